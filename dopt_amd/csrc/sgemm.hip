@@ -25,7 +25,6 @@ struct Gemm {
     int lda, ldb;  // row pitch of A and B as stored
     int mtiles, ntiles, slabs_total, slabs_per_split, splits;
     size_t out_elems;
-    bool quads_a, quads_b;  // sgemm_rows_k: the k-contiguous operand can be read in 16-byte pieces
 };
 
 // An operand tile is BR rows (of M or of N) by BK reduction steps, staged k-major in LDS:
@@ -166,83 +165,100 @@ __global__ __launch_bounds__(kGemmThreads, 2) void sgemm_k(Gemm p)
     }
 }
 
-// The same product with row-major LDS tiles: Xs[r][k], 32 reduction steps per slab at a pitch of 36 floats, so that a
-// lane's operands for eight steps are ONE 128-bit LDS read (lane half h takes steps 8g + 4h .. 8g + 4h + 3 on both
-// operands - any pairing of steps works as long as A and B agree) instead of eight 32-bit reads: 16 LDS reads per
-// 64 matrix instructions where the k-major tiles above need 128.  Every instruction a wavefront issues besides the
-// matrix ones costs the matrix pipe about four cycles, which is what the large products lost.
-//   k-contiguous operand: a thread copies 16-byte pieces, eight lanes per 128-byte row segment (whole cache lines);
-//   r-contiguous operand: a thread gathers four reduction steps of one row with 4-byte loads (64 lanes = 256
-//     contiguous bytes per load) and stores them as one quad - the transposition happens in registers.
-// 128 x 128 tiles, four wavefronts of 64 x 64, two workgroups per CU.  It serves every product of more than 64 rows,
-// whatever the operands' alignment and however they are transposed, so that one (M, N, K) always adds its terms in
-// one order (a plan that reads a transposed operand in place gets the bits of the plan that copies it first).
-constexpr int BK2 = 32, kPitch2 = BK2 + 4;
+// The same product on the bf16 matrix instructions (mfma_core.h): operands are split into three bf16 parts on their way
+// into LDS.  Bound by the power the matrix cores may draw (4096 x 4096 x 4096: the cores busy 71 % of the cycles at 1.6 of
+// 2.4 GHz), then by what a wavefront issues beside its matrix instructions - reading fragments, splitting, arranging
+// operands - which must fit into the slots they leave (eight per instruction); it goes with the sides of a wavefront's
+// tile.  Eight wavefronts of 128 x 64 in 256 x 256 tiles, one workgroup per CU: 1068 -> 640 us for 4096 x 4096 x 4096
+// (129 -> 215 TFLOP/s); 64 x 64 in 128 x 256 and 256 x 128: 755 us; 64 x 32 in 128 x 128: 965 us, for outputs too small
+// to give every CU a larger tile.  The smaller ones have registers for a second set of accumulators.
+// In the largest tile half of the threads stage A, half B, each a block of four rows by four steps: of a k-contiguous operand four 16-byte
+// pieces of four rows (four lanes per 64-byte row segment), of an r-contiguous one four 16-byte pieces of four steps
+// (sixteen lanes per 256 bytes), which become the quads of four rows by naming the registers.
+// It serves every product of more than 64 rows, whatever the operands' alignment and however they are transposed, so
+// that one (M, N, K) always adds its terms in one order (a plan that reads a transposed operand in place gets the bits
+// of the plan that copies it first).
+//
+// A row's 16 steps in LDS are a line of 128 bytes: four pieces of 16 bytes with the (h, m) parts of a quad each, then two
+// pieces with the l parts of two quads each; piece p lies at place p ^ f(row), and the halves of an l piece change places
+// with bit 3 of the row.  f exclusive-ors 4, 2 and 5 for the low three bits of the row, so that the lanes which the LDS
+// serves in one cycle - one piece of eight rows or half a piece of sixteen when reading, four pieces of two rows four
+// apart when writing - touch different banks (a pitch of 112 bytes without the exchange lost a quarter of the loop to
+// conflicts).
+constexpr int kRowBytes = 128, kRowsThreads = 512;
+__device__ __forceinline__ int row_swap(int row) { return (row & 1) << 6 ^ (row & 2) << 4 ^ (row & 4) * 20; }   // 16 f(row)
+__device__ __forceinline__ int hm_at(int row, int quad) { return row * kRowBytes + (16 * quad ^ row_swap(row)); }
+__device__ __forceinline__ int l_at(int row, int quad)
+{
+    return row * kRowBytes + ((64 + 16 * (quad >> 1)) ^ row_swap(row)) + (8 * (quad & 1) ^ (row & 8));
+}
 
 // Loads go through a buffer resource: an element outside the tile's rows or past the end of the reduction is fetched
 // from kOobOffset, where the hardware range check returns zero, so the loop holds no branch and every load of a slab is
 // in flight at once (guarded plain loads compile to one exec-masked region each, with waits in between).
-template <bool kKContig, bool kQuads>
-struct Stage2 {
-    float4 q[4];        // the staged quads: 128 rows x 8 quads over 256 threads
-    unsigned base[4];   // byte offset of quad i at reduction step 0, or kOobOffset when its row is outside the matrix
-    int kq[4];          // first reduction step of quad i inside a slab
-    unsigned step;      // bytes between consecutive reduction steps (r-contiguous: the row pitch)
-    __device__ void init(int ld, int r_base, int r_max, int tid)
+// Pieces are 16 bytes whatever their alignment, and the range check works dword by dword (measured), so a piece may also
+// stick out of the buffer.  One that sticks out of the matrix without leaving the buffer brings rows nobody stores
+// (r-contiguous) or steps past the end of the reduction (k-contiguous, K no multiple of four: kCut), which are zeroed.
+template <bool kCut>
+struct Stage3 {
+    float4 q[4];        // kc: four steps of row i; else four rows of step i
+    unsigned base;      // byte offset of the block at the slab's first step, or kOobOffset when it lies outside the matrix
+    int left;           // kCut: steps of the loaded pieces that lie before the end of the reduction
+    int k0, rows;       // the block's first step inside a slab; how many of its rows lie inside the matrix
+    int hm, l;          // where the parts of its first row go
+    unsigned step, line;   // bytes between consecutive steps; between pieces
+    bool kc;
+    __device__ void init(bool k_contig, int ld, int r_base, int r_max, int t)
     {
-        step = kKContig ? 4u : (unsigned)ld * 4u;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            int row;
-            if (kKContig) {
-                const int idx = tid + 256 * i;
-                row = idx >> 3;
-                kq[i] = 4 * (idx & 7);
-            } else {
-                row = tid & 127;
-                kq[i] = 4 * ((tid >> 7) + 2 * i);
-            }
-            const int r = r_base + row;
-            const unsigned at = kKContig ? ((unsigned)r * (unsigned)ld + (unsigned)kq[i]) * 4u
-                                         : ((unsigned)kq[i] * (unsigned)ld + (unsigned)r) * 4u;
-            base[i] = r < r_max ? at : kOobOffset;
-        }
+        kc = k_contig;
+        line = (unsigned)ld * 4u;
+        step = kc ? 4u : line;
+        k0 = 4 * (t & 3);
+        const int row = t >> 2 << 2, r = r_base + row;
+        rows = r_max - r;
+        hm = hm_at(row, t & 3);
+        l = l_at(row, t & 3);
+        base = rows > 0 ? (unsigned)r * (kc ? line : 4u) + (unsigned)k0 * step : kOobOffset;
     }
-    // kQuads: the rows of a k-contiguous operand are 16-byte addressable (pitch and the reduction's ends multiples of
-    // 4, aligned base); otherwise its pieces are fetched element by element - same values, same order of the sums.
     // A slab wholly past the end of the reduction loads nothing (every offset out of range).
-    __device__ void load(__amdgpu_buffer_rsrc_t rs, int k0, int k_max)
+    __device__ void load(__amdgpu_buffer_rsrc_t rs, int k, int k_max)
     {
-        const unsigned soff = (unsigned)k0 * step;
+        const unsigned soff = (unsigned)k * step;
+        const int steps = k_max - k - k0;
+        const int pieces = !kc ? steps : steps > 0 ? rows : 0;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int k = k0 + kq[i];
-            if (kKContig && kQuads) {
-                q[i] = buffer_load_f32x4(rs, k < k_max ? base[i] : kOobOffset, soff);
-            } else {
-                q[i].x = buffer_load_f32(rs, k + 0 < k_max ? base[i] : kOobOffset, soff);
-                q[i].y = buffer_load_f32(rs, k + 1 < k_max ? base[i] + step : kOobOffset, soff);
-                q[i].z = buffer_load_f32(rs, k + 2 < k_max ? base[i] + 2u * step : kOobOffset, soff);
-                q[i].w = buffer_load_f32(rs, k + 3 < k_max ? base[i] + 3u * step : kOobOffset, soff);
-            }
-        }
+        for (int i = 0; i < 4; i++) q[i] = buffer_load_f32x4(rs, i < pieces ? base : kOobOffset, soff + i * line);
+        if (kCut) left = kc ? steps : 4;
     }
-    __device__ void store(float *Xs, int tid) const
+    // Splits the four steps of the block's row e and stores them.
+    __device__ void store(char *Xs, int e) const
     {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int row = kKContig ? (tid + 256 * i) >> 3 : tid & 127;
-            *(float4 *)&Xs[row * kPitch2 + kq[i]] = q[i];
-        }
+        auto pick = [&](int i) { const float4 v = q[i]; return e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w; };
+        const float4 own = q[e], across = make_float4(pick(0), pick(1), pick(2), pick(3));
+        float4 v = make_float4(kc ? own.x : across.x, kc ? own.y : across.y, kc ? own.z : across.z, kc ? own.w : across.w);
+        if (kCut) v = make_float4(v.x, left > 1 ? v.y : 0.0f, left > 2 ? v.z : 0.0f, left > 3 ? v.w : 0.0f);
+        v4u a;
+        uint2 b;
+        split_quad(v, a, b);
+        *(v4u *)(Xs + (hm ^ row_swap(e)) + e * kRowBytes) = a;
+        *(uint2 *)(Xs + (l ^ row_swap(e)) + e * kRowBytes) = b;
     }
 };
 
-template <bool kTA, bool kTB, bool kQA, bool kQB>
-__global__ __launch_bounds__(kGemmThreads, 2) void sgemm_rows_k(Gemm p)
+// WM x WN wavefronts of MI x NI 32 x 32 pieces each.
+template <int WM_, int WN_, int MI_, int NI_>
+struct RowsTile {
+    static constexpr int WM = WM_, WN = WN_, MI = MI_, NI = NI_, BM = 32 * WM * MI, BN = 32 * WN * NI;
+    static constexpr int kBuf = (BM + BN) * kRowBytes;   // a buffer: the lines of A, then those of B
+    static constexpr bool kLow = MI * NI <= 4;
+    static_assert(WM * WN * 64 == kRowsThreads && BM % 64 == 0 && BN % 64 == 0 && BM + BN <= kRowsThreads, "one block of four rows by four steps per thread");
+};
+
+template <class T, bool kTA, bool kTB, bool kCut>
+__global__ __launch_bounds__(kRowsThreads, 2) void sgemm_rows_k(Gemm p)
 {
-    constexpr int BM = 128, BN = 128;
-    __shared__ __attribute__((aligned(16))) float As[2][BM * kPitch2];
-    __shared__ __attribute__((aligned(16))) float Bs[2][BN * kPitch2];
+    constexpr int MI = T::MI, NI = T::NI, kBuf = T::kBuf;
+    extern __shared__ __attribute__((aligned(16))) char rows_lds[];
 
     unsigned L;
     const unsigned tiles = (unsigned)(p.mtiles * p.ntiles);
@@ -250,89 +266,186 @@ __global__ __launch_bounds__(kGemmThreads, 2) void sgemm_rows_k(Gemm p)
     const int split = (int)(L / tiles);
     const unsigned tile = L - (unsigned)split * tiles;
     const int mt = (int)(tile % (unsigned)p.mtiles), nt = (int)(tile / (unsigned)p.mtiles);
-    const int m0 = mt * BM, n0 = nt * BN;
-    // p.slabs_* count 16-step slabs (the other kernel's unit): two of them per slab here
+    const int m0 = mt * T::BM, n0 = nt * T::BN;
     const int k_begin = split * p.slabs_per_split * BK;
     const int k_end = min(min(k_begin + p.slabs_per_split * BK, p.slabs_total * BK), p.K);
 
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, l32 = lane & 31, kh = lane >> 5;
-    const int wm = w >> 1, wn = w & 1;
-    const int a_frag = (wm * 64 + l32) * kPitch2 + 4 * kh, b_frag = (wn * 64 + l32) * kPitch2 + 4 * kh;
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, kh = lane >> 5;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), wm = w / T::WN, wn = w % T::WN;
+    const int arow = wm * 32 * MI + l32, brow = wn * 32 * NI + l32;
 
-    v16f acc[2][2];
-    zero_acc(acc);
-    const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.A, (size_t)p.M * p.K * sizeof(float));
-    const __amdgpu_buffer_rsrc_t rb = make_rsrc(p.B, (size_t)p.K * p.N * sizeof(float));
-    // Two register sets: while slab s is multiplied out of LDS, slab s + 1 waits in one set to be stored behind it and
-    // slab s + 2 is on its way into the other, so a load has two slabs' worth of matrix work to arrive.  No branch
-    // inside the loop: loads behind the last slab fall out of range and fetch nothing, their stores fill a buffer
-    // nobody reads.
-    Stage2<!kTA, kQA> la[2];   // A as given is k-contiguous
-    Stage2<kTB, kQB> lb[2];    // B transposed is k-contiguous
+    // low: the four smaller kinds of products, where there are registers for them
+    constexpr bool kLow = T::kLow;
+    v16f acc[MI][NI], low[kLow ? MI : 1][kLow ? NI : 1];
+    // Slab s is multiplied out of one LDS buffer in two groups of 3 MI NI matrix instructions (quads 0 and 1, quads 2 and 3).
+    // Between them slab s + 1, fetched an iteration ago, is split and stored into the other buffer, and slab s + 2 is
+    // requested.  A group's fragments are read while the group before it is multiplied; those of the next slab's first
+    // group after the one barrier of the slab, which stands a third into the second group: by then this slab has been
+    // read whole and the next one is stored whole.  Loads behind the last slab fall out of range and fetch nothing, what
+    // is made of them is never multiplied.
+    // the first BM / 64 wavefronts stage A, the next BN / 64 stage B; wavefronts beyond repeat what the first ones do
+    constexpr int kStagers = (T::BM + T::BN) / 64;
+    const int sw = w < kStagers ? w : w - kStagers;
+    const bool for_b = sw >= T::BM / 64;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(for_b ? p.B : p.A, (size_t)(for_b ? p.N : p.M) * p.K * sizeof(float));
+    Stage3<kCut> st;
+    st.init(kTA != kTB ? !kTA : for_b ? kTB : !kTA, for_b ? p.ldb : p.lda, for_b ? n0 : m0, for_b ? p.N : p.M,
+            (for_b ? sw - T::BM / 64 : sw) * 64 + lane);
+    char *const mine = rows_lds + (for_b ? T::BM * kRowBytes : 0);
+    const int ahm = hm_at(arow, kh), al = l_at(arow, kh), bhm = hm_at(T::BM + brow, kh), bl = l_at(T::BM + brow, kh);
+    // The fragments of a group: lane half kh takes quad 2g + kh of its rows.  Which quad differs from quad kh's place by
+    // an exclusive or, made here so that the addresses do not hold registers.
+    v4u fa[2][MI], fb[2][NI];
+    uint2 la[MI], lb[NI];
+    auto read_hm = [&](const char *buf, int g) {
+        int x = 32 * g;
+        asm volatile("" : "+s"(x));
+        const char *const pa = buf + (ahm ^ x), *const pb = buf + (bhm ^ x);
 #pragma unroll
-    for (int u = 0; u < 2; u++) {
-        la[u].init(p.lda, m0, p.M, tid);
-        lb[u].init(p.ldb, n0, p.N, tid);
-    }
-    la[0].load(ra, k_begin, k_end);
-    lb[0].load(rb, k_begin, k_end);
-    la[1].load(ra, k_begin + BK2, k_end);
-    lb[1].load(rb, k_begin + BK2, k_end);
-    la[0].store(As[0], tid);
-    lb[0].store(Bs[0], tid);
-    __syncthreads();
-    auto slab = [&](const float *as, const float *bs) {
+        for (int i = 0; i < MI; i++) fa[g][i] = *(const v4u *)(pa + 32 * i * kRowBytes);
 #pragma unroll
-        for (int g = 0; g < BK2 / 8; g++) {
-            float4 a[2], b[2];
+        for (int j = 0; j < NI; j++) fb[g][j] = *(const v4u *)(pb + 32 * j * kRowBytes);
+    };
+    auto read_l = [&](const char *buf, int g) {
+        int x = 16 * g;
+        asm volatile("" : "+s"(x));
+        const char *const pa = buf + (al ^ x), *const pb = buf + (bl ^ x);
 #pragma unroll
-            for (int i = 0; i < 2; i++) a[i] = *(const float4 *)(as + i * 32 * kPitch2 + 8 * g);
+        for (int i = 0; i < MI; i++) la[i] = *(const uint2 *)(pa + 32 * i * kRowBytes);
 #pragma unroll
-            for (int j = 0; j < 2; j++) b[j] = *(const float4 *)(bs + j * 32 * kPitch2 + 8 * g);
-            // step by step over the four accumulators: consecutive matrix instructions never wait for each other
+        for (int j = 0; j < NI; j++) lb[j] = *(const uint2 *)(pb + 32 * j * kRowBytes);
+    };
+    // The matrix instructions of group g, in three parts: (l, h) . (h, l), (h, m) . (m, h), (h, m) . (h, m)
+    auto part = [&](int g, int kind) {
+        v4u b[NI];
 #pragma unroll
-            for (int e = 0; e < 4; e++)
+        for (int j = 0; j < NI; j++) {
+            const v4u h = fb[g][j];
+            b[j] = kind == 0 ? h : kind == 1 ? v4u{h.z, h.w, h.x, h.y} : v4u{h.x, h.y, lb[j].x, lb[j].y};
+        }
 #pragma unroll
-                for (int i = 0; i < 2; i++)
+        for (int i = 0; i < MI; i++) {
+            const v4u a = kind < 2 ? fa[g][i] : v4u{la[i].x, la[i].y, fa[g][i].x, fa[g][i].y};
 #pragma unroll
-                    for (int j = 0; j < 2; j++) {
-                        const float av = e == 0 ? a[i].x : e == 1 ? a[i].y : e == 2 ? a[i].z : a[i].w;
-                        const float bv = e == 0 ? b[j].x : e == 1 ? b[j].y : e == 2 ? b[j].z : b[j].w;
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc[i][j], 0, 0, 0);
-                    }
+            for (int j = 0; j < NI; j++) {
+                v16f &c = kLow && kind ? low[i % (kLow ? MI : 1)][j % (kLow ? NI : 1)] : acc[i][j];
+                c = mfma_bf16(a, b[j], c);
+            }
         }
     };
-    // iteration pair: slab k0 from buffer 0 (set 1 holds k0 + 32, set 0 is refilled with k0 + 64), then slab k0 + 32
-    // from buffer 1 (set 0 holds k0 + 64, set 1 is refilled with k0 + 96)
-    for (int k0 = k_begin; k0 < k_end; k0 += 2 * BK2) {
-        la[0].load(ra, k0 + 2 * BK2, k_end);
-        lb[0].load(rb, k0 + 2 * BK2, k_end);
-        slab(As[0] + a_frag, Bs[0] + b_frag);
-        la[1].store(As[1], tid);
-        lb[1].store(Bs[1], tid);
-        __syncthreads();
-        if (k0 + BK2 >= k_end) break;   // uniform
-        la[1].load(ra, k0 + 3 * BK2, k_end);
-        lb[1].load(rb, k0 + 3 * BK2, k_end);
-        slab(As[1] + a_frag, Bs[1] + b_frag);
-        la[0].store(As[0], tid);
-        lb[0].store(Bs[0], tid);
-        __syncthreads();
-    }
-
-    float *outp = p.C + (size_t)split * p.out_elems;
+    float *const outp = p.C + (size_t)split * p.out_elems + (size_t)(m0 + wm * 32 * MI) * p.N + n0 + brow;
+    const bool whole = m0 + T::BM <= p.M && n0 + T::BN <= p.N;
+    // C = the accumulators, plus what C holds when `add`; no guards inside the matrix, and a block's loads go out together
+    auto put = [&](bool add) {
+        int pitch = p.N;
+        asm volatile("" : "+s"(pitch));   // no row address is held across the reduction
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int col = n0 + wn * 64 + j * 32 + l32;
-        if (col >= p.N) continue;
+        for (int i = 0; i < MI; i++)
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+            for (int j = 0; j < NI; j++) {
+                float *const at = outp + (size_t)(i * 32 + 4 * kh) * pitch + 32 * j;
+                if (whole) {
+                    float old[16];
+                    if (add) {
 #pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int m = m0 + wm * 64 + i * 32 + acc_row(v, lane);
-                if (m < p.M) outp[(size_t)m * p.N + col] = acc[i][j][v];
+                        for (int v = 0; v < 16; v++) old[v] = at[(size_t)(8 * (v >> 2) + (v & 3)) * pitch];
+#pragma unroll
+                        for (int v = 0; v < 16; v++) acc[i][j][v] += old[v];
+                    }
+#pragma unroll
+                    for (int v = 0; v < 16; v++) at[(size_t)(8 * (v >> 2) + (v & 3)) * pitch] = acc[i][j][v];
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 16; v++) {
+                        const int m = m0 + wm * 32 * MI + i * 32 + acc_row(v, lane);
+                        float *const c = at + (size_t)(8 * (v >> 2) + (v & 3)) * pitch;
+                        if (m < p.M && n0 + brow + 32 * j < p.N) *c = add ? *c + acc[i][j][v] : acc[i][j][v];
+                    }
+                }
             }
+    };
+    // With one accumulator for all products the sum is rounded twelve times per 16 steps, which the fp32 instruction
+    // rounds eight times; two sums over half the steps each have half the error.  The first of them waits in C.  (A
+    // reduction cut over blocks is such sums already.)
+    const int half = kLow || p.splits > 1 ? k_end : k_begin + (k_end - k_begin + 2 * BK - 1) / (2 * BK) * BK;
+    float top = 0.0f;   // NaN once anything is not finite: x * 0 is 0 for finite x only
+#pragma clang loop unroll(disable)
+    for (int from = k_begin, to = half; from < k_end; from = to, to = k_end) {
+        zero_acc(acc);
+        zero_acc(low);
+        st.load(rs, from, to);
+#pragma unroll
+        for (int e = 0; e < 4; e++) st.store(mine, e);
+        st.load(rs, from + BK, to);
+        __syncthreads();
+        read_hm(rows_lds, 0);
+        read_l(rows_lds, 0);
+        for (int k0 = from; k0 < to; k0 += 2 * BK) {
+#pragma unroll
+            for (int cur = 0; cur < 2; cur++) {
+                if (cur && k0 + BK >= to) break;   // uniform
+                char *const now = rows_lds + cur * kBuf, *const next = mine + (cur ^ 1) * kBuf;
+                st.store(next, 0);
+                part(0, 2);
+                __builtin_amdgcn_sched_barrier(0);
+                read_hm(now, 1);
+                st.store(next, 1);
+                part(0, 1);
+                __builtin_amdgcn_sched_barrier(0);
+                read_l(now, 1);
+                st.store(next, 2);
+                part(0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                st.store(next, 3);
+                st.load(rs, k0 + (cur + 2) * BK, to);
+                part(1, 2);
+                __syncthreads();
+                read_hm(rows_lds + (cur ^ 1) * kBuf, 0);
+                part(1, 1);
+                __builtin_amdgcn_sched_barrier(0);
+                read_l(rows_lds + (cur ^ 1) * kBuf, 0);
+                part(1, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __syncthreads();   // the buffers are free for the second half
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NI; j++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    if (kLow) acc[i][j][v] += low[i % (kLow ? MI : 1)][j % (kLow ? NI : 1)][v];
+                    top = __fmaf_rn(acc[i][j][v], 0.0f, top);
+                }
+        put(from != k_begin);
     }
+    if (!__any(top != 0.0f)) return;
+    {   // an operand or a sum that is not finite: this wavefront's part in fp32 instructions
+        const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.A, (size_t)p.M * p.K * sizeof(float));
+        const __amdgpu_buffer_rsrc_t rb = make_rsrc(p.B, (size_t)p.K * p.N * sizeof(float));
+        zero_acc(acc);
+        for (int k = k_begin + kh; k - kh < k_end; k += 2) {
+            float a[MI], b[NI];
+#pragma unroll
+            for (int i = 0; i < MI; i++) {
+                const int r = m0 + arow + 32 * i;
+                const unsigned at = kTA ? (unsigned)k * (unsigned)p.lda + (unsigned)r : (unsigned)r * (unsigned)p.lda + (unsigned)k;
+                a[i] = buffer_load_f32(ra, r < p.M && k < k_end ? at * 4u : kOobOffset, 0);
+            }
+#pragma unroll
+            for (int j = 0; j < NI; j++) {
+                const int c = n0 + brow + 32 * j;
+                const unsigned bt = kTB ? (unsigned)c * (unsigned)p.ldb + (unsigned)k : (unsigned)k * (unsigned)p.ldb + (unsigned)c;
+                b[j] = buffer_load_f32(rb, c < p.N && k < k_end ? bt * 4u : kOobOffset, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int j = 0; j < NI; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+    }
+    put(false);
 }
 
 // Small outputs (a dense layer at batch 128: 128 x 512 values from a 512-deep reduction).  The tile
@@ -830,14 +943,45 @@ int sgemm_bias(int transA, int transB, size_t M, size_t N, size_t K, const float
 // being asked for, which a kernel without one leaves to a pass behind it; operand alignment picks between variants of a
 // kernel that add in the same order (the LDS-resident kernel apart: panel_allowed = false is the route without it).
 struct Route {
-    enum Kind { kNone, kOuter, kGemvRows, kGemvColsShort, kGemvCols, kPanel, kSmall, kTile64, kTile128, kRows } kind;
+    enum Kind { kNone, kOuter, kGemvRows, kGemvColsShort, kGemvCols, kPanel, kSmall, kTile64, kTile128, kRows, kRowsBig } kind;
     size_t cuts;    // partial sums per element that a second pass adds (gemv slices, tile-engine splits)
     size_t depth;   // reduction steps per partial sum (k per slice, slabs per split)
+    size_t bm = 128, bn = 128;   // the tile engines' tile (no part of the order: every tile of a kind adds its elements' terms alike)
 };
+
+template <class T, bool kTA, bool kTB, bool kCut>
+int rows_launch_one(dim3 grid, const Gemm &g)
+{
+    static bool raised = false;   // above 64 KB of dynamic LDS a kernel has to be told once
+    if (!raised)
+        DOPT_HIP_CHECK(hipFuncSetAttribute((const void *)sgemm_rows_k<T, kTA, kTB, kCut>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           2 * T::kBuf));
+    raised = true;
+    hipLaunchKernelGGL((sgemm_rows_k<T, kTA, kTB, kCut>), grid, dim3(kRowsThreads), 2 * T::kBuf, stream(), g);
+    return DOPT_HIP_OK;
+}
+
+template <bool kTA, bool kTB, bool kCut>
+int rows_launch(const Route &r, dim3 grid, const Gemm &g)
+{
+    if (r.bm == 256 && r.bn == 256) return rows_launch_one<RowsTile<2, 4, 4, 2>, kTA, kTB, kCut>(grid, g);
+    if (r.bm == 256) return rows_launch_one<RowsTile<4, 2, 2, 2>, kTA, kTB, kCut>(grid, g);
+    if (r.bn == 256) return rows_launch_one<RowsTile<2, 4, 2, 2>, kTA, kTB, kCut>(grid, g);
+    return rows_launch_one<RowsTile<2, 4, 2, 1>, kTA, kTB, kCut>(grid, g);
+}
+
+
+// What a tile of sgemm_rows_k costs per 16 steps with every CU at work (4096 x 4096 x 4096: 630, 755 and 965 us); a
+// workgroup's own start and end take about 4 us, split copies are written and read at about 5 TB/s.
+struct RowsShape {
+    size_t bm, bn;
+    double slab_us;
+};
+constexpr RowsShape kRowsShapes[] = {{256, 256, 2.4}, {128, 256, 1.45}, {256, 128, 1.45}, {128, 128, 0.93}};
 
 Route sgemm_route(int transA, int transB, size_t M, size_t N, size_t K, bool panel_allowed = true)
 {
-    Route r{Route::kNone, 1, K};
+    Route r{Route::kNone, 1, K, 0, 0};
     if (M * N == 0 || K == 0) return r;
     if (K == 1) { r.kind = Route::kOuter; return r; }
     // matrix-vector products: `rows` reads the matrix row by row (k contiguous), `cols` column-wise
@@ -860,28 +1004,56 @@ Route sgemm_route(int transA, int transB, size_t M, size_t N, size_t K, bool pan
     if (transA && !transB && panel_allowed && panel_shape(M, N, K)) { r.kind = Route::kPanel; return r; }
     // small and medium outputs: one block per 32 x 32 tile, the reduction split over its wavefronts.
     // Each tile reads its own 32 rows of A and 32 columns of B, so the operand traffic grows with the
-    // number of tiles: up to 256 MB of it (served by the L2) this beats the LDS-tiled engine below,
-    // whose 128-wide tiles leave most CUs with one four-wavefront block (1024 x 1024 x 256: 11 against
-    // 22 us; 2048 x 2048 x 128: 21 against 31 us); beyond that the tile engine's operand reuse wins.
+    // number of tiles; it is served by the L2 at about 10 TB/s (1024 x 1024 x 256: 12 us against 20 us with the kernel
+    // below).  A block by itself takes 5.5 ns per reduction step (256 x 256 x 8192: 49 against 28 us), twice that when rows
+    // of a k-contiguous operand start off the 16-byte grid (1700 x 1501 x 333: 69 against 29 us).
+    const bool offsets32 = M * K < ((size_t)1 << 29) && K * N < ((size_t)1 << 29);
     const size_t tiles32 = ceil_div(M, (size_t)32) * ceil_div(N, (size_t)32);
-    if (tiles32 <= 4096 && tiles32 * 64 * K * sizeof(float) <= ((size_t)256 << 20) && M * K < ((size_t)1 << 29) &&
-        K * N < ((size_t)1 << 29)) {   // (32-bit byte offsets into either operand)
-        r.kind = Route::kSmall;
+    const double traffic = (double)tiles32 * 64 * K * sizeof(float);
+    const bool small = offsets32 && tiles32 <= 4096 && traffic <= (double)(256 << 20);   // (32-bit byte offsets)
+    const double small_us = 4 + (K % 4 ? 2 : 1) * (traffic / 10e6 > 5.5e-3 * K ? traffic / 10e6 : 5.5e-3 * K);
+    const size_t slabs_total = ceil_div(K, (size_t)BK);
+    if (M <= 64 || !offsets32) {
+        if (small) { r.kind = Route::kSmall; return r; }
+        r.kind = M <= 64 ? Route::kTile64 : Route::kTile128;
+        r.bm = M <= 64 ? 64 : 128;
+        r.bn = M <= 64 ? 256 : 128;
+        const size_t tiles = ceil_div(M, r.bm) * ceil_div(N, r.bn);
+        size_t splits = (2 * (size_t)num_cus() + tiles - 1) / tiles;
+        if (splits > slabs_total / 4) splits = slabs_total / 4;
+        if (splits > 32) splits = 32;
+        if (splits < 1) splits = 1;
+        r.depth = ceil_div(slabs_total, splits);
+        r.cuts = ceil_div(slabs_total, r.depth);
         return r;
     }
-    const bool big = M > 64;
-    const size_t BM = big ? 128 : 64, BN = big ? 128 : 256;
-    const size_t tiles = ceil_div(M, BM) * ceil_div(N, BN);
-    const size_t slabs_total = ceil_div(K, (size_t)BK);
-    size_t want = ((size_t)2 * num_cus() + tiles - 1) / tiles;
-    const size_t max_by_depth = slabs_total / 4 > 0 ? slabs_total / 4 : 1;
-    size_t splits = want < max_by_depth ? want : max_by_depth;
-    if (splits > 32) splits = 32;
-    if (splits < 1) splits = 1;
-    r.depth = (slabs_total + splits - 1) / splits;
-    r.cuts = (slabs_total + r.depth - 1) / r.depth;
-    // more than 64 rows: row-major LDS tiles (sgemm_rows_k) while byte offsets into either operand fit 32 bits
-    r.kind = !big ? Route::kTile64 : M * K < ((size_t)1 << 29) && K * N < ((size_t)1 << 29) ? Route::kRows : Route::kTile128;
+    r.kind = Route::kRows;
+    double best = 0;
+    for (const RowsShape &t : kRowsShapes) {
+        const size_t tiles = ceil_div(M, t.bm) * ceil_div(N, t.bn);
+        const bool big = t.bm * t.bn == 256 * 256;
+        if (big && K < 1024) continue;   // one accumulator per value: two halves of the reduction have to be long
+        // a sum of more terms than this is cut (the matrix unit rounds down by little: 16384 products of non-negative
+        // values came out 1.2e-6 too small, 4096 by 2e-7, where rounding to nearest is 1.0e-6 and 5e-7 off)
+        const size_t longest = 4096 / BK;
+        size_t least = big && slabs_total <= 2 * longest ? 1 : ceil_div(slabs_total, longest);
+        if (least > 32) least = 32;
+        for (size_t splits = least; splits <= 32 && (splits == least || splits * 4 <= slabs_total); splits++) {
+            const size_t depth = ceil_div(slabs_total, splits), cuts = ceil_div(slabs_total, depth);
+            if (cuts != splits && splits != least) continue;
+            const double us = (double)ceil_div(tiles * cuts, (size_t)num_cus()) * (depth * t.slab_us + 4) +
+                              (double)M * N * 4 / 5e6 * (cuts > 1 ? 2 * cuts + 1 : big ? 3 : 1) + (cuts > 1 ? 5 : 0);
+            if (best == 0 || us < best) {
+                best = us;
+                r.kind = big ? Route::kRowsBig : Route::kRows;
+                r.bm = t.bm;
+                r.bn = t.bn;
+                r.depth = depth;
+                r.cuts = cuts;
+            }
+        }
+    }
+    if (small && small_us < best) r = Route{Route::kSmall, 1, K, 0, 0};
     return r;
 }
 
@@ -975,9 +1147,8 @@ int sgemm_epilogue(int transA, int transB, size_t M, size_t N, size_t K, const f
     g.out_elems = M * N;
     g.slabs_total = (int)ceil_div(K, (size_t)BK);
     const bool big = kind != Route::kTile64;
-    const int BM = big ? 128 : 64, BN = big ? 128 : 256;
-    g.mtiles = (int)ceil_div(M, (size_t)BM);
-    g.ntiles = (int)ceil_div(N, (size_t)BN);
+    g.mtiles = (int)ceil_div(M, route.bm);
+    g.ntiles = (int)ceil_div(N, route.bn);
     const int tiles = g.mtiles * g.ntiles;
     const int splits = (int)route.cuts;
     g.slabs_per_split = (int)route.depth;
@@ -1003,20 +1174,16 @@ int sgemm_epilogue(int transA, int transB, size_t M, size_t N, size_t K, const f
         else if (!transB) DOPT_SGEMM(BMV, true, false);     \
         else DOPT_SGEMM(BMV, true, true);                   \
     } while (0)
-    // more than 64 rows: row-major LDS tiles (sgemm_rows_k)
-    g.quads_a = g.lda % 4 == 0 && K % 4 == 0 && aligned16(A);
-    g.quads_b = g.ldb % 4 == 0 && K % 4 == 0 && aligned16(B);
-    if (kind == Route::kRows) {
-#define DOPT_ROWS(TA, TB, QA, QB) hipLaunchKernelGGL((sgemm_rows_k<TA, TB, QA, QB>), grid, dim3(kGemmThreads), 0, stream(), g)
-        const bool qa = g.quads_a, qb = g.quads_b;   // only a k-contiguous operand has the choice
-        if (!transA && !transB) { if (qa) DOPT_ROWS(false, false, true, false); else DOPT_ROWS(false, false, false, false); }
-        else if (!transA) {
-            if (qa && qb) DOPT_ROWS(false, true, true, true);
-            else if (qa) DOPT_ROWS(false, true, true, false);
-            else if (qb) DOPT_ROWS(false, true, false, true);
-            else DOPT_ROWS(false, true, false, false);
-        } else if (!transB) DOPT_ROWS(true, false, false, false);
-        else { if (qb) DOPT_ROWS(true, true, false, true); else DOPT_ROWS(true, true, false, false); }
+    if (kind == Route::kRows || kind == Route::kRowsBig) {
+        const bool cut = K % 4 != 0;
+#define DOPT_ROWS(TA, TB)                                                                                \
+    do {                                                                                                 \
+        if (int rc = cut ? rows_launch<TA, TB, true>(route, grid, g) : rows_launch<TA, TB, false>(route, grid, g)) return rc; \
+    } while (0)
+        if (!transA && !transB) DOPT_ROWS(false, false);
+        else if (!transA) DOPT_ROWS(false, true);
+        else if (!transB) { if (int rc = rows_launch<true, false, false>(route, grid, g)) return rc; }   // nothing k-contiguous to cut
+        else DOPT_ROWS(true, true);
 #undef DOPT_ROWS
     } else if (big) DOPT_SGEMM_T(128);
     else DOPT_SGEMM_T(64);
@@ -1076,7 +1243,7 @@ int dopt_hip_sgemm_batch(int n, const int *transA, const int *transB, const size
     for (int i = 0; i < n; i++) {
         if (M[i] * N[i] == 0) continue;
         const bool plain = K[i] > 0 && A[i] && B[i] && C[i] && M[i] < ((size_t)1 << 30) && N[i] < ((size_t)1 << 30) && K[i] < ((size_t)1 << 30);
-        const Route r = plain ? sgemm_route(transA[i], transB[i], M[i], N[i], K[i]) : Route{Route::kNone, 1, 0};
+        const Route r = plain ? sgemm_route(transA[i], transB[i], M[i], N[i], K[i]) : Route{Route::kNone, 1, 0, 0, 0};
         if (r.kind == Route::kGemvColsShort && gemvs.size() < (size_t)kGroupJobs) {
             const size_t R = M[i] == 1 ? N[i] : M[i];
             GemvJob q{};
