@@ -478,11 +478,61 @@ constexpr int kWinoXchg = 4 * 64 * 64;   // floats of the exchange area: four wa
 // WK x TH: the eight wavefronts are WK groups of 32 rows x TH groups of 32 tiles x the two halves of the 16 positions:
 // 4 x 1 (128 rows x 32 tiles = 128 pixels) for layers with whole 128-row tiles, 2 x 2 (64 rows x 64 tiles = 256 pixels)
 // for 64-row layers.
+// The four outputs of one tile and row over channels c0 .. c1 - 1, in fp32 without matrix instructions: for the tiles whose
+// operands or results are not finite.  (ih0, iw0): the tile's first input pixel.
+__device__ __forceinline__ void wino_fp32(const PatchConv &p, int n, int m, int ih0, int iw0, int c0, int c1, float (&y)[4])
+{
+    float M[16];
+#pragma unroll
+    for (int x = 0; x < 16; x++) M[x] = 0.0f;
+    const unsigned short *wp = (const unsigned short *)p.wp;
+#pragma unroll 1
+    for (int c = c0; c < c1; c++) {
+        const float *in = p.in + ((size_t)n * p.Cin + c) * p.IH * p.IW;
+        float d[4][4];
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int ih = ih0 + r, iw = iw0 + q;
+                d[r][q] = ih >= 0 && ih < p.IH && iw >= 0 && iw < p.IW ? in[ih * p.IW + iw] : 0.0f;
+            }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float t[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                t[q] = i == 0 ? d[0][q] - d[2][q] : i == 1 ? d[1][q] + d[2][q] : i == 2 ? d[2][q] - d[1][q] : d[1][q] - d[3][q];
+            const float v[4] = {t[0] - t[2], t[1] + t[2], t[2] - t[1], t[1] - t[3]};
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const size_t at = (((size_t)(c / 16) * 16 + i * 4 + j) * 3 * p.Mp + m) * 16 + c % 16, part = (size_t)p.Mp * 16;
+                auto val = [&](size_t a) { return __builtin_bit_cast(float, (unsigned)wp[a] << 16); };
+                M[i * 4 + j] += (val(at) + val(at + part) + val(at + 2 * part)) * v[j];
+            }
+        }
+    }
+    float z[4][2];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        z[i][0] = (M[4 * i] + M[4 * i + 1]) + M[4 * i + 2];
+        z[i][1] = (M[4 * i + 1] - M[4 * i + 2]) - M[4 * i + 3];
+    }
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+        y[b] = (z[0][b] + z[1][b]) + z[2][b];
+        y[2 + b] = (z[1][b] - z[2][b]) - z[3][b];
+    }
+}
+
 template <int NPMAX, int WK, int TH>
 __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
 {
     static_assert(WK * TH == 4 && NPMAX == 16, "eight wavefronts, sixteen channels per chunk");
-    constexpr int BM = 32 * WK, BN = 128 * TH, TT = 32 * TH, CH = 16, LDP = 20, VSZ = 16 * TT * LDP;
+    constexpr int BM = 32 * WK, BN = 128 * TH, TT = 32 * TH, CH = 16, LDP = 20;
+    // V in words: [16 positions][part h, m, l][channel half][tile][8 channels as 4 words] - a lane's fragment of one part is
+    // one 128-bit read and neighbouring lanes' reads are neighbours
+    constexpr int VP = 8 * TT, VX = 3 * VP, VSZ = 16 * VX;
     // 32 tiles per workgroup: V and the raw patch are double-buffered, the transform of the next chunk runs under this
     // chunk's matrix instructions and the workgroup meets once per chunk.  64 tiles: one V (80 KB), transformed between
     // two barriers.
@@ -490,7 +540,7 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int raw_floats = ((p.psz + 1) * LDP + 3) / 4 * 4;   // one spare position absorbs the stores of idle threads
     float *const raw0 = lds;
-    float *const V0 = lds + (DB ? 2 : 1) * raw_floats;          // [16][TT][LDP] (x 2)
+    float *const V0 = lds + (DB ? 2 : 1) * raw_floats;          // (x 2)
 
     unsigned L;
     const unsigned tiles = (unsigned)(p.mtiles * p.ntiles);
@@ -548,13 +598,16 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
     float sg[TH];
 #pragma unroll
     for (int u = 0; u < TH; u++) {
-        const int item = u * 512 + tid, ti = item / (TT * 4), tau_t = (item % (TT * 4)) >> 2, cq = item & 3;
+        // (two of the four channel quads on neighbouring lanes, the other two a multiple of 64 lanes on: neither the reads of
+        // the patch nor the 64-bit writes of the parts meet in a bank)
+        const int item = u * 512 + tid, ti = item / (TT * 4), tau_t = (item >> 1) % TT, cqh = (item / (TT * 2)) & 1;
+        const int cq = 2 * cqh + (item & 1);
         const int img = tau_t / tpi, tl = tau_t - img * tpi, r2 = tl / tcn, c2 = tl - r2 * tcn;
         const int t_in = ((img * p.PR + 2 * r2) * p.PC + 2 * c2) * LDP + cq * 4;
         const int ra = ti == 0 ? 0 : ti == 2 ? 2 : 1, rb = ti == 0 ? 2 : ti == 1 ? 2 : ti == 2 ? 1 : 3;
         t_a[u] = t_in + ra * p.PC * LDP;
         t_b[u] = t_in + rb * p.PC * LDP;
-        t_out[u] = ((ti * 4) * TT + tau_t) * LDP + cq * 4;
+        t_out[u] = ti * 4 * VX + cqh * (4 * TT) + tau_t * 4 + (item & 1) * 2;
         sg[u] = ti == 1 ? 1.0f : -1.0f;
     }
     float4 tt[TH][4];
@@ -567,28 +620,38 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
                                    __builtin_fmaf(sg[u], db.z, da.z), __builtin_fmaf(sg[u], db.w, da.w));
         }
     };
-    auto transform_write = [&](float *Vb) {                      // ... times B: four positions, four channels each
-        auto sub = [](float4 x, float4 y) { return make_float4(x.x - y.x, x.y - y.y, x.z - y.z, x.w - y.w); };
-        auto add = [](float4 x, float4 y) { return make_float4(x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w); };
+    auto transform_write = [&](float *Vb, int j) {               // ... times B, position j of the row, split into its parts
 #pragma unroll
         for (int u = 0; u < TH; u++) {
-            *(float4 *)(Vb + t_out[u]) = sub(tt[u][0], tt[u][2]);
-            *(float4 *)(Vb + t_out[u] + TT * LDP) = add(tt[u][1], tt[u][2]);
-            *(float4 *)(Vb + t_out[u] + 2 * TT * LDP) = sub(tt[u][2], tt[u][1]);
-            *(float4 *)(Vb + t_out[u] + 3 * TT * LDP) = sub(tt[u][1], tt[u][3]);
+            const float4 x = tt[u][j == 0 ? 0 : j == 2 ? 2 : 1], y = tt[u][j < 2 ? 2 : j == 2 ? 1 : 3];
+            const float s = j == 1 ? 1.0f : -1.0f;
+            uint2 h, m, l;
+            split_pair(__builtin_fmaf(s, y.x, x.x), __builtin_fmaf(s, y.y, x.y), h.x, m.x, l.x);
+            split_pair(__builtin_fmaf(s, y.z, x.z), __builtin_fmaf(s, y.w, x.w), h.y, m.y, l.y);
+            float *const o = Vb + t_out[u] + j * VX;
+            *(uint2 *)o = h;
+            *(uint2 *)(o + VP) = m;
+            *(uint2 *)(o + 2 * VP) = l;
         }
     };
 
     // ---- transformed-filter fragments: this lane's 8 channels (kh * 8 ..) of row m0 + 32 wk + l32
-    const unsigned slab_bytes = (unsigned)p.Mp * CH * 4u;
-    const unsigned fa_voff = (unsigned)((m0 + wk * 32 + l32) * CH + kh * 8) * 4u;
-    float4 fa_ring[4][2];
-    auto fa_load = [&](auto slot_tag, int slab) {   // past the last slab the range check returns zeros
+    // [chunk][position][part][row][16 channels]
+    const unsigned part_bytes = (unsigned)p.Mp * CH * 2u, slab_bytes = 3u * part_bytes;
+    const unsigned fa_voff = (unsigned)((m0 + wk * 32 + l32) * CH + kh * 8) * 2u;
+    v4u fa_ring[4][3];
+    auto fa_load = [&](auto slot_tag, int slab) {
         constexpr int slot = decltype(slot_tag)::value;
-        fa_ring[slot][0] = buffer_load_f32x4(rwp, fa_voff, (unsigned)slab * slab_bytes);
-        fa_ring[slot][1] = buffer_load_f32x4(rwp, fa_voff + 16u, (unsigned)slab * slab_bytes);
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+            fa_ring[slot][q] = __builtin_bit_cast(v4u, buffer_load_f32x4(rwp, fa_voff, (unsigned)slab * slab_bytes + q * part_bytes));
     };
-    const int b_frag = (wi * 8 * TT + th * 32 + l32) * LDP + kh * 8;   // position 8 wi, this lane's tile and channels
+    const int b_frag = wi * 8 * VX + kh * (4 * TT) + (th * 32 + l32) * 4;   // position 8 wi, this lane's tile and channels
+    v4u fb_next[3];
+    auto fb_load = [&](const float *Vb, int x) {
+#pragma unroll
+        for (int q = 0; q < 3; q++) fb_next[q] = *(const v4u *)(Vb + b_frag + x * VX + q * VP);
+    };
 
     v16f acc[8];
 #pragma unroll
@@ -625,13 +688,12 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
     __syncthreads();
 #pragma unroll
     for (int b = 0; b < 4; b++) transform_read(b, raw0);
-    transform_write(V0);
+#pragma unroll
+    for (int b = 0; b < 4; b++) transform_write(V0, b);
     __syncthreads();
 
     constexpr int PER = NPMAX / 4;
-    float4 fb_next[2];
-    fb_next[0] = *(const float4 *)(V0 + b_frag);
-    fb_next[1] = *(const float4 *)(V0 + b_frag + 4);
+    fb_load(V0, 0);
     for (int it = 0; it < nch; ++it) {
         const int chunk = cb + it;
         // double-buffered: V of this chunk, raw patch and V of the next one, raw patch of the one after (into the buffer
@@ -642,21 +704,19 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
         float *const raww = raw0 + (DB ? (it & 1) * raw_floats : 0);
         const int ahead = DB ? 2 : 1;
         const bool more = it + 1 < nch, fetch = it + ahead < nch;
+        const int chunk_next = more ? chunk + 1 : chunk;   // (after the last chunk: loaded, not used)
         static_for<0, 8>([&](auto xtag) {
             constexpr int xl = decltype(xtag)::value;
-            const float4 fb0 = fb_next[0], fb1 = fb_next[1];
-            const float4 fa0 = fa_ring[xl % 4][0], fa1 = fa_ring[xl % 4][1];
-            static_for<0, 8>([&](auto stag) {
+            const v4u fb[3] = {fb_next[0], fb_next[1], fb_next[2]};
+            const v4u fa[3] = {fa_ring[xl % 4][0], fa_ring[xl % 4][1], fa_ring[xl % 4][2]};
+            static_for<0, 6>([&](auto stag) {
                 constexpr int ks = decltype(stag)::value;
                 // side work of this step, pinned to it: left to itself the scheduler sinks every load to its first use
                 if constexpr (ks == 0) {
                     // the filter fragments three positions ahead (into the slot of the position before this one)
-                    fa_load(StepTag<(xl + 3) % 4>{}, (xl + 3 < 8 ? chunk * 16 : (chunk + 1) * 16 - 8) + wi * 8 + xl + 3);
+                    fa_load(StepTag<(xl + 3) % 4>{}, (xl + 3 < 8 ? chunk * 16 : chunk_next * 16 - 8) + wi * 8 + xl + 3);
                 }
-                if constexpr (ks == 1 && xl < 7) {   // this lane's tile at the next position
-                    fb_next[0] = *(const float4 *)(Vc + b_frag + (xl + 1) * TT * LDP);
-                    fb_next[1] = *(const float4 *)(Vc + b_frag + (xl + 1) * TT * LDP + 4);
-                }
+                if constexpr (ks == 1 && xl < 7) fb_load(Vc, xl + 1);   // this lane's tile at the next position
                 // the patch `ahead` chunks on: loads during positions 0..3, LDS stores during 4..7
                 if constexpr (xl < 4 && ks >= 2 && ks < 2 + PER) {
                     if (fetch) patch_load(xl * PER + ks - 2, chunk + ahead);
@@ -664,16 +724,15 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
                 if constexpr (xl >= 4 && ks == 2) {
                     if (fetch) patch_store(xl - 4, raww);
                 }
-                if constexpr (DB && ks == 6) {       // the next chunk's transform: a column per position, then the products
+                if constexpr (DB && ks == 4) {       // the next chunk's transform: a column per position, then a product each
                     if (more) {
                         if constexpr (xl < 4) transform_read(xl, rawn);
-                        if constexpr (xl == 4) transform_write(Vn);
+                        if constexpr (xl >= 4) transform_write(Vn, xl - 4);
                     }
                 }
-                const float4 av = ks < 4 ? fa0 : fa1, bv = ks < 4 ? fb0 : fb1;
-                const float a = ks % 4 == 0 ? av.x : ks % 4 == 1 ? av.y : ks % 4 == 2 ? av.z : av.w;
-                const float b = ks % 4 == 0 ? bv.x : ks % 4 == 1 ? bv.y : ks % 4 == 2 ? bv.z : bv.w;
-                acc[xl] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc[xl], 0, 0, 0);
+                // smallest products first: l.h, h.l, m.m, m.h, h.m, h.h
+                constexpr int qa = ks == 0 ? 2 : ks == 2 || ks == 3 ? 1 : 0, qb = ks == 1 ? 2 : ks == 2 || ks == 4 ? 1 : 0;
+                acc[xl] = mfma_bf16(fa[qa], fb[qb], acc[xl]);
                 __builtin_amdgcn_sched_barrier(0);
             });
         });
@@ -682,12 +741,12 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
             if (more) {
 #pragma unroll
                 for (int b = 0; b < 4; b++) transform_read(b, raw0);
-                transform_write(V0);
+#pragma unroll
+                for (int b = 0; b < 4; b++) transform_write(V0, b);
             }
             __syncthreads();
         }
-        fb_next[0] = *(const float4 *)(Vn + b_frag);
-        fb_next[1] = *(const float4 *)(Vn + b_frag + 4);
+        fb_load(Vn, 0);
     }
 
     // ---- inverse transform.  This wavefront's rows of the 4x4 grid are i = 2 wi, 2 wi + 1; acc[4 il + j] = M[i][j].
@@ -718,6 +777,7 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
         const int n = n_first + img;
         if (n >= p.N) return;
         float *base = outp + ((size_t)n * p.Mout * p.OH + (oh0 + 2 * r2)) * p.OW + 2 * c2;
+        unsigned again = 0;
 #pragma unroll
         for (int v = 0; v < 16; v++) {
             const int m = m0 + wk * 32 + acc_row(v, lane);
@@ -725,6 +785,8 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
             const float bias = add_bias ? p.bias[m] : 0.0f;
             const float4 other = *(const float4 *)(xchg + (((w >> 1) * 16 + v) * 64 + lane) * 4);
             float y[4] = {part[v][0] + other.x, part[v][1] + other.y, part[v][2] + other.z, part[v][3] + other.w};
+            // (zero times an infinity or a NaN is a NaN)
+            if ((y[0] * 0.0f + y[1] * 0.0f) + (y[2] * 0.0f + y[3] * 0.0f) != 0.0f) again |= 1u << v;
             if (add_bias) {
 #pragma unroll
                 for (int q = 0; q < 4; q++) y[q] += bias;
@@ -733,11 +795,21 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
             *(float2 *)o = make_float2(y[0], y[1]);
             *(float2 *)(o + p.OW) = make_float2(y[2], y[3]);
         }
+        while (again) {               // the parts of an infinity hold NaNs: formed again in fp32
+            const int m = m0 + wk * 32 + acc_row(__builtin_ctz(again), lane);
+            again &= again - 1;
+            float y[4];
+            wino_fp32(p, n, m, oh0 + 2 * r2 - p.PT, 2 * c2 - p.PL, cb * CH, ce * CH, y);
+            const float bias = add_bias ? p.bias[m] : 0.0f;
+            float *o = base + (size_t)m * OHW;
+            *(float2 *)o = make_float2(y[0] + bias, y[1] + bias);
+            *(float2 *)(o + p.OW) = make_float2(y[2] + bias, y[3] + bias);
+        }
     }
 }
 
-// The transformed filter of the Winograd kernel: U[((chunk*16 + xi)*Mp + m)*16 + j] = (G g Gt)[xi] for row m and
-// channel chunk*16 + j, where g is the filter as the kernel applies it to the patch: g[r][s] multiplies patch offset
+// The transformed filter of the Winograd kernel, split into its bf16 parts q = h, m, l:
+// U[(((chunk*16 + xi)*3 + q)*Mp + m)*16 + j] = (G g Gt)[xi] for row m and channel chunk*16 + j, where g is the filter as the kernel applies it to the patch: g[r][s] multiplies patch offset
 // (r, s), i.e. the stored taps read backwards when the operation is a true convolution (`flip`).  Staged like
 // pack_tile (16 rows of one chunk); G = [1 0 0; .5 .5 .5; .5 -.5 .5; 0 0 1].
 template <bool kBwd>
@@ -784,15 +856,23 @@ __device__ __forceinline__ void wino_pack_tile(int M, int Cred, int Mp, size_t s
             h[2][c] = ((g[0][c] - g[1][c]) + g[2][c]) * 0.5f;
             h[3][c] = g[2][c];
         }
+        // neighbouring channels share a word: the even channel's thread writes the positions of columns 0 and 2, the odd
+        // one's those of columns 1 and 3, each with its neighbour's values
+        const bool odd = j & 1;
+        const size_t part = (size_t)Mp * 8;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const float u0 = h[r][0], u1 = ((h[r][0] + h[r][1]) + h[r][2]) * 0.5f, u2 = ((h[r][0] - h[r][1]) + h[r][2]) * 0.5f,
-                        u3 = h[r][2];
-            float *dst = wp + (((size_t)chunk * 16 + r * 4) * Mp + m0 + ml) * 16 + j;
-            dst[0] = u0;
-            dst[(size_t)Mp * 16] = u1;
-            dst[(size_t)2 * Mp * 16] = u2;
-            dst[(size_t)3 * Mp * 16] = u3;
+            const float u[4] = {h[r][0], ((h[r][0] + h[r][1]) + h[r][2]) * 0.5f, ((h[r][0] - h[r][1]) + h[r][2]) * 0.5f, h[r][2]};
+#pragma unroll
+            for (int e = 0; e < 4; e += 2) {
+                const float other = __shfl_xor(odd ? u[e] : u[e + 1], 1);
+                unsigned ph, pm, pl;
+                split_pair_any(odd ? other : u[e], odd ? u[e + 1] : other, ph, pm, pl);
+                unsigned *dst = (unsigned *)wp + ((((size_t)chunk * 16 + r * 4 + e + odd) * 3) * Mp + m0 + ml) * 8 + (j >> 1);
+                dst[0] = ph;
+                dst[part] = pm;
+                dst[2 * part] = pl;
+            }
         }
     }
 }
@@ -1708,7 +1788,7 @@ PatchSetup patch_setup_as(const dopt_hip_conv_desc *d, size_t P, size_t Q, bool 
     if (wino) {
         if (pc.rows % 2 != 0) return u;   // a pixel tile is whole 2 x 2 tiles
         const size_t buffers = u.BM == 128 ? 2 : 1;   // 32 tiles: raw patch and V are double-buffered
-        const size_t floats = buffers * ((size_t)(((pc.psz + 1) * 20 + 3) / 4 * 4) + (size_t)16 * (u.BN / 4) * 20);
+        const size_t floats = buffers * ((size_t)(((pc.psz + 1) * 20 + 3) / 4 * 4) + (size_t)16 * (u.BN / 4) * 24);
         u.lds_bytes = (floats > (size_t)kWinoXchg ? floats : (size_t)kWinoXchg) * sizeof(float);
     }
     if (u.lds_bytes > 160 * 1024) return u;
@@ -1721,7 +1801,7 @@ PatchSetup patch_setup_as(const dopt_hip_conv_desc *d, size_t P, size_t Q, bool 
     pc.chunks_total = (pc.Cin + 15) / 16;
     pc.out_elems = (size_t)pc.ncols * pc.Mout;
     u.tiles = pc.mtiles * pc.ntiles;
-    u.wp_elems = (size_t)pc.chunks_total * (wino ? 16 : 9) * pc.Mp * 16;
+    u.wp_elems = (size_t)pc.chunks_total * (wino ? 16 * 24 : 9 * 16) * pc.Mp;   // (Winograd: three 16-bit parts a value)
     u.ok = true;
     return u;
 }

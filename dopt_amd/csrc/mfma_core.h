@@ -125,6 +125,25 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsign
     l = __builtin_bit_cast(unsigned, __builtin_convertvector(s, v2bf));
 }
 
+// The same for operands that are laid out once and read again as h + m + l: exact for every value, infinities and values
+// that round to one included (an infinity is its own h part, the other two are zero).
+__device__ __forceinline__ void split_pair_any(float a, float b, unsigned &h, unsigned &m, unsigned &l)
+{
+    split_pair(a, b, h, m, l);
+    auto fix = [](float v, unsigned hv, unsigned shift, unsigned &h, unsigned &m, unsigned &l) {
+        if ((hv & 0x7f80u) != 0x7f80u || v != v) return;   // a finite h; a NaN stays one
+        const unsigned keep = 0xffff0000u >> shift, bits = __builtin_bit_cast(unsigned, v);
+        unsigned h2, m2, l2;
+        const float head = __builtin_bit_cast(float, bits & 0xffff0000u);
+        split_pair(__builtin_isinf(v) ? 0.0f : v - head, 0.0f, h2, m2, l2);   // 16 bits: two parts
+        h = (h & keep) | ((bits >> 16) << shift);
+        m = (m & keep) | (h2 & 0xffffu) << shift;
+        l = (l & keep) | (m2 & 0xffffu) << shift;
+    };
+    fix(a, h & 0xffffu, 0, h, m, l);
+    fix(b, h >> 16, 16, h, m, l);
+}
+
 // Four reduction steps of one row: their h parts in hm.x, .y, their m parts in hm.z, .w, their l parts in l.
 __device__ __forceinline__ void split_quad(float4 q, v4u &hm, uint2 &l)
 {

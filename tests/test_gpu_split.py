@@ -66,3 +66,81 @@ def test_operands_that_are_not_finite():
     fine = np.isfinite(want) & ~over & np.isfinite(got)
     assert fine.sum() > 0.9 * M * N
     assert np.all(np.abs(got[fine] - want[fine]) <= walk(K) * mag[fine])
+
+
+# ---- the Winograd convolution kernel
+
+BT = np.array([[1, 0, -1, 0], [0, 1, 1, 0], [0, -1, 1, 0], [0, 1, 0, -1]], np.float64)
+G = np.array([[1, 0, 0], [.5, .5, .5], [.5, -.5, .5], [0, 0, 1]], np.float64)
+AT = np.array([[1, 1, 1, 0], [0, 1, -1, -1]], np.float64)
+
+
+def sandwich(m, x):
+    """m x m^T over the last two axes, where a zero of m takes nothing from an infinity."""
+    def left(m, x):
+        out = []
+        for row in m:
+            out.append(sum(c * x[..., i, :] for i, c in enumerate(row) if c != 0))
+        return np.stack(out, axis=-2)
+    with np.errstate(all="ignore"):
+        return np.swapaxes(left(m, np.swapaxes(left(m, x), -1, -2)), -1, -2)
+
+
+def winograd(x, w, mag=False):
+    """F(2x2, 3x3) of a true convolution with pad 1 in float64, or the same with every term's absolute value."""
+    f = np.abs if mag else (lambda v: v)
+    N, C, H, W = x.shape
+    g = f(w[:, :, ::-1, ::-1].astype(np.float64))
+    xp = np.pad(f(x.astype(np.float64)), ((0, 0), (0, 0), (1, 1), (1, 1)))
+    d = np.stack([np.stack([xp[:, :, r:r + H:2, q:q + W:2] for q in range(4)], -1) for r in range(4)], -2)
+    u, v = sandwich(f(G), g), sandwich(f(BT), d)
+    with np.errstate(all="ignore"):
+        m = np.stack([np.stack([np.einsum("kc,nchw->nkhw", u[..., i, j], v[..., i, j]) for j in range(4)], -1) for i in range(4)], -2)
+    y = sandwich(f(AT), m)
+    return y.transpose(0, 1, 2, 4, 3, 5).reshape(N, w.shape[0], H, W)
+
+
+def winograd_share(terms):
+    """Of the sum of absolute terms: the sum over the channels, and at most six roundings each in the two transforms before
+    it and the one after."""
+    return walk(terms) + 12 * 2.0 ** -24
+
+
+# 128-row and 64-row tiles; rows of 64 to 4 pixels; the last pixel tile a part of one; one chunk to spare, split reductions
+@pytest.mark.parametrize("shape", [(3, 64, 32, 32, 64), (2, 64, 64, 64, 64), (1, 80, 16, 16, 160), (5, 96, 8, 8, 320),
+                                   (5, 64, 16, 16, 128), (3, 208, 8, 8, 128), (9, 128, 4, 4, 256), (1, 64, 4, 4, 128),
+                                   (2, 640, 8, 8, 128)])
+@pytest.mark.parametrize("backward", [False, True])
+def test_winograd(shape, backward):
+    N, C, H, W, K = shape
+    r = rng(N + C + H)
+    x = np.maximum(r.standard_normal((N, C, H, W)), 0).astype(np.float32)
+    w = r.standard_normal((K, C, 3, 3)).astype(np.float32)
+    if backward:   # the data gradient is the convolution with the filter's transposed and reversed copy
+        got = ops.conv_bwd_data(T(x), T(np.ascontiguousarray(w.transpose(1, 0, 2, 3)[:, :, ::-1, ::-1])), (N, K, H, W), (1, 1), (1, 1)).numpy()
+    else:
+        got = ops.convolution(T(x), T(w), (1, 1), (1, 1)).numpy()
+    want, mag = winograd(x, w), winograd(x, w, True)
+    assert np.all(np.abs(got - want) <= winograd_share(C) * mag), np.max(np.abs(got - want) / mag)
+
+
+@pytest.mark.parametrize("shape", [(2, 64, 16, 16, 64), (2, 64, 16, 16, 128)])
+def test_winograd_operands_that_are_not_finite(shape):
+    N, C, H, W, K = shape
+    r = rng(K)
+    x = np.maximum(r.standard_normal((N, C, H, W)), 0).astype(np.float32)
+    w = (0.1 * r.standard_normal((K, C, 3, 3))).astype(np.float32)
+    x[0, 3, 0, 0], x[0, 5, 9, 9], x[1, 7, 4, 5], x[1, 8, 12, 12] = np.inf, np.nan, -np.inf, 3.4e38
+    w[5, 2, 0, 0], w[6, 9, 1, 1] = np.inf, 3.4e38
+    got = ops.convolution(T(x), T(w), (1, 1), (1, 1)).numpy()
+    want, mag = winograd(x, w), winograd(x, w, True)
+    huge = ~(mag < 3e38)               # where fp32 may overflow on the way, only what float64 says is not finite is known
+    assert np.all(np.isfinite(got[~huge]))
+    bad = ~np.isfinite(want)
+    assert np.array_equal(np.isnan(got[bad]), np.isnan(want[bad]))
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf])
+    assert np.all(np.abs(got[~huge] - want[~huge]) <= winograd_share(C) * mag[~huge])
+    # a value that rounds to infinity in 16 bits but is none
+    fits = huge & np.isfinite(want) & (mag < 3.4e38)
+    assert np.all(np.isfinite(got[fits]))
