@@ -24,6 +24,7 @@
 // the inner loops are branch-free.  Layers with few output tiles split the reduction; partial
 // tiles go to the workspace and are summed in a fixed order -- no float atomics, so results are
 // reproducible.
+#include <algorithm>
 #include <utility>
 #include <vector>
 
@@ -473,7 +474,8 @@ __global__ __launch_bounds__(T::THREADS, T::THREADS / 256) void conv_patch_k(Pat
 // and workgroup, 16/9 the direct kernel's), the V reads, the patch and the transform each add their share, roughly in
 // proportion to their instruction counts (loops without one of them: -0.5, -0.2, -0.3, -0.4 us).  128 rows x 64 tiles
 // would halve filter traffic and fragment loads per matrix instruction and need 256 accumulator registers per wavefront.
-constexpr int kWinoXchg = 4 * 64 * 64;   // floats of the exchange area: four wavefront pairs x 64 values per lane
+// floats of the exchange area: 128 rows: four wavefront pairs x 64 values per lane; 64 rows: eight wavefronts x 64 values
+constexpr int wino_xchg(int bm) { return (bm == 128 ? 4 : 8) * 64 * 64; }
 
 // WK x TH: the eight wavefronts are WK groups of 32 rows x TH groups of 32 tiles x the two halves of the 16 positions:
 // 4 x 1 (128 rows x 32 tiles = 128 pixels) for layers with whole 128-row tiles, 2 x 2 (64 rows x 64 tiles = 256 pixels)
@@ -555,7 +557,9 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wavefront-uniform, and known to be: it enters scalar load offsets
-    const int wi = w & 1, wk = (w >> 1) % WK, th = (w >> 1) / WK;
+    // a wavefront multiplies its rows with XP positions from xb on, the tiles 32 at a time
+    constexpr int XP = 8 / TH;
+    const int wi = TH == 1 ? w & 1 : w >> 1, wk = TH == 1 ? w >> 1 : w & 1, xb = wi * XP;
     const int kh = lane >> 5, l32 = lane & 31;
     const int OHW = p.OH * p.OW;
     const int chan_stride = p.IH * p.IW;
@@ -646,11 +650,11 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
         for (int q = 0; q < 3; q++)
             fa_ring[slot][q] = __builtin_bit_cast(v4u, buffer_load_f32x4(rwp, fa_voff, (unsigned)slab * slab_bytes + q * part_bytes));
     };
-    const int b_frag = wi * 8 * VX + kh * (4 * TT) + (th * 32 + l32) * 4;   // position 8 wi, this lane's tile and channels
+    const int b_frag = xb * VX + kh * (4 * TT) + l32 * 4;   // position xb, this lane's tile and channels
     v4u fb_next[3];
-    auto fb_load = [&](const float *Vb, int x) {
+    auto fb_load = [&](const float *Vb, int x) {   // step x: position x / TH, tiles 32 (x % TH) ..
 #pragma unroll
-        for (int q = 0; q < 3; q++) fb_next[q] = *(const v4u *)(Vb + b_frag + x * VX + q * VP);
+        for (int q = 0; q < 3; q++) fb_next[q] = *(const v4u *)(Vb + b_frag + x / TH * VX + q * VP + x % TH * 128);
     };
 
     v16f acc[8];
@@ -668,9 +672,9 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
 #pragma unroll
         for (int i = 0; i < NPMAX; i++)
             second[i] = i < nslots && nch > 1 ? buffer_load_f32(rin, p_voff, (unsigned)(((cb + 1) * CH + cbase + i) * chan_stride) * 4u) : 0.0f;
-        fa_load(StepTag<0>{}, cb * 16 + wi * 8);
-        fa_load(StepTag<1>{}, cb * 16 + wi * 8 + 1);
-        fa_load(StepTag<2>{}, cb * 16 + wi * 8 + 2);
+        fa_load(StepTag<0>{}, cb * 16 + xb);
+        fa_load(StepTag<1>{}, cb * 16 + xb + 1);
+        fa_load(StepTag<2>{}, cb * 16 + xb + 2);
 #pragma unroll
         for (int g = 0; g < NPMAX / 4; g++) patch_store(g, raw0);
 #pragma unroll
@@ -679,9 +683,9 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
                 *(float4 *)((char *)(raw0 + raw_floats) + p_lds + g * 16) =
                     make_float4(second[4 * g], second[4 * g + 1], second[4 * g + 2], second[4 * g + 3]);
     } else {
-        fa_load(StepTag<0>{}, cb * 16 + wi * 8);
-        fa_load(StepTag<1>{}, cb * 16 + wi * 8 + 1);
-        fa_load(StepTag<2>{}, cb * 16 + wi * 8 + 2);
+        fa_load(StepTag<0>{}, cb * 16 + xb);
+        fa_load(StepTag<1>{}, cb * 16 + xb + 1);
+        fa_load(StepTag<2>{}, cb * 16 + xb + 2);
 #pragma unroll
         for (int g = 0; g < NPMAX / 4; g++) patch_store(g, raw0);
     }
@@ -708,13 +712,14 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
         static_for<0, 8>([&](auto xtag) {
             constexpr int xl = decltype(xtag)::value;
             const v4u fb[3] = {fb_next[0], fb_next[1], fb_next[2]};
-            const v4u fa[3] = {fa_ring[xl % 4][0], fa_ring[xl % 4][1], fa_ring[xl % 4][2]};
+            constexpr int xp = xl / TH;
+            const v4u fa[3] = {fa_ring[xp % 4][0], fa_ring[xp % 4][1], fa_ring[xp % 4][2]};
             static_for<0, 6>([&](auto stag) {
                 constexpr int ks = decltype(stag)::value;
                 // side work of this step, pinned to it: left to itself the scheduler sinks every load to its first use
-                if constexpr (ks == 0) {
+                if constexpr (ks == 0 && xl % TH == 0) {
                     // the filter fragments three positions ahead (into the slot of the position before this one)
-                    fa_load(StepTag<(xl + 3) % 4>{}, (xl + 3 < 8 ? chunk * 16 : chunk_next * 16 - 8) + wi * 8 + xl + 3);
+                    fa_load(StepTag<(xp + 3) % 4>{}, (xp + 3 < XP ? chunk * 16 : chunk_next * 16 - XP) + xb + xp + 3);
                 }
                 if constexpr (ks == 1 && xl < 7) fb_load(Vc, xl + 1);   // this lane's tile at the next position
                 // the patch `ahead` chunks on: loads during positions 0..3, LDS stores during 4..7
@@ -754,56 +759,86 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
     float *const xchg = lds;          // [wavefront pair][accumulator row][lane][4]: the main loop's LDS is free now
     float *outp = p.out + (size_t)split * p.out_elems;
     const bool add_bias = p.bias != nullptr && p.splits == 1;
-    float part[16][4];                // per accumulator row v: this wavefront's share of y[a][b], index 2 a + b
-#pragma unroll
-    for (int v = 0; v < 16; v++) {
-        const float za0 = (acc[0][v] + acc[1][v]) + acc[2][v], za1 = (acc[1][v] - acc[2][v]) - acc[3][v];
-        const float zb0 = (acc[4][v] + acc[5][v]) + acc[6][v], zb1 = (acc[5][v] - acc[6][v]) - acc[7][v];
-        if (wi == 0) {                // rows 0, 1: y[0] += z0 + z1, y[1] += z1
-            part[v][0] = za0 + zb0; part[v][1] = za1 + zb1; part[v][2] = zb0; part[v][3] = zb1;
-        } else {                      // rows 2, 3: y[0] += z2, y[1] += -z2 - z3
-            part[v][0] = za0; part[v][1] = za1; part[v][2] = -za0 - zb0; part[v][3] = -za1 - zb1;
+    unsigned again = 0;               // results that are not finite
+    // the four outputs of accumulator row v of tiles 32 t ..; y: index 2 a + b
+    auto store = [&](int t, int v, float (&y)[4], unsigned flag) {
+        const int tau = t * 32 + l32, img = tau / tpi, tl = tau - img * tpi, r2 = tl / tcn, c2 = tl - r2 * tcn;
+        const int n = n_first + img, m = m0 + wk * 32 + acc_row(v, lane);
+        if (n >= p.N || m >= p.Mout) return;
+        // (zero times an infinity or a NaN is a NaN)
+        if ((y[0] * 0.0f + y[1] * 0.0f) + (y[2] * 0.0f + y[3] * 0.0f) != 0.0f) {
+            if (flag) {               // the parts of an infinity hold NaNs: formed again in fp32 below
+                again |= flag;
+                return;
+            }
         }
-    }
-    if (wi == 1) {   // a lane's four shares of one accumulator row are one 128-bit store
+        if (add_bias) {
+            const float bias = p.bias[m];
 #pragma unroll
-        for (int v = 0; v < 16; v++)
-            *(float4 *)(xchg + (((w >> 1) * 16 + v) * 64 + lane) * 4) = make_float4(part[v][0], part[v][1], part[v][2], part[v][3]);
-    }
-    __syncthreads();
-    if (wi == 1) return;
-    {
-        const int tau = th * 32 + l32, img = tau / tpi, tl = tau - img * tpi, r2 = tl / tcn, c2 = tl - r2 * tcn;
-        const int n = n_first + img;
-        if (n >= p.N) return;
-        float *base = outp + ((size_t)n * p.Mout * p.OH + (oh0 + 2 * r2)) * p.OW + 2 * c2;
-        unsigned again = 0;
+            for (int q = 0; q < 4; q++) y[q] += bias;
+        }
+        float *o = outp + ((size_t)n * p.Mout + m) * OHW + (oh0 + 2 * r2) * p.OW + 2 * c2;
+        *(float2 *)o = make_float2(y[0], y[1]);
+        *(float2 *)(o + p.OW) = make_float2(y[2], y[3]);
+    };
+    auto store_fp32 = [&](int t, int v) {
+        const int tau = t * 32 + l32, img = tau / tpi, tl = tau - img * tpi, r2 = tl / tcn, c2 = tl - r2 * tcn;
+        float y[4];
+        wino_fp32(p, n_first + img, m0 + wk * 32 + acc_row(v, lane), oh0 + 2 * r2 - p.PT, 2 * c2 - p.PL, cb * CH, ce * CH, y);
+        store(t, v, y, 0);
+    };
+    if constexpr (TH == 1) {
+        float part[16][4];            // per accumulator row v: this wavefront's share of y[a][b], index 2 a + b
 #pragma unroll
         for (int v = 0; v < 16; v++) {
-            const int m = m0 + wk * 32 + acc_row(v, lane);
-            if (m >= p.Mout) continue;
-            const float bias = add_bias ? p.bias[m] : 0.0f;
-            const float4 other = *(const float4 *)(xchg + (((w >> 1) * 16 + v) * 64 + lane) * 4);
-            float y[4] = {part[v][0] + other.x, part[v][1] + other.y, part[v][2] + other.z, part[v][3] + other.w};
-            // (zero times an infinity or a NaN is a NaN)
-            if ((y[0] * 0.0f + y[1] * 0.0f) + (y[2] * 0.0f + y[3] * 0.0f) != 0.0f) again |= 1u << v;
-            if (add_bias) {
-#pragma unroll
-                for (int q = 0; q < 4; q++) y[q] += bias;
+            const float za0 = (acc[0][v] + acc[1][v]) + acc[2][v], za1 = (acc[1][v] - acc[2][v]) - acc[3][v];
+            const float zb0 = (acc[4][v] + acc[5][v]) + acc[6][v], zb1 = (acc[5][v] - acc[6][v]) - acc[7][v];
+            if (wi == 0) {            // rows 0, 1: y[0] += z0 + z1, y[1] += z1
+                part[v][0] = za0 + zb0; part[v][1] = za1 + zb1; part[v][2] = zb0; part[v][3] = zb1;
+            } else {                  // rows 2, 3: y[0] += z2, y[1] += -z2 - z3
+                part[v][0] = za0; part[v][1] = za1; part[v][2] = -za0 - zb0; part[v][3] = -za1 - zb1;
             }
-            float *o = base + (size_t)m * OHW;
-            *(float2 *)o = make_float2(y[0], y[1]);
-            *(float2 *)(o + p.OW) = make_float2(y[2], y[3]);
         }
-        while (again) {               // the parts of an infinity hold NaNs: formed again in fp32
-            const int m = m0 + wk * 32 + acc_row(__builtin_ctz(again), lane);
+        if (wi == 1) {   // a lane's four shares of one accumulator row are one 128-bit store
+#pragma unroll
+            for (int v = 0; v < 16; v++)
+                *(float4 *)(xchg + ((wk * 16 + v) * 64 + lane) * 4) = make_float4(part[v][0], part[v][1], part[v][2], part[v][3]);
+        }
+        __syncthreads();
+        if (wi == 1) return;
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const float4 other = *(const float4 *)(xchg + ((wk * 16 + v) * 64 + lane) * 4);
+            float y[4] = {part[v][0] + other.x, part[v][1] + other.y, part[v][2] + other.z, part[v][3] + other.w};
+            store(0, v, y, 1u << v);
+        }
+        while (again) {
+            const int v = __builtin_ctz(again);
             again &= again - 1;
-            float y[4];
-            wino_fp32(p, n, m, oh0 + 2 * r2 - p.PT, 2 * c2 - p.PL, cb * CH, ce * CH, y);
-            const float bias = add_bias ? p.bias[m] : 0.0f;
-            float *o = base + (size_t)m * OHW;
-            *(float2 *)o = make_float2(y[0] + bias, y[1] + bias);
-            *(float2 *)(o + p.OW) = make_float2(y[2] + bias, y[3] + bias);
+            store_fp32(0, v);
+        }
+    } else {
+        // a wavefront holds one row i of the grid: all four put their z in LDS, each finishes eight accumulator rows
+#pragma unroll
+        for (int t = 0; t < TH; t++)
+#pragma unroll
+            for (int v = 0; v < 16; v++)
+                *(float2 *)(xchg + (((wk * 4 + wi) * 32 + t * 16 + v) * 64 + lane) * 2) =
+                    make_float2((acc[t][v] + acc[2 + t][v]) + acc[4 + t][v], (acc[2 + t][v] - acc[4 + t][v]) - acc[6 + t][v]);
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const int tv = wi * 8 + e;
+            float2 z[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) z[i] = *(const float2 *)(xchg + (((wk * 4 + i) * 32 + tv) * 64 + lane) * 2);
+            float y[4] = {(z[0].x + z[1].x) + z[2].x, (z[0].y + z[1].y) + z[2].y, z[1].x + (-z[2].x - z[3].x), z[1].y + (-z[2].y - z[3].y)};
+            store(tv >> 4, tv & 15, y, 1u << e);
+        }
+        while (again) {
+            const int tv = wi * 8 + __builtin_ctz(again);
+            again &= again - 1;
+            store_fp32(tv >> 4, tv & 15);
         }
     }
 }
@@ -1789,7 +1824,7 @@ PatchSetup patch_setup_as(const dopt_hip_conv_desc *d, size_t P, size_t Q, bool 
         if (pc.rows % 2 != 0) return u;   // a pixel tile is whole 2 x 2 tiles
         const size_t buffers = u.BM == 128 ? 2 : 1;   // 32 tiles: raw patch and V are double-buffered
         const size_t floats = buffers * ((size_t)(((pc.psz + 1) * 20 + 3) / 4 * 4) + (size_t)16 * (u.BN / 4) * 24);
-        u.lds_bytes = (floats > (size_t)kWinoXchg ? floats : (size_t)kWinoXchg) * sizeof(float);
+        u.lds_bytes = std::max(floats, (size_t)wino_xchg(u.BM)) * sizeof(float);
     }
     if (u.lds_bytes > 160 * 1024) return u;
     pc.magic_psz = div_magic((unsigned)pc.psz);
