@@ -1342,7 +1342,7 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
     }
     float4 areg[NAQ], breg[NBQ];
     // position of the chunk being FETCHED: first image and, for geometry 0, the band of rows
-    int n_img = kGeo == 0 ? cb / p.bands : cb * p.imgs, band = kGeo == 0 ? cb - n_img * p.bands : 0;
+    int n_img, band;
     auto fetch = [&]() {
         const int p0 = band * p.G;
         const unsigned a_soff = (unsigned)(n_img * p.K * HW + p0 * p.W) * 4u;
@@ -1415,22 +1415,9 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
     __syncthreads();
 
     v16f acc[3];
-#pragma unroll
-    for (int t = 0; t < 3; t++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) acc[t][v] = 0.0f;
-
-    fetch();
-    stash(0);
-    __syncthreads();
-    int cur = 0;
     typedef __attribute__((address_space(3))) float lds_float_t;
     // Fetching runs one chunk ahead and also past the end of this block's range: those loads are
     // range-checked and their data lands in the LDS buffer that is not read again.
-    // The fragments of a step are read one step ahead (the first step's after the barrier that releases the chunk), so
-    // that their LDS latency passes under the previous step's matrix instructions - with twelve wavefronts; fifteen have
-    // 128 registers each and no room for a second set.
-    constexpr bool AHEAD = WM * WC == 4;
     struct Frag {
         float4 a_lo, a_hi, q[4];
         float e[4];
@@ -1457,57 +1444,138 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
         }
         return f;
     };
-    Frag nxt;
-    if constexpr (AHEAD) nxt = read_frag(0, 0);
-    for (int chunk = cb; chunk < ce; ++chunk) {
-        static_for<0, 4>([&](auto stag) {
-            constexpr int s = decltype(stag)::value;
-            if constexpr (s == 0) fetch();
-            Frag f;
-            if constexpr (AHEAD) {
-                f = nxt;
-                if constexpr (s < 3) {
-                    nxt = read_frag(cur, s + 1);
-                    __builtin_amdgcn_sched_barrier(0);   // issued here, not where they are first used
-                }
-            } else {
-                f = read_frag(cur, s);
-            }
-            const float a8[8] = {f.a_lo.x, f.a_lo.y, f.a_lo.z, f.a_lo.w, f.a_hi.x, f.a_hi.y, f.a_hi.z, f.a_hi.w};
-            if constexpr (kGeo == 0) {
-                const float4 b_lo = f.q[0], b_hi = f.q[1];
-                const float win[10] = {f.e[0], b_lo.x, b_lo.y, b_lo.z, b_lo.w, b_hi.x, b_hi.y, b_hi.z, b_hi.w, f.e[1]};
+    auto products_fp32 = [&](const Frag &f) {
+        const float a8[8] = {f.a_lo.x, f.a_lo.y, f.a_lo.z, f.a_lo.w, f.a_hi.x, f.a_hi.y, f.a_hi.z, f.a_hi.w};
+        if constexpr (kGeo == 0) {
+            const float4 b_lo = f.q[0], b_hi = f.q[1];
+            const float win[10] = {f.e[0], b_lo.x, b_lo.y, b_lo.z, b_lo.w, b_hi.x, b_hi.y, b_hi.z, b_hi.w, f.e[1]};
 #pragma unroll
-                for (int ks = 0; ks < 8; ks++)
+            for (int ks = 0; ks < 8; ks++)
 #pragma unroll
-                    for (int ds = 0; ds < 3; ds++)
-                        acc[ds] = __builtin_amdgcn_mfma_f32_32x32x2f32(a8[ks], win[ks + ds], acc[ds], 0, 0, 0);
-            } else if constexpr (kGeo == 1) {
-                const float4 r0 = f.q[0], r1 = f.q[1];
-                const float w0[6] = {f.e[0], r0.x, r0.y, r0.z, r0.w, f.e[1]};
-                const float w1[6] = {f.e[2], r1.x, r1.y, r1.z, r1.w, f.e[3]};
+                for (int ds = 0; ds < 3; ds++)
+                    acc[ds] = __builtin_amdgcn_mfma_f32_32x32x2f32(a8[ks], win[ks + ds], acc[ds], 0, 0, 0);
+        } else if constexpr (kGeo == 1) {
+            const float4 r0 = f.q[0], r1 = f.q[1];
+            const float w0[6] = {f.e[0], r0.x, r0.y, r0.z, r0.w, f.e[1]};
+            const float w1[6] = {f.e[2], r1.x, r1.y, r1.z, r1.w, f.e[3]};
 #pragma unroll
-                for (int ks = 0; ks < 8; ks++)
+            for (int ks = 0; ks < 8; ks++)
 #pragma unroll
-                    for (int ds = 0; ds < 3; ds++)
-                        acc[ds] = __builtin_amdgcn_mfma_f32_32x32x2f32(a8[ks], ks < 4 ? w0[ks + ds] : w1[ks - 4 + ds],
-                                                                       acc[ds], 0, 0, 0);
-            } else {
-                // pixel (row, col) of tap column ds reads element col + ds of the quad of patch row row + dr
-                const float4 q00 = f.q[0], q01 = f.q[1], q10 = f.q[2], q11 = f.q[3];
-                const float win[4][4] = {{q00.x, q00.y, q00.z, q00.w}, {q01.x, q01.y, q01.z, q01.w},
-                                         {q10.x, q10.y, q10.z, q10.w}, {q11.x, q11.y, q11.z, q11.w}};
+                for (int ds = 0; ds < 3; ds++)
+                    acc[ds] = __builtin_amdgcn_mfma_f32_32x32x2f32(a8[ks], ks < 4 ? w0[ks + ds] : w1[ks - 4 + ds],
+                                                                   acc[ds], 0, 0, 0);
+        } else {
+            // pixel (row, col) of tap column ds reads element col + ds of the quad of patch row row + dr
+            const float4 q00 = f.q[0], q01 = f.q[1], q10 = f.q[2], q11 = f.q[3];
+            const float win[4][4] = {{q00.x, q00.y, q00.z, q00.w}, {q01.x, q01.y, q01.z, q01.w},
+                                     {q10.x, q10.y, q10.z, q10.w}, {q11.x, q11.y, q11.z, q11.w}};
 #pragma unroll
-                for (int ks = 0; ks < 8; ks++)
+            for (int ks = 0; ks < 8; ks++)
 #pragma unroll
-                    for (int ds = 0; ds < 3; ds++)
-                        acc[ds] = __builtin_amdgcn_mfma_f32_32x32x2f32(a8[ks], win[ks / 2][(ks & 1) + ds], acc[ds], 0, 0, 0);
-            }
-            if constexpr (s == 3) stash(cur ^ 1);
+                for (int ds = 0; ds < 3; ds++)
+                    acc[ds] = __builtin_amdgcn_mfma_f32_32x32x2f32(a8[ks], win[ks / 2][(ks & 1) + ds], acc[ds], 0, 0, 0);
+        }
+    };
+    // The same sixteen pixels on the bf16 matrix instructions (eighteen of 32 cycles for twenty-four of 64): the fragments are split in registers (mfma_core.h), the x
+    // pixels in pairs that are tap column 1's operands as they are; those of columns 0 and 2 are their neighbouring halves
+    // with the edge pixels.  128 images of 320 -> 320 channels, 16 x 16: 450 -> 318 us (134 -> 190 TFLOP/s); what bounds it
+    // now is the splitting itself, 120 vector instructions a step and wavefront under the 576 cycles of the matrix ones.
+    // (Reading the fragments one step ahead, as the fp32 form did, needs 30 more registers than there are: 399 us.)
+    constexpr int NW = kGeo == 0 ? 5 : kGeo == 1 ? 6 : 8;   // pairs of pixels
+    v4u ap[3];
+    unsigned q[3][NW];
+    auto split_frag = [&](const Frag &f) {
+        {
+            uint2 l0, l1;
+            v4u hm0, hm1;
+            split_quad(f.a_lo, hm0, l0);
+            split_quad(f.a_hi, hm1, l1);
+            ap[0] = v4u{hm0.x, hm0.y, hm1.x, hm1.y};
+            ap[1] = v4u{hm0.z, hm0.w, hm1.z, hm1.w};
+            ap[2] = v4u{l0.x, l0.y, l1.x, l1.y};
+        }
+        static_for<0, kGeo == 2 ? 4 : 2>([&](auto itag) {
+            constexpr int i = decltype(itag)::value;
+            split_pair(f.q[i].x, f.q[i].y, q[0][2 * i], q[1][2 * i], q[2][2 * i]);
+            split_pair(f.q[i].z, f.q[i].w, q[0][2 * i + 1], q[1][2 * i + 1], q[2][2 * i + 1]);
         });
+        if constexpr (kGeo != 2) split_pair(f.e[0], f.e[1], q[0][4], q[1][4], q[2][4]);
+        if constexpr (kGeo == 1) split_pair(f.e[2], f.e[3], q[0][NW - 1], q[1][NW - 1], q[2][NW - 1]);
+    };
+    auto products_split = [&]() {
+        auto mid = [](unsigned hi, unsigned lo) { return __builtin_amdgcn_alignbit(hi, lo, 16); };             // (lo.1, hi.0)
+        auto left = [](unsigned e, unsigned w) { return __builtin_amdgcn_perm(w, e, 0x05040100u); };            // (e.0, w.0)
+        auto right = [](unsigned w, unsigned e) { return __builtin_amdgcn_perm(e, w, 0x07060302u); };           // (w.1, e.1)
+        static_for<0, 3>([&](auto ptag) {
+            constexpr int part = 2 - decltype(ptag)::value;
+            const unsigned *const w = q[part];
+            v4u b[3];
+            if constexpr (kGeo == 0) {
+                const unsigned m0 = mid(w[1], w[0]), m1 = mid(w[2], w[1]), m2 = mid(w[3], w[2]);
+                b[0] = v4u{left(w[4], w[0]), m0, m1, m2};
+                b[1] = v4u{w[0], w[1], w[2], w[3]};
+                b[2] = v4u{m0, m1, m2, right(w[3], w[4])};
+            } else if constexpr (kGeo == 1) {
+                const unsigned m0 = mid(w[1], w[0]), m1 = mid(w[3], w[2]);
+                b[0] = v4u{left(w[4], w[0]), m0, left(w[NW - 1], w[2]), m1};
+                b[1] = v4u{w[0], w[1], w[2], w[3]};
+                b[2] = v4u{m0, right(w[1], w[4]), m1, right(w[3], w[NW - 1])};
+            } else {
+                b[0] = v4u{w[0], w[2], w[4], w[NW - 2]};
+                b[1] = v4u{mid(w[1], w[0]), mid(w[3], w[2]), mid(w[5 % NW], w[4]), mid(w[NW - 1], w[NW - 2])};
+                b[2] = v4u{w[1], w[3], w[5 % NW], w[NW - 1]};
+            }
+            static_for<0, 3 - part>([&](auto atag) {   // x's l with dy's h; m with m, h; h with l, m, h
+                constexpr int pa = 2 - part - decltype(atag)::value;
+#pragma unroll
+                for (int ds = 0; ds < 3; ds++) acc[ds] = mfma_bf16(ap[pa], b[ds], acc[ds]);
+            });
+        });
+    };
+    auto run = [&](auto exact_tag) {
+        constexpr bool exact = decltype(exact_tag)::value != 0;
+        n_img = kGeo == 0 ? cb / p.bands : cb * p.imgs;
+        band = kGeo == 0 ? cb - n_img * p.bands : 0;
+#pragma unroll
+        for (int t = 0; t < 3; t++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[t][v] = 0.0f;
+        fetch();
+        stash(0);
         __syncthreads();
-        cur ^= 1;
-        if constexpr (AHEAD) nxt = read_frag(cur, 0);   // (past the last chunk: the buffer the final, unused prefetch was stored to)
+        int cur = 0;
+        for (int chunk = cb; chunk < ce; ++chunk) {
+            static_for<0, 4>([&](auto stag) {
+                constexpr int s = decltype(stag)::value;
+                if constexpr (s == 0) fetch();
+                if constexpr (exact) {
+                    products_fp32(read_frag(cur, s));
+                } else {
+                    split_frag(read_frag(cur, s));
+                    products_split();
+                }
+                if constexpr (s == 3) stash(cur ^ 1);
+            });
+            __syncthreads();
+            cur ^= 1;
+        }
+    };
+    run(StepTag<0>{});
+    {
+        // the parts of an infinity hold NaNs: a tile that is not finite is formed again with the fp32 instruction
+        float probe = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 3; t++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) probe = __builtin_fmaf(acc[t][v], 0.0f, probe);
+        volatile int *const again = (volatile int *)dummy;
+        if (tid == 0) *again = 0;
+        __syncthreads();
+        if (probe != 0.0f) *again = 1;
+        __syncthreads();
+        const bool redo = *again != 0;
+        __syncthreads();   // (the second pass may store there)
+        if (redo) run(StepTag<1>{});
     }
 
     // Epilogue: the accumulators leave through LDS so that every output row -- the BC*9 values

@@ -144,3 +144,43 @@ def test_winograd_operands_that_are_not_finite(shape):
     # a value that rounds to infinity in 16 bits but is none
     fits = huge & np.isfinite(want) & (mag < 3.4e38)
     assert np.all(np.isfinite(got[fits]))
+
+
+# ---- the filter gradient of 3 x 3 layers
+
+def filter_gradient(dy, x, f=lambda v: v):
+    """dw[k][c][r][s] = sum dy[n][k][p][q] x[n][c][p + 1 - r][q + 1 - s] in float64 (a true convolution, pad 1)."""
+    H, W = x.shape[2:]
+    xp = np.pad(f(x.astype(np.float64)), ((0, 0), (0, 0), (1, 1), (1, 1)))
+    g = f(dy.astype(np.float64)).transpose(1, 0, 2, 3).reshape(dy.shape[1], -1)
+    with np.errstate(all="ignore"):
+        taps = [g @ xp[:, :, 2 - r:2 - r + H, 2 - s:2 - s + W].transpose(0, 2, 3, 1).reshape(-1, x.shape[1])
+                for r in range(3) for s in range(3)]
+    return np.stack(taps, -1).reshape(dy.shape[1], x.shape[1], 3, 3)
+
+
+# 128-, 160- and 64-row tiles; rows of 64 to 8 pixels, whole images of 4 x 4; channels past a tile's edge; one chunk, split sums
+@pytest.mark.parametrize("shape", [(2, 32, 64, 64, 128), (3, 48, 32, 32, 160), (1, 70, 8, 8, 64), (5, 64, 16, 16, 128),
+                                   (3, 33, 8, 8, 320), (8, 64, 4, 4, 64), (4, 160, 4, 4, 160), (20, 128, 4, 4, 128), (2, 16, 32, 32, 20)])
+def test_filter_gradient(shape):
+    N, C, H, W, K = shape
+    r = rng(N + C + H)
+    x = np.maximum(r.standard_normal((N, C, H, W)), 0).astype(np.float32)
+    dy = r.standard_normal((N, K, H, W)).astype(np.float32)
+    got = ops.conv_bwd_filter(T(dy), T(x), (K, C, 3, 3), (1, 1), (1, 1)).numpy()
+    want, mag = filter_gradient(dy, x), filter_gradient(dy, x, np.abs)
+    assert np.all(np.abs(got - want) <= walk(N * H * W) * mag), np.max(np.abs(got - want) / mag)
+
+
+@pytest.mark.parametrize("shape", [(4, 64, 16, 16, 128), (8, 64, 4, 4, 64), (3, 32, 32, 32, 160)])
+def test_filter_gradient_operands_that_are_not_finite(shape):
+    N, C, H, W, K = shape
+    r = rng(K + H)
+    x = r.standard_normal((N, C, H, W)).astype(np.float32)
+    dy = (0.01 * r.standard_normal((N, K, H, W))).astype(np.float32)
+    x[0, 3, 1, 1], x[1, 5, 2, 0], x[2, 9, 3, 3], dy[1, 7, 2, 2], dy[0, 11, 0, 0] = np.inf, np.nan, 3.4e38, -np.inf, 1e-41
+    got = ops.conv_bwd_filter(T(dy), T(x), (K, C, 3, 3), (1, 1), (1, 1)).numpy()
+    want, mag = filter_gradient(dy, x), filter_gradient(dy, x, np.abs)
+    fine = mag < 3e38
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    assert np.all(np.abs(got[fine] - want[fine]) <= walk(N * H * W) * mag[fine])
