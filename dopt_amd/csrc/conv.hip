@@ -455,31 +455,34 @@ __global__ __launch_bounds__(T::THREADS, T::THREADS / 256) void conv_patch_k(Pat
 // images, so the input under them is the same rectangle with the same zero halo) or 64 rows x 64 tiles.
 // Per 16-channel chunk: the raw patch goes to LDS position-major (a thread owns one position and stores its channels
 // as 128-bit pieces); all 512 threads transform it - thread (i, tile, four channels) forms row i of Bt d B for its tile
-// from eight 128-bit reads and writes the four transformed values, four channels each, to V[xi][tile][16 channels];
-// wavefront (wk, wi) multiplies rows 32 wk .. + 31 with the eight positions xi = 8 wi .. 8 wi + 7: per position two
-// 128-bit reads of V (this lane's tile, its eight channels; one position ahead) and two 128-bit loads of the
-// transformed filter U[chunk][xi][row][16 channels] straight into operand registers, three positions ahead, feed
-// eight matrix instructions into the position's own accumulator (128 accumulator registers per wavefront, two
-// wavefronts per SIMD).  With 32 tiles, patch and V are double-buffered and the next chunk's transform runs under
+// from eight 128-bit reads, splits the sixteen values into their three bf16 parts (mfma_core.h) and writes them to
+// V[xi][part][channel half][tile].  The products run on the bf16 matrix instruction: per position and 32 tiles three
+// 128-bit reads of V (one step ahead) and three 128-bit loads of the packed filter's parts U[chunk][xi][part][row]
+// straight into operand registers (three positions ahead) feed six instructions into the position's own accumulator
+// (128 accumulator registers per wavefront, two wavefronts per SIMD).  128 rows: a wavefront takes 32 rows, 32 tiles and
+// eight positions; 64 rows: 32 rows, all 64 tiles and the four positions of one row i, so that a filter fragment serves
+// two steps (32 tiles and eight positions each, every fragment was loaded by two wavefronts: 160 channels on 32 x 32
+// images 259 us instead of 227).  With 32 tiles, patch and V are double-buffered and the next chunk's transform runs under
 // this chunk's matrix instructions; every piece of side work is pinned to a matrix step (sched_barrier), or the
 // scheduler sinks the prefetches to their first use.
 //
-// At the end a lane holds M[xi][row][tile] for its eight positions - two rows i of the 4x4 grid, complete in j - so it
-// applies A along j in registers (z[i][b]), combines its two rows into its share of the four outputs, and the
-// wavefronts of a pair add their shares through LDS: y[a][b] = (At z)[a][b].  Output, split reductions and bias are
-// those of the direct kernel.
+// At the end a lane holds M[xi][row][tile] for its positions, complete rows i of the 4x4 grid: it applies A along j in
+// registers (z[i][b]) and the wavefronts that share an output meet in LDS: y[a][b] = (At z)[a][b].  With 128 rows one of
+// a pair adds the other's share of the four outputs; with 64 rows all four leave their z and finish a quarter of the
+// outputs each.  Output, split reductions and bias are those of the direct kernel.  Outputs that are not finite are
+// formed again in fp32 (wino_fp32).
 //
-// What bounds it: a chunk is 3.4 us of matrix time per workgroup at the nominal rate, 3.95 in a build of this loop with
-// nothing but its matrix instructions, and takes 4.6 .. 5.0 - the filter loads (128 KB per chunk
-// and workgroup, 16/9 the direct kernel's), the V reads, the patch and the transform each add their share, roughly in
-// proportion to their instruction counts (loops without one of them: -0.5, -0.2, -0.3, -0.4 us).  128 rows x 64 tiles
-// would halve filter traffic and fragment loads per matrix instruction and need 256 accumulator registers per wavefront.
+// What bounds it (batch 128 with packing, the fp32 instruction -> this): 640 -> 640 channels on 8 x 8 images, batch 512,
+// 828 -> 627 us; 160 -> 160 on 32 x 32 318 -> 227; 128 -> 128 on 16 x 16, batch 256, 83 -> 66.  A chunk takes 2.9 us per
+// workgroup (fp32: 4.6 .. 5.0), of which 1.8 are matrix time at the rate a product of large matrices reaches.  No single
+// cost is left: filter fragments that hit the L1 would take 10 % off (they are 192 KB per chunk, 26 bytes per cycle from
+// the L2), no transform 8 %, no patch 6 %, no V reads 3 %; with 64 rows, whose single V is transformed between two
+// barriers, no transform 19 %.  64-row tiles in the place of 128-row tiles: 721 us for the first of the layers above.
 // floats of the exchange area: 128 rows: four wavefront pairs x 64 values per lane; 64 rows: eight wavefronts x 64 values
 constexpr int wino_xchg(int bm) { return (bm == 128 ? 4 : 8) * 64 * 64; }
 
-// WK x TH: the eight wavefronts are WK groups of 32 rows x TH groups of 32 tiles x the two halves of the 16 positions:
-// 4 x 1 (128 rows x 32 tiles = 128 pixels) for layers with whole 128-row tiles, 2 x 2 (64 rows x 64 tiles = 256 pixels)
-// for 64-row layers.
+// WK x TH: WK groups of 32 rows, TH groups of 32 tiles: 4 x 1 (128 rows x 32 tiles = 128 pixels) for layers with whole
+// 128-row tiles, 2 x 2 (64 rows x 64 tiles = 256 pixels) for 64-row layers.
 // The four outputs of one tile and row over channels c0 .. c1 - 1, in fp32 without matrix instructions: for the tiles whose
 // operands or results are not finite.  (ih0, iw0): the tile's first input pixel.
 __device__ __forceinline__ void wino_fp32(const PatchConv &p, int n, int m, int ih0, int iw0, int c0, int c1, float (&y)[4])
@@ -536,7 +539,7 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
     // one 128-bit read and neighbouring lanes' reads are neighbours
     constexpr int VP = 8 * TT, VX = 3 * VP, VSZ = 16 * VX;
     // 32 tiles per workgroup: V and the raw patch are double-buffered, the transform of the next chunk runs under this
-    // chunk's matrix instructions and the workgroup meets once per chunk.  64 tiles: one V (80 KB), transformed between
+    // chunk's matrix instructions and the workgroup meets once per chunk.  64 tiles: one V (96 KB), transformed between
     // two barriers.
     constexpr bool DB = TH == 1;
     extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -1930,11 +1933,13 @@ PackJob pack_job(const dopt_hip_conv_desc *d, const PatchSetup &u, const float *
 // in microseconds: rounds x (chunks per block x time per chunk + a fixed prologue/epilogue) plus,
 // when split, writing and re-reading the partial tiles.  The split with the lowest estimate wins;
 // ties go to the smaller one.
-int patch_splits(int tiles, int chunks, int slots, int BM, int BN, size_t out_elems)
+int patch_splits(int tiles, int chunks, int slots, int BM, int BN, size_t out_elems, bool wino)
 {
     const double cu_tflops = 0.47;                                   // what one CU sustains in these main loops
     const double per_cu = (double)slots / num_cus();                 // blocks sharing a CU
-    const double t_chunk = 2.0 * BM * BN * 144 / (cu_tflops * 1e6 / per_cu);   // 16 channels x 9 taps
+    // 16 channels x 9 taps; the Winograd kernel takes 2.9 us (128 rows) to 3.3 us (64 rows) for a chunk of its tile (320 channels
+    // on 16 x 16 images, batch 128, now uncut instead of two ways: 229 -> 223 us; 640 on 8 x 8: 216 -> 212)
+    const double t_chunk = wino ? 3.0 : 2.0 * BM * BN * 144 / (cu_tflops * 1e6 / per_cu);
     int best = 1;
     double best_cost = 0.0;
     for (int sp = 1; sp <= chunks && sp <= 64; sp++) {
@@ -1978,7 +1983,7 @@ int gather_splits(int tiles, int slabs, int slots, int BM, int BN, size_t out_el
 int patch_decide_splits(PatchSetup *u, const float *out)
 {
     PatchConv &pc = u->pc;
-    int splits = patch_splits(u->tiles, pc.chunks_total, u->blocks_wanted, u->BM, u->BN, pc.out_elems);
+    int splits = patch_splits(u->tiles, pc.chunks_total, u->blocks_wanted, u->BM, u->BN, pc.out_elems, u->shape == 4);
     if (pc.out_elems % 4 != 0 || !aligned16(out)) splits = 1;
     pc.chunks_per_split = (pc.chunks_total + splits - 1) / splits;
     splits = (pc.chunks_total + pc.chunks_per_split - 1) / pc.chunks_per_split;
