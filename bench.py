@@ -31,6 +31,7 @@ sys.path.insert(0, ROOT)
 
 BATCH = 128
 MFMA_FP32_PEAK_TFLOPS = 157.3
+MFMA_BF16_PEAK_TFLOPS = 2516.6
 HBM_PEAK_GBS = 8000.0
 
 
@@ -327,8 +328,8 @@ def main():
         # recorded around each launch inside the library, on the stream the kernel runs on (its steps may also run a
         # split sum, which is not part of this figure).  `achieved` counts the layer's FLOPs by the direct algorithm,
         # 2*N*K*C*R*S*P*Q - the algorithmic work of the operation, as the other figures of this file do; the kernel
-        # executes 16/36 of them on the matrix cores (`executed_*`), so `frac` above 1 is the algorithm's gain, not a
-        # measurement error.
+        # executes 16/36 of them, each as six bf16 products of the operands' three parts (`executed_*`, against the bf16
+        # peak), so `frac` above 1 is the algorithm's gain over the fp32 instruction, not a measurement error.
         launches = pl.value / nsteps if nsteps else 0
         tflops = pfl.value / (pus.value * 1e-6) / 1e12 if pus.value else 0.0
         result["roofline"] = {
@@ -337,7 +338,7 @@ def main():
                       "convolution kernels are listed under `kernels`",
             "bound": "mfma", "achieved": round(tflops, 2), "peak": MFMA_FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": round(tflops / MFMA_FP32_PEAK_TFLOPS, 4),
-            "executed_achieved": round(tflops * 16.0 / 36.0, 2), "executed_frac": round(tflops * 16.0 / 36.0 / MFMA_FP32_PEAK_TFLOPS, 4),
+            "executed_achieved": round(tflops * 96.0 / 36.0, 2), "executed_frac": round(tflops * 96.0 / 36.0 / MFMA_BF16_PEAK_TFLOPS, 4),
             "traffic": profile_line("traffic_bytes_per_launch conv_wino_k"),
             "traffic_source": "profiles/conv_kernels_vgg16_b128_hbm_traffic.txt (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE of "
                               "the same %d launches per step; taken from that file, not measured in this run)" % round(launches),
@@ -346,7 +347,7 @@ def main():
             "launches_per_step": int(round(launches)),
             "flops_per_launch": round(pfl.value / pl.value, 1) if pl.value else None,
             "flops_convention": "2*N*K*C*R*S*P*Q per launch, the direct algorithm's count; the kernel's matrix instructions "
-                                "execute 16/36 of it (sixteen products per 2x2 outputs instead of thirty-six)",
+                                "execute 16/36 of it (sixteen products per 2x2 outputs instead of thirty-six), each as six bf16 products",
             "avg_launch_us": round(pus.value / pl.value, 2) if pl.value else None,
             "timing": "HIP events around each launch on the library's stream, %d steps; an event pair also sees the "
                       "boundary to the kernel in front (3-4 us), which the profiler's kernel durations do not" % nsteps,

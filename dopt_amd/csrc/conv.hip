@@ -1240,7 +1240,8 @@ __global__ __launch_bounds__(256) void split_sum_k(size_t n4, int splits, size_t
 // (tap row r): a wavefront keeps the three taps s = 0..2 of its tap row in three 32x32
 // accumulators.  A lane's operands for a 16-pixel slab are pixels kh*8 .. kh*8+7 of the slab
 // (kh = lane / 32): two 128-bit reads of dy, and for x a window that serves all three taps by
-// register selection.
+// register selection.  The products run on the bf16 matrix instruction, each operand split into three parts in registers
+// (mfma_core.h).
 //
 // Geometry of a 64-pixel chunk (kGeo):
 //   0  rows of 8, 16, 32 or 64 pixels: G = 64/W full rows of one image.  Patch rows have pitch W+8
