@@ -516,17 +516,19 @@ __device__ __forceinline__ void wino_fp32(const PatchConv &p, int n, int m, int 
                 M[i * 4 + j] += (val(at) + val(at + part) + val(at + 2 * part)) * v[j];
             }
         }
-    }
-    float z[4][2];
+        float z[4][2];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        z[i][0] = (M[4 * i] + M[4 * i + 1]) + M[4 * i + 2];
-        z[i][1] = (M[4 * i + 1] - M[4 * i + 2]) - M[4 * i + 3];
-    }
+        for (int i = 0; i < 4; i++) {
+            z[i][0] = (M[4 * i] + M[4 * i + 1]) + M[4 * i + 2];
+            z[i][1] = (M[4 * i + 1] - M[4 * i + 2]) - M[4 * i + 3];
+        }
 #pragma unroll
-    for (int b = 0; b < 2; b++) {
-        y[b] = (z[0][b] + z[1][b]) + z[2][b];
-        y[2 + b] = (z[1][b] - z[2][b]) - z[3][b];
+        for (int b = 0; b < 2; b++) {
+            y[b] = (z[0][b] + z[1][b]) + z[2][b];
+            y[2 + b] = (z[1][b] - z[2][b]) - z[3][b];
+        }
+        // a NaN stays one, whatever the channels after it hold: a tile of NaNs costs one channel
+        if (y[0] != y[0] && y[1] != y[1] && y[2] != y[2] && y[3] != y[3]) break;
     }
 }
 
