@@ -184,3 +184,81 @@ def test_filter_gradient_operands_that_are_not_finite(shape):
     fine = mag < 3e38
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
     assert np.all(np.abs(got[fine] - want[fine]) <= walk(N * H * W) * mag[fine])
+
+
+# ---- the general kernels: any filter size, stride and padding
+
+def general(x, w, pad, stride, f=lambda v: v):
+    """A true convolution in float64, tap by tap; a zero of the padding times an infinity is not formed."""
+    N, C, H, W = x.shape
+    K, _, R, S = w.shape
+    P, Q = (H + 2 * pad - R) // stride + 1, (W + 2 * pad - S) // stride + 1
+    xp = np.pad(f(x.astype(np.float64)), ((0, 0), (0, 0), (pad, pad), (pad, pad)))
+    g = f(w.astype(np.float64))
+    y = np.zeros((N, K, P, Q))
+    with np.errstate(all="ignore"):
+        for r in range(R):
+            for s in range(S):
+                a, b = R - 1 - r, S - 1 - s
+                y += np.einsum("kc,nchw->nkhw", g[:, :, r, s], xp[:, :, a:a + stride * P:stride, b:b + stride * Q:stride])
+    return y
+
+
+def general_gradients(x, w, dy, pad, stride, f=lambda v: v):
+    N, C, H, W = x.shape
+    K, _, R, S = w.shape
+    P, Q = dy.shape[2:]
+    xp = np.pad(f(x.astype(np.float64)), ((0, 0), (0, 0), (pad, pad), (pad, pad)))
+    g, d, dx, dw = f(w.astype(np.float64)), f(dy.astype(np.float64)), np.zeros(xp.shape), np.zeros(w.shape)
+    for r in range(R):
+        for s in range(S):
+            at = np.s_[:, :, R - 1 - r:R - 1 - r + stride * P:stride, S - 1 - s:S - 1 - s + stride * Q:stride]
+            dx[at] += np.einsum("kc,nkhw->nchw", g[:, :, r, s], d)
+            dw[:, :, r, s] = np.einsum("nkhw,nchw->kc", d, xp[at])
+    return dx[:, :, pad:pad + H, pad:pad + W], dw
+
+
+# 64-row and 128-row tiles; 1 x 1 and 5 x 5 filters, strides 1 to 3; channel counts off the slab and one past a tile's rows
+@pytest.mark.parametrize("shape", [(2, 48, 13, 11, 100, 5, 2, 2), (3, 20, 9, 9, 64, 5, 2, 1), (4, 160, 16, 16, 320, 3, 1, 2),
+                                   (5, 33, 8, 8, 129, 1, 0, 1), (2, 64, 16, 16, 128, 1, 0, 2), (1, 17, 10, 7, 40, 3, 0, 3)])
+def test_general_convolution(shape):
+    N, C, H, W, K, R, pad, stride = shape
+    r = rng(C + K)
+    x = np.maximum(r.standard_normal((N, C, H, W)), 0).astype(np.float32)
+    w = r.standard_normal((K, C, R, R)).astype(np.float32)
+    got = ops.convolution(T(x), T(w), (pad, pad), (stride, stride)).numpy()
+    dy = r.standard_normal(got.shape).astype(np.float32)
+    want, mag = general(x, w, pad, stride), general(x, w, pad, stride, np.abs)
+    assert np.all(np.abs(got - want) <= walk(C * R * R) * mag)
+    wants, mags = general_gradients(x, w, dy, pad, stride), general_gradients(x, w, dy, pad, stride, np.abs)
+    dx = ops.conv_bwd_data(T(dy), T(w), x.shape, (pad, pad), (stride, stride)).numpy()
+    dw = ops.conv_bwd_filter(T(dy), T(x), w.shape, (pad, pad), (stride, stride)).numpy()
+    assert np.all(np.abs(dx - wants[0]) <= walk(K * R * R) * mags[0])
+    assert np.all(np.abs(dw - wants[1]) <= walk(dy[:, 0].size) * mags[1])
+
+
+def test_general_convolution_operands_that_are_not_finite():
+    """A value far from every bad one is what it is without them; an infinity stays one and a NaN stays one."""
+    r = rng(3)
+    x = np.abs(r.standard_normal((2, 48, 13, 11))).astype(np.float32) + np.float32(0.1)
+    w = np.abs(r.standard_normal((100, 48, 5, 5))).astype(np.float32) + np.float32(0.1)
+    dy = np.abs(r.standard_normal((2, 100, 7, 6))).astype(np.float32) + np.float32(0.1)
+    x[0, 3, 0, 0], x[0, 5, 12, 10], x[1, 7, 6, 5], dy[0, 1, 3, 3], dy[1, 9, 3, 2] = np.inf, np.nan, np.inf, np.inf, np.nan
+    pad = stride = (2, 2)
+    y = ops.convolution(T(x), T(w), pad, stride).numpy()
+    dx = ops.conv_bwd_data(T(dy), T(w), x.shape, pad, stride).numpy()
+    dw = ops.conv_bwd_filter(T(dy), T(x), w.shape, pad, stride).numpy()
+    fx, fdy = np.nan_to_num(x, nan=1.0, posinf=1.0), np.nan_to_num(dy, nan=1.0, posinf=1.0)
+    reach = lambda bad: bad.astype(np.float32)   # how many bad terms an output takes in
+    one_x, one_w, one_dy = np.ones_like(x), np.ones_like(w), np.ones_like(dy)
+    for got, nans, infs, want in (
+            (y, general(reach(np.isnan(x)), one_w, 2, 2), general(reach(np.isinf(x)), one_w, 2, 2), general(fx, w, 2, 2)),
+            (dx, general_gradients(x, one_w, reach(np.isnan(dy)), 2, 2)[0], general_gradients(x, one_w, reach(np.isinf(dy)), 2, 2)[0],
+             general_gradients(fx, w, fdy, 2, 2)[0]),
+            (dw, general_gradients(reach(np.isnan(x)), w, one_dy, 2, 2)[1] + general_gradients(one_x, w, reach(np.isnan(dy)), 2, 2)[1],
+             general_gradients(reach(np.isinf(x)), w, one_dy, 2, 2)[1] + general_gradients(one_x, w, reach(np.isinf(dy)), 2, 2)[1],
+             general_gradients(fx, w, fdy, 2, 2)[1])):
+        assert np.array_equal(np.isnan(got), nans > 0)
+        assert np.array_equal(np.isposinf(got), (infs > 0) & ~(nans > 0))
+        fine = np.isfinite(got)
+        assert np.all(np.abs(got[fine] - want[fine]) <= walk(2500) * want[fine])   # (every term is positive)
