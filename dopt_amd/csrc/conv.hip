@@ -57,7 +57,8 @@ struct GatherConv {
 // The products run on the bf16 matrix instruction, operands split as they are read from LDS (mma_slab_split): the loop was
 // bound by the fp32 instruction, 2048 cycles per slab and 64 x 64 wavefront tile, of which the six bf16 products take 768;
 // the splitting, 704 vector cycles, runs beside the other wavefront's.  50 images of 48 x 45 x 39, 100 filters of 5 x 5 at
-// stride 2, forward and both gradients: 379 -> 270 us.
+// stride 2, forward and both gradients: 379 -> 270 us.  Error against float64 (160 -> 320 channels, stride 2): 2.1e-7 -> 8.5e-8
+// forward, 5.3e-7 -> 1.7e-7 backward-data, 2.2e-7 -> 9.1e-8 filter gradient.
 // kMode: 0 = forward, 1 = backward-data with unit stride (no divisions), 2 = backward-data, any stride.
 // L: the workgroup's item among the problem's (split, tile) pairs, tile fastest.
 template <class T, int kMode>
