@@ -1329,6 +1329,11 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
     const int k0 = mt * BM, c0 = ct * BC;
     const int cb = split * p.chunks_per_split;
     const int ce = min(cb + p.chunks_per_split, p.chunks_total);
+    // The sum over the chunks is formed in kPasses parts of alternating sign, the first of which waits in `out` (see the products below).
+    constexpr bool kLow = WM * WC == 4;
+    constexpr int kPasses = kLow ? 1 : 2;
+    int from = cb, to = kPasses == 1 ? ce : (cb + ce + 1) / 2;
+    float sign = 1.0f;
 
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int kh = lane >> 5, l32 = lane & 31;
@@ -1340,21 +1345,16 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x, p.x_bytes);
 
     // ---- load slots.  dy: quad `quad` of row `row` is pixels 4*quad .. 4*quad+3 of the chunk, which
-    // lie in image quad / qpi of the chunk (qpi = quads of one image inside a chunk).
-    unsigned a_voff[NAQ];
-    int a_lds[NAQ];
+    // lie in image quad / qpi of the chunk (qpi = quads of one image inside a chunk).  Slot i of a thread is the quad AROWS i
+    // rows below its first one, so one offset and one LDS place serve all of them.
+    constexpr int AROWS = THREADS / 16;
     const int qpi = kGeo == 0 ? 16 : HW / 4;
-#pragma unroll
-    for (int i = 0; i < NAQ; i++) {
-        const int a = i * THREADS + tid;
-        const int row = a / 16, quad = a % 16;
-        const int j = quad / qpi, wq = quad - j * qpi;
-        const bool ok = a < BM * 16 && k0 + row < p.K;
-        a_voff[i] = ok ? (unsigned)((j * p.K + k0 + row) * HW + wq * 4) * 4u : kOobOffset;
-        a_lds[i] = a < BM * 16 ? row * APITCH + quad * 4 : -1;
-    }
+    const int a_row = tid / 16, a_quad = tid % 16;
+    const unsigned a_voff = (unsigned)((a_quad / qpi * p.K + k0 + a_row) * HW + a_quad % qpi * 4) * 4u;
+    const int a_lds = a_row * APITCH + a_quad * 4;
+    const int a_rows = min(BM, p.K - k0);
     unsigned b_voff[NBQ];
-    int b_lds[NBQ], b_edge[NBQ];  // b_edge (geometry 0): 1 = top halo row, 2 = bottom halo row
+    int b_lds[NBQ];   // float index inside a patch buffer (a multiple of four) or -1; geometry 0: + 1 = top halo row, + 2 = bottom halo row
 #pragma unroll
     for (int i = 0; i < NBQ; i++) {
         const int b = i * THREADS + tid;
@@ -1365,20 +1365,17 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
             const bool ok = c < BC && c0 + c < p.C;
             // row p0 - 1 + pr of channel c0 + c; p0 and the image are added per chunk
             b_voff[i] = ok ? (unsigned)(((c0 + c) * p.H + pr) * p.W + quad * 4) * 4u : kOobOffset;
-            b_lds[i] = c < BC ? c * p.cstride + pr * p.ppitch + 4 + quad * 4 : -1;
-            b_edge[i] = pr == 0 ? 1 : (pr == p.G + 1 ? 2 : 0);
+            b_lds[i] = c < BC ? c * p.cstride + pr * p.ppitch + 4 + quad * 4 + (pr == 0 ? 1 : pr == p.G + 1 ? 2 : 0) : -1;
         } else if (kGeo == 1) {
             const int c = b / 16, j = (b / 4) % 4, row = b % 4;  // image j of the chunk, image row `row`
             const bool ok = c < BC && c0 + c < p.C;
             b_voff[i] = ok ? (unsigned)((j * p.C + c0 + c) * 16 + row * 4) * 4u : kOobOffset;
             b_lds[i] = c < BC ? c * p.cstride + j * 72 + (row + 1) * 12 + 4 : -1;
-            b_edge[i] = 0;
         } else {
             const int c = b / 16, j = b % 16;  // the whole 2x2 image j is one quad
             const bool ok = c < BC && c0 + c < p.C;
             b_voff[i] = ok ? (unsigned)((j * p.C + c0 + c) * 4) * 4u : kOobOffset;
             b_lds[i] = c < BC ? c * p.cstride + j * 16 + 5 : -1;  // cell (1,1) of the 4x4 block
-            b_edge[i] = 0;
         }
     }
     float4 areg[NAQ], breg[NBQ];
@@ -1388,7 +1385,8 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
         const int p0 = band * p.G;
         const unsigned a_soff = (unsigned)(n_img * p.K * HW + p0 * p.W) * 4u;
 #pragma unroll
-        for (int i = 0; i < NAQ; i++) areg[i] = buffer_load_f32x4(rdy, a_voff[i], a_soff);
+        for (int i = 0; i < NAQ; i++)
+            areg[i] = buffer_load_f32x4(rdy, a_row + AROWS * i < a_rows ? a_voff + (unsigned)(AROWS * i * HW) * 4u : kOobOffset, a_soff);
         if (kGeo == 0) {
             // x row p0 - 1 + pr.  Offsets handed to a buffer load must not go negative: the "- 1" row
             // is taken off the wave-uniform part, except for the very first chunk of the tensor, where
@@ -1400,7 +1398,7 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
             const unsigned b_soff = (unsigned)(n_img * p.C * HW + p0 * p.W) * 4u - (first ? 0u : roww);
 #pragma unroll
             for (int i = 0; i < NBQ; i++) {
-                const bool dead = (b_edge[i] & kill) != 0 || b_voff[i] == kOobOffset;
+                const bool dead = (b_lds[i] & kill) != 0 || b_voff[i] == kOobOffset;
                 breg[i] = buffer_load_f32x4(rx, dead ? kOobOffset : b_voff[i] - (first ? roww : 0u), b_soff);
             }
             if (++band == p.bands) {
@@ -1417,11 +1415,15 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
     auto stash = [&](int buf) {
         float *A = A0 + buf * (BM * APITCH), *B = B0 + buf * bsize;
 #pragma unroll
-        for (int i = 0; i < NAQ; i++) *(float4 *)(a_lds[i] >= 0 ? A + a_lds[i] : dummy) = areg[i];
+        for (int i = 0; i < NAQ; i++) {
+            const float4 v = areg[i];
+            *(float4 *)(AROWS * (i + 1) <= BM || a_row + AROWS * i < BM ? A + a_lds + AROWS * i * APITCH : dummy) =
+                kLow ? v : make_float4(v.x * sign, v.y * sign, v.z * sign, v.w * sign);
+        }
 #pragma unroll
         for (int i = 0; i < NBQ; i++) {
             if (kGeo != 2) {
-                *(float4 *)(b_lds[i] >= 0 ? B + b_lds[i] : dummy) = breg[i];
+                *(float4 *)(b_lds[i] >= 0 ? B + (b_lds[i] & ~3) : dummy) = breg[i];
             } else {
                 float *q = b_lds[i] >= 0 ? B + b_lds[i] : dummy;  // rows 1 and 2 of the cell block, columns 1..2
                 const int down = b_lds[i] >= 0 ? 4 : 0;
@@ -1435,27 +1437,17 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
 
     // ---- fragment addresses
     const int a_frag = (wm * 32 + l32) * APITCH + kh * 8;
-    int b_frag[4];  // float4 index inside a patch buffer, per slab
-    const int chan = (wc * 32 + l32) * p.cstride;
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-        if (kGeo == 0) {
-            // slab s covers the 8-pixel runs 2s (kh = 0) and 2s+1 (kh = 1) of the chunk
-            const int runs_row = p.W / 8;
-            const int u = 2 * s + kh, rho = u / runs_row, q0 = (u - rho * runs_row) * 8;
-            b_frag[s] = (chan + (rho + dr) * p.ppitch + q0) / 4 + 1;  // quad of pixel q0
-        } else if (kGeo == 1) {
-            b_frag[s] = (chan + s * 72 + (2 * kh + dr) * 12) / 4 + 1;  // image s, image rows 2kh and 2kh+1
-        } else {
-            b_frag[s] = (chan + (4 * s + 2 * kh) * 16 + dr * 4) / 4;   // images 4s+2kh and 4s+2kh+1
-        }
-    }
+    // float4 index inside a patch buffer: of slab 0, and how far the other slabs are from it (the same for all lanes)
+    const int runs_row = p.W / 8;
+    const int b_frag = kGeo == 0 ? ((wc * 32 + l32) * p.cstride + (dr + (runs_row == 1 ? kh : 0)) * p.ppitch + (runs_row == 1 ? 0 : kh * 8)) / 4 + 1
+                     : kGeo == 1 ? ((wc * 32 + l32) * p.cstride + (2 * kh + dr) * 12) / 4 + 1   // image s, image rows 2kh and 2kh+1
+                                 : ((wc * 32 + l32) * p.cstride + 2 * kh * 16 + dr * 4) / 4;    // images 4s+2kh and 4s+2kh+1
+    // geometry 0: slab s covers the 8-pixel runs 2s (kh = 0) and 2s+1 (kh = 1) of the chunk
+    auto b_step = [&](int s) {
+        return kGeo == 0 ? (2 * s / runs_row * p.ppitch + 2 * s % runs_row * 8) / 4 : kGeo == 1 ? s * 72 / 4 : s * 64 / 4;
+    };
 
-    // halo cells are never written again: clear both patch buffers once
-    for (int i = tid; i < 2 * bsize; i += THREADS) B0[i] = 0.0f;
-    __syncthreads();
-
-    v16f acc[3];
+    v16f acc[3], low[kLow ? 3 : 1];
     typedef __attribute__((address_space(3))) float lds_float_t;
     // Fetching runs one chunk ahead and also past the end of this block's range: those loads are
     // range-checked and their data lands in the LDS buffer that is not read again.
@@ -1467,7 +1459,7 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
         Frag f;
         const float *A = A0 + buf * (BM * APITCH) + a_frag;
         // float4 indexing keeps the 16-byte alignment of the patch reads visible to the compiler
-        const float4 *bq = (const float4 *)B0 + buf * (bsize / 4) + b_frag[s_];
+        const float4 *bq = (const float4 *)B0 + buf * (bsize / 4) + b_frag + b_step(s_);
         // The edge-column reads are volatile so that the compiler does not fuse a whole window
         // into one run starting at the unaligned edge (it would then read it in 2-dword pieces).
         const volatile lds_float_t *be = (const volatile lds_float_t *)bq;
@@ -1517,11 +1509,19 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
                     acc[ds] = __builtin_amdgcn_mfma_f32_32x32x2f32(a8[ks], win[ks / 2][(ks & 1) + ds], acc[ds], 0, 0, 0);
         }
     };
-    // The same sixteen pixels on the bf16 matrix instructions (eighteen of 32 cycles for twenty-four of 64): the fragments are split in registers (mfma_core.h), the x
-    // pixels in pairs that are tap column 1's operands as they are; those of columns 0 and 2 are their neighbouring halves
-    // with the edge pixels.  128 images of 320 -> 320 channels, 16 x 16: 450 -> 318 us (134 -> 190 TFLOP/s); what bounds it
-    // now is the splitting itself, 120 vector instructions a step and wavefront under the 576 cycles of the matrix ones.
-    // (Reading the fragments one step ahead, as the fp32 form did, needs 30 more registers than there are: 399 us.)
+    // The same sixteen pixels on the bf16 matrix instructions (eighteen of 32 cycles for twenty-four of 64): the fragments are
+    // split in registers (mfma_core.h), the x pixels in pairs that are tap column 1's operands as they are; those of columns 0
+    // and 2 are their neighbouring halves with the edge pixels.  What bounds it is the splitting, 120 vector instructions a step
+    // and wavefront under the 576 cycles of the matrix ones.  (Reading the fragments one step ahead, as the fp32 form did, needs
+    // 30 more registers than there are: 399 us for the first layer below.)
+    // The instruction rounds down what lies below its guard bits.  That is the same way in every block, so no sum over blocks
+    // removes it, and the five small products of a slab suffer it most: with all six in one accumulator 77 % of the error was a
+    // common offset, and it was 1.25 to 1.7 times the fp32 instruction's.  So twelve wavefronts keep the small products in an
+    // accumulator of their own (which fits since a thread's dy slots share an offset and the slabs' places are scalars); fifteen
+    // have no registers for it and add the chunks in two halves of opposite sign instead, whose offsets cancel.
+    // 128 images of 320 -> 320 channels, 16 x 16: fp32 450 us, one accumulator 292, this 296; 160 -> 160, 32 x 32: 486, 302, 327.
+    // Error against float64 (one half of x zero): 64 -> 64 channels, 32 x 32, 2.8e-7 / 4.8e-7 / 1.3e-7; 160 -> 160, 32 x 32,
+    // 6.4e-7 / 1.07e-6 / 5.2e-7; 640 -> 640, 8 x 8, batch 256, 6.7e-7 / 8.4e-7 / 2.6e-7.
     constexpr int NW = kGeo == 0 ? 5 : kGeo == 1 ? 6 : 8;   // pairs of pixels
     v4u ap[3];
     unsigned q[3][NW];
@@ -1569,23 +1569,26 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
             static_for<0, 3 - part>([&](auto atag) {   // x's l with dy's h; m with m, h; h with l, m, h
                 constexpr int pa = 2 - part - decltype(atag)::value;
 #pragma unroll
-                for (int ds = 0; ds < 3; ds++) acc[ds] = mfma_bf16(ap[pa], b[ds], acc[ds]);
+                for (int ds = 0; ds < 3; ds++) {
+                    v16f &c = kLow && part + pa > 0 ? low[kLow ? ds : 0] : acc[ds];
+                    c = mfma_bf16(ap[pa], b[ds], c);
+                }
             });
         });
     };
     auto run = [&](auto exact_tag) {
         constexpr bool exact = decltype(exact_tag)::value != 0;
-        n_img = kGeo == 0 ? cb / p.bands : cb * p.imgs;
-        band = kGeo == 0 ? cb - n_img * p.bands : 0;
+        n_img = kGeo == 0 ? from / p.bands : from * p.imgs;
+        band = kGeo == 0 ? from - n_img * p.bands : 0;
 #pragma unroll
         for (int t = 0; t < 3; t++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) acc[t][v] = 0.0f;
+            for (int v = 0; v < 16; v++) acc[t][v] = low[kLow ? t : 0][v] = 0.0f;
         fetch();
         stash(0);
         __syncthreads();
         int cur = 0;
-        for (int chunk = cb; chunk < ce; ++chunk) {
+        for (int chunk = from; chunk < to; ++chunk) {
             static_for<0, 4>([&](auto stag) {
                 constexpr int s = decltype(stag)::value;
                 if constexpr (s == 0) fetch();
@@ -1600,50 +1603,63 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
             __syncthreads();
             cur ^= 1;
         }
-    };
-    run(StepTag<0>{});
-    {
-        // the parts of an infinity hold NaNs: a tile that is not finite is formed again with the fp32 instruction
-        float probe = 0.0f;
 #pragma unroll
         for (int t = 0; t < 3; t++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) probe = __builtin_fmaf(acc[t][v], 0.0f, probe);
-        volatile int *const again = (volatile int *)dummy;
-        if (tid == 0) *again = 0;
+            for (int v = 0; v < 16; v++) acc[t][v] = kLow ? acc[t][v] + low[kLow ? t : 0][v] : acc[t][v] * sign;
+    };
+    for (int pass = 0;; pass++) {
+        // halo cells are not written by the loop: clear both patch buffers before it
+        for (int i = tid; i < 2 * bsize; i += THREADS) B0[i] = 0.0f;
         __syncthreads();
-        if (probe != 0.0f) *again = 1;
-        __syncthreads();
-        const bool redo = *again != 0;
-        __syncthreads();   // (the second pass may store there)
-        if (redo) run(StepTag<1>{});
-    }
+        run(StepTag<0>{});
+        {
+            // the parts of an infinity hold NaNs: a tile that is not finite is formed again with the fp32 instruction
+            float probe = 0.0f;
+#pragma unroll
+            for (int t = 0; t < 3; t++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) probe = __builtin_fmaf(acc[t][v], 0.0f, probe);
+            volatile int *const again = (volatile int *)dummy;
+            if (tid == 0) *again = 0;
+            __syncthreads();
+            if (probe != 0.0f) *again = 1;
+            __syncthreads();
+            const bool redo = *again != 0;
+            __syncthreads();   // (forming it again may store there)
+            if (redo) run(StepTag<1>{});
+        }
 
-    // Epilogue: the accumulators leave through LDS so that every output row -- the BC*9 values
-    // [c][tap] of one k, contiguous in dw's own layout -- is written as one run.  One group of 32
-    // rows (the wavefronts with the same wm) is staged per pass.  out = dw itself when there is one
-    // split, else this split's partial copy (same layout, summed afterwards in split order).
-    __syncthreads();  // all fragment reads of the last chunk are done: LDS is free
-    constexpr int RP = BC * 9 + 1;  // staging row pitch (odd: the 4-row stride between lane halves spreads over banks)
-    float *outp = p.out + (size_t)split * p.split_stride;
-    const int ncv = min(BC, p.C - c0) * 9;  // valid floats of a staged row
-    for (int g = 0; g < WM; g++) {
-        if (wm == g) {
+        // Epilogue: the accumulators leave through LDS so that every output row -- the BC*9 values
+        // [c][tap] of one k, contiguous in dw's own layout -- is written as one run.  One group of 32
+        // rows (the wavefronts with the same wm) is staged at a time.  out = dw itself when there is one
+        // split, else this split's partial copy (same layout, summed afterwards in split order).
+        __syncthreads();  // all fragment reads of the last chunk are done: LDS is free
+        constexpr int RP = BC * 9 + 1;  // staging row pitch (odd: the 4-row stride between lane halves spreads over banks)
+        float *outp = p.out + (size_t)split * p.split_stride;
+        const int ncv = min(BC, p.C - c0) * 9;  // valid floats of a staged row
+        for (int g = 0; g < WM; g++) {
+            if (wm == g) {
 #pragma unroll
-            for (int ds = 0; ds < 3; ds++) {
-                const int t = (2 - dr) * 3 + (2 - ds);
+                for (int ds = 0; ds < 3; ds++) {
+                    const int t = (2 - dr) * 3 + (2 - ds);
 #pragma unroll
-                for (int v = 0; v < 16; v++) lds[acc_row(v, lane) * RP + (wc * 32 + l32) * 9 + t] = acc[ds][v];
+                    for (int v = 0; v < 16; v++) lds[acc_row(v, lane) * RP + (wc * 32 + l32) * 9 + t] = acc[ds][v];
+                }
             }
+            __syncthreads();
+            for (int r = w; r < 32; r += 3 * WM * WC) {  // one wavefront per row
+                const int k = k0 + g * 32 + r;
+                if (k >= p.K) continue;
+                float *dst = outp + ((size_t)k * p.C + c0) * 9;
+                for (int j = lane; j < ncv; j += 64) dst[j] = pass == 0 ? lds[r * RP + j] : dst[j] + lds[r * RP + j];
+            }
+            __syncthreads();
         }
-        __syncthreads();
-        for (int r = w; r < 32; r += 3 * WM * WC) {  // one wavefront per row
-            const int k = k0 + g * 32 + r;
-            if (k >= p.K) continue;
-            float *dst = outp + ((size_t)k * p.C + c0) * 9;
-            for (int j = lane; j < ncv; j += 64) dst[j] = lds[r * RP + j];
-        }
-        __syncthreads();
+        if (pass + 1 == kPasses || to == ce) break;
+        from = to;
+        to = ce;
+        sign = -sign;
     }
 }
 

@@ -186,6 +186,28 @@ def test_filter_gradient_operands_that_are_not_finite(shape):
     assert np.all(np.abs(got[fine] - want[fine]) <= walk(N * H * W) * mag[fine])
 
 
+def rounded_once_per_term(terms):
+    """Relative error (2-norm) of a sum of `terms` products of zero mean that is rounded after each: a rounding is uniform over
+    one unit in the last place, 0.43 * 2^-24 of the partial sum in the root mean square (the leading digits of the partial sum
+    spread evenly over their logarithm), and the partial sums grow with the root of their length: 0.43 / sqrt(2) * sqrt(terms)."""
+    return 0.30 * 2.0 ** -24 * np.sqrt(terms)
+
+
+# an odd number of filter values, so one block adds all the pixels: 64-, 128- and 160-row tiles, every pixel geometry
+@pytest.mark.parametrize("shape", [(32, 33, 16, 16, 65), (8, 33, 32, 32, 65), (128, 33, 8, 8, 65), (512, 17, 4, 4, 65), (32, 17, 16, 16, 255),
+                                   (2, 17, 64, 64, 255), (512, 17, 4, 4, 255), (8, 17, 32, 32, 159), (128, 17, 8, 8, 159),
+                                   (512, 17, 4, 4, 159)])
+def test_filter_gradient_is_not_further_off_than_one_rounding_per_term(shape):
+    N, C, H, W, K = shape
+    r = rng(N + H + K)
+    x = np.maximum(r.standard_normal((N, C, H, W)), 0).astype(np.float32)
+    dy = r.standard_normal((N, K, H, W)).astype(np.float32)
+    got = ops.conv_bwd_filter(T(dy), T(x), (K, C, 3, 3), (1, 1), (1, 1)).numpy()
+    want = filter_gradient(dy, x)
+    # half of the terms are zero, and a sum is not rounded by adding one
+    assert np.linalg.norm(got - want) <= rounded_once_per_term(N * H * W / 2) * np.linalg.norm(want)
+
+
 # ---- the general kernels: any filter size, stride and padding
 
 def general(x, w, pad, stride, f=lambda v: v):
