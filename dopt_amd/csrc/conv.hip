@@ -1987,13 +1987,15 @@ PackJob pack_job(const dopt_hip_conv_desc *d, const PatchSetup &u, const float *
 // in microseconds: rounds x (chunks per block x time per chunk + a fixed prologue/epilogue) plus,
 // when split, writing and re-reading the partial tiles.  The split with the lowest estimate wins;
 // ties go to the smaller one.
-int patch_splits(int tiles, int chunks, int slots, int BM, int BN, size_t out_elems, bool wino)
+int patch_splits(int tiles, int chunks, int slots, int BM, int BN, size_t out_elems)
 {
     const double cu_tflops = 0.47;                                   // what one CU sustains in these main loops
     const double per_cu = (double)slots / num_cus();                 // blocks sharing a CU
-    // 16 channels x 9 taps; the Winograd kernel takes 2.9 us (128 rows) to 3.3 us (64 rows) for a chunk of its tile (320 channels
-    // on 16 x 16 images, batch 128, now uncut instead of two ways: 229 -> 223 us; 640 on 8 x 8: 216 -> 212)
-    const double t_chunk = wino ? 3.0 : 2.0 * BM * BN * 144 / (cu_tflops * 1e6 / per_cu);
+    // 16 channels x 9 taps.  The Winograd kernel takes a third of that for a chunk, but adds all six parts of a product in one
+    // accumulator: with its own time here it would be cut less and be further off than the fp32 instruction, which was cut by
+    // this estimate (320 channels on 16 x 16 images, error against float64: fp32 2.9e-7, uncut 4.2e-7, cut in two 2.5e-7; batch
+    // 128 216 and 219 us; 160 on 32 x 32 2.5e-7, 2.9e-7, 2.1e-7, and the same time).
+    const double t_chunk = 2.0 * BM * BN * 144 / (cu_tflops * 1e6 / per_cu);
     int best = 1;
     double best_cost = 0.0;
     for (int sp = 1; sp <= chunks && sp <= 64; sp++) {
@@ -2037,7 +2039,7 @@ int gather_splits(int tiles, int slabs, int slots, int BM, int BN, size_t out_el
 int patch_decide_splits(PatchSetup *u, const float *out)
 {
     PatchConv &pc = u->pc;
-    int splits = patch_splits(u->tiles, pc.chunks_total, u->blocks_wanted, u->BM, u->BN, pc.out_elems, u->shape == 4);
+    int splits = patch_splits(u->tiles, pc.chunks_total, u->blocks_wanted, u->BM, u->BN, pc.out_elems);
     if (pc.out_elems % 4 != 0 || !aligned16(out)) splits = 1;
     pc.chunks_per_split = (pc.chunks_total + splits - 1) / splits;
     splits = (pc.chunks_total + pc.chunks_per_split - 1) / pc.chunks_per_split;

@@ -146,6 +146,39 @@ def test_winograd_operands_that_are_not_finite(shape):
     assert np.all(np.isfinite(got[fits]))
 
 
+def winograd_fp32(x, w, halves):
+    """`winograd` in fp32, the channels of each of `halves` added one after the other and rounded after each."""
+    N, C, H, W = x.shape
+    g = w[:, :, ::-1, ::-1]
+    xp = np.pad(x, ((0, 0), (0, 0), (1, 1), (1, 1)))
+    d = np.stack([np.stack([xp[:, :, r:r + H:2, q:q + W:2] for q in range(4)], -1) for r in range(4)], -2)
+    u = sandwich(G.astype(np.float32), g)
+    v = sandwich(BT.astype(np.float32), d).transpose(1, 4, 5, 0, 2, 3).reshape(C, 4, 4, -1)
+    y = 0.0
+    for part in np.array_split(np.arange(C), halves):
+        m = np.zeros((w.shape[0], 4, 4, v.shape[-1]), np.float32)
+        for c in part:
+            m = (m + u[:, c, :, :, None].astype(np.float64) * v[c]).astype(np.float32)
+        t = sandwich(AT.astype(np.float32), m.transpose(0, 3, 1, 2))
+        y = y + t.reshape(-1, N, H // 2, W // 2, 2, 2).transpose(1, 0, 2, 4, 3, 5).reshape(N, -1, H, W)
+    return y
+
+
+# layers whose tiles fill less than half of the chip
+@pytest.mark.parametrize("shape", [(32, 64, 32, 32, 64), (32, 320, 16, 16, 320), (32, 160, 32, 32, 160)])
+def test_winograd_is_not_further_off_than_fp32_in_two_halves(shape):
+    N, C, H, W, K = shape
+    r = rng(C)
+    x = np.maximum(r.standard_normal((N, C, H, W)), 0).astype(np.float32)
+    w = (r.standard_normal((K, C, 3, 3)) * np.sqrt(2 / (9 * C))).astype(np.float32)
+    rows = np.arange(0, K, K // 8)
+    got = ops.convolution(T(x), T(w), (1, 1), (1, 1)).numpy()[:4, rows]
+    x, w = x[:4], w[rows]
+    want, fp32 = winograd(x, w), winograd_fp32(x, w, 2)
+    assert fp32.dtype == np.float32
+    assert np.linalg.norm(got - want) <= np.linalg.norm(fp32 - want)
+
+
 # ---- the filter gradient of 3 x 3 layers
 
 def filter_gradient(dy, x, f=lambda v: v):
