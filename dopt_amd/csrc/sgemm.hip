@@ -24,6 +24,7 @@ struct Gemm {
     int M, N, K;
     int lda, ldb;  // row pitch of A and B as stored
     int mtiles, ntiles, slabs_total, slabs_per_split, splits;
+    int slabs_per_pass;   // sgemm_rows_k: a split is added up in C in passes of so many slabs
     size_t out_elems;
 };
 
@@ -171,7 +172,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void sgemm_k(Gemm p)
 // operands - which must fit into the slots they leave (eight per instruction); it goes with the sides of a wavefront's
 // tile.  Eight wavefronts of 128 x 64 in 256 x 256 tiles, one workgroup per CU: 1068 -> 640 us for 4096 x 4096 x 4096
 // (129 -> 215 TFLOP/s); 64 x 64 in 128 x 256 and 256 x 128: 755 us; 64 x 32 in 128 x 128: 965 us, for outputs too small
-// to give every CU a larger tile.  The smaller ones have registers for a second set of accumulators.
+// to give every CU a larger tile.  The smaller ones have registers for a second set of accumulators, the smallest for a third.
 // In the largest tile half of the threads stage A, half B, each a block of four rows by four steps: of a k-contiguous operand four 16-byte
 // pieces of four rows (four lanes per 64-byte row segment), of an r-contiguous one four 16-byte pieces of four steps
 // (sixteen lanes per 256 bytes), which become the quads of four rows by naming the registers.
@@ -250,7 +251,7 @@ template <int WM_, int WN_, int MI_, int NI_>
 struct RowsTile {
     static constexpr int WM = WM_, WN = WN_, MI = MI_, NI = NI_, BM = 32 * WM * MI, BN = 32 * WN * NI;
     static constexpr int kBuf = (BM + BN) * kRowBytes;   // a buffer: the lines of A, then those of B
-    static constexpr bool kLow = MI * NI <= 4;
+    static constexpr bool kLow = MI * NI <= 4, kTotal = MI * NI <= 2;   // which sets of registers there are beside the accumulators
     static_assert(WM * WN * 64 == kRowsThreads && BM % 64 == 0 && BN % 64 == 0 && BM + BN <= kRowsThreads, "one block of four rows by four steps per thread");
 };
 
@@ -275,8 +276,26 @@ __global__ __launch_bounds__(kRowsThreads, 2) void sgemm_rows_k(Gemm p)
     const int arow = wm * 32 * MI + l32, brow = wn * 32 * NI + l32;
 
     // low: the four smaller kinds of products, where there are registers for them
-    constexpr bool kLow = T::kLow;
-    v16f acc[MI][NI], low[kLow ? MI : 1][kLow ? NI : 1];
+    // total: the finished passes, where there are registers for them too
+    constexpr bool kLow = T::kLow, kTotal = T::kTotal;
+    v16f acc[MI][NI], low[kLow ? MI : 1][kLow ? NI : 1], total[kTotal ? MI : 1][kTotal ? NI : 1];
+    auto add_low = [&]() {
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NI; j++)
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+                    if (kLow) acc[i][j][v] += low[i % (kLow ? MI : 1)][j % (kLow ? NI : 1)][v];
+    };
+    auto add_total = [&]() {
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NI; j++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc[i][j][v] += total[i % (kTotal ? MI : 1)][j % (kTotal ? NI : 1)][v];
+    };
     // Slab s is multiplied out of one LDS buffer in two groups of 3 MI NI matrix instructions (quads 0 and 1, quads 2 and 3).
     // Between them slab s + 1, fetched an iteration ago, is split and stored into the other buffer, and slab s + 2 is
     // requested.  A group's fragments are read while the group before it is multiplied; those of the next slab's first
@@ -364,15 +383,15 @@ __global__ __launch_bounds__(kRowsThreads, 2) void sgemm_rows_k(Gemm p)
                 }
             }
     };
-    // With one accumulator for all products the sum is rounded twelve times per 16 steps, which the fp32 instruction
-    // rounds eight times; two sums over half the steps each have half the error.  The first of them waits in C.  (A
-    // reduction cut over blocks is such sums already.)
-    const int half = kLow || p.splits > 1 ? k_end : k_begin + (k_end - k_begin + 2 * BK - 1) / (2 * BK) * BK;
+    // A split's sum is formed in passes (sgemm_route says how long they are), all but the last of which wait in `total` or in C.
     float top = 0.0f;   // NaN once anything is not finite: x * 0 is 0 for finite x only
 #pragma clang loop unroll(disable)
-    for (int from = k_begin, to = half; from < k_end; from = to, to = k_end) {
+    for (int from = k_begin, to; from < k_end; from = to) {
+        to = kTotal ? k_end : min(from + p.slabs_per_pass * BK, k_end);
+        int left = p.slabs_per_pass;   // kTotal: slabs until the end of the pass
         zero_acc(acc);
         zero_acc(low);
+        zero_acc(total);
         st.load(rs, from, to);
 #pragma unroll
         for (int e = 0; e < 4; e++) st.store(mine, e);
@@ -406,18 +425,28 @@ __global__ __launch_bounds__(kRowsThreads, 2) void sgemm_rows_k(Gemm p)
                 read_l(rows_lds + (cur ^ 1) * kBuf, 0);
                 part(1, 0);
                 __builtin_amdgcn_sched_barrier(0);
+                if (kTotal && --left == 0) {   // uniform
+                    add_low();
+                    add_total();
+#pragma unroll
+                    for (int i = 0; i < (kTotal ? MI : 1); i++)
+#pragma unroll
+                        for (int j = 0; j < (kTotal ? NI : 1); j++) total[i][j] = acc[i][j];
+                    zero_acc(acc);
+                    zero_acc(low);
+                    left = p.slabs_per_pass;
+                }
             }
         }
-        __syncthreads();   // the buffers are free for the second half
+        __syncthreads();   // the buffers are free for the next pass
+        add_low();
+        if (kTotal) add_total();
 #pragma unroll
         for (int i = 0; i < MI; i++)
 #pragma unroll
             for (int j = 0; j < NI; j++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    if (kLow) acc[i][j][v] += low[i % (kLow ? MI : 1)][j % (kLow ? NI : 1)][v];
-                    top = __fmaf_rn(acc[i][j][v], 0.0f, top);
-                }
+                for (int v = 0; v < 16; v++) top = __fmaf_rn(acc[i][j][v], 0.0f, top);
         put(from != k_begin);
     }
     if (!__any(top != 0.0f)) return;
@@ -946,6 +975,7 @@ struct Route {
     enum Kind { kNone, kOuter, kGemvRows, kGemvColsShort, kGemvCols, kPanel, kSmall, kTile64, kTile128, kRows, kRowsBig } kind;
     size_t cuts;    // partial sums per element that a second pass adds (gemv slices, tile-engine splits)
     size_t depth;   // reduction steps per partial sum (k per slice, slabs per split)
+    size_t pass = 0;   // sgemm_rows_k: slabs that are added in its accumulators before they go to C
     size_t bm = 128, bn = 128;   // the tile engines' tile (no part of the order: every tile of a kind adds its elements' terms alike)
 };
 
@@ -972,7 +1002,8 @@ int rows_launch(const Route &r, dim3 grid, const Gemm &g)
 
 
 // What a tile of sgemm_rows_k costs per 16 steps with every CU at work (4096 x 4096 x 4096: 630, 755 and 965 us); a
-// workgroup's own start and end take about 4 us, split copies are written and read at about 5 TB/s.
+// workgroup's own start and end take about 4 us, split copies are written and read at about 5 TB/s, and another pass takes
+// 3 us and its tile twice through a CU's 0.1 TB/s where it waits in C, half a microsecond where it waits in registers.
 struct RowsShape {
     size_t bm, bn;
     double slab_us;
@@ -981,7 +1012,7 @@ constexpr RowsShape kRowsShapes[] = {{256, 256, 2.4}, {128, 256, 1.45}, {256, 12
 
 Route sgemm_route(int transA, int transB, size_t M, size_t N, size_t K, bool panel_allowed = true)
 {
-    Route r{Route::kNone, 1, K, 0, 0};
+    Route r{Route::kNone, 1, K, 0, 0, 0};
     if (M * N == 0 || K == 0) return r;
     if (K == 1) { r.kind = Route::kOuter; return r; }
     // matrix-vector products: `rows` reads the matrix row by row (k contiguous), `cols` column-wise
@@ -1027,22 +1058,36 @@ Route sgemm_route(int transA, int transB, size_t M, size_t N, size_t K, bool pan
         r.cuts = ceil_div(slabs_total, r.depth);
         return r;
     }
+    // How many steps may be added before a sum is rounded and put aside (a pass).  The bf16 instruction rounds down below its
+    // guard bits, so a long sum drifts: 16384 products of non-negative values came out 1.2e-6 too small, 4096 by 2e-7.  And
+    // no result is to be further off than with the fp32 instruction, for which the 32 x 32-tile kernel cuts a reduction in
+    // eight and the tile engine cut it until there were two 128 x 128 tiles for each CU.  At equal lengths the error is 0.5
+    // (A dense) to 0.7 (half of A zero, where the fp32 instruction rounds half as often) of the fp32 instruction's with the
+    // small products in accumulators of their own, 0.7 to 1.15 with one accumulator: sums of twice and of half the length.
+    // 469 x 5446 x 173, half of A zero, error against float64: fp32 8.7e-8, uncut 1.2e-7, so 8.3e-8 (25, 18 and 19 us);
+    // 3818 x 1623 x 2673: 4.6e-7, 5.3e-7, 3.8e-7 (382, 199 and 234 us).
+    const size_t tiles128 = ceil_div(M, (size_t)128) * ceil_div(N, (size_t)128);
+    size_t finest = small ? (size_t)kSmallWaves : ceil_div((size_t)2 * num_cus(), tiles128);
+    if (!small && finest > slabs_total / 4) finest = slabs_total / 4 ? slabs_total / 4 : 1;
+    if (finest > 32) finest = 32;
     r.kind = Route::kRows;
     double best = 0;
     for (const RowsShape &t : kRowsShapes) {
         const size_t tiles = ceil_div(M, t.bm) * ceil_div(N, t.bn);
         const bool big = t.bm * t.bn == 256 * 256;
-        if (big && K < 1024) continue;   // one accumulator per value: two halves of the reduction have to be long
-        // a sum of more terms than this is cut (the matrix unit rounds down by little: 16384 products of non-negative
-        // values came out 1.2e-6 too small, 4096 by 2e-7, where rounding to nearest is 1.0e-6 and 5e-7 off)
-        const size_t longest = 4096 / BK;
-        size_t least = big && slabs_total <= 2 * longest ? 1 : ceil_div(slabs_total, longest);
-        if (least > 32) least = 32;
-        for (size_t splits = least; splits <= 32 && (splits == least || splits * 4 <= slabs_total); splits++) {
+        if (big && K < 1024) continue;   // one accumulator per value: its passes have to be long
+        size_t longest = (big ? slabs_total : 4 * slabs_total) / (2 * finest);
+        if (longest > 4096 / BK) longest = 4096 / BK;
+        if (longest < 1) longest = 1;
+        for (size_t splits = 1; splits <= 32 && (splits == 1 || splits * 4 <= slabs_total); splits++) {
             const size_t depth = ceil_div(slabs_total, splits), cuts = ceil_div(slabs_total, depth);
-            if (cuts != splits && splits != least) continue;
-            const double us = (double)ceil_div(tiles * cuts, (size_t)num_cus()) * (depth * t.slab_us + 4) +
-                              (double)M * N * 4 / 5e6 * (cuts > 1 ? 2 * cuts + 1 : big ? 3 : 1) + (cuts > 1 ? 5 : 0);
+            if (cuts != splits) continue;
+            if (cuts > finest && cuts * M * N > M * K + K * N) break;   // more space than the operands take
+            const size_t passes = ceil_div(depth, longest), pass = ceil_div(depth, passes);
+            const double copy_us = (double)M * N * 4 / 5e6;
+            const double pass_us = t.bm * t.bn == 128 * 128 ? 0.5 : 3 + t.bm * t.bn * 8 / 1e5;   // (the second through C)
+            const double us = (double)ceil_div(tiles * cuts, (size_t)num_cus()) * (depth * t.slab_us + 4 + (passes - 1) * pass_us) +
+                              copy_us * cuts + (cuts > 1 ? (cuts + 1) * copy_us + 5 : 0);
             if (best == 0 || us < best) {
                 best = us;
                 r.kind = big ? Route::kRowsBig : Route::kRows;
@@ -1050,10 +1095,11 @@ Route sgemm_route(int transA, int transB, size_t M, size_t N, size_t K, bool pan
                 r.bn = t.bn;
                 r.depth = depth;
                 r.cuts = cuts;
+                r.pass = pass;
             }
         }
     }
-    if (small && small_us < best) r = Route{Route::kSmall, 1, K, 0, 0};
+    if (small && small_us < best) r = Route{Route::kSmall, 1, K, 0, 0, 0};
     return r;
 }
 
@@ -1152,6 +1198,7 @@ int sgemm_epilogue(int transA, int transB, size_t M, size_t N, size_t K, const f
     const int tiles = g.mtiles * g.ntiles;
     const int splits = (int)route.cuts;
     g.slabs_per_split = (int)route.depth;
+    g.slabs_per_pass = (int)route.pass;
     g.splits = splits;
     float *partial = nullptr;
     if (splits > 1) {
@@ -1243,7 +1290,7 @@ int dopt_hip_sgemm_batch(int n, const int *transA, const int *transB, const size
     for (int i = 0; i < n; i++) {
         if (M[i] * N[i] == 0) continue;
         const bool plain = K[i] > 0 && A[i] && B[i] && C[i] && M[i] < ((size_t)1 << 30) && N[i] < ((size_t)1 << 30) && K[i] < ((size_t)1 << 30);
-        const Route r = plain ? sgemm_route(transA[i], transB[i], M[i], N[i], K[i]) : Route{Route::kNone, 1, 0, 0, 0};
+        const Route r = plain ? sgemm_route(transA[i], transB[i], M[i], N[i], K[i]) : Route{Route::kNone, 1, 0, 0, 0, 0};
         if (r.kind == Route::kGemvColsShort && gemvs.size() < (size_t)kGroupJobs) {
             const size_t R = M[i] == 1 ? N[i] : M[i];
             GemvJob q{};
@@ -1338,7 +1385,7 @@ uint64_t dopt_hip_sgemm_order(int transA, int transB, size_t M, size_t N, size_t
 {
     if (!dopt::ensure_init()) return 0;   // the cut of a reduction follows the device's size
     const dopt::Route r = dopt::sgemm_route(transA, transB, M, N, K);
-    return (uint64_t)r.kind | (uint64_t)r.cuts << 8 | (uint64_t)r.depth << 24;
+    return (uint64_t)r.kind | (uint64_t)r.cuts << 8 | (uint64_t)r.depth << 24 | (uint64_t)r.pass << 52;
 }
 
 int dopt_hip_sgemm_t(int transA, int transB, size_t M, size_t N, size_t K, const float *A, const float *B, float *C)

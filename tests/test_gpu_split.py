@@ -39,6 +39,52 @@ def test_large_products(shape, flags):
         assert np.all(np.abs(got[rows, cols] - want) <= walk(K) * mag), (positive, np.max(np.abs(got[rows, cols] - want) / mag))
 
 
+def fp32_sum(a, b, cuts):
+    """a b, the reduction in `cuts` equal parts, each added term by term and rounded to fp32 after each, then the parts."""
+    K = a.shape[1]
+    depth = -(-K // cuts)
+    pad = np.zeros((a.shape[0], depth * cuts - K))
+    pa = np.hstack([a.astype(np.float64), pad]).reshape(a.shape[0], cuts, depth)
+    pb = np.vstack([b.astype(np.float64), np.zeros((depth * cuts - K, b.shape[1]))]).reshape(cuts, depth, b.shape[1])
+    acc = np.zeros((cuts, a.shape[0], b.shape[1]), np.float32)
+    for k in range(depth):
+        acc = (acc + pa[:, :, k].T[:, :, None] * pb[:, k][:, None, :]).astype(np.float32)
+    total = acc[0]
+    for c in range(1, cuts):
+        total = total + acc[c]
+    return total
+
+
+# (M, N, K, cuts of the fp32 kernels): small outputs, which had eight; larger ones with three, two and none;
+# a reduction too long for the cuts there may be, of non-negative terms
+@pytest.mark.parametrize("shape", [(469, 5446, 173, 8), (2837, 897, 106, 8), (395, 5955, 588, 3), (1066, 2834, 79, 8), (3818, 1623, 2673, 2),
+                                   (3000, 3000, 1400, 1), (3000, 3000, 200, 1), (300, 300, 500000, 32)])
+def test_large_products_are_not_further_off_than_in_fp32(shape):
+    M, N, K, cuts = shape
+    r = rng(M + K)
+    a, b = np.maximum(r.standard_normal((M, K), np.float32), 0), r.standard_normal((K, N), np.float32)
+    if K > 100000:
+        b = np.abs(b)
+    side = 16 if K > 100000 else 48
+    rows, cols = r.choice(M, side, replace=False), r.choice(N, side, replace=False)
+    got = ops.matmul(T(a), T(b)).numpy()[np.ix_(rows, cols)]
+    a, b = a[rows], b[:, cols]
+    want, fp32 = a.astype(np.float64) @ b.astype(np.float64), fp32_sum(a, b, cuts)
+    assert fp32.dtype == np.float32
+    # (four standard deviations of a root mean square over side^2 values)
+    assert np.linalg.norm(got - want) <= np.linalg.norm(fp32 - want) * (1 + 4 / np.sqrt(2 * side * side))
+
+
+@pytest.mark.parametrize("shape", [(16384, 16384, 16384), (8192, 8192, 32768), (4096, 6000, 65536), (16384, 8192, 8208)])
+def test_long_reductions_take_no_more_space_than_their_operands(shape):
+    """A cut needs a copy of the output for each part: 4.3 GB for the first shape in four."""
+    M, N, K = shape
+    for ta in (0, 1):
+        for tb in (0, 1):
+            cuts = capi.load().dopt_hip_sgemm_order(ta, tb, M, N, K) >> 8 & 0xffff
+            assert cuts == 1 or cuts * M * N <= M * K + K * N
+
+
 def test_parts_below_the_bf16_rounding_count():
     """Operands that differ in their last bits only: a product of the leading bf16 parts alone would be the same for both."""
     M, N, K = 300, 2048, 2048
