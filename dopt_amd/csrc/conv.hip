@@ -47,7 +47,7 @@ struct GatherConv {
     int padH, padW, strideH, strideW;
     int CinPad, Mp, ncols;
     int mtiles, ntiles, slabs_total, slabs_per_split, splits;
-    size_t out_elems, in_bytes, wp_bytes;
+    size_t out_elems, in_bytes;
     // where output pixel (oh, ow) of this problem lands: row oh * out_sy + out_oy, column ow * out_sx +
     // out_ox of a plane of out_plane elements and out_OW columns (the whole tensor, or every
     // stride-th pixel of it when a strided backward-data pass is run class by class)
@@ -84,7 +84,6 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
     const int wm = w / T::WN, wn = w % T::WN;
 
     const __amdgpu_buffer_rsrc_t rin = make_rsrc(p.in, p.in_bytes);
-    const __amdgpu_buffer_rsrc_t rwp = make_rsrc(p.wp, p.wp_bytes);
 
     // A: this thread's float4 slots of the [BK][BM] filter tile; byte offset relative to the slab's first row
     unsigned a_voff[NA];
@@ -116,9 +115,10 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
     float breg[NB];
 
     auto load = [&]() {
-        const unsigned a_soff = (unsigned)(kk0 * p.Mp) * 4u;
+        // (the packed filter may be larger than a buffer resource reaches: a resource per slab)
+        const __amdgpu_buffer_rsrc_t rwp = make_rsrc(p.wp + (size_t)kk0 * p.Mp, (size_t)BK * p.Mp * sizeof(float));
 #pragma unroll
-        for (int i = 0; i < NA; i++) areg[i] = buffer_load_f32x4(rwp, a_voff[i], a_soff);
+        for (int i = 0; i < NA; i++) areg[i] = buffer_load_f32x4(rwp, a_voff[i], 0);
         int ih, iw, bad = pix_oob;
         if (kMode == 0) {
             ih = oh * p.strideH - p.padH + (p.R - 1 - tr);
@@ -590,7 +590,6 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
     const int OHW = p.OH * p.OW;
     const int chan_stride = p.IH * p.IW;
     const __amdgpu_buffer_rsrc_t rin = make_rsrc(p.in, p.in_bytes);
-    const __amdgpu_buffer_rsrc_t rwp = make_rsrc(p.wp, p.wp_bytes);
 
     // ---- the patch: a thread owns ONE position and loads `nslots` of the chunk's channels of it, so its sixteen
     // addresses are one per-lane offset plus a wavefront-uniform channel offset (sixteen separate offsets and LDS
@@ -670,11 +669,13 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
     const unsigned part_bytes = (unsigned)p.Mp * CH * 2u, slab_bytes = 3u * part_bytes;
     const unsigned fa_voff = (unsigned)((m0 + wk * 32 + l32) * CH + kh * 8) * 2u;
     v4u fa_ring[4][3];
-    auto fa_load = [&](auto slot_tag, int slab) {
+    // (the packed filter may be larger than a buffer resource reaches: a resource per chunk)
+    auto fa_rsrc = [&](int chunk) { return make_rsrc((const char *)p.wp + (size_t)chunk * 16 * slab_bytes, (size_t)16 * slab_bytes); };
+    auto fa_load = [&](auto slot_tag, __amdgpu_buffer_rsrc_t rwp, int xi) {
         constexpr int slot = decltype(slot_tag)::value;
 #pragma unroll
         for (int q = 0; q < 3; q++)
-            fa_ring[slot][q] = __builtin_bit_cast(v4u, buffer_load_f32x4(rwp, fa_voff, (unsigned)slab * slab_bytes + q * part_bytes));
+            fa_ring[slot][q] = __builtin_bit_cast(v4u, buffer_load_f32x4(rwp, fa_voff, (unsigned)xi * slab_bytes + q * part_bytes));
     };
     const int b_frag = xb * VX + kh * (4 * TT) + l32 * 4;   // position xb, this lane's tile and channels
     v4u fb_next[3];
@@ -698,9 +699,9 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
 #pragma unroll
         for (int i = 0; i < NPMAX; i++)
             second[i] = i < nslots && nch > 1 ? buffer_load_f32(rin, p_voff, (unsigned)(((cb + 1) * CH + cbase + i) * chan_stride) * 4u) : 0.0f;
-        fa_load(StepTag<0>{}, cb * 16 + xb);
-        fa_load(StepTag<1>{}, cb * 16 + xb + 1);
-        fa_load(StepTag<2>{}, cb * 16 + xb + 2);
+        fa_load(StepTag<0>{}, fa_rsrc(cb), xb);
+        fa_load(StepTag<1>{}, fa_rsrc(cb), xb + 1);
+        fa_load(StepTag<2>{}, fa_rsrc(cb), xb + 2);
 #pragma unroll
         for (int g = 0; g < NPMAX / 4; g++) patch_store(g, raw0);
 #pragma unroll
@@ -709,9 +710,9 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
                 *(float4 *)((char *)(raw0 + raw_floats) + p_lds + g * 16) =
                     make_float4(second[4 * g], second[4 * g + 1], second[4 * g + 2], second[4 * g + 3]);
     } else {
-        fa_load(StepTag<0>{}, cb * 16 + xb);
-        fa_load(StepTag<1>{}, cb * 16 + xb + 1);
-        fa_load(StepTag<2>{}, cb * 16 + xb + 2);
+        fa_load(StepTag<0>{}, fa_rsrc(cb), xb);
+        fa_load(StepTag<1>{}, fa_rsrc(cb), xb + 1);
+        fa_load(StepTag<2>{}, fa_rsrc(cb), xb + 2);
 #pragma unroll
         for (int g = 0; g < NPMAX / 4; g++) patch_store(g, raw0);
     }
@@ -734,7 +735,7 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
         float *const raww = raw0 + (DB ? (it & 1) * raw_floats : 0);
         const int ahead = DB ? 2 : 1;
         const bool more = it + 1 < nch, fetch = it + ahead < nch;
-        const int chunk_next = more ? chunk + 1 : chunk;   // (after the last chunk: loaded, not used)
+        const __amdgpu_buffer_rsrc_t rw_now = fa_rsrc(chunk), rw_next = fa_rsrc(more ? chunk + 1 : chunk);   // (after the last chunk: loaded, not used)
         static_for<0, 8>([&](auto xtag) {
             constexpr int xl = decltype(xtag)::value;
             const v4u fb[3] = {fb_next[0], fb_next[1], fb_next[2]};
@@ -745,7 +746,7 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
                 // side work of this step, pinned to it: left to itself the scheduler sinks every load to its first use
                 if constexpr (ks == 0 && xl % TH == 0) {
                     // the filter fragments three positions ahead (into the slot of the position before this one)
-                    fa_load(StepTag<(xp + 3) % 4>{}, (xp + 3 < XP ? chunk * 16 : chunk_next * 16 - XP) + xb + xp + 3);
+                    fa_load(StepTag<(xp + 3) % 4>{}, xp + 3 < XP ? rw_now : rw_next, xb + (xp + 3) % XP);
                 }
                 if constexpr (ks == 1 && xl < 7) fb_load(Vc, xl + 1);   // this lane's tile at the next position
                 // the patch `ahead` chunks on: loads during positions 0..3, LDS stores during 4..7
@@ -1962,6 +1963,9 @@ PatchSetup patch_setup_as(const dopt_hip_conv_desc *d, size_t P, size_t Q, bool 
     pc.out_elems = (size_t)pc.ncols * pc.Mout;
     u.tiles = pc.mtiles * pc.ntiles;
     u.wp_elems = (size_t)pc.chunks_total * (wino ? 16 * 24 : 9 * 16) * pc.Mp;   // (Winograd: three 16-bit parts a value)
+    // the direct kernel's offsets into its packed filter reach 2 GiB (few rows, padded to a tile, of very many channels);
+    // the others' start anew with every chunk
+    if (!wino && u.wp_elems * sizeof(float) > 0x7fffffffu) return u;
     u.ok = true;
     return u;
 }
@@ -2507,6 +2511,8 @@ int gather_launch(GatherConv g, int mode, int K, int C, const float *in, const f
     splits = (g.slabs_total + g.slabs_per_split - 1) / g.slabs_per_split;  // no empty split
     g.splits = splits;
 
+    if ((size_t)BK * g.Mp * sizeof(float) > 0x7fffffffu)
+        return fail(DOPT_HIP_ERR_UNSUPPORTED, "convolution: more than 2^25 output channels are not supported");
     const size_t wp_elems = (size_t)taps * g.CinPad * g.Mp;
     const size_t wp_bytes = (wp_elems * sizeof(float) + 255) / 256 * 256;
     const size_t part_bytes = splits > 1 ? (size_t)splits * g.out_elems * sizeof(float) : 0;
@@ -2533,7 +2539,6 @@ int gather_launch(GatherConv g, int mode, int K, int C, const float *in, const f
     g.in = in;
     g.wp = wp;
     g.in_bytes = (size_t)g.N * g.Cin * g.IH * g.IW * sizeof(float);
-    g.wp_bytes = wp_elems * sizeof(float);
     g.out = splits > 1 ? partial : out;
     dim3 grid(xcd_grid((unsigned)(tiles * splits)));
 #define DOPT_GATHER(TILE)                                                                                      \
@@ -2644,6 +2649,8 @@ int run_bwd_strided(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float
                 std::swap(jobs[j], jobs[j - 1]);
         const int K = (int)d->K, C = (int)d->C;
         const int KPad = round_up(K, BK), Mp = round_up(C, 4);
+        if ((size_t)BK * Mp * sizeof(float) > 0x7fffffffu)
+            return fail(DOPT_HIP_ERR_UNSUPPORTED, "convolution: more than 2^25 output channels are not supported");
         size_t wp_off[kGatherJobs + 1] = {0};
         for (int j = 0; j < njobs; j++) {
             const size_t elems = (size_t)jobs[j].ch.taps * jobs[j].cw.taps * KPad * Mp;
@@ -2686,7 +2693,6 @@ int run_bwd_strided(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float
             g.wp = subs.f[j].wp;
             g.out = dx;
             g.in_bytes = (size_t)g.N * g.Cin * g.IH * g.IW * sizeof(float);
-            g.wp_bytes = (size_t)g.R * g.S * KPad * Mp * sizeof(float);
             gg.per[j] = ((unsigned)(g.mtiles * g.ntiles) + 7u) / 8u;
             blocks += 8u * gg.per[j];
             tiles_all += (unsigned)(g.mtiles * g.ntiles);

@@ -363,3 +363,58 @@ def test_general_convolution_operands_that_are_not_finite():
         assert np.array_equal(np.isposinf(got), (infs > 0) & ~(nans > 0))
         fine = np.isfinite(got)
         assert np.all(np.abs(got[fine] - want[fine]) <= walk(2500) * want[fine])   # (every term is positive)
+
+
+# ---- packed filters beyond 2 GiB
+
+def cheap(r, *shape):
+    """Values of mean zero that are made faster than normal ones."""
+    out = r.random(shape, np.float32)
+    out -= np.float32(0.5)
+    return out
+
+
+def test_winograd_filter_of_more_than_2_gib():
+    N, C, K = 2, 5120, 5120   # 2.5 GB in three 16-bit parts
+    r = rng(1)
+    d = capi.ConvDesc(N, C, 4, 4, K, 3, 3, 1, 1, 1, 1)
+    assert capi.load().dopt_hip_conv_packed_bytes(d, 0) == capi.load().dopt_hip_conv_packed_bytes(d, 1) == 96 * C * K > 2 ** 31
+    x, dy, w = cheap(r, N, C, 4, 4), cheap(r, N, K, 4, 4), cheap(r, K, C, 3, 3)
+    dw = T(w)
+    rows = np.array([0, 77, 2600, K - 1])
+    got = ops.convolution(T(x), dw, (1, 1), (1, 1)).numpy()[:, rows]
+    want, mag = winograd(x, w[rows]), winograd(x, w[rows], True)
+    assert np.all(np.abs(got - want) <= winograd_share(C) * mag)
+    got = ops.conv_bwd_data(T(dy), dw, x.shape, (1, 1), (1, 1)).numpy()[:, rows]
+    flipped = np.ascontiguousarray(w[:, rows].transpose(1, 0, 2, 3)[:, :, ::-1, ::-1])
+    want, mag = winograd(dy, flipped), winograd(dy, flipped, True)
+    assert np.all(np.abs(got - want) <= winograd_share(K) * mag)
+
+
+def test_general_filter_of_more_than_2_gib():
+    M = 1400000   # 25 taps x 16 (padded) x M values: 2.2 GB
+    r = rng(2)
+    w, x = cheap(r, M, 1, 5, 5), cheap(r, 1, 1, 6, 6)
+    y = ops.convolution(T(x), T(w), (2, 2), (1, 1)).numpy()
+    for rows in (np.arange(100), np.arange(M - 100, M)):
+        want, mag = general(x, w[rows], 2, 1), general(x, w[rows], 2, 1, np.abs)
+        assert np.all(np.abs(y[:, rows] - want) <= walk(25) * mag)
+    del y
+    w = w.reshape(1, M, 5, 5)
+    dx = ops.conv_bwd_data(T(x), T(w), (1, M, 6, 6), (2, 2), (1, 1)).numpy()
+    for rows in (np.arange(100), np.arange(M - 100, M)):
+        part, zero = np.ascontiguousarray(w[:, rows]), np.zeros((1, 100, 6, 6), np.float32)
+        want, mag = general_gradients(zero, part, x, 2, 1)[0], general_gradients(zero, part, x, 2, 1, np.abs)[0]
+        assert np.all(np.abs(dx[:, rows] - want) <= walk(25) * mag)
+
+
+def test_direct_filter_of_more_than_2_gib():
+    """One output channel, padded to a tile of 64 rows: the direct kernel's copy would be 2.2 GB, its last channels out of reach."""
+    C = 940000
+    r = rng(3)
+    assert capi.load().dopt_hip_conv_packed_bytes(capi.ConvDesc(1, C, 16, 16, 1, 3, 3, 1, 1, 1, 1), 0) == 0
+    w, x = cheap(r, 1, C, 3, 3), np.zeros((1, C, 16, 16), np.float32)
+    x[:, -64:] = cheap(r, 1, 64, 16, 16)
+    y = ops.convolution(T(x), T(w), (1, 1), (1, 1)).numpy()
+    want, mag = general(x[:, -64:], w[:, -64:], 1, 1), general(x[:, -64:], w[:, -64:], 1, 1, np.abs)
+    assert np.all(np.abs(y - want) <= walk(9 * 64) * mag)
