@@ -152,16 +152,17 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
             }
         }
     };
-    auto store = [&](int buf) {
+    auto store = [&](int buf, float up) {
 #pragma unroll
-        for (int i = 0; i < NA; i++) *(float4 *)&As[buf][a_lds[i]] = areg[i];
+        for (int i = 0; i < NA; i++) *(float4 *)&As[buf][a_lds[i]] = make_float4(areg[i].x * up, areg[i].y * up, areg[i].z * up, areg[i].w * up);
 #pragma unroll
-        for (int i = 0; i < NB; i++) Bs[buf][(brow0 + RSTEP * i) * LDB + bcol] = breg[i];
+        for (int i = 0; i < NB; i++) Bs[buf][(brow0 + RSTEP * i) * LDB + bcol] = breg[i] * up;
     };
 
     v16f acc[T::MI][T::NI];
     auto run = [&](auto exact_tag) {
         constexpr bool exact = decltype(exact_tag)::value != 0;
+        constexpr float up = exact ? 1.0f : kSplitUp;
         kk0 = slab_begin * BK;
         tap = kk0 / p.CinPad;
         ci0 = kk0 - tap * p.CinPad;
@@ -175,14 +176,14 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
             else mma_slab_split<LDA, LDB>(As[buf], Bs[buf], wm * (BM / T::WM), wn * (BN / T::WN), acc, low, lane);
         };
         load();
-        store(0);
+        store(0, up);
         __syncthreads();
         int cur = 0;
         // steady state: no data-dependent branches inside
         for (int slab = slab_begin; slab < slab_end - 1; ++slab) {
             load();
             slab_products(cur);
-            store(cur ^ 1);
+            store(cur ^ 1, up);
             __syncthreads();
             cur ^= 1;
         }
@@ -502,6 +503,10 @@ __global__ __launch_bounds__(T::THREADS, T::THREADS / 256) void conv_patch_k(Pat
 // floats of the exchange area: 128 rows: four wavefront pairs x 64 values per lane; 64 rows: eight wavefronts x 64 values
 constexpr int wino_xchg(int bm) { return (bm == 128 ? 4 : 8) * 64 * 64; }
 
+// A packed filter value whose parts are no numbers (2^103 and more, infinities, NaNs) has this NaN for its h part and its bits as
+// they are in the other two.
+constexpr unsigned short kWinoRaw = 0x7fff;
+
 // WK x TH: WK groups of 32 rows, TH groups of 32 tiles: 4 x 1 (128 rows x 32 tiles = 128 pixels) for layers with whole
 // 128-row tiles, 2 x 2 (64 rows x 64 tiles = 256 pixels) for 64-row layers.
 // The four outputs of one tile and row over channels c0 .. c1 - 1, in fp32 without matrix instructions: for the tiles whose
@@ -534,7 +539,9 @@ __device__ __forceinline__ void wino_fp32(const PatchConv &p, int n, int m, int 
             for (int j = 0; j < 4; j++) {
                 const size_t at = (((size_t)(c / 16) * 16 + i * 4 + j) * 3 * p.Mp + m) * 16 + c % 16, part = (size_t)p.Mp * 16;
                 auto val = [&](size_t a) { return __builtin_bit_cast(float, (unsigned)wp[a] << 16); };
-                M[i * 4 + j] += (val(at) + val(at + part) + val(at + 2 * part)) * v[j];
+                const float u = wp[at] == kWinoRaw ? __builtin_bit_cast(float, (unsigned)wp[at + part] << 16 | wp[at + 2 * part])
+                                                   : (val(at) + val(at + part) + val(at + 2 * part)) * (1.0f / kSplitUp);
+                M[i * 4 + j] += u * v[j];
             }
         }
         float z[4][2];
@@ -617,7 +624,8 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
     };
     auto patch_store = [&](int g, float *rawb) {   // channels 4 g .. 4 g + 3 of the position: one 128-bit store
         if (4 * g < nslots)
-            *(float4 *)((char *)rawb + p_lds + g * 16) = make_float4(preg[4 * g], preg[4 * g + 1], preg[4 * g + 2], preg[4 * g + 3]);
+            *(float4 *)((char *)rawb + p_lds + g * 16) =
+                make_float4(preg[4 * g] * kSplitUp, preg[4 * g + 1] * kSplitUp, preg[4 * g + 2] * kSplitUp, preg[4 * g + 3] * kSplitUp);
     };
 
     // ---- the transform items of this thread (TH of them): row ti of Bt d B for tile tau, channels 4 cq .. 4 cq + 3
@@ -698,7 +706,9 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
         float second[NPMAX];
 #pragma unroll
         for (int i = 0; i < NPMAX; i++)
-            second[i] = i < nslots && nch > 1 ? buffer_load_f32(rin, p_voff, (unsigned)(((cb + 1) * CH + cbase + i) * chan_stride) * 4u) : 0.0f;
+            // (no branch: what is done to the values would move into it, and each load be waited for there)
+            second[i] = buffer_load_f32(rin, i < nslots && nch > 1 ? p_voff : kOobOffset,
+                                        (unsigned)(((nch > 1 ? cb + 1 : cb) * CH + cbase + (i < nslots ? i : 0)) * chan_stride) * 4u);
         fa_load(StepTag<0>{}, fa_rsrc(cb), xb);
         fa_load(StepTag<1>{}, fa_rsrc(cb), xb + 1);
         fa_load(StepTag<2>{}, fa_rsrc(cb), xb + 2);
@@ -708,7 +718,8 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
         for (int g = 0; g < NPMAX / 4; g++)
             if (4 * g < nslots)
                 *(float4 *)((char *)(raw0 + raw_floats) + p_lds + g * 16) =
-                    make_float4(second[4 * g], second[4 * g + 1], second[4 * g + 2], second[4 * g + 3]);
+                    make_float4(second[4 * g] * kSplitUp, second[4 * g + 1] * kSplitUp, second[4 * g + 2] * kSplitUp,
+                                second[4 * g + 3] * kSplitUp);
     } else {
         fa_load(StepTag<0>{}, fa_rsrc(cb), xb);
         fa_load(StepTag<1>{}, fa_rsrc(cb), xb + 1);
@@ -836,7 +847,8 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
 #pragma unroll
         for (int v = 0; v < 16; v++) {
             const float4 other = *(const float4 *)(xchg + ((wk * 16 + v) * 64 + lane) * 4);
-            float y[4] = {part[v][0] + other.x, part[v][1] + other.y, part[v][2] + other.z, part[v][3] + other.w};
+            float y[4] = {(part[v][0] + other.x) * kSplitDown, (part[v][1] + other.y) * kSplitDown, (part[v][2] + other.z) * kSplitDown,
+                          (part[v][3] + other.w) * kSplitDown};
             store(0, v, y, 1u << v);
         }
         while (again) {
@@ -859,7 +871,8 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
             float2 z[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) z[i] = *(const float2 *)(xchg + (((wk * 4 + i) * 32 + tv) * 64 + lane) * 2);
-            float y[4] = {(z[0].x + z[1].x) + z[2].x, (z[0].y + z[1].y) + z[2].y, z[1].x + (-z[2].x - z[3].x), z[1].y + (-z[2].y - z[3].y)};
+            float y[4] = {((z[0].x + z[1].x) + z[2].x) * kSplitDown, ((z[0].y + z[1].y) + z[2].y) * kSplitDown,
+                          (z[1].x + (-z[2].x - z[3].x)) * kSplitDown, (z[1].y + (-z[2].y - z[3].y)) * kSplitDown};
             store(tv >> 4, tv & 15, y, 1u << e);
         }
         while (again) {
@@ -870,7 +883,7 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
     }
 }
 
-// The transformed filter of the Winograd kernel, split into its bf16 parts q = h, m, l:
+// The transformed filter of the Winograd kernel, multiplied by kSplitUp and split into its bf16 parts q = h, m, l:
 // U[(((chunk*16 + xi)*3 + q)*Mp + m)*16 + j] = (G g Gt)[xi] for row m and channel chunk*16 + j, where g is the filter as the kernel applies it to the patch: g[r][s] multiplies patch offset
 // (r, s), i.e. the stored taps read backwards when the operation is a true convolution (`flip`).  Staged like
 // pack_tile (16 rows of one chunk); G = [1 0 0; .5 .5 .5; .5 -.5 .5; 0 0 1].
@@ -929,7 +942,20 @@ __device__ __forceinline__ void wino_pack_tile(int M, int Cred, int Mp, size_t s
             for (int e = 0; e < 4; e += 2) {
                 const float other = __shfl_xor(odd ? u[e] : u[e + 1], 1);
                 unsigned ph, pm, pl;
-                split_pair_any(odd ? other : u[e], odd ? u[e + 1] : other, ph, pm, pl);
+                const float a = odd ? other : u[e], b = odd ? u[e + 1] : other;
+                split_pair(a * kSplitUp, b * kSplitUp, ph, pm, pl);
+                const unsigned bits[2] = {__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b)};
+                constexpr unsigned kTop = 0x73000000u;   // 2^103
+                if (__any(max(bits[0] & 0x7fffffffu, bits[1] & 0x7fffffffu) >= kTop)) {
+#pragma unroll
+                    for (int v = 0; v < 2; v++) {
+                        const unsigned shift = 16 * v, keep = 0xffff0000u >> shift;
+                        if ((bits[v] & 0x7fffffffu) < kTop) continue;
+                        ph = (ph & keep) | (unsigned)kWinoRaw << shift;
+                        pm = (pm & keep) | bits[v] >> 16 << shift;
+                        pl = (pl & keep) | (bits[v] & 0xffffu) << shift;
+                    }
+                }
                 unsigned *dst = (unsigned *)wp + ((((size_t)chunk * 16 + r * 4 + e + odd) * 3) * Mp + m0 + ml) * 8 + (j >> 1);
                 dst[0] = ph;
                 dst[part] = pm;
@@ -1133,16 +1159,17 @@ __global__ __launch_bounds__(T::THREADS, T::THREADS / 128) void conv_wgrad_k(Fil
             }
         }
     };
-    auto store = [&](int buf) {
+    auto store = [&](int buf, float up) {
 #pragma unroll
-        for (int i = 0; i < NA; i++) As[buf][kl * LDA + r0 + 16 * i] = areg[i];
+        for (int i = 0; i < NA; i++) As[buf][kl * LDA + r0 + 16 * i] = areg[i] * up;
 #pragma unroll
-        for (int i = 0; i < NB; i++) Bs[buf][kl * LDB + r0 + 16 * i] = breg[i];
+        for (int i = 0; i < NB; i++) Bs[buf][kl * LDB + r0 + 16 * i] = breg[i] * up;
     };
 
     v16f acc[T::MI][T::NI];
     auto run = [&](auto exact_tag) {
         constexpr bool exact = decltype(exact_tag)::value != 0;
+        constexpr float up = exact ? 1.0f : kSplitUp;
         v16f low[T::MI][T::NI];
         zero_acc(acc);
         zero_acc(low);
@@ -1151,13 +1178,13 @@ __global__ __launch_bounds__(T::THREADS, T::THREADS / 128) void conv_wgrad_k(Fil
             else mma_slab_split<LDA, LDB>(As[buf], Bs[buf], wm * (BM / T::WM), wn * (BN / T::WN), acc, low, lane);
         };
         load(slab_begin);
-        store(0);
+        store(0, up);
         __syncthreads();
         int cur = 0;
         for (int slab = slab_begin; slab < slab_end - 1; ++slab) {
             load(slab + 1);
             slab_products(cur);
-            store(cur ^ 1);
+            store(cur ^ 1, up);
             __syncthreads();
             cur ^= 1;
         }
@@ -1334,7 +1361,7 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
     constexpr bool kLow = WM * WC == 4;
     constexpr int kPasses = kLow ? 1 : 2;
     int from = cb, to = kPasses == 1 ? ce : (cb + ce + 1) / 2;
-    float sign = 1.0f;
+    float up = kSplitUp;   // its sign alternates
 
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int kh = lane >> 5, l32 = lane & 31;
@@ -1413,25 +1440,28 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
             n_img += p.imgs;
         }
     };
-    auto stash = [&](int buf) {
+    auto stash = [&](int buf, auto exact_tag) {
+        constexpr bool exact = decltype(exact_tag)::value != 0;
         float *A = A0 + buf * (BM * APITCH), *B = B0 + buf * bsize;
 #pragma unroll
         for (int i = 0; i < NAQ; i++) {
             const float4 v = areg[i];
+            const float by = kLow ? kSplitUp : up;
             *(float4 *)(AROWS * (i + 1) <= BM || a_row + AROWS * i < BM ? A + a_lds + AROWS * i * APITCH : dummy) =
-                kLow ? v : make_float4(v.x * sign, v.y * sign, v.z * sign, v.w * sign);
+                exact ? v : make_float4(v.x * by, v.y * by, v.z * by, v.w * by);
         }
 #pragma unroll
         for (int i = 0; i < NBQ; i++) {
+            const float4 v = exact ? breg[i] : make_float4(breg[i].x * kSplitUp, breg[i].y * kSplitUp, breg[i].z * kSplitUp, breg[i].w * kSplitUp);
             if (kGeo != 2) {
-                *(float4 *)(b_lds[i] >= 0 ? B + (b_lds[i] & ~3) : dummy) = breg[i];
+                *(float4 *)(b_lds[i] >= 0 ? B + (b_lds[i] & ~3) : dummy) = v;
             } else {
                 float *q = b_lds[i] >= 0 ? B + b_lds[i] : dummy;  // rows 1 and 2 of the cell block, columns 1..2
                 const int down = b_lds[i] >= 0 ? 4 : 0;
-                q[0] = breg[i].x;
-                q[1] = breg[i].y;
-                q[down] = breg[i].z;
-                q[down + 1] = breg[i].w;
+                q[0] = v.x;
+                q[1] = v.y;
+                q[down] = v.z;
+                q[down + 1] = v.w;
             }
         }
     };
@@ -1586,7 +1616,7 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[t][v] = low[kLow ? t : 0][v] = 0.0f;
         fetch();
-        stash(0);
+        stash(0, exact_tag);
         __syncthreads();
         int cur = 0;
         for (int chunk = from; chunk < to; ++chunk) {
@@ -1599,15 +1629,17 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
                     split_frag(read_frag(cur, s));
                     products_split();
                 }
-                if constexpr (s == 3) stash(cur ^ 1);
+                if constexpr (s == 3) stash(cur ^ 1, exact_tag);
             });
             __syncthreads();
             cur ^= 1;
         }
+        if (exact) return;
 #pragma unroll
         for (int t = 0; t < 3; t++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) acc[t][v] = kLow ? acc[t][v] + low[kLow ? t : 0][v] : acc[t][v] * sign;
+            for (int v = 0; v < 16; v++)
+                acc[t][v] = kLow ? (acc[t][v] + low[kLow ? t : 0][v]) * kSplitDown : acc[t][v] * (up * (kSplitDown / kSplitUp));
     };
     for (int pass = 0;; pass++) {
         // halo cells are not written by the loop: clear both patch buffers before it
@@ -1660,7 +1692,7 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
         if (pass + 1 == kPasses || to == ce) break;
         from = to;
         to = ce;
-        sign = -sign;
+        up = -up;
     }
 }
 

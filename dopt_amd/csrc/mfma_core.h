@@ -90,9 +90,13 @@ __device__ inline void zero_acc(v16f (&acc)[MI][NI])
 //
 // v_mfma_f32_32x32x16_bf16 multiplies 16 reduction steps in half the cycles that v_mfma_f32_32x32x2_f32 takes for two
 // (measured on this chip: 1770 against 124 TFLOP/s), so six of them per sixteen steps still run at 2.4 times the fp32
-// rate.  An fp32 value is the exact sum of three bf16 values: h = bf16(a), m = bf16(a - h), l = bf16(a - h - m), each
-// rounded to nearest; 24 significand bits are three times 8, so nothing is left over.  Of the nine products of two such
-// sums the six largest are taken; the three left out (m.l, l.m, l.l) are together at most 2^-24 of |a.b|, what ONE
+// rate.  An fp32 value of ordinary size is the exact sum of three bf16 values: h = bf16(a), m = bf16(a - h), l = bf16(a - h - m),
+// each rounded to nearest; 24 significand bits are three times 8, so nothing is left over (Henry, Tang and Heinecke,
+// "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations", 2019).  bf16 has the exponents
+// of fp32 but not its small steps: the parts of a value below 2^-110 would fall under the smallest bf16 number.  So operands
+// are multiplied by 2^24 (kSplitUp) on their way to the split, which makes every nonzero part of every fp32 value a normal
+// bf16 number, and sums by 2^-48 (kSplitDown); both are exact, and no other bit changes.
+// Of the nine products of two such sums the six largest are taken; the three left out (m.l, l.m, l.l) are together at most 2^-24 of |a.b|, what ONE
 // fp32 rounding of the product may be off by, and 2^-28 of it on average.  Every product of two bf16 values is exact
 // in fp32, and all sums are fp32.  Against float64 the result is not less accurate than the fp32 instruction's, because
 // it is rounded less often; with the large products and the small rest in accumulators of their own, where registers
@@ -100,9 +104,9 @@ __device__ inline void zero_acc(v16f (&acc)[MI][NI])
 // 4096 terms: 5.0e-8 / 1.3e-7 / 3.8e-7, the fp32 instruction 1.4e-7 / 4.0e-7 / 1.2e-6, one accumulator for all six
 // 1.1e-7 / 3.4e-7 / 9.8e-7).
 //
-// The split of an infinity or of a value above the bf16 range holds NaNs.  Kernels that use it look at their finished
-// accumulators and form a tile that is not finite a second time with the fp32 instruction, so infinities and NaNs of
-// the operands give what they always gave.
+// The split of an infinity, or of a value that is one after the multiplication (2^104 and more), holds NaNs, and a sum of 2^80
+// and more overflows.  Kernels that use it look at their finished accumulators and form a tile that is not finite a second time
+// with the fp32 instruction, so such operands and sums give what they always gave.
 //
 // The instruction adds the eight products of a lane half's eight slots in one go, whatever their order (measured: no
 // permutation of the eight changes a bit).  So the six products of FOUR reduction steps fill the eight slots of three
@@ -114,6 +118,8 @@ typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
+constexpr float kSplitUp = 0x1p24f, kSplitDown = 0x1p-48f;
+
 // Two values' h, m and l parts, each pair packed into one word (first value in the low half): 11 VALU instructions.
 __device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsigned &m, unsigned &l)
 {
@@ -123,25 +129,6 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsign
     m = __builtin_bit_cast(unsigned, __builtin_convertvector(r, v2bf));
     const v2f s = {r.x - __builtin_bit_cast(float, m << 16), r.y - __builtin_bit_cast(float, m & 0xffff0000u)};
     l = __builtin_bit_cast(unsigned, __builtin_convertvector(s, v2bf));
-}
-
-// The same for operands that are laid out once and read again as h + m + l: exact for every value, infinities and values
-// that round to one included (an infinity is its own h part, the other two are zero).
-__device__ __forceinline__ void split_pair_any(float a, float b, unsigned &h, unsigned &m, unsigned &l)
-{
-    split_pair(a, b, h, m, l);
-    auto fix = [](float v, unsigned hv, unsigned shift, unsigned &h, unsigned &m, unsigned &l) {
-        if ((hv & 0x7f80u) != 0x7f80u || v != v) return;   // a finite h; a NaN stays one
-        const unsigned keep = 0xffff0000u >> shift, bits = __builtin_bit_cast(unsigned, v);
-        unsigned h2, m2, l2;
-        const float head = __builtin_bit_cast(float, bits & 0xffff0000u);
-        split_pair(__builtin_isinf(v) ? 0.0f : v - head, 0.0f, h2, m2, l2);   // 16 bits: two parts
-        h = (h & keep) | ((bits >> 16) << shift);
-        m = (m & keep) | (h2 & 0xffffu) << shift;
-        l = (l & keep) | (m2 & 0xffffu) << shift;
-    };
-    fix(a, h & 0xffffu, 0, h, m, l);
-    fix(b, h >> 16, 16, h, m, l);
 }
 
 // Four reduction steps of one row: their h parts in hm.x, .y, their m parts in hm.z, .w, their l parts in l.
@@ -158,6 +145,7 @@ __device__ __forceinline__ v16f mfma_bf16(v4u a, v4u b, v16f c)
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
 }
 
+// The finished sums of mma_slab_split.
 template <int MI, int NI>
 __device__ __forceinline__ void add_acc(v16f (&acc)[MI][NI], const v16f (&low)[MI][NI])
 {
@@ -166,7 +154,7 @@ __device__ __forceinline__ void add_acc(v16f (&acc)[MI][NI], const v16f (&low)[M
 #pragma unroll
         for (int j = 0; j < NI; j++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] += low[i][j][v];
+            for (int v = 0; v < 16; v++) acc[i][j][v] = (acc[i][j][v] + low[i][j][v]) * kSplitDown;
 }
 
 // Whether this lane's accumulators hold an infinity or a NaN: x * 0 is 0 for finite x only.
@@ -184,7 +172,7 @@ __device__ __forceinline__ int not_finite(const v16f (&acc)[MI][NI])
 }
 
 // mma_slab on the bf16 matrix instruction: from the same k-major fp32 slab of sixteen steps a lane reads its eight steps of
-// each fragment and splits them in registers.  h.h goes to acc, the five small products to low.
+// each fragment (multiplied by kSplitUp) and splits them in registers.  h.h goes to acc, the five small products to low.
 template <int LDA, int LDB, int MI, int NI>
 __device__ __forceinline__ void mma_slab_split(const float *As, const float *Bs, int a_off, int b_off, v16f (&acc)[MI][NI],
                                                v16f (&low)[MI][NI], int lane)

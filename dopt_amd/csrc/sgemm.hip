@@ -240,7 +240,7 @@ struct Stage3 {
         if (kCut) v = make_float4(v.x, left > 1 ? v.y : 0.0f, left > 2 ? v.z : 0.0f, left > 3 ? v.w : 0.0f);
         v4u a;
         uint2 b;
-        split_quad(v, a, b);
+        split_quad(make_float4(v.x * kSplitUp, v.y * kSplitUp, v.z * kSplitUp, v.w * kSplitUp), a, b);
         *(v4u *)(Xs + (hm ^ row_swap(e)) + e * kRowBytes) = a;
         *(uint2 *)(Xs + (l ^ row_swap(e)) + e * kRowBytes) = b;
     }
@@ -446,7 +446,10 @@ __global__ __launch_bounds__(kRowsThreads, 2) void sgemm_rows_k(Gemm p)
 #pragma unroll
             for (int j = 0; j < NI; j++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) top = __fmaf_rn(acc[i][j][v], 0.0f, top);
+                for (int v = 0; v < 16; v++) {
+                    top = __fmaf_rn(acc[i][j][v], 0.0f, top);
+                    acc[i][j][v] *= kSplitDown;
+                }
         put(from != k_begin);
     }
     if (!__any(top != 0.0f)) return;

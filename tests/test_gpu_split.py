@@ -365,6 +365,65 @@ def test_general_convolution_operands_that_are_not_finite():
         assert np.all(np.abs(got[fine] - want[fine]) <= walk(2500) * want[fine])   # (every term is positive)
 
 
+# ---- operands and sums at the ends of the range of fp32, where bf16 parts would be lost or overflow
+
+def scaled_pairs(p, q, least_q=-149):
+    """The two operands of a product at very different scales: (p, q) with finite products between 1e-12 and 1e+35."""
+    for ep, eq in ((-112, 100), (-120, 100), (-130, 100), (-140, 100), (60, 40), (-20, 110), (-80, 120)):
+        for swap in (False, True):
+            if swap and ep < least_q:
+                continue
+            with np.errstate(under="ignore"):
+                yield (ep, eq, swap), np.ldexp(p, eq if swap else ep), np.ldexp(q, ep if swap else eq)
+
+
+def check_norm(got, want, terms, what):
+    """Against float64 in the 2-norm.  Not further off than one rounding per term, plus the roundings of the values themselves (four
+    of a result: the Winograd transforms, the parts' sum and the last)."""
+    got = got.astype(np.float64)
+    assert np.all(np.isfinite(got)), what
+    assert np.linalg.norm(got - want) <= (rounded_once_per_term(terms) + 4 * 2.0 ** -24) * np.linalg.norm(want), what
+
+
+def test_products_of_operands_at_the_ends_of_the_range():
+    r = rng(17)
+    for M, N, K in ((300, 2048, 700), (2304, 2304, 1100)):   # the smaller tiles, 256 x 256
+        p, q = r.standard_normal((M, K), np.float32), r.standard_normal((K, N), np.float32)
+        for what, a, b in scaled_pairs(p, q):
+            got = ops.matmul(T(a), T(b)).numpy()[:256:5]
+            check_norm(got, a[:256:5].astype(np.float64) @ b.astype(np.float64), K, (M, what))
+
+
+@pytest.mark.parametrize("shape", [(2, 64, 16, 16, 64), (2, 64, 8, 8, 128)])
+def test_winograd_operands_at_the_ends_of_the_range(shape):
+    N, C, H, W, K = shape
+    r = rng(K)
+    # (the filter's transform is in fp32: of subnormal values it is rounded to steps of 2^-149, with every instruction)
+    for what, x, w in scaled_pairs(r.standard_normal((N, C, H, W), np.float32), r.standard_normal((K, C, 3, 3), np.float32), -122):
+        check_norm(ops.convolution(T(x), T(w), (1, 1), (1, 1)).numpy(), winograd(x, w), 9 * C, what)
+
+
+# 64-, 128- and 160-row tiles
+@pytest.mark.parametrize("shape", [(4, 33, 16, 16, 65), (8, 32, 4, 4, 128), (4, 32, 32, 32, 160)])
+def test_filter_gradient_operands_at_the_ends_of_the_range(shape):
+    N, C, H, W, K = shape
+    r = rng(K)
+    for what, x, dy in scaled_pairs(r.standard_normal((N, C, H, W), np.float32), r.standard_normal((N, K, H, W), np.float32)):
+        check_norm(ops.conv_bwd_filter(T(dy), T(x), (K, C, 3, 3), (1, 1), (1, 1)).numpy(), filter_gradient(dy, x), N * H * W, what)
+
+
+def test_general_convolution_operands_at_the_ends_of_the_range():
+    r = rng(23)
+    x, w = r.standard_normal((2, 48, 13, 11), np.float32), r.standard_normal((100, 48, 5, 5), np.float32)
+    dy, pad = r.standard_normal((2, 100, 7, 6), np.float32), (2, 2)
+    for what, p, q in scaled_pairs(x, w):
+        check_norm(ops.convolution(T(p), T(q), pad, pad).numpy(), general(p, q, 2, 2), 48 * 25, what)
+    for what, p, q in scaled_pairs(dy, w):
+        check_norm(ops.conv_bwd_data(T(p), T(q), x.shape, pad, pad).numpy(), general_gradients(x, q, p, 2, 2)[0], 100 * 9, what)
+    for what, p, q in scaled_pairs(x, dy):
+        check_norm(ops.conv_bwd_filter(T(q), T(p), w.shape, pad, pad).numpy(), general_gradients(p, w, q, 2, 2)[1], 84, what)
+
+
 # ---- packed filters beyond 2 GiB
 
 def cheap(r, *shape):
