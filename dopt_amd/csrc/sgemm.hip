@@ -453,7 +453,8 @@ __global__ __launch_bounds__(kRowsThreads, 2) void sgemm_rows_k(Gemm p)
         put(from != k_begin);
     }
     if (!__any(top != 0.0f)) return;
-    {   // an operand or a sum that is not finite: this wavefront's part in fp32 instructions
+    {   // an operand or a sum that is not finite: this wavefront's part in fp32 instructions, of which those values are taken that
+        // are not finite in C (the others have the bits that they have beside finite ones, whatever tile they lie in)
         const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.A, (size_t)p.M * p.K * sizeof(float));
         const __amdgpu_buffer_rsrc_t rb = make_rsrc(p.B, (size_t)p.K * p.N * sizeof(float));
         zero_acc(acc);
@@ -477,7 +478,16 @@ __global__ __launch_bounds__(kRowsThreads, 2) void sgemm_rows_k(Gemm p)
                 for (int j = 0; j < NI; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
         }
     }
-    put(false);
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+        for (int j = 0; j < NI; j++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const int m = m0 + wm * 32 * MI + i * 32 + acc_row(v, lane);
+                float *const c = outp + (size_t)(i * 32 + 4 * kh + 8 * (v >> 2) + (v & 3)) * p.N + 32 * j;
+                if (m < p.M && n0 + brow + 32 * j < p.N && *c * 0.0f != 0.0f) *c = acc[i][j][v];
+            }
 }
 
 // Small outputs (a dense layer at batch 128: 128 x 512 values from a 512-deep reduction).  The tile

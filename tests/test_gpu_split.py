@@ -114,6 +114,34 @@ def test_operands_that_are_not_finite():
     assert np.all(np.abs(got[fine] - want[fine]) <= walk(K) * mag[fine])
 
 
+@pytest.mark.parametrize("shape", [(2304, 2304, 1100), (2049, 2560, 1030), (300, 2048, 700)])
+def test_finite_values_keep_their_bits_beside_others(shape):
+    """An infinity or a NaN changes its own row or column: what dopt_hip_sgemm_order promises, equal bits whichever way the operands
+    are stored and for the transposed product, holds for the values beside it, and they are what they are without it."""
+    M, N, K = shape
+    r = rng(M)
+    a, b = r.standard_normal((M, K), np.float32), r.standard_normal((K, N), np.float32)
+    plain = ops.matmul(T(a), T(b)).numpy()
+    a[3, 5], a[200, 7], b[9, 1000], a[10, 0] = np.inf, np.nan, -np.inf, 1e36
+    lib = capi.load()
+    order = lib.dopt_hip_sgemm_order(0, 0, M, N, K)
+    got = ops.matmul(T(a), T(b)).numpy()
+    rows, cols = np.delete(np.arange(M), [3, 10, 200]), np.delete(np.arange(N), 1000)
+    assert np.array_equal(got[np.ix_(rows, cols)], plain[np.ix_(rows, cols)])
+    at, bt = np.ascontiguousarray(a.T), np.ascontiguousarray(b.T)
+    seen = 0
+    for ta, tb in ((False, True), (True, False), (True, True)):
+        if lib.dopt_hip_sgemm_order(int(ta), int(tb), M, N, K) == order:
+            again = ops.matmul_t(T(at if ta else a), T(bt if tb else b), ta, tb).numpy()
+            assert np.array_equal(again, got, equal_nan=True), (ta, tb)
+            seen += 1
+        if lib.dopt_hip_sgemm_order(int(ta), int(tb), N, M, K) == order:
+            again = ops.matmul_t(T(b if ta else bt), T(a if tb else at), ta, tb).numpy().T
+            assert np.array_equal(again, got, equal_nan=True), ("transposed", ta, tb)
+            seen += 1
+    assert seen >= 3
+
+
 # ---- the Winograd convolution kernel
 
 BT = np.array([[1, 0, -1, 0], [0, 1, 1, 0], [0, -1, 1, 0], [0, 1, 0, -1]], np.float64)
