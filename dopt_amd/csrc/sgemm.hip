@@ -1089,7 +1089,7 @@ Route sgemm_route(int transA, int transB, size_t M, size_t N, size_t K, bool pan
         const size_t tiles = ceil_div(M, t.bm) * ceil_div(N, t.bn);
         const bool big = t.bm * t.bn == 256 * 256;
         if (big && K < 1024) continue;   // one accumulator per value: its passes have to be long
-        size_t longest = (big ? slabs_total : 4 * slabs_total) / (2 * finest);
+        size_t longest = big ? ceil_div(slabs_total, 2 * finest) : 2 * slabs_total / finest;
         if (longest > 4096 / BK) longest = 4096 / BK;
         if (longest < 1) longest = 1;
         for (size_t splits = 1; splits <= 32 && (splits == 1 || splits * 4 <= slabs_total); splits++) {

@@ -19,6 +19,21 @@ def walk(terms):
     return (6 * np.sqrt(0.75 * terms) + 1) * 2.0 ** -24
 
 
+def rounded_once_per_term(terms):
+    """Relative error (2-norm) of a sum of `terms` products of zero mean that is rounded after each: a rounding is uniform over
+    one unit in the last place, 0.43 * 2^-24 of the partial sum in the root mean square (the leading digits of the partial sum
+    spread evenly over their logarithm), and the partial sums grow with the root of their length: 0.43 / sqrt(2) * sqrt(terms)."""
+    return 0.30 * 2.0 ** -24 * np.sqrt(terms)
+
+
+def check_norm(got, want, terms, what):
+    """Against float64 in the 2-norm.  Not further off than one rounding per term, plus the roundings of the values themselves (four
+    of a result: the Winograd transforms, the parts' sum and the last)."""
+    got = got.astype(np.float64)
+    assert np.all(np.isfinite(got)), what
+    assert np.linalg.norm(got - want) <= (rounded_once_per_term(terms) + 4 * 2.0 ** -24) * np.linalg.norm(want), what
+
+
 # one tile of every size and one value more; reductions of one slab, a part of one, several cuts; no multiple of four
 @pytest.mark.parametrize("shape", [(65, 2048, 2100), (256, 256, 20000), (257, 1024, 4099), (130, 3001, 1030), (2049, 2047, 17),
                                    (1030, 4100, 1025), (4096, 4096, 64), (1537, 1538, 2050)])
@@ -142,6 +157,61 @@ def test_finite_values_keep_their_bits_beside_others(shape):
     assert seen >= 3
 
 
+ROUTES = {9: "rows", 10: "rows 256 x 256"}   # the kernels of the first byte of dopt_hip_sgemm_order that split their operands
+
+
+def route(ta, tb, M, N, K):
+    """(kernel, cuts, slabs of 16 steps per cut, slabs per pass)"""
+    o = capi.load().dopt_hip_sgemm_order(int(ta), int(tb), M, N, K)
+    return ROUTES.get(o & 0xff), o >> 8 & 0xffff, o >> 24 & 0xfffffff, o >> 52
+
+
+# every tile, with the sum in one pass, in passes that wait in registers (128 x 128) and in C (the others), and cut: whole tiles and
+# ragged ones, reductions of an odd number of slabs and no multiple of four
+@pytest.mark.parametrize("shape,kernel,cuts,passes", [
+    ((3072, 2816, 1104), "rows 256 x 256", 1, 2), ((3001, 2879, 1101), "rows 256 x 256", 1, 2), ((4096, 2304, 5000), "rows 256 x 256", 3, 1),
+    ((1500, 1500, 2050), "rows", None, None), ((3000, 3000, 200), "rows", 1, 1), ((4100, 2050, 190), "rows", 1, 1),
+    ((469, 5446, 173), "rows", 1, 6), ((130, 6001, 1030), "rows", None, None), ((2837, 897, 106), "rows", 1, 7),
+    ((257, 300, 40000), "rows", None, None)])
+def test_every_part_counts(shape, kernel, cuts, passes):
+    """In the 2-norm: leaving out the l parts of one operand would be 2e-6 off, one of the six products of parts more than that."""
+    M, N, K = shape
+    r = rng(M + N)
+    a, b = r.standard_normal((M, K), np.float32), r.standard_normal((K, N), np.float32)
+    rows, cols = np.append(r.choice(M, 61, replace=False), [0, M - 1, M - 2]), np.append(r.choice(N, 61, replace=False), [0, N - 1, N - 2])
+    want = a[rows].astype(np.float64) @ b[:, cols].astype(np.float64)
+    at, bt = np.ascontiguousarray(a.T), np.ascontiguousarray(b.T)
+    seen = {}
+    for ta in (False, True):
+        for tb in (False, True):
+            name, c, depth, length = route(ta, tb, M, N, K)
+            assert name == kernel and cuts in (None, c) and passes in (None, -(-depth // length)), (name, c, depth, length)
+            got = ops.matmul_t(T(at if ta else a), T(bt if tb else b), ta, tb).numpy()
+            assert np.linalg.norm(got[np.ix_(rows, cols)] - want) <= min(rounded_once_per_term(K), 1e-6) * np.linalg.norm(want)
+            first = seen.setdefault((c, depth, length), got)
+            assert np.array_equal(got, first), (ta, tb)
+
+
+@pytest.mark.parametrize("shape", [(3072, 2816, 1104), (3001, 2879, 1101)])
+def test_not_finite_in_either_pass(shape):
+    M, N, K = shape
+    assert route(0, 0, M, N, K)[:2] == ("rows 256 x 256", 1)
+    r = rng(M)
+    a, b = r.standard_normal((M, K), np.float32), r.standard_normal((K, N), np.float32)
+    a[3, 5], a[700, K - 5], b[9, 1000], b[K - 3, 77], a[10, 0], a[11, K - 1] = np.inf, np.nan, -np.inf, np.nan, 1e36, 3.4e38
+    got = ops.matmul(T(a), T(b)).numpy()
+    rows, cols = np.append(r.choice(M, 50, replace=False), [3, 700, 10, 11]), np.append(r.choice(N, 50, replace=False), [1000, 77])
+    with np.errstate(all="ignore"):
+        want = a[rows].astype(np.float64) @ b[:, cols].astype(np.float64)
+        mag = np.abs(a[rows]).astype(np.float64) @ np.abs(b[:, cols]).astype(np.float64)
+    got = got[np.ix_(rows, cols)]
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf])
+    fine = np.isfinite(want) & (mag < 3.4e38)
+    assert np.all(np.isfinite(got[fine])) and np.all(np.abs(got[fine] - want[fine]) <= walk(K) * mag[fine])
+
+
 # ---- the Winograd convolution kernel
 
 BT = np.array([[1, 0, -1, 0], [0, 1, 1, 0], [0, -1, 1, 0], [0, 1, 0, -1]], np.float64)
@@ -196,6 +266,7 @@ def test_winograd(shape, backward):
         got = ops.convolution(T(x), T(w), (1, 1), (1, 1)).numpy()
     want, mag = winograd(x, w), winograd(x, w, True)
     assert np.all(np.abs(got - want) <= winograd_share(C) * mag), np.max(np.abs(got - want) / mag)
+    check_norm(got, want, 9 * C, shape)   # (every part counts: without the l parts of one operand it would be 2e-6 off)
 
 
 @pytest.mark.parametrize("shape", [(2, 64, 16, 16, 64), (2, 64, 16, 16, 128)])
@@ -277,6 +348,7 @@ def test_filter_gradient(shape):
     got = ops.conv_bwd_filter(T(dy), T(x), (K, C, 3, 3), (1, 1), (1, 1)).numpy()
     want, mag = filter_gradient(dy, x), filter_gradient(dy, x, np.abs)
     assert np.all(np.abs(got - want) <= walk(N * H * W) * mag), np.max(np.abs(got - want) / mag)
+    check_norm(got, want, N * H * W / 2, shape)
 
 
 @pytest.mark.parametrize("shape", [(4, 64, 16, 16, 128), (8, 64, 4, 4, 64), (3, 32, 32, 32, 160)])
@@ -291,13 +363,6 @@ def test_filter_gradient_operands_that_are_not_finite(shape):
     fine = mag < 3e38
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
     assert np.all(np.abs(got[fine] - want[fine]) <= walk(N * H * W) * mag[fine])
-
-
-def rounded_once_per_term(terms):
-    """Relative error (2-norm) of a sum of `terms` products of zero mean that is rounded after each: a rounding is uniform over
-    one unit in the last place, 0.43 * 2^-24 of the partial sum in the root mean square (the leading digits of the partial sum
-    spread evenly over their logarithm), and the partial sums grow with the root of their length: 0.43 / sqrt(2) * sqrt(terms)."""
-    return 0.30 * 2.0 ** -24 * np.sqrt(terms)
 
 
 # an odd number of filter values, so one block adds all the pixels: 64-, 128- and 160-row tiles, every pixel geometry
@@ -359,11 +424,14 @@ def test_general_convolution(shape):
     dy = r.standard_normal(got.shape).astype(np.float32)
     want, mag = general(x, w, pad, stride), general(x, w, pad, stride, np.abs)
     assert np.all(np.abs(got - want) <= walk(C * R * R) * mag)
+    check_norm(got, want, C * R * R / 2, shape)
     wants, mags = general_gradients(x, w, dy, pad, stride), general_gradients(x, w, dy, pad, stride, np.abs)
     dx = ops.conv_bwd_data(T(dy), T(w), x.shape, (pad, pad), (stride, stride)).numpy()
     dw = ops.conv_bwd_filter(T(dy), T(x), w.shape, (pad, pad), (stride, stride)).numpy()
     assert np.all(np.abs(dx - wants[0]) <= walk(K * R * R) * mags[0])
     assert np.all(np.abs(dw - wants[1]) <= walk(dy[:, 0].size) * mags[1])
+    check_norm(dx, wants[0], K * R * R / stride ** 2, shape)
+    check_norm(dw, wants[1], dy[:, 0].size / 2, shape)
 
 
 def test_general_convolution_operands_that_are_not_finite():
@@ -403,14 +471,6 @@ def scaled_pairs(p, q, least_q=-149):
                 continue
             with np.errstate(under="ignore"):
                 yield (ep, eq, swap), np.ldexp(p, eq if swap else ep), np.ldexp(q, ep if swap else eq)
-
-
-def check_norm(got, want, terms, what):
-    """Against float64 in the 2-norm.  Not further off than one rounding per term, plus the roundings of the values themselves (four
-    of a result: the Winograd transforms, the parts' sum and the last)."""
-    got = got.astype(np.float64)
-    assert np.all(np.isfinite(got)), what
-    assert np.linalg.norm(got - want) <= (rounded_once_per_term(terms) + 4 * 2.0 ** -24) * np.linalg.norm(want), what
 
 
 def test_products_of_operands_at_the_ends_of_the_range():
