@@ -326,19 +326,20 @@ def main():
         # 128-row tiles that runs the forward pass of layers 3-10 and the backward-data pass of layers 4-10 (15 launches
         # per step; the 64-row instantiation of layers 2-3 is not part of this figure).  Timed by events
         # recorded around each launch inside the library, on the stream the kernel runs on (its steps may also run a
-        # split sum, which is not part of this figure).  `achieved` counts the layer's FLOPs by the direct algorithm,
-        # 2*N*K*C*R*S*P*Q - the algorithmic work of the operation, as the other figures of this file do; the kernel
-        # executes 16/36 of them, each as six bf16 products of the operands' three parts (`executed_*`, against the bf16
-        # peak), so `frac` above 1 is the algorithm's gain over the fp32 instruction, not a measurement error.
+        # split sum, which is not part of this figure).  `achieved` counts what the matrix instructions execute, against the
+        # peak of the instruction that they are: 16/36 of the direct algorithm's products, each as six bf16 products of the
+        # operands' three parts.  `direct_*` counts the layer's FLOPs by the direct algorithm, 2*N*K*C*R*S*P*Q - the work of
+        # the operation, as the other figures of this file do - against the peak of the fp32 instruction, which a kernel of
+        # that algorithm and instruction could not pass.
         launches = pl.value / nsteps if nsteps else 0
         tflops = pfl.value / (pus.value * 1e-6) / 1e12 if pus.value else 0.0
         result["roofline"] = {
             "kernel": "conv_wino_k<16, 4, 1>: Winograd F(2x2, 3x3) convolution on the transformed filter, 128 rows x 32 tiles of 2x2 "
                       "pixels per workgroup: forward of layers 3-10 and backward-data of layers 4-10 of the 13; the other "
                       "convolution kernels are listed under `kernels`",
-            "bound": "mfma", "achieved": round(tflops, 2), "peak": MFMA_FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
-            "frac": round(tflops / MFMA_FP32_PEAK_TFLOPS, 4),
-            "executed_achieved": round(tflops * 96.0 / 36.0, 2), "executed_frac": round(tflops * 96.0 / 36.0 / MFMA_BF16_PEAK_TFLOPS, 4),
+            "bound": "mfma", "achieved": round(tflops * 96.0 / 36.0, 2), "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
+            "frac": round(tflops * 96.0 / 36.0 / MFMA_BF16_PEAK_TFLOPS, 4),
+            "direct_achieved": round(tflops, 2), "direct_frac_of_fp32_peak": round(tflops / MFMA_FP32_PEAK_TFLOPS, 4),
             "traffic": profile_line("traffic_bytes_per_launch conv_wino_k"),
             "traffic_source": "profiles/conv_kernels_vgg16_b128_hbm_traffic.txt (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE of "
                               "the same %d launches per step; taken from that file, not measured in this run)" % round(launches),
@@ -376,14 +377,14 @@ def main():
         result["kernels"] = {
             "forward convolutions of layers 3-10 (conv_wino_k; FLOPs by the direct algorithm's count)": {
                 "achieved_TFLOPs": round(flops / (us * 1e-6) / 1e12, 2) if us else None,
-                "frac_of_mfma_peak": round(flops / (us * 1e-6) / 1e12 / MFMA_FP32_PEAK_TFLOPS, 4) if us else None,
+                "frac_of_fp32_mfma_peak": round(flops / (us * 1e-6) / 1e12 / MFMA_FP32_PEAK_TFLOPS, 4) if us else None,
                 "launches_per_step": n128, "avg_launch_us": round(us / n128, 2) if n128 else None,
                 "algorithmic_bytes_per_launch": int(bytes_alg / n128) if n128 else None,
                 "traffic": profile_line("traffic_bytes_per_launch conv_wino_k")},
             "all 38 convolution operations of the step incl. filter packing and split sums (2x2-image layers counted at the "
             "conventional 9-tap FLOPs although their dense route executes 4/9 of them)": {
                 "achieved_TFLOPs": round((2 * fwd + bwd_data) / (allconv_us * 1e-6) / 1e12, 2),
-                "frac_of_mfma_peak": round((2 * fwd + bwd_data) / (allconv_us * 1e-6) / 1e12 / MFMA_FP32_PEAK_TFLOPS, 4),
+                "frac_of_fp32_mfma_peak": round((2 * fwd + bwd_data) / (allconv_us * 1e-6) / 1e12 / MFMA_FP32_PEAK_TFLOPS, 4),
                 "us_per_step": round(allconv_us, 1)},
             "device_us_per_step_by_op": {k: round(v[0], 1) for k, v in sorted(per_op.items(), key=lambda kv: -kv[1][0])},
             "device_us_per_step_total": round(sum(v[0] for v in per_op.values()), 1),

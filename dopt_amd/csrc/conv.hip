@@ -1,4 +1,5 @@
-// Convolution forward, backward-data and backward-filter as implicit GEMMs on fp32 MFMA.
+// Convolution forward, backward-data and backward-filter as implicit GEMMs on matrix instructions: most kernels on the bf16 one
+// with each fp32 value split into three parts (mfma_core.h), the direct 3 x 3 and the 2 x 2-image kernels on the fp32 one.
 // Replaces cudnnConvolutionForward / BackwardData / BackwardFilter as called at
 // cuda/source/dopt/cuda/nnet/cudnn7.d:154, :199, :244.  The reference configures cuDNN with
 // CUDNN_CONVOLUTION (cudnn7.d:87), i.e. a TRUE convolution: the filter is flipped,
@@ -57,7 +58,7 @@ struct GatherConv {
 // The products run on the bf16 matrix instruction, operands split as they are read from LDS (mma_slab_split): the loop was
 // bound by the fp32 instruction, 2048 cycles per slab and 64 x 64 wavefront tile, of which the six bf16 products take 768;
 // the splitting, 704 vector cycles, runs beside the other wavefront's.  50 images of 48 x 45 x 39, 100 filters of 5 x 5 at
-// stride 2, forward and both gradients: 379 -> 270 us.  Error against float64 (160 -> 320 channels, stride 2): 2.1e-7 -> 8.5e-8
+// stride 2, forward and both gradients: 379 -> 274 us.  Error against float64 (160 -> 320 channels, stride 2): 2.1e-7 -> 8.5e-8
 // forward, 5.3e-7 -> 1.7e-7 backward-data, 2.2e-7 -> 9.1e-8 filter gradient.
 // kMode: 0 = forward, 1 = backward-data with unit stride (no divisions), 2 = backward-data, any stride.
 // L: the workgroup's item among the problem's (split, tile) pairs, tile fastest.
@@ -2048,8 +2049,9 @@ int patch_splits(int tiles, int chunks, int slots, int BM, int BN, size_t out_el
     return best;
 }
 
-// The same estimate for the general kernels, whose unit is a slab of 16 reduction steps and whose main loops
-// sustain less (k-major LDS tiles, 32-bit fragment reads).
+// The same estimate for the general kernels, whose unit is a slab of 16 reduction steps.  0.33 TFLOP/s per CU is what their loops
+// sustained on the fp32 instruction; on the bf16 one they are about 1.4 times as fast, and with 0.5 here nearly every layer is
+// cut the same (Wide-ResNet-28-10 step 21.87 against 21.89 ms, the 5 x 5 layers above 271.4 against 271.5 us).
 int gather_splits(int tiles, int slabs, int slots, int BM, int BN, size_t out_elems, int cap = 64)
 {
     const double cu_tflops = 0.33;
@@ -2909,6 +2911,8 @@ WgradSetup wgrad_patch_setup(const dopt_hip_conv_desc *d, const float *dw)
     int splits = 1;
     {
         const int max_by_depth = wp.chunks_total / 2 > 0 ? wp.chunks_total / 2 : 1;  // two chunks amortise the set-up
+        // (0.45 TFLOP/s per CU was the fp32 instruction's loop, this one sustains 0.8; with 0.7 here the layers of VGG-16 and
+        // Wide-ResNet-28-10 at batch 128 are cut the same)
         const double t_chunk = 2.0 * BM * BC * 9 * 64 / 0.45e6;
         double best = 0.0;
         for (int sp = 1; sp <= max_by_depth && sp <= 512; sp++) {

@@ -5,7 +5,8 @@
 // broadcast is a product with a ones vector (core/source/dopt/core/ops/basic.d:370-381,
 // core/source/dopt/core/ops/package.d:96-103) and rank-2 row / column sums are products with a
 // ones vector too (core/source/dopt/core/ops/math.d:257-279).  Those degenerate shapes are
-// HBM-bound and get their own kernels here; everything else runs on the fp32 MFMA tile engine.
+// HBM-bound and get their own kernels here; everything else runs on matrix instructions: small outputs on the fp32 one, large
+// ones on the bf16 one with each fp32 value split into three parts (mfma_core.h).
 #include <vector>
 
 #include "common.h"
@@ -899,9 +900,10 @@ unsigned flat_grid(size_t n)
     return (unsigned)(blocks < 1 ? 1 : (blocks > cap ? cap : blocks));
 }
 
-// The LDS-resident kernel wins where its 128 x 128 tiles give every CU one or two blocks and the
-// operands take 128-bit loads (2048 x 2048 x 128: 17 us against 22 us for the 32 x 32 tiles); with
-// fewer tiles CUs idle, with more the tile engine's two resident blocks per CU overlap better.
+// The LDS-resident kernel is taken where its 128 x 128 tiles give every CU one or two blocks and the operands take 128-bit loads.
+// Against what those shapes take without it (an operand off the 16-byte grid): 2048 x 2048 x 64 11 and 18 us, 1024 x 4096 x
+// 100 15 and 21, 2048 x 2048 x 128 17 and 17, 2880 x 2880 x 32 20 and 20; with two blocks on some CUs and 128 steps it is
+// behind, 2816 x 2816 28 and 20, 2048 x 4096 27 and 20.
 bool panel_shape(size_t M, size_t N, size_t K)
 {
     const size_t tiles = ceil_div(M, (size_t)kPanelTile) * ceil_div(N, (size_t)kPanelTile);

@@ -159,7 +159,7 @@ def main():
         if args.json:
             print(json.dumps(res))
             return
-        print("%-28s %10s %10s %8s" % ("matmul [M,K] x [K,N]", "us", "TFLOP/s", "of peak"))
+        print("%-28s %10s %10s %12s" % ("matmul [M,K] x [K,N]", "us", "TFLOP/s", "of fp32 peak"))
         for r in res:
             print("%-28s %10.1f %10.1f %7.1f%%" % ("[%d,%d] x [%d,%d]" % (r["M"], r["K"], r["K"], r["N"]), r["us"], r["TFLOP/s"],
                                                     100 * r["frac_of_157.3"]))

@@ -237,6 +237,9 @@ int dopt_hip_sgemm_t(int transA, int transB, size_t M, size_t N, size_t K, const
    of another job: the order inside the batch is not kept. */
 int dopt_hip_sgemm_batch(int n, const int *transA, const int *transB, const size_t *M, const size_t *N, const size_t *K,
                          const float *const *A, const float *const *B, float *const *C);
+/* Large products and convolutions form their fp32 products from three 16-bit parts of each operand, to at least the accuracy
+   of the fp32 matrix instruction over the whole range of fp32.  Operands of 2^104 (2e31) and sums of 2^80 (1e24) and more,
+   infinities and NaNs take a second pass in fp32: the values are those of fp32, the call takes several times as long. */
 /* Names the order in which dopt_hip_sgemm_t adds the K terms of an output element for these flags and dimensions
    (which kernel runs, and where it cuts the reduction): two calls with equal values give equal bits for equal
    operand values, also when one computes the transpose of the other's product, (A B)^T = B^T A^T with M and N
@@ -288,7 +291,8 @@ int dopt_hip_conv_bwd_data(const dopt_hip_conv_desc *d, const float *dy, const f
    the unpacked entry points).  A packed copy depends on the descriptor, the direction and the
    device, and is valid until the filter changes.  Layers that run the Winograd F(2x2, 3x3) kernel (pad 1, even
    image sides of 4 and more, whole 16-channel chunks and at least 64 reduction channels, rows in whole 128s or
-   in 64s padded by at most a fifth) get the transformed filter G g Gt as their packed copy, 16/9 the size. */
+   in 64s padded by at most a fifth) get the transformed filter G g Gt as their packed copy, each value in three 16-bit
+   parts: 8/3 the size. */
 size_t dopt_hip_conv_packed_bytes(const dopt_hip_conv_desc *d, int bwd_data);
 /* Which layout that packed copy has, or -1 when there is none: two packed copies of the same filter
    under the same descriptor and with equal layout ids are identical, so a caller needs only one.
