@@ -588,6 +588,8 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
     const int cb = split * p.chunks_per_split;
     const int ce = min(cb + p.chunks_per_split, p.chunks_total);
     const int nch = ce - cb;
+    // The bf16 instruction rounds down below its guard bits; partial sums of alternating sign take that out of their total.
+    const float up = split & 1 ? -kSplitUp : kSplitUp, down = split & 1 ? -kSplitDown : kSplitDown;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wavefront-uniform, and known to be: it enters scalar load offsets
@@ -626,7 +628,7 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
     auto patch_store = [&](int g, float *rawb) {   // channels 4 g .. 4 g + 3 of the position: one 128-bit store
         if (4 * g < nslots)
             *(float4 *)((char *)rawb + p_lds + g * 16) =
-                make_float4(preg[4 * g] * kSplitUp, preg[4 * g + 1] * kSplitUp, preg[4 * g + 2] * kSplitUp, preg[4 * g + 3] * kSplitUp);
+                make_float4(preg[4 * g] * up, preg[4 * g + 1] * up, preg[4 * g + 2] * up, preg[4 * g + 3] * up);
     };
 
     // ---- the transform items of this thread (TH of them): row ti of Bt d B for tile tau, channels 4 cq .. 4 cq + 3
@@ -719,8 +721,8 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
         for (int g = 0; g < NPMAX / 4; g++)
             if (4 * g < nslots)
                 *(float4 *)((char *)(raw0 + raw_floats) + p_lds + g * 16) =
-                    make_float4(second[4 * g] * kSplitUp, second[4 * g + 1] * kSplitUp, second[4 * g + 2] * kSplitUp,
-                                second[4 * g + 3] * kSplitUp);
+                    make_float4(second[4 * g] * up, second[4 * g + 1] * up, second[4 * g + 2] * up,
+                                second[4 * g + 3] * up);
     } else {
         fa_load(StepTag<0>{}, fa_rsrc(cb), xb);
         fa_load(StepTag<1>{}, fa_rsrc(cb), xb + 1);
@@ -848,8 +850,8 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
 #pragma unroll
         for (int v = 0; v < 16; v++) {
             const float4 other = *(const float4 *)(xchg + ((wk * 16 + v) * 64 + lane) * 4);
-            float y[4] = {(part[v][0] + other.x) * kSplitDown, (part[v][1] + other.y) * kSplitDown, (part[v][2] + other.z) * kSplitDown,
-                          (part[v][3] + other.w) * kSplitDown};
+            float y[4] = {(part[v][0] + other.x) * down, (part[v][1] + other.y) * down, (part[v][2] + other.z) * down,
+                          (part[v][3] + other.w) * down};
             store(0, v, y, 1u << v);
         }
         while (again) {
@@ -872,8 +874,8 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
             float2 z[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) z[i] = *(const float2 *)(xchg + (((wk * 4 + i) * 32 + tv) * 64 + lane) * 2);
-            float y[4] = {((z[0].x + z[1].x) + z[2].x) * kSplitDown, ((z[0].y + z[1].y) + z[2].y) * kSplitDown,
-                          (z[1].x + (-z[2].x - z[3].x)) * kSplitDown, (z[1].y + (-z[2].y - z[3].y)) * kSplitDown};
+            float y[4] = {((z[0].x + z[1].x) + z[2].x) * down, ((z[0].y + z[1].y) + z[2].y) * down,
+                          (z[1].x + (-z[2].x - z[3].x)) * down, (z[1].y + (-z[2].y - z[3].y)) * down};
             store(tv >> 4, tv & 15, y, 1u << e);
         }
         while (again) {

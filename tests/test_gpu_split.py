@@ -291,8 +291,8 @@ def test_winograd_operands_that_are_not_finite(shape):
     assert np.all(np.isfinite(got[fits]))
 
 
-def winograd_fp32(x, w, halves):
-    """`winograd` in fp32, the channels of each of `halves` added one after the other and rounded after each."""
+def winograd_fp32(x, w, cuts):
+    """`winograd` in fp32, the channels of each of `cuts` parts added one after the other and rounded after each, then the parts."""
     N, C, H, W = x.shape
     g = w[:, :, ::-1, ::-1]
     xp = np.pad(x, ((0, 0), (0, 0), (1, 1), (1, 1)))
@@ -300,7 +300,7 @@ def winograd_fp32(x, w, halves):
     u = sandwich(G.astype(np.float32), g)
     v = sandwich(BT.astype(np.float32), d).transpose(1, 4, 5, 0, 2, 3).reshape(C, 4, 4, -1)
     y = 0.0
-    for part in np.array_split(np.arange(C), halves):
+    for part in np.array_split(np.arange(C), cuts):
         m = np.zeros((w.shape[0], 4, 4, v.shape[-1]), np.float32)
         for c in part:
             m = (m + u[:, c, :, :, None].astype(np.float64) * v[c]).astype(np.float32)
@@ -309,17 +309,19 @@ def winograd_fp32(x, w, halves):
     return y
 
 
-# layers whose tiles fill less than half of the chip
-@pytest.mark.parametrize("shape", [(32, 64, 32, 32, 64), (32, 320, 16, 16, 320), (32, 160, 32, 32, 160)])
-def test_winograd_is_not_further_off_than_fp32_in_two_halves(shape):
-    N, C, H, W, K = shape
+# (images, channels, rows, columns, filters, cuts of the reduction): layers whose tiles fill less than half of the chip, and a few
+# tiles, whose reduction is cut into single chunks
+@pytest.mark.parametrize("shape", [(32, 64, 32, 32, 64, 2), (32, 320, 16, 16, 320, 2), (32, 160, 32, 32, 160, 2), (1, 640, 8, 8, 640, 40),
+                                   (18, 432, 4, 4, 128, 27), (2, 512, 4, 4, 512, 32)])
+def test_winograd_is_not_further_off_than_fp32_with_the_same_cuts(shape):
+    N, C, H, W, K, cuts = shape
     r = rng(C)
     x = np.maximum(r.standard_normal((N, C, H, W)), 0).astype(np.float32)
     w = (r.standard_normal((K, C, 3, 3)) * np.sqrt(2 / (9 * C))).astype(np.float32)
-    rows = np.arange(0, K, K // 8)
+    rows = np.arange(0, K, K // 32 if H < 16 else K // 8)
     got = ops.convolution(T(x), T(w), (1, 1), (1, 1)).numpy()[:4, rows]
     x, w = x[:4], w[rows]
-    want, fp32 = winograd(x, w), winograd_fp32(x, w, 2)
+    want, fp32 = winograd(x, w), winograd_fp32(x, w, cuts)
     assert fp32.dtype == np.float32
     assert np.linalg.norm(got - want) <= np.linalg.norm(fp32 - want)
 
