@@ -382,6 +382,19 @@ def test_filter_gradient_is_not_further_off_than_one_rounding_per_term(shape):
     assert np.linalg.norm(got - want) <= rounded_once_per_term(N * H * W / 2) * np.linalg.norm(want)
 
 
+# 65536 pixels and more in one block, every product non-negative
+@pytest.mark.parametrize("shape", [(128, 33, 32, 32, 65), (16, 17, 64, 64, 255), (64, 17, 32, 32, 159)])
+def test_long_filter_gradient_of_one_sign(shape):
+    """Rounded after each term, the partial sums grow with their length: 0.43 * 2^-24 * sqrt(terms / 3) of the sum."""
+    N, C, H, W, K = shape
+    r = rng(K)
+    x = np.maximum(r.standard_normal((N, C, H, W), np.float32), 0)
+    dy = np.abs(r.standard_normal((N, K, H, W), np.float32))
+    got = ops.conv_bwd_filter(T(dy), T(x), (K, C, 3, 3), (1, 1), (1, 1)).numpy()
+    want = filter_gradient(dy, x)
+    assert np.linalg.norm(got - want) <= 0.25 * 2.0 ** -24 * np.sqrt(N * H * W / 2) * np.linalg.norm(want)
+
+
 # ---- the general kernels: any filter size, stride and padding
 
 def general(x, w, pad, stride, f=lambda v: v):
