@@ -492,8 +492,7 @@ __global__ __launch_bounds__(T::THREADS, T::THREADS / 256) void conv_patch_k(Pat
 // At the end a lane holds M[xi][row][tile] for its positions, complete rows i of the 4x4 grid: it applies A along j in
 // registers (z[i][b]) and the wavefronts that share an output meet in LDS: y[a][b] = (At z)[a][b].  With 128 rows one of
 // a pair adds the other's share of the four outputs; with 64 rows all four leave their z and finish a quarter of the
-// outputs each.  Output, split reductions and bias are those of the direct kernel.  Outputs that are not finite are
-// formed again in fp32 (wino_fp32).
+// outputs each.  Output, split reductions and bias are those of the direct kernel.
 //
 // What bounds it (batch 128 with packing, the fp32 instruction -> this): 640 -> 640 channels on 8 x 8 images, batch 512,
 // 828 -> 627 us; 160 -> 160 on 32 x 32 318 -> 227; 128 -> 128 on 16 x 16, batch 256, 83 -> 66.  A chunk takes 2.9 us per
@@ -510,57 +509,6 @@ constexpr unsigned short kWinoRaw = 0x7fff;
 
 // WK x TH: WK groups of 32 rows, TH groups of 32 tiles: 4 x 1 (128 rows x 32 tiles = 128 pixels) for layers with whole
 // 128-row tiles, 2 x 2 (64 rows x 64 tiles = 256 pixels) for 64-row layers.
-// The four outputs of one tile and row over channels c0 .. c1 - 1, in fp32 without matrix instructions: for the tiles whose
-// operands or results are not finite.  (ih0, iw0): the tile's first input pixel.
-__device__ __forceinline__ void wino_fp32(const PatchConv &p, int n, int m, int ih0, int iw0, int c0, int c1, float (&y)[4])
-{
-    float M[16];
-#pragma unroll
-    for (int x = 0; x < 16; x++) M[x] = 0.0f;
-    const unsigned short *wp = (const unsigned short *)p.wp;
-#pragma unroll 1
-    for (int c = c0; c < c1; c++) {
-        const float *in = p.in + ((size_t)n * p.Cin + c) * p.IH * p.IW;
-        float d[4][4];
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int ih = ih0 + r, iw = iw0 + q;
-                d[r][q] = ih >= 0 && ih < p.IH && iw >= 0 && iw < p.IW ? in[ih * p.IW + iw] : 0.0f;
-            }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            float t[4];
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-                t[q] = i == 0 ? d[0][q] - d[2][q] : i == 1 ? d[1][q] + d[2][q] : i == 2 ? d[2][q] - d[1][q] : d[1][q] - d[3][q];
-            const float v[4] = {t[0] - t[2], t[1] + t[2], t[2] - t[1], t[1] - t[3]};
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const size_t at = (((size_t)(c / 16) * 16 + i * 4 + j) * 3 * p.Mp + m) * 16 + c % 16, part = (size_t)p.Mp * 16;
-                auto val = [&](size_t a) { return __builtin_bit_cast(float, (unsigned)wp[a] << 16); };
-                const float u = wp[at] == kWinoRaw ? __builtin_bit_cast(float, (unsigned)wp[at + part] << 16 | wp[at + 2 * part])
-                                                   : (val(at) + val(at + part) + val(at + 2 * part)) * (1.0f / kSplitUp);
-                M[i * 4 + j] += u * v[j];
-            }
-        }
-        float z[4][2];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            z[i][0] = (M[4 * i] + M[4 * i + 1]) + M[4 * i + 2];
-            z[i][1] = (M[4 * i + 1] - M[4 * i + 2]) - M[4 * i + 3];
-        }
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-            y[b] = (z[0][b] + z[1][b]) + z[2][b];
-            y[2 + b] = (z[1][b] - z[2][b]) - z[3][b];
-        }
-        // a NaN stays one, whatever the channels after it hold: a tile of NaNs costs one channel
-        if (y[0] != y[0] && y[1] != y[1] && y[2] != y[2] && y[3] != y[3]) break;
-    }
-}
-
 template <int NPMAX, int WK, int TH>
 __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
 {
@@ -800,19 +748,18 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
     float *const xchg = lds;          // [wavefront pair][accumulator row][lane][4]: the main loop's LDS is free now
     float *outp = p.out + (size_t)split * p.out_elems;
     const bool add_bias = p.bias != nullptr && p.splits == 1;
-    unsigned again = 0;               // results that are not finite
     // the four outputs of accumulator row v of tiles 32 t ..; y: index 2 a + b
-    auto store = [&](int t, int v, float (&y)[4], unsigned flag) {
+    float scale = down, probe = 0.0f;   // probe: NaN once anything is not finite, x * 0 is 0 for finite x only
+    auto store = [&](int t, int v, const float (&sum)[4]) {
+        float y[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            probe = __builtin_fmaf(sum[q], 0.0f, probe);
+            y[q] = sum[q] * scale;
+        }
         const int tau = t * 32 + l32, img = tau / tpi, tl = tau - img * tpi, r2 = tl / tcn, c2 = tl - r2 * tcn;
         const int n = n_first + img, m = m0 + wk * 32 + acc_row(v, lane);
         if (n >= p.N || m >= p.Mout) return;
-        // (zero times an infinity or a NaN is a NaN)
-        if ((y[0] * 0.0f + y[1] * 0.0f) + (y[2] * 0.0f + y[3] * 0.0f) != 0.0f) {
-            if (flag) {               // the parts of an infinity hold NaNs: formed again in fp32 below
-                again |= flag;
-                return;
-            }
-        }
         if (add_bias) {
             const float bias = p.bias[m];
 #pragma unroll
@@ -822,67 +769,112 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
         *(float2 *)o = make_float2(y[0], y[1]);
         *(float2 *)(o + p.OW) = make_float2(y[2], y[3]);
     };
-    auto store_fp32 = [&](int t, int v) {
-        const int tau = t * 32 + l32, img = tau / tpi, tl = tau - img * tpi, r2 = tl / tcn, c2 = tl - r2 * tcn;
-        float y[4];
-        wino_fp32(p, n_first + img, m0 + wk * 32 + acc_row(v, lane), oh0 + 2 * r2 - p.PT, 2 * c2 - p.PL, cb * CH, ce * CH, y);
-        store(t, v, y, 0);
-    };
-    if constexpr (TH == 1) {
-        float part[16][4];            // per accumulator row v: this wavefront's share of y[a][b], index 2 a + b
+    for (int pass = 0;; pass++) {
+        if constexpr (TH == 1) {
+            float part[16][4];            // per accumulator row v: this wavefront's share of y[a][b], index 2 a + b
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const float za0 = (acc[0][v] + acc[1][v]) + acc[2][v], za1 = (acc[1][v] - acc[2][v]) - acc[3][v];
-            const float zb0 = (acc[4][v] + acc[5][v]) + acc[6][v], zb1 = (acc[5][v] - acc[6][v]) - acc[7][v];
-            if (wi == 0) {            // rows 0, 1: y[0] += z0 + z1, y[1] += z1
-                part[v][0] = za0 + zb0; part[v][1] = za1 + zb1; part[v][2] = zb0; part[v][3] = zb1;
-            } else {                  // rows 2, 3: y[0] += z2, y[1] += -z2 - z3
-                part[v][0] = za0; part[v][1] = za1; part[v][2] = -za0 - zb0; part[v][3] = -za1 - zb1;
+            for (int v = 0; v < 16; v++) {
+                const float za0 = (acc[0][v] + acc[1][v]) + acc[2][v], za1 = (acc[1][v] - acc[2][v]) - acc[3][v];
+                const float zb0 = (acc[4][v] + acc[5][v]) + acc[6][v], zb1 = (acc[5][v] - acc[6][v]) - acc[7][v];
+                if (wi == 0) {            // rows 0, 1: y[0] += z0 + z1, y[1] += z1
+                    part[v][0] = za0 + zb0; part[v][1] = za1 + zb1; part[v][2] = zb0; part[v][3] = zb1;
+                } else {                  // rows 2, 3: y[0] += z2, y[1] += -z2 - z3
+                    part[v][0] = za0; part[v][1] = za1; part[v][2] = -za0 - zb0; part[v][3] = -za1 - zb1;
+                }
+            }
+            if (wi == 1) {   // a lane's four shares of one accumulator row are one 128-bit store
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+                    *(float4 *)(xchg + ((wk * 16 + v) * 64 + lane) * 4) = make_float4(part[v][0], part[v][1], part[v][2], part[v][3]);
+            }
+            __syncthreads();
+            if (wi == 0) {
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    const float4 other = *(const float4 *)(xchg + ((wk * 16 + v) * 64 + lane) * 4);
+                    const float y[4] = {part[v][0] + other.x, part[v][1] + other.y, part[v][2] + other.z, part[v][3] + other.w};
+                    store(0, v, y);
+                }
+            }
+        } else {
+            // a wavefront holds one row i of the grid: all four put their z in LDS, each finishes eight accumulator rows
+#pragma unroll
+            for (int t = 0; t < TH; t++)
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+                    *(float2 *)(xchg + (((wk * 4 + wi) * 32 + t * 16 + v) * 64 + lane) * 2) =
+                        make_float2((acc[t][v] + acc[2 + t][v]) + acc[4 + t][v], (acc[2 + t][v] - acc[4 + t][v]) - acc[6 + t][v]);
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const int tv = wi * 8 + e;
+                float2 z[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) z[i] = *(const float2 *)(xchg + (((wk * 4 + i) * 32 + tv) * 64 + lane) * 2);
+                const float y[4] = {(z[0].x + z[1].x) + z[2].x, (z[0].y + z[1].y) + z[2].y, z[1].x + (-z[2].x - z[3].x), z[1].y + (-z[2].y - z[3].y)};
+                store(tv >> 4, tv & 15, y);
             }
         }
-        if (wi == 1) {   // a lane's four shares of one accumulator row are one 128-bit store
+        if (pass == 1) break;
+        // the parts of an infinity hold NaNs: a tile that is not finite is formed again with the fp32 instruction, one chunk and
+        // one position after the other (each wavefront's word lies behind the exchange area)
+        int *const bad = (int *)(lds + wino_xchg(BM));
+        const int mine = __any(probe != 0.0f);
+        if (lane == 0) bad[w] = mine;
+        __syncthreads();
+        const int4 bad0 = *(const int4 *)bad, bad1 = *(const int4 *)(bad + 4);
+        if (((bad0.x | bad0.y | bad0.z | bad0.w) | (bad1.x | bad1.y | bad1.z | bad1.w)) == 0) break;
+        constexpr int LDV = 20;   // V here: [16 positions][tile][16 channels (+ 4 pad)]
 #pragma unroll
-            for (int v = 0; v < 16; v++)
-                *(float4 *)(xchg + ((wk * 16 + v) * 64 + lane) * 4) = make_float4(part[v][0], part[v][1], part[v][2], part[v][3]);
+        for (int x = 0; x < 8; x++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[x][v] = 0.0f;
+#pragma unroll 1
+        for (int chunk = cb; chunk < ce; chunk++) {
+#pragma unroll
+            for (int i = 0; i < NPMAX; i++) patch_load(i, chunk);
+#pragma unroll
+            for (int g = 0; g < NPMAX / 4; g++)
+                if (4 * g < nslots)
+                    *(float4 *)((char *)raw0 + p_lds + g * 16) = make_float4(preg[4 * g], preg[4 * g + 1], preg[4 * g + 2], preg[4 * g + 3]);
+            __syncthreads();
+#pragma unroll
+            for (int b = 0; b < 4; b++) transform_read(b, raw0);
+#pragma unroll
+            for (int u = 0; u < TH; u++) {
+                const int item = u * 512 + tid, ti = item / (TT * 4), tau_t = (item >> 1) % TT, cq = 2 * ((item / (TT * 2)) & 1) + (item & 1);
+                float *const o = V0 + (ti * 4 * TT + tau_t) * LDV + cq * 4;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float4 x = tt[u][j == 0 ? 0 : j == 2 ? 2 : 1], y = tt[u][j < 2 ? 2 : j == 2 ? 1 : 3];
+                    const float s = j == 1 ? 1.0f : -1.0f;
+                    *(float4 *)(o + j * TT * LDV) = make_float4(__builtin_fmaf(s, y.x, x.x), __builtin_fmaf(s, y.y, x.y),
+                                                               __builtin_fmaf(s, y.z, x.z), __builtin_fmaf(s, y.w, x.w));
+                }
+            }
+            __syncthreads();
+            const __amdgpu_buffer_rsrc_t rw = fa_rsrc(chunk);
+            static_for<0, 8>([&](auto xtag) {
+                constexpr int xl = decltype(xtag)::value;
+                fa_load(StepTag<0>{}, rw, xb + xl / TH);
+                const float *const src = V0 + ((xb + xl / TH) * TT + xl % TH * 32 + l32) * LDV + kh * 8;
+                const float4 b0 = *(const float4 *)src, b1 = *(const float4 *)(src + 4);
+                const float b8[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    unsigned q[3];
+#pragma unroll
+                    for (int t = 0; t < 3; t++) q[t] = e & 1 ? fa_ring[0][t][e / 2] >> 16 : fa_ring[0][t][e / 2] & 0xffffu;
+                    auto val = [&](int t) { return __builtin_bit_cast(float, q[t] << 16); };
+                    const float a = q[0] == kWinoRaw ? __builtin_bit_cast(float, q[1] << 16 | q[2])
+                                                     : (val(0) + val(1) + val(2)) * (1.0f / kSplitUp);
+                    acc[xl] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b8[e], acc[xl], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
         }
         __syncthreads();
-        if (wi == 1) return;
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const float4 other = *(const float4 *)(xchg + ((wk * 16 + v) * 64 + lane) * 4);
-            float y[4] = {(part[v][0] + other.x) * down, (part[v][1] + other.y) * down, (part[v][2] + other.z) * down,
-                          (part[v][3] + other.w) * down};
-            store(0, v, y, 1u << v);
-        }
-        while (again) {
-            const int v = __builtin_ctz(again);
-            again &= again - 1;
-            store_fp32(0, v);
-        }
-    } else {
-        // a wavefront holds one row i of the grid: all four put their z in LDS, each finishes eight accumulator rows
-#pragma unroll
-        for (int t = 0; t < TH; t++)
-#pragma unroll
-            for (int v = 0; v < 16; v++)
-                *(float2 *)(xchg + (((wk * 4 + wi) * 32 + t * 16 + v) * 64 + lane) * 2) =
-                    make_float2((acc[t][v] + acc[2 + t][v]) + acc[4 + t][v], (acc[2 + t][v] - acc[4 + t][v]) - acc[6 + t][v]);
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const int tv = wi * 8 + e;
-            float2 z[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) z[i] = *(const float2 *)(xchg + (((wk * 4 + i) * 32 + tv) * 64 + lane) * 2);
-            float y[4] = {((z[0].x + z[1].x) + z[2].x) * down, ((z[0].y + z[1].y) + z[2].y) * down,
-                          (z[1].x + (-z[2].x - z[3].x)) * down, (z[1].y + (-z[2].y - z[3].y)) * down};
-            store(tv >> 4, tv & 15, y, 1u << e);
-        }
-        while (again) {
-            const int tv = wi * 8 + __builtin_ctz(again);
-            again &= again - 1;
-            store_fp32(tv >> 4, tv & 15);
-        }
+        scale = 1.0f;
     }
 }
 
@@ -1985,7 +1977,7 @@ PatchSetup patch_setup_as(const dopt_hip_conv_desc *d, size_t P, size_t Q, bool 
         if (pc.rows % 2 != 0) return u;   // a pixel tile is whole 2 x 2 tiles
         const size_t buffers = u.BM == 128 ? 2 : 1;   // 32 tiles: raw patch and V are double-buffered
         const size_t floats = buffers * ((size_t)(((pc.psz + 1) * 20 + 3) / 4 * 4) + (size_t)16 * (u.BN / 4) * 24);
-        u.lds_bytes = std::max(floats, (size_t)wino_xchg(u.BM)) * sizeof(float);
+        u.lds_bytes = std::max(floats, (size_t)wino_xchg(u.BM) + 8) * sizeof(float);
     }
     if (u.lds_bytes > 160 * 1024) return u;
     pc.magic_psz = div_magic((unsigned)pc.psz);
