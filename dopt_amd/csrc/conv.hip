@@ -276,6 +276,7 @@ struct PatchConv {
     int nimg, rows;    // images per pixel tile; output rows of each image in the tile
     int PR, PC, psz;   // patch rows and columns per image; patch positions per tile = nimg*PR*PC
     unsigned magic_psz, magic_img, magic_pc;  // floor(2^32/d)+1 for d = psz, PR*PC, PC (exact for x*d < 2^32)
+    unsigned magic_tpi, magic_tcn;            // Winograd: the same for the 2 x 2 tiles of one image in the pixel tile, and of one row
     int Mp;            // rows of one packed filter slab (Mout rounded up to the tile height)
     int ncols, mtiles, ntiles, chunks_total, chunks_per_split, splits;
     size_t out_elems, in_bytes, wp_bytes;
@@ -581,6 +582,12 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
 
     // ---- the transform items of this thread (TH of them): row ti of Bt d B for tile tau, channels 4 cq .. 4 cq + 3
     const int tcn = p.OW >> 1, tpi = (p.rows >> 1) * tcn;          // tiles per row of tiles, per image of the pixel tile
+    auto tile_at = [&](int tau, int &img, int &r2, int &c2) {
+        img = (int)fast_div((unsigned)tau, p.magic_tpi);
+        const int tl = tau - img * tpi;
+        r2 = (int)fast_div((unsigned)tl, p.magic_tcn);
+        c2 = tl - r2 * tcn;
+    };
     // Bt = [1 0 -1 0; 0 1 1 0; 0 -1 1 0; 0 1 0 -1]: row ti is d[ra] + sg * d[rb]
     int t_a[TH], t_b[TH], t_out[TH];
     float sg[TH];
@@ -590,7 +597,8 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
         // the patch nor the 64-bit writes of the parts meet in a bank)
         const int item = u * 512 + tid, ti = item / (TT * 4), tau_t = (item >> 1) % TT, cqh = (item / (TT * 2)) & 1;
         const int cq = 2 * cqh + (item & 1);
-        const int img = tau_t / tpi, tl = tau_t - img * tpi, r2 = tl / tcn, c2 = tl - r2 * tcn;
+        int img, r2, c2;
+        tile_at(tau_t, img, r2, c2);
         const int t_in = ((img * p.PR + 2 * r2) * p.PC + 2 * c2) * LDP + cq * 4;
         const int ra = ti == 0 ? 0 : ti == 2 ? 2 : 1, rb = ti == 0 ? 2 : ti == 1 ? 2 : ti == 2 ? 1 : 3;
         t_a[u] = t_in + ra * p.PC * LDP;
@@ -757,7 +765,8 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
             probe = __builtin_fmaf(sum[q], 0.0f, probe);
             y[q] = sum[q] * scale;
         }
-        const int tau = t * 32 + l32, img = tau / tpi, tl = tau - img * tpi, r2 = tl / tcn, c2 = tl - r2 * tcn;
+        int img, r2, c2;
+        tile_at(t * 32 + l32, img, r2, c2);
         const int n = n_first + img, m = m0 + wk * 32 + acc_row(v, lane);
         if (n >= p.N || m >= p.Mout) return;
         if (add_bias) {
@@ -1975,6 +1984,8 @@ PatchSetup patch_setup_as(const dopt_hip_conv_desc *d, size_t P, size_t Q, bool 
     u.lds_bytes = (size_t)2 * (pc.psz + 1) * 20 * sizeof(float);
     if (wino) {
         if (pc.rows % 2 != 0) return u;   // a pixel tile is whole 2 x 2 tiles
+        pc.magic_tpi = div_magic((unsigned)(pc.rows / 2 * (pc.OW / 2)));
+        pc.magic_tcn = div_magic((unsigned)(pc.OW / 2));
         const size_t buffers = u.BM == 128 ? 2 : 1;   // 32 tiles: raw patch and V are double-buffered
         const size_t floats = buffers * ((size_t)(((pc.psz + 1) * 20 + 3) / 4 * 4) + (size_t)16 * (u.BN / 4) * 24);
         u.lds_bytes = std::max(floats, (size_t)wino_xchg(u.BM) + 8) * sizeof(float);
