@@ -2192,8 +2192,17 @@ int HIPPlan::resolve(int nargs, const int *argOps, const void *const *argPtrs, c
                 if (mArgUsed[slot]) DOPT_HIP_CHECK(hipEventSynchronize(mArgDone[slot]));
             }
             HostArg &h = mHostArgs[slot][id];
-            if (!h.dev && bytes)
+            if (!h.dev && bytes) {
                 if (int rc = dopt_hip_malloc(&h.dev, bytes)) return rc;
+                // The fill of a new block, and the kernels of whoever had it before, are on the main queue; the uploads run
+                // beside it, and one that overtook the fill was lost.
+                hipEvent_t filled = nullptr;
+                DOPT_HIP_CHECK(hipEventCreateWithFlags(&filled, hipEventDisableTiming));
+                const hipError_t recorded = hipEventRecord(filled, lane_stream(0));
+                const hipError_t waits = recorded == hipSuccess ? hipStreamWaitEvent(lane_stream(1), filled, 0) : recorded;
+                (void)hipEventDestroy(filled);
+                DOPT_HIP_CHECK(waits);
+            }
             if (!h.pinned && bytes)
                 if (int rc = dopt_hip_host_alloc(&h.pinned, bytes)) return rc;
             if (bytes) {

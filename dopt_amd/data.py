@@ -157,6 +157,7 @@ class DeviceFeed:
                 "g_host": PinnedArray([batch_size, 3], np.int32),
                 "raw": ops.Tensor([batch_size] + list(fshape)), "f": ops.Tensor([batch_size] + list(fshape)),
                 "l": ops.Tensor([batch_size] + list(lshape)), "g": ops.Tensor([batch_size, 3], np.int32)})
+        ops.sync()   # the new buffers are filled on the first queue: the uploads on the second must not overtake that
         self._turn = 0
         self._marks = []
         for _ in range(2):

@@ -99,3 +99,28 @@ def test_checkpoint_round_trip_through_device_parameters(tmp_path):
     after, = plan2.execute({x2: xs, y2: ys})             # the registered variables now hold the loaded values
     want, = core.compile([loss]).execute({x: xs, y: ys})
     assert after == want and after != before
+
+
+def test_first_uploads_do_not_overtake_the_fill_of_their_buffers():
+    """The buffers that host arguments and fed batches are uploaded to are new on first use, and filled on the main queue
+    behind whatever is queued there; the uploads run on the second queue."""
+    r = np.random.default_rng(3)
+    x = r.standard_normal((64, 3, 32, 32)).astype(np.float32)
+    y = r.standard_normal((64, 10)).astype(np.float32)
+    big = ops.tensor(r.standard_normal((4096, 4096)).astype(np.float32))
+    out = ops.Tensor([4096, 4096])
+
+    def busy():
+        for _ in range(8):   # some milliseconds of work in front of the fills
+            ops.matmul(big, big, out=out)
+
+    a, b = core.float32([64, 3, 32, 32]), core.float32([64, 10])
+    plan = core.compile([a + a, b + b])
+    for _ in range(2):
+        busy()
+        got = plan.execute({a: x, b: y})
+        assert np.array_equal(got[0], x + x) and np.array_equal(got[1], y + y)
+    busy()
+    feed = data.DeviceFeed(data.SupervisedBatchIterator(x, y, [(3, 32, 32), (10,)], shuffle=False), 64)
+    f, l = feed.next()
+    assert np.array_equal(f.numpy(), x) and np.array_equal(l.numpy(), y)
