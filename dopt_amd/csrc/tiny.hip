@@ -76,6 +76,48 @@ __device__ __forceinline__ void pw_loop(int n, AP a, AP b, int ka, int kb, int i
     }
 }
 
+// Operands and result all start on a quad: four consecutive elements a thread, so that the most a node can have is one pass
+// (four single ones a thread were four times the instructions, and a node of 2560 elements 0.9 us instead of 0.4).  The
+// elements behind the last of an n that is no multiple of four are read and written in LDS, where every place ends on a
+// quad, and left alone in memory.
+__device__ __forceinline__ float4 quad_at(const float *p, int i, int n, bool single)
+{
+    (void)n;
+    if (single) return make_float4(*p, *p, *p, *p);
+    return *(const float4 *)(p + i);
+}
+
+__device__ __forceinline__ float4 quad_at(const gfloat *p, int i, int n, bool single)
+{
+    if (single) return make_float4(*p, *p, *p, *p);
+    if (i + 3 < n) {
+        typedef float Quad __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(1))) Quad gquad;
+        const Quad v = *(const gquad *)(p + i);
+        return make_float4(v.x, v.y, v.z, v.w);
+    }
+    return make_float4(p[i], p[min(i + 1, n - 1)], p[min(i + 2, n - 1)], 0.0f);
+}
+
+template <int kOp, class AP>
+__device__ __forceinline__ void pw_quads(int n, AP a, AP b, int ka, int kb, float *dstL, gfloat *dstG)
+{
+    const int i = 4 * (int)threadIdx.x;
+    if (i >= n) return;
+    const float4 x = quad_at(a, i, n, ka == 1), y = quad_at(b, i, n, kb == 1);
+    const float4 r = make_float4(pw_apply<kOp>(x.x, y.x), pw_apply<kOp>(x.y, y.y), pw_apply<kOp>(x.z, y.z), pw_apply<kOp>(x.w, y.w));
+    if (dstL) *(float4 *)(dstL + i) = r;
+    if (i + 3 < n) {
+        typedef float Quad __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(1))) Quad gquad;
+        *(gquad *)(dstG + i) = Quad{r.x, r.y, r.z, r.w};
+    } else {
+        dstG[i] = r.x;
+        if (i + 1 < n) dstG[i + 1] = r.y;
+        if (i + 2 < n) dstG[i + 2] = r.z;
+    }
+}
+
 // Everything a node reads comes from LDS.  A load from memory waits for every store the wavefront issued before it
 // (one counter tracks both), so a node that reads what the node before it has just stored to memory waits for that
 // store to reach the L2 and for its own load to come back: 3-4 us per node, and a chain of thirteen nodes took as long
@@ -88,7 +130,6 @@ constexpr int kArenaFloats = 12288;
 constexpr int kTinyStaged = 16;
 struct TinyLds {
     short dst, a, b;   // float offsets into the arena, or -1
-    short pad;
 };
 struct TinyStage {
     const float *src;
@@ -96,16 +137,31 @@ struct TinyStage {
     short n;
     int pad;
 };
+// A node as the kernels read it, addresses resolved by the host.  `threads`: how many threads have something to do (all of
+// them where the node has barriers of its own); wavefronts past it go on to the next barrier.  `meet`: whether the workgroup
+// meets in front of the node.  It does not between two nodes that only the first wavefront takes part in and that find
+// their operands in LDS.
+struct TinyAddress {
+    unsigned lo, hi;
+};
+struct TinyNode {
+    TinyAddress dst;
+    TinyLds lds;
+    short threads;
+    unsigned char kind, op, a_kind, b_kind;
+    short n;
+    unsigned char meet, quads;
+    TinyAddress a, b;
+    short dims[4], reps[4];
+    unsigned odd[3];           // seventeen words: see Description
+};
 struct TinyProgram {
-    void *slot[DOPT_HIP_TINY_SLOTS];
-    dopt_hip_tiny_node node[DOPT_HIP_TINY_NODES];
-    TinyLds lds[DOPT_HIP_TINY_NODES];
-    int nnodes;
+    TinyNode node[DOPT_HIP_TINY_NODES];
+    TinyStage in[kTinyStaged];   // what enters the arena from outside
+    int nnodes, staged;
 };
-struct TinyStaging {
-    TinyStage in[kTinyStaged];
-    int n;
-};
+static_assert(sizeof(TinyNode) == 17 * 4 && DOPT_HIP_TINY_NODES <= 64 && DOPT_HIP_TINY_ELEMS < 32768, "a lane a node; counts fit 16 bits");
+static_assert(sizeof(TinyProgram) <= 4 * kTinyThreads, "fetched with one load a thread");
 
 template <bool kSum>
 __device__ inline float fold(float a, float b)
@@ -171,7 +227,7 @@ __device__ __forceinline__ void reduce_row(AP row, int R, bool quads, float *out
 }
 
 template <bool kSum, class AP>
-__device__ __forceinline__ void reduce_node(const dopt_hip_tiny_node &nd, AP in, bool in_aligned, float *out, gfloat *out2, float *part)
+__device__ __forceinline__ void reduce_node(const TinyNode &nd, AP in, float *out, gfloat *out2, float *part)
 {
     const int outer = nd.dims[0], R = nd.dims[1], inner = nd.dims[2];
     if (inner > 1 || R <= 64) {   // red_cols: thread (o, j) folds in ascending r from the identity
@@ -186,24 +242,87 @@ __device__ __forceinline__ void reduce_node(const dopt_hip_tiny_node &nd, AP in,
         }
         return;
     }
-    (void)in_aligned;
     const bool quads = R % 4 == 0;   // dopt_hip_reduce's test: the order does not depend on where the row starts in memory
     for (int o = 0; o < outer; o++) reduce_row<kSum, AP>(in + (size_t)o * R, R, quads, out ? out + o : nullptr, out2 ? out2 + o : nullptr, part);
 }
 
+// The part of a node's description that every node needs, in scalar registers.
+struct Node {
+    gfloat *dst;
+    int lds_dst, lds_a, lds_b, threads, kind, op, a_kind, b_kind, n, meet, quads;
+    const gfloat *a, *b;
+    const TinyNode *rest;   // extents, in LDS
+};
+
+// What a wavefront holds of the run: lane l keeps the words of node l, so that the description of the node it comes to is a
+// few register reads away.  Read from LDS when the node is reached, in steps that depend on each other, it took 0.6 us a node
+// whatever the node did (sixteen nodes on one element 13.0 us, now 10.3, on 2560 elements 17.8, now 13.8; a register read also
+// makes the switch over the operation a scalar branch).  Lanes are seventeen words apart, so that the words of sixty-four nodes lie in different banks.
+template <bool kThroughMemory>
+struct Description {
+    unsigned w[kThroughMemory ? 10 : 6];
+    __device__ __forceinline__ void load(const TinyProgram &pr)
+    {
+        const unsigned *p = (const unsigned *)&pr.node[min((int)threadIdx.x & 63, DOPT_HIP_TINY_NODES - 1)];
+#pragma unroll
+        for (int i = 0; i < (kThroughMemory ? 10 : 6); i++) w[i] = p[i];
+    }
+    __device__ __forceinline__ int word(int i, int k) const { return __builtin_amdgcn_readlane((int)w[i], k); }
+    __device__ __forceinline__ gfloat *address(int i, int k) const
+    {
+        return (gfloat *)(uintptr_t)((unsigned)word(i, k) | (unsigned long long)(unsigned)word(i + 1, k) << 32);
+    }
+    __device__ __forceinline__ Node node(int k, const TinyProgram &pr) const
+    {
+        const int at = word(2, k), rest = word(3, k), kinds = word(4, k), count = word(5, k);
+        Node nd;
+        nd.dst = address(0, k);
+        nd.lds_dst = (short)at;
+        nd.lds_a = at >> 16;
+        nd.lds_b = (short)rest;
+        nd.threads = rest >> 16;
+        nd.kind = kinds & 255;
+        nd.op = kinds >> 8 & 255;
+        nd.a_kind = kinds >> 16 & 255;
+        nd.b_kind = (unsigned)kinds >> 24;
+        nd.n = (short)count;
+        nd.meet = count >> 16 & 255;
+        nd.quads = (unsigned)count >> 24;
+        nd.a = nd.b = nullptr;
+        if constexpr (kThroughMemory) {
+            nd.a = address(6, k);
+            nd.b = address(8, k);
+        }
+        nd.rest = &pr.node[k];
+        return nd;
+    }
+};
+
 // One node.  a, b: where its operands lie; dstL: the result's place in LDS (or null), dstG: its buffer in memory (or
 // null).  The softmax keeps its exponentials where it will leave the result: in LDS when it has a place there.
 template <class AP>
-__device__ __forceinline__ void run_node(const dopt_hip_tiny_node &nd, AP a, AP b, bool a_aligned, float *dstL, gfloat *dstG,
+__device__ __forceinline__ void run_node(const Node &of, AP a, AP b, float *dstL, gfloat *dstG,
                                          float *part)
 {
-    const int n = nd.n;
-    switch (nd.kind) {
+    const int n = of.n;
+    const TinyNode &nd = *of.rest;
+    switch (of.kind) {
     case DOPT_HIP_TINY_POINTWISE: {
         // where result i finds an operand: 0 at i, 1 at its only element, 2 at its row, 3 at its column of [n / dims[0], dims[0]]
-        const int inner = nd.dims[0] > 0 ? nd.dims[0] : 1;
-        const int ka = nd.a_kind, kb = nd.b < 0 ? nd.a_kind : nd.b_kind;
-        switch (nd.op) {
+        const int inner = of.a_kind < 2 && of.b_kind < 2 ? 1 : nd.dims[0];
+        const int ka = of.a_kind, kb = of.b_kind;
+        if (of.quads) {
+            switch (of.op) {
+#define DOPT_PW_CASE(name, arity, f32, i32) \
+            case OP_##name:                 \
+                pw_quads<OP_##name, AP>(n, a, b, ka, kb, dstL, dstG); \
+                break;
+                DOPT_PW_OPS(DOPT_PW_CASE)
+#undef DOPT_PW_CASE
+            }
+            break;
+        }
+        switch (of.op) {
 #define DOPT_PW_CASE(name, arity, f32, i32) \
         case OP_##name:                         \
             pw_loop<OP_##name, AP>(n, a, b, ka, kb, inner, dstL, dstG); \
@@ -214,8 +333,8 @@ __device__ __forceinline__ void run_node(const dopt_hip_tiny_node &nd, AP a, AP 
         break;
     }
     case DOPT_HIP_TINY_REDUCE:
-        if (nd.op == 0) reduce_node<true, AP>(nd, a, a_aligned, dstL, dstG, part);
-        else reduce_node<false, AP>(nd, a, a_aligned, dstL, dstG, part);
+        if (of.op == 0) reduce_node<true, AP>(nd, a, dstL, dstG, part);
+        else reduce_node<false, AP>(nd, a, dstL, dstG, part);
         break;
     case DOPT_HIP_TINY_SOFTMAX: {
         const int N = nd.dims[0], C = nd.dims[1], inner = nd.dims[2];
@@ -333,14 +452,27 @@ __device__ __forceinline__ void run_node(const dopt_hip_tiny_node &nd, AP a, AP 
 // Through memory: every node reads its operands from, and writes its result to, the buffers themselves.
 // The run's description arrives as kernel arguments, which live in host-visible memory: read node by node as the loop
 // reaches them, every node waited a microsecond or two for its own description.  All threads fetch it together instead,
-// 16 bytes each, into LDS, and the loop reads it from there.
-template <class T>
-__device__ __forceinline__ void fetch_args(const T &args, T *to)
+// a word each, into LDS, and the loop reads it from there.
+__device__ __forceinline__ void fetch_args(const TinyProgram &args, TinyProgram *to)
 {
-    static_assert(sizeof(T) % 4 == 0, "copied in words");
-    const unsigned *src = (const unsigned *)&args;
-    unsigned *dst = (unsigned *)to;
-    for (unsigned i = threadIdx.x; i < sizeof(T) / 4; i += kTinyThreads) dst[i] = src[i];
+    if (threadIdx.x < sizeof(TinyProgram) / 4) ((unsigned *)to)[threadIdx.x] = ((const unsigned *)&args)[threadIdx.x];
+    __syncthreads();
+}
+
+// The nodes one after the other: run(node) by the wavefronts that have something to do.  Instructions of idle wavefronts cost
+// as much as those of busy ones (four wavefronts share a SIMD), so a wavefront past `threads` goes on at once.
+template <bool kThroughMemory, class Run>
+__device__ __forceinline__ void run_nodes(const TinyProgram &pr, Run &&run)
+{
+    const int first = __builtin_amdgcn_readfirstlane((int)threadIdx.x) & ~63, nnodes = __builtin_amdgcn_readfirstlane(pr.nnodes);
+    Description<kThroughMemory> all;
+    all.load(pr);
+    for (int k = 0; k < nnodes; k++) {
+        const Node nd = all.node(k, pr);
+        if (nd.meet) __syncthreads();
+        else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // (LDS serves a wavefront in order)
+        if (first < nd.threads) run(nd);
+    }
 }
 
 __global__ __launch_bounds__(kTinyThreads) void tiny_graph_mem_k(TinyProgram args)
@@ -348,63 +480,48 @@ __global__ __launch_bounds__(kTinyThreads) void tiny_graph_mem_k(TinyProgram arg
     __shared__ float part[kTinyBlock / 64];
     __shared__ TinyProgram pr;
     fetch_args(args, &pr);
-    __syncthreads();
-    for (int k = 0; k < pr.nnodes; k++) {
-        const dopt_hip_tiny_node &nd = pr.node[k];
-        gfloat *mem = (gfloat *)((uintptr_t)pr.slot[nd.dst] + (uintptr_t)nd.dst_offset);
-        const gfloat *a = (const gfloat *)((uintptr_t)pr.slot[nd.a] + (uintptr_t)nd.a_offset);
-        const gfloat *b = nd.b < 0 ? a : (const gfloat *)((uintptr_t)pr.slot[nd.b] + (uintptr_t)nd.b_offset);
-        run_node<const gfloat *>(nd, a, b, ((uintptr_t)a & 15u) == 0, nullptr, mem, part);
-        __syncthreads();   // the next node reads what this one wrote (stores of a workgroup are ordered by its barrier)
-    }
+    run_nodes<true>(pr, [&](const Node &nd) { run_node<const gfloat *>(nd, nd.a, nd.b, nullptr, nd.dst, part); });
 }
 
 // Through LDS: every operand has a place in the arena (see above).
-__global__ __launch_bounds__(kTinyThreads) void tiny_graph_lds_k(TinyProgram args, TinyStaging staged)
+__global__ __launch_bounds__(kTinyThreads) void tiny_graph_lds_k(TinyProgram args)
 {
     __shared__ float part[kTinyBlock / 64];
     __shared__ __attribute__((aligned(16))) float arena[kArenaFloats];
     __shared__ TinyProgram pr;
-    __shared__ TinyStaging st;
     fetch_args(args, &pr);
-    fetch_args(staged, &st);
-    __syncthreads();
-    if (st.n > 0) {   // what enters from outside: the loads of ALL ranges in flight together (one after the other, each range cost a
+    const int entering = __builtin_amdgcn_readfirstlane(pr.staged), first = __builtin_amdgcn_readfirstlane((int)threadIdx.x) & ~63;
+    if (entering > 0) {   // what enters from outside: the loads of ALL ranges in flight together (one after the other, each range cost a
         // trip to memory), two per range and thread, then a loop for what is left of ranges beyond 2048 values
         float v[kTinyStaged][2];
 #pragma unroll
         for (int e = 0; e < kTinyStaged; e++) {
-            const int ee = min(e, st.n - 1), n = st.in[ee].n;
-            const gfloat *src = (const gfloat *)(uintptr_t)st.in[ee].src;
+            if (e >= entering) break;
+            const int n = __builtin_amdgcn_readfirstlane(pr.in[e].n);
+            const gfloat *src = (const gfloat *)(uintptr_t)pr.in[e].src;
 #pragma unroll
-            for (int u = 0; u < 2; u++) v[e][u] = src[min((int)threadIdx.x + u * kTinyThreads, n - 1)];
+            for (int u = 0; u < 2; u++)
+                if (first + u * kTinyThreads < n) v[e][u] = src[min((int)threadIdx.x + u * kTinyThreads, n - 1)];
         }
 #pragma unroll
         for (int e = 0; e < kTinyStaged; e++) {
-            if (e >= st.n) break;
-            float *to = arena + st.in[e].at;
+            if (e >= entering) break;
+            const int n = __builtin_amdgcn_readfirstlane(pr.in[e].n);
+            float *to = arena + pr.in[e].at;
 #pragma unroll
             for (int u = 0; u < 2; u++)
-                if ((int)threadIdx.x + u * kTinyThreads < st.in[e].n) to[threadIdx.x + u * kTinyThreads] = v[e][u];
+                if (first + u * kTinyThreads < n && (int)threadIdx.x + u * kTinyThreads < n) to[threadIdx.x + u * kTinyThreads] = v[e][u];
         }
-        for (int e = 0; e < st.n; e++) {
-            const gfloat *src = (const gfloat *)(uintptr_t)st.in[e].src;
-            float *to = arena + st.in[e].at;
-            for (int i = threadIdx.x + 2 * kTinyThreads; i < st.in[e].n; i += kTinyThreads) to[i] = src[i];
+        for (int e = 0; e < entering; e++) {
+            const gfloat *src = (const gfloat *)(uintptr_t)pr.in[e].src;
+            float *to = arena + pr.in[e].at;
+            for (int i = threadIdx.x + 2 * kTinyThreads; i < pr.in[e].n; i += kTinyThreads) to[i] = src[i];
         }
     }
     __syncthreads();
-    for (int k = 0; k < pr.nnodes; k++) {
-        const dopt_hip_tiny_node &nd = pr.node[k];
-        const TinyLds &ld = pr.lds[k];
-        gfloat *mem = (gfloat *)((uintptr_t)pr.slot[nd.dst] + (uintptr_t)nd.dst_offset);
-        const float *a = arena + ld.a;
-        const float *b = nd.b < 0 ? a : arena + ld.b;
-        // (the row sums take quads where the tensor in memory would allow it)
-        const bool aligned = (((uintptr_t)pr.slot[nd.a] + (uintptr_t)nd.a_offset) & 15u) == 0;
-        run_node<const float *>(nd, a, b, aligned, ld.dst >= 0 ? arena + ld.dst : nullptr, mem, part);
-        __syncthreads();
-    }
+    run_nodes<false>(pr, [&](const Node &nd) {
+        run_node<const float *>(nd, arena + nd.lds_a, arena + nd.lds_b, nd.lds_dst >= 0 ? arena + nd.lds_dst : nullptr, nd.dst, part);
+    });
 }
 
 // How many values a node reads from operand a (which = 0) or b (1).
@@ -425,7 +542,7 @@ int operand_extent(const dopt_hip_tiny_node &nd, int which)
 // name one buffer), or the range of memory it enters the run from; for every result the span of nodes that read it; then
 // first fit in node order, places given back when their last reader has run.  False when something finds no room (or
 // an operand overlaps an earlier result only in part): the run then goes through memory.
-bool assign_lds(int nnodes, const dopt_hip_tiny_node *nodes, void *const *slots, TinyLds *lds, TinyStaging *st)
+bool assign_lds(int nnodes, const dopt_hip_tiny_node *nodes, void *const *slots, TinyLds *lds, TinyStage *staged, int *nstaged)
 {
     int producer[DOPT_HIP_TINY_NODES][2], last_reader[DOPT_HIP_TINY_NODES];
     struct Ext { const char *lo, *hi; int at; };
@@ -433,7 +550,7 @@ bool assign_lds(int nnodes, const dopt_hip_tiny_node *nodes, void *const *slots,
     int ext_of[DOPT_HIP_TINY_NODES][2];
     for (int k = 0; k < nnodes; k++) {
         last_reader[k] = -1;
-        lds[k] = TinyLds{-1, -1, -1, 0};
+        lds[k] = TinyLds{-1, -1, -1};
         for (int w = 0; w < 2; w++) {
             producer[k][w] = ext_of[k][w] = -1;
             const int slot = w == 0 ? nodes[k].a : nodes[k].b;
@@ -463,14 +580,14 @@ bool assign_lds(int nnodes, const dopt_hip_tiny_node *nodes, void *const *slots,
     // what comes from outside stays for the whole run, at the bottom of the arena; 16-byte aligned copies of 16-byte
     // aligned ranges (a row sum reads quads from its copy exactly where it would from memory)
     int floor = 0;
-    st->n = 0;
+    *nstaged = 0;
     for (Ext &e : exts) {
         const int n = (int)((e.hi - e.lo) / 4);
         const int skew = (int)(((uintptr_t)e.lo & 15u) / 4);   // the copy starts as far into a quad as the range does
         e.at = floor + skew;
         floor += (skew + n + 3) / 4 * 4;
         if (floor > kArenaFloats || n > 32767) return false;
-        st->in[st->n++] = TinyStage{(const float *)e.lo, (short)e.at, (short)n, 0};
+        staged[(*nstaged)++] = TinyStage{(const float *)e.lo, (short)e.at, (short)n, 0};
     }
     struct Span { int at, len, until; };
     std::vector<Span> held;
@@ -521,8 +638,7 @@ int dopt_hip_tiny_graph(int nslots, void *const *slots, int nnodes, const dopt_h
                  "dopt_hip_tiny_graph: %d buffers and %d nodes (at most %d and %d)", nslots, nnodes, DOPT_HIP_TINY_SLOTS,
                  DOPT_HIP_TINY_NODES);
     DOPT_ENSURE_INIT();
-    TinyProgram pr{};
-    for (int i = 0; i < nslots; i++) pr.slot[i] = slots[i];
+    std::vector<dopt_hip_tiny_node> plain_nodes(nodes, nodes + nnodes);
     for (int k = 0; k < nnodes; k++) {
         const dopt_hip_tiny_node &nd = nodes[k];
         const bool binary = nd.kind == DOPT_HIP_TINY_SOFTMAX_GRAD || (nd.kind == DOPT_HIP_TINY_POINTWISE && nd.b >= 0);
@@ -555,18 +671,54 @@ int dopt_hip_tiny_graph(int nslots, void *const *slots, int nnodes, const dopt_h
             DOPT_REQUIRE(nd.dims[0] >= 0 && nd.dims[1] >= 1 && nd.dims[2] >= 1 && (long long)nd.dims[0] * nd.dims[1] * nd.dims[2] == nd.n,
                          "dopt_hip_tiny_graph: node %d: softmax over [%d, %d, %d] does not have %d elements", k, nd.dims[0], nd.dims[1], nd.dims[2], nd.n);
         }
-        pr.node[k] = nd;
         if (nd.kind == DOPT_HIP_TINY_POINTWISE && nd.dims[0] >= 1) {   // a grid of one column or one row needs no division
-            dopt_hip_tiny_node &q = pr.node[k];
+            dopt_hip_tiny_node &q = plain_nodes[(size_t)k];
             const int inner = nd.dims[0], rows = nd.n / inner;
             auto plain = [&](int kind) { return kind == 2 ? (inner == 1 ? 0 : rows == 1 ? 1 : 2) : kind == 3 ? (inner == 1 ? 1 : rows == 1 ? 0 : 3) : kind; };
             q.a_kind = plain(nd.a_kind);
             q.b_kind = plain(nd.b_kind);
         }
     }
+    TinyProgram pr{};
     pr.nnodes = nnodes;
-    TinyStaging st{};
-    if (assign_lds(nnodes, pr.node, slots, pr.lds, &st)) hipLaunchKernelGGL(tiny_graph_lds_k, dim3(1), dim3(kTinyThreads), 0, stream(), pr, st);
+    TinyLds lds[DOPT_HIP_TINY_NODES];
+    const bool in_lds = assign_lds(nnodes, plain_nodes.data(), slots, lds, pr.in, &pr.staged);
+    bool alone = false;   // whether the node before is the first wavefront's alone
+    for (int k = 0; k < nnodes; k++) {
+        const dopt_hip_tiny_node &nd = plain_nodes[(size_t)k];
+        TinyNode &to = pr.node[k];
+        auto words = [&](int slot, int offset) {
+            const unsigned long long p = (unsigned long long)(uintptr_t)slots[slot] + (unsigned long long)offset;
+            return TinyAddress{(unsigned)p, (unsigned)(p >> 32)};
+        };
+        to.dst = words(nd.dst, nd.dst_offset);
+        to.a = words(nd.a, nd.a_offset);
+        to.b = nd.b < 0 ? to.a : words(nd.b, nd.b_offset);
+        to.lds = lds[k];
+        if (nd.b < 0) to.lds.b = to.lds.a;
+        to.kind = (unsigned char)nd.kind;
+        to.op = (unsigned char)nd.op;
+        to.a_kind = (unsigned char)nd.a_kind;
+        to.b_kind = (unsigned char)(nd.b < 0 ? nd.a_kind : nd.b_kind);
+        to.n = (short)nd.n;
+        for (int d = 0; d < 4; d++) {
+            to.dims[d] = (short)nd.dims[d];
+            to.reps[d] = (short)nd.reps[d];
+        }
+        long long busy = nd.n;
+        if (nd.kind == DOPT_HIP_TINY_SOFTMAX || nd.kind == DOPT_HIP_TINY_SOFTMAX_GRAD) busy = (long long)nd.dims[0] * nd.dims[2];
+        else if (nd.kind == DOPT_HIP_TINY_REDUCE && nd.dims[2] == 1 && nd.dims[1] > 64) busy = kTinyThreads;   // rows: the block folds them together
+        // quads: an operand that is read element by element, and the result, start on one in memory and in LDS
+        auto on_quad = [](const TinyAddress &m, int at, bool single) { return single || ((m.lo & 15u) == 0 && (at & 3) == 0); };
+        to.quads = nd.kind == DOPT_HIP_TINY_POINTWISE && to.a_kind < 2 && to.b_kind < 2 && on_quad(to.a, in_lds ? to.lds.a : 0, to.a_kind == 1) &&
+                   on_quad(to.b, in_lds ? to.lds.b : 0, to.b_kind == 1) && on_quad(to.dst, in_lds && to.lds.dst >= 0 ? to.lds.dst : 0, false);
+        if (to.quads) busy = (nd.n + 3) / 4;
+        to.threads = (short)(busy < kTinyThreads ? busy : kTinyThreads);
+        const bool one = in_lds && to.threads <= 64;
+        to.meet = k > 0 && !(one && alone);
+        alone = one;
+    }
+    if (in_lds) hipLaunchKernelGGL(tiny_graph_lds_k, dim3(1), dim3(kTinyThreads), 0, stream(), pr);
     else hipLaunchKernelGGL(tiny_graph_mem_k, dim3(1), dim3(kTinyThreads), 0, stream(), pr);
     DOPT_LAUNCH_CHECK();
     return DOPT_HIP_OK;
