@@ -361,20 +361,50 @@ __global__ __launch_bounds__(kBlock) void image_transform_k(uint32_t total, uint
     out[idx] = in[((size_t)(n * C + c) * H + sy) * W + sx];
 }
 
-// ---- many small device-to-device copies in one launch -----------------------------------------
-constexpr int kBatchCopies = 48;
+// ---- many device-to-device copies in one launch ------------------------------------------------
+// The outputs of a plan on their way to the caller's buffers: a hundred tensors of 10 to some million values.  A workgroup
+// finds its copy by its block number and moves 16 KB of it; a copy that is not on quads goes word by word, 4 KB a workgroup.
+constexpr int kBatchCopies = 128;
 struct CopyBatch {  // passed by value: no table to upload
     const void *src[kBatchCopies];
     void *dst[kBatchCopies];
     unsigned words[kBatchCopies];  // 4-byte words
+    unsigned first[kBatchCopies];  // the copy's first block; bit 31: on quads
+    int n;
 };
+constexpr unsigned kOnQuads = 0x80000000u;
+constexpr unsigned kCopyWords = 4096, kCopyLoose = 1024;   // words a block moves
 
 __global__ __launch_bounds__(256) void copy_batch_k(CopyBatch b)
 {
-    const unsigned *s = (const unsigned *)b.src[blockIdx.x];
-    unsigned *d = (unsigned *)b.dst[blockIdx.x];
-    const unsigned n = b.words[blockIdx.x];
-    for (unsigned i = threadIdx.x; i < n; i += 256) d[i] = s[i];
+    const int lane = threadIdx.x & 63;
+    const bool low = lane < b.n && (b.first[lane] & ~kOnQuads) <= blockIdx.x;
+    const bool high = lane + 64 < b.n && (b.first[lane + 64] & ~kOnQuads) <= blockIdx.x;
+    const int at = __popcll(__ballot(low)) + __popcll(__ballot(high)) - 1;
+    const unsigned n = b.words[at], first = b.first[at], block = blockIdx.x - (first & ~kOnQuads);
+    if (first & kOnQuads) {
+        const uint4 *s = (const uint4 *)b.src[at];
+        uint4 *d = (uint4 *)b.dst[at];
+        const unsigned quads = n / 4, q = block * (kCopyWords / 4) + threadIdx.x;
+        if (block * (kCopyWords / 4) + kCopyWords / 4 <= quads) {
+            const uint4 v0 = s[q], v1 = s[q + 256], v2 = s[q + 512], v3 = s[q + 768];
+            d[q] = v0;
+            d[q + 256] = v1;
+            d[q + 512] = v2;
+            d[q + 768] = v3;
+        } else {
+            for (unsigned i = q; i < quads; i += 256) d[i] = s[i];
+        }
+        if (block == 0 && threadIdx.x < n % 4) ((unsigned *)d)[quads * 4 + threadIdx.x] = ((const unsigned *)s)[quads * 4 + threadIdx.x];
+        return;
+    }
+    const unsigned *s = (const unsigned *)b.src[at];
+    unsigned *d = (unsigned *)b.dst[at];
+#pragma unroll
+    for (unsigned u = 0; u < 4; u++) {
+        const unsigned i = block * kCopyLoose + u * 256 + threadIdx.x;
+        if (i < n) d[i] = s[i];
+    }
 }
 
 }  // namespace
@@ -515,19 +545,24 @@ int dopt_hip_copy_d2d_batch(int n, void *const *dst, const void *const *src, con
     DOPT_ENSURE_INIT();
     CopyBatch b;
     int filled = 0;
+    size_t blocks = 0;
     auto flush = [&]() -> int {
         if (filled == 0) return DOPT_HIP_OK;
-        hipLaunchKernelGGL(copy_batch_k, dim3((unsigned)filled), dim3(256), 0, stream(), b);
+        b.n = filled;
+        hipLaunchKernelGGL(copy_batch_k, dim3((unsigned)blocks), dim3(256), 0, stream(), b);
         DOPT_LAUNCH_CHECK();
         filled = 0;
+        blocks = 0;
         return DOPT_HIP_OK;
     };
     for (int i = 0; i < n; i++) {
         if (bytes[i] == 0) continue;
         DOPT_REQUIRE(dst[i] && src[i], "dopt_hip_copy_d2d_batch: null pointer");
-        const bool small = bytes[i] <= 65536 && bytes[i] % 4 == 0 &&
+        const bool words = bytes[i] % 4 == 0 && bytes[i] / 4 < (1u << 31) &&
                            (reinterpret_cast<uintptr_t>(dst[i]) & 3u) == 0 && (reinterpret_cast<uintptr_t>(src[i]) & 3u) == 0;
-        if (!small) {
+        const char *s0 = (const char *)src[i], *t0 = (const char *)dst[i];
+        const bool apart = s0 + bytes[i] <= t0 || t0 + bytes[i] <= s0;
+        if (!words || !apart) {
             // the copies are sequential: what is still waiting in the batch goes first
             if (int rc = flush()) return rc;
             if (int rc = dopt_hip_copy_d2d(dst[i], src[i], bytes[i])) return rc;
@@ -539,15 +574,18 @@ int dopt_hip_copy_d2d_batch(int n, void *const *dst, const void *const *src, con
             const size_t len = (size_t)b.words[j] * 4;
             const char *d0 = (const char *)b.dst[j], *d1 = d0 + len;
             const char *r0 = (const char *)b.src[j], *r1 = r0 + len;
-            const char *s0 = (const char *)src[i], *t0 = (const char *)dst[i];
             if ((s0 < d1 && s0 + bytes[i] > d0) || (t0 < d1 && t0 + bytes[i] > d0) || (t0 < r1 && t0 + bytes[i] > r0)) {
                 if (int rc = flush()) return rc;
                 break;
             }
         }
+        const bool quads = aligned16(src[i]) && aligned16(dst[i]);
         b.src[filled] = src[i];
         b.dst[filled] = dst[i];
         b.words[filled] = (unsigned)(bytes[i] / 4);
+        b.first[filled] = (unsigned)blocks | (quads ? kOnQuads : 0u);
+        blocks += ceil_div(bytes[i] / 4, quads ? kCopyWords : kCopyLoose);
+        // (blocks of one launch stay far below 2^31: a copy adds at most 2^21 of them)
         if (++filled == kBatchCopies)
             if (int rc = flush()) return rc;
     }

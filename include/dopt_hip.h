@@ -89,7 +89,7 @@ int dopt_hip_copy_h2d_async(void *dst, const void *pinned_src, size_t bytes);
    reader).  No counterpart in the reference, whose uploads block (cuda/package.d:172-176). */
 int dopt_hip_copy_h2d_beside(void *dst, const void *pinned_src, size_t bytes);
 int dopt_hip_upload_join(void);
-/* n device-to-device copies, in order; copies of at most 64 KiB share kernel launches.  Stands
+/* n device-to-device copies, in order; up to 128 of them share a kernel launch.  Stands
    for the loop of cuMemcpy calls that hands a plan's outputs to the caller's buffers
    (cuda/package.d:419-422): most of them are a few hundred bytes of batch-norm statistics. */
 int dopt_hip_copy_d2d_batch(int n, void *const *dst, const void *const *src, const size_t *bytes);
