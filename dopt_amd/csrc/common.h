@@ -8,6 +8,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <string>
+#include <vector>
 
 #include "../../include/dopt_hip.h"
 
@@ -80,8 +81,32 @@ int num_cus();
 inline size_t ceil_div(size_t a, size_t b) { return (a + b - 1) / b; }
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// rtc_ops.cpp: the same pointwise program over many tensors as one launch (more, when their addresses do not fit a launch's
+// arguments).  Operand k < kind.size() of a node is input k - kind 0 an n-element tensor, 1 one element - and operand
+// kind.size() + j is node j; `outs` are the nodes that are stored, each to a buffer of its own.  Every node rounds by itself, as
+// the kernel of its operation does.
+struct PointwiseProgram {
+    std::vector<unsigned char> kind;
+    struct Node { std::string op; int lhs, rhs; };
+    std::vector<Node> nodes;
+    std::vector<int> outs;
+};
+struct PointwiseItem {
+    size_t n;
+    std::vector<const void *> in;   // one per input of the program
+    std::vector<void *> out;
+};
+constexpr int kGroupInputs = 48, kGroupNodes = 64, kGroupOuts = 8;
+int pointwise_group(const PointwiseProgram &program, const std::vector<PointwiseItem> &items);
+int pointwise_group_compile_only(const PointwiseProgram &program, const char *arch);
+
+// rtc_ops.cpp: out[i] = the sum of the squares of the n[i] (more than 64) values at in[i], each the value that
+// dopt_hip_reduce_squares gives.
+int reduce_squares_batch(int count, const float *const *in, const size_t *n, float *const *out);
+
 // hipRTC: compile `source` (once per distinct `key`) and return the named kernel.
 int rtc_get(const std::string &key, const std::string &source, const char *kernel_name, hipFunction_t *fn);
+bool rtc_find(const std::string &key, hipFunction_t *fn);   // a kernel compiled before (its source need not be put together again)
 int rtc_compile_only(const std::string &source, const char *arch, std::string *log);
 int rtc_launch(hipFunction_t fn, unsigned grid, unsigned block, void **args);
 

@@ -554,6 +554,10 @@ std::unique_ptr<HIPKernel> make_fused(const Graph &g, int id, int kind, void *ex
     }
     // batchNormGrad, with reluGrad folded in (kind 3: inputs [dy, y, x, scale]; else [dy, x, scale])
     // and/or the bias gradient of the preceding addBias written to `extra`
+    if ((kind != 0 && kind != 3) || op.opType != "batchNormGrad" || !need_deps(op, 3)) {
+        fail(DOPT_HIP_ERR_RUNTIME, "operation '%s' is part of another operation's kernel", op.opType.c_str());
+        return nullptr;
+    }
     size_t N, C, inner;
     nci(g.ops[op.deps[1]].shape, &N, &C, &inner);
     const bool relu = kind == 3;
@@ -580,7 +584,7 @@ struct HIPPlan::Builder {
     std::vector<Alias> alias;
     // inputsOf[id]: the operations whose buffers feed id's kernel (its deps, unless fused);
     // fusedKind[id]: 1 conv+bias, 2 bn+relu, 3 relugrad+bngrad, 6 matmul with transposes, 7 pointwise chain,
-    // 8 maxpoolgrad+relugrad+bngrad, 9 matmul+relugrad, 10 member of a tiny run, 11 sum of squares
+    // 8 maxpoolgrad+relugrad+bngrad, 9 matmul+relugrad, 10 member of a tiny run, 11 sum of squares, 12 member of a group
     std::vector<std::vector<int>> inputsOf;
     std::vector<int> fusedKind;
     std::vector<std::unique_ptr<HIPKernel>> prebuilt;
@@ -596,7 +600,8 @@ struct HIPPlan::Builder {
     std::vector<int> pairLead;                  // the operation of such a pair that comes first in the order -> the backward-data op
     std::vector<char> pairLater;                // the operation of such a pair that comes second: no step of its own
     std::vector<char> absorbed;
-    std::vector<std::vector<int>> tinyWrites;   // last member of a run of tiny operations -> the other members
+    std::vector<char> groupReads;               // operations whose buffers a group's kernel reads: they must be stored
+    std::vector<std::vector<int>> tinyWrites;   // last member of a run of tiny operations or of a group -> the others whose buffers it fills
     std::vector<char> needed;
     // late: the copy is made right in front of its first reader instead of at the start of the run
     struct Prepack { int op, filter; int bwd; dopt_hip_conv_desc d; void *buf; bool owner, late; };
@@ -615,7 +620,7 @@ struct HIPPlan::Builder {
           inputsOf((size_t)nops), fusedKind((size_t)nops, 0), prebuilt((size_t)nops), prebuiltLabel((size_t)nops),
           live((size_t)nops, 0), uses((size_t)nops), exposed((size_t)nops), biasGradOf((size_t)nops, -1), poolOf((size_t)nops, -1), pairOf((size_t)nops, -1), pairLead((size_t)nops, -1),
           pairLater((size_t)nops, 0),
-          absorbed((size_t)nops, 0), tinyWrites((size_t)nops), needed((size_t)nops, 0), packOf((size_t)nops, -1), mmInfo((size_t)nops)
+          absorbed((size_t)nops, 0), groupReads((size_t)nops, 0), tinyWrites((size_t)nops), needed((size_t)nops, 0), packOf((size_t)nops, -1), mmInfo((size_t)nops)
     {
     }
 
@@ -638,6 +643,7 @@ struct HIPPlan::Builder {
     void fuseDenseLayers();
     void fuseDenseBackward();
     bool plainProduct(int id, MatmulInfo *mi, bool sole_reader) const;
+    void formGroups();
     void formTinyRuns();
     void fuseSquareSums();
     void formChains();
@@ -977,6 +983,204 @@ void HIPPlan::Builder::fuseDenseBackward()
     }
 }
 
+// The tail of a training graph is the same for every parameter: the gradient's penalty term and the update rule, pointwise
+// operations whose values nothing reads but other such operations and the plan's outputs (online/source/dopt/online/*.d build
+// the rules that way).  Nothing waits for them, so they can all run last: each connected piece of them becomes a program
+// that reads every operand once and stores only what leaves the plan, and pieces with the same program, one per parameter,
+// become one step (pointwise_group): one or two launches for the update of a network instead of several per parameter.
+// One-element values (a rate, a bias correction) do not connect pieces.  Where they are pointwise values of one-element
+// tensors and only pieces read them, every piece computes them again from those; else they are operands.
+// A step stands where the last of its members stood; everything it reads is older.
+void HIPPlan::Builder::formGroups()
+{
+    auto one_element = [&](int id) { return g.ops[id].volume() == 1 && g.ops[id].dtype == DOPT_HIP_F32; };
+    // a column times a row of which one is a single element (the reference's scalar broadcast, core/ops/basic.d:370-381)
+    auto scaling = [&](const Operation &o) {
+        if (o.opType != "matmul" || o.deps.size() != 2 || o.rank() != 2) return false;
+        const Operation &l = g.ops[o.deps[0]], &r = g.ops[o.deps[1]];
+        return l.rank() == 2 && r.rank() == 2 && l.shape[1] == 1 && r.shape[0] == 1 && (o.shape[0] == 1 || o.shape[1] == 1);
+    };
+    auto is_node = [&](int id) {
+        const Operation &o = g.ops[id];
+        if (!live[id] || alias[id].source >= 0 || fusedKind[id] || prebuilt[id] || o.dtype != DOPT_HIP_F32 || o.volume() < 2) return false;
+        for (int d : o.deps)
+            if (g.ops[d].dtype != DOPT_HIP_F32) return false;
+        if (scaling(o)) return true;
+        const int arity = dopt_hip_pointwise_arity(o.opType.c_str());
+        if (arity <= 0 || arity != (int)o.deps.size() || o.opType == "reluGrad") return false;
+        for (int d : o.deps)
+            if (g.ops[d].volume() != o.volume()) return false;
+        return true;
+    };
+    std::vector<char> last((size_t)nops, 0);   // operations that may run after everything else
+    for (auto it = p->mOps.rbegin(); it != p->mOps.rend(); ++it) {
+        const int id = *it;
+        if (!is_node(id)) continue;
+        bool ok = isOutput(id) || !uses[id].empty();
+        for (const Use &u : uses[id]) ok = ok && last[u.op] && u.off == 0 && g.ops[u.op].volume() == g.ops[id].volume();
+        last[id] = ok;
+    }
+    // one-element values that pieces compute for themselves: all that reads one is a piece, as the element it scales or
+    // broadcasts, or another such value
+    std::vector<char> scalar((size_t)nops, 0);
+    auto scales = [&](const Use &u) {
+        const Operation &o = g.ops[u.op];
+        return last[u.op] && scaling(o) && u.off == 0 && g.ops[o.deps[(size_t)u.slot]].volume() == 1;
+    };
+    for (auto it = p->mOps.rbegin(); it != p->mOps.rend(); ++it) {
+        const int id = *it;
+        const Operation &o = g.ops[id];
+        if (!live[id] || alias[id].source >= 0 || fusedKind[id] || prebuilt[id] || !one_element(id) || isOutput(id) || uses[id].empty()) continue;
+        const int arity = dopt_hip_pointwise_arity(o.opType.c_str());
+        bool ok = arity > 0 && arity == (int)o.deps.size() && o.opType != "reluGrad";
+        for (int d : o.deps) ok = ok && one_element(d);
+        for (const Use &u : uses[id]) {
+            const Operation &ro = g.ops[u.op];
+            if (ro.opType == "repeat" && ro.deps.size() == 1 && alias[u.op].source < 0 && !isOutput(u.op) && !fusedKind[u.op] && u.off == 0) {
+                for (const Use &v : uses[u.op]) ok = ok && last[v.op] && v.off == 0 && g.ops[v.op].volume() == ro.volume();
+                continue;
+            }
+            ok = ok && u.off == 0 && (scales(u) || scalar[u.op]);
+        }
+        scalar[id] = ok;
+    }
+    // connected pieces, in execution order
+    std::vector<int> parent((size_t)nops);
+    for (int i = 0; i < nops; i++) parent[i] = i;
+    std::function<int(int)> find = [&](int i) { return parent[i] == i ? i : parent[i] = find(parent[i]); };
+    for (int id : p->mOps) {
+        if (!last[id]) continue;
+        for (int d : g.ops[id].deps) {
+            size_t off;
+            const int r = root(d, &off);
+            if (last[r] && g.ops[r].volume() == g.ops[id].volume()) parent[find(r)] = find(id);
+        }
+    }
+    std::vector<std::vector<int>> pieces;
+    std::vector<int> pieceOf((size_t)nops, -1);
+    for (int id : p->mOps) {
+        if (!last[id]) continue;
+        int &k = pieceOf[find(id)];
+        if (k < 0) {
+            k = (int)pieces.size();
+            pieces.emplace_back();
+        }
+        pieces[(size_t)k].push_back(id);
+    }
+    struct Group { PointwiseProgram program; std::vector<size_t> members; std::vector<std::vector<int>> inputs, outs; };
+    std::vector<Group> groups;
+    std::unordered_map<std::string, size_t> byProgram;
+    for (size_t k = 0; k < pieces.size(); k++) {
+        PointwiseProgram prog;
+        std::vector<int> inputs;              // operations whose buffers the piece reads
+        std::unordered_map<int, int> nodeOf;
+        std::function<int(int)> add;          // an operation as a node of the program
+        auto input = [&](int op, int kind) {
+            for (size_t i = 0; i < inputs.size(); i++)
+                if (inputs[i] == op && prog.kind[i] == kind) return (int)i;
+            inputs.push_back(op);
+            prog.kind.push_back((unsigned char)kind);
+            return (int)inputs.size() - 1;
+        };
+        std::function<int(int)> operand = [&](int dep) {   // >= 0: an input; -2 and below: a node
+            size_t off, soff;
+            const int r = root(dep, &off);
+            auto at = nodeOf.find(r);
+            if (at != nodeOf.end() && off == 0) return -2 - at->second;
+            const Operation &ro = g.ops[r];
+            if (ro.opType == "repeat" && ro.deps.size() == 1 && off == 0 && alias[r].source < 0 && one_element(ro.deps[0]) &&
+                g.ops[root(ro.deps[0], &soff)].dtype == DOPT_HIP_F32)
+                return operand(ro.deps[0]);
+            if (scalar[r] && off == 0) return -2 - add(r);
+            return input(dep, g.ops[dep].volume() == 1 ? 1 : 0);
+        };
+        add = [&](int id) {
+            const Operation &o = g.ops[id];
+            PointwiseProgram::Node node{o.opType == "matmul" ? "mul" : o.opType, 0, 0};
+            node.lhs = operand(o.deps[0]);
+            node.rhs = o.deps.size() > 1 ? operand(o.deps[1]) : node.lhs;
+            prog.nodes.push_back(node);
+            return nodeOf[id] = (int)prog.nodes.size() - 1;
+        };
+        std::vector<int> outOps;
+        for (int id : pieces[k]) {
+            const int node = add(id);
+            if (!isOutput(id)) continue;
+            prog.outs.push_back(node);
+            outOps.push_back(id);
+        }
+        const int nin = (int)inputs.size();
+        if (nin > kGroupInputs || prog.nodes.size() > (size_t)kGroupNodes || prog.outs.size() > (size_t)kGroupOuts) continue;   // other passes take its operations
+        std::string key;
+        for (unsigned char kind : prog.kind) key += kind ? 's' : 'v';
+        for (PointwiseProgram::Node &n : prog.nodes) {
+            if (n.lhs < 0) n.lhs = nin + (-2 - n.lhs);
+            if (n.rhs < 0) n.rhs = nin + (-2 - n.rhs);
+            key += "|" + n.op + "," + std::to_string(n.lhs) + "," + std::to_string(n.rhs);
+        }
+        for (int o : prog.outs) key += ">" + std::to_string(o);
+        const auto seen = byProgram.emplace(key, groups.size());
+        if (seen.second) groups.push_back(Group{prog, {}, {}, {}});
+        groups[seen.first->second].members.push_back(k);
+        groups[seen.first->second].inputs.push_back(inputs);
+        groups[seen.first->second].outs.push_back(outOps);
+    }
+    std::vector<int> pos((size_t)nops, -1);
+    for (size_t i = 0; i < p->mOps.size(); i++) pos[p->mOps[i]] = (int)i;
+    for (Group &gr : groups) {
+        // A single piece gains nothing as a group of one node; a short one on a tiny tensor costs less as part of a run of
+        // tiny operations (0.4 us a node) than as a launch (4 us).
+        const size_t nodes = gr.program.nodes.size(), volume = g.ops[pieces[gr.members[0]][0]].volume();
+        if (gr.members.size() == 1 && (nodes < 2 || (volume <= DOPT_HIP_TINY_ELEMS && nodes < 10))) continue;
+        struct Item { size_t n; std::vector<int> in, out; };   // places in the step's inputs; a result of -1 is the step's own
+        int lead = -1;
+        for (size_t k : gr.members)
+            for (int id : pieces[k])
+                if (lead < 0 || pos[id] > pos[lead]) lead = id;   // (nothing reads the last one, so it is an output)
+        std::vector<int> ins;
+        std::unordered_map<int, int> inAt;
+        auto place = [&](int op) {
+            const auto seen = inAt.emplace(op, (int)ins.size());
+            if (seen.second) ins.push_back(op);
+            return seen.first->second;
+        };
+        std::vector<Item> layout;
+        tinyWrites[lead].clear();
+        for (size_t m = 0; m < gr.members.size(); m++) {
+            const std::vector<int> &piece = pieces[gr.members[m]];
+            Item it{g.ops[piece[0]].volume(), {}, {}};
+            for (int op : gr.inputs[m]) {
+                size_t off;
+                groupReads[root(op, &off)] = 1;   // (also through a scalar that the piece computes for itself: not among its `uses`)
+                it.in.push_back(place(op));
+            }
+            for (int id : gr.outs[m]) {
+                it.out.push_back(id == lead ? -1 : place(id));
+                if (id == lead) continue;
+                tinyWrites[lead].push_back(id);
+                absorbed[id] = 1;
+            }
+            for (int id : piece) {
+                fusedKind[id] = 12;
+                inputsOf[id] = {lead};
+            }
+            layout.push_back(std::move(it));
+        }
+        inputsOf[lead] = ins;
+        const PointwiseProgram program = gr.program;
+        prebuilt[lead] = make([=](const std::vector<const void *> &in, void *out) {
+            std::vector<PointwiseItem> items(layout.size());
+            for (size_t m = 0; m < layout.size(); m++) {
+                items[m].n = layout[m].n;
+                for (int i : layout[m].in) items[m].in.push_back(in[(size_t)i]);
+                for (int o : layout[m].out) items[m].out.push_back(o < 0 ? out : const_cast<void *>(in[(size_t)o]));
+            }
+            return pointwise_group(program, items);
+        });
+        prebuiltLabel[lead] = "pointwise*" + std::to_string(nodes) + "x" + std::to_string(layout.size());
+    }
+}
+
 // Runs of operations on tiny tensors (a softmax over ten classes, the loss behind it, the scalars of an update rule):
 // each would be a kernel that lasts as long as the gap between two kernels.  Walking the order, operations that
 // dopt_hip_tiny_graph can compute (every tensor involved of at most DOPT_HIP_TINY_ELEMS fp32 values) collect into a
@@ -1184,8 +1388,11 @@ void HIPPlan::Builder::formTinyRuns()
 // (dopt_hip_reduce_squares), the product rounded to fp32 before it is added and the sums in the reduction's own order,
 // so the value is the one the two kernels give; the product is never stored.  Tensors small enough for a tiny run have
 // been taken by one already (DOPT_HIP_PLAN_FUSE).
+// The penalties of a whole network are one step (reduce_squares_batch) where the first of them stood: they read variables and
+// constants, which no step writes.
 void HIPPlan::Builder::fuseSquareSums()
 {
+    std::vector<int> whole;   // such sums over whole variables or constants
     for (int id : p->mOps) {
         const Operation &op = g.ops[id];
         if (!live[id] || alias[id].source >= 0 || fusedKind[id] || prebuilt[id] || op.opType != "sum" || op.deps.size() != 1 ||
@@ -1220,7 +1427,37 @@ void HIPPlan::Builder::fuseSquareSums()
                                            (float *)out);
         });
         prebuiltLabel[id] = "mul+sum";
+        size_t xoff;
+        if (op.volume() == 1 && mo.volume() > 64 && mo.volume() < (size_t)1 << 40 && is_leaf(g.ops[root(mo.deps[0], &xoff)])) whole.push_back(id);
     }
+    if (whole.size() < 3) return;   // a pair stays two steps, which a profile tells apart
+    const int lead = whole[0];
+    std::vector<int> ins;
+    std::vector<size_t> counts;
+    for (int id : whole) {
+        ins.push_back(inputsOf[id][0]);
+        counts.push_back(g.ops[inputsOf[id][0]].volume());
+    }
+    tinyWrites[lead].assign(whole.begin() + 1, whole.end());
+    for (int id : tinyWrites[lead]) {
+        ins.push_back(id);
+        inputsOf[id] = {lead};
+        prebuilt[id].reset();
+        prebuiltLabel[id].clear();
+        absorbed[id] = 1;   // keeps its buffer, filled by the one step
+    }
+    inputsOf[lead] = ins;
+    const size_t n = whole.size();
+    prebuilt[lead] = make([=](const std::vector<const void *> &in, void *out) {
+        std::vector<const float *> from(n);
+        std::vector<float *> to(n);
+        for (size_t i = 0; i < n; i++) {
+            from[i] = (const float *)in[i];
+            to[i] = i == 0 ? (float *)out : (float *)const_cast<void *>(in[n + i - 1]);
+        }
+        return reduce_squares_batch((int)n, from.data(), counts.data(), to.data());
+    });
+    prebuiltLabel[lead] = "mul+sum*" + std::to_string(n);
 }
 
 void HIPPlan::Builder::formChains()
@@ -1265,7 +1502,7 @@ void HIPPlan::Builder::formChains()
         const int id = *it;
         if (!is_pw(id)) continue;
         int target = -1;
-        bool joins = !isOutput(id) && !uses[id].empty();
+        bool joins = !isOutput(id) && !uses[id].empty() && !groupReads[id];
         auto reader_joins = [&](const Use &u, size_t volume) {   // the reader is a member of the one chain, and reads all of it
             if (chainOf[u.op] < 0 || u.off != 0 || g.ops[u.op].volume() != volume) joins = false;
             else if (g.ops[u.op].opType == "reluGrad" && u.slot == 1) joins = false;   // the y operand is not part of the node
@@ -2102,6 +2339,7 @@ int HIPPlan::create(Graph *graph, const std::vector<int> &outputs, unsigned flag
         b.foldTransposes();
         b.fuseDenseLayers();
         b.fuseDenseBackward();
+        b.formGroups();
         b.formTinyRuns();
         b.fuseSquareSums();
         b.formChains();

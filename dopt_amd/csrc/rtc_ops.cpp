@@ -4,6 +4,7 @@
 // independent loads in flight per lane and no host synchronisation.  Semantics follow the CPU
 // evaluator, cpu/source/dopt/cpu/math.d:312-437 (pointwise), :90-247 (sum / maxElement) and
 // :249-310 (argmin).
+#include <algorithm>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -230,6 +231,113 @@ __device__ inline int dopt_ipow(int x, int n)
     return s;
 }
 
+// ------------------------------------------------------------------------------ pointwise groups
+// One program over many tensors: a workgroup finds its tensor by its block number and computes 1024 elements of it, every
+// operand read once and every result stored once.  Bound by memory traffic where the tensors are large and by one kernel
+// boundary where they are small.  The arguments travel by value (at most 4 KB): addresses, counts and first block per
+// tensor, and the single elements that all tensors share.  16-byte loads for tensors whose operands all allow them.
+struct GroupShape {
+    std::vector<int> own, shared;   // inputs with an address per tensor; single elements at one address for all
+    int nptr = 0, items = 0;        // addresses per tensor; tensors per launch
+};
+
+GroupShape group_shape(const PointwiseProgram &p, const std::vector<char> &common)
+{
+    GroupShape g;
+    for (int k = 0; k < (int)p.kind.size(); k++) (p.kind[k] == 1 && common[k] ? g.shared : g.own).push_back(k);
+    g.nptr = (int)(g.own.size() + p.outs.size());
+    g.items = std::min(64, (4000 - 8 * (int)g.shared.size()) / (8 * g.nptr + 16));   // (64: a lane a tensor)
+    return g;
+}
+
+std::string group_key(const PointwiseProgram &p, const std::vector<char> &common)
+{
+    std::string key = "group:f32";
+    for (size_t k = 0; k < p.kind.size(); k++) key += p.kind[k] == 0 ? ":v" : common[k] ? ":S" : ":s";
+    for (const auto &n : p.nodes) key += "|" + n.op + "," + std::to_string(n.lhs) + "," + std::to_string(n.rhs);
+    for (int o : p.outs) key += ">" + std::to_string(o);
+    return key;
+}
+
+std::string group_source(const PointwiseProgram &p, const GroupShape &g)
+{
+    const int nin = (int)p.kind.size(), nout = (int)p.outs.size(), nown = (int)g.own.size();
+    auto str = [](int v) { return std::to_string(v); };
+    std::string s = "typedef float T;\ntypedef T T4 __attribute__((ext_vector_type(4)));\n";
+    s += "#define ITEMS " + str(g.items) + "\n#define PTRS " + str(g.nptr) + "\n#define SHARED " + str(std::max(1, (int)g.shared.size())) + "\n";
+    s += "struct Args {\n    T *p[ITEMS * PTRS];\n    size_t n[ITEMS];\n    const T *shared[SHARED];\n    unsigned first[ITEMS];   // bit 31: quads\n    int items;\n};\n";
+    for (int j = 0; j < (int)p.nodes.size(); j++) s += "__device__ inline T f" + str(j) + "(T a, T b) { return (T)(" + find_op(p.nodes[j].op.c_str())->expr_f32 + "); }\n";
+    std::vector<int> own_of(nin, -1), shared_of(nin, -1);
+    for (int i = 0; i < nown; i++) own_of[g.own[i]] = i;
+    for (int i = 0; i < (int)g.shared.size(); i++) shared_of[g.shared[i]] = i;
+    // nodes whose operands are all single elements: the same for every element, computed once a thread
+    std::vector<char> single(p.nodes.size(), 0);
+    auto is_single = [&](int k) { return k < nin ? p.kind[k] == 1 : single[k - nin] != 0; };
+    for (size_t j = 0; j < p.nodes.size(); j++) single[j] = is_single(p.nodes[j].lhs) && is_single(p.nodes[j].rhs);
+    auto body = [&](const char *lane, const char *indent) {
+        std::string b = std::string(indent) + "{\n";
+        auto operand = [&](int k) -> std::string {
+            if (k >= nin) return "t" + str(k - nin);
+            return p.kind[k] == 1 ? "s" + str(k) : "x" + str(k) + lane;
+        };
+        for (int j = 0; j < (int)p.nodes.size(); j++)
+            if (!single[j]) b += std::string(indent) + "    const T t" + str(j) + " = f" + str(j) + "(" + operand(p.nodes[j].lhs) + ", " + operand(p.nodes[j].rhs) + ");\n";
+        for (int o = 0; o < nout; o++) b += std::string(indent) + "    r" + str(o) + lane + " = t" + str(p.outs[o]) + ";\n";
+        return b + indent + "}\n";
+    };
+    auto element = [&](const char *indent) {   // element e
+        std::string b;
+        for (int k = 0; k < nin; k++)
+            if (p.kind[k] == 0) b += std::string(indent) + "const T x" + str(k) + " = p[" + str(own_of[k]) + "][e];\n";
+        for (int o = 0; o < nout; o++) b += std::string(indent) + "T r" + str(o) + ";\n";
+        b += body("", indent);
+        for (int o = 0; o < nout; o++) b += std::string(indent) + "p[" + str(nown + o) + "][e] = r" + str(o) + ";\n";
+        return b;
+    };
+    s += R"SRC(
+extern "C" __global__ __launch_bounds__(256) void group_k(const Args a)
+{
+    const int lane = threadIdx.x & 63;
+    const unsigned start = lane < a.items ? a.first[lane] & 0x7fffffffu : 0xffffffffu;
+    const int item = __builtin_popcountll(__ballot(start <= blockIdx.x)) - 1;
+    T *const *p = a.p + item * PTRS;
+    const size_t n = a.n[item];
+    const size_t block = blockIdx.x - (a.first[item] & 0x7fffffffu);
+)SRC";
+    for (int k = 0; k < nin; k++)
+        if (p.kind[k] == 1) s += "    const T s" + str(k) + " = " + (shared_of[k] >= 0 ? "a.shared[" + str(shared_of[k]) + "][0]" : "p[" + str(own_of[k]) + "][0]") + ";\n";
+    for (int j = 0; j < (int)p.nodes.size(); j++) {
+        auto operand = [&](int k) { return (k >= nin ? "t" + str(k - nin) : "s" + str(k)); };
+        if (single[j]) s += "    const T t" + str(j) + " = f" + str(j) + "(" + operand(p.nodes[j].lhs) + ", " + operand(p.nodes[j].rhs) + ");\n";
+    }
+    s += "    if (a.first[item] >> 31) {\n        const size_t n4 = n >> 2, q = block * 256 + threadIdx.x;\n        if (q < n4) {\n";
+    for (int k = 0; k < nin; k++)
+        if (p.kind[k] == 0) s += "            const T4 x" + str(k) + " = ((const T4 *)p[" + str(own_of[k]) + "])[q];\n";
+    for (int o = 0; o < nout; o++) s += "            T4 r" + str(o) + ";\n";
+    for (const char *lane : {".x", ".y", ".z", ".w"}) s += body(lane, "            ");
+    for (int o = 0; o < nout; o++) s += "            ((T4 *)p[" + str(nown + o) + "])[q] = r" + str(o) + ";\n";
+    s += "        } else if (q < n4 + (n & 3)) {   // the last n % 4 elements\n            const size_t e = 3 * n4 + q;\n" + element("            ");
+    s += "        }\n    } else {\n        for (size_t e = block * 1024 + threadIdx.x; e < n && e < block * 1024 + 1024; e += 256) {\n" + element("            ");
+    return s + "        }\n    }\n}\n";
+}
+
+// Whether the program is one that group_source can write; the message says what is wrong.
+int group_check(const PointwiseProgram &p)
+{
+    const int nin = (int)p.kind.size();
+    DOPT_REQUIRE(nin >= 1 && nin <= kGroupInputs && !p.nodes.empty() && (int)p.nodes.size() <= kGroupNodes && !p.outs.empty() &&
+                     (int)p.outs.size() <= kGroupOuts,
+                 "pointwise_group: %d inputs, %zu nodes, %zu results", nin, p.nodes.size(), p.outs.size());
+    for (size_t j = 0; j < p.nodes.size(); j++) {
+        const OpInfo *info = find_op(p.nodes[j].op.c_str());
+        if (!info) return fail(DOPT_HIP_ERR_UNSUPPORTED, "pointwise_group: unknown operation '%s'", p.nodes[j].op.c_str());
+        DOPT_REQUIRE(p.nodes[j].lhs >= 0 && p.nodes[j].lhs < nin + (int)j && p.nodes[j].rhs >= 0 && p.nodes[j].rhs < nin + (int)j,
+                     "pointwise_group: node %zu reads an operand that is not computed before it", j);
+    }
+    for (int o : p.outs) DOPT_REQUIRE(o >= 0 && o < (int)p.nodes.size(), "pointwise_group: no node %d", o);
+    return DOPT_HIP_OK;
+}
+
 // ------------------------------------------------------------------------------ reductions
 
 const char *kReduceBody = R"SRC(
@@ -268,15 +376,11 @@ __device__ inline T block_reduce(T v)
     return v;  // valid in thread 0
 }
 
-// Contiguous rows: block (row o, chunk c) reduces in[o*R + c*chunk ... ) into out[o*nchunks + c].
-extern "C" __global__ __launch_bounds__(BLOCK) void red_rows(const T *in, T *out, size_t R, size_t chunk,
-                                                              size_t nchunks)
+// One thread's part of row[start .. end): element by element, or by quads (start a multiple of four; end too), loaded whole
+// from a 16-byte aligned row, word by word from any other (a view into a larger tensor), in the same order of sums, so that a
+// value does not depend on where its operand happens to start.
+__device__ inline T fold_words(const T *row, size_t start, size_t end)
 {
-    const size_t o = blockIdx.x / nchunks, c = blockIdx.x % nchunks;
-    const size_t start = c * chunk;
-    size_t end = start + chunk;
-    if (end > R) end = R;
-    const T *row = in + o * R;
     T acc0 = (T)(IDENT), acc1 = (T)(IDENT), acc2 = (T)(IDENT), acc3 = (T)(IDENT);
     size_t i = start + threadIdx.x;
     for (; i + 3 * BLOCK < end; i += 4 * BLOCK) {
@@ -287,72 +391,76 @@ extern "C" __global__ __launch_bounds__(BLOCK) void red_rows(const T *in, T *out
         acc3 = combine(acc3, v3);
     }
     for (; i < end; i += BLOCK) acc0 = combine(acc0, PRE(row[i]));
-    T acc = combine(combine(acc0, acc1), combine(acc2, acc3));
-    acc = block_reduce(acc);
-    if (threadIdx.x == 0) out[blockIdx.x] = acc;
+    return combine(combine(acc0, acc1), combine(acc2, acc3));
 }
 
-// The same with 128-bit loads: R and chunk are multiples of 4 and `in` is 16-byte aligned.
-extern "C" __global__ __launch_bounds__(BLOCK) void red_rows4(const T *in, T *out, size_t R, size_t chunk,
-                                                               size_t nchunks)
+__device__ inline T4 quad_whole(const T *row, size_t q) { return pre4(((const T4 *)row)[q]); }
+__device__ inline T4 quad_words(const T *row, size_t q)
 {
-    const size_t o = blockIdx.x / nchunks, c = blockIdx.x % nchunks;
-    const size_t start = c * chunk;
-    size_t end = start + chunk;
-    if (end > R) end = R;
-    const T4 *row = (const T4 *)(in + o * R);
-    const size_t q0 = start / 4, q1 = end / 4;
-    T acc0 = (T)(IDENT), acc1 = (T)(IDENT), acc2 = (T)(IDENT), acc3 = (T)(IDENT);
-    size_t i = q0 + threadIdx.x;
-    for (; i + 3 * BLOCK < q1; i += 4 * BLOCK) {
-        T4 v0 = pre4(row[i]), v1 = pre4(row[i + BLOCK]), v2 = pre4(row[i + 2 * BLOCK]), v3 = pre4(row[i + 3 * BLOCK]);
-        acc0 = combine(acc0, combine(combine(v0.x, v0.y), combine(v0.z, v0.w)));
-        acc1 = combine(acc1, combine(combine(v1.x, v1.y), combine(v1.z, v1.w)));
-        acc2 = combine(acc2, combine(combine(v2.x, v2.y), combine(v2.z, v2.w)));
-        acc3 = combine(acc3, combine(combine(v3.x, v3.y), combine(v3.z, v3.w)));
-    }
-    for (; i < q1; i += BLOCK) {
-        T4 v0 = pre4(row[i]);
-        acc0 = combine(acc0, combine(combine(v0.x, v0.y), combine(v0.z, v0.w)));
-    }
-    T acc = combine(combine(acc0, acc1), combine(acc2, acc3));
-    acc = block_reduce(acc);
-    if (threadIdx.x == 0) out[blockIdx.x] = acc;
-}
-
-// The same order of sums from a buffer that is not 16-byte aligned (a view into a larger tensor): four 32-bit loads
-// per quad, so that a value does not depend on where its operand happens to start.
-__device__ inline T4 ld4(const T *p)
-{
+    const T *p = row + 4 * q;
     T4 r;
     r.x = PRE(p[0]); r.y = PRE(p[1]); r.z = PRE(p[2]); r.w = PRE(p[3]);
     return r;
 }
-extern "C" __global__ __launch_bounds__(BLOCK) void red_rows4u(const T *in, T *out, size_t R, size_t chunk,
-                                                                size_t nchunks)
+
+#define FOLD_QUADS(name, LOAD)                                                                          \
+    __device__ inline T name(const T *row, size_t start, size_t end)                                    \
+    {                                                                                                   \
+        const size_t q1 = end / 4;                                                                      \
+        T acc0 = (T)(IDENT), acc1 = (T)(IDENT), acc2 = (T)(IDENT), acc3 = (T)(IDENT);                   \
+        size_t i = start / 4 + threadIdx.x;                                                             \
+        for (; i + 3 * BLOCK < q1; i += 4 * BLOCK) {                                                    \
+            T4 v0 = LOAD(row, i), v1 = LOAD(row, i + BLOCK), v2 = LOAD(row, i + 2 * BLOCK), v3 = LOAD(row, i + 3 * BLOCK); \
+            acc0 = combine(acc0, combine(combine(v0.x, v0.y), combine(v0.z, v0.w)));                    \
+            acc1 = combine(acc1, combine(combine(v1.x, v1.y), combine(v1.z, v1.w)));                    \
+            acc2 = combine(acc2, combine(combine(v2.x, v2.y), combine(v2.z, v2.w)));                    \
+            acc3 = combine(acc3, combine(combine(v3.x, v3.y), combine(v3.z, v3.w)));                    \
+        }                                                                                               \
+        for (; i < q1; i += BLOCK) {                                                                    \
+            T4 v0 = LOAD(row, i);                                                                       \
+            acc0 = combine(acc0, combine(combine(v0.x, v0.y), combine(v0.z, v0.w)));                    \
+        }                                                                                               \
+        return combine(combine(acc0, acc1), combine(acc2, acc3));                                       \
+    }
+FOLD_QUADS(fold_quads, quad_whole)
+FOLD_QUADS(fold_quads_loose, quad_words)
+
+// Contiguous rows: block (row o, chunk c) reduces in[o*R + c*chunk ... ) into out[o*nchunks + c].  rows4 and rows4u: R and
+// chunk are multiples of 4; rows4: `in` is 16-byte aligned.
+#define RED_ROWS(name, FOLD)                                                                            \
+    extern "C" __global__ __launch_bounds__(BLOCK) void name(const T *in, T *out, size_t R, size_t chunk, size_t nchunks) \
+    {                                                                                                   \
+        const size_t o = blockIdx.x / nchunks, c = blockIdx.x % nchunks;                                \
+        const size_t start = c * chunk, end = start + chunk < R ? start + chunk : R;                    \
+        const T acc = block_reduce(FOLD(in + o * R, start, end));                                       \
+        if (threadIdx.x == 0) out[blockIdx.x] = acc;                                                    \
+    }
+RED_ROWS(red_rows, fold_words)
+RED_ROWS(red_rows4, fold_quads)
+RED_ROWS(red_rows4u, fold_quads_loose)
+
+// Whole tensors, many in one launch: a block finds its tensor by its number and folds the chunk that block of red_rows /
+// red_rows4 / red_rows4u would fold (mode 0, 1, 2), to where its result goes (out + the chunk's number).
+#define ITEMS 64
+struct Rows {
+    const T *in[ITEMS];
+    T *out[ITEMS];
+    size_t R[ITEMS];
+    unsigned chunk[ITEMS];
+    unsigned first[ITEMS];   // bits 30 and 31: the mode
+    int items;
+};
+extern "C" __global__ __launch_bounds__(BLOCK) void red_batch(const Rows a)
 {
-    const size_t o = blockIdx.x / nchunks, c = blockIdx.x % nchunks;
-    const size_t start = c * chunk;
-    size_t end = start + chunk;
-    if (end > R) end = R;
-    const T *row = in + o * R;
-    const size_t q0 = start / 4, q1 = end / 4;
-    T acc0 = (T)(IDENT), acc1 = (T)(IDENT), acc2 = (T)(IDENT), acc3 = (T)(IDENT);
-    size_t i = q0 + threadIdx.x;
-    for (; i + 3 * BLOCK < q1; i += 4 * BLOCK) {
-        T4 v0 = ld4(row + 4 * i), v1 = ld4(row + 4 * (i + BLOCK)), v2 = ld4(row + 4 * (i + 2 * BLOCK)), v3 = ld4(row + 4 * (i + 3 * BLOCK));
-        acc0 = combine(acc0, combine(combine(v0.x, v0.y), combine(v0.z, v0.w)));
-        acc1 = combine(acc1, combine(combine(v1.x, v1.y), combine(v1.z, v1.w)));
-        acc2 = combine(acc2, combine(combine(v2.x, v2.y), combine(v2.z, v2.w)));
-        acc3 = combine(acc3, combine(combine(v3.x, v3.y), combine(v3.z, v3.w)));
-    }
-    for (; i < q1; i += BLOCK) {
-        T4 v0 = ld4(row + 4 * i);
-        acc0 = combine(acc0, combine(combine(v0.x, v0.y), combine(v0.z, v0.w)));
-    }
-    T acc = combine(combine(acc0, acc1), combine(acc2, acc3));
+    const int lane = threadIdx.x & 63;
+    const unsigned begin = lane < a.items ? a.first[lane] & 0x3fffffffu : 0xffffffffu;
+    const int item = __builtin_popcountll(__ballot(begin <= blockIdx.x)) - 1;
+    const unsigned c = blockIdx.x - (a.first[item] & 0x3fffffffu), mode = a.first[item] >> 30;
+    const T *in = a.in[item];
+    const size_t R = a.R[item], start = (size_t)c * a.chunk[item], stop = start + a.chunk[item], end = stop < R ? stop : R;
+    T acc = mode == 0 ? fold_words(in, start, end) : mode == 1 ? fold_quads(in, start, end) : fold_quads_loose(in, start, end);
     acc = block_reduce(acc);
-    if (threadIdx.x == 0) out[blockIdx.x] = acc;
+    if (threadIdx.x == 0) a.out[item][c] = acc;
 }
 
 // Strided lanes: thread (o, j) folds in[(o*R + r)*inner + j] over r in ascending r (the order of
@@ -532,12 +640,29 @@ int check_dtype(int dtype)
 struct ReduceKernels {
     hipFunction_t rows, rows4, rows4u, cols;
 };
-int reduce_kernels(const std::string &key, const std::string &src, ReduceKernels *k)
+int reduce_kernels(const std::string &key, bool is_sum, int dtype, bool square, ReduceKernels *k)
 {
+    if (rtc_find(key + ":rows", &k->rows) && rtc_find(key + ":rows4", &k->rows4) && rtc_find(key + ":rows4u", &k->rows4u) &&
+        rtc_find(key + ":cols", &k->cols))
+        return DOPT_HIP_OK;
+    const std::string src = reduce_source(is_sum, dtype, square);
     if (int rc = rtc_get(key + ":rows", src, "red_rows", &k->rows)) return rc;
     if (int rc = rtc_get(key + ":rows4", src, "red_rows4", &k->rows4)) return rc;
     if (int rc = rtc_get(key + ":rows4u", src, "red_rows4u", &k->rows4u)) return rc;
     return rtc_get(key + ":cols", src, "red_cols", &k->cols);
+}
+
+// How much of a contiguous row of R values one workgroup folds.
+size_t row_chunk(size_t outer, size_t R)
+{
+    size_t nchunks = 1;
+    if (outer < 1024) {
+        size_t want = ceil_div((size_t)num_cus() * 4, outer);
+        size_t maxc = ceil_div(R, (size_t)256 * 16);
+        nchunks = want < maxc ? want : maxc;
+        if (nchunks < 1) nchunks = 1;
+    }
+    return (ceil_div(R, nchunks) + 1023) / 1024 * 1024;
 }
 
 int reduce_pass(const ReduceKernels &k, const void *in, void *out, size_t outer, size_t R, size_t inner, size_t esize,
@@ -552,16 +677,7 @@ int reduce_pass(const ReduceKernels &k, const void *in, void *out, size_t outer,
         return rtc_launch(cols, grid, 256, args);
     }
     // contiguous rows
-    size_t nchunks = 1;
-    if (outer < 1024) {
-        size_t want = ceil_div((size_t)num_cus() * 4, outer);
-        size_t maxc = ceil_div(R, (size_t)256 * 16);
-        nchunks = want < maxc ? want : maxc;
-        if (nchunks < 1) nchunks = 1;
-    }
-    size_t chunk = ceil_div(R, nchunks);
-    chunk = (chunk + 1023) / 1024 * 1024;
-    nchunks = ceil_div(R, chunk);
+    size_t chunk = row_chunk(outer, R), nchunks = ceil_div(R, chunk);
     hipFunction_t first = R % 4 == 0 ? (aligned16(in) ? rows4 : k.rows4u) : rows;
     if (nchunks == 1) {
         void *args[] = {(void *)&in, (void *)&out, (void *)&R, (void *)&chunk, (void *)&nchunks};
@@ -582,6 +698,80 @@ int reduce_pass(const ReduceKernels &k, const void *in, void *out, size_t outer,
 
 }  // namespace
 
+namespace dopt {
+
+int pointwise_group(const PointwiseProgram &p, const std::vector<PointwiseItem> &items)
+{
+    if (int rc = group_check(p)) return rc;
+    const int nin = (int)p.kind.size();
+    std::vector<const PointwiseItem *> todo;
+    for (const PointwiseItem &it : items) {
+        DOPT_REQUIRE((int)it.in.size() == nin && it.out.size() == p.outs.size(), "pointwise_group: an item with %zu inputs and %zu results", it.in.size(),
+                     it.out.size());
+        if (it.n == 0) continue;
+        for (const void *q : it.in) DOPT_REQUIRE(q != nullptr, "pointwise_group: null input");
+        for (const void *q : it.out) DOPT_REQUIRE(q != nullptr, "pointwise_group: null result");
+        DOPT_REQUIRE(it.n < (size_t)1 << 40, "pointwise_group: %zu elements", it.n);
+        todo.push_back(&it);
+    }
+    if (todo.empty()) return DOPT_HIP_OK;
+    DOPT_ENSURE_INIT();
+    std::vector<char> common((size_t)nin, 0);
+    for (int k = 0; k < nin; k++) {
+        common[k] = p.kind[k] == 1;
+        for (const PointwiseItem *it : todo) common[k] = common[k] && it->in[k] == todo[0]->in[k];
+    }
+    const GroupShape g = group_shape(p, common);
+    hipFunction_t fn;
+    const std::string key = group_key(p, common);
+    if (!rtc_find(key, &fn))
+        if (int rc = rtc_get(key, group_source(p, g), "group_k", &fn)) return rc;
+    // struct Args of the source, field by field
+    const size_t at_n = (size_t)g.items * g.nptr * 8, at_shared = at_n + (size_t)g.items * 8;
+    const size_t at_first = at_shared + std::max<size_t>(1, g.shared.size()) * 8, at_count = at_first + (size_t)g.items * 4;
+    std::vector<char> args(at_count + 8, 0);
+    auto put = [&](size_t at, const void *from, size_t bytes) { std::memcpy(args.data() + at, from, bytes); };
+    for (size_t i = 0; i < g.shared.size(); i++) put(at_shared + 8 * i, &todo[0]->in[(size_t)g.shared[i]], 8);
+    int filled = 0;
+    size_t blocks = 0;
+    auto flush = [&]() -> int {
+        if (filled == 0) return DOPT_HIP_OK;
+        put(at_count, &filled, 4);
+        void *argv[] = {args.data()};
+        const int rc = rtc_launch(fn, (unsigned)blocks, 256, argv);
+        filled = 0;
+        blocks = 0;
+        return rc;
+    };
+    for (const PointwiseItem *it : todo) {
+        bool quads = true;
+        for (int k = 0; k < nin; k++) quads = quads && (p.kind[k] == 1 || aligned16(it->in[k]));
+        for (const void *q : it->out) quads = quads && aligned16(q);
+        const size_t need = quads ? ceil_div(it->n / 4 + it->n % 4, 256) : ceil_div(it->n, 1024);
+        if (filled == g.items || blocks + need > 0x3fffffffu)
+            if (int rc = flush()) return rc;
+        DOPT_REQUIRE(need <= 0x3fffffffu, "pointwise_group: %zu elements", it->n);
+        char *ptrs = args.data() + (size_t)filled * g.nptr * 8;
+        for (size_t i = 0; i < g.own.size(); i++) std::memcpy(ptrs + 8 * i, &it->in[(size_t)g.own[i]], 8);
+        for (size_t o = 0; o < it->out.size(); o++) std::memcpy(ptrs + 8 * (g.own.size() + o), &it->out[o], 8);
+        put(at_n + 8 * (size_t)filled, &it->n, 8);
+        const unsigned first = (unsigned)blocks | (quads ? 0x80000000u : 0u);
+        put(at_first + 4 * (size_t)filled, &first, 4);
+        blocks += need;
+        filled++;
+    }
+    return flush();
+}
+
+int pointwise_group_compile_only(const PointwiseProgram &p, const char *arch)
+{
+    if (int rc = group_check(p)) return rc;
+    const std::vector<char> common(p.kind.size(), 0);
+    return rtc_compile_only(group_source(p, group_shape(p, common)), arch, nullptr);
+}
+
+}  // namespace dopt
+
 extern "C" {
 
 int dopt_hip_pointwise(const char *op, int dtype, size_t n, const void *a, const void *b, void *out)
@@ -599,14 +789,15 @@ int dopt_hip_pointwise(const char *op, int dtype, size_t n, const void *a, const
     const char *kname = vec ? "pw_vec" : "pw_scalar";
     std::string key = std::string("pw:") + op + (dtype == DOPT_HIP_F32 ? ":f32:" : ":i32:") + kname;
     hipFunction_t fn;
-    if (int rc = rtc_get(key, pointwise_source(*info, dtype), kname, &fn)) return rc;
+    if (!rtc_find(key, &fn))
+        if (int rc = rtc_get(key, pointwise_source(*info, dtype), kname, &fn)) return rc;
     const void *bb = b ? b : a;
     unsigned grid = vec ? grid_for(256 * 4, ceil_div(n, 4)) : grid_for(256, n);
     void *args[] = {(void *)&n, (void *)&a, (void *)&bb, (void *)&out};
     return rtc_launch(fn, grid, 256, args);
 }
 
-// Checks a chain description and produces its cache key and source.
+// Checks a chain description and produces its cache key and, where `source` is given, its source.
 static int chain_prepare(int dtype, int nin, const unsigned char *in_is_scalar, int nnodes, const char *const *node_op,
                          const int *node_lhs, const int *node_rhs, std::string *key, std::string *source)
 {
@@ -630,7 +821,7 @@ static int chain_prepare(int dtype, int nin, const unsigned char *in_is_scalar, 
         *key += std::string("|") + node_op[j] + "," + std::to_string(node_lhs[j]) + "," +
                 std::to_string(ops[j]->arity == 2 ? node_rhs[j] : -1);
     }
-    *source = chain_source(dtype, nin, in_is_scalar, nnodes, ops, node_lhs, node_rhs);
+    if (source) *source = chain_source(dtype, nin, in_is_scalar, nnodes, ops, node_lhs, node_rhs);
     return DOPT_HIP_OK;
 }
 
@@ -639,7 +830,7 @@ int dopt_hip_pointwise_chain(int dtype, size_t n, size_t inner, int nin, const v
                              const int *node_rhs, void *out)
 {
     std::string key, source;
-    if (int rc = chain_prepare(dtype, nin, in_is_scalar, nnodes, node_op, node_lhs, node_rhs, &key, &source)) return rc;
+    if (int rc = chain_prepare(dtype, nin, in_is_scalar, nnodes, node_op, node_lhs, node_rhs, &key, nullptr)) return rc;
     if (n == 0) return DOPT_HIP_OK;
     DOPT_REQUIRE(in && out, "dopt_hip_pointwise_chain: null argument");
     bool vec = aligned16(out), grid_kinds = false;
@@ -657,7 +848,10 @@ int dopt_hip_pointwise_chain(int dtype, size_t n, size_t inner, int nin, const v
     DOPT_ENSURE_INIT();
     const char *kname = vec ? "chain_vec" : "chain_scalar";
     hipFunction_t fn;
-    if (int rc = rtc_get(key + ":" + kname, source, kname, &fn)) return rc;
+    if (!rtc_find(key + ":" + kname, &fn)) {
+        if (int rc = chain_prepare(dtype, nin, in_is_scalar, nnodes, node_op, node_lhs, node_rhs, &key, &source)) return rc;
+        if (int rc = rtc_get(key + ":" + kname, source, kname, &fn)) return rc;
+    }
     const void *ptrs[16];
     void *args[19];
     args[0] = (void *)&n;
@@ -763,11 +957,10 @@ int reduce_impl(const char *op, int dtype, const size_t *shape, int rank, const 
         if (channel_sum(N, C, inner, (const float *)in, (float *)out, &crc)) return crc;
     }
     std::string key = std::string("red:") + op + (dtype == DOPT_HIP_F32 ? ":f32" : ":i32");
-    std::string src = reduce_source(is_sum, dtype);
     ReduceKernels plain{}, squares{};   // `squares`: the first pass of a sum of squares
-    if (int rc = reduce_kernels(key, src, &plain)) return rc;
+    if (int rc = reduce_kernels(key, is_sum, dtype, false, &plain)) return rc;
     if (square)
-        if (int rc = reduce_kernels("red:sumsq:f32", reduce_source(true, dtype, true), &squares)) return rc;
+        if (int rc = reduce_kernels("red:sumsq:f32", true, dtype, true, &squares)) return rc;
     const void *src_ptr = in;
     void *tmp_prev = nullptr;
     int rc = DOPT_HIP_OK;
@@ -830,6 +1023,74 @@ int dopt_hip_reduce_squares(const size_t *shape, int rank, const size_t *axes, i
     dopt_hip_free(product);
     return rc;
 }
+
+}  // extern "C"
+
+namespace dopt {
+
+// out[i] = the sum of the squares of the n[i] values at in[i], each as dopt_hip_reduce_squares gives it (same chunks, same
+// order); two launches for up to 64 tensors instead of two each.
+int reduce_squares_batch(int count, const float *const *in, const size_t *n, float *const *out)
+{
+    struct Rows {   // struct Rows of the kernel source
+        const float *in[64];
+        float *out[64];
+        size_t R[64];
+        unsigned chunk[64], first[64];
+        int items;
+    };
+    DOPT_ENSURE_INIT();
+    hipFunction_t squares, plain;
+    if (!rtc_find("red:sumsq:f32:batch", &squares))
+        if (int rc = rtc_get("red:sumsq:f32:batch", reduce_source(true, DOPT_HIP_F32, true), "red_batch", &squares)) return rc;
+    if (!rtc_find("red:sum:f32:batch", &plain))
+        if (int rc = rtc_get("red:sum:f32:batch", reduce_source(true, DOPT_HIP_F32), "red_batch", &plain)) return rc;
+    for (int begin = 0; begin < count; begin += 64) {
+        const int items = std::min(64, count - begin);
+        size_t partials = 0;
+        for (int i = 0; i < items; i++) {
+            DOPT_REQUIRE(in[begin + i] && out[begin + i] && n[begin + i] > 64 && n[begin + i] < (size_t)1 << 40, "reduce_squares_batch: tensor %d", begin + i);
+            const size_t nchunks = ceil_div(n[begin + i], row_chunk(1, n[begin + i]));
+            if (nchunks > 1) partials += nchunks;
+        }
+        float *partial = nullptr;
+        if (partials > 0) {
+            partial = (float *)workspace(partials * sizeof(float));
+            if (!partial) return DOPT_HIP_ERR_OOM;
+        }
+        Rows a{}, b{};
+        size_t blocks = 0;
+        for (int i = 0; i < items; i++) {
+            const float *src = in[begin + i];
+            const size_t R = n[begin + i], chunk = row_chunk(1, R), nchunks = ceil_div(R, chunk);
+            const unsigned mode = R % 4 != 0 ? 0 : aligned16(src) ? 1 : 2;
+            a.in[i] = src;
+            a.out[i] = nchunks > 1 ? partial : out[begin + i];
+            a.R[i] = R;
+            a.chunk[i] = (unsigned)chunk;   // (at most 2^40 / 2^10 values)
+            a.first[i] = (unsigned)blocks | mode << 30;
+            blocks += nchunks;
+            if (nchunks == 1) continue;
+            b.in[b.items] = partial;
+            b.out[b.items] = out[begin + i];
+            b.R[b.items] = nchunks;
+            b.chunk[b.items] = (unsigned)((nchunks + 255) / 256 * 256);
+            b.first[b.items] = (unsigned)b.items;
+            b.items++;
+            partial += nchunks;
+        }
+        a.items = items;
+        void *aargs[] = {&a}, *bargs[] = {&b};
+        if (int rc = rtc_launch(squares, (unsigned)blocks, 256, aargs)) return rc;
+        if (b.items > 0)
+            if (int rc = rtc_launch(plain, (unsigned)b.items, 256, bargs)) return rc;
+    }
+    return DOPT_HIP_OK;
+}
+
+}  // namespace dopt
+
+extern "C" {
 
 int dopt_hip_argmin(int dtype, const size_t *shape, int rank, size_t axis, const void *in, int32_t *out)
 {

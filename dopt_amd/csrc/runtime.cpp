@@ -213,6 +213,15 @@ int rtc_compile_only(const std::string &source, const char *arch, std::string *l
     return rtc_compile(source, arch, nullptr, log);
 }
 
+bool rtc_find(const std::string &key, hipFunction_t *fn)
+{
+    Runtime &r = rt();
+    auto it = r.kernels.find(key);
+    if (it == r.kernels.end()) return false;
+    *fn = it->second;
+    return true;
+}
+
 int rtc_get(const std::string &key, const std::string &source, const char *kernel_name, hipFunction_t *fn)
 {
     Runtime &r = rt();

@@ -208,3 +208,81 @@ def test_random_graphs_give_the_same_values_with_every_rewrite(seed):
             plan.execute(None, bufs)
             for got, w in zip(bufs, want):
                 assert np.array_equal(got.numpy(), w, equal_nan=True), flags
+
+
+# sizes around a quad, a workgroup's 256 quads and its 1024 loose elements; more tensors than one launch's arguments hold
+GROUPS = [[2, 3], [5, 64, 1023, 1024, 1025, 4099, 100003], list(range(2, 150, 2)), [7] * 3 + [4096, 4100]]
+
+
+@pytest.mark.parametrize("sizes", GROUPS, ids=lambda s: "%d_tensors" % len(s))
+@pytest.mark.parametrize("offset", [0, 1, 4])
+def test_update_rules_of_many_tensors_as_one_step(sizes, offset):
+    """Pointwise pieces that only feed outputs, one per tensor: one step for all that share a program.  Gradients arrive as
+    views into a larger tensor (`offset` elements in: 1 is no quad), scalars as products with ones vectors, through `repeat`
+    and as one-element arithmetic; a value is an output and read on, one is a view of an output.  Bits of the plan without
+    rewrites, also at the second execution, which replays a recording."""
+    r = np.random.default_rng(len(sizes) + offset)
+    rate, decay, unit = core.float32([], [0.3]), core.float32([], [0.05]), core.float32([1], [0.7])
+    outs = []
+    for n in sizes:
+        w, m = (core.float32([n], r.standard_normal(n).astype(np.float32)) for _ in range(2))
+        packed = core.float32([n + offset + 3], r.standard_normal(n + offset + 3).astype(np.float32))
+        g = core.slice(packed, [offset], [offset + n])
+        nm = m * rate + (1.0 - rate) * g               # 1 - rate: arithmetic on one element, for every tensor anew
+        nw = w - (decay * 2.0) * (nm / (core.sqrt(core.abs(nm)) + core.repeat(unit, [n])))
+        outs += [nw, core.reshape(nm, [n, 1]), core.max(nm, g)]
+    want = core.compile(outs).execute()
+    for flags in (core.PLAN_VIEWS | core.PLAN_FUSE | core.PLAN_TIMING, core.PLAN_VIEWS | core.PLAN_FUSE | core.PLAN_GRAPH,
+                  core.PLAN_VIEWS | core.PLAN_FUSE | core.PLAN_OVERLAP, core.PLAN_FUSE):
+        plan = core.compile(outs, flags)
+        bufs = [ops.Tensor(o.shape) for o in outs]
+        for _ in range(3):
+            plan.execute(None, bufs)
+            for got, b in zip(bufs, want):
+                assert np.array_equal(got.numpy(), b), flags
+        if flags & core.PLAN_TIMING:
+            assert any(k.startswith("pointwise*") and k.endswith("x%d" % len(sizes)) for k in plan.profile()), plan.profile()
+
+
+def test_values_that_something_else_reads_stay_out_of_a_group():
+    """A reduction, a narrower view and a value broadcast from one element of a tensor end what may run last."""
+    r = np.random.default_rng(9)
+    a, b = (core.float32([300], r.standard_normal(300).astype(np.float32)) for _ in range(2))
+    s = a * b
+    outs = [s - a, core.sum(s + b), core.slice(s, [10], [20]) * core.slice(a, [0], [10]), core.exp(b) + a]
+    one = core.sum(a * 0.5)
+    outs += [(one * 0.25) * a, (one * 0.25) * b, one * 0.25]
+    want = core.compile(outs).execute()
+    got = core.compile(outs, core.PLAN_VIEWS | core.PLAN_FUSE).execute()
+    for g, w in zip(got, want):
+        assert np.array_equal(g, w)
+
+
+def test_penalties_of_many_tensors_as_one_step():
+    """sum(w * w) of three and more variables: the sums of dopt_hip_reduce_squares, bit for bit, whatever the size (one
+    workgroup's chunk of 4096, several, no multiple of four)."""
+    r = np.random.default_rng(2)
+    ws = [core.float32([n], r.standard_normal(n).astype(np.float32)) for n in (65, 66, 4096, 4097, 50001, 1 << 20) + tuple(range(80, 160))]
+    outs = [core.sum(w * w) for w in ws]
+    want = core.compile(outs).execute()
+    plan = core.compile(outs, core.PLAN_VIEWS | core.PLAN_FUSE | core.PLAN_TIMING)
+    for g, w in zip(plan.execute(), want):
+        assert np.array_equal(g, w)
+    assert any(k.startswith("mul+sum*") for k in plan.profile()), plan.profile()
+
+
+def test_batched_copies_of_every_length_and_alignment():
+    lib = capi.load()
+    r = np.random.default_rng(4)
+    lengths = [1, 3, 4, 5, 1023, 1024, 1025, 4095, 4096, 4100, 16384, 70001] + [int(v) for v in r.integers(1, 9000, 140)]
+    src = [ops.tensor(r.standard_normal(n + 8).astype(np.float32)) for n in lengths]
+    dst = [ops.tensor(np.zeros(n + 8, np.float32)) for n in lengths]
+    at = [(int(r.integers(0, 3)) * 2, int(r.integers(0, 5))) for _ in lengths]
+    n = len(lengths)
+    capi.check(lib.dopt_hip_copy_d2d_batch(n, (C.c_void_p * n)(*[d.ptr + 4 * j for d, (_, j) in zip(dst, at)]),
+                                           (C.c_void_p * n)(*[s.ptr + 4 * i for s, (i, _) in zip(src, at)]),
+                                           (C.c_size_t * n)(*[4 * k for k in lengths])))
+    for s, d, (i, j), k in zip(src, dst, at, lengths):
+        want = np.zeros(k + 8, np.float32)
+        want[j:j + k] = s.numpy()[i:i + k]
+        assert np.array_equal(d.numpy(), want)
