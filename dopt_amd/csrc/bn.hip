@@ -272,39 +272,113 @@ __global__ __launch_bounds__(kBlock) void bn_infer_prepare_k(size_t C, double ep
     coef[c] = k;
 }
 
-// Inference in one launch: block (c, slice) derives its channel's coefficients itself (one float64
-// reciprocal square root per thread) and streams that channel's rows of images slice, slice + S, ...
-// with four 128-bit loads in flight per thread.  Same arithmetic as the coefficient table + bn_apply_k.
-__global__ __launch_bounds__(kBlock) void bn_infer_chan_k(unsigned N, unsigned C, unsigned inner4, unsigned S, double eps,
-                                                           const float *x, const float *scale, const float *bias,
-                                                           const float *mean, const float *var, float *y)
+// Inference in one launch, with the relu behind it, the 2 x 2 max-pool behind that, and the partial copies of the convolution
+// in front of it: y = relu(a * (x - mean) + b) and / or its pooled tensor.  Bound by memory traffic where the tensor is large
+// and by the kernel boundary where it is small, so what counts is that these are one pass and one launch: a layer of a
+// single image was three to five launches (sum of copies, coefficient table, batch norm, relu, pool).
+// A block takes kU * 256 units of consecutive quads - a unit is one quad, or, pooled, the quads of one or two windows - and
+// first puts the coefficients of the channels they lie in into LDS (one float64 reciprocal square root each; rows of
+// the [N * C, inner] view, so at most as many as it has units).  Same arithmetic as bn_infer_prepare_k, bn_apply_k, relu_fwd_k
+// and maxpool2x2_fwd_k; the copies are added as splitk_reduce_k adds them.
+struct InferArgs {
+    const float4 *x;         // the operand, or null: [splits] copies of it at `partial`, to be added, and `addend` per channel
+    const float4 *partial;
+    const float *addend;
+    int splits;
+    unsigned n4, C, inner4, units, upr, W;   // quads; channels; quads of a row; units in all and of a row; pixels of an image row
+    double eps;
+    const float *scale, *bias, *mean, *var;
+    float4 *y;               // either may be null
+    float *pooled;
+    int relu;
+};
+
+__device__ inline float4 infer_load(const InferArgs &g, unsigned i, unsigned c)
 {
-    const unsigned c = blockIdx.x % C, s = blockIdx.x / C;
-    const double rstd = 1.0 / sqrt((double)var[c] + eps);
-    const float m = mean[c], a = (float)((double)scale[c] * rstd), b = bias[c];
-    const unsigned nimg = (N - s + S - 1) / S, tot = nimg * inner4;
-    const float4 *x4 = (const float4 *)x;
-    float4 *y4 = (float4 *)y;
-    for (unsigned base = threadIdx.x; base < tot; base += kUnroll * kBlock) {
-        float4 v[kUnroll];
-        size_t at[kUnroll];
+    if (g.x) return g.x[i];
+    float4 acc = g.partial[i];
+    const int last = g.splits - 1;
+    for (int s = 1; s < g.splits; s += 4) {   // four loads in flight, added in ascending order
+        const float4 v0 = g.partial[(size_t)s * g.n4 + i];
+        const float4 v1 = g.partial[(size_t)min(s + 1, last) * g.n4 + i];
+        const float4 v2 = g.partial[(size_t)min(s + 2, last) * g.n4 + i];
+        const float4 v3 = g.partial[(size_t)min(s + 3, last) * g.n4 + i];
+        acc = make_float4(acc.x + v0.x, acc.y + v0.y, acc.z + v0.z, acc.w + v0.w);
+        if (s + 1 <= last) acc = make_float4(acc.x + v1.x, acc.y + v1.y, acc.z + v1.z, acc.w + v1.w);
+        if (s + 2 <= last) acc = make_float4(acc.x + v2.x, acc.y + v2.y, acc.z + v2.z, acc.w + v2.w);
+        if (s + 3 <= last) acc = make_float4(acc.x + v3.x, acc.y + v3.y, acc.z + v3.z, acc.w + v3.w);
+    }
+    if (g.addend) {
+        const float b = g.addend[c];
+        acc = make_float4(acc.x + b, acc.y + b, acc.z + b, acc.w + b);
+    }
+    return acc;
+}
+
+__device__ inline float4 infer_value(const InferArgs &g, float4 v, const Coef &k)
+{
+    float4 r;
+    r.x = k.a * ((v.x - k.mean) - k.mean_lo) + k.b;
+    r.y = k.a * ((v.y - k.mean) - k.mean_lo) + k.b;
+    r.z = k.a * ((v.z - k.mean) - k.mean_lo) + k.b;
+    r.w = k.a * ((v.w - k.mean) - k.mean_lo) + k.b;
+    return g.relu ? make_float4(relu1(r.x), relu1(r.y), relu1(r.z), relu1(r.w)) : r;
+}
+
+template <int kU, bool kPool>
+__global__ __launch_bounds__(kBlock) void bn_infer_k(InferArgs g)
+{
+    __shared__ Coef coef[kU * kBlock + 1];
+    __shared__ unsigned channel[kU * kBlock + 1];
+    const unsigned begin = blockIdx.x * (kU * kBlock), end = min(begin + kU * kBlock, g.units);
+    const unsigned row0 = begin / g.upr, rows = (end - 1) / g.upr - row0 + 1;
+    for (unsigned k = threadIdx.x; k < rows; k += kBlock) {
+        const unsigned c = (row0 + k) % g.C;
+        const double rstd = 1.0 / sqrt((double)g.var[c] + g.eps);
+        Coef q;
+        q.mean = g.mean[c];
+        q.a = (float)((double)g.scale[c] * rstd);
+        q.b = g.bias[c];
+        q.mean_lo = 0.0f;
+        coef[k] = q;
+        channel[k] = c;
+    }
+    __syncthreads();
+    if constexpr (!kPool) {
+        float4 v[kU];
+        unsigned at[kU];
 #pragma unroll
-        for (int u = 0; u < kUnroll; u++) {
-            const unsigned t = base + u * kBlock;
-            const unsigned j = t / inner4, i = t - j * inner4;
-            at[u] = ((size_t)(s + j * S) * C + c) * inner4 + i;
-            if (t < tot) v[u] = x4[at[u]];
+        for (int u = 0; u < kU; u++) {
+            const unsigned i = begin + u * kBlock + threadIdx.x;
+            if (i >= end) break;
+            at[u] = i / g.upr - row0;
+            v[u] = infer_load(g, i, channel[at[u]]);
         }
 #pragma unroll
-        for (int u = 0; u < kUnroll; u++) {
-            if (base + u * kBlock >= tot) continue;
-            float4 r;
-            r.x = a * ((v[u].x - m) - 0.0f) + b;
-            r.y = a * ((v[u].y - m) - 0.0f) + b;
-            r.z = a * ((v[u].z - m) - 0.0f) + b;
-            r.w = a * ((v[u].w - m) - 0.0f) + b;
-            y4[at[u]] = r;
+        for (int u = 0; u < kU; u++) {
+            const unsigned i = begin + u * kBlock + threadIdx.x;
+            if (i >= end) break;
+            g.y[i] = infer_value(g, v[u], coef[at[u]]);
         }
+    } else {
+        const unsigned i = begin + threadIdx.x;   // (kU is 1)
+        if (i >= end) return;
+        const unsigned row = i / g.upr, j = i - row * g.upr, k = row - row0;
+        if (g.W == 2) {   // a quad is a window
+            const unsigned q = row * g.inner4 + j;
+            const float4 r = infer_value(g, infer_load(g, q, channel[k]), coef[k]);
+            if (g.y) g.y[q] = r;
+            g.pooled[i] = pool2x2(r.x, r.y, r.z, r.w);
+            return;
+        }
+        const unsigned W4 = g.W / 4, p = j / W4, q = row * g.inner4 + 2 * p * W4 + (j - p * W4);
+        const float4 v0 = infer_load(g, q, channel[k]), v1 = infer_load(g, q + W4, channel[k]);
+        const float4 a = infer_value(g, v0, coef[k]), b = infer_value(g, v1, coef[k]);
+        if (g.y) {
+            g.y[q] = a;
+            g.y[q + W4] = b;
+        }
+        ((float2 *)g.pooled)[i] = make_float2(pool2x2(a.x, a.y, b.x, b.y), pool2x2(a.z, a.w, b.z, b.w));
     }
 }
 
@@ -1399,6 +1473,45 @@ int bn_grad_impl(size_t N, size_t C, size_t inner, const float *dy, const float 
     return DOPT_HIP_OK;
 }
 
+// Whether bn_infer_k takes a tensor: whole quads within a channel's row, 32-bit indices.
+bool infer_takes(size_t total, size_t inner, const float *x, const float *y)
+{
+    return inner % 4 == 0 && total < 0x7fffffffull && aligned16(x) && aligned16(y);
+}
+
+// W: pixels of an image row (pooled given).
+int launch_infer(size_t N, size_t C, size_t inner, size_t W, const float *x, const dopt_hip_split_sum *open, const float *scale,
+                 const float *bias, const float *mean, const float *var, int relu, float *y, float *pooled)
+{
+    InferArgs g{};
+    const bool split = open && open->splits > 0;
+    g.x = split ? nullptr : (const float4 *)x;
+    if (split) {
+        g.partial = (const float4 *)open->partial;
+        g.splits = open->splits;
+        g.addend = open->bias;
+    }
+    g.n4 = (unsigned)(N * C * inner / 4);
+    g.C = (unsigned)C;
+    g.inner4 = (unsigned)(inner / 4);
+    g.W = (unsigned)W;
+    g.upr = !pooled ? g.inner4 : W == 2 ? g.inner4 : g.inner4 / 2;
+    g.units = (unsigned)(N * C) * g.upr;
+    g.eps = 1e-5;   // cudnn7.d:652
+    g.scale = scale; g.bias = bias; g.mean = mean; g.var = var;
+    g.y = (float4 *)y;
+    g.pooled = pooled;
+    g.relu = relu;
+    if (split) open_split_clear(open->partial);
+    // four quads a thread once that still gives every CU two blocks
+    if (pooled) hipLaunchKernelGGL((bn_infer_k<1, true>), dim3((unsigned)ceil_div(g.units, kBlock)), dim3(kBlock), 0, stream(), g);
+    else if (g.units >= 2u * 4 * kBlock * (unsigned)num_cus())
+        hipLaunchKernelGGL((bn_infer_k<4, false>), dim3((unsigned)ceil_div(g.units, 4 * kBlock)), dim3(kBlock), 0, stream(), g);
+    else hipLaunchKernelGGL((bn_infer_k<1, false>), dim3((unsigned)ceil_div(g.units, kBlock)), dim3(kBlock), 0, stream(), g);
+    DOPT_LAUNCH_CHECK();
+    return DOPT_HIP_OK;
+}
+
 }  // namespace
 
 namespace dopt {
@@ -1554,14 +1667,7 @@ int dopt_hip_bn_infer(size_t N, size_t C, size_t inner, const float *x, const fl
     if (total == 0) return DOPT_HIP_OK;
     DOPT_REQUIRE(x && scale && bias && mean && var && y, "dopt_hip_bn_infer: null argument");
     DOPT_ENSURE_INIT();
-    if ((inner & 3) == 0 && inner >= 256 && aligned16(x) && aligned16(y) && total / 4 < 0xffffffffull && N < (1u << 24) &&
-        C <= 0x7fffffffu / kMaxSlices) {
-        const size_t S = pick_slices(N, C);
-        hipLaunchKernelGGL(bn_infer_chan_k, dim3((unsigned)(C * S)), dim3(kBlock), 0, stream(), (unsigned)N, (unsigned)C,
-                           (unsigned)(inner / 4), (unsigned)S, 1e-5 /* cudnn7.d:652 */, x, scale, bias, mean, var, y);
-        DOPT_LAUNCH_CHECK();
-        return DOPT_HIP_OK;
-    }
+    if (infer_takes(total, inner, x, y)) return launch_infer(N, C, inner, 1, x, nullptr, scale, bias, mean, var, 0, y, nullptr);
     Coef *coef = (Coef *)workspace(C * sizeof(Coef));
     if (!coef) return DOPT_HIP_ERR_OOM;
     hipLaunchKernelGGL(bn_infer_prepare_k, dim3((unsigned)ceil_div(C, (size_t)kBlock)), dim3(kBlock), 0, stream(), C,
@@ -1571,3 +1677,29 @@ int dopt_hip_bn_infer(size_t N, size_t C, size_t inner, const float *x, const fl
 }
 
 }  // extern "C"
+
+namespace dopt {
+
+int bn_infer_fused(size_t N, size_t C, size_t H, size_t W, const float *x, const dopt_hip_split_sum *open, const float *scale, const float *bias,
+                   const float *mean, const float *var, int relu, float *y, int keep_y, float *pooled)
+{
+    const size_t inner = H * W, total = N * C * inner;
+    if (total == 0) return DOPT_HIP_OK;
+    DOPT_REQUIRE(x && scale && bias && mean && var && y, "bn_infer_fused: null argument");
+    DOPT_ENSURE_INIT();
+    const bool split = open && open->splits > 0;
+    if (split)
+        DOPT_REQUIRE(open->partial && open->value == x && open->elems == total && open->C == C && open->inner == inner && open->lanes == 0,
+                     "bn_infer_fused: the open convolution result is not the batch norm's operand");
+    const bool windows = H % 2 == 0 && (W % 4 == 0 || W == 2);
+    if (infer_takes(total, inner, split ? open->partial : x, y) && (!pooled || (windows && aligned16(pooled))))
+        return launch_infer(N, C, inner, W, x, open, scale, bias, mean, var, relu, pooled && !keep_y ? nullptr : y, pooled);
+    if (split)
+        if (int rc = dopt_hip_split_sum_close(open)) return rc;
+    if (int rc = dopt_hip_bn_infer(N, C, inner, x, scale, bias, mean, var, y)) return rc;
+    if (relu)
+        if (int rc = dopt_hip_relu_fwd(total, y, y)) return rc;
+    return pooled ? dopt_hip_maxpool_fwd(N, C, H, W, 2, 2, y, pooled) : DOPT_HIP_OK;
+}
+
+}  // namespace dopt

@@ -54,6 +54,11 @@ bool sgemm_fold2x2(size_t C, size_t K, size_t N, const float *x, const float *dy
 // The same for up to 8 layers in one launch; false, with nothing launched, unless every layer suits that kernel.
 bool sgemm_fold2x2_batch(int n, const size_t *C, const size_t *K, const size_t *N, const float *const *x,
                          const float *const *dy, float *const *dw, int *rc);
+// bn.hip: batchNormInference of [N, C, H, W] with what surrounds it in one launch: its operand x may be an open convolution
+// result (`open`, value == x), relu != 0 clamps, `pooled` (or null) receives the 2 x 2 max-pool.  y receives the (clamped) value;
+// with keep_y == 0 it is scratch that only the pool reads.
+int bn_infer_fused(size_t N, size_t C, size_t H, size_t W, const float *x, const dopt_hip_split_sum *open, const float *scale, const float *bias,
+                   const float *mean, const float *var, int relu, float *y, int keep_y, float *pooled);
 // conv_smallc.hip: 3x3 pad-1 unit-stride convolutions over at most three input channels.  `done`
 // stays false when the shape is not theirs (the caller then uses the general kernels).
 bool conv_smallc_takes(const dopt_hip_conv_desc *d);

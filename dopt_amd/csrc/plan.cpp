@@ -584,7 +584,8 @@ struct HIPPlan::Builder {
     std::vector<Alias> alias;
     // inputsOf[id]: the operations whose buffers feed id's kernel (its deps, unless fused);
     // fusedKind[id]: 1 conv+bias, 2 bn+relu, 3 relugrad+bngrad, 6 matmul with transposes, 7 pointwise chain,
-    // 8 maxpoolgrad+relugrad+bngrad, 9 matmul+relugrad, 10 member of a tiny run, 11 sum of squares, 12 member of a group
+    // 8 maxpoolgrad+relugrad+bngrad, 9 matmul+relugrad, 10 member of a tiny run, 11 sum of squares, 12 member of a group,
+    // 13 batchNormInference whose kernel clamps
     std::vector<std::vector<int>> inputsOf;
     std::vector<int> fusedKind;
     std::vector<std::unique_ptr<HIPKernel>> prebuilt;
@@ -595,7 +596,8 @@ struct HIPPlan::Builder {
     std::vector<std::vector<Use>> uses;
     std::vector<std::vector<size_t>> exposed;   // byte offsets at which plan outputs (or aliases of them) expose a buffer
     std::vector<int> biasGradOf;                // batchNormGrad op -> the addBiasGrad op it serves
-    std::vector<int> poolOf;                    // batchNormTrain op -> the 2 x 2 maxpool op whose buffer its kernel fills too
+    std::vector<int> reluOf;                    // batchNormInference op of kind 13 -> the relu op whose value its buffer holds
+    std::vector<int> poolOf;                    // batchNormTrain or batchNormInference op -> the 2 x 2 maxpool op whose buffer its kernel fills too
     std::vector<int> pairOf;                    // packed convolutionFeaturesGrad op -> the convolutionFiltersGrad op of the same layer
     std::vector<int> pairLead;                  // the operation of such a pair that comes first in the order -> the backward-data op
     std::vector<char> pairLater;                // the operation of such a pair that comes second: no step of its own
@@ -618,7 +620,7 @@ struct HIPPlan::Builder {
     Builder(const Graph &graph, HIPPlan *plan, const std::vector<int> &outs, unsigned f)
         : g(graph), p(plan), outputs(outs), flags(f), nops((int)graph.ops.size()), alias((size_t)nops),
           inputsOf((size_t)nops), fusedKind((size_t)nops, 0), prebuilt((size_t)nops), prebuiltLabel((size_t)nops),
-          live((size_t)nops, 0), uses((size_t)nops), exposed((size_t)nops), biasGradOf((size_t)nops, -1), poolOf((size_t)nops, -1), pairOf((size_t)nops, -1), pairLead((size_t)nops, -1),
+          live((size_t)nops, 0), uses((size_t)nops), exposed((size_t)nops), biasGradOf((size_t)nops, -1), reluOf((size_t)nops, -1), poolOf((size_t)nops, -1), pairOf((size_t)nops, -1), pairLead((size_t)nops, -1),
           pairLater((size_t)nops, 0),
           absorbed((size_t)nops, 0), groupReads((size_t)nops, 0), tinyWrites((size_t)nops), needed((size_t)nops, 0), packOf((size_t)nops, -1), mmInfo((size_t)nops)
     {
@@ -651,6 +653,7 @@ struct HIPPlan::Builder {
     void absorbPools();
     void pairBackward();
     std::unique_ptr<HIPKernel> makePooledTrain(int id, std::shared_ptr<dopt_hip_split_sum> open, std::string *label);
+    std::unique_ptr<HIPKernel> makeInference(int id, std::shared_ptr<dopt_hip_split_sum> open, std::string *label);
     void markNeeded();
     int prepackFilters();
     int allocateBuffers();
@@ -744,6 +747,14 @@ void HIPPlan::Builder::fusePairs()
             size_t off;
             const int b = root(op.deps[0], &off);
             const Operation &bn = g.ops[b];
+            if (bn.opType == "batchNormInference" && bn.deps.size() == 5 && off == 0 && !fusedKind[b] && bn.dtype == DOPT_HIP_F32 &&
+                op.volume() == bn.volume() && !isOutput(b) && uses[b].size() == 1) {
+                fusedKind[b] = 13;
+                reluOf[b] = id;
+                alias[id].source = b;  // the buffer holds the clamped value
+                alias[id].offset = 0;
+                continue;
+            }
             if (bn.opType != "batchNormTrain" || bn.deps.size() != 5 || off != 0 || fusedKind[b] ||
                 op.volume() != g.ops[bn.deps[0]].volume())
                 continue;
@@ -1647,8 +1658,8 @@ void HIPPlan::Builder::absorbBiasGrads()
 
 void HIPPlan::Builder::absorbPools()
 {
-    // maxpool [2, 2] of a batch norm's y part (through the relu that became an alias of it, or directly): the
-    // batch-norm kernel has the values in registers and writes the pooled tensor too.  The maxpool operation
+    // maxpool [2, 2] of a batch norm's y part (through the relu that became an alias of it, or directly; training or
+    // inference): the batch-norm kernel has the values in registers and writes the pooled tensor too.  The maxpool operation
     // keeps its buffer but gets no kernel of its own.
     if (!(flags & DOPT_HIP_PLAN_FUSE)) return;
     for (int id : p->mOps) {
@@ -1660,8 +1671,9 @@ void HIPPlan::Builder::absorbPools()
         size_t off;
         const int b = root(op.deps[0], &off);
         const Operation &bn = g.ops[b];
-        if (bn.opType != "batchNormTrain" || bn.deps.size() != 5 || off != 0 || poolOf[b] >= 0 || prebuilt[b] ||
-            (fusedKind[b] != 0 && fusedKind[b] != 2) || g.ops[bn.deps[0]].shape != xs || op.volume() == 0)
+        const bool infer = bn.opType == "batchNormInference";
+        if ((bn.opType != "batchNormTrain" && !infer) || bn.deps.size() != 5 || off != 0 || poolOf[b] >= 0 || prebuilt[b] ||
+            (fusedKind[b] != 0 && fusedKind[b] != (infer ? 13 : 2)) || g.ops[bn.deps[0]].shape != xs || op.volume() == 0)
             continue;
         poolOf[b] = id;
         absorbed[id] = 1;
@@ -1856,6 +1868,29 @@ std::unique_ptr<HIPKernel> HIPPlan::Builder::makePooledTrain(int id, std::shared
     });
 }
 
+// batchNormInference with the relu (kind 13) and the maxpool that became part of it; `open`: as above.
+std::unique_ptr<HIPKernel> HIPPlan::Builder::makeInference(int id, std::shared_ptr<dopt_hip_split_sum> open, std::string *label)
+{
+    const Operation &op = g.ops[id];
+    if (!need_deps(op, 5) || !need_f32(op)) return nullptr;
+    const auto &xs = op.shape;
+    const bool image = xs.size() == 4;
+    size_t N, C, inner;
+    nci(xs, &N, &C, &inner);
+    const size_t H = image ? xs[2] : inner, W = image ? xs[3] : 1;
+    const int relu = fusedKind[id] == 13, pool = poolOf[id];
+    float *pooled = pool >= 0 && needed[pool] ? (float *)p->mResults[pool] : nullptr;
+    // the value itself is stored unless the pool is all that reads it
+    const int value = relu ? reluOf[id] : id;
+    const int keep = !pooled || isOutput(value) || uses[value].size() != 1;
+    *label = std::string("batchNormInference") + (relu ? "+relu" : "") + (pooled ? "+maxpool" : "");
+    return make([=](const std::vector<const void *> &in, void *out) {
+        if (open && open->value != in[0]) return fail(DOPT_HIP_ERR_RUNTIME, "plan: open convolution result is not the batch norm's input");
+        return bn_infer_fused(N, C, H, W, (const float *)in[0], open.get(), (const float *)in[1], (const float *)in[2], (const float *)in[3],
+                              (const float *)in[4], relu, (float *)out, keep, pooled);
+    });
+}
+
 int HIPPlan::Builder::buildSteps()
 {
     // kernels and buffers
@@ -1920,6 +1955,8 @@ int HIPPlan::Builder::buildSteps()
         } else if (prebuilt[id]) {
             k = std::move(prebuilt[id]);
             label = prebuiltLabel[id];
+        } else if (op.opType == "batchNormInference" && (fusedKind[id] == 13 || (poolOf[id] >= 0 && needed[poolOf[id]]))) {
+            k = makeInference(id, nullptr, &label);
         } else if (poolOf[id] >= 0 && needed[poolOf[id]]) {
             k = makePooledTrain(id, nullptr, &label);
         } else if (fusedKind[id] || extra) {
@@ -2109,6 +2146,15 @@ void HIPPlan::Builder::openSplitSums()
                                                   (const float *)in[3], (const float *)in[4], (float *)out, relu);
                 });
             }
+        } else if (!cs.bwd && bo.opType == "batchNormInference" && bo.deps.size() == 5 && next.inputOps.size() == 5 &&
+                   (fusedKind[b] == 0 || fusedKind[b] == 13) && bo.dtype == DOPT_HIP_F32 && uses[cs.op].size() == 1 && !isOutput(cs.op)) {
+            const bool bias = cs.bias;
+            conv.kernel = make([=](const std::vector<const void *> &in, void *out) {
+                return dopt_hip_conv_fwd_bias_packed_open(&d, (const float *)in[0], fi >= 0 ? (const float *)in[fi] : packed,
+                                                          bias ? (const float *)in[1] : nullptr, (float *)out, open.get());
+            });
+            std::string unused;
+            next.kernel = makeInference(b, open, &unused);
         } else if (cs.bwd && bo.opType == "batchNormGrad" && bo.deps.size() == 3 &&
                    (((fusedKind[b] == 3 || fusedKind[b] == 8) && next.inputOps.size() == 4) ||
                     (fusedKind[b] == 0 && next.inputOps.size() == 3))) {

@@ -77,7 +77,7 @@ __device__ __forceinline__ void pw_loop(int n, AP a, AP b, int ka, int kb, int i
 }
 
 // Operands and result all start on a quad: four consecutive elements a thread, so that the most a node can have is one pass
-// (four single ones a thread were four times the instructions, and a node of 2560 elements 0.9 us instead of 0.4).  The
+// (four single ones a thread were four times the instructions, and a node of 2560 elements 0.9 us instead of 0.6).  The
 // elements behind the last of an n that is no multiple of four are read and written in LDS, where every place ends on a
 // quad, and left alone in memory.
 __device__ __forceinline__ float4 quad_at(const float *p, int i, int n, bool single)

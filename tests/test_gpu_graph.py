@@ -1184,3 +1184,42 @@ def test_graph_flag_leaves_plans_with_random_draws_direct():
         plan.execute(None, [out])
         draws.append(out.numpy().copy())
     assert all(not np.array_equal(draws[0], d) for d in draws[1:])     # a replayed kernel would repeat its draws
+
+
+@pytest.mark.parametrize("shape", [(1, 512, 2, 2), (3, 64, 4, 4), (1, 96, 16, 16), (2, 5, 6, 6), (5, 7, 3, 3), (2, 16, 8, 4), (7, 24, 2, 4),
+                                   (40, 300, 32, 32), (1, 4, 64, 64)], ids=str)
+@pytest.mark.parametrize("conv", [0, 1], ids=["plain", "behind a convolution"])
+def test_inference_batch_norm_with_its_neighbours_as_one_kernel(shape, conv):
+    """batchNormInference, the relu and the 2 x 2 max-pool behind it, and the sum of the copies of the convolution in front of
+    it: bits of the plan without rewrites, for every layout of quads and windows and for those that have none; with values
+    that something else reads, and with the batch norm's own value an output."""
+    r = np.random.default_rng(shape[1])
+    n, c, h, w = shape
+    x = float32(shape, r.standard_normal(shape).astype(np.float32))
+
+    def layer(y, relu=True):
+        p = [float32([1, c, 1, 1], r.standard_normal(c).astype(np.float32)), float32([c], r.standard_normal(c).astype(np.float32)),
+             float32([c], r.standard_normal(c).astype(np.float32)), float32([c], (r.random(c) + 0.5).astype(np.float32))]
+        if conv and c <= 100:
+            f = float32([c, c, 3, 3], (r.standard_normal((c, c, 3, 3)) * np.sqrt(2.0 / (9 * c))).astype(np.float32))
+            y = core.addBias(core.convolution(y, f, [1, 1], [1, 1]), float32([c], r.standard_normal(c).astype(np.float32)))
+        b = core.batchNormInference(y, *p)
+        return core.relu(b) if relu else b
+
+    a = layer(x)
+    b = layer(a)                                     # a is read twice: by this layer and below
+    outs = [core.maxpool(b, [2, 2]), a + b, core.maxpool(layer(b, relu=False), [2, 2]) if h > 1 else b, layer(a)]
+    d = layer(b)
+    pooled = core.maxpool(d, [2, 2])                 # only the pool reads d
+    outs += [core.sum(pooled), layer(b, relu=False)]
+    e = layer(a)
+    outs += [e, core.maxpool(e, [2, 2])]             # the value is an output as well
+    want = core.compile(outs).execute()
+    for flags in (core.PLAN_VIEWS | core.PLAN_FUSE, core.PLAN_VIEWS | core.PLAN_FUSE | core.PLAN_GRAPH,
+                  core.PLAN_VIEWS | core.PLAN_FUSE | core.PLAN_OVERLAP_LIGHT):
+        plan = core.compile(outs, flags)
+        bufs = [ops.Tensor(o.shape) for o in outs]
+        for _ in range(3):
+            plan.execute(None, bufs)
+            for got, v in zip(bufs, want):
+                assert np.array_equal(got.numpy(), v), flags
