@@ -1,5 +1,5 @@
 // Convolution forward, backward-data and backward-filter as implicit GEMMs on matrix instructions: most kernels on the bf16 one
-// with each fp32 value split into three parts (mfma_core.h), the direct 3 x 3 and the 2 x 2-image kernels on the fp32 one.
+// with each fp32 value split into three parts (mfma_core.h), the 2 x 2-image kernels on the fp32 one.
 // Replaces cudnnConvolutionForward / BackwardData / BackwardFilter as called at
 // cuda/source/dopt/cuda/nnet/cudnn7.d:154, :199, :244.  The reference configures cuDNN with
 // CUDNN_CONVOLUTION (cudnn7.d:87), i.e. a TRUE convolution: the filter is flipped,
@@ -256,18 +256,14 @@ __global__ __launch_bounds__(T::THREADS, T::THREADS / 128) void conv_gather_grou
 // Forward and backward-data of 3x3 unit-stride convolutions.  The gathered operand is not
 // re-fetched per filter tap: for a chunk of 16 input channels the block loads the input patch
 // under its pixel tile ONCE -- the tile's rows plus a one-pixel halo, zero-filled outside the
-// image by the buffer range check -- and the nine taps read it at nine offsets.  LDS holds the
-// patch position-major, Bp[pos][16 channels (+4 pad)], so that a lane's pixel operands for a whole
-// 16-channel slab are two 128-bit LDS reads per 32-wide fragment; the packed filter,
-// wp[slab][m][16 channels], has the same shape per row, and a lane's filter operands are two 128-bit
-// loads straight from it.  Lane half kh (= lane / 32) multiplies channels kh*8 .. kh*8+7 of the
-// chunk over the slab's eight matrix steps (the same channel permutation on both operands, so
-// every channel is counted once).  Per 32 matrix instructions a wavefront issues 4 patch fragment
-// reads, 4 filter loads and ~5 patch loads and stores.
+// image by the buffer range check -- and the nine taps read it at nine offsets.  LDS holds the patch by channel half and
+// position, so that a lane's pixel operands for a whole 16-channel slab are 128-bit LDS reads; the packed filter,
+// wp[slab][part][m][16 channels], has the same shape per row, and a lane's filter operands are 128-bit
+// loads straight from it.  Lane half kh (= lane / 32) multiplies channels kh*8 .. kh*8+7 of the chunk.
 
 struct PatchConv {
     const float *in;   // gathered operand [N, Cin, IH, IW]
-    const float *wp;   // packed filter [chunks][9][Mp][16]
+    const float *wp;   // packed filter [chunks][9][3 parts][Mp][16], bf16 (Winograd: 16 positions in the place of 9 taps)
     float *out;        // [N, Mout, OH, OW], or `splits` partial copies of it
     const float *bias; // optional [Mout], added to the finished sums (by the split reduction when there is one)
     int N, Cin, IH, IW, Mout, OH, OW;
@@ -275,28 +271,67 @@ struct PatchConv {
     int flip;          // 1: tap (tr,ts) reads patch offset (2-tr, 2-ts); 0: (tr, ts)
     int nimg, rows;    // images per pixel tile; output rows of each image in the tile
     int PR, PC, psz;   // patch rows and columns per image; patch positions per tile = nimg*PR*PC
-    unsigned magic_psz, magic_img, magic_pc;  // floor(2^32/d)+1 for d = psz, PR*PC, PC (exact for x*d < 2^32)
+    unsigned magic_img, magic_pc;  // floor(2^32/d)+1 for d = PR*PC, PC (exact for x*d < 2^32)
     unsigned magic_tpi, magic_tcn;            // Winograd: the same for the 2 x 2 tiles of one image in the pixel tile, and of one row
     int Mp;            // rows of one packed filter slab (Mout rounded up to the tile height)
     int ncols, mtiles, ntiles, chunks_total, chunks_per_split, splits;
-    size_t out_elems, in_bytes, wp_bytes;
+    size_t out_elems, in_bytes;
 };
+
+// Filters packed as bf16 parts.  A value whose parts are no numbers (2^103 and more, infinities, NaNs) has this NaN for its h part
+// and its bits as they are in the other two.
+constexpr unsigned short kPackedRaw = 0x7fff;
+
+// Two neighbouring channels' parts, each pair one word.
+__device__ __forceinline__ void split_packed(float a, float b, unsigned &h, unsigned &m, unsigned &l)
+{
+    split_pair(a * kSplitUp, b * kSplitUp, h, m, l);
+    const unsigned bits[2] = {__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b)};
+    constexpr unsigned kTop = 0x73000000u;   // 2^103
+    if (__any(max(bits[0] & 0x7fffffffu, bits[1] & 0x7fffffffu) >= kTop)) {
+#pragma unroll
+        for (int v = 0; v < 2; v++) {
+            const unsigned shift = 16 * v, keep = 0xffff0000u >> shift;
+            if ((bits[v] & 0x7fffffffu) < kTop) continue;
+            h = (h & keep) | (unsigned)kPackedRaw << shift;
+            m = (m & keep) | bits[v] >> 16 << shift;
+            l = (l & keep) | (bits[v] & 0xffffu) << shift;
+        }
+    }
+}
+
+// The fp32 value e of a fragment's eight.
+__device__ __forceinline__ float packed_value(const v4u (&f)[3], int e)
+{
+    unsigned q[3];
+#pragma unroll
+    for (int t = 0; t < 3; t++) q[t] = e & 1 ? f[t][e / 2] >> 16 : f[t][e / 2] & 0xffffu;
+    auto val = [&](int t) { return __builtin_bit_cast(float, q[t] << 16); };
+    return q[0] == kPackedRaw ? __builtin_bit_cast(float, q[1] << 16 | q[2]) : (val(0) + val(1) + val(2)) * (1.0f / kSplitUp);
+}
 
 __device__ inline unsigned fast_div(unsigned x, unsigned magic) { return __umulhi(x, magic); }
 
-// The filter fragments go from memory straight into the registers the matrix cores read: the
-// packed layout is the fragment layout (a wavefront fetches 32 rows x 64 bytes, 2 KB contiguous, per
-// 32 output channels and tap; the four wavefronts of a tile row fetch the same lines, three of them
-// from the L1), one tap ahead.  Only the patch goes through LDS, double buffered, so the workgroup
-// meets once per 16-channel chunk, when the patch buffers swap.  (Staging the filter slab in LDS as
-// well costs a barrier per tap: 1.1 % slower on the VGG step.)
-template <class T, int NPMAX, bool kCFull>
+// The products run on the bf16 matrix instruction (mfma_core.h).  A patch value is split once, when it is stored, and its parts
+// serve all nine taps of all rows, so splitting is a tenth of the loop.  The filter's parts are packed; its fragments go from
+// memory straight into the registers the matrix cores read: the packed layout is the fragment layout (a wavefront fetches 32
+// rows x 32 bytes, 1 KB contiguous, per part; wavefronts of a tile row fetch the same lines, all but one from the L1), one or two
+// taps ahead.  Only the patch goes through LDS, double buffered: [part][channel half][position][8 channels], a lane's fragment
+// of one part is one 128-bit read and neighbouring lanes' reads are neighbours.  The workgroup meets once per 16-channel chunk.
+// The h.h products have an accumulator of their own, the five small ones another.
+// Batch 128 on 32 x 32 images, the fp32 instruction -> this: 160 -> 16 channels 172 -> 54 us (tiles of 32 rows instead of 64: half
+// of that), 16 -> 160 78 -> 52, 32 -> 32 43 -> 19.  48 -> 48 channels: 40 us, of which 25 are matrix time at the rate that a large
+// product reaches; the rest is the first patch and the last stores of a workgroup (half as large tiles, two workgroups per CU: 41).
+template <class T, int NS, bool kCFull>
 __device__ __forceinline__ void conv_patch_body(const PatchConv &p, const unsigned block_id)
 {
     constexpr int BM = T::BM, BN = T::BN, THREADS = T::THREADS, MI = T::MI, NI = T::NI;
-    constexpr int TAPS = 9, CH = 16, LDP = 20;
+    constexpr int TAPS = 9, CH = 16;
+    constexpr int AHEAD = MI == 1 ? 2 : 1, RING = AHEAD + 1;   // filter fragments on their way: a tap of MI = 1 lasts half as long
+    static_assert(TAPS % RING == 0 || RING == 2, "the ring slot of a tap follows from its number");
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    const int pstride = (p.psz + 1) * LDP;  // one spare position absorbs the stores of unused slots
+    const int area = p.psz + 1;              // one spare position absorbs the stores of unused slots
+    const int pstride = area * 24;           // floats of one patch buffer: 3 parts x 2 halves x 4 words a position
     float *const Bp0 = lds;                  // [2][pstride]
 
     unsigned L;
@@ -309,138 +344,201 @@ __device__ __forceinline__ void conv_patch_body(const PatchConv &p, const unsign
     const int cb = split * p.chunks_per_split;
     const int ce = min(cb + p.chunks_per_split, p.chunks_total);
 
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = w / T::WN, wn = w % T::WN;
     const int kh = lane >> 5, l32 = lane & 31;
     const int OHW = p.OH * p.OW;
     const int chan_stride = p.IH * p.IW;
 
     const __amdgpu_buffer_rsrc_t rin = make_rsrc(p.in, p.in_bytes);
-    const __amdgpu_buffer_rsrc_t rwp = make_rsrc(p.wp, p.wp_bytes);
 
-    // ---- patch slots of this thread: element e = i*THREADS + tid -> (channel e / psz, position e % psz)
+    // ---- patch slots of this thread: eight channels (one half of the chunk) of one position each
     const int n_first = n0 / OHW, oh0 = (n0 - n_first * OHW) / p.OW;
-    unsigned p_voff[NPMAX];  // byte offset of the element inside channel chunk 0, or kOobOffset
-    int p_lds[NPMAX];        // byte offset inside a patch buffer
-    int p_chan[NPMAX];       // channel inside the chunk (only read when the last chunk is ragged)
+    unsigned p_voff[NS];   // byte offset of the slot's first channel inside chunk 0, or kOobOffset
+    int p_lds[NS];         // float offset inside a patch buffer
+    int p_left[NS];        // channels from the slot's first one to the last (only read when the last chunk is ragged)
 #pragma unroll
-    for (int i = 0; i < NPMAX; i++) {
-        const unsigned e = (unsigned)(i * THREADS + tid);
-        const unsigned c = fast_div(e, p.magic_psz);
-        const unsigned pos = e - c * (unsigned)p.psz;
+    for (int i = 0; i < NS; i++) {
+        const int e = i * THREADS + tid, half = e >= 2 * p.psz ? 2 : e >= p.psz ? 1 : 0;
+        const unsigned pos = (unsigned)(half == 2 ? 0 : e - half * p.psz);
         const unsigned img = fast_div(pos, p.magic_img);
         const unsigned rem = pos - img * (unsigned)(p.PR * p.PC);
         const unsigned pr = fast_div(rem, p.magic_pc);
         const unsigned pc = rem - pr * (unsigned)p.PC;
         const int n = n_first + (int)img, ih = oh0 + (int)pr - p.PT, iw = (int)pc - p.PL;
-        const int bad = (CH - 1 - (int)c) | (p.N - 1 - n) | ih | (p.IH - 1 - ih) | iw | (p.IW - 1 - iw);
-        p_voff[i] = bad < 0 ? kOobOffset : (unsigned)(((n * p.Cin + (int)c) * p.IH + ih) * p.IW + iw) * 4u;
-        p_lds[i] = c < (unsigned)CH ? (int)(pos * LDP + c) * 4 : (p.psz * LDP + (tid & 15)) * 4;
-        p_chan[i] = (int)c;
+        const int bad = (1 - half) | (p.N - 1 - n) | ih | (p.IH - 1 - ih) | iw | (p.IW - 1 - iw);
+        p_voff[i] = bad < 0 ? kOobOffset : (unsigned)(((n * p.Cin + half * 8) * p.IH + ih) * p.IW + iw) * 4u;
+        p_lds[i] = half == 2 ? p.psz * 4 : (half * area + (int)pos) * 4;
+        p_left[i] = p.Cin - half * 8;
     }
-    float preg[NPMAX];
-    auto patch_load = [&](int i, int chunk) {
+    float preg[NS][8];
+    auto patch_load = [&](int i, int c, int chunk) {
         unsigned voff = p_voff[i];
-        if (!kCFull) voff = chunk * CH + p_chan[i] < p.Cin ? voff : kOobOffset;
-        preg[i] = buffer_load_f32(rin, voff, (unsigned)(chunk * CH * chan_stride) * 4u);
+        if (!kCFull) voff = chunk * CH + c < p_left[i] ? voff : kOobOffset;
+        preg[i][c] = buffer_load_f32(rin, voff, (unsigned)((chunk * CH + c) * chan_stride) * 4u);
     };
-    auto patch_store = [&](int i, float *buf) { *(float *)((char *)buf + p_lds[i]) = preg[i]; };
-
-    // ---- filter fragments: this lane's 8 channels (kh * 8 ..) of row l32 of each 32-row group
-    const unsigned slab_bytes = (unsigned)p.Mp * CH * 4u;
-    const unsigned fa_voff = (unsigned)((m0 + wm * (BM / T::WM) + l32) * CH + kh * 8) * 4u;   // m0 + row < Mp always
-    // three sets of filter fragments: the tap being multiplied, the next one, and the one after it on its way (a tap
-    // lasts ~0.4 us per wavefront, less than a load from the L2 can take under load)
-    float4 fa_ring[3][MI][2];
-    auto fa_load = [&](auto slot_tag, int slab) {   // past the last slab the range check returns zeros
-        constexpr int slot = decltype(slot_tag)::value;
+    auto patch_store = [&](int i, float *buf, const unsigned (&q)[3][4]) {
 #pragma unroll
-        for (int i = 0; i < MI; i++) {
-            fa_ring[slot][i][0] = buffer_load_f32x4(rwp, fa_voff + (unsigned)(i * 32 * CH) * 4u, (unsigned)slab * slab_bytes);
-            fa_ring[slot][i][1] = buffer_load_f32x4(rwp, fa_voff + (unsigned)(i * 32 * CH) * 4u + 16u, (unsigned)slab * slab_bytes);
-        }
+        for (int t = 0; t < 3; t++) *(v4u *)(buf + p_lds[i] + t * 2 * area * 4) = v4u{q[t][0], q[t][1], q[t][2], q[t][3]};
     };
-    int b_frag[NI];  // float offset inside a patch buffer of this lane's pixel, tap offset (0,0)
+    auto patch_split = [&](int i, int e, unsigned (&q)[3][4]) {
+        split_pair(preg[i][2 * e] * kSplitUp, preg[i][2 * e + 1] * kSplitUp, q[0][e], q[1][e], q[2][e]);
+    };
+
+    // ---- filter fragments: this lane's 8 channels (kh * 8 ..) of row l32 of each 32-row group: [chunk][tap][part][row][16]
+    const unsigned part_bytes = (unsigned)p.Mp * CH * 2u, slab_bytes = 3u * part_bytes;
+    const unsigned fa_voff = (unsigned)((m0 + wm * (BM / T::WM) + l32) * CH + kh * 8) * 2u;   // m0 + row < Mp always
+    v4u fa_ring[RING][MI][3];
+    // (the packed filter may be larger than a buffer resource reaches: a resource per chunk)
+    auto fa_rsrc = [&](int chunk) { return make_rsrc((const char *)p.wp + (size_t)chunk * TAPS * slab_bytes, (size_t)TAPS * slab_bytes); };
+    auto fa_load = [&](int slot, __amdgpu_buffer_rsrc_t rwp, int tap) {
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int t = 0; t < 3; t++)
+                fa_ring[slot][i][t] = __builtin_bit_cast(v4u, buffer_load_f32x4(rwp, fa_voff + (unsigned)(i * 32 * CH) * 2u,
+                                                                               (unsigned)tap * slab_bytes + t * part_bytes));
+    };
+    int b_pos[NI];  // this lane's pixel and channel half in the area of a part, in positions, tap offset (0,0)
 #pragma unroll
     for (int j = 0; j < NI; j++) {
         const int q = wn * (BN / T::WN) + j * 32 + l32;  // pixel inside the tile
         const int img = q / (p.rows * p.OW), r = q / p.OW - img * p.rows, col = q % p.OW;
-        b_frag[j] = ((img * p.PR + r) * p.PC + col) * LDP + kh * 8;
+        b_pos[j] = kh * area + (img * p.PR + r) * p.PC + col;
     }
+    auto tap_offset = [&](int t) { return p.flip ? (2 - t / 3) * p.PC + (2 - t % 3) : t / 3 * p.PC + t % 3; };
 
-    v16f acc[MI][NI];
+    v16f acc[MI][NI], low[MI][NI];
     zero_acc(acc);
+    zero_acc(low);
 
-    // prologue: the first patch and the first filter slab
+    // prologue: the first patch and the first filter slabs
 #pragma unroll
-    for (int i = 0; i < NPMAX; i++) patch_load(i, cb);
-    fa_load(StepTag<0>{}, cb * TAPS);
-    fa_load(StepTag<1>{}, cb * TAPS + 1);
+    for (int i = 0; i < NS; i++)
 #pragma unroll
-    for (int i = 0; i < NPMAX; i++) patch_store(i, Bp0);
+        for (int c = 0; c < 8; c++) patch_load(i, c, cb);
+#pragma unroll
+    for (int t = 0; t < AHEAD; t++) fa_load(t, fa_rsrc(cb), t);
+#pragma unroll
+    for (int i = 0; i < NS; i++) {
+        unsigned q[3][4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) patch_split(i, e, q);
+        patch_store(i, Bp0, q);
+    }
     __syncthreads();
 
-    int pcur = 0;
-    int sidx = cb * TAPS;  // filter slab being multiplied
-    // loads of the next patch are issued during taps 0..3 of a chunk, its LDS stores during taps 5..8
-    constexpr int PER = (NPMAX + 3) / 4;
-    for (int chunk = cb; chunk < ce; ++chunk) {
-        float *const bp_cur = Bp0 + pcur * pstride;
-        float *const bp_nxt = Bp0 + (pcur ^ 1) * pstride;
+    v4u fb[NI][3];
+    auto fb_load = [&](int part, const float *bp, int t) {
+        const int off = part * 2 * area + tap_offset(t);
+#pragma unroll
+        for (int j = 0; j < NI; j++) fb[j][part] = *(const v4u *)(bp + (off + b_pos[j]) * 4);
+    };
+    fb_load(2, Bp0, 0);
+    fb_load(1, Bp0, 0);
+
+    // The next patch is loaded during taps 0 .. 3 of a chunk and split and stored during taps 5 .. 7; the workgroup meets in
+    // tap 8, behind the last reads of the patch being multiplied.
+    constexpr int PER = NS * 2;   // loads of a tap
+    static_assert(NS <= 3, "a slot per tap 5 .. 7");
+    int ring = 0;   // (two slots: nine taps leave the ring turned)
+    auto chunk_products = [&](int chunk, const float *bp_cur, float *bp_nxt, auto turned_tag) {
+        constexpr int turned = decltype(turned_tag)::value;
+        const __amdgpu_buffer_rsrc_t rw_now = fa_rsrc(chunk), rw_next = fa_rsrc(chunk + 1 < ce ? chunk + 1 : chunk);   // (after the last chunk: loaded, not used)
+        unsigned q[3][4];
+#pragma unroll
+        for (int j = 0; j < NI; j++) asm volatile("" : "+v"(b_pos[j]));   // (or the fifty-four addresses of a chunk are kept in registers)
         static_for<0, TAPS>([&](auto ttag) {
             constexpr int t = decltype(ttag)::value;
-            constexpr int tr = t / 3, ts = t % 3;
-            const int tapoff = (p.flip ? (2 - tr) * p.PC + (2 - ts) : tr * p.PC + ts) * LDP;
-            float4 fa[MI][2], fb[NI][2];
-#pragma unroll
-            for (int i = 0; i < MI; i++) {   // nine taps per chunk: the ring slot of a tap is the same in every chunk
-                fa[i][0] = fa_ring[t % 3][i][0];
-                fa[i][1] = fa_ring[t % 3][i][1];
-            }
-#pragma unroll
-            for (int j = 0; j < NI; j++) {
-                fb[j][0] = *(const float4 *)(bp_cur + b_frag[j] + tapoff);
-                fb[j][1] = *(const float4 *)(bp_cur + b_frag[j] + tapoff + 4);
-            }
-            static_for<0, 8>([&](auto stag) {
+            constexpr int slot = (t + turned) % RING;
+            // the pixel part that is used last is read first again: l after its one product, m after its two, h at the tap's start
+            static_for<0, 6>([&](auto stag) {
                 constexpr int ks = decltype(stag)::value;
-                // side work of this step
-                if constexpr (ks == 0) fa_load(StepTag<(t + 2) % 3>{}, sidx + 2);
-                if constexpr (t < 4 && ks >= 1 && ks <= 6) {
-                    // PER loads of tap t, dealt over steps 1..6
-                    constexpr int first = t * PER + (ks - 1) * ((PER + 5) / 6);
-                    constexpr int last = first + (PER + 5) / 6;
-#pragma unroll
-                    for (int i = first; i < last; i++)
-                        if (i < (t + 1) * PER && i < NPMAX) patch_load(i, chunk + 1);
+                constexpr int qb = ks == 0 ? 2 : ks <= 2 ? 1 : 0;
+                constexpr int qa = ks == 0 ? 0 : ks == 1 ? 1 : ks == 2 ? 0 : ks == 3 ? 2 : ks == 4 ? 1 : 0;
+                // side work of this step, pinned to it
+                if constexpr (ks == 0) {
+                    fa_load((t + AHEAD + turned) % RING, t + AHEAD < TAPS ? rw_now : rw_next, (t + AHEAD) % TAPS);
+                    fb_load(0, bp_cur, t);
+                    if constexpr (t == TAPS - 1) __syncthreads();
                 }
-                if constexpr (t >= 5 && ks >= 1 && ks <= 6) {
-                    constexpr int first = (t - 5) * PER + (ks - 1) * ((PER + 5) / 6);
-                    constexpr int last = first + (PER + 5) / 6;
+                if constexpr (ks == 1) fb_load(2, t == TAPS - 1 ? bp_nxt : bp_cur, (t + 1) % TAPS);
+                if constexpr (ks == 3) fb_load(1, t == TAPS - 1 ? bp_nxt : bp_cur, (t + 1) % TAPS);
+                if constexpr (t < 4) {
 #pragma unroll
-                    for (int i = first; i < last; i++)
-                        if (i < (t - 4) * PER && i < NPMAX) patch_store(i, bp_nxt);
+                    for (int i = ks * PER / 6; i < (ks + 1) * PER / 6; i++) patch_load((t * PER + i) / 8, (t * PER + i) % 8, chunk + 1);
+                }
+                if constexpr (t >= 5 && t - 5 < NS) {
+                    if constexpr (ks < 4) patch_split(t - 5, ks, q);
+                    if constexpr (ks == 4) patch_store(t - 5, bp_nxt, q);
                 }
 #pragma unroll
                 for (int i = 0; i < MI; i++)
 #pragma unroll
                     for (int j = 0; j < NI; j++) {
-                        const float4 av = fa[i][ks / 4], bv = fb[j][ks / 4];
-                        const float a = ks % 4 == 0 ? av.x : ks % 4 == 1 ? av.y : ks % 4 == 2 ? av.z : av.w;
-                        const float b = ks % 4 == 0 ? bv.x : ks % 4 == 1 ? bv.y : ks % 4 == 2 ? bv.z : bv.w;
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc[i][j], 0, 0, 0);
+                        v16f &c = ks < 5 ? low[i][j] : acc[i][j];
+                        c = mfma_bf16(fa_ring[slot][i][qa], fb[j][qb], c);
                     }
-#pragma unroll
-                for (int g = 0; g < MI * NI; g++) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x216, 2, 0);
-                }
                 __builtin_amdgcn_sched_barrier(0);
             });
-            if constexpr (t == TAPS - 1) __syncthreads();
-            ++sidx;
         });
-        pcur ^= 1;
+    };
+    for (int chunk = cb; chunk < ce; ++chunk) {
+        float *const bp_cur = Bp0 + ((chunk - cb) & 1) * pstride;
+        float *const bp_nxt = Bp0 + ((chunk - cb + 1) & 1) * pstride;
+        if (RING == 2 && ring) chunk_products(chunk, bp_cur, bp_nxt, StepTag<1>{});
+        else chunk_products(chunk, bp_cur, bp_nxt, StepTag<0>{});
+        ring ^= 1;
+    }
+    add_acc(acc, low);
+
+    // the parts of an infinity hold NaNs: a tile that is not finite is formed again with the fp32 instruction, one chunk after the
+    // other (a word per wavefront: in a backward pair the workgroup's surplus wavefronts have ended)
+    __syncthreads();
+    {
+        const int mine = __any(not_finite(acc));
+        if (lane == 0) ((int *)lds)[w] = mine;
+        __syncthreads();
+        int bad = 0;
+#pragma unroll
+        for (int i = 0; i < THREADS / 64; i++) bad |= ((const int *)lds)[i];
+        if (bad) {
+            zero_acc(acc);
+#pragma unroll 1
+            for (int chunk = cb; chunk < ce; chunk++) {
+                __syncthreads();
+#pragma unroll
+                for (int i = 0; i < NS; i++) {   // patch here: [half][position][8 channels]
+#pragma unroll
+                    for (int c = 0; c < 8; c++) patch_load(i, c, chunk);
+                    *(float4 *)(Bp0 + p_lds[i] * 2) = make_float4(preg[i][0], preg[i][1], preg[i][2], preg[i][3]);
+                    *(float4 *)(Bp0 + p_lds[i] * 2 + 4) = make_float4(preg[i][4], preg[i][5], preg[i][6], preg[i][7]);
+                }
+                __syncthreads();
+                const __amdgpu_buffer_rsrc_t rw = fa_rsrc(chunk);
+#pragma unroll 1
+                for (int t = 0; t < TAPS; t++) {
+                    fa_load(0, rw, t);
+                    const int off = tap_offset(t);
+                    float b8[NI][8];
+#pragma unroll
+                    for (int j = 0; j < NI; j++) {
+                        const float4 b0 = *(const float4 *)(Bp0 + (off + b_pos[j]) * 8), b1 = *(const float4 *)(Bp0 + (off + b_pos[j]) * 8 + 4);
+                        b8[j][0] = b0.x; b8[j][1] = b0.y; b8[j][2] = b0.z; b8[j][3] = b0.w;
+                        b8[j][4] = b1.x; b8[j][5] = b1.y; b8[j][6] = b1.z; b8[j][7] = b1.w;
+                    }
+#pragma unroll
+                    for (int i = 0; i < MI; i++)
+#pragma unroll
+                        for (int e = 0; e < 8; e++) {
+                            const float a = packed_value(fa_ring[0][i], e);
+#pragma unroll
+                            for (int j = 0; j < NI; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b8[j][e], acc[i][j], 0, 0, 0);
+                        }
+                }
+            }
+        }
     }
 
     float *outp = p.out + (size_t)split * p.out_elems;
@@ -461,10 +559,11 @@ __device__ __forceinline__ void conv_patch_body(const PatchConv &p, const unsign
     }
 }
 
-template <class T, int NPMAX, bool kCFull>
-__global__ __launch_bounds__(T::THREADS, T::THREADS / 256) void conv_patch_k(PatchConv p)
+// (two wavefronts per SIMD: as one workgroup of eight, or two of four)
+template <class T, int NS, bool kCFull>
+__global__ __launch_bounds__(T::THREADS, 2) void conv_patch_k(PatchConv p)
 {
-    conv_patch_body<T, NPMAX, kCFull>(p, blockIdx.x);
+    conv_patch_body<T, NS, kCFull>(p, blockIdx.x);
 }
 
 // ------------------------------------------------------------------------------------ Winograd F(2x2, 3x3)
@@ -503,10 +602,6 @@ __global__ __launch_bounds__(T::THREADS, T::THREADS / 256) void conv_patch_k(Pat
 // barriers, no transform 19 %.  64-row tiles in the place of 128-row tiles: 721 us for the first of the layers above.
 // floats of the exchange area: 128 rows: four wavefront pairs x 64 values per lane; 64 rows: eight wavefronts x 64 values
 constexpr int wino_xchg(int bm) { return (bm == 128 ? 4 : 8) * 64 * 64; }
-
-// A packed filter value whose parts are no numbers (2^103 and more, infinities, NaNs) has this NaN for its h part and its bits as
-// they are in the other two.
-constexpr unsigned short kWinoRaw = 0x7fff;
 
 // WK x TH: WK groups of 32 rows, TH groups of 32 tiles: 4 x 1 (128 rows x 32 tiles = 128 pixels) for layers with whole
 // 128-row tiles, 2 x 2 (64 rows x 64 tiles = 256 pixels) for 64-row layers.
@@ -871,12 +966,7 @@ __global__ __launch_bounds__(512, 1) void conv_wino_k(PatchConv p)
                 const float b8[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
-                    unsigned q[3];
-#pragma unroll
-                    for (int t = 0; t < 3; t++) q[t] = e & 1 ? fa_ring[0][t][e / 2] >> 16 : fa_ring[0][t][e / 2] & 0xffffu;
-                    auto val = [&](int t) { return __builtin_bit_cast(float, q[t] << 16); };
-                    const float a = q[0] == kWinoRaw ? __builtin_bit_cast(float, q[1] << 16 | q[2])
-                                                     : (val(0) + val(1) + val(2)) * (1.0f / kSplitUp);
+                    const float a = packed_value(fa_ring[0], e);
                     acc[xl] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b8[e], acc[xl], 0, 0, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -947,19 +1037,7 @@ __device__ __forceinline__ void wino_pack_tile(int M, int Cred, int Mp, size_t s
                 const float other = __shfl_xor(odd ? u[e] : u[e + 1], 1);
                 unsigned ph, pm, pl;
                 const float a = odd ? other : u[e], b = odd ? u[e + 1] : other;
-                split_pair(a * kSplitUp, b * kSplitUp, ph, pm, pl);
-                const unsigned bits[2] = {__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b)};
-                constexpr unsigned kTop = 0x73000000u;   // 2^103
-                if (__any(max(bits[0] & 0x7fffffffu, bits[1] & 0x7fffffffu) >= kTop)) {
-#pragma unroll
-                    for (int v = 0; v < 2; v++) {
-                        const unsigned shift = 16 * v, keep = 0xffff0000u >> shift;
-                        if ((bits[v] & 0x7fffffffu) < kTop) continue;
-                        ph = (ph & keep) | (unsigned)kWinoRaw << shift;
-                        pm = (pm & keep) | bits[v] >> 16 << shift;
-                        pl = (pl & keep) | (bits[v] & 0xffffu) << shift;
-                    }
-                }
+                split_packed(a, b, ph, pm, pl);
                 unsigned *dst = (unsigned *)wp + ((((size_t)chunk * 16 + r * 4 + e + odd) * 3) * Mp + m0 + ml) * 8 + (j >> 1);
                 dst[0] = ph;
                 dst[part] = pm;
@@ -969,8 +1047,8 @@ __device__ __forceinline__ void wino_pack_tile(int M, int Cred, int Mp, size_t s
     }
 }
 
-// Packed filter of the patch kernel: wp[((chunk*9 + tap)*Mp + m)*16 + j] = w[m*sm + (chunk*16+j)*sc + tap]
-// (zero where m >= M or the channel is past the end).  Forward: m = output channel k (sm = C*9,
+// Packed filter of the patch kernel: wp[(((chunk*9 + tap)*3 + part)*Mp + m)*16 + j], the bf16 parts of w[m*sm + (chunk*16+j)*sc + tap]
+// times kSplitUp (zero where m >= M or the channel is past the end).  Forward: m = output channel k (sm = C*9,
 // sc = 9); backward-data: m = input channel c (sm = 9, sc = C*9), reduction over k.
 // A block transposes 16 rows of one chunk through LDS.  Its source is 16 contiguous runs of 144
 // floats (forward: one per row, its 16 channels x 9 taps; backward: one per reduction channel,
@@ -1004,7 +1082,7 @@ __device__ __forceinline__ void pack_tile(int M, int Cred, int Mp, size_t sm, si
         stage[(f / 144) * PITCH + f % 144] = v[i];
     }
     __syncthreads();
-    // one float4 (four channels of one row and tap) per thread and pass
+    // four channels of one row and tap per thread and pass
     for (int o = threadIdx.x; o < 9 * 16 * 4; o += 256) {
         const int j4 = o & 3, ml = (o >> 2) & 15, tap = o >> 6;
         float4 q;
@@ -1015,7 +1093,12 @@ __device__ __forceinline__ void pack_tile(int M, int Cred, int Mp, size_t sm, si
             const float *s = stage + (j4 * 4) * PITCH + ml * 9 + tap;
             q = make_float4(s[0], s[PITCH], s[2 * PITCH], s[3 * PITCH]);
         }
-        *(float4 *)&wp[(((size_t)chunk * 9 + tap) * Mp + m0 + ml) * 16 + j4 * 4] = q;
+        uint2 part[3];
+        split_packed(q.x, q.y, part[0].x, part[1].x, part[2].x);
+        split_packed(q.z, q.w, part[0].y, part[1].y, part[2].y);
+        uint2 *dst = (uint2 *)wp + ((((size_t)chunk * 9 + tap) * 3) * Mp + m0 + ml) * 4 + j4;
+#pragma unroll
+        for (int t = 0; t < 3; t++) dst[(size_t)t * Mp * 4] = part[t];
     }
 }
 
@@ -1712,12 +1795,12 @@ __global__ __launch_bounds__(64 * 3 * WM * WC, 1) void conv_wgrad_patch_k(WgradP
 // tile at once instead of idling until the slowest tile of the launch is done and the next launch has ramped up.
 // Launched with the filter gradient's 768 threads: the wavefronts a backward-data workgroup does not need end
 // at once (a barrier waits for the surviving wavefronts only).
-template <class T, int NPMAX, int WM, int WC, int kGeo>
+template <class T, int NS, int WM, int WC, int kGeo>
 __global__ __launch_bounds__(768, 1) void conv_bwd_pair_k(PatchConv a, WgradPatch b, unsigned grid_a)
 {
     if (blockIdx.x < grid_a) {
         if (threadIdx.x >= (unsigned)T::THREADS) return;
-        conv_patch_body<T, NPMAX, true>(a, blockIdx.x);
+        conv_patch_body<T, NS, true>(a, blockIdx.x);
     } else {
         conv_wgrad_patch_body<WM, WC, kGeo>(b, blockIdx.x - grid_a);
     }
@@ -1866,18 +1949,24 @@ using GatherTall = Tile<160, 128, 1, 4>;    // 160 output channels (and 480, ...
 
 unsigned div_magic(unsigned d) { return (unsigned)((((unsigned long long)1 << 32) / d) + 1); }
 
-template <class T, int NPMAX>
+// Tiles of the direct 3 x 3 kernel.
+using PatchNarrow = Tile<32, 256, 1, 4>;    // up to 32 output channels: 64 rows would multiply as many zeros
+using PatchWide = Tile<64, 256, 2, 4>;
+using PatchDeep = Tile<128, 128, 4, 2>;
+using PatchTall = Tile<160, 128, 5, 2>;     // 160 output channels (and 480, ...)
+
+template <class T, int NS>
 int launch_patch(const PatchConv &pc, bool c_full, dim3 grid, size_t lds_bytes)
 {
     // above 64 KB of dynamic LDS a kernel has to be told once
     static bool raised[2] = {false, false};
     if (!raised[c_full]) {
-        const void *fn = c_full ? (const void *)conv_patch_k<T, NPMAX, true> : (const void *)conv_patch_k<T, NPMAX, false>;
+        const void *fn = c_full ? (const void *)conv_patch_k<T, NS, true> : (const void *)conv_patch_k<T, NS, false>;
         DOPT_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         raised[c_full] = true;
     }
-    if (c_full) hipLaunchKernelGGL((conv_patch_k<T, NPMAX, true>), grid, dim3(T::THREADS), lds_bytes, stream(), pc);
-    else hipLaunchKernelGGL((conv_patch_k<T, NPMAX, false>), grid, dim3(T::THREADS), lds_bytes, stream(), pc);
+    if (c_full) hipLaunchKernelGGL((conv_patch_k<T, NS, true>), grid, dim3(T::THREADS), lds_bytes, stream(), pc);
+    else hipLaunchKernelGGL((conv_patch_k<T, NS, false>), grid, dim3(T::THREADS), lds_bytes, stream(), pc);
     DOPT_LAUNCH_CHECK();
     return DOPT_HIP_OK;
 }
@@ -1889,8 +1978,9 @@ int launch_patch(const PatchConv &pc, bool c_full, dim3 grid, size_t lds_bytes)
 struct PatchSetup {
     bool ok;
     PatchConv pc;
-    int shape;            // 0 wide, 1 square, 2 deep, 3 tall, 4 Winograd (BM 128: 128 rows x 32 tiles of 2x2 pixels, BM 64: 64 rows x 64 tiles)
+    int shape;            // 0 wide, 1 narrow, 2 deep, 3 tall, 4 Winograd (BM 128: 128 rows x 32 tiles of 2x2 pixels, BM 64: 64 rows x 64 tiles)
     int BM, BN, blocks_wanted, tiles;
+    int positions;        // of a patch that the workgroup's load slots hold
     size_t lds_bytes, wp_elems;
 };
 
@@ -1937,7 +2027,6 @@ PatchSetup patch_setup_as(const dopt_hip_conv_desc *d, size_t P, size_t Q, bool 
         pc.PT = 2 - (int)d->padH; pc.PL = 2 - (int)d->padW; pc.flip = 0;
     }
     pc.ncols = pc.N * pc.OH * pc.OW;
-    int npmax, threads;
     // 160-row tiles where they pad no more than both other heights (160 channels: 160 rows, not 192 or 256; 320 and 640
     // channels: two and four such tiles - on 8 x 8 images 640 channels are then exactly 256 tiles, one per compute unit
     // with no split of the reduction, where 128-row tiles gave 320 and a four-way split); 64-row tiles for up to 64 output
@@ -1955,17 +2044,16 @@ PatchSetup patch_setup_as(const dopt_hip_conv_desc *d, size_t P, size_t Q, bool 
         if (pc.Mout % wino != 0 && !(wino == 64 && pc.Mout > 64 && up64 * 5 <= pc.Mout * 6)) return u;
         // whole 128-row tiles of 32 tiles (128 pixels), or whole 64-row tiles of 64 tiles (256 pixels)
         u.shape = 4; u.BM = wino; u.BN = u.BM == 128 ? 128 : 256;
-        u.blocks_wanted = num_cus(); npmax = 16; threads = 512;
+        u.blocks_wanted = num_cus(); u.positions = 512;
     } else if (allow_tall && pc.Mout > 64 && up160 <= up64 && up160 <= up128 && tall_tiles >= num_cus() &&
         !no_tall_tiles()) {
-        u.shape = 3; u.BM = 160; u.BN = 128; u.blocks_wanted = num_cus(); npmax = 16; threads = 256;
+        u.shape = 3; u.BM = 160; u.BN = 128; u.blocks_wanted = num_cus(); u.positions = 256;
+    } else if (pc.Mout <= 32) {   // (16 -> 16 channels on 32 x 32 images, batch 64: 18 us with 64 rows in fp32, 10 us)
+        u.shape = 1; u.BM = 32; u.BN = 256; u.blocks_wanted = 2 * num_cus(); u.positions = 384;
     } else if (pc.Mout <= 64 || up64 < up128) {
-        u.shape = 0; u.BM = 64; u.BN = 256; u.blocks_wanted = 2 * num_cus(); npmax = 24; threads = 256;
+        u.shape = 0; u.BM = 64; u.BN = 256; u.blocks_wanted = num_cus(); u.positions = 384;
     } else {
-        u.BM = 128; u.BN = 128;
-        const int t = ((pc.Mout + 127) / 128) * ((pc.ncols + 127) / 128);
-        if (t >= 2 * num_cus()) { u.shape = 1; u.blocks_wanted = 2 * num_cus(); npmax = 16; threads = 256; }
-        else { u.shape = 2; u.blocks_wanted = num_cus(); npmax = 16; threads = 512; }
+        u.shape = 2; u.BM = 128; u.BN = 128; u.blocks_wanted = num_cus(); u.positions = 512;
     }
     const int BM = u.BM, BN = u.BN;
     // pixel tile = `rows` full rows of one image, or `nimg` whole images
@@ -1980,8 +2068,8 @@ PatchSetup patch_setup_as(const dopt_hip_conv_desc *d, size_t P, size_t Q, bool 
     }
     pc.PR = pc.rows + 2; pc.PC = pc.OW + 2;
     pc.psz = pc.nimg * pc.PR * pc.PC;
-    if ((size_t)pc.psz * 16 > (size_t)npmax * threads) return u;
-    u.lds_bytes = (size_t)2 * (pc.psz + 1) * 20 * sizeof(float);
+    if (pc.psz > u.positions) return u;
+    u.lds_bytes = (size_t)2 * (pc.psz + 1) * 24 * sizeof(float);
     if (wino) {
         if (pc.rows % 2 != 0) return u;   // a pixel tile is whole 2 x 2 tiles
         pc.magic_tpi = div_magic((unsigned)(pc.rows / 2 * (pc.OW / 2)));
@@ -1991,7 +2079,6 @@ PatchSetup patch_setup_as(const dopt_hip_conv_desc *d, size_t P, size_t Q, bool 
         u.lds_bytes = std::max(floats, (size_t)wino_xchg(u.BM) + 8) * sizeof(float);
     }
     if (u.lds_bytes > 160 * 1024) return u;
-    pc.magic_psz = div_magic((unsigned)pc.psz);
     pc.magic_img = div_magic((unsigned)(pc.PR * pc.PC));
     pc.magic_pc = div_magic((unsigned)pc.PC);
     pc.mtiles = (pc.Mout + BM - 1) / BM;
@@ -2000,10 +2087,9 @@ PatchSetup patch_setup_as(const dopt_hip_conv_desc *d, size_t P, size_t Q, bool 
     pc.chunks_total = (pc.Cin + 15) / 16;
     pc.out_elems = (size_t)pc.ncols * pc.Mout;
     u.tiles = pc.mtiles * pc.ntiles;
-    u.wp_elems = (size_t)pc.chunks_total * (wino ? 16 * 24 : 9 * 16) * pc.Mp;   // (Winograd: three 16-bit parts a value)
-    // the direct kernel's offsets into its packed filter reach 2 GiB (few rows, padded to a tile, of very many channels);
-    // the others' start anew with every chunk
-    if (!wino && u.wp_elems * sizeof(float) > 0x7fffffffu) return u;
+    u.wp_elems = (size_t)pc.chunks_total * (wino ? 16 : 9) * 24 * pc.Mp;   // three 16-bit parts a value
+    // (few rows of very many channels, whose copy in fp32, padded to 64 rows, would reach 2 GiB, are the general kernels')
+    if (!wino && (size_t)pc.chunks_total * 9 * 64 * std::max(pc.Mp, 64) > 0x7fffffffu) return u;
     u.ok = true;
     return u;
 }
@@ -2029,9 +2115,9 @@ PackJob pack_job(const dopt_hip_conv_desc *d, const PatchSetup &u, const float *
 // in microseconds: rounds x (chunks per block x time per chunk + a fixed prologue/epilogue) plus,
 // when split, writing and re-reading the partial tiles.  The split with the lowest estimate wins;
 // ties go to the smaller one.
-int patch_splits(int tiles, int chunks, int slots, int BM, int BN, size_t out_elems)
+int patch_splits(int tiles, int chunks, int slots, int BM, int BN, size_t out_elems, bool wino)
 {
-    const double cu_tflops = 0.47;                                   // what one CU sustains in these main loops
+    const double cu_tflops = wino ? 0.47 : 0.8;                      // what one CU sustains in these main loops (direct: 0.47 in fp32)
     const double per_cu = (double)slots / num_cus();                 // blocks sharing a CU
     // 16 channels x 9 taps.  The Winograd kernel takes a third of that for a chunk, but adds all six parts of a product in one
     // accumulator: with its own time here it would be cut less and be further off than the fp32 instruction, which was cut by
@@ -2082,7 +2168,7 @@ int gather_splits(int tiles, int slabs, int slots, int BM, int BN, size_t out_el
 int patch_decide_splits(PatchSetup *u, const float *out)
 {
     PatchConv &pc = u->pc;
-    int splits = patch_splits(u->tiles, pc.chunks_total, u->blocks_wanted, u->BM, u->BN, pc.out_elems);
+    int splits = patch_splits(u->tiles, pc.chunks_total, u->blocks_wanted, u->BM, u->BN, pc.out_elems, u->shape == 4);
     if (pc.out_elems % 4 != 0 || !aligned16(out)) splits = 1;
     pc.chunks_per_split = (pc.chunks_total + splits - 1) / splits;
     splits = (pc.chunks_total + pc.chunks_per_split - 1) / pc.chunks_per_split;
@@ -2121,9 +2207,9 @@ int dispatch_patch(const PatchSetup &u, int splits)
     const PatchConv &pc = u.pc;
     const dim3 grid(xcd_grid((unsigned)(u.tiles * splits)));
     const bool c_full = pc.Cin % 16 == 0;
-    if (u.shape == 0) return launch_patch<GatherWide, 24>(pc, c_full, grid, u.lds_bytes);
-    if (u.shape == 1) return launch_patch<GatherSquare, 16>(pc, c_full, grid, u.lds_bytes);
-    if (u.shape == 3) return launch_patch<GatherTall, 16>(pc, c_full, grid, u.lds_bytes);
+    if (u.shape == 0) return launch_patch<PatchWide, 2>(pc, c_full, grid, u.lds_bytes);
+    if (u.shape == 3) return launch_patch<PatchTall, 2>(pc, c_full, grid, u.lds_bytes);
+    if (u.shape == 1) return launch_patch<PatchNarrow, 3>(pc, c_full, grid, u.lds_bytes);
     if (u.shape == 4) {
         static bool raised = false;
         if (!raised) {
@@ -2146,7 +2232,7 @@ int dispatch_patch(const PatchSetup &u, int splits)
         }
         return DOPT_HIP_OK;
     }
-    return launch_patch<GatherDeep, 16>(pc, c_full, grid, u.lds_bytes);
+    return launch_patch<PatchDeep, 2>(pc, c_full, grid, u.lds_bytes);
 }
 
 template <bool kBwd>
@@ -2157,7 +2243,6 @@ int run_patch(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float *in, 
     PatchSetup u = patch_setup<kBwd>(d, P, Q);
     if (!u.ok) return DOPT_HIP_OK;
     PatchConv &pc = u.pc;
-    const int tiles = u.tiles;
     const int splits = patch_decide_splits(&u, out);
 
     const size_t wp_bytes = prepacked ? 0 : (u.wp_elems * sizeof(float) + 255) / 256 * 256;
@@ -2179,7 +2264,6 @@ int run_patch(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float *in, 
     pc.wp = prepacked;
     pc.bias = bias;
     pc.in_bytes = (size_t)pc.N * pc.Cin * pc.IH * pc.IW * sizeof(float);
-    pc.wp_bytes = u.wp_elems * sizeof(float);
     pc.out = splits > 1 ? partial : out;
     if (int rc = dispatch_patch(u, splits)) return rc;
     *done = true;
@@ -3011,16 +3095,16 @@ int run_wgrad_patch(const dopt_hip_conv_desc *d, const float *dy, const float *x
 // Backward-data (on a packed filter) and filter gradient of one 3x3 layer as one launch (conv_bwd_pair_k).
 // *done = false: one of the two is not a patch-kernel shape, or a combination that is not built; the
 // caller runs them one after the other.  `open` as in run_patch.
-template <class T, int NPMAX, int WM, int WC, int kGeo>
+template <class T, int NS, int WM, int WC, int kGeo>
 int launch_bwd_pair(const PatchConv &pc, const WgradPatch &wp, unsigned grid_a, unsigned grid_b, size_t lds_bytes)
 {
     static bool raised = false;
     if (!raised) {
-        DOPT_HIP_CHECK(hipFuncSetAttribute((const void *)conv_bwd_pair_k<T, NPMAX, WM, WC, kGeo>,
+        DOPT_HIP_CHECK(hipFuncSetAttribute((const void *)conv_bwd_pair_k<T, NS, WM, WC, kGeo>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         raised = true;
     }
-    hipLaunchKernelGGL((conv_bwd_pair_k<T, NPMAX, WM, WC, kGeo>), dim3(grid_a + grid_b), dim3(768), lds_bytes, stream(), pc,
+    hipLaunchKernelGGL((conv_bwd_pair_k<T, NS, WM, WC, kGeo>), dim3(grid_a + grid_b), dim3(768), lds_bytes, stream(), pc,
                        wp, grid_a);
     DOPT_LAUNCH_CHECK();
     return DOPT_HIP_OK;
@@ -3059,7 +3143,6 @@ int run_bwd_pair(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float *d
     pc.wp = prepacked;
     pc.bias = nullptr;
     pc.in_bytes = (size_t)pc.N * pc.Cin * pc.IH * pc.IW * sizeof(float);
-    pc.wp_bytes = a.wp_elems * sizeof(float);
     pc.out = splits_a > 1 ? partial_a : dx;
     wp.dy = dy; wp.x = x;
     wp.out = b.splits > 1 ? partial_b : dw;
@@ -3073,8 +3156,8 @@ int run_bwd_pair(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float *d
     if (two) {
         rc = dispatch_wgrad_patch(b);
         if (!rc) rc = dispatch_patch(a, splits_a);
-    } else if (combo == 0) rc = launch_bwd_pair<GatherDeep, 16, 4, 1, 0>(pc, wp, grid_a, grid_b, lds_bytes);
-    else rc = launch_bwd_pair<GatherDeep, 16, 4, 1, 1>(pc, wp, grid_a, grid_b, lds_bytes);
+    } else if (combo == 0) rc = launch_bwd_pair<PatchDeep, 2, 4, 1, 0>(pc, wp, grid_a, grid_b, lds_bytes);
+    else rc = launch_bwd_pair<PatchDeep, 2, 4, 1, 1>(pc, wp, grid_a, grid_b, lds_bytes);
     if (rc) return rc;
     if (probing) {
         DOPT_HIP_CHECK(hipEventRecord(probe.events[probe.used++].second, stream()));

@@ -527,6 +527,53 @@ def test_general_convolution_operands_at_the_ends_of_the_range():
         check_norm(ops.conv_bwd_filter(T(q), T(p), w.shape, pad, pad).numpy(), general_gradients(p, w, q, 2, 2)[1], 84, what)
 
 
+# ---- the direct 3 x 3 kernel: tiles of 32, 64, 128 and 160 rows, forward and (channels swapped) backward-data
+
+# one and several chunks of channels, ragged and whole; rows one past a tile; whole images and rows of an image; every padding
+DIRECT = [(2, 16, 16, 16, 16, 1), (3, 33, 32, 32, 17, 1), (1, 160, 16, 16, 32, 1), (2, 20, 16, 16, 48, 1), (1, 33, 64, 64, 64, 1),
+          (3, 40, 8, 8, 100, 1), (1, 48, 16, 16, 256, 1), (2, 24, 10, 10, 80, 0), (5, 24, 6, 6, 20, 2), (33, 24, 32, 32, 160, 1),
+          (9, 96, 4, 4, 30, 1)]
+
+
+@pytest.mark.parametrize("shape", DIRECT)
+def test_direct_convolution(shape):
+    N, C, H, W, K, pad = shape
+    r = rng(C + K)
+    x = np.maximum(r.standard_normal((N, C, H, W)), 0).astype(np.float32)
+    w = r.standard_normal((K, C, 3, 3)).astype(np.float32)
+    got = ops.convolution(T(x), T(w), (pad, pad), (1, 1)).numpy()
+    dy = r.standard_normal(got.shape).astype(np.float32)
+    dx = ops.conv_bwd_data(T(dy), T(w), x.shape, (pad, pad), (1, 1)).numpy()
+    want, mag = general(x, w, pad, 1), general(x, w, pad, 1, np.abs)
+    assert np.all(np.abs(got - want) <= walk(C * 9) * mag)
+    check_norm(got, want, C * 9 / 2, shape)
+    want, mag = general_gradients(x, w, dy, pad, 1)[0], general_gradients(x, w, dy, pad, 1, np.abs)[0]
+    assert np.all(np.abs(dx - want) <= walk(K * 9) * mag)
+    check_norm(dx, want, K * 9, shape)
+
+
+# a tile of every height; every term is positive
+@pytest.mark.parametrize("shape", [(2, 20, 16, 16, 17, 1), (2, 20, 16, 16, 48, 1), (4, 40, 8, 8, 100, 1), (33, 17, 32, 32, 160, 1)])
+def test_direct_convolution_operands_that_are_not_finite(shape):
+    N, C, H, W, K, pad = shape
+    r = rng(K)
+    x, w = (np.abs(r.standard_normal(s)).astype(np.float32) + np.float32(0.1) for s in ((N, C, H, W), (K, C, 3, 3)))
+    x[0, 3, 0, 0], x[N - 1, C - 1, H - 1, 2], w[K - 1, 2, 1, 1], w[1, C - 1, 0, 2], w[2, 5, 1, 0] = np.inf, np.nan, np.inf, np.nan, 2.0 ** 120
+    got = ops.convolution(T(x), T(w), (pad, pad), (1, 1)).numpy()
+    want = general(x, w, pad, 1)   # (zeros of the padding times an infinity are NaNs in both)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+    fine = np.isfinite(got)
+    assert np.all(np.abs(got[fine] - want[fine]) <= walk(C * 9) * want[fine])
+
+
+@pytest.mark.parametrize("shape", [(2, 20, 16, 16, 17), (2, 20, 16, 16, 48), (2, 40, 8, 8, 100)])
+def test_direct_convolution_operands_at_the_ends_of_the_range(shape):
+    N, C, H, W, K = shape
+    r = rng(K)
+    for what, x, w in scaled_pairs(r.standard_normal((N, C, H, W), np.float32), r.standard_normal((K, C, 3, 3), np.float32)):
+        check_norm(ops.convolution(T(x), T(w), (1, 1), (1, 1)).numpy(), general(x, w, 1, 1), 9 * C, what)
+
+
 # ---- packed filters beyond 2 GiB
 
 def cheap(r, *shape):
