@@ -13,8 +13,8 @@
 // GEMM view: M = output channels of the op, columns = output pixels (n,oh,ow), reduction =
 // (tap, ci) with ci padded to a multiple of 16 so that a 16-deep slab has ONE tap: the input
 // offset and the bounds mask are then uniform over the slab, and a lane's loads for successive
-// channels differ by a wave-uniform offset.  Wp is the filter re-packed once per call into
-// [tap*ci][m] (m contiguous), so the A tile goes global -> LDS with 128-bit accesses.
+// channels differ by a wave-uniform offset.  Wp is the filter re-packed once per call as its bf16 parts, in the order
+// the tile has in LDS, so the A tile goes global -> LDS with 128-bit accesses.
 //
 // Backward-filter is a GEMM with M = K (output channels), columns = (r', s', c) tap-major with c
 // padded to 16, reduction = output pixels (n,p,q); both operands are gathered with lanes along
@@ -37,246 +37,6 @@ namespace {
 using namespace dopt;
 
 constexpr int BK = 16;
-
-// ------------------------------------------------------------------------------------ gather
-
-struct GatherConv {
-    const float *in;   // gathered operand [N, Cin, IH, IW]
-    const float *wp;   // packed filter [taps * CinPad][Mp]
-    float *out;        // [N, Mout, OH, OW], or `splits` partial copies of it
-    int N, Cin, IH, IW, Mout, OH, OW, R, S;
-    int padH, padW, strideH, strideW;
-    int CinPad, Mp, ncols;
-    int mtiles, ntiles, slabs_total, slabs_per_split, splits;
-    size_t out_elems, in_bytes;
-    // where output pixel (oh, ow) of this problem lands: row oh * out_sy + out_oy, column ow * out_sx +
-    // out_ox of a plane of out_plane elements and out_OW columns (the whole tensor, or every
-    // stride-th pixel of it when a strided backward-data pass is run class by class)
-    int out_plane, out_OW, out_sy, out_sx, out_oy, out_ox;
-};
-
-// The products run on the bf16 matrix instruction, operands split as they are read from LDS (mma_slab_split): the loop was
-// bound by the fp32 instruction, 2048 cycles per slab and 64 x 64 wavefront tile, of which the six bf16 products take 768;
-// the splitting, 704 vector cycles, runs beside the other wavefront's.  50 images of 48 x 45 x 39, 100 filters of 5 x 5 at
-// stride 2, forward and both gradients: 379 -> 274 us.  Error against float64 (160 -> 320 channels, stride 2): 2.1e-7 -> 8.5e-8
-// forward, 5.3e-7 -> 1.7e-7 backward-data, 2.2e-7 -> 9.1e-8 filter gradient.
-// kMode: 0 = forward, 1 = backward-data with unit stride (no divisions), 2 = backward-data, any stride.
-// L: the workgroup's item among the problem's (split, tile) pairs, tile fastest.
-template <class T, int kMode>
-__device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L)
-{
-    constexpr int BM = T::BM, BN = T::BN, LDA = T::LDA, LDB = T::LDB, THREADS = T::THREADS;
-    constexpr int NA = BM * BK / 4 / THREADS;  // float4 loads of A per thread
-    constexpr int RSTEP = THREADS / BN;        // reduction rows covered by one pass of B loads
-    constexpr int NB = BK / RSTEP;             // scalar loads of B per thread
-    static_assert(NA >= 1 && NB >= 1 && RSTEP >= 1, "tile too small for the thread count");
-    __shared__ __attribute__((aligned(16))) float As[2][BK * LDA];
-    __shared__ __attribute__((aligned(16))) float Bs[2][BK * LDB];
-
-    const unsigned tiles = (unsigned)(p.mtiles * p.ntiles);
-    const int split = (int)(L / tiles);
-    const unsigned tile = L - (unsigned)split * tiles;
-    const int mt = (int)(tile % (unsigned)p.mtiles), nt = (int)(tile / (unsigned)p.mtiles);
-    const int m0 = mt * BM, n0 = nt * BN;
-    const int slab_begin = split * p.slabs_per_split;
-    const int slab_end = min(slab_begin + p.slabs_per_split, p.slabs_total);
-
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int wm = w / T::WN, wn = w % T::WN;
-
-    const __amdgpu_buffer_rsrc_t rin = make_rsrc(p.in, p.in_bytes);
-
-    // A: this thread's float4 slots of the [BK][BM] filter tile; byte offset relative to the slab's first row
-    unsigned a_voff[NA];
-    int a_lds[NA];
-#pragma unroll
-    for (int i = 0; i < NA; i++) {
-        const int f = tid + THREADS * i;
-        const int row = f / (BM / 4), gm = m0 + (f % (BM / 4)) * 4;
-        a_voff[i] = gm < p.Mp ? (unsigned)(row * p.Mp + gm) * 4u : kOobOffset;
-        a_lds[i] = row * LDA + (f % (BM / 4)) * 4;
-    }
-
-    // B: the output pixel this thread gathers for
-    const int bcol = tid % BN, brow0 = tid / BN;
-    const int pix = n0 + bcol;
-    const int pix_oob = p.ncols - 1 - pix;  // negative past the last pixel
-    const int OHW = p.OH * p.OW;
-    const int n_img = pix / OHW, pq = pix - n_img * OHW;
-    const int oh = pq / p.OW, ow = pq - oh * p.OW;
-    const int chan_stride = p.IH * p.IW;
-    const int pix_base = (n_img * p.Cin + brow0) * chan_stride;  // element offset of (n, channel brow0, 0, 0)
-    const int row_limit = p.Cin - brow0;                          // rows with ci0 + RSTEP*i >= row_limit are padding
-    const bool c_full = p.CinPad == p.Cin;
-
-    // running position in the (tap, channel) reduction, advanced slab by slab without divisions
-    int kk0, tap, ci0, tr, ts;
-
-    float4 areg[NA];
-    float breg[NB];
-
-    auto load = [&]() {
-        // (the packed filter may be larger than a buffer resource reaches: a resource per slab)
-        const __amdgpu_buffer_rsrc_t rwp = make_rsrc(p.wp + (size_t)kk0 * p.Mp, (size_t)BK * p.Mp * sizeof(float));
-#pragma unroll
-        for (int i = 0; i < NA; i++) areg[i] = buffer_load_f32x4(rwp, a_voff[i], 0);
-        int ih, iw, bad = pix_oob;
-        if (kMode == 0) {
-            ih = oh * p.strideH - p.padH + (p.R - 1 - tr);
-            iw = ow * p.strideW - p.padW + (p.S - 1 - ts);
-        } else if (kMode == 1) {
-            ih = oh + p.padH - (p.R - 1 - tr);
-            iw = ow + p.padW - (p.S - 1 - ts);
-        } else {
-            // out = dx[.., h, w]; in = dy[.., ph, qw] with h = ph*stride - pad + r, r = R-1-tr
-            const int nh = oh + p.padH - (p.R - 1 - tr), nw = ow + p.padW - (p.S - 1 - ts);
-            ih = nh / p.strideH;
-            iw = nw / p.strideW;
-            // negative numerators, and numerators that are not multiples of the stride, hit no input
-            bad |= nh | nw | -(int)(ih * p.strideH != nh) | -(int)(iw * p.strideW != nw);
-        }
-        bad |= ih | (p.IH - 1 - ih) | iw | (p.IW - 1 - iw);  // sign bit set: outside the input
-        const unsigned b_voff = bad < 0 ? kOobOffset : (unsigned)(pix_base + ih * p.IW + iw) * 4u;
-#pragma unroll
-        for (int i = 0; i < NB; i++) {
-            const int ci = ci0 + RSTEP * i;  // wave-uniform
-            const unsigned voff = (c_full || ci < row_limit) ? b_voff : kOobOffset;
-            breg[i] = buffer_load_f32(rin, voff, (unsigned)(ci * chan_stride) * 4u);
-        }
-        kk0 += BK;
-        ci0 += BK;
-        if (ci0 == p.CinPad) {
-            ci0 = 0;
-            if (++ts == p.S) {
-                ts = 0;
-                ++tr;
-            }
-        }
-    };
-    auto store = [&](int buf, float up) {
-#pragma unroll
-        for (int i = 0; i < NA; i++) *(float4 *)&As[buf][a_lds[i]] = make_float4(areg[i].x * up, areg[i].y * up, areg[i].z * up, areg[i].w * up);
-#pragma unroll
-        for (int i = 0; i < NB; i++) Bs[buf][(brow0 + RSTEP * i) * LDB + bcol] = breg[i] * up;
-    };
-
-    v16f acc[T::MI][T::NI];
-    auto run = [&](auto exact_tag) {
-        constexpr bool exact = decltype(exact_tag)::value != 0;
-        constexpr float up = exact ? 1.0f : kSplitUp;
-        kk0 = slab_begin * BK;
-        tap = kk0 / p.CinPad;
-        ci0 = kk0 - tap * p.CinPad;
-        tr = tap / p.S;
-        ts = tap - tr * p.S;
-        v16f low[T::MI][T::NI];
-        zero_acc(acc);
-        zero_acc(low);
-        auto slab_products = [&](int buf) {
-            if constexpr (exact) mma_slab<BK, LDA, LDB>(As[buf], Bs[buf], wm * (BM / T::WM), wn * (BN / T::WN), acc, lane);
-            else mma_slab_split<LDA, LDB>(As[buf], Bs[buf], wm * (BM / T::WM), wn * (BN / T::WN), acc, low, lane);
-        };
-        load();
-        store(0, up);
-        __syncthreads();
-        int cur = 0;
-        // steady state: no data-dependent branches inside
-        for (int slab = slab_begin; slab < slab_end - 1; ++slab) {
-            load();
-            slab_products(cur);
-            store(cur ^ 1, up);
-            __syncthreads();
-            cur ^= 1;
-        }
-        slab_products(cur);
-        if constexpr (!exact) add_acc(acc, low);
-    };
-    run(StepTag<0>{});
-    // the parts of an infinity hold NaNs: a tile that is not finite is formed again with the fp32 instruction
-    if (__syncthreads_or(not_finite(acc))) run(StepTag<1>{});
-
-    float *outp = p.out + (size_t)split * p.out_elems;
-#pragma unroll
-    for (int j = 0; j < T::NI; j++) {
-        const int col = n0 + wn * (BN / T::WN) + j * 32 + (lane & 31);
-        if (col >= p.ncols) continue;
-        const int n2 = col / OHW, pq2 = col - n2 * OHW;
-        const int oh2 = pq2 / p.OW, ow2 = pq2 - oh2 * p.OW;
-        float *base = outp + (size_t)n2 * p.Mout * p.out_plane + (size_t)(oh2 * p.out_sy + p.out_oy) * p.out_OW +
-                      ow2 * p.out_sx + p.out_ox;
-#pragma unroll
-        for (int i = 0; i < T::MI; i++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int m = m0 + wm * (BM / T::WM) + i * 32 + acc_row(v, lane);
-                if (m < p.Mout) base[(size_t)m * p.out_plane] = acc[i][j][v];
-            }
-    }
-}
-
-template <class T, int kMode>
-__global__ __launch_bounds__(T::THREADS, T::THREADS / 128) void conv_gather_k(GatherConv p)
-{
-    // 1-D grid over (split, tile), tile fastest: the blocks an XCD receives work on neighbouring
-    // tiles of the same slice of the reduction, whatever the ratio of tiles to splits
-    unsigned L;
-    if (!xcd_remap(blockIdx.x, (unsigned)(p.mtiles * p.ntiles) * (unsigned)p.splits, &L)) return;
-    conv_gather_body<T, kMode>(p, L);
-}
-
-// Up to nine problems that do not depend on each other in ONE launch (the residue classes of a strided backward-data
-// pass - four at stride 2, nine at stride 3: same operands, different sub-filters, interleaved output pixels).  Every workgroup runs conv_gather_body on one
-// tile of one problem, so each problem's values are those of a launch of its own; what changes is that the chip is not
-// drained and refilled between problems that each fill only part of it.  An XCD takes the same share of every problem
-// (its tiles of a problem are neighbours, as in a single launch), longest problem first.
-constexpr int kGatherJobs = 9;
-struct GatherGroup {
-    GatherConv g[kGatherJobs];
-    unsigned per[kGatherJobs];   // workgroups of problem j on each XCD: ceil(tiles * splits / 8)
-    int n;
-};
-
-template <class T, int kMode>
-__global__ __launch_bounds__(T::THREADS, T::THREADS / 128) void conv_gather_group_k(GatherGroup gg)
-{
-    const unsigned xcd = blockIdx.x & 7u;
-    unsigned i = blockIdx.x >> 3;
-    int j = 0;
-    while (j < gg.n - 1 && i >= gg.per[j]) {
-        i -= gg.per[j];
-        j++;
-    }
-    const unsigned L = xcd * gg.per[j] + i;
-    if (i >= gg.per[j] || L >= (unsigned)(gg.g[j].mtiles * gg.g[j].ntiles) * (unsigned)gg.g[j].splits) return;
-    conv_gather_body<T, kMode>(gg.g[j], L);
-}
-
-// ------------------------------------------------------------------------------------ patch (3x3, unit stride)
-//
-// Forward and backward-data of 3x3 unit-stride convolutions.  The gathered operand is not
-// re-fetched per filter tap: for a chunk of 16 input channels the block loads the input patch
-// under its pixel tile ONCE -- the tile's rows plus a one-pixel halo, zero-filled outside the
-// image by the buffer range check -- and the nine taps read it at nine offsets.  LDS holds the patch by channel half and
-// position, so that a lane's pixel operands for a whole 16-channel slab are 128-bit LDS reads; the packed filter,
-// wp[slab][part][m][16 channels], has the same shape per row, and a lane's filter operands are 128-bit
-// loads straight from it.  Lane half kh (= lane / 32) multiplies channels kh*8 .. kh*8+7 of the chunk.
-
-struct PatchConv {
-    const float *in;   // gathered operand [N, Cin, IH, IW]
-    const float *wp;   // packed filter [chunks][9][3 parts][Mp][16], bf16 (Winograd: 16 positions in the place of 9 taps)
-    float *out;        // [N, Mout, OH, OW], or `splits` partial copies of it
-    const float *bias; // optional [Mout], added to the finished sums (by the split reduction when there is one)
-    int N, Cin, IH, IW, Mout, OH, OW;
-    int PT, PL;        // input row / column of patch position (0,0) is (oh0 - PT, -PL)
-    int flip;          // 1: tap (tr,ts) reads patch offset (2-tr, 2-ts); 0: (tr, ts)
-    int nimg, rows;    // images per pixel tile; output rows of each image in the tile
-    int PR, PC, psz;   // patch rows and columns per image; patch positions per tile = nimg*PR*PC
-    unsigned magic_img, magic_pc;  // floor(2^32/d)+1 for d = PR*PC, PC (exact for x*d < 2^32)
-    unsigned magic_tpi, magic_tcn;            // Winograd: the same for the 2 x 2 tiles of one image in the pixel tile, and of one row
-    int Mp;            // rows of one packed filter slab (Mout rounded up to the tile height)
-    int ncols, mtiles, ntiles, chunks_total, chunks_per_split, splits;
-    size_t out_elems, in_bytes;
-};
 
 // Filters packed as bf16 parts.  A value whose parts are no numbers (2^103 and more, infinities, NaNs) has this NaN for its h part
 // and its bits as they are in the other two.
@@ -309,6 +69,363 @@ __device__ __forceinline__ float packed_value(const v4u (&f)[3], int e)
     auto val = [&](int t) { return __builtin_bit_cast(float, q[t] << 16); };
     return q[0] == kPackedRaw ? __builtin_bit_cast(float, q[1] << 16 | q[2]) : (val(0) + val(1) + val(2)) * (1.0f / kSplitUp);
 }
+
+// ------------------------------------------------------------------------------------ gather
+
+struct GatherConv {
+    const float *in;   // gathered operand [N, Cin, IH, IW]
+    const float *wp;   // packed filter [16-channel chunk][tap][Mp / 4][3 parts][2 halves][4 rows][8 channels], bf16
+    float *out;        // [N, Mout, OH, OW], or `splits` partial copies of it
+    int N, Cin, IH, IW, Mout, OH, OW, R, S;
+    int padH, padW, strideH, strideW;
+    int CinPad, Mp, ncols;
+    int mtiles, ntiles, slabs_total, slabs_per_split, splits;
+    size_t out_elems, in_bytes;
+    // where output pixel (oh, ow) of this problem lands: row oh * out_sy + out_oy, column ow * out_sx +
+    // out_ox of a plane of out_plane elements and out_OW columns (the whole tensor, or every
+    // stride-th pixel of it when a strided backward-data pass is run class by class)
+    int out_plane, out_OW, out_sy, out_sx, out_oy, out_ox;
+};
+
+// The products run on the bf16 matrix instruction (mfma_core.h).  The filter is packed as bf16 parts; an input value is split
+// once, when it is stored in LDS.  (Split by every wavefront that reads a value, splitting took 700 vector cycles of a slab beside
+// 384 to 768 matrix cycles.)  LDS holds both operands as [part][half][row][8 channels], so a fragment of one part is one
+// 128-bit read and neighbouring lanes' reads are neighbours.  A stage is SL slabs; under the matrix instructions of one the next is
+// split and stored and the one after it is loaded, each piece pinned to a step, and the workgroup meets once per stage.  Split
+// behind the products instead, with every wavefront at the same place: 5 x 5 layers below 101 and 69 us, now 75 and 58.
+// 50 images of 48 x 45 x 39, 100 filters of 5 x 5 at stride 2: forward 103 -> 58 us, backward-data 95 -> 75; 64 -> 64 channels of 3 x 3
+// on 64 images of 33 x 31 46 -> 37 us; Wide-ResNet-28-10's two strided 3 x 3 layers backward 270 -> 240 us.  A stage of a
+// 64 x 256 tile takes 1.7 us of which 0.9 are matrix time at the rate of a large product; it reads 144 KB of fragments from LDS.
+// Error against float64 (160 -> 320 channels, stride 2): 8.5e-8 forward, 1.7e-7 backward-data (the fp32 instruction: 2.1e-7, 5.3e-7).
+// kMode: 0 = forward, 1 = backward-data with unit stride (no divisions), 2 = backward-data, any stride.
+// L: the workgroup's item among the problem's (split, tile) pairs, tile fastest.
+template <class T, int SL>
+struct GatherLds {
+    static constexpr int PA = T::BM + 4, PB = T::BN;   // rows of a part's half (four more: a chunk's parts go to different banks)
+    static constexpr int A = SL * 6 * PA * 4, STAGE = A + SL * 6 * PB * 4;   // floats
+    static constexpr size_t BYTES = 2 * STAGE * sizeof(float);
+};
+
+template <class T, int SL, int kMode>
+__device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L)
+{
+    constexpr int BM = T::BM, BN = T::BN, THREADS = T::THREADS, MI = T::MI, NI = T::NI;
+    constexpr int CHUNKS = SL * BM * 6;                      // 16-byte pieces of a stage's filter tile
+    constexpr int NA = (CHUNKS + THREADS - 1) / THREADS;     // ... of each thread
+    constexpr int CPT = 16 * BN / THREADS;                   // channels of a slab that a thread gathers for its pixel
+    constexpr int PA = GatherLds<T, SL>::PA, PB = GatherLds<T, SL>::PB, STAGE = GatherLds<T, SL>::STAGE, BOFF = GatherLds<T, SL>::A;
+    static_assert((CPT == 4 || CPT == 8) && SL <= 2, "half a piece of LDS or a whole one; two sets of fragments");
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+
+    const unsigned tiles = (unsigned)(p.mtiles * p.ntiles);
+    const int split = (int)(L / tiles);
+    const unsigned tile = L - (unsigned)split * tiles;
+    const int mt = (int)(tile % (unsigned)p.mtiles), nt = (int)(tile / (unsigned)p.mtiles);
+    const int m0 = mt * BM, n0 = nt * BN;
+    const int slab_begin = split * p.slabs_per_split;
+    const int slab_end = min(slab_begin + p.slabs_per_split, p.slabs_total);
+
+    const int tid = threadIdx.x, lane = tid & 63, kh = lane >> 5, l32 = lane & 31;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = w / T::WN, wn = w % T::WN;
+
+    const __amdgpu_buffer_rsrc_t rin = make_rsrc(p.in, p.in_bytes);
+
+    // A: this thread's pieces of the stage's filter tile, which lies in memory as one run of 96 bytes a row per slab
+    const unsigned a_rows = (unsigned)min(BM, p.Mp - m0);   // rows past the packed ones are zeros (range check)
+    unsigned a_voff[NA];
+    int a_lds[NA];
+#pragma unroll
+    for (int i = 0; i < NA; i++) {
+        const int f = i * THREADS + tid, sl = f / (BM * 6), g = f - sl * (BM * 6);
+        const int block = g / 24, half_part = g / 4 % 6, row = block * 4 + g % 4;
+        a_voff[i] = (unsigned)g * 16u;
+        a_lds[i] = ((sl * 6 + half_part) * PA + row) * 4;
+    }
+
+    // B: the output pixel this thread gathers for, CPT channels of a slab from c0 on
+    const int bcol = tid % BN, c0 = tid / BN * CPT;
+    const int pix = n0 + bcol;
+    const int pix_oob = p.ncols - 1 - pix;  // negative past the last pixel
+    const int OHW = p.OH * p.OW;
+    const int n_img = pix / OHW, pq = pix - n_img * OHW;
+    const int oh = pq / p.OW, ow = pq - oh * p.OW;
+    const int chan_stride = p.IH * p.IW;
+    const int pix_base = (n_img * p.Cin + c0) * chan_stride;  // element offset of (n, channel c0, 0, 0)
+    const int row_limit = p.Cin - c0;                          // channels ci0 + i >= row_limit are padding
+    const int b_lds = BOFF + (c0 / 8 * PB + bcol) * 4 + c0 % 8 / 2;
+
+    // running position in the reduction, advanced slab by slab without divisions: all taps of sixteen channels, then the next
+    // sixteen, so that a tap finds most of its pixels where the one before left them in the L1
+    int slab, ci0, tr, ts;
+    auto rewind = [&]() {
+        slab = slab_begin;
+        const int taps = p.R * p.S, chunk = slab_begin / taps, tap = slab_begin - chunk * taps;
+        ci0 = chunk * BK;
+        tr = tap / p.S;
+        ts = tap - tr * p.S;
+    };
+
+    float4 areg[NA];
+    float breg[SL][CPT];
+    auto load_a = [&](int first) {   // the filter's pieces of the stage that begins with slab `first`
+#pragma unroll
+        for (int i = 0; i < NA; i++) {
+            // (the packed filter may be larger than a buffer resource reaches: a resource per slab; which slab of the stage
+            // is the same for a whole wavefront)
+            const int sl = SL == 1 ? 0 : (i * THREADS + w * 64) / (BM * 6);
+            const bool have = first + sl < slab_end && (CHUNKS % THREADS == 0 || i * THREADS + w * 64 < CHUNKS);
+            const __amdgpu_buffer_rsrc_t rwp = make_rsrc(p.wp + ((size_t)(have ? first + sl : 0) * p.Mp + m0) * 24, have ? (size_t)a_rows * 96 : 0);
+            areg[i] = buffer_load_f32x4(rwp, a_voff[i], 0);
+        }
+    };
+    auto pixel = [&]() {   // byte offset of this thread's input pixel for the slab at the running position, or kOobOffset
+        int ih, iw, bad = pix_oob | (slab_end - 1 - slab);
+        if (kMode == 0) {
+            ih = oh * p.strideH - p.padH + (p.R - 1 - tr);
+            iw = ow * p.strideW - p.padW + (p.S - 1 - ts);
+        } else if (kMode == 1) {
+            ih = oh + p.padH - (p.R - 1 - tr);
+            iw = ow + p.padW - (p.S - 1 - ts);
+        } else {
+            // out = dx[.., h, w]; in = dy[.., ph, qw] with h = ph*stride - pad + r, r = R-1-tr
+            const int nh = oh + p.padH - (p.R - 1 - tr), nw = ow + p.padW - (p.S - 1 - ts);
+            ih = nh / p.strideH;
+            iw = nw / p.strideW;
+            // negative numerators, and numerators that are not multiples of the stride, hit no input
+            bad |= nh | nw | -(int)(ih * p.strideH != nh) | -(int)(iw * p.strideW != nw);
+        }
+        bad |= ih | (p.IH - 1 - ih) | iw | (p.IW - 1 - iw);  // sign bit set: outside the input
+        return bad < 0 ? kOobOffset : (unsigned)(pix_base + ih * p.IW + iw) * 4u;
+    };
+    auto next_slab = [&]() {
+        ++slab;
+        if (++ts == p.S) {
+            ts = 0;
+            if (++tr == p.R) {
+                tr = 0;
+                ci0 += BK;
+            }
+        }
+    };
+    // Channels past the last one are read as they lie (another image's, or zeros past the tensor): their filter values are zeros.
+    // Only the fp32 pass, which a product of such a zero with an infinity leads to, has to leave them out.
+    auto load_b = [&](int sl, int i, unsigned voff) { breg[sl][i] = buffer_load_f32(rin, voff, (unsigned)((ci0 + i) * chan_stride) * 4u); };
+    auto store_a = [&](float *buf) {
+#pragma unroll
+        for (int i = 0; i < NA; i++)
+            if (CHUNKS % THREADS == 0 || i * THREADS + tid < CHUNKS) *(float4 *)(buf + a_lds[i]) = areg[i];
+    };
+    constexpr int PAIRS = CPT / 2;   // of a slab: four make a 16-byte piece per part, two half of one
+    unsigned q[3][PAIRS];
+    auto split_b = [&](int sl, int e) {
+        split_pair(breg[sl][2 * e] * kSplitUp, breg[sl][2 * e + 1] * kSplitUp, q[0][e], q[1][e], q[2][e]);
+    };
+    auto store_b = [&](float *buf, int sl) {
+#pragma unroll
+        for (int t = 0; t < 3; t++) {
+            float *const o = buf + b_lds + (sl * 6 + t * 2) * PB * 4;
+            if constexpr (PAIRS == 4) *(v4u *)o = v4u{q[t][0], q[t][1], q[t][2], q[t][3]};
+            else *(uint2 *)o = make_uint2(q[t][0], q[t][1]);
+        }
+    };
+
+    v16f acc[MI][NI], low[MI][NI];
+    zero_acc(acc);
+    zero_acc(low);
+    const int a_frag = (kh * PA + wm * (BM / T::WM) + l32) * 4, b_frag = BOFF + (kh * PB + wn * (BN / T::WN) + l32) * 4;
+    v4u a[2][MI][3], b[2][NI][3];
+    auto fragments = [&](const float *buf, int sl) {
+#pragma unroll
+        for (int t = 0; t < 3; t++) {
+#pragma unroll
+            for (int i = 0; i < MI; i++) a[sl & 1][i][t] = *(const v4u *)(buf + a_frag + ((sl * 6 + t * 2) * PA + 32 * i) * 4);
+#pragma unroll
+            for (int j = 0; j < NI; j++) b[sl & 1][j][t] = *(const v4u *)(buf + b_frag + ((sl * 6 + t * 2) * PB + 32 * j) * 4);
+        }
+    };
+    // Under the matrix instructions of a stage the next one, which is in registers, is split and stored, and the one after
+    // it is loaded: a slab's values as soon as the slab before in those registers is stored.
+    auto stage = [&](const float *cur, float *nxt) {
+        fragments(cur, 0);
+        unsigned voff = 0;
+        static_for<0, SL>([&](auto sl_tag) {
+            constexpr int sl = decltype(sl_tag)::value;
+            static_for<0, 6>([&](auto tag) {
+                constexpr int s = decltype(tag)::value;
+                if constexpr (s == 0 && sl + 1 < SL) fragments(cur, sl + 1);
+                if constexpr (s < PAIRS) split_b(sl, s);
+                if constexpr (s == 0 && sl == 0) {
+                    store_a(nxt);
+                    load_a(slab);
+                }
+                if constexpr (s == PAIRS) {
+                    store_b(nxt, sl);
+                    voff = pixel();
+                }
+                if constexpr (s == PAIRS + 1) {
+#pragma unroll
+                    for (int i = 0; i < CPT; i++) load_b(sl, i, voff);
+                    next_slab();
+                }
+                // smallest products first: l.h, h.l, m.m, m.h, h.m, h.h
+                constexpr int qa = s == 0 ? 2 : s == 2 || s == 3 ? 1 : 0, qb = s == 1 ? 2 : s == 2 || s == 4 ? 1 : 0;
+#pragma unroll
+                for (int i = 0; i < MI; i++)
+#pragma unroll
+                    for (int j = 0; j < NI; j++) {
+                        v16f &c = s < 5 ? low[i][j] : acc[i][j];
+                        c = mfma_bf16(a[sl & 1][i][qa], b[sl & 1][j][qb], c);
+                    }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        });
+        __syncthreads();
+    };
+    auto load_stage = [&](auto masked_tag) {   // all of it at once
+        load_a(slab);
+#pragma unroll
+        for (int sl = 0; sl < SL; sl++) {
+            const unsigned voff = pixel();
+#pragma unroll
+            for (int i = 0; i < CPT; i++) load_b(sl, i, decltype(masked_tag)::value && ci0 + i >= row_limit ? kOobOffset : voff);
+            next_slab();
+        }
+    };
+    rewind();
+    load_stage(StepTag<0>{});
+    store_a(lds);
+#pragma unroll
+    for (int sl = 0; sl < SL; sl++) {
+#pragma unroll
+        for (int e = 0; e < PAIRS; e++) split_b(sl, e);
+        store_b(lds, sl);
+    }
+    load_stage(StepTag<0>{});   // (past the last slab: zeros)
+    __syncthreads();
+    const int stages = (slab_end - slab_begin + SL - 1) / SL;
+    for (int st = 0; st < stages; ++st) stage(lds + (st & 1) * STAGE, lds + (~st & 1) * STAGE);
+    add_acc(acc, low);
+
+    // the parts of an infinity hold NaNs: a tile that is not finite is formed again with the fp32 instruction, a stage at a time
+    if (__syncthreads_or(not_finite(acc))) {
+        zero_acc(acc);
+        rewind();
+#pragma unroll 1
+        for (int st = 0; st < stages; ++st) {
+            load_stage(StepTag<1>{});
+            __syncthreads();
+            store_a(lds);
+            // B here: [half][pixel][8 channels]
+#pragma unroll
+            for (int sl = 0; sl < SL; sl++)
+#pragma unroll
+                for (int i = 0; i < CPT; i += 4)
+                    *(float4 *)(lds + BOFF + sl * 6 * PB * 4 + (((c0 + i) / 8 * PB + bcol) * 8 + (c0 + i) % 8)) =
+                        make_float4(breg[sl][i], breg[sl][i + 1], breg[sl][i + 2], breg[sl][i + 3]);
+            __syncthreads();
+#pragma unroll 1
+            for (int sl = 0; sl < SL; sl++)
+#pragma unroll
+                for (int i = 0; i < MI; i++) {
+                    v4u f[3];
+#pragma unroll
+                    for (int t = 0; t < 3; t++) f[t] = *(const v4u *)(lds + a_frag + ((sl * 6 + t * 2) * PA + 32 * i) * 4);
+#pragma unroll
+                    for (int j = 0; j < NI; j++) {
+                        const float *const src = lds + BOFF + sl * 6 * PB * 4 + (kh * PB + wn * (BN / T::WN) + 32 * j + l32) * 8;
+                        const float4 b0 = *(const float4 *)src, b1 = *(const float4 *)(src + 4);
+                        const float b8[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+#pragma unroll
+                        for (int e = 0; e < 8; e++)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(packed_value(f, e), b8[e], acc[i][j], 0, 0, 0);
+                    }
+                }
+        }
+    }
+
+    float *outp = p.out + (size_t)split * p.out_elems;
+#pragma unroll
+    for (int j = 0; j < NI; j++) {
+        const int col = n0 + wn * (BN / T::WN) + j * 32 + l32;
+        if (col >= p.ncols) continue;
+        const int n2 = col / OHW, pq2 = col - n2 * OHW;
+        const int oh2 = pq2 / p.OW, ow2 = pq2 - oh2 * p.OW;
+        float *base = outp + (size_t)n2 * p.Mout * p.out_plane + (size_t)(oh2 * p.out_sy + p.out_oy) * p.out_OW +
+                      ow2 * p.out_sx + p.out_ox;
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const int m = m0 + wm * (BM / T::WM) + i * 32 + acc_row(v, lane);
+                if (m < p.Mout) base[(size_t)m * p.out_plane] = acc[i][j][v];
+            }
+    }
+}
+
+template <class T, int SL, int kMode>
+__global__ __launch_bounds__(T::THREADS, 2) void conv_gather_k(GatherConv p)
+{
+    // 1-D grid over (split, tile), tile fastest: the blocks an XCD receives work on neighbouring
+    // tiles of the same slice of the reduction, whatever the ratio of tiles to splits
+    unsigned L;
+    if (!xcd_remap(blockIdx.x, (unsigned)(p.mtiles * p.ntiles) * (unsigned)p.splits, &L)) return;
+    conv_gather_body<T, SL, kMode>(p, L);
+}
+
+// Up to nine problems that do not depend on each other in ONE launch (the residue classes of a strided backward-data
+// pass - four at stride 2, nine at stride 3: same operands, different sub-filters, interleaved output pixels).  Every workgroup runs conv_gather_body on one
+// tile of one problem, so each problem's values are those of a launch of its own; what changes is that the chip is not
+// drained and refilled between problems that each fill only part of it.  An XCD takes the same share of every problem
+// (its tiles of a problem are neighbours, as in a single launch), longest problem first.
+constexpr int kGatherJobs = 9;
+struct GatherGroup {
+    GatherConv g[kGatherJobs];
+    unsigned per[kGatherJobs];   // workgroups of problem j on each XCD: ceil(tiles * splits / 8)
+    int n;
+};
+
+template <class T, int SL, int kMode>
+__global__ __launch_bounds__(T::THREADS, 2) void conv_gather_group_k(GatherGroup gg)
+{
+    const unsigned xcd = blockIdx.x & 7u;
+    unsigned i = blockIdx.x >> 3;
+    int j = 0;
+    while (j < gg.n - 1 && i >= gg.per[j]) {
+        i -= gg.per[j];
+        j++;
+    }
+    const unsigned L = xcd * gg.per[j] + i;
+    if (i >= gg.per[j] || L >= (unsigned)(gg.g[j].mtiles * gg.g[j].ntiles) * (unsigned)gg.g[j].splits) return;
+    conv_gather_body<T, SL, kMode>(gg.g[j], L);
+}
+
+// ------------------------------------------------------------------------------------ patch (3x3, unit stride)
+//
+// Forward and backward-data of 3x3 unit-stride convolutions.  The gathered operand is not
+// re-fetched per filter tap: for a chunk of 16 input channels the block loads the input patch
+// under its pixel tile ONCE -- the tile's rows plus a one-pixel halo, zero-filled outside the
+// image by the buffer range check -- and the nine taps read it at nine offsets.  LDS holds the patch by channel half and
+// position, so that a lane's pixel operands for a whole 16-channel slab are 128-bit LDS reads; the packed filter,
+// wp[slab][part][m][16 channels], has the same shape per row, and a lane's filter operands are 128-bit
+// loads straight from it.  Lane half kh (= lane / 32) multiplies channels kh*8 .. kh*8+7 of the chunk.
+
+struct PatchConv {
+    const float *in;   // gathered operand [N, Cin, IH, IW]
+    const float *wp;   // packed filter [chunks][9][3 parts][Mp][16], bf16 (Winograd: 16 positions in the place of 9 taps)
+    float *out;        // [N, Mout, OH, OW], or `splits` partial copies of it
+    const float *bias; // optional [Mout], added to the finished sums (by the split reduction when there is one)
+    int N, Cin, IH, IW, Mout, OH, OW;
+    int PT, PL;        // input row / column of patch position (0,0) is (oh0 - PT, -PL)
+    int flip;          // 1: tap (tr,ts) reads patch offset (2-tr, 2-ts); 0: (tr, ts)
+    int nimg, rows;    // images per pixel tile; output rows of each image in the tile
+    int PR, PC, psz;   // patch rows and columns per image; patch positions per tile = nimg*PR*PC
+    unsigned magic_img, magic_pc;  // floor(2^32/d)+1 for d = PR*PC, PC (exact for x*d < 2^32)
+    unsigned magic_tpi, magic_tcn;            // Winograd: the same for the 2 x 2 tiles of one image in the pixel tile, and of one row
+    int Mp;            // rows of one packed filter slab (Mout rounded up to the tile height)
+    int ncols, mtiles, ntiles, chunks_total, chunks_per_split, splits;
+    size_t out_elems, in_bytes;
+};
 
 __device__ inline unsigned fast_div(unsigned x, unsigned magic) { return __umulhi(x, magic); }
 
@@ -1857,44 +1974,66 @@ __global__ __launch_bounds__(256) void splitk_reduce_k(size_t n4, int splits, co
     }
 }
 
-// Forward pack: w[K][C][taps] -> Wp[(tap*CinPad + c)][Mp] (m = k contiguous), through a 64x64 LDS tile.
-__global__ __launch_bounds__(256) void pack_fwd_k(int K, int C, int taps, int CinPad, int Mp, const float *w,
-                                                   float *wp)
+// The general kernels' packed filters (GatherConv::wp) from w[K][C][R][S]: of the whole filter (one class with R2 = R, S2 = S, no
+// stride) or of the sub-filters that the residue classes of a strided backward-data pass multiply.  Forward: rows = K, reduction
+// over C; backward: rows = C, reduction over K.  Rows up to Mp and channels up to a multiple of 16 are written, zeros where the
+// filter has none.  A block takes 16 rows and 8 channels: they are contiguous runs in w (forward a run per row, backward one per
+// channel), staged through LDS; then a thread splits eight values of one row and tap and writes a 16-byte piece per part.
+struct SubFilter {
+    float *wp;            // packed copy of this class
+    int R2, S2, r0, s0;   // tap rows / columns of the class and its first tap offsets
+};
+struct SubFilters {
+    SubFilter f[kGatherJobs];
+    int n;
+};
+template <bool kBwd>
+__global__ __launch_bounds__(256) void pack_gather_k(int M, int Cred, int Mp, int R, int S, int sH, int sW, size_t sm, size_t sc,
+                                                      const float *w, SubFilters subs)
 {
-    __shared__ float tile[64][65];
-    const int CT = C * taps;
-    const int m0 = blockIdx.x * 64, col0 = blockIdx.y * 64;
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
-        const int m = m0 + ty + 4 * k, cc = col0 + tx;
-        tile[ty + 4 * k][tx] = (m < K && cc < CT) ? w[(size_t)m * CT + cc] : 0.0f;
+    extern __shared__ float stage[];
+    const unsigned mblocks = (unsigned)(Mp + 15) / 16;
+    const int RS = R * S, m0 = (int)(blockIdx.x % mblocks) * 16, c0 = (int)(blockIdx.x / mblocks) * 8;
+    const int len = (kBwd ? 16 : 8) * RS, pitch = len + 1;   // of a run; backward: channel c0 + run, rows m0 ..; forward: row m0 + run, channels c0 ..
+    for (int i = threadIdx.x; i < (kBwd ? 8 : 16) * len; i += 256) {
+        const int run = i / len, r = i - run * len;
+        const int m = m0 + (kBwd ? r / RS : run), c = c0 + (kBwd ? run : r / RS);
+        stage[run * pitch + r] = m < M && c < Cred ? w[(size_t)m * sm + (size_t)c * sc + r % RS] : 0.0f;
     }
     __syncthreads();
+    for (int j = 0; j < subs.n; j++) {
+        const SubFilter f = subs.f[j];
+        for (int i = threadIdx.x; i < 16 * f.R2 * f.S2; i += 256) {
+            const int t = i / 16, ml = i % 16, tr = t / f.S2, ts = t - tr * f.S2;
+            // stored tap (tr, ts) stands for offsets r = r0 + (R2 - 1 - tr) * sH, s likewise, and the element
+            // that multiplies offset (r, s) is the flipped one (see subfilter_k)
+            const int r = f.r0 + (f.R2 - 1 - tr) * sH, s = f.s0 + (f.S2 - 1 - ts) * sW;
+            const float *const src = stage + (kBwd ? ml * RS : ml * pitch) + (R - 1 - r) * S + (S - 1 - s);
+            unsigned q[3][4];
 #pragma unroll
-    for (int k = 0; k < 16; k++) {
-        const int cc = col0 + ty + 4 * k, m = m0 + tx;
-        if (cc < CT && m < K) {
-            const int c = cc / taps, t = cc - c * taps;
-            wp[(size_t)(t * CinPad + c) * Mp + m] = tile[tx][ty + 4 * k];
+            for (int e = 0; e < 4; e++) {
+                const int step = kBwd ? pitch : RS;
+                split_packed(src[2 * e * step], src[(2 * e + 1) * step], q[0][e], q[1][e], q[2][e]);
+            }
+            const int m = m0 + ml;
+            if (m >= Mp) continue;
+            v4u *const dst = (v4u *)f.wp + ((size_t)(c0 / 16 * (f.R2 * f.S2) + t) * Mp + m / 4 * 4) * 6 + c0 / 8 % 2 * 4 + m % 4;
+#pragma unroll
+            for (int part = 0; part < 3; part++) dst[part * 8] = v4u{q[part][0], q[part][1], q[part][2], q[part][3]};
         }
     }
 }
 
-// Backward-data pack: w[K][C][taps] -> Wp[(tap*KPad + k)][Mp] (m = c contiguous).
-// Block (k, 64-channel chunk) stages w[k][c0 .. c0+64][*] (contiguous) in LDS.
-__global__ __launch_bounds__(256) void pack_bwd_k(int K, int C, int taps, int KPad, int Mp, const float *w, float *wp)
+int launch_pack_gather(bool bwd, int K, int C, int R, int S, int sH, int sW, int Mp, const float *w, const SubFilters &subs)
 {
-    extern __shared__ float stage[];  // 64 * taps floats
-    const int k = blockIdx.x, c0 = blockIdx.y * 64;
-    const int nc = min(64, C - c0);
-    const float *src = w + ((size_t)k * C + c0) * taps;
-    for (int i = threadIdx.x; i < nc * taps; i += 256) stage[i] = src[i];
-    __syncthreads();
-    for (int i = threadIdx.x; i < nc * taps; i += 256) {
-        const int t = i / nc, c = i - t * nc;
-        wp[(size_t)(t * KPad + k) * Mp + c0 + c] = stage[c * taps + t];
-    }
+    const int M = bwd ? C : K, Cred = bwd ? K : C, chunks = (Cred + BK - 1) / BK, RS = R * S;
+    const size_t sm = bwd ? (size_t)RS : (size_t)C * RS, sc = bwd ? (size_t)C * RS : (size_t)RS;
+    const dim3 grid((unsigned)((Mp + 15) / 16) * (unsigned)(2 * chunks));
+    const size_t lds = (bwd ? (size_t)8 * (16 * RS + 1) : (size_t)16 * (8 * RS + 1)) * sizeof(float);   // at most 33 KB: 64 taps
+    if (bwd) hipLaunchKernelGGL(pack_gather_k<true>, grid, dim3(256), lds, stream(), M, Cred, Mp, R, S, sH, sW, sm, sc, w, subs);
+    else hipLaunchKernelGGL(pack_gather_k<false>, grid, dim3(256), lds, stream(), M, Cred, Mp, R, S, sH, sW, sm, sc, w, subs);
+    DOPT_LAUNCH_CHECK();
+    return DOPT_HIP_OK;
 }
 
 int round_up(int v, int to) { return (v + to - 1) / to * to; }
@@ -1942,10 +2081,10 @@ int launch_splitk_reduce(size_t elems, int splits, const float *partial, float *
     return DOPT_HIP_OK;
 }
 
-using GatherWide = Tile<64, 256, 1, 4>;     // few output channels, many pixels
-using GatherSquare = Tile<128, 128, 2, 2>;  // enough tiles for two workgroups per CU
-using GatherDeep = Tile<128, 128, 2, 4>;    // few tiles: 8 wavefronts per workgroup, one workgroup per CU
-using GatherTall = Tile<160, 128, 1, 4>;    // 160 output channels (and 480, ...): 64- and 128-row tiles would multiply a fifth more rows than there are
+// Eight wavefronts of 32 x 64, one workgroup per CU.  (Four of 64 x 64, two workgroups per CU, hid their loads as well but had
+// twice the values to split per wavefront: 5 x 5 layers backward-data 104 against 101 us before the splitting was overlapped.)
+using GatherWide = Tile<64, 256, 2, 4>;     // few output channels, many pixels
+using GatherSquare = Tile<128, 128, 4, 2>;
 
 unsigned div_magic(unsigned d) { return (unsigned)((((unsigned long long)1 << 32) / d) + 1); }
 
@@ -2140,12 +2279,10 @@ int patch_splits(int tiles, int chunks, int slots, int BM, int BN, size_t out_el
     return best;
 }
 
-// The same estimate for the general kernels, whose unit is a slab of 16 reduction steps.  0.33 TFLOP/s per CU is what their loops
-// sustained on the fp32 instruction; on the bf16 one they are about 1.4 times as fast, and with 0.5 here nearly every layer is
-// cut the same (Wide-ResNet-28-10 step 21.87 against 21.89 ms, the 5 x 5 layers above 271.4 against 271.5 us).
-int gather_splits(int tiles, int slabs, int slots, int BM, int BN, size_t out_elems, int cap = 64)
+// The same estimate for the general kernels, whose unit is a slab of 16 reduction steps, at the rate that one CU sustains.
+constexpr double kGatherRate = 0.6, kWgradRate = 0.33;
+int gather_splits(int tiles, int slabs, int slots, int BM, int BN, size_t out_elems, double cu_tflops, int cap)
 {
-    const double cu_tflops = 0.33;
     const double per_cu = (double)slots / num_cus();
     const double t_slab = 2.0 * BM * BN * 16 / (cu_tflops * 1e6 / per_cu);
     int best = 1;
@@ -2598,6 +2735,30 @@ int run_dense2x2_wgrad(const dopt_hip_conv_desc *d, const float *dy, const float
     return rc;
 }
 
+template <class T, int SL, auto kKernel, class Args>
+int launch_gather_kernel(const Args &args, dim3 grid)
+{
+    constexpr size_t lds = GatherLds<T, SL>::BYTES;
+    if constexpr (lds > 64 * 1024) {   // a kernel has to be told once
+        static bool raised = false;
+        if (!raised) {
+            DOPT_HIP_CHECK(hipFuncSetAttribute((const void *)kKernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            raised = true;
+        }
+    }
+    hipLaunchKernelGGL(kKernel, grid, dim3(T::THREADS), lds, stream(), args);
+    DOPT_LAUNCH_CHECK();
+    return DOPT_HIP_OK;
+}
+
+template <class T, int SL>
+int launch_gather(int mode, const GatherConv &g, dim3 grid)
+{
+    if (mode == 0) return launch_gather_kernel<T, SL, conv_gather_k<T, SL, 0>>(g, grid);
+    if (mode == 1) return launch_gather_kernel<T, SL, conv_gather_k<T, SL, 1>>(g, grid);
+    return launch_gather_kernel<T, SL, conv_gather_k<T, SL, 2>>(g, grid);
+}
+
 // Packs the filter w[K][C][g.R * g.S] and runs conv_gather_k on a problem whose geometry the caller
 // has filled in (dimensions, padding, stride, output placement).  mode as conv_gather_k's kMode.
 int gather_launch(GatherConv g, int mode, int K, int C, const float *in, const float *w, float *out)
@@ -2612,22 +2773,13 @@ int gather_launch(GatherConv g, int mode, int K, int C, const float *in, const f
     const bool dense = g.out_sy == 1 && g.out_sx == 1 && g.out_plane == g.OH * g.OW;
 
     // tile shape: 64-row tiles for <= 64 output channels and wherever 128-row tiles would pad more;
-    // otherwise 128x128, with 8 wavefronts per workgroup when there are too few tiles to give every
-    // CU two 4-wavefront workgroups
-    enum { kWide, kSquare, kDeep } shape;
-    int BM, BN, blocks_wanted;
-    if (g.Mout <= 64 || (g.Mout + 63) / 64 * 64 < (g.Mout + 127) / 128 * 128) {
-        shape = kWide; BM = 64; BN = 256; blocks_wanted = 2 * num_cus();
-    } else {
-        BM = 128; BN = 128;
-        const int t = ((g.Mout + 127) / 128) * ((g.ncols + 127) / 128);
-        if (t >= 2 * num_cus()) { shape = kSquare; blocks_wanted = 2 * num_cus(); }
-        else { shape = kDeep; blocks_wanted = num_cus(); }
-    }
+    // otherwise 128x128
+    const bool wide = g.Mout <= 64 || (g.Mout + 63) / 64 * 64 < (g.Mout + 127) / 128 * 128;
+    const int BM = wide ? 64 : 128, BN = wide ? 256 : 128;
     g.mtiles = (g.Mout + BM - 1) / BM;
     g.ntiles = (g.ncols + BN - 1) / BN;
     const int tiles = g.mtiles * g.ntiles;
-    int splits = gather_splits(tiles, g.slabs_total, blocks_wanted, BM, BN, g.out_elems);
+    int splits = gather_splits(tiles, g.slabs_total, num_cus(), BM, BN, g.out_elems, kGatherRate, 64);
     // the split reduction works on float4 over a dense output
     if (g.out_elems % 4 != 0 || !aligned16(out) || !dense) splits = 1;
     g.slabs_per_split = (g.slabs_total + splits - 1) / splits;
@@ -2636,45 +2788,23 @@ int gather_launch(GatherConv g, int mode, int K, int C, const float *in, const f
 
     if ((size_t)BK * g.Mp * sizeof(float) > 0x7fffffffu)
         return fail(DOPT_HIP_ERR_UNSUPPORTED, "convolution: more than 2^25 output channels are not supported");
-    const size_t wp_elems = (size_t)taps * g.CinPad * g.Mp;
-    const size_t wp_bytes = (wp_elems * sizeof(float) + 255) / 256 * 256;
+    const size_t wp_bytes = ((size_t)g.slabs_total * g.Mp * 96 + 255) / 256 * 256;
     const size_t part_bytes = splits > 1 ? (size_t)splits * g.out_elems * sizeof(float) : 0;
     char *ws = (char *)workspace(wp_bytes + part_bytes);
     if (!ws) return DOPT_HIP_ERR_OOM;
     float *wp = (float *)ws;
     float *partial = (float *)(ws + wp_bytes);
-
-    // pack the filter
-    if (g.CinPad != g.Cin || g.Mp != g.Mout) {
-        if (capturing()) return fail(DOPT_HIP_ERR_UNSUPPORTED, "convolution: a fill cannot be recorded into a graph");
-        DOPT_HIP_CHECK(hipMemsetAsync(wp, 0, wp_elems * sizeof(float), stream()));
-    }
-    if (!bwd) {
-        dim3 grid((unsigned)((K + 63) / 64), (unsigned)((C * taps + 63) / 64));
-        hipLaunchKernelGGL(pack_fwd_k, grid, dim3(256), 0, stream(), K, C, taps, g.CinPad, g.Mp, w, wp);
-    } else {
-        dim3 grid((unsigned)K, (unsigned)((C + 63) / 64));
-        hipLaunchKernelGGL(pack_bwd_k, grid, dim3(256), (size_t)64 * taps * sizeof(float), stream(), K, C, taps,
-                           g.CinPad, g.Mp, w, wp);
-    }
-    DOPT_LAUNCH_CHECK();
+    SubFilters subs{};
+    subs.n = 1;
+    subs.f[0] = SubFilter{wp, g.R, g.S, 0, 0};
+    if (int rc = launch_pack_gather(bwd, K, C, g.R, g.S, 1, 1, g.Mp, w, subs)) return rc;
 
     g.in = in;
     g.wp = wp;
     g.in_bytes = (size_t)g.N * g.Cin * g.IH * g.IW * sizeof(float);
     g.out = splits > 1 ? partial : out;
     dim3 grid(xcd_grid((unsigned)(tiles * splits)));
-#define DOPT_GATHER(TILE)                                                                                      \
-    do {                                                                                                       \
-        if (mode == 0) hipLaunchKernelGGL((conv_gather_k<TILE, 0>), grid, dim3(TILE::THREADS), 0, stream(), g); \
-        else if (mode == 1) hipLaunchKernelGGL((conv_gather_k<TILE, 1>), grid, dim3(TILE::THREADS), 0, stream(), g); \
-        else hipLaunchKernelGGL((conv_gather_k<TILE, 2>), grid, dim3(TILE::THREADS), 0, stream(), g);          \
-    } while (0)
-    if (shape == kWide) DOPT_GATHER(GatherWide);
-    else if (shape == kSquare) DOPT_GATHER(GatherSquare);
-    else DOPT_GATHER(GatherDeep);
-#undef DOPT_GATHER
-    DOPT_LAUNCH_CHECK();
+    if (int rc = wide ? launch_gather<GatherWide, 2>(mode, g, grid) : launch_gather<GatherSquare, 2>(mode, g, grid)) return rc;
     if (splits > 1) return launch_splitk_reduce(g.out_elems, splits, partial, out);
     return DOPT_HIP_OK;
 }
@@ -2700,38 +2830,6 @@ __global__ __launch_bounds__(256) void subfilter_k(int KC, int R, int S, int R2,
         // element that multiplies offset r is the flipped one, w[.., R - 1 - r, S - 1 - s]
         const int r = r0 + (R2 - 1 - tr) * sH, sc = s0 + (S2 - 1 - ts) * sW;
         sub[i] = w[(size_t)kc * (R * S) + (R - 1 - r) * S + (S - 1 - sc)];
-    }
-}
-
-// The packed sub-filters of all classes in one launch: block (k, 64-channel chunk) stages w[k][c0 .. c0+64][*]
-// once and writes each class's taps as pack_bwd_k would write them from that class's sub-filter.
-struct SubFilter {
-    float *wp;            // [(tap * KPad + k)][Mp] of this class
-    int R2, S2, r0, s0;   // tap rows / columns of the class and its first tap offsets
-};
-struct SubFilters {
-    SubFilter f[kGatherJobs];
-    int n;
-};
-__global__ __launch_bounds__(256) void pack_bwd_classes_k(int K, int C, int R, int S, int sH, int sW, int KPad, int Mp,
-                                                           const float *w, SubFilters subs)
-{
-    extern __shared__ float stage[];  // 64 * R * S floats
-    const int k = blockIdx.x, c0 = blockIdx.y * 64, RS = R * S;
-    const int nc = min(64, C - c0);
-    const float *src = w + ((size_t)k * C + c0) * RS;
-    for (int i = threadIdx.x; i < nc * RS; i += 256) stage[i] = src[i];
-    __syncthreads();
-    for (int j = 0; j < subs.n; j++) {
-        const SubFilter f = subs.f[j];
-        const int taps = f.R2 * f.S2;
-        for (int i = threadIdx.x; i < nc * taps; i += 256) {
-            const int t = i / nc, c = i - t * nc, tr = t / f.S2, ts = t - tr * f.S2;
-            // stored tap (tr, ts) stands for offsets r = r0 + (R2 - 1 - tr) * sH, s likewise, and the element
-            // that multiplies offset (r, s) is the flipped one (see subfilter_k)
-            const int r = f.r0 + (f.R2 - 1 - tr) * sH, sc = f.s0 + (f.S2 - 1 - ts) * sW;
-            f.wp[(size_t)(t * KPad + k) * Mp + c0 + c] = stage[c * RS + (R - 1 - r) * S + (S - 1 - sc)];
-        }
     }
 }
 
@@ -2776,21 +2874,17 @@ int run_bwd_strided(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float
             return fail(DOPT_HIP_ERR_UNSUPPORTED, "convolution: more than 2^25 output channels are not supported");
         size_t wp_off[kGatherJobs + 1] = {0};
         for (int j = 0; j < njobs; j++) {
-            const size_t elems = (size_t)jobs[j].ch.taps * jobs[j].cw.taps * KPad * Mp;
-            wp_off[j + 1] = wp_off[j] + (elems * sizeof(float) + 255) / 256 * 256;
+            const size_t slabs = (size_t)jobs[j].ch.taps * jobs[j].cw.taps * KPad / BK;
+            wp_off[j + 1] = wp_off[j] + (slabs * Mp * 96 + 255) / 256 * 256;
         }
         char *ws = (char *)workspace(wp_off[njobs]);
         if (!ws) return DOPT_HIP_ERR_OOM;
-        if (KPad != K || Mp != C) {
-            if (capturing()) return fail(DOPT_HIP_ERR_UNSUPPORTED, "convolution: a fill cannot be recorded into a graph");
-            DOPT_HIP_CHECK(hipMemsetAsync(ws, 0, wp_off[njobs], stream()));
-        }
         const bool wide = C <= 64 || (C + 63) / 64 * 64 < (C + 127) / 128 * 128;
         const int BM = wide ? 64 : 128, BN = wide ? 256 : 128;
         SubFilters subs{};
         GatherGroup gg{};
         subs.n = gg.n = njobs;
-        unsigned blocks = 0, tiles_all = 0;
+        unsigned blocks = 0;
         for (int j = 0; j < njobs; j++) {
             const Job &jb = jobs[j];
             subs.f[j] = SubFilter{(float *)(ws + wp_off[j]), jb.ch.taps, jb.cw.taps, jb.ch.first, jb.cw.first};
@@ -2818,19 +2912,10 @@ int run_bwd_strided(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float
             g.in_bytes = (size_t)g.N * g.Cin * g.IH * g.IW * sizeof(float);
             gg.per[j] = ((unsigned)(g.mtiles * g.ntiles) + 7u) / 8u;
             blocks += 8u * gg.per[j];
-            tiles_all += (unsigned)(g.mtiles * g.ntiles);
         }
-        hipLaunchKernelGGL(pack_bwd_classes_k, dim3((unsigned)K, (unsigned)((C + 63) / 64)), dim3(256),
-                           (size_t)64 * R * S * sizeof(float), stream(), K, C, R, S, sH, sW, KPad, Mp, w, subs);
-        DOPT_LAUNCH_CHECK();
-        if (wide)
-            hipLaunchKernelGGL((conv_gather_group_k<GatherWide, 1>), dim3(blocks), dim3(GatherWide::THREADS), 0, stream(), gg);
-        else if (tiles_all >= 2u * (unsigned)num_cus())
-            hipLaunchKernelGGL((conv_gather_group_k<GatherSquare, 1>), dim3(blocks), dim3(GatherSquare::THREADS), 0, stream(), gg);
-        else
-            hipLaunchKernelGGL((conv_gather_group_k<GatherDeep, 1>), dim3(blocks), dim3(GatherDeep::THREADS), 0, stream(), gg);
-        DOPT_LAUNCH_CHECK();
-        return DOPT_HIP_OK;
+        if (int rc = launch_pack_gather(true, K, C, R, S, sH, sW, Mp, w, subs)) return rc;
+        if (wide) return launch_gather_kernel<GatherWide, 2, conv_gather_group_k<GatherWide, 2, 1>>(gg, blocks);
+        return launch_gather_kernel<GatherSquare, 2, conv_gather_group_k<GatherSquare, 2, 1>>(gg, blocks);
     }
     void *sub = nullptr;
     if (int rc = scratch_alloc(&sub, d->K * d->C * d->R * d->S * sizeof(float))) return rc;
@@ -3484,7 +3569,7 @@ int dopt_hip_conv_bwd_filter(const dopt_hip_conv_desc *d, const float *dy, const
     f.ntiles = (f.ncols + BN - 1) / BN;
     const int tiles = f.mtiles * f.ntiles;
     // filter gradients are short and wide (small output, long pixel reduction): allow deep splits
-    int splits = gather_splits(tiles, f.slabs_total, 2 * num_cus(), BM, BN, f.out_elems, 512);
+    int splits = gather_splits(tiles, f.slabs_total, 2 * num_cus(), BM, BN, f.out_elems, kWgradRate, 512);
     f.slabs_per_split = (f.slabs_total + splits - 1) / splits;
     splits = (f.slabs_total + f.slabs_per_split - 1) / f.slabs_per_split;
     f.splits = splits;
