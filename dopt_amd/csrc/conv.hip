@@ -1509,7 +1509,7 @@ __global__ __launch_bounds__(256) void split_sum_k(size_t n4, int splits, size_t
 // (tap row r): a wavefront keeps the three taps s = 0..2 of its tap row in three 32x32
 // accumulators.  A lane's operands for a 16-pixel slab are pixels kh*8 .. kh*8+7 of the slab
 // (kh = lane / 32): two 128-bit reads of dy, and for x a window that serves all three taps by
-// register selection.  The products run on the bf16 matrix instruction, each operand split into three parts in registers
+// register selection.  The products run on the bf16 matrix instruction, each operand split into three parts
 // (mfma_core.h).
 //
 // Geometry of a 64-pixel chunk (kGeo):
@@ -1537,7 +1537,7 @@ struct WgradPatch {
     size_t dy_bytes, x_bytes;
 };
 
-template <int WM, int WC, int kGeo>
+template <int WM, int WC, int kGeo, bool kPre>
 __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const unsigned block_id)
 {
     constexpr int BM = 32 * WM, BC = 32 * WC, THREADS = 64 * 3 * WM * WC, NPIX = 64, APITCH = NPIX + 4;
@@ -1547,10 +1547,13 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
     constexpr int NBQ = kGeo == 0 ? (WC == 1 ? 2 : 3) : (BC * 16 + THREADS - 1) / THREADS;
     static_assert(WM * WC == 4 || WM * WC == 5, "twelve or fifteen wavefronts: 4 or 5 (row, channel) groups x 3 tap rows");
     extern __shared__ __attribute__((aligned(16))) float lds[];
+    // first column of a patch row; pitch of the rows of a 4 x 4 image, and its distance to the next image
+    constexpr int COL0 = kPre && kGeo == 0 ? 8 : 4, RP1 = kPre ? 8 : 12, IP1 = kPre ? 40 : 72;
     const int bsize = BC * p.cstride;
-    float *const A0 = lds;                     // [2][BM * APITCH]
-    float *const B0 = lds + 2 * BM * APITCH;   // [2][bsize]
-    float *const dummy = B0 + 2 * bsize;       // 4 floats absorbing the stores of unused slots
+    const int bstride = kPre ? bsize / 2 * 3 : bsize;           // floats of a patch buffer: three 16-bit parts a value
+    float *const A0 = lds;                                      // [2][BM * APITCH]
+    float *const B0 = lds + 2 * BM * APITCH - (kPre ? 4 : 0);   // [2][bstride] (the pad of the last row before it is not used)
+    float *const dummy = B0 + 2 * bstride;                      // 4 floats absorbing the stores of unused slots
 
     unsigned L;
     const unsigned tiles = (unsigned)(p.mtiles * p.ctiles);
@@ -1586,7 +1589,7 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
     const int a_lds = a_row * APITCH + a_quad * 4;
     const int a_rows = min(BM, p.K - k0);
     unsigned b_voff[NBQ];
-    int b_lds[NBQ];   // float index inside a patch buffer (a multiple of four) or -1; geometry 0: + 1 = top halo row, + 2 = bottom halo row
+    int b_lds[NBQ];   // index of the value inside a patch buffer (a multiple of four) or -1; geometry 0: + 1 = top halo row, + 2 = bottom halo row
 #pragma unroll
     for (int i = 0; i < NBQ; i++) {
         const int b = i * THREADS + tid;
@@ -1597,12 +1600,12 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
             const bool ok = c < BC && c0 + c < p.C;
             // row p0 - 1 + pr of channel c0 + c; p0 and the image are added per chunk
             b_voff[i] = ok ? (unsigned)(((c0 + c) * p.H + pr) * p.W + quad * 4) * 4u : kOobOffset;
-            b_lds[i] = c < BC ? c * p.cstride + pr * p.ppitch + 4 + quad * 4 + (pr == 0 ? 1 : pr == p.G + 1 ? 2 : 0) : -1;
+            b_lds[i] = c < BC ? c * p.cstride + pr * p.ppitch + COL0 + quad * 4 + (pr == 0 ? 1 : pr == p.G + 1 ? 2 : 0) : -1;
         } else if (kGeo == 1) {
             const int c = b / 16, j = (b / 4) % 4, row = b % 4;  // image j of the chunk, image row `row`
             const bool ok = c < BC && c0 + c < p.C;
             b_voff[i] = ok ? (unsigned)((j * p.C + c0 + c) * 16 + row * 4) * 4u : kOobOffset;
-            b_lds[i] = c < BC ? c * p.cstride + j * 72 + (row + 1) * 12 + 4 : -1;
+            b_lds[i] = c < BC ? c * p.cstride + j * IP1 + (row + 1) * RP1 + COL0 : -1;
         } else {
             const int c = b / 16, j = b % 16;  // the whole 2x2 image j is one quad
             const bool ok = c < BC && c0 + c < p.C;
@@ -1646,7 +1649,7 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
     };
     auto stash = [&](int buf, auto exact_tag) {
         constexpr bool exact = decltype(exact_tag)::value != 0;
-        float *A = A0 + buf * (BM * APITCH), *B = B0 + buf * bsize;
+        float *A = A0 + buf * (BM * APITCH), *B = B0 + buf * bstride;
 #pragma unroll
         for (int i = 0; i < NAQ; i++) {
             const float4 v = areg[i];
@@ -1657,7 +1660,13 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
 #pragma unroll
         for (int i = 0; i < NBQ; i++) {
             const float4 v = exact ? breg[i] : make_float4(breg[i].x * kSplitUp, breg[i].y * kSplitUp, breg[i].z * kSplitUp, breg[i].w * kSplitUp);
-            if (kGeo != 2) {
+            if constexpr (kPre && !exact) {
+                uint2 q3[3];
+                split_pair(v.x, v.y, q3[0].x, q3[1].x, q3[2].x);
+                split_pair(v.z, v.w, q3[0].y, q3[1].y, q3[2].y);
+#pragma unroll
+                for (int t = 0; t < 3; t++) *(uint2 *)(b_lds[i] >= 0 ? B + t * (bsize / 2) + (b_lds[i] & ~3) / 2 : dummy) = q3[t];
+            } else if constexpr (kGeo != 2) {
                 *(float4 *)(b_lds[i] >= 0 ? B + (b_lds[i] & ~3) : dummy) = v;
             } else {
                 float *q = b_lds[i] >= 0 ? B + b_lds[i] : dummy;  // rows 1 and 2 of the cell block, columns 1..2
@@ -1672,40 +1681,44 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
 
     // ---- fragment addresses
     const int a_frag = (wm * 32 + l32) * APITCH + kh * 8;
-    // float4 index inside a patch buffer: of slab 0, and how far the other slabs are from it (the same for all lanes)
+    // index inside a patch buffer: of slab 0, and how far the other slabs are from it (the same for all lanes)
     const int runs_row = p.W / 8;
-    const int b_frag = kGeo == 0 ? ((wc * 32 + l32) * p.cstride + (dr + (runs_row == 1 ? kh : 0)) * p.ppitch + (runs_row == 1 ? 0 : kh * 8)) / 4 + 1
-                     : kGeo == 1 ? ((wc * 32 + l32) * p.cstride + (2 * kh + dr) * 12) / 4 + 1   // image s, image rows 2kh and 2kh+1
-                                 : ((wc * 32 + l32) * p.cstride + 2 * kh * 16 + dr * 4) / 4;    // images 4s+2kh and 4s+2kh+1
+    const int b_frag = kGeo == 0 ? (wc * 32 + l32) * p.cstride + (dr + (runs_row == 1 ? kh : 0)) * p.ppitch + (runs_row == 1 ? 0 : kh * 8) + COL0
+                     : kGeo == 1 ? (wc * 32 + l32) * p.cstride + (2 * kh + dr) * RP1 + COL0     // image s, image rows 2kh and 2kh+1
+                                 : (wc * 32 + l32) * p.cstride + 2 * kh * 16 + dr * 4;          // images 4s+2kh and 4s+2kh+1
     // geometry 0: slab s covers the 8-pixel runs 2s (kh = 0) and 2s+1 (kh = 1) of the chunk
-    auto b_step = [&](int s) {
-        return kGeo == 0 ? (2 * s / runs_row * p.ppitch + 2 * s % runs_row * 8) / 4 : kGeo == 1 ? s * 72 / 4 : s * 64 / 4;
-    };
+    auto b_step = [&](int s) { return kGeo == 0 ? 2 * s / runs_row * p.ppitch + 2 * s % runs_row * 8 : kGeo == 1 ? s * IP1 : s * 64; };
 
     v16f acc[3], low[kLow ? 3 : 1];
     typedef __attribute__((address_space(3))) float lds_float_t;
-    // Fetching runs one chunk ahead and also past the end of this block's range: those loads are
+    // Fetching runs one chunk ahead, or two, and also past the end of this block's range: those loads are
     // range-checked and their data lands in the LDS buffer that is not read again.
+    // Two chunks ahead a chunk is stored at the beginning of the one before it, and the wavefronts of a SIMD, which have
+    // drifted apart behind the barrier by then, store under each other's matrix instructions; one ahead, at its end, they all
+    // store at once.  It takes registers: not with fifteen wavefronts.
+    constexpr bool kEarly = kPre && kLow;
     struct Frag {
         float4 a_lo, a_hi, q[4];
         float e[4];
     };
-    auto read_frag = [&](int buf, int s_) {
+    auto read_frag = [&](int buf, int s_, auto parts_tag) {
+        constexpr bool parts = decltype(parts_tag)::value != 0;   // dy alone
         Frag f;
         const float *A = A0 + buf * (BM * APITCH) + a_frag;
         // float4 indexing keeps the 16-byte alignment of the patch reads visible to the compiler
-        const float4 *bq = (const float4 *)B0 + buf * (bsize / 4) + b_frag + b_step(s_);
+        const float4 *bq = (const float4 *)B0 + (buf * bstride + b_frag + b_step(s_)) / 4;
         // The edge-column reads are volatile so that the compiler does not fuse a whole window
         // into one run starting at the unaligned edge (it would then read it in 2-dword pieces).
         const volatile lds_float_t *be = (const volatile lds_float_t *)bq;
         f.a_lo = *(const float4 *)(A + s_ * 16);
         f.a_hi = *(const float4 *)(A + s_ * 16 + 4);
+        if constexpr (parts) return f;
         if constexpr (kGeo == 0) {
             f.q[0] = bq[0]; f.q[1] = bq[1];
             f.e[0] = be[-1]; f.e[1] = be[8];
         } else if constexpr (kGeo == 1) {
-            f.q[0] = bq[0]; f.q[1] = bq[3];   // the next patch row is 12 floats on
-            f.e[0] = be[-1]; f.e[1] = be[4]; f.e[2] = be[11]; f.e[3] = be[16];
+            f.q[0] = bq[0]; f.q[1] = bq[RP1 / 4];
+            f.e[0] = be[-1]; f.e[1] = be[4]; f.e[2] = be[RP1 - 1]; f.e[3] = be[RP1 + 4];
         } else {
             // (image, row) quads: image 0 rows 0, 1 then image 1 rows 0, 1
             f.q[0] = bq[0]; f.q[1] = bq[1]; f.q[2] = bq[4]; f.q[3] = bq[5];
@@ -1744,11 +1757,12 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
                     acc[ds] = __builtin_amdgcn_mfma_f32_32x32x2f32(a8[ks], win[ks / 2][(ks & 1) + ds], acc[ds], 0, 0, 0);
         }
     };
-    // The same sixteen pixels on the bf16 matrix instructions (eighteen of 32 cycles for twenty-four of 64): the fragments are
-    // split in registers (mfma_core.h), the x pixels in pairs that are tap column 1's operands as they are; those of columns 0
-    // and 2 are their neighbouring halves with the edge pixels.  What bounds it is the splitting, 120 vector instructions a step
-    // and wavefront under the 576 cycles of the matrix ones.  (Reading the fragments one step ahead, as the fp32 form did, needs
-    // 30 more registers than there are: 399 us for the first layer below.)
+    // The same sixteen pixels on the bf16 matrix instructions (eighteen of 32 cycles for twenty-four of 64): dy's fragments are
+    // split in registers (mfma_core.h); x, which twelve wavefronts read, when it is stored (kPre), in pairs of pixels that are tap
+    // column 1's operands as they are; those of columns 0 and 2 are their neighbouring halves with the edge pixels.  320 -> 320
+    // channels on 16 x 16, batch 128: both split in registers 296 us, x when stored 289, stored at the beginning of a chunk 278;
+    // 640 -> 640 on 8 x 8 305, 296, 279; of them 205 us are matrix time at the rate of a large product.  (Reading the fragments one step
+    // ahead, as the fp32 form did, needs 30 more registers than there are.)
     // The instruction rounds down what lies below its guard bits.  That is the same way in every block, so no sum over blocks
     // removes it, and the five small products of a slab suffer it most: with all six in one accumulator 77 % of the error was a
     // common offset, and it was 1.25 to 1.7 times the fp32 instruction's.  So twelve wavefronts keep the small products in an
@@ -1757,7 +1771,7 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
     // 128 images of 320 -> 320 channels, 16 x 16: fp32 450 us, one accumulator 292, this 296; 160 -> 160, 32 x 32: 486, 302, 327.
     // Error against float64 (one half of x zero): 64 -> 64 channels, 32 x 32, 2.8e-7 / 4.8e-7 / 1.3e-7; 160 -> 160, 32 x 32,
     // 6.4e-7 / 1.07e-6 / 5.2e-7; 640 -> 640, 8 x 8, batch 256, 6.7e-7 / 8.4e-7 / 2.6e-7.
-    constexpr int NW = kGeo == 0 ? 5 : kGeo == 1 ? 6 : 8;   // pairs of pixels
+    constexpr int NW = kPre ? 6 : kGeo == 0 ? 5 : kGeo == 1 ? 6 : 8;   // pairs of pixels
     v4u ap[3];
     unsigned q[3][NW];
     auto split_frag = [&](const Frag &f) {
@@ -1770,6 +1784,7 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
             ap[1] = v4u{hm0.z, hm0.w, hm1.z, hm1.w};
             ap[2] = v4u{l0.x, l0.y, l1.x, l1.y};
         }
+        if constexpr (kPre) return;
         static_for<0, kGeo == 2 ? 4 : 2>([&](auto itag) {
             constexpr int i = decltype(itag)::value;
             split_pair(f.q[i].x, f.q[i].y, q[0][2 * i], q[1][2 * i], q[2][2 * i]);
@@ -1777,6 +1792,21 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
         });
         if constexpr (kGeo != 2) split_pair(f.e[0], f.e[1], q[0][4], q[1][4], q[2][4]);
         if constexpr (kGeo == 1) split_pair(f.e[2], f.e[3], q[0][NW - 1], q[1][NW - 1], q[2][NW - 1]);
+    };
+    auto read_parts = [&](int buf, int s_) {   // the x window's pairs where they were split when stored
+        const unsigned *const first = (const unsigned *)B0 + buf * bstride + (b_frag + b_step(s_)) / 2;
+#pragma unroll
+        for (int t = 0; t < 3; t++) {
+            const unsigned *const w = first + t * (bsize / 2);
+            if constexpr (kGeo == 0) {
+                const v4u m = *(const v4u *)w;
+                q[t][0] = m.x; q[t][1] = m.y; q[t][2] = m.z; q[t][3] = m.w;
+                q[t][4] = w[-1]; q[t][NW - 1] = w[4];
+            } else {
+                const uint2 r0 = *(const uint2 *)w, r1 = *(const uint2 *)(w + RP1 / 2);
+                q[t][0] = r0.x; q[t][1] = r0.y; q[t][2] = r1.x; q[t][3] = r1.y;
+            }
+        }
     };
     auto products_split = [&]() {
         auto mid = [](unsigned hi, unsigned lo) { return __builtin_amdgcn_alignbit(hi, lo, 16); };             // (lo.1, hi.0)
@@ -1786,7 +1816,17 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
             constexpr int part = 2 - decltype(ptag)::value;
             const unsigned *const w = q[part];
             v4u b[3];
-            if constexpr (kGeo == 0) {
+            if constexpr (kPre && kGeo == 0) {   // (the edge words hold two pixels of which one is the window's)
+                const unsigned m0 = mid(w[1], w[0]), m1 = mid(w[2], w[1]), m2 = mid(w[3], w[2]);
+                b[0] = v4u{mid(w[0], w[4]), m0, m1, m2};
+                b[1] = v4u{w[0], w[1], w[2], w[3]};
+                b[2] = v4u{m0, m1, m2, mid(w[NW - 1], w[3])};
+            } else if constexpr (kPre) {         // (what is left and right of a 4 x 4 image's row is zero)
+                const unsigned m0 = mid(w[1], w[0]), m1 = mid(w[3], w[2]);
+                b[0] = v4u{w[0] << 16, m0, w[2] << 16, m1};
+                b[1] = v4u{w[0], w[1], w[2], w[3]};
+                b[2] = v4u{m0, w[1] >> 16, m1, w[3] >> 16};
+            } else if constexpr (kGeo == 0) {
                 const unsigned m0 = mid(w[1], w[0]), m1 = mid(w[2], w[1]), m2 = mid(w[3], w[2]);
                 b[0] = v4u{left(w[4], w[0]), m0, m1, m2};
                 b[1] = v4u{w[0], w[1], w[2], w[3]};
@@ -1819,21 +1859,27 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
         for (int t = 0; t < 3; t++)
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[t][v] = low[kLow ? t : 0][v] = 0.0f;
+        // halo cells are not written by the loop
+        for (int i = tid; i < 2 * bstride; i += THREADS) B0[i] = 0.0f;
         fetch();
+        __syncthreads();
         stash(0, exact_tag);
+        if (kEarly) fetch();
         __syncthreads();
         int cur = 0;
         for (int chunk = from; chunk < to; ++chunk) {
             static_for<0, 4>([&](auto stag) {
                 constexpr int s = decltype(stag)::value;
-                if constexpr (s == 0) fetch();
+                if constexpr (!kEarly && s == 0) fetch();
                 if constexpr (exact) {
-                    products_fp32(read_frag(cur, s));
+                    products_fp32(read_frag(cur, s, StepTag<0>{}));
                 } else {
-                    split_frag(read_frag(cur, s));
+                    if constexpr (kPre) read_parts(cur, s);
+                    split_frag(read_frag(cur, s, StepTag<kPre>{}));
                     products_split();
                 }
-                if constexpr (s == 3) stash(cur ^ 1, exact_tag);
+                if constexpr (s == (kEarly ? 0 : 3)) stash(cur ^ 1, exact_tag);
+                if constexpr (kEarly && s == 1) fetch();
             });
             __syncthreads();
             cur ^= 1;
@@ -1846,9 +1892,6 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
                 acc[t][v] = kLow ? (acc[t][v] + low[kLow ? t : 0][v]) * kSplitDown : acc[t][v] * (up * (kSplitDown / kSplitUp));
     };
     for (int pass = 0;; pass++) {
-        // halo cells are not written by the loop: clear both patch buffers before it
-        for (int i = tid; i < 2 * bsize; i += THREADS) B0[i] = 0.0f;
-        __syncthreads();
         run(StepTag<0>{});
         {
             // the parts of an infinity hold NaNs: a tile that is not finite is formed again with the fp32 instruction
@@ -1900,10 +1943,10 @@ __device__ __forceinline__ void conv_wgrad_patch_body(const WgradPatch &p, const
     }
 }
 
-template <int WM, int WC, int kGeo>
+template <int WM, int WC, int kGeo, bool kPre>
 __global__ __launch_bounds__(64 * 3 * WM * WC, 1) void conv_wgrad_patch_k(WgradPatch p)
 {
-    conv_wgrad_patch_body<WM, WC, kGeo>(p, blockIdx.x);
+    conv_wgrad_patch_body<WM, WC, kGeo, kPre>(p, blockIdx.x);
 }
 
 // Backward-data and filter gradient of one layer in ONE launch: both read dy and nothing of each other.
@@ -1919,7 +1962,7 @@ __global__ __launch_bounds__(768, 1) void conv_bwd_pair_k(PatchConv a, WgradPatc
         if (threadIdx.x >= (unsigned)T::THREADS) return;
         conv_patch_body<T, NS, true>(a, blockIdx.x);
     } else {
-        conv_wgrad_patch_body<WM, WC, kGeo>(b, blockIdx.x - grid_a);
+        conv_wgrad_patch_body<WM, WC, kGeo, true>(b, blockIdx.x - grid_a);
     }
 }
 
@@ -2993,16 +3036,16 @@ int run_gather(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float *in,
     return gather_launch(g, kBwd ? 1 : 0, (int)d->K, (int)d->C, in, w, out);
 }
 
-template <int WM, int WC, int kGeo>
+template <int WM, int WC, int kGeo, bool kPre = kGeo != 2>
 int launch_wgrad_patch(const WgradPatch &wp, dim3 grid, size_t lds_bytes)
 {
     static bool raised = false;
     if (!raised) {
-        DOPT_HIP_CHECK(hipFuncSetAttribute((const void *)conv_wgrad_patch_k<WM, WC, kGeo>,
+        DOPT_HIP_CHECK(hipFuncSetAttribute((const void *)conv_wgrad_patch_k<WM, WC, kGeo, kPre>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         raised = true;
     }
-    hipLaunchKernelGGL((conv_wgrad_patch_k<WM, WC, kGeo>), grid, dim3(64 * 3 * WM * WC), lds_bytes, stream(), wp);
+    hipLaunchKernelGGL((conv_wgrad_patch_k<WM, WC, kGeo, kPre>), grid, dim3(64 * 3 * WM * WC), lds_bytes, stream(), wp);
     DOPT_LAUNCH_CHECK();
     return DOPT_HIP_OK;
 }
@@ -3024,6 +3067,7 @@ struct WgradSetup {
     bool ok;
     WgradPatch wp;
     bool tall;            // 128 rows x 32 channels per block
+    bool pre;             // x is split when it is stored
     int rows;             // output channels per block: 128 (tall), 160 (x 32 channels) or 64 (x 64 channels)
     int geo, tiles, splits;
     size_t out_elems, lds_bytes;
@@ -3058,7 +3102,6 @@ WgradSetup wgrad_patch_setup(const dopt_hip_conv_desc *d, const float *dw)
     } else {
         return u;
     }
-    while (wp.cstride % 8 != 4) wp.cstride += 4;  // 128-bit reads by 32 channels at this stride touch every LDS bank once
     // 128 rows x 32 channels, or 64 x 64 when that pads the output channels less (160 -> 192, not 256)
     // ... or 160 x 32 where that pads them less than both (160 channels: 160 rows, not 192 or 256)
     const int up64 = (int)((d->K + 63) / 64 * 64), up128 = (int)((d->K + 127) / 128 * 128), up160 = (int)((d->K + 159) / 160 * 160);
@@ -3068,6 +3111,13 @@ WgradSetup wgrad_patch_setup(const dopt_hip_conv_desc *d, const float *dw)
     const bool tall = !rows160 && d->K >= 128 && up128 <= up64;
     if (!tall && !rows160 && W == 64) return u;
     const int BM = rows160 ? 160 : tall ? 128 : 64, BC = BM == 64 ? 64 : 32;
+    // x is split when it is stored: not with 2 x 2 images, whose values are single 16-bit ones, nor where the parts of 160 rows
+    // and of rows of 64 pixels do not fit the LDS together
+    const bool pre = geo != 2 && !(rows160 && W == 64);
+    // 128-bit reads by 32 channels at these strides touch every LDS bank once: an odd number of 16-byte pieces (with parts, of
+    // 16-bit values; one piece at least behind the last row, which holds its right edge)
+    if (pre) wp.cstride = geo == 0 ? ((wp.G + 2) * wp.ppitch / 8 + 1 | 1) * 8 : 21 * 8;
+    else while (wp.cstride % 8 != 4) wp.cstride += 4;
     wp.N = (int)d->N; wp.C = (int)d->C; wp.K = (int)d->K; wp.H = H; wp.W = W;
     wp.quads_row = W / 4;
     wp.mtiles = (wp.K + BM - 1) / BM;
@@ -3105,12 +3155,12 @@ WgradSetup wgrad_patch_setup(const dopt_hip_conv_desc *d, const float *dw)
     wp.chunks_per_split = (wp.chunks_total + splits - 1) / splits;
     splits = (wp.chunks_total + wp.chunks_per_split - 1) / wp.chunks_per_split;
     wp.splits = splits;
-    const size_t lds_main = ((size_t)2 * BM * 68 + (size_t)2 * BC * wp.cstride + 4) * sizeof(float);
+    const size_t lds_main = ((size_t)2 * BM * 68 + (pre ? (size_t)3 * BC * wp.cstride : (size_t)2 * BC * wp.cstride + 4)) * sizeof(float);
     const size_t lds_epi = (size_t)32 * (BC * 9 + 1) * sizeof(float);
     u.lds_bytes = lds_main > lds_epi ? lds_main : lds_epi;
     if (u.lds_bytes > 160 * 1024) return u;
     wp.split_stride = out_elems;
-    u.tall = tall; u.rows = BM; u.geo = geo; u.tiles = tiles; u.splits = splits; u.out_elems = out_elems;
+    u.tall = tall; u.pre = pre; u.rows = BM; u.geo = geo; u.tiles = tiles; u.splits = splits; u.out_elems = out_elems;
     u.ok = true;
     return u;
 }
@@ -3147,6 +3197,7 @@ int dispatch_wgrad_patch(const WgradSetup &u)
     const WgradPatch &wp = u.wp;
     const dim3 grid(xcd_grid((unsigned)(u.tiles * u.splits)));
     const int geo = u.geo;
+    if (u.rows == 160 && geo == 0 && !u.pre) return launch_wgrad_patch<5, 1, 0, false>(wp, grid, u.lds_bytes);
     if (u.rows == 160) return geo == 0 ? launch_wgrad_patch<5, 1, 0>(wp, grid, u.lds_bytes)
                             : geo == 1 ? launch_wgrad_patch<5, 1, 1>(wp, grid, u.lds_bytes)
                                        : launch_wgrad_patch<5, 1, 2>(wp, grid, u.lds_bytes);
