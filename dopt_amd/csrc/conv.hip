@@ -93,7 +93,8 @@ struct GatherConv {
 // 128-bit read and neighbouring lanes' reads are neighbours.  A stage is SL slabs; under the matrix instructions of one the next is
 // split and stored and the one after it is loaded, each piece pinned to a step, and the workgroup meets once per stage.  Split
 // behind the products instead, with every wavefront at the same place: 5 x 5 layers below 101 and 69 us, now 75 and 58.
-// 50 images of 48 x 45 x 39, 100 filters of 5 x 5 at stride 2: forward 103 -> 58 us, backward-data 95 -> 75; 64 -> 64 channels of 3 x 3
+// 50 images of 48 x 45 x 39, 100 filters of 5 x 5 at stride 2: forward 103 -> 58 us, backward-data 95 -> 75 (with a last stage that
+// only multiplies 9 -> 7 us for 2 images of 19 x 46 x 14, as before); 64 -> 64 channels of 3 x 3
 // on 64 images of 33 x 31 46 -> 37 us; Wide-ResNet-28-10's two strided 3 x 3 layers backward 270 -> 240 us.  A stage of a
 // 64 x 256 tile takes 1.7 us of which 0.9 are matrix time at the rate of a large product; it reads 144 KB of fragments from LDS.
 // Error against float64 (160 -> 320 channels, stride 2): 8.5e-8 forward, 1.7e-7 backward-data (the fp32 instruction: 2.1e-7, 5.3e-7).
@@ -246,7 +247,9 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
     };
     // Under the matrix instructions of a stage the next one, which is in registers, is split and stored, and the one after
     // it is loaded: a slab's values as soon as the slab before in those registers is stored.
-    auto stage = [&](const float *cur, float *nxt) {
+    // The last stage has only its products: with few slabs a block would wait for loads of nothing.
+    auto stage = [&](const float *cur, float *nxt, auto more_tag) {
+        constexpr bool more = decltype(more_tag)::value != 0;
         fragments(cur, 0);
         unsigned voff = 0;
         static_for<0, SL>([&](auto sl_tag) {
@@ -254,16 +257,16 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
             static_for<0, 6>([&](auto tag) {
                 constexpr int s = decltype(tag)::value;
                 if constexpr (s == 0 && sl + 1 < SL) fragments(cur, sl + 1);
-                if constexpr (s < PAIRS) split_b(sl, s);
-                if constexpr (s == 0 && sl == 0) {
+                if constexpr (more && s < PAIRS) split_b(sl, s);
+                if constexpr (more && s == 0 && sl == 0) {
                     store_a(nxt);
                     load_a(slab);
                 }
-                if constexpr (s == PAIRS) {
+                if constexpr (more && s == PAIRS) {
                     store_b(nxt, sl);
                     voff = pixel();
                 }
-                if constexpr (s == PAIRS + 1) {
+                if constexpr (more && s == PAIRS + 1) {
 #pragma unroll
                     for (int i = 0; i < CPT; i++) load_b(sl, i, voff);
                     next_slab();
@@ -280,7 +283,7 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
                 __builtin_amdgcn_sched_barrier(0);
             });
         });
-        __syncthreads();
+        if constexpr (more) __syncthreads();
     };
     auto load_stage = [&](auto masked_tag) {   // all of it at once
         load_a(slab);
@@ -301,10 +304,11 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
         for (int e = 0; e < PAIRS; e++) split_b(sl, e);
         store_b(lds, sl);
     }
-    load_stage(StepTag<0>{});   // (past the last slab: zeros)
-    __syncthreads();
     const int stages = (slab_end - slab_begin + SL - 1) / SL;
-    for (int st = 0; st < stages; ++st) stage(lds + (st & 1) * STAGE, lds + (~st & 1) * STAGE);
+    if (stages > 1) load_stage(StepTag<0>{});
+    __syncthreads();
+    for (int st = 0; st < stages - 1; ++st) stage(lds + (st & 1) * STAGE, lds + (~st & 1) * STAGE, StepTag<1>{});
+    stage(lds + ((stages - 1) & 1) * STAGE, nullptr, StepTag<0>{});
     add_acc(acc, low);
 
     // the parts of an infinity hold NaNs: a tile that is not finite is formed again with the fp32 instruction, a stage at a time
@@ -1274,19 +1278,23 @@ struct FilterGrad {
     size_t out_elems, dy_bytes, x_bytes;
 };
 
-// Products as in conv_gather_body, with the same bound before and now.
+// Products, LDS and stages as in conv_gather_body; here both operands are split when they are stored.  A lane loads one pixel of a
+// stage's 32, lane and lane + 32 neighbouring ones: v_permlane32_swap gives either lane both pixels of one of two rows, and a
+// pair of pixels is a word of each part.  (Split in every wavefront that read a
+// value: 64 -> 64 channels of 3 x 3 on 64 images of 33 x 31 72 us, now 57; 5 x 5 at stride 2, 48 -> 100 on 50 images of 45 x 39, 80 -> 78; the
+// strided layers of Wide-ResNet-28-10 410 + 355 + 76 -> 357 + 353 + 68.  What bounds those now are the gathered loads of x.)
 // TPT = number of column groups of a tile that may belong to different taps (BN / gcd(BN, Cp)):
 // the input displacement and the bounds test are per group, not per element.
 template <class T, int TPT>
-__global__ __launch_bounds__(T::THREADS, T::THREADS / 128) void conv_wgrad_k(FilterGrad p)
+__global__ __launch_bounds__(T::THREADS, 2) void conv_wgrad_k(FilterGrad p)
 {
-    constexpr int BM = T::BM, BN = T::BN, LDA = T::LDA, LDB = T::LDB;
-    static_assert(T::THREADS == 256, "lanes run along 16 pixels, 16 rows per pass");
+    constexpr int BM = T::BM, BN = T::BN, MI = T::MI, NI = T::NI, SL = 2;
+    static_assert(T::THREADS == 512, "lanes run along 32 pixels, 16 rows per pass");
     constexpr int NA = BM / 16, NB = BN / 16;  // scalar loads per thread
     constexpr int GSZ = NB / TPT;              // loads per tap group
-    static_assert(GSZ * TPT == NB, "TPT must divide the loads per thread");
-    __shared__ float As[2][BK * LDA];
-    __shared__ float Bs[2][BK * LDB];
+    static_assert(GSZ * TPT == NB && NA % 2 == 0 && NB % 2 == 0, "TPT must divide the loads per thread");
+    constexpr int PA = BM + 4, PB = BN + 4, BOFF = SL * 6 * PA * 4, STAGE = BOFF + SL * 6 * PB * 4;   // as GatherLds
+    extern __shared__ __attribute__((aligned(16))) float lds[];
 
     unsigned L;
     const unsigned tiles = (unsigned)(p.mtiles * p.ntiles);
@@ -1298,20 +1306,16 @@ __global__ __launch_bounds__(T::THREADS, T::THREADS / 128) void conv_wgrad_k(Fil
     const int slab_begin = split * p.slabs_per_split;
     const int slab_end = min(slab_begin + p.slabs_per_split, p.slabs_total);
 
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, kh = lane >> 5, l32 = lane & 31;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = w / T::WN, wn = w % T::WN;
-    const int kl = tid & 15, r0 = tid >> 4;  // reduction row inside the slab; first tile row/column
+    // this lane's pixel of the stage, and its first tile row / column (others are multiples of 16 further on)
+    const int px = 2 * (lane & 15) + kh, r0 = 2 * w + ((lane >> 4) & 1);
     const int PQ = p.P * p.Q, HW = p.H * p.W;
 
     const __amdgpu_buffer_rsrc_t rdy = make_rsrc(p.dy, p.dy_bytes);
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x, p.x_bytes);
-
-    // rows (output channels) at or past K are masked
-    unsigned row_oob = 0;
-#pragma unroll
-    for (int i = 0; i < NA; i++)
-        if (m0 + r0 + 16 * i >= p.K) row_oob |= 1u << i;
-    const bool k_full = m0 + BM <= p.K;  // wave-uniform: every row of this tile exists
+    // (rows past K and columns past C are read as they lie, or as zeros past the tensor: their sums are not used)
 
     // wave-uniform description of each tap group of this tile
     int g_dr[TPT], g_ds[TPT], g_disp[TPT], g_c0[TPT];
@@ -1331,73 +1335,132 @@ __global__ __launch_bounds__(T::THREADS, T::THREADS / 128) void conv_wgrad_k(Fil
         }
         g_disp[g] = g_dr[g] * p.W + g_ds[g];
     }
-    const bool c_full = p.C == p.Cp;
 
     float areg[NA], breg[NB];
-    auto load = [&](int slab) {
-        const int kk = slab * BK + kl;
-        const int oob_pix = (p.npix - 1 - kk);  // negative past the last pixel
+    int slab;                       // first slab of the stage that is loaded next
+    int ih0, iw0, x_pix, oob_pix;   // of that stage's pixel
+    auto load_a = [&]() {           // and where the pixel lies
+        const int kk = slab * BK + px;
+        oob_pix = min(p.npix, slab_end * BK) - 1 - kk;  // negative past the last pixel
         const int n = kk / PQ, pq = kk - n * PQ;
         const int ph = pq / p.Q, qw = pq - ph * p.Q;
-        const unsigned a_raw = (unsigned)((n * p.K + m0 + r0) * PQ + pq) * 4u;
-        const unsigned a_voff = oob_pix < 0 ? kOobOffset : a_raw;
+        const unsigned voff = oob_pix < 0 ? kOobOffset : (unsigned)((n * p.K + m0 + r0) * PQ + pq) * 4u;
 #pragma unroll
-        for (int i = 0; i < NA; i++) {
-            unsigned v = a_voff;
-            if (!k_full) v = ((row_oob >> i) & 1u) ? kOobOffset : a_voff;
-            areg[i] = buffer_load_f32(rdy, v, (unsigned)(16 * i * PQ) * 4u);
-        }
-        const int ih0 = ph * p.strideH, iw0 = qw * p.strideW;
-        const int x_pix = (n * p.C + r0) * HW + ih0 * p.W + iw0;  // element offset of (n, channel r0, ih0, iw0)
+        for (int i = 0; i < NA; i++) areg[i] = buffer_load_f32(rdy, voff, (unsigned)(16 * i * PQ) * 4u);
+        ih0 = ph * p.strideH;
+        iw0 = qw * p.strideW;
+        x_pix = (n * p.C + r0) * HW + ih0 * p.W + iw0;  // element offset of (n, channel r0, ih0, iw0)
+        slab += SL;
+    };
+    auto load_b = [&]() {
 #pragma unroll
         for (int g = 0; g < TPT; g++) {
             const int ih = ih0 + g_dr[g], iw = iw0 + g_ds[g];
             const int bad = ih | (p.H - 1 - ih) | iw | (p.W - 1 - iw) | oob_pix;  // sign bit: outside
-            const unsigned g_voff = bad < 0 ? kOobOffset : (unsigned)(x_pix + g_disp[g]) * 4u;
+            const unsigned voff = bad < 0 ? kOobOffset : (unsigned)(x_pix + g_disp[g]) * 4u;
 #pragma unroll
-            for (int ii = 0; ii < GSZ; ii++) {
-                const int c_uni = g_c0[g] + 16 * ii;  // wave-uniform first channel of this load
-                unsigned v = g_voff;
-                if (!c_full) v = (c_uni + r0 < p.C) ? g_voff : kOobOffset;
-                breg[g * GSZ + ii] = buffer_load_f32(rx, v, (unsigned)(c_uni * HW) * 4u);
-            }
+            for (int ii = 0; ii < GSZ; ii++)
+                breg[g * GSZ + ii] = buffer_load_f32(rx, voff, (unsigned)((g_c0[g] + 16 * ii) * HW) * 4u);
         }
     };
-    auto store = [&](int buf, float up) {
+    // rows (or columns) r0 + 32 e and r0 + 32 e + 16: after the swap lanes 0 .. 31 hold both pixels of the first, the others of the second
+    const int half = (lane & 15) / 4;   // eight pixels: slab half / 2, half of the slab half % 2
+    const int w_lds = half / 2 * 6, w_half = half % 2, w_row = r0 + 16 * kh, w_word = lane & 3;
+    auto store = [&](float v0, float v1, int e, float *operand, int pitch) {
+        const auto both = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v0 * kSplitUp), __builtin_bit_cast(unsigned, v1 * kSplitUp), false, false);
+        unsigned q[3];
+        const unsigned even = both[0], odd = both[1];   // (a bit cast of a vector's element takes its first one)
+        split_pair(__builtin_bit_cast(float, even), __builtin_bit_cast(float, odd), q[0], q[1], q[2]);
 #pragma unroll
-        for (int i = 0; i < NA; i++) As[buf][kl * LDA + r0 + 16 * i] = areg[i] * up;
-#pragma unroll
-        for (int i = 0; i < NB; i++) Bs[buf][kl * LDB + r0 + 16 * i] = breg[i] * up;
+        for (int t = 0; t < 3; t++) ((unsigned *)operand)[((w_lds + t * 2 + w_half) * pitch + w_row + 32 * e) * 4 + w_word] = q[t];
+    };
+    auto store_pair = [&](float *buf, int e) {   // pair e of A's and then of B's
+        if (e < NA / 2) store(areg[2 * e], areg[2 * e + 1], e, buf, PA);
+        else store(breg[2 * e - NA], breg[2 * e - NA + 1], e - NA / 2, buf + BOFF, PB);
     };
 
-    v16f acc[T::MI][T::NI];
-    auto run = [&](auto exact_tag) {
-        constexpr bool exact = decltype(exact_tag)::value != 0;
-        constexpr float up = exact ? 1.0f : kSplitUp;
-        v16f low[T::MI][T::NI];
-        zero_acc(acc);
-        zero_acc(low);
-        auto slab_products = [&](int buf) {
-            if constexpr (exact) mma_slab<BK, LDA, LDB>(As[buf], Bs[buf], wm * (BM / T::WM), wn * (BN / T::WN), acc, lane);
-            else mma_slab_split<LDA, LDB>(As[buf], Bs[buf], wm * (BM / T::WM), wn * (BN / T::WN), acc, low, lane);
-        };
-        load(slab_begin);
-        store(0, up);
-        __syncthreads();
-        int cur = 0;
-        for (int slab = slab_begin; slab < slab_end - 1; ++slab) {
-            load(slab + 1);
-            slab_products(cur);
-            store(cur ^ 1, up);
-            __syncthreads();
-            cur ^= 1;
+    v16f acc[MI][NI], low[MI][NI];
+    zero_acc(acc);
+    zero_acc(low);
+    const int a_frag = (kh * PA + wm * (BM / T::WM) + l32) * 4, b_frag = BOFF + (kh * PB + wn * (BN / T::WN) + l32) * 4;
+    v4u a[2][MI][3], b[2][NI][3];
+    auto fragments = [&](const float *buf, int sl) {
+#pragma unroll
+        for (int t = 0; t < 3; t++) {
+#pragma unroll
+            for (int i = 0; i < MI; i++) a[sl][i][t] = *(const v4u *)(buf + a_frag + ((sl * 6 + t * 2) * PA + 32 * i) * 4);
+#pragma unroll
+            for (int j = 0; j < NI; j++) b[sl][j][t] = *(const v4u *)(buf + b_frag + ((sl * 6 + t * 2) * PB + 32 * j) * 4);
         }
-        slab_products(cur);
-        if constexpr (!exact) add_acc(acc, low);
     };
-    run(StepTag<0>{});
-    // the parts of an infinity hold NaNs: a tile that is not finite is formed again with the fp32 instruction
-    if (__syncthreads_or(not_finite(acc))) run(StepTag<1>{});
+    constexpr int PAIRS = (NA + NB) / 2;
+    static_assert(PAIRS <= 10, "a pair per step, the loads behind them");
+    slab = slab_begin;
+    load_a();
+    load_b();
+#pragma unroll
+    for (int e = 0; e < PAIRS; e++) store_pair(lds, e);
+    const int stages = (slab_end - slab_begin + SL - 1) / SL;
+    if (stages > 1) {
+        load_a();
+        load_b();
+    }
+    __syncthreads();
+    auto stage = [&](const float *cur, float *nxt, auto more_tag) {
+        constexpr bool more = decltype(more_tag)::value != 0;
+        fragments(cur, 0);
+        static_for<0, 6 * SL>([&](auto tag) {
+            constexpr int step = decltype(tag)::value, sl = step / 6, s = step % 6;
+            if constexpr (step == 0) fragments(cur, 1);
+            if constexpr (more && step < PAIRS) store_pair(nxt, step);
+            if constexpr (more && step == NA / 2) load_a();   // (the registers' last values have just been stored)
+            if constexpr (more && step == PAIRS) load_b();
+            // smallest products first: l.h, h.l, m.m, m.h, h.m, h.h
+            constexpr int qa = s == 0 ? 2 : s == 2 || s == 3 ? 1 : 0, qb = s == 1 ? 2 : s == 2 || s == 4 ? 1 : 0;
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int j = 0; j < NI; j++) {
+                    v16f &c = s < 5 ? low[i][j] : acc[i][j];
+                    c = mfma_bf16(a[sl][i][qa], b[sl][j][qb], c);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        if constexpr (more) __syncthreads();
+    };
+    for (int st = 0; st < stages - 1; ++st) stage(lds + (st & 1) * STAGE, lds + (~st & 1) * STAGE, StepTag<1>{});
+    stage(lds + ((stages - 1) & 1) * STAGE, nullptr, StepTag<0>{});
+    add_acc(acc, low);
+
+    // the parts of an infinity hold NaNs: a tile that is not finite is formed again with the fp32 instruction, a stage at a time
+    if (__syncthreads_or(not_finite(acc))) {
+        zero_acc(acc);
+        slab = slab_begin;
+#pragma unroll 1
+        for (int st = 0; st < stages; ++st) {
+            load_a();
+            load_b();
+            __syncthreads();
+            // here [slab][half][row][8 pixels]
+            const int at = px / 16 * 2 + px / 8 % 2;
+#pragma unroll
+            for (int i = 0; i < NA; i++) lds[(at * PA + r0 + 16 * i) * 8 + px % 8] = areg[i];
+#pragma unroll
+            for (int i = 0; i < NB; i++) lds[BOFF + (at * PB + r0 + 16 * i) * 8 + px % 8] = breg[i];
+            __syncthreads();
+#pragma unroll 1
+            for (int sl = 0; sl < SL; sl++)
+#pragma unroll 1
+                for (int e = 0; e < 8; e++)
+#pragma unroll
+                    for (int i = 0; i < MI; i++)
+#pragma unroll
+                        for (int j = 0; j < NI; j++)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(lds[((sl * 2 + kh) * PA + wm * (BM / T::WM) + l32 + 32 * i) * 8 + e],
+                                                                              lds[BOFF + ((sl * 2 + kh) * PB + wn * (BN / T::WN) + l32 + 32 * j) * 8 + e],
+                                                                              acc[i][j], 0, 0, 0);
+        }
+    }
 
     float *outp = p.out + (size_t)split * p.out_elems;
 #pragma unroll
@@ -2323,7 +2386,7 @@ int patch_splits(int tiles, int chunks, int slots, int BM, int BN, size_t out_el
 }
 
 // The same estimate for the general kernels, whose unit is a slab of 16 reduction steps, at the rate that one CU sustains.
-constexpr double kGatherRate = 0.6, kWgradRate = 0.33;
+constexpr double kGatherRate = 0.6;
 int gather_splits(int tiles, int slabs, int slots, int BM, int BN, size_t out_elems, double cu_tflops, int cap)
 {
     const double per_cu = (double)slots / num_cus();
@@ -3050,6 +3113,20 @@ int launch_wgrad_patch(const WgradPatch &wp, dim3 grid, size_t lds_bytes)
     return DOPT_HIP_OK;
 }
 
+template <class T, int TPT>
+int launch_wgrad(const FilterGrad &f, dim3 grid)
+{
+    constexpr size_t lds = (size_t)2 * 2 * 6 * (T::BM + 4 + T::BN + 4) * 16;
+    static bool raised = false;
+    if (!raised) {   // above 64 KB of dynamic LDS a kernel has to be told once
+        DOPT_HIP_CHECK(hipFuncSetAttribute((const void *)conv_wgrad_k<T, TPT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        raised = true;
+    }
+    hipLaunchKernelGGL((conv_wgrad_k<T, TPT>), grid, dim3(T::THREADS), lds, stream(), f);
+    DOPT_LAUNCH_CHECK();
+    return DOPT_HIP_OK;
+}
+
 int launch_wgrad_reduce(int K, int C, int Cp, int taps, int splits, size_t out_elems, const float *partial, float *dw)
 {
     // 64-channel chunks when that still leaves >= 1024 workgroups and the LDS staging stays small
@@ -3328,8 +3405,8 @@ int run_bwd_pair(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float *d
     return DOPT_HIP_OK;
 }
 
-using WgradSquare = Tile<128, 128, 2, 2>;
-using WgradNarrow = Tile<64, 128, 1, 4>;  // K <= 64
+using WgradSquare = Tile<128, 128, 4, 2>;
+using WgradNarrow = Tile<64, 128, 2, 4>;  // K <= 64: two workgroups per CU
 
 }  // namespace
 
@@ -3620,7 +3697,7 @@ int dopt_hip_conv_bwd_filter(const dopt_hip_conv_desc *d, const float *dy, const
     f.ntiles = (f.ncols + BN - 1) / BN;
     const int tiles = f.mtiles * f.ntiles;
     // filter gradients are short and wide (small output, long pixel reduction): allow deep splits
-    int splits = gather_splits(tiles, f.slabs_total, 2 * num_cus(), BM, BN, f.out_elems, kWgradRate, 512);
+    int splits = gather_splits(tiles, f.slabs_total, big ? num_cus() : 2 * num_cus(), BM, BN, f.out_elems, kGatherRate, 512);
     f.slabs_per_split = (f.slabs_total + splits - 1) / splits;
     splits = (f.slabs_total + f.slabs_per_split - 1) / f.slabs_per_split;
     f.splits = splits;
@@ -3632,20 +3709,11 @@ int dopt_hip_conv_bwd_filter(const dopt_hip_conv_desc *d, const float *dy, const
     while (f.Cp % gw != 0) gw /= 2;  // largest power-of-two divisor of Cp not above BN (>= 16)
     const int tpt = BN / gw;         // 1, 2, 4 or 8
     dim3 grid(xcd_grid((unsigned)(tiles * splits)));
-#define DOPT_WGRAD(TILE, TPTV) hipLaunchKernelGGL((conv_wgrad_k<TILE, TPTV>), grid, dim3(TILE::THREADS), 0, stream(), f)
-    if (big) {
-        if (tpt == 1) DOPT_WGRAD(WgradSquare, 1);
-        else if (tpt == 2) DOPT_WGRAD(WgradSquare, 2);
-        else if (tpt == 4) DOPT_WGRAD(WgradSquare, 4);
-        else DOPT_WGRAD(WgradSquare, 8);
-    } else {
-        if (tpt == 1) DOPT_WGRAD(WgradNarrow, 1);
-        else if (tpt == 2) DOPT_WGRAD(WgradNarrow, 2);
-        else if (tpt == 4) DOPT_WGRAD(WgradNarrow, 4);
-        else DOPT_WGRAD(WgradNarrow, 8);
-    }
-#undef DOPT_WGRAD
-    DOPT_LAUNCH_CHECK();
+    auto run = [&](auto tile_tag) {
+        using T = decltype(tile_tag);
+        return tpt == 1 ? launch_wgrad<T, 1>(f, grid) : tpt == 2 ? launch_wgrad<T, 2>(f, grid) : tpt == 4 ? launch_wgrad<T, 4>(f, grid) : launch_wgrad<T, 8>(f, grid);
+    };
+    if (int rc = big ? run(WgradSquare{}) : run(WgradNarrow{})) return rc;
     return launch_wgrad_reduce(f.K, f.C, f.Cp, taps, splits, f.out_elems, partial, dw);
 }
 

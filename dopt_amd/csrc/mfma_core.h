@@ -145,7 +145,7 @@ __device__ __forceinline__ v16f mfma_bf16(v4u a, v4u b, v16f c)
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
 }
 
-// The finished sums of mma_slab_split.
+// The finished sums: of the h.h products and of the five small ones.
 template <int MI, int NI>
 __device__ __forceinline__ void add_acc(v16f (&acc)[MI][NI], const v16f (&low)[MI][NI])
 {
@@ -169,42 +169,6 @@ __device__ __forceinline__ int not_finite(const v16f (&acc)[MI][NI])
 #pragma unroll
             for (int v = 0; v < 16; v++) probe = __builtin_fmaf(acc[i][j][v], 0.0f, probe);
     return probe != 0.0f;
-}
-
-// mma_slab on the bf16 matrix instruction: from the same k-major fp32 slab of sixteen steps a lane reads its eight steps of
-// each fragment (multiplied by kSplitUp) and splits them in registers.  h.h goes to acc, the five small products to low.
-template <int LDA, int LDB, int MI, int NI>
-__device__ __forceinline__ void mma_slab_split(const float *As, const float *Bs, int a_off, int b_off, v16f (&acc)[MI][NI],
-                                               v16f (&low)[MI][NI], int lane)
-{
-    const int kh = lane >> 5, l32 = lane & 31;
-    auto fragment = [](const float *s, int pitch, v4u (&f)[3]) {
-        float v[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) v[e] = s[e * pitch];
-        unsigned q[3][4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) split_pair(v[2 * e], v[2 * e + 1], q[0][e], q[1][e], q[2][e]);
-#pragma unroll
-        for (int t = 0; t < 3; t++) f[t] = v4u{q[t][0], q[t][1], q[t][2], q[t][3]};
-    };
-    v4u a[MI][3], b[NI][3];
-#pragma unroll
-    for (int i = 0; i < MI; i++) fragment(As + kh * 8 * LDA + a_off + 32 * i + l32, LDA, a[i]);
-#pragma unroll
-    for (int j = 0; j < NI; j++) fragment(Bs + kh * 8 * LDB + b_off + 32 * j + l32, LDB, b[j]);
-    // smallest products first: l.h, h.l, m.m, m.h, h.m, h.h
-    static_for<0, 6>([&](auto tag) {
-        constexpr int s = decltype(tag)::value;
-        constexpr int qa = s == 0 ? 2 : s == 2 || s == 3 ? 1 : 0, qb = s == 1 ? 2 : s == 2 || s == 4 ? 1 : 0;
-#pragma unroll
-        for (int i = 0; i < MI; i++)
-#pragma unroll
-            for (int j = 0; j < NI; j++) {
-                v16f &c = s < 5 ? low[i][j] : acc[i][j];
-                c = mfma_bf16(a[i][qa], b[j][qb], c);
-            }
-    });
 }
 
 // Row of accumulator register v of a 32x32 tile for this lane; the column is lane % 32.
