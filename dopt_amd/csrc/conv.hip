@@ -3332,11 +3332,12 @@ int run_bwd_pair(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float *d
     WgradSetup b = wgrad_patch_setup(d, dw);
     if (!a.ok || !b.ok || !prepacked || a.pc.Cin % 16 != 0) return DOPT_HIP_OK;
     // The combinations that are built: 128 x 128 backward-data tiles on eight wavefronts, one workgroup per CU
-    // (the 64 x 256 tiles of layers with up to 64 input channels run two 256-thread workgroups per CU, which a
-    // launch shaped for the filter gradient's 768 threads cannot hold), with 128 x 32 filter-gradient tiles on
+    // (the 64 x 256 and 32 x 256 tiles of layers with up to 64 input channels are not built), with 128 x 32 filter-gradient tiles on
     // rows of 8 .. 64 pixels or on 4 x 4 images.
     // (a layer the Winograd kernel takes has its filter packed for that kernel: shape 4, not a pair)
-    const int combo = a.shape == 2 && b.tall && b.geo == 0 ? 0 : a.shape == 2 && b.tall && b.geo == 1 ? 1 : -1;
+    // (only where the launch needs it: with two rounds of backward-data tiles and more the two run one after the other)
+    const bool few = a.shape == 2 && a.tiles < 2 * num_cus();
+    const int combo = few && b.tall && b.geo == 0 ? 0 : few && b.tall && b.geo == 1 ? 1 : -1;
     // A layer whose backward-data is the Winograd kernel on 128-row tiles: two launches, each as it would run alone, but out of ONE
     // workspace request, so that both results can stay open for the launch behind them - the filter gradient's split
     // sum rides in the batch-norm gradient there instead of being a launch of its own.  (The same for the 64-row layers
