@@ -1023,12 +1023,14 @@ void HIPPlan::Builder::formGroups()
             if (g.ops[d].volume() != o.volume()) return false;
         return true;
     };
+    // whether a use reads all of the value: a view of its first element or rows starts at offset 0 as well
+    auto whole = [&](const Use &u, int id) { return u.off == 0 && g.ops[g.ops[u.op].deps[(size_t)u.slot]].volume() == g.ops[id].volume(); };
     std::vector<char> last((size_t)nops, 0);   // operations that may run after everything else
     for (auto it = p->mOps.rbegin(); it != p->mOps.rend(); ++it) {
         const int id = *it;
         if (!is_node(id)) continue;
         bool ok = isOutput(id) || !uses[id].empty();
-        for (const Use &u : uses[id]) ok = ok && last[u.op] && u.off == 0 && g.ops[u.op].volume() == g.ops[id].volume();
+        for (const Use &u : uses[id]) ok = ok && last[u.op] && whole(u, id) && g.ops[u.op].volume() == g.ops[id].volume();
         last[id] = ok;
     }
     // one-element values that pieces compute for themselves: all that reads one is a piece, as the element it scales or

@@ -245,7 +245,8 @@ def test_update_rules_of_many_tensors_as_one_step(sizes, offset):
 
 
 def test_values_that_something_else_reads_stay_out_of_a_group():
-    """A reduction, a narrower view and a value broadcast from one element of a tensor end what may run last."""
+    """A reduction and a narrower view end what may run last; a one-element value that leaves the plan is an operand.  (A value
+    scaled by one of its own elements: below.)"""
     r = np.random.default_rng(9)
     a, b = (core.float32([300], r.standard_normal(300).astype(np.float32)) for _ in range(2))
     s = a * b
@@ -256,6 +257,31 @@ def test_values_that_something_else_reads_stay_out_of_a_group():
     got = core.compile(outs, core.PLAN_VIEWS | core.PLAN_FUSE).execute()
     for g, w in zip(got, want):
         assert np.array_equal(g, w)
+
+
+@pytest.mark.parametrize("tensors", [1, 3])
+def test_a_tensor_scaled_by_its_own_first_element(tensors):
+    """A view of a value's first element starts where the value does, and a view of its first rows too: what reads one does not
+    read the whole.  As a product with [1, 1] from either side, through the scalar broadcast and through `repeat`; 5000 elements
+    are no run of tiny operations."""
+    r = np.random.default_rng(11)
+    n, outs = 5000, []
+    first = lambda v: core.slice(v, [0], [1])
+    forms = [lambda v: core.matmul(core.reshape(v, [n, 1]), core.reshape(first(v), [1, 1])), lambda v: v * core.reshape(first(v), []),
+             lambda v: v - core.repeat(first(v), [n]), lambda v: core.matmul(core.reshape(first(v), [1, 1]), core.reshape(v, [1, n]))]
+    for _ in range(tensors):
+        a, b = (core.float32([n], r.standard_normal(n).astype(np.float32)) for _ in range(2))
+        for k, form in enumerate(forms):
+            y, z = a * b + (0.5 + k), a - b * (0.5 + k)   # values of their own for each form
+            outs += [y, z, form(y), core.sum(form(z))]
+    want = core.compile(outs).execute()
+    for flags in (core.PLAN_VIEWS | core.PLAN_FUSE, core.PLAN_VIEWS | core.PLAN_FUSE | core.PLAN_GRAPH):
+        plan = core.compile(outs, flags)
+        bufs = [ops.Tensor(o.shape) for o in outs]
+        for _ in range(3):
+            plan.execute(None, bufs)
+            for k, (got, w) in enumerate(zip(bufs, want)):
+                assert np.array_equal(got.numpy(), w), (flags, k)
 
 
 def test_penalties_of_many_tensors_as_one_step():
