@@ -1516,8 +1516,11 @@ void HIPPlan::Builder::formChains()
         if (!is_pw(id)) continue;
         int target = -1;
         bool joins = !isOutput(id) && !uses[id].empty() && !groupReads[id];
-        auto reader_joins = [&](const Use &u, size_t volume) {   // the reader is a member of the one chain, and reads all of it
-            if (chainOf[u.op] < 0 || u.off != 0 || g.ops[u.op].volume() != volume) joins = false;
+        // the reader is a member of the one chain, has `volume` elements and reads `part` of the value: all of it, not a view of its
+        // first element or rows, which starts at offset 0 as well
+        auto reader_joins = [&](const Use &u, size_t volume, size_t part) {
+            if (chainOf[u.op] < 0 || u.off != 0 || g.ops[u.op].volume() != volume || g.ops[g.ops[u.op].deps[(size_t)u.slot]].volume() != part)
+                joins = false;
             else if (g.ops[u.op].opType == "reluGrad" && u.slot == 1) joins = false;   // the y operand is not part of the node
             else if (target < 0) target = chainOf[u.op];
             else if (target != chainOf[u.op]) joins = false;
@@ -1532,7 +1535,7 @@ void HIPPlan::Builder::formChains()
                 ro.volume() > 1 && alias[u.op].source < 0 && !isOutput(u.op) && live[u.op] && !fusedKind[u.op] && !uses[u.op].empty()) {
                 for (const Use &u2 : uses[u.op]) {
                     if (!joins) break;
-                    reader_joins(u2, ro.volume());
+                    reader_joins(u2, ro.volume(), ro.volume());
                 }
                 continue;
             }
@@ -1540,10 +1543,10 @@ void HIPPlan::Builder::formChains()
             // [1,1] x [1,n], core/ops/basic.d:370-381): the member reads the value as its one-element operand
             if (g.ops[id].volume() == 1 && ro.volume() > 1 && outer_cols(u.op) && chainOf[u.op] >= 0 && u.off == 0 &&
                 ((u.slot == 1 && ro.shape[1] == 1) || (u.slot == 0 && ro.shape[0] == 1))) {
-                reader_joins(u, ro.volume());
+                reader_joins(u, ro.volume(), 1);
                 continue;
             }
-            reader_joins(u, g.ops[id].volume());
+            reader_joins(u, g.ops[id].volume(), g.ops[id].volume());
         }
         if (joins && chainOps[target].size() >= 48) joins = false;
         const size_t cols = outer_grid(id);

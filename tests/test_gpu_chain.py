@@ -260,7 +260,8 @@ def test_values_that_something_else_reads_stay_out_of_a_group():
 
 
 @pytest.mark.parametrize("tensors", [1, 3])
-def test_a_tensor_scaled_by_its_own_first_element(tensors):
+@pytest.mark.parametrize("read_on", [True, False], ids=["an output as well", "only read by its product"])
+def test_a_tensor_scaled_by_its_own_first_element(tensors, read_on):
     """A view of a value's first element starts where the value does, and a view of its first rows too: what reads one does not
     read the whole.  As a product with [1, 1] from either side, through the scalar broadcast and through `repeat`; 5000 elements
     are no run of tiny operations."""
@@ -273,7 +274,10 @@ def test_a_tensor_scaled_by_its_own_first_element(tensors):
         a, b = (core.float32([n], r.standard_normal(n).astype(np.float32)) for _ in range(2))
         for k, form in enumerate(forms):
             y, z = a * b + (0.5 + k), a - b * (0.5 + k)   # values of their own for each form
-            outs += [y, z, form(y), core.sum(form(z))]
+            outs += ([y, z] if read_on else []) + [form(y), core.sum(form(z))]
+        if not read_on:
+            column, row = a * b, core.float32([1, 100], r.standard_normal(100).astype(np.float32))
+            outs.append(core.matmul(core.reshape(core.slice(column, [0], [50]), [50, 1]), row) + core.reshape(column, [50, 100]))
     want = core.compile(outs).execute()
     for flags in (core.PLAN_VIEWS | core.PLAN_FUSE, core.PLAN_VIEWS | core.PLAN_FUSE | core.PLAN_GRAPH):
         plan = core.compile(outs, flags)
