@@ -615,7 +615,8 @@ __device__ __forceinline__ void conv_patch_body(const PatchConv &p, const unsign
     add_acc(acc, low);
 
     // the parts of an infinity hold NaNs: a tile that is not finite is formed again with the fp32 instruction, one chunk after the
-    // other (a word per wavefront: in a backward pair the workgroup's surplus wavefronts have ended)
+    // other, for its values that are not finite (a word per wavefront: in a backward pair the workgroup's surplus wavefronts have
+    // ended)
     __syncthreads();
     {
         const int mine = __any(not_finite(acc));
@@ -625,7 +626,7 @@ __device__ __forceinline__ void conv_patch_body(const PatchConv &p, const unsign
 #pragma unroll
         for (int i = 0; i < THREADS / 64; i++) bad |= ((const int *)lds)[i];
         if (bad) {
-            zero_acc(acc);
+            zero_acc(low);
 #pragma unroll 1
             for (int chunk = cb; chunk < ce; chunk++) {
                 __syncthreads();
@@ -655,10 +656,11 @@ __device__ __forceinline__ void conv_patch_body(const PatchConv &p, const unsign
                         for (int e = 0; e < 8; e++) {
                             const float a = packed_value(fa_ring[0][i], e);
 #pragma unroll
-                            for (int j = 0; j < NI; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b8[j][e], acc[i][j], 0, 0, 0);
+                            for (int j = 0; j < NI; j++) low[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b8[j][e], low[i][j], 0, 0, 0);
                         }
                 }
             }
+            keep_finite(acc, low);
         }
     }
 

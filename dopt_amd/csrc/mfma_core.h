@@ -171,6 +171,19 @@ __device__ __forceinline__ int not_finite(const v16f (&acc)[MI][NI])
     return probe != 0.0f;
 }
 
+// The sums of a tile that was formed twice: the first time's where they are finite, so that a finite value does not depend on
+// what else lies in its tile.
+template <int MI, int NI>
+__device__ __forceinline__ void keep_finite(v16f (&acc)[MI][NI], const v16f (&again)[MI][NI])
+{
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+        for (int j = 0; j < NI; j++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[i][j][v] = acc[i][j][v] * 0.0f == 0.0f ? acc[i][j][v] : again[i][j][v];
+}
+
 // Row of accumulator register v of a 32x32 tile for this lane; the column is lane % 32.
 __device__ inline int acc_row(int v, int lane) { return 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3); }
 

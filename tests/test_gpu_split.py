@@ -566,6 +566,25 @@ def test_direct_convolution_operands_that_are_not_finite(shape):
     assert np.all(np.abs(got[fine] - want[fine]) <= walk(C * 9) * want[fine])
 
 
+# a tile of every height with whole and ragged channels, and one reduction that is cut
+@pytest.mark.parametrize("shape", [(2, 20, 16, 16, 17), (2, 16, 16, 16, 32), (2, 20, 16, 16, 48), (4, 72, 8, 8, 100), (4, 200, 8, 8, 100),
+                                   (33, 17, 32, 32, 160)])
+def test_direct_convolution_finite_values_keep_their_bits_beside_others(shape):
+    N, C, H, W, K = shape
+    r = rng(K)
+    x, w, dy = (np.abs(r.standard_normal(s)).astype(np.float32) + np.float32(0.1) for s in ((N, C, H, W), (K, C, 3, 3), (N, K, H, W)))
+    both = lambda: (ops.convolution(T(x), T(w), (1, 1), (1, 1)).numpy(), ops.conv_bwd_data(T(dy), T(w), x.shape, (1, 1), (1, 1)).numpy())
+    plain = both()
+    x[0, 3, 0, 0], x[N - 1, C - 1, H - 1, 2], dy[0, 1, 3, 3], dy[1, K - 1, 3, 2] = np.inf, np.nan, np.inf, np.nan
+    for got, want in zip(both(), plain):
+        fine = np.isfinite(got)
+        assert 0.8 < fine.mean() < 1.0 and np.array_equal(got[fine], want[fine])
+    w[K - 1, 2, 1, 1], w[1, C - 1, 0, 2] = np.inf, np.nan
+    for got, want in zip(both(), plain):
+        fine = np.isfinite(got)
+        assert 0.7 < fine.mean() < 1.0 and np.array_equal(got[fine], want[fine])
+
+
 @pytest.mark.parametrize("shape", [(2, 20, 16, 16, 17), (2, 20, 16, 16, 48), (2, 40, 8, 8, 100)])
 def test_direct_convolution_operands_at_the_ends_of_the_range(shape):
     N, C, H, W, K = shape
