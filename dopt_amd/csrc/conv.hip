@@ -145,7 +145,7 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
     }
 
     // B: the output pixel this thread gathers for, CPT channels of a slab from c0 on
-    const int bcol = tid % BN, c0 = tid / BN * CPT;
+    const int bcol = tid % BN, c0 = w * 64 / BN * CPT;
     const int pix = n0 + bcol;
     const int pix_oob = p.ncols - 1 - pix;  // negative past the last pixel
     const int OHW = p.OH * p.OW;
@@ -210,8 +210,12 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
         }
     };
     // Channels past the last one are read as they lie (another image's, or zeros past the tensor): their filter values are zeros.
-    // Only the fp32 pass, which a product of such a zero with an infinity leads to, has to leave them out.
-    auto load_b = [&](int sl, int i, unsigned voff) { breg[sl][i] = buffer_load_f32(rin, voff, (unsigned)((ci0 + i) * chan_stride) * 4u); };
+    // Where that makes a NaN of an infinity the sums are formed again without them: masked.  (Left out at once, by a select per
+    // load, they cost 6 % of the 5 x 5 layers' time; by one per load of the last sixteen channels 3 %.)
+    auto load_b = [&](int sl, int i, unsigned voff, auto masked_tag) {
+        if (decltype(masked_tag)::value) voff = ci0 + i < row_limit ? voff : kOobOffset;
+        breg[sl][i] = buffer_load_f32(rin, voff, (unsigned)((ci0 + i) * chan_stride) * 4u);
+    };
     auto store_a = [&](float *buf) {
 #pragma unroll
         for (int i = 0; i < NA; i++)
@@ -232,8 +236,6 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
     };
 
     v16f acc[MI][NI], low[MI][NI];
-    zero_acc(acc);
-    zero_acc(low);
     const int a_frag = (kh * PA + wm * (BM / T::WM) + l32) * 4, b_frag = BOFF + (kh * PB + wn * (BN / T::WN) + l32) * 4;
     v4u a[2][MI][3], b[2][NI][3];
     auto fragments = [&](const float *buf, int sl) {
@@ -248,7 +250,7 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
     // Under the matrix instructions of a stage the next one, which is in registers, is split and stored, and the one after
     // it is loaded: a slab's values as soon as the slab before in those registers is stored.
     // The last stage has only its products: with few slabs a block would wait for loads of nothing.
-    auto stage = [&](const float *cur, float *nxt, auto more_tag) {
+    auto stage = [&](const float *cur, float *nxt, auto more_tag, auto masked_tag) {
         constexpr bool more = decltype(more_tag)::value != 0;
         fragments(cur, 0);
         unsigned voff = 0;
@@ -268,7 +270,7 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
                 }
                 if constexpr (more && s == PAIRS + 1) {
 #pragma unroll
-                    for (int i = 0; i < CPT; i++) load_b(sl, i, voff);
+                    for (int i = 0; i < CPT; i++) load_b(sl, i, voff, masked_tag);
                     next_slab();
                 }
                 // smallest products first: l.h, h.l, m.m, m.h, h.m, h.h
@@ -291,29 +293,40 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
         for (int sl = 0; sl < SL; sl++) {
             const unsigned voff = pixel();
 #pragma unroll
-            for (int i = 0; i < CPT; i++) load_b(sl, i, decltype(masked_tag)::value && ci0 + i >= row_limit ? kOobOffset : voff);
+            for (int i = 0; i < CPT; i++) load_b(sl, i, voff, masked_tag);
             next_slab();
         }
     };
-    rewind();
-    load_stage(StepTag<0>{});
-    store_a(lds);
-#pragma unroll
-    for (int sl = 0; sl < SL; sl++) {
-#pragma unroll
-        for (int e = 0; e < PAIRS; e++) split_b(sl, e);
-        store_b(lds, sl);
-    }
     const int stages = (slab_end - slab_begin + SL - 1) / SL;
-    if (stages > 1) load_stage(StepTag<0>{});
-    __syncthreads();
-    for (int st = 0; st < stages - 1; ++st) stage(lds + (st & 1) * STAGE, lds + (~st & 1) * STAGE, StepTag<1>{});
-    stage(lds + ((stages - 1) & 1) * STAGE, nullptr, StepTag<0>{});
-    add_acc(acc, low);
-
-    // the parts of an infinity hold NaNs: a tile that is not finite is formed again with the fp32 instruction, a stage at a time
-    if (__syncthreads_or(not_finite(acc))) {
+    auto sums = [&](auto masked_tag) {
         zero_acc(acc);
+        zero_acc(low);
+        rewind();
+        load_stage(masked_tag);
+        store_a(lds);
+#pragma unroll
+        for (int sl = 0; sl < SL; sl++) {
+#pragma unroll
+            for (int e = 0; e < PAIRS; e++) split_b(sl, e);
+            store_b(lds, sl);
+        }
+        if (stages > 1) load_stage(masked_tag);
+        __syncthreads();
+        for (int st = 0; st < stages - 1; ++st) stage(lds + (st & 1) * STAGE, lds + (~st & 1) * STAGE, StepTag<1>{}, masked_tag);
+        stage(lds + ((stages - 1) & 1) * STAGE, nullptr, StepTag<0>{}, masked_tag);
+        add_acc(acc, low);
+    };
+    sums(StepTag<0>{});
+    int again = __syncthreads_or(not_finite(acc));
+    if (again && p.CinPad != p.Cin) {
+        sums(StepTag<1>{});
+        again = __syncthreads_or(not_finite(acc));
+    }
+
+    // the parts of an infinity hold NaNs: a tile that is not finite is formed again with the fp32 instruction, a stage at a time,
+    // for its values that are not finite
+    if (again) {
+        zero_acc(low);
         rewind();
 #pragma unroll 1
         for (int st = 0; st < stages; ++st) {
@@ -342,10 +355,11 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
                         const float b8[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
 #pragma unroll
                         for (int e = 0; e < 8; e++)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(packed_value(f, e), b8[e], acc[i][j], 0, 0, 0);
+                            low[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(packed_value(f, e), b8[e], low[i][j], 0, 0, 0);
                     }
                 }
         }
+        keep_finite(acc, low);
     }
 
     float *outp = p.out + (size_t)split * p.out_elems;

@@ -476,6 +476,23 @@ def test_general_convolution_operands_that_are_not_finite():
         assert np.all(np.abs(got[fine] - want[fine]) <= walk(2500) * want[fine])   # (every term is positive)
 
 
+# channel counts off the slab, of x and of dy; images of one 256-pixel tile each, and several in a tile
+@pytest.mark.parametrize("shape", [(3, 17, 16, 16, 23, 5, 2, 1), (3, 33, 16, 16, 20, 1, 0, 1), (4, 40, 8, 8, 130, 5, 2, 1), (3, 17, 32, 32, 24, 3, 1, 2),
+                                   (2, 150, 7, 9, 70, 3, 0, 2)])
+def test_general_convolution_finite_values_keep_their_bits_beside_others(shape):
+    N, C, H, W, K, R, pad, stride = shape
+    r = rng(K)
+    x, w = (np.abs(r.standard_normal(s)).astype(np.float32) + np.float32(0.1) for s in ((N, C, H, W), (K, C, R, R)))
+    y = ops.convolution(T(x), T(w), (pad, pad), (stride, stride)).numpy()
+    dy = np.abs(r.standard_normal(y.shape)).astype(np.float32) + np.float32(0.1)
+    gradient = lambda: ops.conv_bwd_data(T(dy), T(w), x.shape, (pad, pad), (stride, stride)).numpy()
+    plain = y, gradient()
+    x[1, 0, 3, 3], x[N - 1, C - 1, 0, 0], dy[1, 0, 1, 1], dy[N - 1, K - 1, 0, 2] = np.inf, np.nan, np.nan, np.inf
+    for got, want in zip((ops.convolution(T(x), T(w), (pad, pad), (stride, stride)).numpy(), gradient()), plain):
+        fine = np.isfinite(got)
+        assert fine[0].all() and not fine.all() and np.array_equal(got[fine], want[fine])
+
+
 # ---- operands and sums at the ends of the range of fp32, where bf16 parts would be lost or overflow
 
 def scaled_pairs(p, q, least_q=-149):
