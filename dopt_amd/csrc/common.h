@@ -83,6 +83,8 @@ int nn_device_setup();
 // Number of compute units of the active device (256 on MI355X); used to size grids.
 int num_cus();
 
+// Workgroups of 256 threads that a launch of ours is given at most (a launch takes fewer than 2^32 threads along a dimension).
+constexpr size_t kLaunchBlocks = (size_t)1 << 22;
 inline size_t ceil_div(size_t a, size_t b) { return (a + b - 1) / b; }
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 

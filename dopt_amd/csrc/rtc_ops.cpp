@@ -6,6 +6,7 @@
 // :249-310 (argmin).
 #include <algorithm>
 #include <cstring>
+#include <deque>
 #include <string>
 #include <vector>
 
@@ -704,7 +705,9 @@ int pointwise_group(const PointwiseProgram &p, const std::vector<PointwiseItem> 
 {
     if (int rc = group_check(p)) return rc;
     const int nin = (int)p.kind.size();
+    constexpr size_t kPart = kLaunchBlocks * 1024;   // elements: a tensor of more goes part by part
     std::vector<const PointwiseItem *> todo;
+    std::deque<PointwiseItem> parts;
     for (const PointwiseItem &it : items) {
         DOPT_REQUIRE((int)it.in.size() == nin && it.out.size() == p.outs.size(), "pointwise_group: an item with %zu inputs and %zu results", it.in.size(),
                      it.out.size());
@@ -712,7 +715,19 @@ int pointwise_group(const PointwiseProgram &p, const std::vector<PointwiseItem> 
         for (const void *q : it.in) DOPT_REQUIRE(q != nullptr, "pointwise_group: null input");
         for (const void *q : it.out) DOPT_REQUIRE(q != nullptr, "pointwise_group: null result");
         DOPT_REQUIRE(it.n < (size_t)1 << 40, "pointwise_group: %zu elements", it.n);
-        todo.push_back(&it);
+        if (it.n <= kPart) {
+            todo.push_back(&it);
+            continue;
+        }
+        for (size_t from = 0; from < it.n; from += kPart) {
+            parts.push_back(it);
+            PointwiseItem &part = parts.back();
+            part.n = std::min(it.n - from, kPart);
+            for (int k = 0; k < nin; k++)
+                if (p.kind[k] == 0) part.in[k] = (const float *)it.in[k] + from;
+            for (void *&q : part.out) q = (float *)q + from;
+            todo.push_back(&part);
+        }
     }
     if (todo.empty()) return DOPT_HIP_OK;
     DOPT_ENSURE_INIT();
@@ -748,9 +763,8 @@ int pointwise_group(const PointwiseProgram &p, const std::vector<PointwiseItem> 
         for (int k = 0; k < nin; k++) quads = quads && (p.kind[k] == 1 || aligned16(it->in[k]));
         for (const void *q : it->out) quads = quads && aligned16(q);
         const size_t need = quads ? ceil_div(it->n / 4 + it->n % 4, 256) : ceil_div(it->n, 1024);
-        if (filled == g.items || blocks + need > 0x3fffffffu)
+        if (filled == g.items || blocks + need > kLaunchBlocks)
             if (int rc = flush()) return rc;
-        DOPT_REQUIRE(need <= 0x3fffffffu, "pointwise_group: %zu elements", it->n);
         char *ptrs = args.data() + (size_t)filled * g.nptr * 8;
         for (size_t i = 0; i < g.own.size(); i++) std::memcpy(ptrs + 8 * i, &it->in[(size_t)g.own[i]], 8);
         for (size_t o = 0; o < it->out.size(); o++) std::memcpy(ptrs + 8 * (g.own.size() + o), &it->out[o], 8);

@@ -288,6 +288,28 @@ def test_a_tensor_scaled_by_its_own_first_element(tensors, read_on):
                 assert np.array_equal(got.numpy(), w), (flags, k)
 
 
+# more workgroups than one launch can have, 2^24 of them; and a tensor of more elements than go into a launch
+@pytest.mark.parametrize("tensors, base, times", [(17, 2 ** 20, 1024), (1, 2 ** 20 + 1, 4097)])
+def test_groups_of_more_than_a_launch(tensors, base, times):
+    values, n = np.random.default_rng(2).standard_normal(base).astype(np.float32), base * times
+    x = core.repeat(core.float32([base], values), [times])
+    cs = [core.float32([1], [0.25 * (k + 1)]) for k in range(tensors)]
+    outs = [(x + core.repeat(c, [n])) * x for c in cs]
+    try:
+        plan, ret = core.compile(outs, core.PLAN_VIEWS | core.PLAN_FUSE), ops.Tensor([n])
+    except capi.HipError as e:
+        if e.code != 4:
+            raise
+        pytest.skip("not enough device memory")
+    for k in sorted({0, tensors - 1}):
+        rets = [None] * tensors
+        rets[k] = ret
+        plan.execute(None, rets)
+        want = (values + np.float32(0.25 * (k + 1))) * values
+        for block in (0, times // 2, times - 2, times - 1):
+            assert np.array_equal(ret.view(block * base, [base]).numpy(), want), (k, block)
+
+
 def test_penalties_of_many_tensors_as_one_step():
     """sum(w * w) of three and more variables: the sums of dopt_hip_reduce_squares, bit for bit, whatever the size (one
     workgroup's chunk of 4096, several, no multiple of four)."""
