@@ -580,12 +580,14 @@ int dopt_hip_copy_d2d_batch(int n, void *const *dst, const void *const *src, con
             }
         }
         const bool quads = aligned16(src[i]) && aligned16(dst[i]);
+        const size_t need = ceil_div(bytes[i] / 4, quads ? kCopyWords : kCopyLoose);   // (at most 2^21)
+        if (blocks + need > kLaunchBlocks)
+            if (int rc = flush()) return rc;
         b.src[filled] = src[i];
         b.dst[filled] = dst[i];
         b.words[filled] = (unsigned)(bytes[i] / 4);
         b.first[filled] = (unsigned)blocks | (quads ? kOnQuads : 0u);
-        blocks += ceil_div(bytes[i] / 4, quads ? kCopyWords : kCopyLoose);
-        // (blocks of one launch stay far below 2^31: a copy adds at most 2^21 of them)
+        blocks += need;
         if (++filled == kBatchCopies)
             if (int rc = flush()) return rc;
     }

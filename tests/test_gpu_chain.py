@@ -338,3 +338,25 @@ def test_batched_copies_of_every_length_and_alignment():
         want = np.zeros(k + 8, np.float32)
         want[j:j + k] = s.numpy()[i:i + k]
         assert np.array_equal(d.numpy(), want)
+
+
+def test_batched_copies_of_more_than_a_launch():
+    """Nine copies of 2^31 - 1 words that are not on quads: more workgroups than one launch can have, 2^24 of them."""
+    n, edge = 2 ** 31 - 1, 4096
+    r = np.random.default_rng(6)
+    try:
+        src, dst = ops.Tensor([n + 8]), [ops.Tensor([n + 8]) for _ in range(9)]
+    except capi.HipError as e:
+        if e.code != 4:
+            raise
+        pytest.skip("not enough device memory")
+    places = [0, n // 2, n + 8 - edge]
+    values = [r.standard_normal(edge).astype(np.float32) for _ in places]
+    for p, v in zip(places, values):
+        src.view(p, [edge]).set(v)
+    capi.check(capi.load().dopt_hip_copy_d2d_batch(9, (C.c_void_p * 9)(*[d.ptr + 4 * 3 for d in dst]), (C.c_void_p * 9)(*[src.ptr + 4 * 2] * 9),
+                                                   (C.c_size_t * 9)(*[4 * n] * 9)))
+    for k, d in enumerate(dst):   # words 2 .. 2 + n of the source at 3 .. 3 + n
+        assert np.array_equal(d.view(0, [edge]).numpy(), np.concatenate([np.zeros(3, np.float32), values[0][2:-1]])), k
+        assert np.array_equal(d.view(n // 2 + 1, [edge]).numpy(), values[1]), k
+        assert np.array_equal(d.view(n + 8 - edge, [edge]).numpy(), np.concatenate([[0], values[2][:-6], np.zeros(5)]).astype(np.float32)), k
