@@ -2111,11 +2111,12 @@ struct SubFilters {
 };
 template <bool kBwd>
 __global__ __launch_bounds__(256) void pack_gather_k(int M, int Cred, int Mp, int R, int S, int sH, int sW, size_t sm, size_t sc,
-                                                      const float *w, SubFilters subs)
+                                                      const float *w, SubFilters subs, unsigned begin)
 {
     extern __shared__ float stage[];
     const unsigned mblocks = (unsigned)(Mp + 15) / 16;
-    const int RS = R * S, m0 = (int)(blockIdx.x % mblocks) * 16, c0 = (int)(blockIdx.x / mblocks) * 8;
+    const unsigned block = begin + blockIdx.x;
+    const int RS = R * S, m0 = (int)(block % mblocks) * 16, c0 = (int)(block / mblocks) * 8;
     const int len = (kBwd ? 16 : 8) * RS, pitch = len + 1;   // of a run; backward: channel c0 + run, rows m0 ..; forward: row m0 + run, channels c0 ..
     for (int i = threadIdx.x; i < (kBwd ? 8 : 16) * len; i += 256) {
         const int run = i / len, r = i - run * len;
@@ -2150,11 +2151,14 @@ int launch_pack_gather(bool bwd, int K, int C, int R, int S, int sH, int sW, int
 {
     const int M = bwd ? C : K, Cred = bwd ? K : C, chunks = (Cred + BK - 1) / BK, RS = R * S;
     const size_t sm = bwd ? (size_t)RS : (size_t)C * RS, sc = bwd ? (size_t)C * RS : (size_t)RS;
-    const dim3 grid((unsigned)((Mp + 15) / 16) * (unsigned)(2 * chunks));
+    const size_t blocks = (size_t)((Mp + 15) / 16) * (size_t)(2 * chunks);   // (filters have less than 2^29 values: below 2^27)
     const size_t lds = (bwd ? (size_t)8 * (16 * RS + 1) : (size_t)16 * (8 * RS + 1)) * sizeof(float);   // at most 33 KB: 64 taps
-    if (bwd) hipLaunchKernelGGL(pack_gather_k<true>, grid, dim3(256), lds, stream(), M, Cred, Mp, R, S, sH, sW, sm, sc, w, subs);
-    else hipLaunchKernelGGL(pack_gather_k<false>, grid, dim3(256), lds, stream(), M, Cred, Mp, R, S, sH, sW, sm, sc, w, subs);
-    DOPT_LAUNCH_CHECK();
+    for (size_t begin = 0; begin < blocks; begin += kLaunchBlocks) {
+        const dim3 grid((unsigned)std::min(blocks - begin, kLaunchBlocks));
+        if (bwd) hipLaunchKernelGGL(pack_gather_k<true>, grid, dim3(256), lds, stream(), M, Cred, Mp, R, S, sH, sW, sm, sc, w, subs, (unsigned)begin);
+        else hipLaunchKernelGGL(pack_gather_k<false>, grid, dim3(256), lds, stream(), M, Cred, Mp, R, S, sH, sW, sm, sc, w, subs, (unsigned)begin);
+        DOPT_LAUNCH_CHECK();
+    }
     return DOPT_HIP_OK;
 }
 

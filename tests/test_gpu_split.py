@@ -653,6 +653,19 @@ def test_general_filter_of_more_than_2_gib():
         assert np.all(np.abs(dx[:, rows] - want) <= walk(25) * mag)
 
 
+def test_general_filter_of_2_27_channels():
+    """Its packing takes as many workgroups as one launch cannot have, 2^24 of 256 threads."""
+    N, C = 4, 2 ** 27 - 1
+    r = rng(4)
+    w, x, edge = np.zeros((1, C, 1, 1), np.float32), np.zeros((N, C, 1, 1), np.float32), 200
+    for at in (0, C // 2, C - edge):
+        w[:, at:at + edge], x[:, at:at + edge] = cheap(r, 1, edge, 1, 1), cheap(r, N, edge, 1, 1)
+    y = ops.convolution(T(x), T(w), (0, 0), (1, 1)).numpy()
+    used = np.flatnonzero(w[0, :, 0, 0])
+    a, b = x[:, used, 0, 0].astype(np.float64), w[0, used, 0, 0].astype(np.float64)
+    assert np.all(np.abs(y[:, 0, 0, 0] - a @ b) <= walk(3 * edge) * (np.abs(a) @ np.abs(b)))
+
+
 def test_direct_filter_of_more_than_2_gib():
     """One output channel, padded to a tile of 64 rows: the direct kernel's copy would be 2.2 GB, its last channels out of reach."""
     C = 940000
