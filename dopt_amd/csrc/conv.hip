@@ -97,7 +97,11 @@ struct GatherConv {
 // only multiplies 9 -> 7 us for 2 images of 19 x 46 x 14, as before); 64 -> 64 channels of 3 x 3
 // on 64 images of 33 x 31 46 -> 37 us; Wide-ResNet-28-10's two strided 3 x 3 layers backward 270 -> 240 us.  A stage of a
 // 64 x 256 tile takes 1.7 us of which 0.9 are matrix time at the rate of a large product; it reads 144 KB of fragments from LDS.
-// Error against float64 (160 -> 320 channels, stride 2): 8.5e-8 forward, 1.7e-7 backward-data (the fp32 instruction: 2.1e-7, 5.3e-7).
+// A chain of sums ends after eight slabs and is added to `sum`: the error grows with the root of a chain's length, and with few
+// cuts of the reduction a chain was the whole of it.  Drawn layers (3 to 640 channels, filters of 1, 3 and 5) are 0.8 times as far off float64
+// as when it was cut for twice as many workgroups, at most 1.15 times, without the chains up to 1.8 times.  160 -> 320 channels,
+// stride 2: 8.5e-8 forward and 8.4e-8 backward-data, without 1.7e-7 both (the fp32 instruction: 2.1e-7, 5.3e-7).  It costs
+// 1 to 2 % of the time; four stages in a row, so that nothing is decided within, instead of a test per stage, 3 %.
 // kMode: 0 = forward, 1 = backward-data with unit stride (no divisions), 2 = backward-data, any stride.
 // L: the workgroup's item among the problem's (split, tile) pairs, tile fastest.
 template <class T, int SL>
@@ -235,7 +239,7 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
         }
     };
 
-    v16f acc[MI][NI], low[MI][NI];
+    v16f acc[MI][NI], low[MI][NI], sum[MI][NI];
     const int a_frag = (kh * PA + wm * (BM / T::WM) + l32) * 4, b_frag = BOFF + (kh * PB + wn * (BN / T::WN) + l32) * 4;
     v4u a[2][MI][3], b[2][NI][3];
     auto fragments = [&](const float *buf, int sl) {
@@ -298,9 +302,10 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
         }
     };
     const int stages = (slab_end - slab_begin + SL - 1) / SL;
-    auto sums = [&](auto masked_tag) {
+    auto sums = [&](auto masked_tag) {   // (masked or not: the same order)
         zero_acc(acc);
         zero_acc(low);
+        zero_acc(sum);
         rewind();
         load_stage(masked_tag);
         store_a(lds);
@@ -312,15 +317,24 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
         }
         if (stages > 1) load_stage(masked_tag);
         __syncthreads();
-        for (int st = 0; st < stages - 1; ++st) stage(lds + (st & 1) * STAGE, lds + (~st & 1) * STAGE, StepTag<1>{}, masked_tag);
+        int st = 0;
+        for (; st + 4 <= stages - 1; st += 4) {
+            static_for<0, 4>([&](auto tag) {
+                constexpr int cur = decltype(tag)::value % 2;
+                stage(lds + cur * STAGE, lds + (1 - cur) * STAGE, StepTag<1>{}, masked_tag);
+            });
+            move_acc(sum, acc);
+        }
+        for (; st < stages - 1; ++st) stage(lds + (st & 1) * STAGE, lds + (~st & 1) * STAGE, StepTag<1>{}, masked_tag);
         stage(lds + ((stages - 1) & 1) * STAGE, nullptr, StepTag<0>{}, masked_tag);
-        add_acc(acc, low);
+        move_acc(sum, acc);
+        add_acc(sum, low);
     };
     sums(StepTag<0>{});
-    int again = __syncthreads_or(not_finite(acc));
+    int again = __syncthreads_or(not_finite(sum));
     if (again && p.CinPad != p.Cin) {
         sums(StepTag<1>{});
-        again = __syncthreads_or(not_finite(acc));
+        again = __syncthreads_or(not_finite(sum));
     }
 
     // the parts of an infinity hold NaNs: a tile that is not finite is formed again with the fp32 instruction, a stage at a time,
@@ -359,7 +373,7 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
                     }
                 }
         }
-        keep_finite(acc, low);
+        keep_finite(sum, low);
     }
 
     float *outp = p.out + (size_t)split * p.out_elems;
@@ -376,7 +390,7 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
 #pragma unroll
             for (int v = 0; v < 16; v++) {
                 const int m = m0 + wm * (BM / T::WM) + i * 32 + acc_row(v, lane);
-                if (m < p.Mout) base[(size_t)m * p.out_plane] = acc[i][j][v];
+                if (m < p.Mout) base[(size_t)m * p.out_plane] = sum[i][j][v];
             }
     }
 }
@@ -1395,9 +1409,14 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_wgrad_k(FilterGrad p)
         else store(breg[2 * e - NA], breg[2 * e - NA + 1], e - NA / 2, buf + BOFF, PB);
     };
 
-    v16f acc[MI][NI], low[MI][NI];
+    // Chains of sixteen slabs (see conv_gather_body), in pairs of stages, whose places in LDS are then fixed: 5 x 5 at
+    // stride 2, 48 -> 100 on 50 images of 45 x 39, 75 -> 72 us.  0.83 times as far off float64 as when the reduction was cut for twice
+    // as many workgroups, without the chains 1.1 and up to 1.5 times.  Tiles of 64 rows run as two workgroups per CU, which leaves no registers for a second accumulator.
+    constexpr bool kChains = BM > 64;
+    v16f acc[MI][NI], low[MI][NI], sum[MI][NI];
     zero_acc(acc);
     zero_acc(low);
+    zero_acc(sum);
     const int a_frag = (kh * PA + wm * (BM / T::WM) + l32) * 4, b_frag = BOFF + (kh * PB + wn * (BN / T::WN) + l32) * 4;
     v4u a[2][MI][3], b[2][NI][3];
     auto fragments = [&](const float *buf, int sl) {
@@ -1444,13 +1463,25 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_wgrad_k(FilterGrad p)
         });
         if constexpr (more) __syncthreads();
     };
-    for (int st = 0; st < stages - 1; ++st) stage(lds + (st & 1) * STAGE, lds + (~st & 1) * STAGE, StepTag<1>{});
+    int st = 0;
+    if constexpr (kChains) {
+        while (st + 8 <= stages - 1) {
+#pragma unroll 1
+            for (int pair = 0; pair < 4; pair++, st += 2) {
+                stage(lds, lds + STAGE, StepTag<1>{});
+                stage(lds + STAGE, lds, StepTag<1>{});
+            }
+            move_acc(sum, acc);
+        }
+    }
+    for (; st < stages - 1; ++st) stage(lds + (st & 1) * STAGE, lds + (~st & 1) * STAGE, StepTag<1>{});
     stage(lds + ((stages - 1) & 1) * STAGE, nullptr, StepTag<0>{});
-    add_acc(acc, low);
+    move_acc(sum, acc);
+    add_acc(sum, low);
 
     // the parts of an infinity hold NaNs: a tile that is not finite is formed again with the fp32 instruction, a stage at a time
-    if (__syncthreads_or(not_finite(acc))) {
-        zero_acc(acc);
+    if (__syncthreads_or(not_finite(sum))) {
+        zero_acc(sum);
         slab = slab_begin;
 #pragma unroll 1
         for (int st = 0; st < stages; ++st) {
@@ -1472,9 +1503,9 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_wgrad_k(FilterGrad p)
                     for (int i = 0; i < MI; i++)
 #pragma unroll
                         for (int j = 0; j < NI; j++)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(lds[((sl * 2 + kh) * PA + wm * (BM / T::WM) + l32 + 32 * i) * 8 + e],
+                            sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(lds[((sl * 2 + kh) * PA + wm * (BM / T::WM) + l32 + 32 * i) * 8 + e],
                                                                               lds[BOFF + ((sl * 2 + kh) * PB + wn * (BN / T::WN) + l32 + 32 * j) * 8 + e],
-                                                                              acc[i][j], 0, 0, 0);
+                                                                              sum[i][j], 0, 0, 0);
         }
     }
 
@@ -1488,7 +1519,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_wgrad_k(FilterGrad p)
 #pragma unroll
             for (int v = 0; v < 16; v++) {
                 const int m = m0 + wm * (BM / T::WM) + i * 32 + acc_row(v, lane);
-                if (m < p.K) outp[(size_t)m * p.ncols + col] = acc[i][j][v];
+                if (m < p.K) outp[(size_t)m * p.ncols + col] = sum[i][j][v];
             }
     }
 }

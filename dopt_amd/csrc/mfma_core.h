@@ -157,6 +157,21 @@ __device__ __forceinline__ void add_acc(v16f (&acc)[MI][NI], const v16f (&low)[M
             for (int v = 0; v < 16; v++) acc[i][j][v] = (acc[i][j][v] + low[i][j][v]) * kSplitDown;
 }
 
+// Ends a chain of sums: what it holds goes to `sum`, and the next one begins.
+template <int MI, int NI>
+__device__ __forceinline__ void move_acc(v16f (&sum)[MI][NI], v16f (&acc)[MI][NI])
+{
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+        for (int j = 0; j < NI; j++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                sum[i][j][v] += acc[i][j][v];
+                acc[i][j][v] = 0.0f;
+            }
+}
+
 // Whether this lane's accumulators hold an infinity or a NaN: x * 0 is 0 for finite x only.
 template <int MI, int NI>
 __device__ __forceinline__ int not_finite(const v16f (&acc)[MI][NI])

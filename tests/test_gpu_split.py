@@ -476,6 +476,28 @@ def test_general_convolution_operands_that_are_not_finite():
         assert np.all(np.abs(got[fine] - want[fine]) <= walk(2500) * want[fine])   # (every term is positive)
 
 
+def test_general_convolution_error_grows_with_chains_not_with_the_reduction():
+    """Reductions that are not cut (256 tiles and more): a sum is added up in chains of at most 16 slabs of 16 terms, and the chains
+    one after the other, each rounded once.  So it is not further off float64 than a reduction of nine slabs whose roundings are as many
+    as a chain's, and the roundings of the chains (0.43 / sqrt(2) of 2^-24 each, see rounded_once_per_term)."""
+    r = rng(12)
+    N, C, H, W, K = 64, 256, 17, 15, 256
+    off = lambda got, want: np.linalg.norm(got - want) / np.linalg.norm(want)
+    x, w = r.standard_normal((N, C, H, W), np.float32), r.standard_normal((K, C, 3, 3), np.float32)
+    y = ops.convolution(T(x), T(w), (1, 1), (1, 1)).numpy()
+    dy = r.standard_normal(y.shape, np.float32)
+    dx = ops.conv_bwd_data(T(dy), T(w), x.shape, (1, 1), (1, 1)).numpy()
+    dw = ops.conv_bwd_filter(T(dy), T(x), w.shape, (1, 1), (1, 1)).numpy()
+    x9, w9 = np.ascontiguousarray(x[:, :16]), np.ascontiguousarray(w[:, :16])
+    nine = off(ops.convolution(T(x9), T(w9), (1, 1), (1, 1)).numpy()[:4], general(x9[:4], w9, 1, 1))
+    bound = lambda slabs, chain: 1.1 * np.hypot(nine * np.sqrt(chain / 9), 0.30 * 2.0 ** -24 * np.sqrt(slabs / chain))
+    assert off(y[:4], general(x[:4], w, 1, 1)) <= bound(144, 8)
+    few = np.zeros((4, C, H, W), np.float32)
+    assert off(dx[:4], general_gradients(few, w, dy[:4], 1, 1)[0]) <= bound(144, 8)
+    want = general_gradients(x, w[:32], np.ascontiguousarray(dy[:, :32]), 1, 1)[1]
+    assert off(dw[:32], want) <= bound(N * H * W / 16, 16)
+
+
 # channel counts off the slab, of x and of dy; images of one 256-pixel tile each, and several in a tile
 @pytest.mark.parametrize("shape", [(3, 17, 16, 16, 23, 5, 2, 1), (3, 33, 16, 16, 20, 1, 0, 1), (4, 40, 8, 8, 130, 5, 2, 1), (3, 17, 32, 32, 24, 3, 1, 2),
                                    (2, 150, 7, 9, 70, 3, 0, 2)])
