@@ -3279,7 +3279,12 @@ WgradSetup wgrad_patch_setup(const dopt_hip_conv_desc *d, const float *dw)
             }
         }
     }
-    if (out_elems % 4 != 0 || !aligned16(dw)) splits = 1;  // the split sum works on float4
+    const bool whole = out_elems % 4 != 0 || !aligned16(dw);
+    if (whole) splits = 1;  // the split sum works on float4
+    // 64-row tiles on 4 x 4 images: few workgroups of a long set-up unless the layer or the batch is large, and one without a split
+    // (16 images, 64 -> 64 channels: 20 us, the general kernel 10; 140, 62 -> 27: 135 and 18; 128, 128 -> 48: 21 and 18; but 256, 16 -> 16:
+    // 18 and 26; 512, 64 -> 64: 25 and 29; 128, 320 -> 320: 41 and 59; 192 -> 192, nine tiles, 8 to 128 images: within a tenth)
+    if (geo == 1 && BM == 64 && (whole || (tiles < 8 && d->N < 256))) return u;
     wp.chunks_per_split = (wp.chunks_total + splits - 1) / splits;
     splits = (wp.chunks_total + wp.chunks_per_split - 1) / wp.chunks_per_split;
     wp.splits = splits;

@@ -1,5 +1,7 @@
 """fp32 products formed on the bf16 matrix instructions (three bf16 parts per value): the tile edges, the cuts of the
 reduction and operands that are not finite, against float64."""
+import time
+
 import numpy as np
 import pytest
 
@@ -351,6 +353,29 @@ def test_filter_gradient(shape):
     want, mag = filter_gradient(dy, x), filter_gradient(dy, x, np.abs)
     assert np.all(np.abs(got - want) <= walk(N * H * W) * mag), np.max(np.abs(got - want) / mag)
     check_norm(got, want, N * H * W / 2, shape)
+
+
+# 4 x 4 images, either side of the lines between the kernels
+@pytest.mark.parametrize("shape", [(252, 64, 4, 4, 64), (256, 64, 4, 4, 64), (256, 62, 4, 4, 27), (8, 192, 4, 4, 192), (12, 191, 4, 4, 65)])
+def test_filter_gradient_of_small_images(shape):
+    test_filter_gradient(shape)
+
+
+def test_filter_gradient_without_a_split_takes_no_longer_than_with_one():
+    """4 x 4 images, an odd and an even number of quads of filter values: one workgroup added the 35 chunks of the odd one, seven
+    times as long."""
+    def best(N, C, H, W, K):
+        dy, x, dw = T(np.ones((N, K, H, W), np.float32)), T(np.ones((N, C, H, W), np.float32)), ops.Tensor([K, C, 3, 3])
+        times = []
+        for _ in range(12):
+            ops.sync()
+            start = time.perf_counter()
+            for _ in range(10):
+                ops.conv_bwd_filter(dy, x, dw.shape, (1, 1), (1, 1), out=dw)
+            ops.sync()
+            times.append(time.perf_counter() - start)
+        return min(times)
+    assert best(140, 62, 4, 4, 27) < 3 * best(140, 64, 4, 4, 28)
 
 
 @pytest.mark.parametrize("shape", [(4, 64, 16, 16, 128), (8, 64, 4, 4, 64), (3, 32, 32, 32, 160)])
