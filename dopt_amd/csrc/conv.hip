@@ -102,6 +102,8 @@ struct GatherConv {
 // as when it was cut for twice as many workgroups, at most 1.15 times, without the chains up to 1.8 times.  160 -> 320 channels,
 // stride 2: 8.5e-8 forward and 8.4e-8 backward-data, without 1.7e-7 both (the fp32 instruction: 2.1e-7, 5.3e-7).  It costs
 // 1 to 2 % of the time; four stages in a row, so that nothing is decided within, instead of a test per stage, 3 %.
+// Stages of one slab (SL = 1) are for short reductions (see gather_launch): no chains, and registers for two workgroups
+// per CU, of which one stores its results or loads its first stage while the other multiplies.
 // kMode: 0 = forward, 1 = backward-data with unit stride (no divisions), 2 = backward-data, any stride.
 // L: the workgroup's item among the problem's (split, tile) pairs, tile fastest.
 template <class T, int SL>
@@ -318,7 +320,7 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
         if (stages > 1) load_stage(masked_tag);
         __syncthreads();
         int st = 0;
-        for (; st + 4 <= stages - 1; st += 4) {
+        if constexpr (SL > 1) for (; st + 4 <= stages - 1; st += 4) {
             static_for<0, 4>([&](auto tag) {
                 constexpr int cur = decltype(tag)::value % 2;
                 stage(lds + cur * STAGE, lds + (1 - cur) * STAGE, StepTag<1>{}, masked_tag);
@@ -396,7 +398,7 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
 }
 
 template <class T, int SL, int kMode>
-__global__ __launch_bounds__(T::THREADS, 2) void conv_gather_k(GatherConv p)
+__global__ __launch_bounds__(T::THREADS, SL > 1 ? 2 : 4) void conv_gather_k(GatherConv p)
 {
     // 1-D grid over (split, tile), tile fastest: the blocks an XCD receives work on neighbouring
     // tiles of the same slice of the reduction, whatever the ratio of tiles to splits
@@ -2961,7 +2963,16 @@ int gather_launch(GatherConv g, int mode, int K, int C, const float *in, const f
     g.in_bytes = (size_t)g.N * g.Cin * g.IH * g.IW * sizeof(float);
     g.out = splits > 1 ? partial : out;
     dim3 grid(xcd_grid((unsigned)(tiles * splits)));
-    if (int rc = wide ? launch_gather<GatherWide, 2>(mode, g, grid) : launch_gather<GatherSquare, 2>(mode, g, grid)) return rc;
+    // Short reductions that are not cut: in stages of one slab, two workgroups per CU, where there are two tiles per CU or a second
+    // slab would be half of the work.  1 x 1 on 128 images of 32 x 32, stages of two slabs -> of one: 16 -> 160 channels 37 -> 28 us,
+    // 112 -> 160 63 -> 53; 145 images of 29 x 25, 15 -> 7 14 -> 12; but 3 x 3 on 64 of 33 x 31, 16 -> 32, 256 tiles of nine slabs, 17 -> 19.  Beyond nine
+    // slabs only from four tiles per CU on, where reductions were not cut before either: without chains the error is that of
+    // the whole reduction (320 -> 320 196 -> 191 us, 480 -> 320, thirty slabs, 275 -> 266; but 42 -> 592, 3 x 3, 515 tiles of 27 slabs, 1.3 times as far off).
+    const int tiles_per_cu = tiles / num_cus();
+    const bool brief = splits == 1 && g.slabs_total <= (tiles_per_cu >= 4 ? 32 : tiles_per_cu >= 2 ? 9 : 3);
+    if (int rc = brief ? (wide ? launch_gather<GatherWide, 1>(mode, g, grid) : launch_gather<GatherSquare, 1>(mode, g, grid))
+                       : (wide ? launch_gather<GatherWide, 2>(mode, g, grid) : launch_gather<GatherSquare, 2>(mode, g, grid)))
+        return rc;
     if (splits > 1) return launch_splitk_reduce(g.out_elems, splits, partial, out);
     return DOPT_HIP_OK;
 }

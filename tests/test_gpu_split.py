@@ -474,6 +474,26 @@ def test_general_convolution(shape):
     check_norm(dw, wants[1], dy[:, 0].size / 2, shape)
 
 
+# short reductions in stages of one slab: one slab, nine, many tiles of ten and of thirty-two; and one slab more than each, few tiles of ten
+@pytest.mark.parametrize("shape", [(5, 16, 31, 9, 70, 1, 0, 1), (2, 3, 17, 15, 130, 3, 1, 1), (64, 145, 32, 32, 250, 1, 0, 1), (64, 500, 33, 31, 250, 1, 0, 1),
+                                   (2, 145, 31, 9, 70, 1, 0, 1), (64, 520, 33, 31, 250, 1, 0, 1)])
+def test_general_convolution_of_short_reductions(shape):
+    N, C, H, W, K, R, pad, stride = shape
+    r = rng(C + K)
+    x, w = r.standard_normal((N, C, H, W), np.float32), r.standard_normal((K, C, R, R), np.float32)
+    got = ops.convolution(T(x), T(w), (pad, pad), (stride, stride)).numpy()
+    dy = r.standard_normal(got.shape, np.float32)
+    dx = ops.conv_bwd_data(T(dy), T(w), x.shape, (pad, pad), (stride, stride)).numpy()
+    for part in (slice(0, 1), slice(N - 1, N)):
+        check_norm(got[part], general(x[part], w, pad, stride), C * R * R, shape)
+        check_norm(dx[part], general_gradients(x[part], w, dy[part], pad, stride)[0], K * R * R, shape)
+    x[N - 1, C - 1, 0, 0], dy[0, 0, 1, 1] = np.inf, np.nan   # the pass that forms a tile again, in stages of one slab too
+    for again, plain in ((ops.convolution(T(x), T(w), (pad, pad), (stride, stride)).numpy(), got),
+                         (ops.conv_bwd_data(T(dy), T(w), x.shape, (pad, pad), (stride, stride)).numpy(), dx)):
+        fine = np.isfinite(again)
+        assert not fine.all() and fine.mean() > 0.9 and np.array_equal(again[fine], plain[fine])
+
+
 def test_general_convolution_operands_that_are_not_finite():
     """A value far from every bad one is what it is without them; an infinity stays one and a NaN stays one."""
     r = rng(3)
