@@ -105,7 +105,6 @@ struct PointwiseItem {
 };
 constexpr int kGroupInputs = 48, kGroupNodes = 64, kGroupOuts = 8;
 int pointwise_group(const PointwiseProgram &program, const std::vector<PointwiseItem> &items);
-int pointwise_group_compile_only(const PointwiseProgram &program, const char *arch);
 
 // rtc_ops.cpp: out[i] = the sum of the squares of the n[i] (more than 64) values at in[i], each the value that
 // dopt_hip_reduce_squares gives.

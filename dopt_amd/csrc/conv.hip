@@ -104,7 +104,7 @@ struct GatherConv {
 // 1 to 2 % of the time; four stages in a row, so that nothing is decided within, instead of a test per stage, 3 %.
 // Stages of one slab (SL = 1) are for short reductions (see gather_launch): no chains, and registers for two workgroups
 // per CU, of which one stores its results or loads its first stage while the other multiplies.
-// kMode: 0 = forward, 1 = backward-data with unit stride (no divisions), 2 = backward-data, any stride.
+// kBwd: backward-data, of unit stride.
 // L: the workgroup's item among the problem's (split, tile) pairs, tile fastest.
 template <class T, int SL>
 struct GatherLds {
@@ -113,7 +113,7 @@ struct GatherLds {
     static constexpr size_t BYTES = 2 * STAGE * sizeof(float);
 };
 
-template <class T, int SL, int kMode>
+template <class T, int SL, bool kBwd>
 __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L)
 {
     constexpr int BM = T::BM, BN = T::BN, THREADS = T::THREADS, MI = T::MI, NI = T::NI;
@@ -188,19 +188,12 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
     };
     auto pixel = [&]() {   // byte offset of this thread's input pixel for the slab at the running position, or kOobOffset
         int ih, iw, bad = pix_oob | (slab_end - 1 - slab);
-        if (kMode == 0) {
+        if constexpr (!kBwd) {
             ih = oh * p.strideH - p.padH + (p.R - 1 - tr);
             iw = ow * p.strideW - p.padW + (p.S - 1 - ts);
-        } else if (kMode == 1) {
+        } else {
             ih = oh + p.padH - (p.R - 1 - tr);
             iw = ow + p.padW - (p.S - 1 - ts);
-        } else {
-            // out = dx[.., h, w]; in = dy[.., ph, qw] with h = ph*stride - pad + r, r = R-1-tr
-            const int nh = oh + p.padH - (p.R - 1 - tr), nw = ow + p.padW - (p.S - 1 - ts);
-            ih = nh / p.strideH;
-            iw = nw / p.strideW;
-            // negative numerators, and numerators that are not multiples of the stride, hit no input
-            bad |= nh | nw | -(int)(ih * p.strideH != nh) | -(int)(iw * p.strideW != nw);
         }
         bad |= ih | (p.IH - 1 - ih) | iw | (p.IW - 1 - iw);  // sign bit set: outside the input
         return bad < 0 ? kOobOffset : (unsigned)(pix_base + ih * p.IW + iw) * 4u;
@@ -397,14 +390,14 @@ __device__ __forceinline__ void conv_gather_body(const GatherConv &p, unsigned L
     }
 }
 
-template <class T, int SL, int kMode>
+template <class T, int SL, bool kBwd>
 __global__ __launch_bounds__(T::THREADS, SL > 1 ? 2 : 4) void conv_gather_k(GatherConv p)
 {
     // 1-D grid over (split, tile), tile fastest: the blocks an XCD receives work on neighbouring
     // tiles of the same slice of the reduction, whatever the ratio of tiles to splits
     unsigned L;
     if (!xcd_remap(blockIdx.x, (unsigned)(p.mtiles * p.ntiles) * (unsigned)p.splits, &L)) return;
-    conv_gather_body<T, SL, kMode>(p, L);
+    conv_gather_body<T, SL, kBwd>(p, L);
 }
 
 // Up to nine problems that do not depend on each other in ONE launch (the residue classes of a strided backward-data
@@ -419,7 +412,7 @@ struct GatherGroup {
     int n;
 };
 
-template <class T, int SL, int kMode>
+template <class T, int SL, bool kBwd>
 __global__ __launch_bounds__(T::THREADS, 2) void conv_gather_group_k(GatherGroup gg)
 {
     const unsigned xcd = blockIdx.x & 7u;
@@ -431,7 +424,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_gather_group_k(GatherGroup
     }
     const unsigned L = xcd * gg.per[j] + i;
     if (i >= gg.per[j] || L >= (unsigned)(gg.g[j].mtiles * gg.g[j].ntiles) * (unsigned)gg.g[j].splits) return;
-    conv_gather_body<T, SL, kMode>(gg.g[j], L);
+    conv_gather_body<T, SL, kBwd>(gg.g[j], L);
 }
 
 // ------------------------------------------------------------------------------------ patch (3x3, unit stride)
@@ -466,7 +459,7 @@ __device__ inline unsigned fast_div(unsigned x, unsigned magic) { return __umulh
 // The products run on the bf16 matrix instruction (mfma_core.h).  A patch value is split once, when it is stored, and its parts
 // serve all nine taps of all rows, so splitting is a tenth of the loop.  The filter's parts are packed; its fragments go from
 // memory straight into the registers the matrix cores read: the packed layout is the fragment layout (a wavefront fetches 32
-// rows x 32 bytes, 1 KB contiguous, per part; wavefronts of a tile row fetch the same lines, all but one from the L1), one or two
+// rows x 32 bytes, 1 KB contiguous, per part; wavefronts of a tile row fetch the same lines, all but one from the L1), two
 // taps ahead.  Only the patch goes through LDS, double buffered: [part][channel half][position][8 channels], a lane's fragment
 // of one part is one 128-bit read and neighbouring lanes' reads are neighbours.  The workgroup meets once per 16-channel chunk.
 // The h.h products have an accumulator of their own, the five small ones another.
@@ -478,8 +471,8 @@ __device__ __forceinline__ void conv_patch_body(const PatchConv &p, const unsign
 {
     constexpr int BM = T::BM, BN = T::BN, THREADS = T::THREADS, MI = T::MI, NI = T::NI;
     constexpr int TAPS = 9, CH = 16;
-    constexpr int AHEAD = MI == 1 ? 2 : 1, RING = AHEAD + 1;   // filter fragments on their way: a tap of MI = 1 lasts half as long
-    static_assert(TAPS % RING == 0 || RING == 2, "the ring slot of a tap follows from its number");
+    constexpr int AHEAD = 2, RING = AHEAD + 1;   // filter fragments on their way
+    static_assert(MI == 1 && TAPS % RING == 0, "two taps of one row group ahead; the ring slot of a tap follows from its number");
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int area = p.psz + 1;              // one spare position absorbs the stores of unused slots
     const int pstride = area * 24;           // floats of one patch buffer: 3 parts x 2 halves x 4 words a position
@@ -593,16 +586,14 @@ __device__ __forceinline__ void conv_patch_body(const PatchConv &p, const unsign
     // tap 8, behind the last reads of the patch being multiplied.
     constexpr int PER = NS * 2;   // loads of a tap
     static_assert(NS <= 3, "a slot per tap 5 .. 7");
-    int ring = 0;   // (two slots: nine taps leave the ring turned)
-    auto chunk_products = [&](int chunk, const float *bp_cur, float *bp_nxt, auto turned_tag) {
-        constexpr int turned = decltype(turned_tag)::value;
+    auto chunk_products = [&](int chunk, const float *bp_cur, float *bp_nxt) {
         const __amdgpu_buffer_rsrc_t rw_now = fa_rsrc(chunk), rw_next = fa_rsrc(chunk + 1 < ce ? chunk + 1 : chunk);   // (after the last chunk: loaded, not used)
         unsigned q[3][4];
 #pragma unroll
         for (int j = 0; j < NI; j++) asm volatile("" : "+v"(b_pos[j]));   // (or the fifty-four addresses of a chunk are kept in registers)
         static_for<0, TAPS>([&](auto ttag) {
             constexpr int t = decltype(ttag)::value;
-            constexpr int slot = (t + turned) % RING;
+            constexpr int slot = t % RING;
             // the pixel part that is used last is read first again: l after its one product, m after its two, h at the tap's start
             static_for<0, 6>([&](auto stag) {
                 constexpr int ks = decltype(stag)::value;
@@ -610,7 +601,7 @@ __device__ __forceinline__ void conv_patch_body(const PatchConv &p, const unsign
                 constexpr int qa = ks == 0 ? 0 : ks == 1 ? 1 : ks == 2 ? 0 : ks == 3 ? 2 : ks == 4 ? 1 : 0;
                 // side work of this step, pinned to it
                 if constexpr (ks == 0) {
-                    fa_load((t + AHEAD + turned) % RING, t + AHEAD < TAPS ? rw_now : rw_next, (t + AHEAD) % TAPS);
+                    fa_load((t + AHEAD) % RING, t + AHEAD < TAPS ? rw_now : rw_next, (t + AHEAD) % TAPS);
                     fb_load(0, bp_cur, t);
                     if constexpr (t == TAPS - 1) __syncthreads();
                 }
@@ -638,9 +629,7 @@ __device__ __forceinline__ void conv_patch_body(const PatchConv &p, const unsign
     for (int chunk = cb; chunk < ce; ++chunk) {
         float *const bp_cur = Bp0 + ((chunk - cb) & 1) * pstride;
         float *const bp_nxt = Bp0 + ((chunk - cb + 1) & 1) * pstride;
-        if (RING == 2 && ring) chunk_products(chunk, bp_cur, bp_nxt, StepTag<1>{});
-        else chunk_products(chunk, bp_cur, bp_nxt, StepTag<0>{});
-        ring ^= 1;
+        chunk_products(chunk, bp_cur, bp_nxt);
     }
     add_acc(acc, low);
 
@@ -2911,18 +2900,15 @@ int launch_gather_kernel(const Args &args, dim3 grid)
 }
 
 template <class T, int SL>
-int launch_gather(int mode, const GatherConv &g, dim3 grid)
+int launch_gather(bool bwd, const GatherConv &g, dim3 grid)
 {
-    if (mode == 0) return launch_gather_kernel<T, SL, conv_gather_k<T, SL, 0>>(g, grid);
-    if (mode == 1) return launch_gather_kernel<T, SL, conv_gather_k<T, SL, 1>>(g, grid);
-    return launch_gather_kernel<T, SL, conv_gather_k<T, SL, 2>>(g, grid);
+    return bwd ? launch_gather_kernel<T, SL, conv_gather_k<T, SL, true>>(g, grid) : launch_gather_kernel<T, SL, conv_gather_k<T, SL, false>>(g, grid);
 }
 
 // Packs the filter w[K][C][g.R * g.S] and runs conv_gather_k on a problem whose geometry the caller
-// has filled in (dimensions, padding, stride, output placement).  mode as conv_gather_k's kMode.
-int gather_launch(GatherConv g, int mode, int K, int C, const float *in, const float *w, float *out)
+// has filled in (dimensions, padding, stride, output placement).
+int gather_launch(GatherConv g, bool bwd, int K, int C, const float *in, const float *w, float *out)
 {
-    const bool bwd = mode != 0;
     const int taps = g.R * g.S;
     g.CinPad = round_up(g.Cin, BK);
     g.Mp = round_up(g.Mout, 4);
@@ -2970,8 +2956,8 @@ int gather_launch(GatherConv g, int mode, int K, int C, const float *in, const f
     // the whole reduction (320 -> 320 196 -> 191 us, 480 -> 320, thirty slabs, 275 -> 266; but 42 -> 592, 3 x 3, 515 tiles of 27 slabs, 1.3 times as far off).
     const int tiles_per_cu = tiles / num_cus();
     const bool brief = splits == 1 && g.slabs_total <= (tiles_per_cu >= 4 ? 32 : tiles_per_cu >= 2 ? 9 : 3);
-    if (int rc = brief ? (wide ? launch_gather<GatherWide, 1>(mode, g, grid) : launch_gather<GatherSquare, 1>(mode, g, grid))
-                       : (wide ? launch_gather<GatherWide, 2>(mode, g, grid) : launch_gather<GatherSquare, 2>(mode, g, grid)))
+    if (int rc = brief ? (wide ? launch_gather<GatherWide, 1>(bwd, g, grid) : launch_gather<GatherSquare, 1>(bwd, g, grid))
+                       : (wide ? launch_gather<GatherWide, 2>(bwd, g, grid) : launch_gather<GatherSquare, 2>(bwd, g, grid)))
         return rc;
     if (splits > 1) return launch_splitk_reduce(g.out_elems, splits, partial, out);
     return DOPT_HIP_OK;
@@ -2980,7 +2966,7 @@ int gather_launch(GatherConv g, int mode, int K, int C, const float *in, const f
 // ---- backward-data with a stride, one residue class of output pixels at a time -------------------
 // dx[n, c, h, w] = sum over k, r, s with (h + padH - r) and (w + padW - s) multiples of the stride of
 // dy[n, k, (h + padH - r) / sH, (w + padW - s) / sW] * w[k, c, R - 1 - r, S - 1 - s] (the flipped filter).  Which taps qualify depends only
-// on (h mod sH, w mod sW).  Taking all pixels together (conv_gather_k mode 2) multiplies every pixel
+// on (h mod sH, w mod sW).  Taking all pixels together multiplies every pixel
 // by every tap and masks three quarters of the products of a stride-2 3x3 layer; taking the pixels
 // of one class (a, b) = (h mod sH, w mod sW) at a time, only its taps r = r0, r0 + sH, ... and s = s0,
 // s0 + sW, ... are multiplied, and the class is a UNIT-stride problem on the grid (i, j) = (h / sH, w / sW):
@@ -3082,8 +3068,8 @@ int run_bwd_strided(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float
             blocks += 8u * gg.per[j];
         }
         if (int rc = launch_pack_gather(true, K, C, R, S, sH, sW, Mp, w, subs)) return rc;
-        if (wide) return launch_gather_kernel<GatherWide, 2, conv_gather_group_k<GatherWide, 2, 1>>(gg, blocks);
-        return launch_gather_kernel<GatherSquare, 2, conv_gather_group_k<GatherSquare, 2, 1>>(gg, blocks);
+        if (wide) return launch_gather_kernel<GatherWide, 2, conv_gather_group_k<GatherWide, 2, true>>(gg, blocks);
+        return launch_gather_kernel<GatherSquare, 2, conv_gather_group_k<GatherSquare, 2, true>>(gg, blocks);
     }
     void *sub = nullptr;
     if (int rc = scratch_alloc(&sub, d->K * d->C * d->R * d->S * sizeof(float))) return rc;
@@ -3108,7 +3094,7 @@ int run_bwd_strided(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float
             g.Mout = (int)d->C; g.OH = ch.n; g.OW = cw.n;
             g.out_plane = H * W; g.out_OW = W;
             g.out_sy = sH; g.out_sx = sW; g.out_oy = a; g.out_ox = b;
-            rc = gather_launch(g, 1, (int)d->K, (int)d->C, dy, (const float *)sub, dx);
+            rc = gather_launch(g, true, (int)d->K, (int)d->C, dy, (const float *)sub, dx);
         }
     dopt_hip_free(sub);
     return rc;
@@ -3158,7 +3144,7 @@ int run_gather(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float *in,
     g.out_plane = g.OH * g.OW;
     g.out_OW = g.OW;
     g.out_sy = g.out_sx = 1;
-    return gather_launch(g, kBwd ? 1 : 0, (int)d->K, (int)d->C, in, w, out);
+    return gather_launch(g, kBwd, (int)d->K, (int)d->C, in, w, out);
 }
 
 template <int WM, int WC, int kGeo, bool kPre = kGeo != 2>

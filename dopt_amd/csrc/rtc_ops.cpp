@@ -777,13 +777,6 @@ int pointwise_group(const PointwiseProgram &p, const std::vector<PointwiseItem> 
     return flush();
 }
 
-int pointwise_group_compile_only(const PointwiseProgram &p, const char *arch)
-{
-    if (int rc = group_check(p)) return rc;
-    const std::vector<char> common(p.kind.size(), 0);
-    return rtc_compile_only(group_source(p, group_shape(p, common)), arch, nullptr);
-}
-
 }  // namespace dopt
 
 extern "C" {
