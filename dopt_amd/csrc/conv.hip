@@ -713,8 +713,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_patch_k(PatchConv p)
 // The same layers (3x3, unit stride, pad 1, even image sides, whole 16-channel chunks) with 16 instead of 36
 // multiplications per 2x2 output pixels (Lavin & Gray): Y = At [ (G g Gt) . (Bt d B) ] A, the element-wise product summed
 // over the channels - sixteen independent [rows x channels] . [channels x tiles] products, one per position xi of the
-// 4x4 transformed tile.  The direct kernels run at three quarters of the fp32 matrix peak, so what is left to remove is
-// arithmetic.
+// 4x4 transformed tile.
 //
 // A workgroup owns 128 rows x 32 tiles (the 128 pixels of the direct kernel's column tile: whole image rows or whole
 // images, so the input under them is the same rectangle with the same zero halo) or 64 rows x 64 tiles.
@@ -2267,7 +2266,7 @@ struct PatchSetup {
     PatchConv pc;
     int shape;            // 0 wide, 1 narrow, 2 deep, 3 tall, 4 Winograd (BM 128: 128 rows x 32 tiles of 2x2 pixels, BM 64: 64 rows x 64 tiles)
     int BM, BN, blocks_wanted, tiles;
-    int positions;        // of a patch that the workgroup's load slots hold
+    int positions;        // of a patch, at most (the load slots of some tiles hold more: wider patches are the general kernels')
     size_t lds_bytes, wp_elems;
 };
 
@@ -2375,7 +2374,8 @@ PatchSetup patch_setup_as(const dopt_hip_conv_desc *d, size_t P, size_t Q, bool 
     pc.out_elems = (size_t)pc.ncols * pc.Mout;
     u.tiles = pc.mtiles * pc.ntiles;
     u.wp_elems = (size_t)pc.chunks_total * (wino ? 16 : 9) * 24 * pc.Mp;   // three 16-bit parts a value
-    // (few rows of very many channels, whose copy in fp32, padded to 64 rows, would reach 2 GiB, are the general kernels')
+    // (few rows of very many channels, from 2 GiB at four bytes a value and 64 rows on, stay the general kernels', as they were
+    // when the copy was one of fp32 values and reached by 32-bit offsets; not measured against the direct kernel since)
     if (!wino && (size_t)pc.chunks_total * 9 * 64 * std::max(pc.Mp, 64) > 0x7fffffffu) return u;
     u.ok = true;
     return u;
@@ -2404,7 +2404,9 @@ PackJob pack_job(const dopt_hip_conv_desc *d, const PatchSetup &u, const float *
 // ties go to the smaller one.
 int patch_splits(int tiles, int chunks, int slots, int BM, int BN, size_t out_elems, bool wino)
 {
-    const double cu_tflops = wino ? 0.47 : 0.8;                      // what one CU sustains in these main loops (direct: 0.47 in fp32)
+    // what one CU sustains in these main loops (direct: 0.47 in fp32.  With 0.47 here, and 0.33 in place of kGatherRate, the half-width
+    // VGG-16 step is 0.4 % and that of Wide-ResNet-10-2 2.4 % longer, Wide-ResNet-28-10's and the 5 x 5 layers' the same)
+    const double cu_tflops = wino ? 0.47 : 0.8;
     const double per_cu = (double)slots / num_cus();                 // blocks sharing a CU
     // 16 channels x 9 taps.  The Winograd kernel takes a third of that for a chunk, but adds all six parts of a product in one
     // accumulator: with its own time here it would be cut less and be further off than the fp32 instruction, which was cut by
@@ -2427,7 +2429,8 @@ int patch_splits(int tiles, int chunks, int slots, int BM, int BN, size_t out_el
     return best;
 }
 
-// The same estimate for the general kernels, whose unit is a slab of 16 reduction steps, at the rate that one CU sustains.
+// The same estimate for the general kernels, whose unit is a slab of 16 reduction steps, at the rate that one CU sustains (0.33 on the
+// fp32 instruction; measured above).
 constexpr double kGatherRate = 0.6;
 int gather_splits(int tiles, int slabs, int slots, int BM, int BN, size_t out_elems, double cu_tflops, int cap)
 {
@@ -3388,7 +3391,8 @@ int run_bwd_pair(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float *d
     // (the 64 x 256 and 32 x 256 tiles of layers with up to 64 input channels are not built), with 128 x 32 filter-gradient tiles on
     // rows of 8 .. 64 pixels or on 4 x 4 images.
     // (a layer the Winograd kernel takes has its filter packed for that kernel: shape 4, not a pair)
-    // (only where the launch needs it: with two rounds of backward-data tiles and more the two run one after the other)
+    // (only where the launch needs it: with two rounds of backward-data tiles and more the two run one after the other, which
+    // took as long or 1 % less: 64 images of 100 x 32 x 32, 128 filters, 350 and 348 us for the whole step; 256 of 200 x 16 x 16, 384, 1460 and 1450)
     const bool few = a.shape == 2 && a.tiles < 2 * num_cus();
     const int combo = few && b.tall && b.geo == 0 ? 0 : few && b.tall && b.geo == 1 ? 1 : -1;
     // A layer whose backward-data is the Winograd kernel on 128-row tiles: two launches, each as it would run alone, but out of ONE

@@ -3,7 +3,7 @@
 // The tail of a training graph - softmax, the loss's logarithm, product with the labels, sum, scaling, and the way
 // back through the same operations - is a chain of kernels on a few hundred values each.  Every one of them lasts as
 // long as a kernel boundary does (4-5 us between dependent kernels of one queue), whatever it computes.  Here a
-// single block of 256 threads walks the chain: node after node, each node's elements dealt over the threads, a
+// single block walks the chain: node after node, each node's elements dealt over the threads, a
 // workgroup barrier between nodes, every value in the buffer the plan gave its operation (so anything outside the run
 // that reads one finds it where it always was).
 //
