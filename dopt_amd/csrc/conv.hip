@@ -2952,13 +2952,14 @@ int gather_launch(GatherConv g, bool bwd, int K, int C, const float *in, const f
     g.in_bytes = (size_t)g.N * g.Cin * g.IH * g.IW * sizeof(float);
     g.out = splits > 1 ? partial : out;
     dim3 grid(xcd_grid((unsigned)(tiles * splits)));
-    // Short reductions that are not cut: in stages of one slab, two workgroups per CU, where there are two tiles per CU or a second
-    // slab would be half of the work.  1 x 1 on 128 images of 32 x 32, stages of two slabs -> of one: 16 -> 160 channels 37 -> 28 us,
-    // 112 -> 160 63 -> 53; 145 images of 29 x 25, 15 -> 7 14 -> 12; but 3 x 3 on 64 of 33 x 31, 16 -> 32, 256 tiles of nine slabs, 17 -> 19.  Beyond nine
-    // slabs only from four tiles per CU on, where reductions were not cut before either: without chains the error is that of
-    // the whole reduction (320 -> 320 196 -> 191 us, 480 -> 320, thirty slabs, 275 -> 266; but 42 -> 592, 3 x 3, 515 tiles of 27 slabs, 1.3 times as far off).
-    const int tiles_per_cu = tiles / num_cus();
-    const bool brief = splits == 1 && g.slabs_total <= (tiles_per_cu >= 4 ? 32 : tiles_per_cu >= 2 ? 9 : 3);
+    // Short reductions that are not cut: in stages of one slab, two workgroups per CU, where there are two tiles per CU, or more than
+    // one and a second slab would be half of the work.  1 x 1 on 128 images of 32 x 32, stages of two slabs -> of one: 16 -> 160 channels
+    // 37 -> 28 us, 112 -> 160 63 -> 53; 145 images of 29 x 25, 15 -> 7, 411 tiles, 14 -> 12; but 64 of 32 x 32, 16 -> 32, 256 tiles, 7.4 -> 8.7, and
+    // 3 x 3 on 64 of 33 x 31, 16 -> 32, 256 tiles of nine slabs, 17 -> 19.  Beyond nine slabs only from four tiles per CU on, where reductions
+    // were not cut before either: without chains the error is that of the whole reduction (320 -> 320 196 -> 191 us, 480 -> 320, thirty
+    // slabs, 275 -> 266; but 42 -> 592, 3 x 3, 515 tiles of 27 slabs, 1.3 times as far off).
+    const int cus = num_cus();
+    const bool brief = splits == 1 && g.slabs_total <= (tiles >= 4 * cus ? 32 : tiles >= 2 * cus ? 9 : tiles > cus ? 3 : 0);
     if (int rc = brief ? (wide ? launch_gather<GatherWide, 1>(bwd, g, grid) : launch_gather<GatherSquare, 1>(bwd, g, grid))
                        : (wide ? launch_gather<GatherWide, 2>(bwd, g, grid) : launch_gather<GatherSquare, 2>(bwd, g, grid)))
         return rc;

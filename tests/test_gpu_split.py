@@ -474,9 +474,11 @@ def test_general_convolution(shape):
     check_norm(dw, wants[1], dy[:, 0].size / 2, shape)
 
 
-# short reductions in stages of one slab: one slab, nine, many tiles of ten and of thirty-two; and one slab more than each, few tiles of ten
-@pytest.mark.parametrize("shape", [(5, 16, 31, 9, 70, 1, 0, 1), (2, 3, 17, 15, 130, 3, 1, 1), (64, 145, 32, 32, 250, 1, 0, 1), (64, 500, 33, 31, 250, 1, 0, 1),
-                                   (2, 145, 31, 9, 70, 1, 0, 1), (64, 520, 33, 31, 250, 1, 0, 1)])
+# either side of the lines between stages of one slab and of two: 411 tiles of one slab, 578 of nine, 1024 of ten and of thirty-two; 256 of one,
+# 411 of four, 578 of ten, 1024 of thirty-three, a few
+@pytest.mark.parametrize("shape", [(145, 7, 29, 25, 15, 1, 0, 1), (145, 16, 30, 34, 40, 3, 1, 1), (64, 145, 32, 32, 250, 1, 0, 1), (64, 500, 33, 31, 250, 1, 0, 1),
+                                   (64, 16, 32, 32, 32, 1, 0, 1), (145, 60, 29, 25, 50, 1, 0, 1), (145, 150, 30, 34, 150, 1, 0, 1), (64, 520, 33, 31, 250, 1, 0, 1),
+                                   (5, 16, 31, 9, 70, 1, 0, 1), (2, 3, 17, 15, 130, 3, 1, 1)])
 def test_general_convolution_of_short_reductions(shape):
     N, C, H, W, K, R, pad, stride = shape
     r = rng(C + K)
