@@ -361,6 +361,11 @@ def test_filter_gradient_of_small_images(shape):
     test_filter_gradient(shape)
 
 
+@pytest.mark.parametrize("shape", [(8, 64, 4, 4, 128), (256, 64, 4, 4, 64)])
+def test_filter_gradient_of_small_images_that_are_not_finite(shape):
+    test_filter_gradient_operands_that_are_not_finite(shape)
+
+
 def test_filter_gradient_without_a_split_takes_no_longer_than_with_one():
     """4 x 4 images, an odd and an even number of quads of filter values: one workgroup added the 35 chunks of the odd one, seven
     times as long."""
@@ -392,7 +397,8 @@ def test_filter_gradient_operands_that_are_not_finite(shape):
     assert np.all(np.abs(got[fine] - want[fine]) <= walk(N * H * W) * mag[fine])
 
 
-# an odd number of filter values, so one block adds all the pixels: 64-, 128- and 160-row tiles, every pixel geometry
+# an odd number of filter values, so one block adds all the pixels: 64-, 128- and 160-row tiles, every pixel geometry (64-row tiles on
+# 4 x 4 images: the general kernel, whose result can be split)
 @pytest.mark.parametrize("shape", [(32, 33, 16, 16, 65), (8, 33, 32, 32, 65), (128, 33, 8, 8, 65), (512, 17, 4, 4, 65), (32, 17, 16, 16, 255),
                                    (2, 17, 64, 64, 255), (512, 17, 4, 4, 255), (8, 17, 32, 32, 159), (128, 17, 8, 8, 159),
                                    (512, 17, 4, 4, 159)])
