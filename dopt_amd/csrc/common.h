@@ -27,6 +27,9 @@ bool is_initialised();   // dopt_hip_init (or a lazily initialising entry point)
 // cuda/nnet/cudnn7.d:111).  Valid until the next call that asks for more; all users enqueue on
 // the one library stream, so consecutive users never overlap.
 void *workspace(size_t bytes);
+// The same for callers that can do without: null, with no error recorded, where partial sums are parked in it (open_split_set) or
+// it would have to grow while a graph is recorded.
+void *workspace_if_free(size_t bytes);
 // Changes whenever a workspace is reallocated (its address may have changed): whoever keeps the
 // address beyond one call -- a recorded HIP graph -- compares generations before using it again.
 unsigned long workspace_generation();

@@ -487,6 +487,43 @@ extern "C" __global__ __launch_bounds__(BLOCK) void red_cols(const T *in, T *out
         out[idx] = acc;
     }
 }
+
+// The same for few columns of many rows, where red_cols would keep a handful of wavefronts busy one row after the other (HBM
+// latency times R / 8).  A block folds rows [s * rows_per, + rows_per) of `width` columns of one outer index: its threads are
+// blockDim / width rows side by side (consecutive threads, consecutive addresses where a row is one tile), each folds every
+// blockDim / width-th row, and the rows meet in LDS pairwise.  A slice's fold goes to out[(o * slices + s) * inner + j].
+// Bound by memory from a few MB on; sum of [17310, 17] over its rows 572 -> 6 us, of [7550, 786] 336 -> 9 us (both launches).
+extern "C" __global__ __launch_bounds__(1024) void red_cols_split(const T *in, T *out, size_t R, size_t inner, size_t rows_per,
+                                                                   unsigned width, unsigned tiles, unsigned slices)
+{
+    __shared__ T part[1024];
+    const unsigned tile = blockIdx.x % tiles, os = blockIdx.x / tiles, s = os % slices, o = os / slices;
+    const unsigned rows = blockDim.x / width, ty = threadIdx.x / width, tx = threadIdx.x - ty * width;
+    const size_t j = (size_t)tile * width + tx;
+    const bool mine = ty < rows && j < inner;
+    T acc = (T)(IDENT);
+    if (mine) {
+        const size_t r0 = (size_t)s * rows_per, r1 = r0 + rows_per < R ? r0 + rows_per : R;
+        const T *p = in + (size_t)o * R * inner + j;
+        size_t r = r0 + ty;
+        for (; r + 7 * rows < r1; r += 8 * rows) {
+            T v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = PRE(p[(r + u * rows) * inner]);
+#pragma unroll
+            for (int u = 0; u < 8; u++) acc = combine(acc, v[u]);
+        }
+        for (; r < r1; r += rows) acc = combine(acc, PRE(p[r * inner]));
+    }
+    part[threadIdx.x] = acc;
+    for (unsigned n = rows; n > 1;) {
+        const unsigned half = (n + 1) / 2;
+        __syncthreads();
+        if (mine && ty + half < n) part[threadIdx.x] = acc = combine(acc, part[threadIdx.x + half * width]);
+        n = half;
+    }
+    if (mine && ty == 0) out[(size_t)os * inner + j] = acc;
+}
 )SRC";
 
 const char *kArgminBody = R"SRC(
@@ -637,20 +674,21 @@ int check_dtype(int dtype)
 }
 
 // One (outer, R, inner) reduction pass on the device.
-// `rows_plain` adds the partial results of a split row: the first stage may fold PRE(element), the second never does.
+// `later` folds partial results: the first stage may fold PRE(element), the second never does.
 struct ReduceKernels {
-    hipFunction_t rows, rows4, rows4u, cols;
+    hipFunction_t rows, rows4, rows4u, cols, split;
 };
 int reduce_kernels(const std::string &key, bool is_sum, int dtype, bool square, ReduceKernels *k)
 {
     if (rtc_find(key + ":rows", &k->rows) && rtc_find(key + ":rows4", &k->rows4) && rtc_find(key + ":rows4u", &k->rows4u) &&
-        rtc_find(key + ":cols", &k->cols))
+        rtc_find(key + ":cols", &k->cols) && rtc_find(key + ":split", &k->split))
         return DOPT_HIP_OK;
     const std::string src = reduce_source(is_sum, dtype, square);
     if (int rc = rtc_get(key + ":rows", src, "red_rows", &k->rows)) return rc;
     if (int rc = rtc_get(key + ":rows4", src, "red_rows4", &k->rows4)) return rc;
     if (int rc = rtc_get(key + ":rows4u", src, "red_rows4u", &k->rows4u)) return rc;
-    return rtc_get(key + ":cols", src, "red_cols", &k->cols);
+    if (int rc = rtc_get(key + ":cols", src, "red_cols", &k->cols)) return rc;
+    return rtc_get(key + ":split", src, "red_cols_split", &k->split);
 }
 
 // How much of a contiguous row of R values one workgroup folds.
@@ -666,12 +704,53 @@ size_t row_chunk(size_t outer, size_t R)
     return (ceil_div(R, nchunks) + 1023) / 1024 * 1024;
 }
 
-int reduce_pass(const ReduceKernels &k, const void *in, void *out, size_t outer, size_t R, size_t inner, size_t esize,
-                hipFunction_t rows_plain = nullptr)
+// Folding [outer, R, inner] over R in slices of rows.  Worth it where a thread per column leaves the chip idle (fewer columns than
+// 256 threads on every CU) and is long enough at it: red_cols takes 20 to 40 ns a row, a launch of red_cols_split 3 to 4 us.
+// A tensor of up to 4096 values stays with red_cols, whose ascending order runs of tiny operations reproduce bit by bit.
+struct ColsSplit {
+    unsigned width, tiles, slices;
+    size_t rows_per;
+};
+bool cols_split(size_t outer, size_t R, size_t inner, ColsSplit *c)
 {
-    const hipFunction_t rows = k.rows, rows4 = k.rows4, cols = k.cols;
-    if (!rows_plain) rows_plain = rows;
+    if (inner < 2 || R <= 128 || outer * inner >= (size_t)num_cus() * 256 || outer * R * inner <= 4096) return false;
+    const size_t tiles = ceil_div(inner, (size_t)64);   // (fewer than 2^16 columns)
+    c->tiles = (unsigned)tiles;
+    c->width = (unsigned)ceil_div(inner, tiles);
+    // one launch while a thread has no more than 64 rows; else two blocks on every CU with at least 8 rows a thread, and no more
+    // slices than the launch that adds them folds in 16 rows a thread
+    const size_t side = 1024 / c->width;
+    size_t slices = 1;
+    if (R > side * 64) slices = std::min({ceil_div((size_t)num_cus() * 2, outer * tiles), ceil_div(R, side * 8), side * 16});
+    c->rows_per = ceil_div(R, slices);
+    c->slices = (unsigned)ceil_div(R, c->rows_per);
+    return true;
+}
+
+int reduce_pass(const ReduceKernels &k, const void *in, void *out, size_t outer, size_t R, size_t inner, size_t esize,
+                const ReduceKernels *later = nullptr)
+{
+    if (!later) later = &k;
+    const hipFunction_t rows = k.rows, rows4 = k.rows4, cols = k.cols, rows_plain = later->rows;
     if (outer * inner == 0) return DOPT_HIP_OK;
+    ColsSplit c;
+    if (cols_split(outer, R, inner, &c)) {
+        void *first = out;
+        if (c.slices > 1 && !(first = workspace_if_free(outer * c.slices * inner * esize))) {
+            first = out;
+            c.slices = 1;
+            c.rows_per = R;
+        }
+        void *args[] = {(void *)&in, (void *)&first, (void *)&R, (void *)&inner, (void *)&c.rows_per, (void *)&c.width, (void *)&c.tiles,
+                        (void *)&c.slices};
+        if (int rc = rtc_launch(k.split, (unsigned)(outer * c.slices * c.tiles), 1024, args)) return rc;
+        if (c.slices == 1) return DOPT_HIP_OK;
+        size_t r2 = c.slices;
+        unsigned one = 1;
+        void *args2[] = {(void *)&first, (void *)&out, (void *)&r2, (void *)&inner, (void *)&r2, (void *)&c.width, (void *)&c.tiles,
+                         (void *)&one};
+        return rtc_launch(later->split, (unsigned)(outer * c.tiles), 1024, args2);
+    }
     if (inner > 1 || R <= 64) {
         unsigned grid = grid_for(256, outer * inner);
         void *args[] = {(void *)&in, (void *)&out, (void *)&outer, (void *)&R, (void *)&inner};
@@ -985,7 +1064,7 @@ int reduce_impl(const char *op, int dtype, const size_t *shape, int rank, const 
             dst = tmp;
         }
         const bool first = square && ri == (int)runs.size() - 1;   // only what is read from `in` is squared
-        rc = first ? reduce_pass(squares, src_ptr, dst, outer, R, inner, 4, plain.rows)
+        rc = first ? reduce_pass(squares, src_ptr, dst, outer, R, inner, 4, &plain)
                    : reduce_pass(plain, src_ptr, dst, outer, R, inner, 4);
         if (tmp_prev) dopt_hip_free(tmp_prev);
         tmp_prev = tmp;

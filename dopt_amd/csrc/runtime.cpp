@@ -176,6 +176,14 @@ void *workspace(size_t bytes)
     return r.ws[l];
 }
 
+void *workspace_if_free(size_t bytes)
+{
+    Runtime &r = rt();
+    const int l = r.lane;
+    if (r.open_split[l][0] || r.open_split[l][1] || (r.capturing && bytes > r.ws_bytes[l])) return nullptr;
+    return workspace(bytes);
+}
+
 // ------------------------------------------------------------------------------- hipRTC
 
 static int rtc_compile(const std::string &source, const char *arch, std::vector<char> *code, std::string *log)

@@ -172,6 +172,34 @@ def test_sum_of_squares_is_the_sum_of_the_stored_product(shape, axes):
             assert np.array_equal(ops.sum(whole.view(1, shape), axes).numpy(), ops.sum(T(x), axes).numpy())
 
 
+@pytest.mark.parametrize("outer,rows,inner", [
+    (1, 129, 32), (1, 1000, 2), (3, 700, 17), (1, 1480, 11), (2, 2049, 64), (1, 1025, 65), (1, 20001, 3), (1, 17310, 17),
+    (1, 9000, 305), (2, 40000, 64), (1, 300, 65535), (1, 129, 65537), (5, 65, 200), (1, 4096, 1024)])
+def test_folds_of_few_columns_over_many_rows(outer, rows, inner):
+    """Sums and maxima over a middle or leading axis: one thread per column, a workgroup per tile of columns, or slices of rows
+    that a second launch adds.  Bound for sums: six standard deviations of 256 roundings (the longest chain) of partial sums that
+    are no larger than sqrt(rows); maxima and int32 sums are exact."""
+    r = rng(outer + rows + inner)
+    x = r.standard_normal((outer, rows, inner)).astype(np.float32)
+    want = x.astype(np.float64).sum(1)
+    got = ops.sum(T(x), [1]).numpy()
+    assert np.abs(got - want).max() <= 2.0 ** -24 * 6 * 16 * np.sqrt(rows)
+    assert np.array_equal(ops.max_element(T(x), [1]).numpy(), x.max(1))
+    squares = ops.sum_of_squares(T(x), [1]).numpy()
+    assert np.array_equal(squares, ops.sum(ops.pointwise("mul", T(x), T(x)), [1]).numpy())
+    nan = x.copy()
+    nan[:, ::3] = np.nan
+    nan[:, :, 0] = np.nan
+    assert np.array_equal(ops.max_element(T(nan), [1]).numpy(), O.max_element(nan, [1]))
+    xi = r.integers(-2**31, 2**31 - 1, x.shape).astype(np.int32)
+    with np.errstate(over="ignore"):
+        assert np.array_equal(ops.sum(T(xi), [1]).numpy(), xi.sum(1, dtype=np.int32))
+    assert np.array_equal(ops.max_element(T(xi), [1]).numpy(), xi.max(1))
+    if outer == 1 and inner <= 2000:   # the same values from a view off the 16-byte grid
+        whole = T(np.concatenate([[3.0], x.ravel()]).astype(np.float32))
+        assert np.array_equal(ops.sum(whole.view(1, x.shape), [1]).numpy(), got)
+
+
 def test_max_identity_is_minus_type_max():
     x = np.full((3, 5), -2**31, np.int32)
     assert np.array_equal(ops.max_element(T(x), (1,)).numpy(), O.max_element(x, (1,)))
