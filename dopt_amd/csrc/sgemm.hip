@@ -511,32 +511,41 @@ constexpr int kGroupJobs = 8;   // jobs one grouped launch may hold (its descrip
 
 // The lane's four reductions kk .. kk + 3 of row / column r.  `base`: byte offset of (r, reduction 0), or kOobOffset
 // when r lies outside the matrix; `pitch`: bytes between consecutive reductions of an r-contiguous operand.
-template <bool kKContig, bool kVec>
+// A k-contiguous operand is loaded as one 16-byte piece whatever its alignment (see Stage3): word by word, each load touched a
+// line per row, and [29 x 2146] x [2146 x 2424], B stored [2424][2146], took 49 us instead of 20.
+// kCut: the reduction is no multiple of four; what a piece holds past its end is zeroed.
+template <bool kKContig, bool kCut>
 __device__ __forceinline__ void small_load(__amdgpu_buffer_rsrc_t rs, unsigned base, unsigned pitch, int kk, int k_end,
                                            float (&v)[4])
 {
-    if (kKContig && kVec) {   // rows are whole quads: the end of the reduction never cuts one
+    if (kKContig) {
         const float4 q = buffer_load_f32x4(rs, kk < k_end ? base + (unsigned)kk * 4u : kOobOffset, 0);
         v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
     } else {
-        const unsigned step = kKContig ? 4u : pitch;
 #pragma unroll
-        for (int e = 0; e < 4; e++) v[e] = buffer_load_f32(rs, kk + e < k_end ? base + (unsigned)(kk + e) * step : kOobOffset, 0);
+        for (int e = 0; e < 4; e++) v[e] = buffer_load_f32(rs, kk + e < k_end ? base + (unsigned)(kk + e) * pitch : kOobOffset, 0);
     }
 }
 
-// kVA / kVB: the rows of a k-contiguous A / B are 16-byte addressable (an r-contiguous operand has no use for the flag).
-template <bool kTA, bool kTB, bool kVA, bool kVB>
+// What the last pieces of a k-contiguous operand hold past the end of the reduction counts as zero.
+template <bool kKContig, bool kCut>
+__device__ __forceinline__ float small_value(const float (&v)[4], int e, int kk, int k_end)
+{
+    return kKContig && kCut && e > 0 ? (kk + e < k_end ? v[e] : 0.0f) : v[e];
+}
+
+// kCut: a k-contiguous operand's rows are no whole quads.
+template <bool kTA, bool kTB, bool kCut>
 __device__ __forceinline__ void sgemm_small_body(int M, int N, int K, int lda, int ldb, int kslice, const float *A,
                                                  const float *B, float *C, const float *colbias, int bias_shift,
-                                                 const float *rowvec, int relu, const float *mask, int bx, int by,
+                                                 const float *rowvec, int relu, const float *mask, int bx, int by, int k0, int k1,
                                                  float (*red)[32 * 33])
 {
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, r = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // the same in every lane: loop bounds stay scalar
     const int m0 = by * 32, n0 = bx * 32;
     const int row = m0 + r, col = n0 + r;
-    const int k_begin = wave * kslice, k_end = min(K, k_begin + kslice);
+    const int k_begin = k0 + wave * kslice, k_end = min(k1, k_begin + kslice);   // the block's part of the reduction: [k0, k1)
     const __amdgpu_buffer_rsrc_t rsa = make_rsrc(A, (size_t)M * K * sizeof(float)), rsb = make_rsrc(B, (size_t)K * N * sizeof(float));
     // A is k-contiguous as given, B when it is read transposed
     const unsigned abase = row < M ? (kTA ? (unsigned)row * 4u : (unsigned)row * (unsigned)lda * 4u) : kOobOffset;
@@ -550,10 +559,12 @@ __device__ __forceinline__ void sgemm_small_body(int M, int N, int K, int lda, i
     const int nsteps = k_begin < k_end ? (k_end - k_begin + 7) / 8 : 0;
 #pragma unroll
     for (int j = 0; j < kSmallDepth; j++) {   // steps past the end fetch nothing
-        small_load<!kTA, kVA>(rsa, abase, apitch, k_begin + 8 * j + 4 * half, k_end, a[j]);
-        small_load<kTB, kVB>(rsb, bbase, bpitch, k_begin + 8 * j + 4 * half, k_end, b[j]);
+        small_load<!kTA, kCut>(rsa, abase, apitch, k_begin + 8 * j + 4 * half, k_end, a[j]);
+        small_load<kTB, kCut>(rsb, bbase, bpitch, k_begin + 8 * j + 4 * half, k_end, b[j]);
         __builtin_amdgcn_sched_barrier(0);   // in this order: the first step's operands are waited for first
     }
+    auto value_a = [&](int j, int s, int e) { return small_value<!kTA, kCut>(a[j], e, k_begin + 8 * (s + j) + 4 * half, k_end); };
+    auto value_b = [&](int j, int s, int e) { return small_value<kTB, kCut>(b[j], e, k_begin + 8 * (s + j) + 4 * half, k_end); };
     // Whole rounds of kSmallDepth steps without a branch inside (a branch per step made the compiler wait for every
     // load in flight at the top of the loop), then the steps left over, whose operands are in their registers or on
     // their way already.
@@ -562,10 +573,10 @@ __device__ __forceinline__ void sgemm_small_body(int M, int N, int K, int lda, i
 #pragma unroll
         for (int j = 0; j < kSmallDepth; j++) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j][e], b[j][e], acc, 0, 0, 0);
+            for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(value_a(j, s, e), value_b(j, s, e), acc, 0, 0, 0);
             const int kk = k_begin + 8 * (s + j + kSmallDepth) + 4 * half;   // this register set's next step
-            small_load<!kTA, kVA>(rsa, abase, apitch, kk, k_end, a[j]);
-            small_load<kTB, kVB>(rsb, bbase, bpitch, kk, k_end, b[j]);
+            small_load<!kTA, kCut>(rsa, abase, apitch, kk, k_end, a[j]);
+            small_load<kTB, kCut>(rsb, bbase, bpitch, kk, k_end, b[j]);
             __builtin_amdgcn_sched_barrier(0);   // keep each refill behind its own step: sunk to the loop's end, all of them are waited for at once
         }
     }
@@ -573,7 +584,7 @@ __device__ __forceinline__ void sgemm_small_body(int M, int N, int K, int lda, i
     for (int j = 0; j < kSmallDepth - 1; j++)
         if (whole + j < nsteps) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j][e], b[j][e], acc, 0, 0, 0);
+            for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(value_a(j, whole, e), value_b(j, whole, e), acc, 0, 0, 0);
         }
 #pragma unroll
     for (int v = 0; v < 16; v++) red[wave][acc_row(v, lane) * 33 + r] = acc[v];
@@ -597,15 +608,17 @@ __device__ __forceinline__ void sgemm_small_body(int M, int N, int K, int lda, i
     }
 }
 
-template <bool kTA, bool kTB, bool kVA, bool kVB>
+// blockIdx.z: the part of the reduction (8 kslice steps each); the parts' sums go to consecutive copies of C.
+template <bool kTA, bool kTB, bool kCut>
 __global__ __launch_bounds__(64 * kSmallWaves) void sgemm_small_k(int M, int N, int K, int lda, int ldb, int kslice,
                                                                    const float *A, const float *B, float *C,
                                                                    const float *colbias, int bias_shift,
                                                                    const float *rowvec, int relu, const float *mask)
 {
     __shared__ float red[kSmallWaves][32 * 33];
-    sgemm_small_body<kTA, kTB, kVA, kVB>(M, N, K, lda, ldb, kslice, A, B, C, colbias, bias_shift, rowvec, relu, mask,
-                                         (int)blockIdx.x, (int)blockIdx.y, red);
+    const int k0 = (int)blockIdx.z * kSmallWaves * kslice;
+    sgemm_small_body<kTA, kTB, kCut>(M, N, K, lda, ldb, kslice, A, B, C + (size_t)blockIdx.z * M * N, colbias, bias_shift, rowvec, relu,
+                                     mask, (int)blockIdx.x, (int)blockIdx.y, k0, min(K, k0 + kSmallWaves * kslice), red);
 }
 
 // Short reductions over large outputs with both operands stored k-major (A as [K][M], B as [K][N]:
@@ -763,6 +776,32 @@ __global__ __launch_bounds__(256) void splitk_reduce_k(size_t n, int splits, con
     }
 }
 
+// ... and the epilogue of sgemm_small_k behind it.
+__global__ __launch_bounds__(256) void splitk_epilogue_k(size_t M, size_t N, int splits, const float *partial, float *out,
+                                                          const float *colbias, int bias_shift, const float *rowvec, int relu,
+                                                          const float *mask)
+{
+    const size_t n = M * N;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        float acc = 0.f;
+        const int last = splits - 1;
+        for (int s = 0; s < splits; s += 4) {
+            const float v0 = partial[(size_t)s * n + i], v1 = partial[(size_t)min(s + 1, last) * n + i];
+            const float v2 = partial[(size_t)min(s + 2, last) * n + i], v3 = partial[(size_t)min(s + 3, last) * n + i];
+            acc = (((acc + v0) + (s + 1 <= last ? v1 : 0.f)) + (s + 2 <= last ? v2 : 0.f)) + (s + 3 <= last ? v3 : 0.f);
+        }
+        if (colbias) {
+            const size_t row = i / N, col = i - row * N;
+            float add = colbias[col >> bias_shift];
+            if (rowvec) add = __fmul_rn(rowvec[row], add);
+            acc += add;
+        }
+        if (relu) acc = acc < 0.0f ? 0.0f : acc;
+        if (mask) acc = mask[i] > 0.0f ? acc : 0.0f;
+        out[i] = acc;
+    }
+}
+
 // K == 1: C[m][n] = a[m] * b[n] -- the broadcast product.  One rounding per element, so a
 // product with 1.0f reproduces the broadcast value exactly.
 __global__ __launch_bounds__(256) void outer_k(size_t M, size_t N, const float *a, const float *b, float *c)
@@ -858,7 +897,7 @@ struct SmallGroup {
     int ns, nv;
 };
 
-template <bool kTA, bool kTB, bool kVA, bool kVB>
+template <bool kTA, bool kTB, bool kCut>
 __global__ __launch_bounds__(64 * kSmallWaves) void sgemm_small_group_k(SmallGroup g)
 {
     __shared__ float red[kSmallWaves][32 * 33];
@@ -875,8 +914,8 @@ __global__ __launch_bounds__(64 * kSmallWaves) void sgemm_small_group_k(SmallGro
     while (j + 1 < g.ns && b >= g.s[j + 1].first) j++;
     const SmallJob &q = g.s[j];
     const int local = b - q.first;
-    sgemm_small_body<kTA, kTB, kVA, kVB>(q.M, q.N, q.K, q.lda, q.ldb, q.kslice, q.A, q.B, q.C, nullptr, 0, nullptr, 0, nullptr,
-                                         local % q.nx, local / q.nx, red);
+    sgemm_small_body<kTA, kTB, kCut>(q.M, q.N, q.K, q.lda, q.ldb, q.kslice, q.A, q.B, q.C, nullptr, 0, nullptr, 0, nullptr,
+                                     local % q.nx, local / q.nx, 0, q.K, red);
 }
 
 // c[m][n] = relu?(c[m][n] + u[m] * v[n]): the epilogue of dopt_hip_sgemm_rank1 as a pass of its own, for the
@@ -899,6 +938,9 @@ unsigned flat_grid(size_t n)
     size_t cap = (size_t)num_cus() * 16;
     return (unsigned)(blocks < 1 ? 1 : (blocks > cap ? cap : blocks));
 }
+
+// Steps of the reduction per wavefront of a 32 x 32-tile block that takes `depth` of them.
+size_t small_slice(size_t depth) { return ceil_div(ceil_div(depth, (size_t)kSmallWaves), (size_t)8) * 8; }
 
 // The LDS-resident kernel is taken where its 128 x 128 tiles give every CU one or two blocks and the operands take 128-bit loads.
 // Against what those shapes take without it (an operand off the 16-byte grid): 2048 x 2048 x 64 11 and 18 us, 1024 x 4096 x
@@ -1025,6 +1067,29 @@ struct RowsShape {
 };
 constexpr RowsShape kRowsShapes[] = {{256, 256, 2.4}, {128, 256, 1.45}, {256, 128, 1.45}, {128, 128, 0.93}};
 
+// How many blocks share the reduction of a 32 x 32 tile: a few tiles over a long reduction leave most of the chip idle (a block
+// takes 5.5 ns per step whatever runs beside it).  Another launch adds the parts.  [61 x 41] from 3673 steps: 21 us uncut, 8.6 in 29
+// parts; [16 x 132] from 944 6.7 us uncut, 8.1 in eight.  The parts take no more space than the operands.
+// `us`: what has to be undercut; `longest`: steps of a part.
+Route small_cuts(size_t M, size_t N, size_t K, size_t tiles, double traffic_us, double us, size_t longest = ~(size_t)0)
+{
+    Route r{Route::kSmall, 1, K, 0, 0, 0};
+    const unsigned slots = 2 * (unsigned)num_cus(), k = (unsigned)K, t = (unsigned)tiles;
+    const double copy_us = 8.0 * M * N / 5e6;
+    for (unsigned cuts = 2; cuts <= 32; cuts++) {
+        const unsigned depth = ((k + cuts - 1) / cuts + 63) / 64 * 64;
+        if (depth < 128 || cuts * M * N > M * K + K * N) break;
+        if (depth > longest || (k + depth - 1) / depth != cuts) continue;
+        const unsigned rounds = (t * cuts + slots - 1) / slots;
+        const double cost = 9.5 + std::max(traffic_us, 5.5e-3 * depth * rounds) + copy_us * cuts;
+        if (cost >= us) continue;
+        us = cost;
+        r.cuts = cuts;
+        r.depth = depth;
+    }
+    return r;
+}
+
 Route sgemm_route(int transA, int transB, size_t M, size_t N, size_t K, bool panel_allowed = true)
 {
     Route r{Route::kNone, 1, K, 0, 0, 0};
@@ -1051,16 +1116,17 @@ Route sgemm_route(int transA, int transB, size_t M, size_t N, size_t K, bool pan
     // small and medium outputs: one block per 32 x 32 tile, the reduction split over its wavefronts.
     // Each tile reads its own 32 rows of A and 32 columns of B, so the operand traffic grows with the
     // number of tiles; it is served by the L2 at about 10 TB/s (1024 x 1024 x 256: 12 us against 20 us with the kernel
-    // below).  A block by itself takes 5.5 ns per reduction step (256 x 256 x 8192: 49 against 28 us), twice that when rows
-    // of a k-contiguous operand start off the 16-byte grid (1700 x 1501 x 333: 69 against 29 us).
+    // below), at half that when rows of a k-contiguous operand start off the 16-byte grid (91 x 1900 x 4674: 56 against 32 us).
+    // A block by itself takes 5.5 ns per reduction step (256 x 256 x 8192: 49 against 28 us).
     const bool offsets32 = M * K < ((size_t)1 << 29) && K * N < ((size_t)1 << 29);
     const size_t tiles32 = ceil_div(M, (size_t)32) * ceil_div(N, (size_t)32);
     const double traffic = (double)tiles32 * 64 * K * sizeof(float);
     const bool small = offsets32 && tiles32 <= 4096 && traffic <= (double)(256 << 20);   // (32-bit byte offsets)
-    const double small_us = 4 + (K % 4 ? 2 : 1) * (traffic / 10e6 > 5.5e-3 * K ? traffic / 10e6 : 5.5e-3 * K);
+    const double traffic_us = traffic / (K % 4 ? 4.5e6 : 10e6);
+    const double small_us = 4 + (K % 4 ? 2 : 1) * std::max(traffic / 10e6, 5.5e-3 * K);
     const size_t slabs_total = ceil_div(K, (size_t)BK);
     if (M <= 64 || !offsets32) {
-        if (small) { r.kind = Route::kSmall; return r; }
+        if (small) return small_cuts(M, N, K, tiles32, traffic_us, small_us);
         r.kind = M <= 64 ? Route::kTile64 : Route::kTile128;
         r.bm = M <= 64 ? 64 : 128;
         r.bn = M <= 64 ? 256 : 128;
@@ -1114,7 +1180,13 @@ Route sgemm_route(int transA, int transB, size_t M, size_t N, size_t K, bool pan
             }
         }
     }
-    if (small && small_us < best) r = Route{Route::kSmall, 1, K, 0, 0, 0};
+    if (small && small_us < best) return small_cuts(M, N, K, tiles32, traffic_us, small_us);
+    // Else the 32 x 32 tiles only where the reduction is cut into parts whose sums are as close as sgemm_rows_k's: 506 x 36 from 1127
+    // steps 13 us and 1.2e-7 off float64; in parts of 256 steps 8 us and 1.2e-7; uncut 9 us and 2.2e-7.
+    if (small) {
+        const Route cut = small_cuts(M, N, K, tiles32, traffic_us, best, 256);
+        if (cut.cuts > 1) return cut;
+    }
     return r;
 }
 
@@ -1176,24 +1248,29 @@ int sgemm_epilogue(int transA, int transB, size_t M, size_t N, size_t K, const f
     if (kind == Route::kPanel) return panel_launch(false, M, N, K, A, B, C);
     if (kind == Route::kSmall) {
         const int lda = (int)(transA ? M : K), ldb = (int)(transB ? K : N);
-        int kslice = (int)ceil_div(ceil_div(K, (size_t)kSmallWaves), (size_t)8) * 8;
-        // 128-bit loads for a k-contiguous operand whose rows start on 16-byte boundaries
-        const bool va = !transA && aligned16(A) && lda % 4 == 0, vb = transB && aligned16(B) && ldb % 4 == 0;
-        const dim3 grid((unsigned)ceil_div(N, (size_t)32), (unsigned)ceil_div(M, (size_t)32)), block(64 * kSmallWaves);
-#define DOPT_SMALL(TA, TB, VA, VB)                                                                                       \
-    hipLaunchKernelGGL((sgemm_small_k<TA, TB, VA, VB>), grid, block, 0, stream(), (int)M, (int)N, (int)K, lda, ldb, kslice, \
-                       A, B, C, colbias, bias_shift, rowvec, relu, ex.mask)
-        if (transA && transB) { if (vb) DOPT_SMALL(true, true, false, true); else DOPT_SMALL(true, true, false, false); }
-        else if (transA) DOPT_SMALL(true, false, false, false);
-        else if (transB) {
-            if (va && vb) DOPT_SMALL(false, true, true, true);
-            else if (va) DOPT_SMALL(false, true, true, false);
-            else if (vb) DOPT_SMALL(false, true, false, true);
-            else DOPT_SMALL(false, true, false, false);
-        } else { if (va) DOPT_SMALL(false, false, true, false); else DOPT_SMALL(false, false, false, false); }
+        const size_t cuts = route.cuts;
+        const int kslice = (int)small_slice(route.depth);
+        float *to = C;
+        if (cuts > 1 && !(to = (float *)workspace(cuts * M * N * sizeof(float)))) return DOPT_HIP_ERR_OOM;
+        const bool fused = cuts == 1;   // the epilogue runs behind the last sum
+        const dim3 grid((unsigned)ceil_div(N, (size_t)32), (unsigned)ceil_div(M, (size_t)32), (unsigned)cuts), block(64 * kSmallWaves);
+#define DOPT_SMALL(TA, TB, CUT)                                                                                          \
+    hipLaunchKernelGGL((sgemm_small_k<TA, TB, CUT>), grid, block, 0, stream(), (int)M, (int)N, (int)K, lda, ldb, kslice, \
+                       A, B, to, fused ? colbias : nullptr, bias_shift, fused ? rowvec : nullptr, fused ? relu : 0,      \
+                       fused ? ex.mask : nullptr)
+        const bool cut = K % 4 != 0;
+        if (transA && transB) { if (cut) DOPT_SMALL(true, true, true); else DOPT_SMALL(true, true, false); }
+        else if (transA) DOPT_SMALL(true, false, false);   // nothing k-contiguous to cut
+        else if (transB) { if (cut) DOPT_SMALL(false, true, true); else DOPT_SMALL(false, true, false); }
+        else { if (cut) DOPT_SMALL(false, false, true); else DOPT_SMALL(false, false, false); }
 #undef DOPT_SMALL
         DOPT_LAUNCH_CHECK();
-        *biased = true;   // whatever epilogue was asked for (the extras included), this kernel applied it
+        if (!fused) {
+            hipLaunchKernelGGL(splitk_epilogue_k, dim3(flat_grid(M * N)), dim3(256), 0, stream(), M, N, (int)cuts, to, C, colbias,
+                               bias_shift, rowvec, relu, ex.mask);
+            DOPT_LAUNCH_CHECK();
+        }
+        *biased = true;   // whatever epilogue was asked for (the extras included), it has been applied
         return DOPT_HIP_OK;
     }
 
@@ -1298,7 +1375,7 @@ int dopt_hip_sgemm_batch(int n, const int *transA, const int *transB, const size
     DOPT_ENSURE_INIT();
     // Products that take the 32 x 32-tile kernel (grouped per template instance) or the short column sum share launches;
     // the others run one by one.  Outputs must not overlap any operand of the batch: the order inside it is not kept.
-    struct Inst { bool ta, tb, va, vb; SmallGroup g; unsigned blocks; bool used; };
+    struct Inst { bool ta, tb, cut; SmallGroup g; unsigned blocks; bool used; };
     std::vector<Inst> insts;
     std::vector<GemvJob> gemvs;
     std::vector<int> single;
@@ -1314,22 +1391,19 @@ int dopt_hip_sgemm_batch(int n, const int *transA, const int *transB, const size
             q.B = M[i] == 1 ? B[i] : A[i];
             q.c = C[i];
             gemvs.push_back(q);
-        } else if (r.kind == Route::kSmall) {
+        } else if (r.kind == Route::kSmall && r.cuts == 1) {
             const int lda = (int)(transA[i] ? M[i] : K[i]), ldb = (int)(transB[i] ? K[i] : N[i]);
-            const bool ta = transA[i] != 0, tb = transB[i] != 0;
-            const bool va = !ta && aligned16(A[i]) && lda % 4 == 0, vb = tb && aligned16(B[i]) && ldb % 4 == 0;
-            // the instance the product would take alone (flags an instance does not read are false there)
-            const bool iva = ta ? false : va, ivb = tb ? vb : false;
+            const bool ta = transA[i] != 0, tb = transB[i] != 0, cut = K[i] % 4 != 0 && (!ta || tb);   // the instance the product would take alone
             Inst *in = nullptr;
             for (Inst &c : insts)
-                if (c.ta == ta && c.tb == tb && c.va == iva && c.vb == ivb && c.g.ns < kGroupJobs) in = &c;
+                if (c.ta == ta && c.tb == tb && c.cut == cut && c.g.ns < kGroupJobs) in = &c;
             if (!in) {
-                insts.push_back(Inst{ta, tb, iva, ivb, SmallGroup{}, 0, false});
+                insts.push_back(Inst{ta, tb, cut, SmallGroup{}, 0, false});
                 in = &insts.back();
             }
             SmallJob &q = in->g.s[in->g.ns++];
             q.M = (int)M[i]; q.N = (int)N[i]; q.K = (int)K[i]; q.lda = lda; q.ldb = ldb;
-            q.kslice = (int)ceil_div(ceil_div(K[i], (size_t)kSmallWaves), (size_t)8) * 8;
+            q.kslice = (int)small_slice(K[i]);
             q.nx = (int)ceil_div(N[i], (size_t)32);
             q.first = (int)in->blocks;
             q.A = A[i]; q.B = B[i]; q.C = C[i];
@@ -1350,15 +1424,11 @@ int dopt_hip_sgemm_batch(int n, const int *transA, const int *transB, const size
             gemvs.clear();
         }
         const dim3 grid(in.blocks), block(64 * kSmallWaves);
-#define DOPT_GROUP(TA, TB, VA, VB) hipLaunchKernelGGL((sgemm_small_group_k<TA, TB, VA, VB>), grid, block, 0, stream(), in.g)
-        if (in.ta && in.tb) { if (in.vb) DOPT_GROUP(true, true, false, true); else DOPT_GROUP(true, true, false, false); }
-        else if (in.ta) DOPT_GROUP(true, false, false, false);
-        else if (in.tb) {
-            if (in.va && in.vb) DOPT_GROUP(false, true, true, true);
-            else if (in.va) DOPT_GROUP(false, true, true, false);
-            else if (in.vb) DOPT_GROUP(false, true, false, true);
-            else DOPT_GROUP(false, true, false, false);
-        } else { if (in.va) DOPT_GROUP(false, false, true, false); else DOPT_GROUP(false, false, false, false); }
+#define DOPT_GROUP(TA, TB, CUT) hipLaunchKernelGGL((sgemm_small_group_k<TA, TB, CUT>), grid, block, 0, stream(), in.g)
+        if (in.ta && in.tb) { if (in.cut) DOPT_GROUP(true, true, true); else DOPT_GROUP(true, true, false); }
+        else if (in.ta) DOPT_GROUP(true, false, false);
+        else if (in.tb) { if (in.cut) DOPT_GROUP(false, true, true); else DOPT_GROUP(false, true, false); }
+        else { if (in.cut) DOPT_GROUP(false, false, true); else DOPT_GROUP(false, false, false); }
 #undef DOPT_GROUP
         DOPT_LAUNCH_CHECK();
     }

@@ -919,6 +919,36 @@ def test_sgemm_large_products_all_operand_layouts(shape):
             assert np.array_equal(got, plain), (ta, tb, "unaligned")
 
 
+@pytest.mark.parametrize("shape", [(41, 375, 4819), (16, 23, 2000), (64, 33, 1283), (1000, 2, 1601), (32, 32, 4095), (20, 696, 3029),
+                                   (506, 36, 1127), (65, 31, 8190), (29, 2424, 2146), (7, 5, 1537)])
+def test_products_of_few_tiles_cut_their_reduction(shape):
+    """32 x 32 tiles whose reduction is shared by several workgroups: every way of storing the operands, on and off the 16-byte
+    grid, with the epilogues behind the last sum.  Bound: six standard deviations of 64 roundings (a chain in a wavefront, the
+    wavefronts, the parts) of partial sums no larger than sqrt(K)."""
+    M, N, K = shape
+    r = rng(M + N + K)
+    a, b = r.standard_normal((M, K)).astype(np.float32), r.standard_normal((K, N)).astype(np.float32)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    tol = 2.0 ** -24 * 6 * 8 * np.sqrt(K)
+    from dopt_amd import capi
+    ta_, tb_ = np.ascontiguousarray(a.T), np.ascontiguousarray(b.T)
+    u, v = r.standard_normal(M).astype(np.float32), r.standard_normal(N).astype(np.float32)
+    mask = r.standard_normal((M, N)).astype(np.float32)
+    for ta in (0, 1):
+        for tb in (0, 1):
+            A, B = T(ta_ if ta else a), T(tb_ if tb else b)
+            got = ops.matmul_t(A, B, trans_a=bool(ta), trans_b=bool(tb)).numpy()
+            assert np.abs(got - want).max() <= tol, (ta, tb)
+            la, lb = T(np.concatenate([[9.0], (ta_ if ta else a).ravel()]).astype(np.float32)), T(np.concatenate([[9.0] * 3, (tb_ if tb else b).ravel()]).astype(np.float32))
+            loose = ops.matmul_t(la.view(1, (K, M) if ta else (M, K)), lb.view(3, (N, K) if tb else (K, N)), trans_a=bool(ta), trans_b=bool(tb)).numpy()
+            assert np.array_equal(loose, got), (ta, tb)
+            f = np.maximum(got + (u[:, None] * v[None, :]).astype(np.float32), np.float32(0))
+            assert np.array_equal(ops.matmul_rank1(A, B, T(u), T(v), relu=True, trans_a=bool(ta), trans_b=bool(tb)).numpy(), f)
+            g, x = ops.Tensor((M, N)), T(mask)
+            capi.check(capi.load().dopt_hip_sgemm_relu_grad(ta, tb, M, N, K, A.ptr, B.ptr, x.ptr, g.ptr))
+            assert np.array_equal(g.numpy(), np.where(mask > 0, got, np.float32(0)))
+
+
 @pytest.mark.parametrize("shape", [(12, 32768, 32), (32768, 12, 16), (12, 32768, 100), (64, 8192, 512), (8192, 64, 512),
                                    (33, 70000, 40), (70000, 33, 40), (128, 2048, 2048), (2048, 128, 2048),
                                    (256, 256, 8192), (1, 3000, 77), (3000, 1, 77), (1, 5000, 700), (5000, 1, 700),
