@@ -22,6 +22,7 @@
 #include <cstring>
 #include <functional>
 #include <set>
+#include <unordered_set>
 
 #include "../../include/dopt_hip_plan.h"
 
@@ -647,7 +648,7 @@ struct HIPPlan::Builder {
     bool plainProduct(int id, MatmulInfo *mi, bool sole_reader) const;
     void formGroups();
     void formTinyRuns();
-    void fuseSquareSums();
+    void fuseSquareSums(bool many);
     void formChains();
     void absorbBiasGrads();
     void absorbPools();
@@ -1222,7 +1223,8 @@ void HIPPlan::Builder::formTinyRuns()
     // what a member is to the kernel; false when it cannot be one
     auto describe = [&](int id, dopt_hip_tiny_node *nd, int (&operands)[2]) -> bool {
         const Operation &o = g.ops[id];
-        if (!live[id] || alias[id].source >= 0 || fusedKind[id] || prebuilt[id] || !small_f32(id)) return false;
+        const bool product = fusedKind[id] == 6 && o.opType == "matmul" && mmInfo[id].valid;   // one that reads its operands through transposes
+        if (!live[id] || alias[id].source >= 0 || (!product && (fusedKind[id] || prebuilt[id])) || !small_f32(id)) return false;
         if (!read[id]) return false;
         for (int d : o.deps)
             if (!small_f32(d)) return false;
@@ -1240,16 +1242,26 @@ void HIPPlan::Builder::formTinyRuns()
             operands[1] = o.deps[2];
             return true;
         }
-        if (o.opType == "matmul" && o.deps.size() == 2 && o.rank() == 2) {   // [m,1] x [1,n]: a column times a row
+        if (o.opType == "matmul" && o.deps.size() == 2 && o.rank() == 2) {
             const Operation &l = g.ops[o.deps[0]], &r = g.ops[o.deps[1]];
-            if (l.rank() != 2 || r.rank() != 2 || l.shape[1] != 1 || r.shape[0] != 1) return false;
-            nd->kind = DOPT_HIP_TINY_POINTWISE;
-            nd->op = dopt_hip_pointwise_index("mul");
-            nd->a_kind = 2;
-            nd->b_kind = 3;
-            nd->dims[0] = (int)o.shape[1];
-            operands[0] = o.deps[0];
-            operands[1] = o.deps[1];
+            if (l.rank() != 2 || r.rank() != 2) return false;
+            const MatmulInfo &mi = mmInfo[id];   // as it runs: a transposed vector is the same memory
+            const bool folded = fusedKind[id] == 6;
+            const size_t K = folded ? mi.K : l.shape[1], M = folded ? mi.M : o.shape[0], N = folded ? mi.N : o.shape[1];
+            if (M * N != o.volume() || (folded && (!small_f32(mi.a) || !small_f32(mi.b)))) return false;
+            operands[0] = folded ? mi.a : o.deps[0];
+            operands[1] = folded ? mi.b : o.deps[1];
+            if (K == 1) {   // [m,1] x [1,n]: a column times a row
+                nd->kind = DOPT_HIP_TINY_POINTWISE;
+                nd->op = dopt_hip_pointwise_index("mul");
+                nd->a_kind = 2;
+                nd->b_kind = 3;
+                nd->dims[0] = (int)N;
+                return true;
+            }
+            if (N != 1 || K < 2 || (folded && mi.tA)) return false;
+            nd->kind = DOPT_HIP_TINY_MATVEC;   // [m,k] x [k,1]: the rows' weighted sums
+            nd->dims[0] = (int)K;
             return true;
         }
         const int arity = o.opType == "relu" ? 1 : dopt_hip_pointwise_arity(o.opType.c_str());
@@ -1272,11 +1284,21 @@ void HIPPlan::Builder::formTinyRuns()
                 if (a >= sh.size() || red[a]) return false;
                 red[a] = 1;
             }
-            size_t first = sh.size(), last = 0;
-            for (size_t i = 0; i < sh.size(); i++)
-                if (red[i]) { first = std::min(first, i); last = i; }
-            for (size_t i = first; i <= last; i++)
-                if (!red[i]) return false;   // more than one run of reduced axes: passes with a temporary in between
+            // one run of reduced axes (several are passes with a temporary in between), or one beside axes of extent one; a sum
+            // around a kept middle has a kernel of its own
+            size_t runs = 0, first = sh.size(), last = 0;
+            bool one = true;
+            for (size_t i = 0; i < sh.size(); i++) runs += red[i] && (i == 0 || !red[i - 1]);
+            if (runs == 2 && red[0] && red[sh.size() - 1]) return false;
+            for (int pass = 0; pass < 2 && first == sh.size(); pass++)
+                for (size_t i = 0; i < sh.size(); i++)
+                    if (red[i] && (pass == 1 || runs == 1 || sh[i] != 1)) {
+                        first = std::min(first, i);
+                        last = i;
+                        if (pass == 1) break;   // nothing but extents of one
+                    }
+            for (size_t i = first; i <= last; i++) one = one && red[i];
+            if (!one) return false;
             size_t outer = 1, R = 1, inner = 1;
             for (size_t i = 0; i < first; i++) outer *= sh[i];
             for (size_t i = first; i <= last; i++) R *= sh[i];
@@ -1319,6 +1341,7 @@ void HIPPlan::Builder::formTinyRuns()
     struct Member { int op; dopt_hip_tiny_node nd; int operands[2]; };
     std::vector<Member> run;
     std::vector<char> inRun((size_t)nops, 0);
+    std::unordered_set<int> named;   // the buffers that the run's members read or write
     auto close = [&]() {
         if (run.size() >= 2) {
             // buffers: the members' own, and whatever else they read (by owner of the buffer, with the byte offset in the node)
@@ -1348,6 +1371,8 @@ void HIPPlan::Builder::formTinyRuns()
                 const int last = run.back().op;
                 for (const Member &m : run) {
                     fusedKind[m.op] = 10;
+                    prebuilt[m.op].reset();
+                    prebuiltLabel[m.op].clear();
                     if (m.op != last) absorbed[m.op] = 1;   // keeps its buffer, filled by the run's kernel
                 }
                 // every buffer is an input of the step (the members' too: that is what keeps them allocated), except the
@@ -1374,13 +1399,29 @@ void HIPPlan::Builder::formTinyRuns()
         }
         for (const Member &m : run) inRun[m.op] = 0;
         run.clear();
+        named.clear();
     };
     for (int id : p->mOps) {
         if (!live[id]) continue;
         Member m{};
         m.op = id;
         if (describe(id, &m.nd, m.operands)) {
-            if (run.size() >= (size_t)DOPT_HIP_TINY_NODES || run.size() * 3 + 3 > (size_t)DOPT_HIP_TINY_SLOTS) close();
+            std::vector<int> more;   // buffers that the run does not name yet
+            auto names = [&]() {
+                more.assign(1, id);
+                for (int op : m.operands) {
+                    if (op < 0) continue;
+                    size_t off;
+                    const int owner = root(op, &off);
+                    if (!named.count(owner) && std::find(more.begin(), more.end(), owner) == more.end()) more.push_back(owner);
+                }
+            };
+            names();
+            if (run.size() >= (size_t)DOPT_HIP_TINY_NODES || named.size() + more.size() > (size_t)DOPT_HIP_TINY_SLOTS) {
+                close();
+                names();
+            }
+            named.insert(more.begin(), more.end());
             run.push_back(m);
             inRun[id] = 1;
             continue;
@@ -1403,7 +1444,9 @@ void HIPPlan::Builder::formTinyRuns()
 // been taken by one already (DOPT_HIP_PLAN_FUSE).
 // The penalties of a whole network are one step (reduce_squares_batch) where the first of them stood: they read variables and
 // constants, which no step writes.
-void HIPPlan::Builder::fuseSquareSums()
+// Called once before the tiny runs are formed, for the step of a whole network (`many`: small tensors too, whose squares and sums
+// would be two nodes of a run each, one after the other: 18 us for eight of them), and once behind, for what is left.
+void HIPPlan::Builder::fuseSquareSums(bool many)
 {
     std::vector<int> whole;   // such sums over whole variables or constants
     for (int id : p->mOps) {
@@ -1433,6 +1476,11 @@ void HIPPlan::Builder::fuseSquareSums()
         for (size_t i = 0; valid && i < shape.size(); i++)
             if (red[i] && (i == 0 || !red[i - 1])) runs++;
         if (!valid || runs != 1) continue;
+        if (many) {
+            size_t xoff;
+            if (op.volume() == 1 && mo.volume() > 64 && mo.volume() < (size_t)1 << 40 && is_leaf(g.ops[root(mo.deps[0], &xoff)])) whole.push_back(id);
+            continue;
+        }
         fusedKind[id] = 11;
         inputsOf[id] = {mo.deps[0]};
         prebuilt[id] = make([=](const std::vector<const void *> &in, void *out) {
@@ -1440,23 +1488,26 @@ void HIPPlan::Builder::fuseSquareSums()
                                            (float *)out);
         });
         prebuiltLabel[id] = "mul+sum";
-        size_t xoff;
-        if (op.volume() == 1 && mo.volume() > 64 && mo.volume() < (size_t)1 << 40 && is_leaf(g.ops[root(mo.deps[0], &xoff)])) whole.push_back(id);
     }
-    if (whole.size() < 3) return;   // a pair stays two steps, which a profile tells apart
+    if (std::count_if(whole.begin(), whole.end(), [&](int id) {
+            size_t off;
+            return g.ops[root(g.ops[id].deps[0], &off)].volume() > DOPT_HIP_TINY_ELEMS;
+        }) < 3)
+        return;   // a pair stays two steps, which a profile tells apart, and small ones are nodes of a run
     const int lead = whole[0];
     std::vector<int> ins;
     std::vector<size_t> counts;
     for (int id : whole) {
-        ins.push_back(inputsOf[id][0]);
-        counts.push_back(g.ops[inputsOf[id][0]].volume());
+        size_t off;
+        const int squared = g.ops[root(g.ops[id].deps[0], &off)].deps[0];
+        fusedKind[id] = 11;
+        ins.push_back(squared);
+        counts.push_back(g.ops[squared].volume());
     }
     tinyWrites[lead].assign(whole.begin() + 1, whole.end());
     for (int id : tinyWrites[lead]) {
         ins.push_back(id);
         inputsOf[id] = {lead};
-        prebuilt[id].reset();
-        prebuiltLabel[id].clear();
         absorbed[id] = 1;   // keeps its buffer, filled by the one step
     }
     inputsOf[lead] = ins;
@@ -2011,12 +2062,12 @@ void HIPPlan::Builder::batchIndependent()
     auto base_label = [](const std::string &l) { return l.substr(0, l.find('@')); };
     struct Product { size_t step; MatmulInfo mi; };
     struct Wgrad { size_t step; dopt_hip_conv_desc d; };
-    std::vector<Product> products;
+    std::vector<Product> products, fed;   // fed: read by a later step
     std::vector<Wgrad> wgrads;
     for (size_t i = 0; i < p->mSteps.size(); i++) {
         const Step &st = p->mSteps[i];
         const int id = st.op;
-        if (id < 0 || !uses[id].empty() || !dynamic_cast<FnKernel *>(st.kernel.get())) continue;
+        if (id < 0 || !dynamic_cast<FnKernel *>(st.kernel.get())) continue;
         if (biasGradOf[id] >= 0 || poolOf[id] >= 0 || pairOf[id] >= 0 || pairLead[id] >= 0 || pairLater[id] || packOf[id] >= 0) continue;
         const Operation &op = g.ops[id];
         const std::string label = base_label(st.label);
@@ -2024,7 +2075,9 @@ void HIPPlan::Builder::batchIndependent()
         if ((label == "matmul" || label == "matmul+transpose") && (fusedKind[id] == 0 || fusedKind[id] == 6) &&
             plainProduct(id, &mi, false) && st.inputOps.size() == 2 && st.inputOps[0] == mi.a && st.inputOps[1] == mi.b &&
             products.size() < 64) {
-            products.push_back({i, mi});
+            (uses[id].empty() ? products : fed).push_back({i, mi});
+        } else if (!uses[id].empty()) {
+            continue;
         } else if (label == "convolutionFiltersGrad" && op.opType == "convolutionFiltersGrad" && fusedKind[id] == 0 &&
                    op.deps.size() == 2 && op.dtype == DOPT_HIP_F32 && st.inputOps == op.deps && wgrads.size() < 64) {
             const auto *pad = sizes_attr(op, "padding"), *stride = sizes_attr(op, "stride");
@@ -2095,6 +2148,58 @@ void HIPPlan::Builder::batchIndependent()
         const size_t at = wgrads.back().step;
         drop[at] = 0;
         p->mSteps[at] = std::move(b);
+    }
+    // Products that a later step reads (a dense layer's gradients in front of an update rule) can wait for each other while no
+    // step in between reads one of them.
+    for (size_t from = 0; from < fed.size();) {
+        size_t to = from + 1;
+        std::vector<char> made((size_t)nops, 0);
+        made[p->mSteps[fed[from].step].op] = 1;
+        for (; to < fed.size() && to - from < 64; to++) {
+            bool waits = true;
+            for (size_t s = fed[to - 1].step + 1; s <= fed[to].step && waits; s++)
+                for (int in : p->mSteps[s].inputOps) {
+                    size_t off;
+                    if (in >= 0 && made[root(in, &off)]) waits = false;
+                }
+            if (!waits) break;
+            made[p->mSteps[fed[to].step].op] = 1;
+        }
+        if (to - from >= 2) {
+            const size_t n = to - from, at = fed[to - 1].step;
+            Step b;
+            b.op = p->mSteps[at].op;
+            b.label = "matmul*" + std::to_string(n) + (shapes ? "@" : "");
+            std::vector<int> tA, tB;
+            std::vector<size_t> M, N, K;
+            for (size_t k = from; k < to; k++) {
+                const MatmulInfo &mi = fed[k].mi;
+                tA.push_back(mi.tA); tB.push_back(mi.tB);
+                M.push_back(mi.M); N.push_back(mi.N); K.push_back(mi.K);
+                b.inputOps.push_back(mi.a);
+                b.inputOps.push_back(mi.b);
+            }
+            for (size_t k = from; k + 1 < to; k++) {   // (their buffers come as inputs, as those of a group's members do)
+                b.inputOps.push_back(p->mSteps[fed[k].step].op);
+                b.writes.push_back(p->mSteps[fed[k].step].op);
+                drop[fed[k].step] = 1;
+            }
+            b.kernel = make([=](const std::vector<const void *> &in, void *out) {
+                std::vector<const float *> A(n), B(n);
+                std::vector<float *> C(n);
+                for (size_t j = 0; j < n; j++) {
+                    A[j] = (const float *)in[2 * j];
+                    B[j] = (const float *)in[2 * j + 1];
+                    C[j] = j + 1 < n ? (float *)const_cast<void *>(in[2 * n + j]) : (float *)out;
+                }
+                return dopt_hip_sgemm_batch((int)n, tA.data(), tB.data(), M.data(), N.data(), K.data(), A.data(), B.data(), C.data());
+            });
+            b.inputs.resize(b.inputOps.size());
+            b.inputBytes.resize(b.inputOps.size());
+            for (size_t i = 0; i < b.inputOps.size(); i++) b.inputBytes[i] = g.ops[b.inputOps[i]].bytes();
+            p->mSteps[at] = std::move(b);
+        }
+        from = to;
     }
     // close the ranks; the convolution steps remembered for openSplitSums move with them
     std::vector<size_t> moved(p->mSteps.size(), 0);
@@ -2391,8 +2496,9 @@ int HIPPlan::create(Graph *graph, const std::vector<int> &outputs, unsigned flag
         b.fuseDenseLayers();
         b.fuseDenseBackward();
         b.formGroups();
+        b.fuseSquareSums(true);
         b.formTinyRuns();
-        b.fuseSquareSums();
+        b.fuseSquareSums(false);
         b.formChains();
         b.absorbBiasGrads();
         b.absorbPools();

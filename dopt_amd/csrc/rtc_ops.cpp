@@ -1042,6 +1042,18 @@ int reduce_impl(const char *op, int dtype, const size_t *shape, int rank, const 
         int crc = DOPT_HIP_OK;
         if (channel_sum(N, C, inner, (const float *)in, (float *)out, &crc)) return crc;
     }
+    // Runs of axes of extent one need no pass beside another run: folding one value into the start value changes nothing that a
+    // fold has gone over already (a gradient of repeat sums [1, 100, 10, 1] over axes 0 and 2).
+    if (!square && runs.size() > 1) {
+        auto trivial = [&](const std::pair<int, int> &run) {
+            size_t extent = 1;
+            for (int i = run.first; i <= run.second; i++) extent *= cur[i];
+            return extent == 1;
+        };
+        const std::pair<int, int> last = runs.back();
+        runs.erase(std::remove_if(runs.begin(), runs.end(), trivial), runs.end());
+        if (runs.empty()) runs.push_back(last);
+    }
     std::string key = std::string("red:") + op + (dtype == DOPT_HIP_F32 ? ":f32" : ":i32");
     ReduceKernels plain{}, squares{};   // `squares`: the first pass of a sum of squares
     if (int rc = reduce_kernels(key, is_sum, dtype, false, &plain)) return rc;

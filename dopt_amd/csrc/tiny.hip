@@ -15,7 +15,8 @@
 //                 wavefront shuffles, wavefronts in order);
 //   softmax(Grad) one thread per (n, inner) lane, channels in the order of cpu/nnet.d:129-166 (softmax_fwd_k,
 //                 softmax_bwd_k of nn.hip, which rows of fewer than 64 classes take);
-//   repeat        a copy (core/ops/basic.d:336-356).
+//   repeat        a copy (core/ops/basic.d:336-356);
+//   matrix times vector, the reference's way to sum rows (core/ops/basic.d:370-381): the order of gemv_rows_k.
 // So a plan that runs such a chain as one launch returns the bits of the plan that runs it kernel by kernel.
 #include <vector>
 
@@ -426,6 +427,38 @@ __device__ __forceinline__ void run_node(const Node &of, AP a, AP b, float *dstL
         }
         break;
     }
+    case DOPT_HIP_TINY_MATVEC: {   // a: [n, K], b: [K], as gemv_rows_k: lane l of a wavefront adds every 64th product from l on, then
+        // the lanes' sums meet in halves.  A short row is one thread's, which adds what the lanes past its end would (zeros).
+        const int K = nd.dims[0];
+        if (K <= 16) {
+            for (int r = threadIdx.x; r < n; r += kTinyThreads) {
+                float q[16];
+#pragma unroll
+                for (int c = 0; c < 16; c++) q[c] = c < K ? 0.0f + a[(size_t)r * K + c] * b[c] : 0.0f;
+#pragma unroll
+                for (int c = 0; c < 16; c++) q[c] += 0.0f;   // (lanes 32 to 63, then 16 to 31: zeros)
+#pragma unroll
+                for (int half = 8; half > 0; half /= 2)
+#pragma unroll
+                    for (int c = 0; c < half; c++) q[c] += q[c + half];
+                if (dstL) dstL[r] = q[0];
+                if (dstG) dstG[r] = q[0];
+            }
+            break;
+        }
+        const int lane = threadIdx.x & 63;
+        for (int r = threadIdx.x >> 6; r < n; r += kTinyThreads / 64) {
+            float acc = 0.0f;
+            for (int c = lane; c < K; c += 64) acc += a[(size_t)r * K + c] * b[c];
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
+            if (lane == 0) {
+                if (dstL) dstL[r] = acc;
+                if (dstG) dstG[r] = acc;
+            }
+        }
+        break;
+    }
     case DOPT_HIP_TINY_REPEAT: {   // dims = the input's extents (leading 1s for ranks below 4), reps beside them
         if (nd.dims[0] * nd.dims[1] * nd.dims[2] * nd.dims[3] == 1) {   // one value, n times
             const float r = a[0];
@@ -533,6 +566,7 @@ int operand_extent(const dopt_hip_tiny_node &nd, int which)
         return kind == 0 ? nd.n : kind == 1 ? 1 : kind == 2 ? nd.n / inner : inner;
     }
     case DOPT_HIP_TINY_REDUCE: return nd.dims[0] * nd.dims[1] * nd.dims[2];
+    case DOPT_HIP_TINY_MATVEC: return which == 0 ? nd.n * nd.dims[0] : nd.dims[0];
     case DOPT_HIP_TINY_REPEAT: return nd.dims[0] * nd.dims[1] * nd.dims[2] * nd.dims[3];
     default: return nd.n;
     }
@@ -641,8 +675,8 @@ int dopt_hip_tiny_graph(int nslots, void *const *slots, int nnodes, const dopt_h
     std::vector<dopt_hip_tiny_node> plain_nodes(nodes, nodes + nnodes);
     for (int k = 0; k < nnodes; k++) {
         const dopt_hip_tiny_node &nd = nodes[k];
-        const bool binary = nd.kind == DOPT_HIP_TINY_SOFTMAX_GRAD || (nd.kind == DOPT_HIP_TINY_POINTWISE && nd.b >= 0);
-        DOPT_REQUIRE(nd.kind >= DOPT_HIP_TINY_POINTWISE && nd.kind <= DOPT_HIP_TINY_REPEAT, "dopt_hip_tiny_graph: node %d has unknown kind %d", k, nd.kind);
+        const bool binary = nd.kind == DOPT_HIP_TINY_SOFTMAX_GRAD || nd.kind == DOPT_HIP_TINY_MATVEC || (nd.kind == DOPT_HIP_TINY_POINTWISE && nd.b >= 0);
+        DOPT_REQUIRE(nd.kind >= DOPT_HIP_TINY_POINTWISE && nd.kind <= DOPT_HIP_TINY_MATVEC, "dopt_hip_tiny_graph: node %d has unknown kind %d", k, nd.kind);
         DOPT_REQUIRE(nd.dst >= 0 && nd.dst < nslots && nd.a >= 0 && nd.a < nslots && nd.b < nslots && (!binary || nd.b >= 0),
                      "dopt_hip_tiny_graph: node %d names a buffer that was not passed", k);
         DOPT_REQUIRE(slots[nd.dst] && slots[nd.a] && (nd.b < 0 || slots[nd.b]), "dopt_hip_tiny_graph: node %d: null buffer", k);
@@ -660,6 +694,9 @@ int dopt_hip_tiny_graph(int nslots, void *const *slots, int nnodes, const dopt_h
             DOPT_REQUIRE(nd.dims[0] >= 0 && nd.dims[1] >= 1 && nd.dims[2] >= 1 && (long long)nd.dims[0] * nd.dims[2] == nd.n &&
                              (long long)nd.dims[0] * nd.dims[1] * nd.dims[2] <= DOPT_HIP_TINY_ELEMS,
                          "dopt_hip_tiny_graph: node %d: a reduction of [%d, %d, %d] does not give %d values", k, nd.dims[0], nd.dims[1], nd.dims[2], nd.n);
+        } else if (nd.kind == DOPT_HIP_TINY_MATVEC) {
+            DOPT_REQUIRE(nd.dims[0] >= 2 && (long long)nd.n * nd.dims[0] <= DOPT_HIP_TINY_ELEMS,
+                         "dopt_hip_tiny_graph: node %d: a product of [%d, %d] and a vector", k, nd.n, nd.dims[0]);
         } else if (nd.kind == DOPT_HIP_TINY_REPEAT) {
             long long vol = 1;
             for (int d = 0; d < 4; d++) {
@@ -708,6 +745,7 @@ int dopt_hip_tiny_graph(int nslots, void *const *slots, int nnodes, const dopt_h
         long long busy = nd.n;
         if (nd.kind == DOPT_HIP_TINY_SOFTMAX || nd.kind == DOPT_HIP_TINY_SOFTMAX_GRAD) busy = (long long)nd.dims[0] * nd.dims[2];
         else if (nd.kind == DOPT_HIP_TINY_REDUCE && nd.dims[2] == 1 && nd.dims[1] > 64) busy = kTinyThreads;   // rows: the block folds them together
+        else if (nd.kind == DOPT_HIP_TINY_MATVEC && nd.dims[0] > 16) busy = 64ll * nd.n;
         // quads: an operand that is read element by element, and the result, start on one in memory and in LDS
         auto on_quad = [](const TinyAddress &m, int at, bool single) { return single || ((m.lo & 15u) == 0 && (at & 3) == 0); };
         to.quads = nd.kind == DOPT_HIP_TINY_POINTWISE && to.a_kind < 2 && to.b_kind < 2 && on_quad(to.a, in_lds ? to.lds.a : 0, to.a_kind == 1) &&

@@ -161,14 +161,16 @@ int dopt_hip_pointwise_index(const char *op);
      SOFTMAX       the operand is [dims[0], dims[1], dims[2]] = [N, C, inner], normalised over C as dopt_hip_softmax_fwd
                    does for rows of fewer than 64 classes (or inner > 1)
      SOFTMAX_GRAD  a = dy, b = y, same layout, as dopt_hip_softmax_bwd
-     REPEAT        the operand has extents dims[0..3] (leading 1s for lower ranks) and is tiled reps[0..3] times */
+     REPEAT        the operand has extents dims[0..3] (leading 1s for lower ranks) and is tiled reps[0..3] times
+     MATVEC        a = matrix [n, dims[0]], b = vector [dims[0]]: their product as dopt_hip_sgemm gives it (dims[0] >= 2) */
 typedef enum { DOPT_HIP_TINY_SLOTS = 48, DOPT_HIP_TINY_NODES = 40, DOPT_HIP_TINY_ELEMS = 4096 } dopt_hip_tiny_limits;
 typedef enum {
     DOPT_HIP_TINY_POINTWISE = 0,
     DOPT_HIP_TINY_REDUCE = 1,
     DOPT_HIP_TINY_SOFTMAX = 2,
     DOPT_HIP_TINY_SOFTMAX_GRAD = 3,
-    DOPT_HIP_TINY_REPEAT = 4
+    DOPT_HIP_TINY_REPEAT = 4,
+    DOPT_HIP_TINY_MATVEC = 5
 } dopt_hip_tiny_kind;
 typedef struct {
     int kind, op;

@@ -669,6 +669,48 @@ def test_host_arguments_are_consumed_when_the_call_returns():
         assert np.all(np.isfinite(u)) and np.array_equal(u, v)
 
 
+@pytest.mark.parametrize("batch,width", [(100, 10), (59, 10), (300, 10), (20, 200)])
+def test_softmax_regression_with_sums_as_products(batch, width):
+    """The softmax of examples/mnistlogit.d, whose row sums are products with a vector of ones and whose gradients sum over axes of
+    extent one beside another: the same bits with and without the rewrites, in fewer steps, replayed and after new values."""
+    def build():
+        feats, labels = core.float32([batch, 64]), core.float32([batch, width])
+        W, b = core.float32([64, width]), core.float32([width])
+        linear = core.matmul(feats, W) + core.repeat(b, batch)
+        numer = core.exp(linear - core.maxElement(linear))
+        denom = core.repeat(core.sum(numer, [1]).reshape([batch, 1]), [1, width])
+        loss = nnet.crossEntropy(numer / denom, labels)
+        step = [p - core.repeat(core.float32([1], [0.5]), p.volume).reshape(p.shape) * g for p, g in zip((W, b), core.grad(loss, [W, b]))]
+        return feats, labels, W, b, [loss] + step
+    feats, labels, W, b, outs = build()
+    plans = [core.compile(outs, f) for f in (0, core.PLAN_VIEWS | core.PLAN_FUSE, core.PLAN_VIEWS | core.PLAN_FUSE | core.PLAN_OVERLAP,
+                                             core.PLAN_VIEWS | core.PLAN_FUSE | core.PLAN_OVERLAP_LIGHT, core.PLAN_VIEWS | core.PLAN_FUSE | core.PLAN_GRAPH)]
+    for seed in range(4):
+        r = np.random.default_rng(seed)
+        args = {feats: r.random((batch, 64), np.float32), labels: np.eye(width, dtype=np.float32)[r.integers(0, width, batch)],
+                W: (r.standard_normal((64, width)) * 0.1).astype(np.float32), b: r.standard_normal(width).astype(np.float32)}
+        want = plans[0].execute(args)
+        for p in plans[1:]:
+            for x, y in zip(want, p.execute(args)):
+                assert np.array_equal(x, y)
+    if width == 10 and batch * width <= 4096:
+        assert plans[1].stats()["kernels"] <= 6 < plans[0].stats()["kernels"]
+
+
+@pytest.mark.parametrize("shape,axes", [((1, 100, 10, 1), (0, 2)), ((1, 7, 1, 5), (0, 2)), ((3, 1, 4), (0, 2)), ((1, 4, 1), (0, 2)), ((2, 1, 3, 1, 2), (0, 2, 4))])
+def test_sums_over_axes_of_extent_one_beside_others(shape, axes):
+    r = np.random.default_rng(3)
+    x = r.standard_normal(shape).astype(np.float32)
+    x.ravel()[:2] = -0.0
+    for op, want in ((core.sum, x.astype(np.float64).sum(axes)), (core.maxElement, x.max(axes))):
+        v = core.float32(list(shape))
+        outs = [op(v * v, list(axes)) + op(v, list(axes)), op(v, list(axes))]
+        a, b = (core.compile(outs, f).execute({v: x}) for f in (0, core.PLAN_VIEWS | core.PLAN_FUSE))
+        for p, q in zip(a, b):
+            assert np.array_equal(p.view(np.uint32), q.view(np.uint32))
+        assert np.allclose(a[1], want, rtol=1e-5, atol=1e-6)
+
+
 def test_weight_decay_terms_square_on_load():
     """`weightDecay * sum(filters * filters)` (nnet/layers/conv.d:117): with the rewrites on the product is never stored
     (`mul+sum`, one pass over the filter); loss and gradients are those of the plan without rewrites, bit for bit.

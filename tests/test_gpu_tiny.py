@@ -12,7 +12,7 @@ from util import assert_close
 
 pytestmark = pytest.mark.gpu
 
-PW, RED, SMAX, SMAXG, REP = range(5)
+PW, RED, SMAX, SMAXG, REP, MATVEC = range(6)
 
 
 def _node(kind, dst, a, b=-1, op=0, n=0, a_kind=0, b_kind=0, dims=(0, 0, 0, 0), reps=(0, 0, 0, 0), offs=(0, 0, 0)):
@@ -123,6 +123,17 @@ def test_repeat_node_equals_dopt_hip_repeat(shape, reps):
     _run([tx, out], [_node(REP, 1, 0, n=want.size, dims=(1,) * lead + tuple(shape), reps=(1,) * lead + tuple(reps))])
     assert np.array_equal(out.numpy(), want)
     assert np.array_equal(want, np.tile(x, reps))
+
+
+@pytest.mark.parametrize("rows,k", [(100, 10), (1, 2), (256, 16), (240, 17), (63, 65), (1, 4096), (31, 130), (2048, 2), (1024, 3)])
+def test_matrix_vector_node_equals_the_product(rows, k):
+    r = np.random.default_rng(rows + k)
+    a, b = r.standard_normal((rows, k)).astype(np.float32), r.standard_normal((k, 1)).astype(np.float32)
+    a[0] = -0.0
+    ta, tb, out = ops.tensor(a), ops.tensor(b), ops.Tensor([rows, 1])
+    _run([ta, tb, out], [_node(MATVEC, 2, 0, 1, n=rows, dims=(k, 0, 0, 0))])
+    want = ops.matmul(ta, tb).numpy()
+    assert np.array_equal(out.numpy().view(np.uint32), want.view(np.uint32))
 
 
 def test_a_loss_tail_as_one_launch_matches_the_oracle():
