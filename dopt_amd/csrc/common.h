@@ -113,6 +113,20 @@ int pointwise_group(const PointwiseProgram &program, const std::vector<Pointwise
 // dopt_hip_reduce_squares gives.
 int reduce_squares_batch(int count, const float *const *in, const size_t *n, float *const *out);
 
+// tiny_rtc.cpp: a run of operations on tiny tensors (dopt_hip_tiny_graph's nodes) as a kernel of its own, compiled when it is first
+// launched.  The results' buffers must not overlap each other, which a plan's own do not.  `done` stays false, with nothing
+// launched, for runs it does not take and where what is read from outside overlaps a result: those are dopt_hip_tiny_graph's.
+struct TinyRun {
+    TinyRun(int nslots, const std::vector<dopt_hip_tiny_node> &nodes);
+    int launch(void *const *slots, bool *done) const;
+
+private:
+    struct Range { int slot, offset, bytes; };
+    int slots, threads = 0;
+    std::string source, key;
+    std::vector<Range> reads, writes;
+};
+
 // hipRTC: compile `source` (once per distinct `key`) and return the named kernel.
 int rtc_get(const std::string &key, const std::string &source, const char *kernel_name, hipFunction_t *fn);
 bool rtc_find(const std::string &key, hipFunction_t *fn);   // a kernel compiled before (its source need not be put together again)

@@ -174,3 +174,84 @@ def test_a_loss_tail_as_one_launch_matches_the_oracle():
     assert lib.dopt_hip_tiny_graph(2, (C.c_void_p * 2)(tl.ptr, work.ptr), 1, (capi.TinyNode * 1)(bad)) != 0
     assert b"at most" in lib.dopt_hip_last_error()
     ops.sync()
+
+
+UNARY, BINARY = ["neg", "abs", "sgn", "exp", "sqrt", "tanh", "relu"], ["add", "sub", "mul", "div", "max", "min", "lt", "pow"]
+
+
+def _random_run(seed):
+    """A graph of tiny operations of every kind a run may hold, over tensors of odd and even sizes, and its variables."""
+    from dopt_amd import core, nnet
+    r = np.random.default_rng(seed)
+    rows, cols = int(r.choice([1, 2, 7, 33, 64, 100, 257, 400])), int(r.choice([1, 2, 3, 8, 10, 16, 40]))
+    if rows * cols > 4096:
+        cols = 4096 // rows
+    var = [core.float32([rows, cols]) for _ in range(3)] + [core.float32([1]), core.float32([rows, 1]), core.float32([1, cols])]
+    full, single = list(var[:3]), [var[3]]
+    outs = []
+    for _ in range(int(r.integers(6, 22))):
+        k, x = r.integers(0, 11), full[r.integers(len(full))]
+        y = full[r.integers(len(full))]
+        if k < 3:
+            op = BINARY[r.integers(len(BINARY))]
+            full.append(core.Operation(op, [x, y], {}) if not hasattr(core, op) else getattr(core, op)(x, y))
+        elif k == 3:
+            op = UNARY[r.integers(len(UNARY) - 1)]
+            full.append(core.Operation(op, [x], {}) if not hasattr(core, op) else getattr(core, op)(x))
+        elif k == 4:
+            full.append(core.softmax(x) if cols < 64 else x)
+        elif k == 5:
+            single.append(core.sum(x).reshape([1]) if r.random() < 0.5 else core.maxElement(x).reshape([1]))
+        elif k == 6:
+            full.append(core.repeat(core.sum(x, [0]).reshape([1, cols]), [rows, 1]))
+        elif k == 7:
+            full.append(core.repeat(core.maxElement(x, [1]).reshape([rows, 1]), [1, cols]))
+        elif k == 8:
+            full.append(core.matmul(core.matmul(x, core.float32([cols, 1], np.ones(cols, np.float32))), var[5]))
+        elif k == 9:
+            full.append(core.repeat(single[r.integers(len(single))], [rows * cols]).reshape([rows, cols]) * x)
+        else:
+            single.append(single[r.integers(len(single))] * single[r.integers(len(single))] + var[3])
+        if r.random() < 0.3:
+            outs.append(full[-1])
+    outs += [full[-1], single[-1], core.sum(full[-1] * full[0], [1])]
+    return var, outs
+
+
+@pytest.mark.parametrize("seed", range(40))
+def test_runs_compiled_for_a_plan_equal_their_operations(seed):
+    """The kernel that a plan compiles for a run against the plan that runs every operation by itself, bit for bit (NaNs by
+    their place), with values that are not finite in every other case."""
+    from dopt_amd import core
+    var, outs = _random_run(seed)
+    r = np.random.default_rng(1000 + seed)
+    plain, fused = core.compile(outs, 0), core.compile(outs, core.PLAN_VIEWS | core.PLAN_FUSE)
+    for case in range(2):
+        args = {v: r.standard_normal(v.shape).astype(np.float32) for v in var}
+        if case == 1 and seed % 2:
+            a = args[var[0]].ravel()
+            a[:: max(1, a.size // 3)] = np.nan
+            a[a.size // 2] = np.inf
+        for x, y in zip(plain.execute(args), fused.execute(args)):
+            assert np.array_equal(x, y, equal_nan=True)
+
+
+def test_a_run_whose_argument_lies_in_its_own_result():
+    """An argument at the address of a buffer that the run fills: what it reads is what was there before."""
+    from dopt_amd import core
+    x, w = core.float32([10, 10]), core.float32([10, 10])
+    a = x * w
+    b = core.sum(a, [0])
+    c = core.repeat(b.reshape([1, 10]), [10, 1]) + a * x
+    plan = core.compile([a, b, c], core.PLAN_VIEWS | core.PLAN_FUSE)
+    r = np.random.default_rng(0)
+    X, Wv = r.standard_normal((10, 10)).astype(np.float32), r.standard_normal((10, 10)).astype(np.float32)
+    first = plan.execute({x: X, w: Wv})
+    ptr, _ = plan.result_ptr(c)
+    before = first[2]
+    again = plan.execute({x: ops.Tensor((10, 10), _ptr=ptr, _owner=plan), w: Wv})
+    A = before * Wv
+    assert np.array_equal(again[0], A)
+    plain = core.compile([a, b, c], 0).execute({x: before, w: Wv})
+    for p, q in zip(plain, again):
+        assert np.array_equal(p, q)
