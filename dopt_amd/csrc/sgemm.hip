@@ -813,67 +813,128 @@ __global__ __launch_bounds__(256) void outer_k(size_t M, size_t N, const float *
     }
 }
 
-// N == 1: C[m] = sum_k A[m][k] * b[k]; one wavefront per row, lanes along k.
-__global__ __launch_bounds__(256) void gemv_rows_k(size_t M, size_t K, const float *A, const float *b, float *c)
+// Matrix times vector, either way the matrix is stored, in one order: the reduction falls into slices of kGemvSlice steps; of a
+// slice, chain l (of 64) adds the products l, l + 64, l + 128 .., the chains' sums meet in halves (l and l + 32, then l and
+// l + 16 ..), and slices are added from the first on.  So a plan that reads a transposed matrix in place gets the bits of the
+// plan that copies it first.  Bound by the matrix' bytes from a few MB on.
+constexpr int kGemvSlice = 1024;
+
+struct VectorEpilogue {   // + rowvec[row] * colbias[col >> shift], relu, mask, as sgemm_small_k's
+    const float *colbias, *rowvec, *mask;
+    int shift, relu;
+    size_t N;   // columns of the result
+    __device__ __forceinline__ float operator()(float sum, size_t i) const
+    {
+        if (colbias) {
+            const size_t row = i / N, col = i - row * N;
+            float add = colbias[col >> shift];
+            if (rowvec) add = __fmul_rn(rowvec[row], add);
+            sum += add;
+        }
+        if (relu) sum = sum < 0.0f ? 0.0f : sum;
+        if (mask) sum = mask[i] > 0.0f ? sum : 0.0f;
+        return sum;
+    }
+};
+
+// The matrix is stored row by row along the reduction: a wavefront per result, a lane per chain.
+__global__ __launch_bounds__(256) void gemv_rows_k(size_t M, size_t K, const float *A, const float *b, float *c, VectorEpilogue ep)
 {
     const size_t row = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= M) return;
     const int lane = threadIdx.x & 63;
     const float *ar = A + row * K;
-    float acc = 0.0f;
-    for (size_t k = lane; k < K; k += 64) acc += ar[k] * b[k];
+    float total = 0.0f;
+    for (size_t k0 = 0; k0 < K; k0 += kGemvSlice) {
+        const size_t k1 = min(K, k0 + kGemvSlice);
+        float acc = 0.0f;
+        size_t k = k0 + lane;
+        for (; k + 448 < k1; k += 512) {   // eight steps in flight
+            float x[8], y[8];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
-    if (lane == 0) c[row] = acc;
-}
-
-// M == 1: C[n] = sum_k a[k] * B[k][n]; lanes along n, a block folds a slice of k; slices are then
-// summed in a fixed order.
-__global__ __launch_bounds__(256) void gemv_cols_k(size_t K, size_t N, size_t kslice, const float *a, const float *B,
-                                                    float *partial)
-{
-    const size_t n = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (n >= N) return;
-    const size_t k0 = (size_t)blockIdx.y * kslice;
-    const size_t k1 = k0 + kslice < K ? k0 + kslice : K;
-    float acc = 0.0f;
-    for (size_t k = k0; k < k1; k++) acc += a[k] * B[k * N + n];
-    partial[(size_t)blockIdx.y * N + n] = acc;
-}
-
-// The same for a short reduction (K <= 256) in one launch: a block takes 64 columns, its four
-// groups of 64 threads take every fourth k, sixteen loads in flight per thread (clamped, not
-// branched), and the four sums are added in group order through LDS.
-// (`on`: false for the threads of a larger block that only keep the barrier company)
-__device__ __forceinline__ void gemv_cols_short_body(int K, int N, const float *a, const float *B, float *c, int bx, bool on,
-                                                     float (*part)[64])
-{
-    const int col = threadIdx.x & 63, kl = (threadIdx.x >> 6) & 3;
-    const int n = min(bx * 64 + col, N - 1);
-    float acc = 0.0f;
-    if (on) {
-        for (int k0 = kl; k0 < K; k0 += 64) {
-            float av[16], bv[16];
-#pragma unroll
-            for (int u = 0; u < 16; u++) {
-                const int k = min(k0 + 4 * u, K - 1);
-                av[u] = a[k];
-                bv[u] = B[(size_t)k * N + n];
+            for (int u = 0; u < 8; u++) {
+                x[u] = ar[k + 64 * u];
+                y[u] = b[k + 64 * u];
             }
 #pragma unroll
-            for (int u = 0; u < 16; u++)
-                if (k0 + 4 * u < K) acc += av[u] * bv[u];
+            for (int u = 0; u < 8; u++) acc += x[u] * y[u];
         }
-        part[kl][col] = acc;
+        float x[7], y[7];   // what is left: up to seven steps, together as well
+#pragma unroll
+        for (int u = 0; u < 7; u++) {
+            const size_t at = min(k + 64 * u, K - 1);
+            x[u] = ar[at];
+            y[u] = b[at];
+        }
+#pragma unroll
+        for (int u = 0; u < 7; u++)
+            if (k + 64 * u < k1) acc += x[u] * y[u];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
+        total = k0 == 0 ? acc : total + acc;
     }
-    __syncthreads();
-    if (on && kl == 0 && bx * 64 + col < N) c[n] = ((part[0][col] + part[1][col]) + part[2][col]) + part[3][col];
+    if (lane == 0) c[row] = ep(total, row);
 }
 
-__global__ __launch_bounds__(256) void gemv_cols_short_k(int K, int N, const float *a, const float *B, float *c)
+// The matrix is stored [K][N]: a block folds one slice of 32 columns, a thread eight neighbouring chains of a column.
+constexpr int kGemvCols = 32;
+struct GemvLds {
+    float chain[8][8][kGemvCols];   // group of chains, chain, column
+};
+// (`on`: false for the threads of a larger block that only keep the barriers company)
+template <class Store>
+__device__ __forceinline__ void gemv_cols_body(int K, int N, const float *a, const float *B, int bx, int k0, bool on, GemvLds &lds, Store &&store)
 {
-    __shared__ float part[4][64];
-    gemv_cols_short_body(K, N, a, B, c, (int)blockIdx.x, true, part);
+    const int col = threadIdx.x & 31, g = (threadIdx.x >> 5) & 7, k1 = min(K, k0 + kGemvSlice);
+    const int n = min(bx * kGemvCols + col, N - 1);
+    float acc[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) acc[j] = 0.0f;
+    if (on) {
+        for (int k = k0 + 8 * g; k < k1; k += 128) {   // sixteen loads in flight (clamped, not branched)
+            float av[2][8], bv[2][8];
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const int at = min(k + 64 * u + j, K - 1);
+                    av[u][j] = a[at];
+                    bv[u][j] = B[(size_t)at * N + n];
+                }
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    if (k + 64 * u + j < k1) acc[j] += av[u][j] * bv[u][j];
+        }
+    }
+#pragma unroll
+    for (int half = 4; half > 0; half >>= 1) {   // chains 32, 16 and 8 apart: groups
+        if (on && g >= half && g < 2 * half) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) lds.chain[g][j][col] = acc[j];
+        }
+        __syncthreads();
+        if (on && g < half) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) acc[j] += lds.chain[g + half][j][col];
+        }
+    }
+#pragma unroll
+    for (int half = 4; half > 0; half >>= 1)
+#pragma unroll
+        for (int j = 0; j < half; j++) acc[j] += acc[j + half];
+    if (on && g == 0 && bx * kGemvCols + col < N) store(bx * kGemvCols + col, acc[0]);
+}
+
+// blockIdx.y: the slice.  With more than one their sums go to consecutive copies of the result, which splitk_epilogue_k adds
+// (and `ep` does nothing).
+__global__ __launch_bounds__(256) void gemv_cols_k(int K, int N, const float *a, const float *B, float *c, VectorEpilogue ep)
+{
+    __shared__ GemvLds lds;
+    float *const to = c + (size_t)blockIdx.y * N;
+    gemv_cols_body(K, N, a, B, (int)blockIdx.x, (int)blockIdx.y * kGemvSlice, true, lds,
+                   [&](int n, float v) { to[n] = ep(v, (size_t)n); });
 }
 
 // Several independent small products in ONE launch: the weight and bias gradients of a dense head are six kernels of a
@@ -900,14 +961,16 @@ struct SmallGroup {
 template <bool kTA, bool kTB, bool kCut>
 __global__ __launch_bounds__(64 * kSmallWaves) void sgemm_small_group_k(SmallGroup g)
 {
-    __shared__ float red[kSmallWaves][32 * 33];
-    __shared__ float part[4][64];
+    __shared__ union {
+        float red[kSmallWaves][32 * 33];
+        GemvLds gemv;
+    } lds;
     const int b = (int)blockIdx.x;   // uniform: the scans below stay scalar
     if (g.nv > 0 && b >= g.v[0].first) {
         int j = 0;
         while (j + 1 < g.nv && b >= g.v[j + 1].first) j++;
         const GemvJob &q = g.v[j];
-        gemv_cols_short_body(q.K, q.N, q.a, q.B, q.c, b - q.first, threadIdx.x < 256, part);
+        gemv_cols_body(q.K, q.N, q.a, q.B, b - q.first, 0, threadIdx.x < 256, lds.gemv, [&](int n, float v) { q.c[n] = v; });
         return;
     }
     int j = 0;
@@ -915,7 +978,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void sgemm_small_group_k(SmallGro
     const SmallJob &q = g.s[j];
     const int local = b - q.first;
     sgemm_small_body<kTA, kTB, kCut>(q.M, q.N, q.K, q.lda, q.ldb, q.kslice, q.A, q.B, q.C, nullptr, 0, nullptr, 0, nullptr,
-                                     local % q.nx, local / q.nx, 0, q.K, red);
+                                     local % q.nx, local / q.nx, 0, q.K, lds.red);
 }
 
 // c[m][n] = relu?(c[m][n] + u[m] * v[n]): the epilogue of dopt_hip_sgemm_rank1 as a pass of its own, for the
@@ -1015,6 +1078,9 @@ struct Extras {
     const float *mask = nullptr;
 };
 
+// Whether a matrix times a vector finds the matrix stored row by row along the reduction (where both sides are vectors it does).
+bool gemv_by_rows(int transA, int transB, size_t M, size_t N) { return (N == 1 && !transA) || (M == 1 && transB) || (M == 1 && N == 1); }
+
 int sgemm_epilogue(int transA, int transB, size_t M, size_t N, size_t K, const float *A, const float *B, float *C,
                    const float *colbias, int bias_shift, const float *rowvec, int relu, bool *biased, const Extras &ex = Extras{});
 
@@ -1029,7 +1095,7 @@ int sgemm_bias(int transA, int transB, size_t M, size_t N, size_t K, const float
 // being asked for, which a kernel without one leaves to a pass behind it; operand alignment picks between variants of a
 // kernel that add in the same order (the LDS-resident kernel apart: panel_allowed = false is the route without it).
 struct Route {
-    enum Kind { kNone, kOuter, kGemvRows, kGemvColsShort, kGemvCols, kPanel, kSmall, kTile64, kTile128, kRows, kRowsBig } kind;
+    enum Kind { kNone, kOuter, kGemv, kPanel = 5, kSmall, kTile64, kTile128, kRows, kRowsBig } kind;
     size_t cuts;    // partial sums per element that a second pass adds (gemv slices, tile-engine splits)
     size_t depth;   // reduction steps per partial sum (k per slice, slabs per split)
     size_t pass = 0;   // sgemm_rows_k: slabs that are added in its accumulators before they go to C
@@ -1095,18 +1161,9 @@ Route sgemm_route(int transA, int transB, size_t M, size_t N, size_t K, bool pan
     Route r{Route::kNone, 1, K, 0, 0, 0};
     if (M * N == 0 || K == 0) return r;
     if (K == 1) { r.kind = Route::kOuter; return r; }
-    // matrix-vector products: `rows` reads the matrix row by row (k contiguous), `cols` column-wise
-    if ((N == 1 && !transA) || (M == 1 && transB)) { r.kind = Route::kGemvRows; return r; }
-    if ((M == 1 && !transB) || (N == 1 && transA)) {
-        const size_t R = M == 1 ? N : M;
-        if (K <= 256 && R < ((size_t)1 << 30)) { r.kind = Route::kGemvColsShort; return r; }   // one launch, no partial sums
-        const size_t nblocks = ceil_div(R, (size_t)256);
-        size_t slices = ceil_div((size_t)num_cus() * 2, nblocks);
-        if (slices > ceil_div(K, (size_t)32)) slices = ceil_div(K, (size_t)32);
-        if (slices > 64) slices = 64;
-        if (slices < 1) slices = 1;
-        r.kind = Route::kGemvCols;
-        r.depth = ceil_div(K, slices);
+    if (M == 1 || N == 1) {   // matrix times vector: one order however the matrix is stored
+        r.kind = Route::kGemv;
+        r.depth = kGemvSlice;
         r.cuts = ceil_div(K, r.depth);
         return r;
     }
@@ -1214,33 +1271,25 @@ int sgemm_epilogue(int transA, int transB, size_t M, size_t N, size_t K, const f
         DOPT_LAUNCH_CHECK();
         return DOPT_HIP_OK;
     }
-    if (kind == Route::kGemvRows) {
-        const size_t R = N == 1 ? M : N;
+    if (kind == Route::kGemv) {
+        const size_t R = N == 1 ? M : N, slices = route.cuts;
         const float *mat = N == 1 ? A : B, *vec = N == 1 ? B : A;
-        hipLaunchKernelGGL(gemv_rows_k, dim3((unsigned)ceil_div(R, (size_t)4)), dim3(256), 0, stream(), R, K, mat, vec, C);
-        DOPT_LAUNCH_CHECK();
-        return DOPT_HIP_OK;
-    }
-    if (kind == Route::kGemvColsShort || kind == Route::kGemvCols) {
-        const size_t R = M == 1 ? N : M;
-        const float *mat = M == 1 ? B : A, *vec = M == 1 ? A : B;
-        if (kind == Route::kGemvColsShort) {
-            hipLaunchKernelGGL(gemv_cols_short_k, dim3((unsigned)ceil_div(R, (size_t)64)), dim3(256), 0, stream(), (int)K, (int)R,
-                               vec, mat, C);
+        const VectorEpilogue ep{colbias, rowvec, ex.mask, bias_shift, relu, N}, none{nullptr, nullptr, nullptr, 0, 0, 1};
+        *biased = true;
+        if (gemv_by_rows(transA, transB, M, N)) {
+            hipLaunchKernelGGL(gemv_rows_k, dim3((unsigned)ceil_div(R, (size_t)4)), dim3(256), 0, stream(), R, K, mat, vec, C, ep);
             DOPT_LAUNCH_CHECK();
             return DOPT_HIP_OK;
         }
-        const size_t nblocks = ceil_div(R, (size_t)256), slices = route.cuts, kslice = route.depth;
-        float *partial = C;
-        if (slices > 1) {
-            partial = (float *)workspace(slices * R * sizeof(float));
-            if (!partial) return DOPT_HIP_ERR_OOM;
-        }
-        hipLaunchKernelGGL(gemv_cols_k, dim3((unsigned)nblocks, (unsigned)slices), dim3(256), 0, stream(), K, R, kslice,
-                           vec, mat, partial);
+        float *to = C;
+        if (slices > 1 && !(to = (float *)workspace(slices * R * sizeof(float)))) return DOPT_HIP_ERR_OOM;
+        for (size_t s0 = 0; s0 < slices; s0 += 65535)   // (a grid's second dimension)
+            hipLaunchKernelGGL(gemv_cols_k, dim3((unsigned)ceil_div(R, (size_t)kGemvCols), (unsigned)std::min(slices - s0, (size_t)65535)), dim3(256), 0, stream(),
+                               (int)(K - s0 * kGemvSlice), (int)R, vec + s0 * kGemvSlice, mat + s0 * kGemvSlice * R, to + s0 * R, slices > 1 ? none : ep);
         DOPT_LAUNCH_CHECK();
         if (slices > 1) {
-            hipLaunchKernelGGL(splitk_reduce_k, dim3(flat_grid(R)), dim3(256), 0, stream(), R, (int)slices, partial, C);
+            hipLaunchKernelGGL(splitk_epilogue_k, dim3(flat_grid(R)), dim3(256), 0, stream(), M, N, (int)slices, to, C, colbias, bias_shift, rowvec, relu,
+                               ex.mask);
             DOPT_LAUNCH_CHECK();
         }
         return DOPT_HIP_OK;
@@ -1383,7 +1432,7 @@ int dopt_hip_sgemm_batch(int n, const int *transA, const int *transB, const size
         if (M[i] * N[i] == 0) continue;
         const bool plain = K[i] > 0 && A[i] && B[i] && C[i] && M[i] < ((size_t)1 << 30) && N[i] < ((size_t)1 << 30) && K[i] < ((size_t)1 << 30);
         const Route r = plain ? sgemm_route(transA[i], transB[i], M[i], N[i], K[i]) : Route{Route::kNone, 1, 0, 0, 0, 0};
-        if (r.kind == Route::kGemvColsShort && gemvs.size() < (size_t)kGroupJobs) {
+        if (r.kind == Route::kGemv && r.cuts == 1 && !gemv_by_rows(transA[i], transB[i], M[i], N[i]) && gemvs.size() < (size_t)kGroupJobs) {
             const size_t R = M[i] == 1 ? N[i] : M[i];
             GemvJob q{};
             q.K = (int)K[i]; q.N = (int)R;
@@ -1419,7 +1468,7 @@ int dopt_hip_sgemm_batch(int n, const int *transA, const int *transB, const size
                 GemvJob &q = in.g.v[in.g.nv++];
                 q = v;
                 q.first = (int)in.blocks;
-                in.blocks += (unsigned)ceil_div((size_t)v.N, (size_t)64);
+                in.blocks += (unsigned)ceil_div((size_t)v.N, (size_t)kGemvCols);
             }
             gemvs.clear();
         }
@@ -1433,8 +1482,8 @@ int dopt_hip_sgemm_batch(int n, const int *transA, const int *transB, const size
         DOPT_LAUNCH_CHECK();
     }
     for (const GemvJob &v : gemvs) {   // no 32 x 32-tile launch to ride in
-        hipLaunchKernelGGL(gemv_cols_short_k, dim3((unsigned)ceil_div((size_t)v.N, (size_t)64)), dim3(256), 0, stream(), v.K, v.N,
-                           v.a, v.B, v.c);
+        hipLaunchKernelGGL(gemv_cols_k, dim3((unsigned)ceil_div((size_t)v.N, (size_t)kGemvCols)), dim3(256), 0, stream(), v.K, v.N, v.a, v.B, v.c,
+                           VectorEpilogue{nullptr, nullptr, nullptr, 0, 0, 1});
         DOPT_LAUNCH_CHECK();
     }
     for (int i : single)

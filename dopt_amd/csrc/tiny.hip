@@ -430,8 +430,8 @@ __device__ __forceinline__ void run_node(const Node &of, AP a, AP b, float *dstL
         }
         break;
     }
-    case DOPT_HIP_TINY_MATVEC: {   // a: [n, K], b: [K], as gemv_rows_k: lane l of a wavefront adds every 64th product from l on, then
-        // the lanes' sums meet in halves.  A short row is one thread's, which adds what the lanes past its end would (zeros).
+    case DOPT_HIP_TINY_MATVEC: {   // a: [n, K], b: [K], as gemv_rows_k: of 1024 products lane l of a wavefront adds every 64th from l on,
+        // then the lanes' sums meet in halves.  A short row is one thread's, which adds what the lanes past its end would (zeros).
         const int K = nd.dims[0];
         if (K <= 16) {
             for (int r = threadIdx.x; r < n; r += kTinyThreads) {
@@ -451,13 +451,18 @@ __device__ __forceinline__ void run_node(const Node &of, AP a, AP b, float *dstL
         }
         const int lane = threadIdx.x & 63;
         for (int r = threadIdx.x >> 6; r < n; r += kTinyThreads / 64) {
-            float acc = 0.0f;
-            for (int c = lane; c < K; c += 64) acc += a[(size_t)r * K + c] * b[c];
+            float total = 0.0f;
+            for (int k0 = 0; k0 < K; k0 += 1024) {
+                const int k1 = min(K, k0 + 1024);
+                float acc = 0.0f;
+                for (int c = k0 + lane; c < k1; c += 64) acc += a[(size_t)r * K + c] * b[c];
 #pragma unroll
-            for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
+                for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
+                total = k0 == 0 ? acc : total + acc;
+            }
             if (lane == 0) {
-                if (dstL) dstL[r] = acc;
-                if (dstG) dstG[r] = acc;
+                if (dstL) dstL[r] = total;
+                if (dstG) dstG[r] = total;
             }
         }
         break;

@@ -332,10 +332,10 @@ struct Generator {
                 publish(k);
                 break;
             }
-            put("    for (int r = t >> 6; r < " + num(n) + "; r += " + num(threads / 64) + ") {\n        float acc = 0.0f;\n        for (int c = t & 63; c < " + num(K) +
-                "; c += 64) acc += " + at(a, "r * " + num(K) + " + c") + " * " + at(b, "c") +
-                ";\n#pragma unroll\n        for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);\n        if ((t & 63) == 0) L[" + num(out.at) +
-                " + r] = acc;\n    }\n");
+            put("    for (int r = t >> 6; r < " + num(n) + "; r += " + num(threads / 64) + ") {\n        float total = 0.0f;\n        for (int k0 = 0; k0 < " + num(K) +
+                "; k0 += 1024) {\n            float acc = 0.0f;\n            for (int c = k0 + (t & 63); c < min(" + num(K) + ", k0 + 1024); c += 64) acc += " +
+                at(a, "r * " + num(K) + " + c") + " * " + at(b, "c") + ";\n#pragma unroll\n            for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);\n" +
+                "            total = k0 == 0 ? acc : total + acc;\n        }\n        if ((t & 63) == 0) L[" + num(out.at) + " + r] = total;\n    }\n");
             out.made = epoch;
             unstored.push_back(k);
             break;

@@ -949,6 +949,34 @@ def test_products_of_few_tiles_cut_their_reduction(shape):
             assert np.array_equal(g.numpy(), np.where(mask > 0, got, np.float32(0)))
 
 
+@pytest.mark.parametrize("n,k", [(512, 512), (1252, 784), (10, 25088), (777, 2500), (1, 70000), (33, 65), (5000, 3), (7, 1025), (31, 1024),
+                                 (64, 2), (1, 2), (100001, 130), (3, 5000), (32, 63)])
+def test_vector_products_have_one_order(n, k):
+    """A matrix times a vector: the same bits whether the matrix is stored by rows or by columns, whichever side it stands on, with
+    the epilogues and in a batch.  Bound: six standard deviations of 32 roundings of partial sums no larger than sqrt(k)."""
+    from dopt_amd import capi
+    r = rng(n + k)
+    m, v = r.standard_normal((n, k)).astype(np.float32), r.standard_normal(k).astype(np.float32)
+    mT = np.ascontiguousarray(m.T)
+    want = m.astype(np.float64) @ v.astype(np.float64)
+    tm, tmT, row, col = T(m), T(mT), T(v.reshape(1, k)), T(v.reshape(k, 1))
+    got = ops.matmul(tm, col).numpy().ravel()
+    assert np.abs(got - want).max() <= 2.0 ** -24 * 6 * np.sqrt(32) * np.sqrt(k)
+    lib = capi.load()
+    loose = T(np.concatenate([[1.0], mT.ravel()]).astype(np.float32)).view(1, (k, n))
+    forms = [(tmT, col, 1, 0, n, 1), (row, tmT, 0, 0, 1, n), (row, tm, 0, 1, 1, n), (col, tm, 1, 1, 1, n), (loose, row, 1, 1, n, 1)]
+    bias, scale, mask = r.standard_normal(n).astype(np.float32), np.float32(0.75), r.standard_normal(n).astype(np.float32)
+    for a, b, ta, tb, M, N in forms:
+        assert lib.dopt_hip_sgemm_order(ta, tb, M, N, k) == lib.dopt_hip_sgemm_order(0, 0, n, 1, k) or n == 1
+        assert np.array_equal(ops.matmul_t(a, b, trans_a=bool(ta), trans_b=bool(tb)).numpy().ravel(), got), (ta, tb, M, N)
+        u, w = (T(bias), T(np.array([scale]))) if N == 1 else (T(np.array([scale])), T(bias))
+        f = ops.matmul_rank1(a, b, u, w, relu=True, trans_a=bool(ta), trans_b=bool(tb)).numpy().ravel()
+        assert np.array_equal(f, np.maximum(got + scale * bias, np.float32(0)))
+        g, x = ops.Tensor((n,)), T(mask)
+        capi.check(lib.dopt_hip_sgemm_relu_grad(ta, tb, M, N, k, a.ptr, b.ptr, x.ptr, g.ptr))
+        assert np.array_equal(g.numpy(), np.where(mask > 0, got, np.float32(0)))
+
+
 @pytest.mark.parametrize("shape", [(12, 32768, 32), (32768, 12, 16), (12, 32768, 100), (64, 8192, 512), (8192, 64, 512),
                                    (33, 70000, 40), (70000, 33, 40), (128, 2048, 2048), (2048, 128, 2048),
                                    (256, 256, 8192), (1, 3000, 77), (3000, 1, 77), (1, 5000, 700), (5000, 1, 700),
