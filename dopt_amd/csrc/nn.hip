@@ -324,6 +324,32 @@ __global__ __launch_bounds__(kBlock) void softmax_fwd_k(size_t N, size_t C, size
     }
 }
 
+// The same for at most kMost channels, kept in registers: all loads together, then the operations above in their order (one after
+// the other they went to memory three times a channel: ten classes of one row 5.4 us, now 3.5; 17310 rows of 17 14.0 -> 8.9).
+template <int kMost>
+__global__ __launch_bounds__(kBlock) void softmax_few_fwd_k(size_t N, int C, size_t inner, const float *x, float *y)
+{
+    const size_t total = N * inner;
+    for (size_t idx = (size_t)blockIdx.x * kBlock + threadIdx.x; idx < total; idx += (size_t)gridDim.x * kBlock) {
+        const size_t n = idx / inner, i = idx % inner, base = n * C * inner + i;
+        float v[kMost], m = -FLT_MAX, s = 0.0f;
+#pragma unroll
+        for (int c = 0; c < kMost; c++) v[c] = x[base + (size_t)min(c, C - 1) * inner];
+#pragma unroll
+        for (int c = 0; c < kMost; c++)
+            if (c < C) m = dmax(m, v[c]);
+#pragma unroll
+        for (int c = 0; c < kMost; c++)
+            if (c < C) {
+                v[c] = expf(v[c] - m);
+                s += v[c];
+            }
+#pragma unroll
+        for (int c = 0; c < kMost; c++)
+            if (c < C) y[base + (size_t)c * inner] = v[c] / s;
+    }
+}
+
 // Rows of at least 64 contiguous channels (inner == 1): one wavefront per row, lanes stride along
 // the channels, maximum / sum / dot product folded with wavefront shuffles.  Sums are tree-ordered
 // here (the lane-per-row kernels sum in channel order).
@@ -719,6 +745,10 @@ int dopt_hip_softmax_fwd(size_t N, size_t C, size_t inner, const float *x, float
     } else if (inner == 1 && C >= 64)
         hipLaunchKernelGGL(softmax_rows_fwd_k, dim3((unsigned)ceil_div(N, (size_t)(kBlock / 64))), dim3(kBlock), 0, stream(),
                            N, C, x, y);
+    else if (C <= 16)
+        hipLaunchKernelGGL(softmax_few_fwd_k<16>, dim3(flat_grid(N * inner)), dim3(kBlock), 0, stream(), N, (int)C, inner, x, y);
+    else if (C <= 32)
+        hipLaunchKernelGGL(softmax_few_fwd_k<32>, dim3(flat_grid(N * inner)), dim3(kBlock), 0, stream(), N, (int)C, inner, x, y);
     else
         hipLaunchKernelGGL(softmax_fwd_k, dim3(flat_grid(N * inner)), dim3(kBlock), 0, stream(), N, C, inner, x, y);
     DOPT_LAUNCH_CHECK();

@@ -95,6 +95,19 @@ def test_reductions_as_nodes_equal_dopt_hip_reduce(shape, axes, op):
     assert np.array_equal(out.numpy().ravel(), want.ravel(), equal_nan=True)
 
 
+@pytest.mark.parametrize("shape", [(5, 1), (300, 2), (33, 15), (3, 16), (200, 17), (9, 31), (4, 32), (11, 33), (3, 16, 5), (2, 17, 3, 2)])
+def test_softmax_of_few_classes(shape):
+    """Kept in registers up to 16 and 32 classes: the bits of the node, which takes the classes in the reference's order."""
+    r = np.random.default_rng(int(np.prod(shape)))
+    x = (r.standard_normal(shape) * 5).astype(np.float32)
+    x.ravel()[0] = np.inf
+    x.ravel()[-1] = np.nan
+    inner = int(np.prod(shape[2:], dtype=np.int64))
+    tx, got = ops.tensor(x), ops.Tensor(shape)
+    _run([tx, got], [_node(SMAX, 1, 0, n=x.size, dims=(shape[0], shape[1], inner, 0))])
+    assert np.array_equal(ops.softmax(tx).numpy(), got.numpy(), equal_nan=True)
+
+
 @pytest.mark.parametrize("shape", [(128, 10), (100, 10), (7, 63), (4, 5, 3, 3), (2, 70, 2, 2)])
 def test_softmax_nodes_equal_their_kernels(shape):
     r = np.random.default_rng(3)
