@@ -1554,13 +1554,22 @@ __global__ __launch_bounds__(256) void wgrad_reduce_k(int K, int C, int Cp, int 
     for (int i = threadIdx.x; i < nelem; i += 256) dst[i] = stage[i];
 }
 
+// Quad i of a result of n values that may start anywhere and end inside a quad.
+__device__ __forceinline__ void store_loose(float *out, size_t n, size_t i, float4 v)
+{
+    const float q[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        if (4 * i + e < n) out[4 * i + e] = q[e];
+}
+
 // out[i] = sum over s of partial[s * stride + i], in a fixed order: split lane sl of a block folds
 // the splits s = sl, sl + SL, ... (four independent chains, then ((a0+a1)+(a2+a3))), and the SL
 // lane sums are added in lane order.  256 threads = (256 / SL) float4 columns x SL split lanes; SL
 // is chosen by the host so that small outputs with hundreds of splits still fill the machine.
-template <int SL>
+template <int SL, bool kLoose = false>
 __global__ __launch_bounds__(256) void split_sum_k(size_t n4, int splits, size_t stride4, const float4 *partial,
-                                                    float4 *out)
+                                                    float4 *out, size_t n = 0)
 {
     constexpr int EL = 256 / SL;
     __shared__ float4 part[SL][EL];
@@ -1593,7 +1602,8 @@ __global__ __launch_bounds__(256) void split_sum_k(size_t n4, int splits, size_t
             const float4 v = part[k][el];
             r.x += v.x; r.y += v.y; r.z += v.z; r.w += v.w;
         }
-        out[i] = r;
+        if constexpr (kLoose) store_loose((float *)out, n, i, r);
+        else out[i] = r;
     }
 }
 
@@ -2117,6 +2127,35 @@ __global__ __launch_bounds__(256) void splitk_reduce_k(size_t n4, int splits, co
     }
 }
 
+// The same for the general kernels, whose reductions are cut into up to sixty-four parts: added in float64 and rounded once (one fp32
+// rounding per part was most of the error: 66 -> 13 channels, 3 x 3, one image of 23 x 7, 1.3e-7 off float64, so 0.7e-7; the time
+// is that of the copies' bytes).  kLoose: the result's n values are no whole quads, or not on the 16-byte grid.
+template <bool kLoose>
+__global__ __launch_bounds__(256) void splitk_exact_k(size_t n4, int splits, const float4 *partial, float4 *out, size_t n)
+{
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256) {
+        double x = 0, y = 0, z = 0, w = 0;
+        const int last = splits - 1;
+        for (int s = 0; s < splits; s += 8) {   // eight loads in flight (indices clamped to the last part, surplus values dropped)
+            float4 v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = partial[(size_t)min(s + u, last) * n4 + i];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                if (s + u > last) continue;
+                if (s + u == 0) {   // not 0 + v: the sum of negative zeros stays a negative zero
+                    x = v[0].x, y = v[0].y, z = v[0].z, w = v[0].w;
+                } else {
+                    x += v[u].x, y += v[u].y, z += v[u].z, w += v[u].w;
+                }
+            }
+        }
+        const float4 sum = make_float4((float)x, (float)y, (float)z, (float)w);
+        if constexpr (kLoose) store_loose((float *)out, n, i, sum);
+        else out[i] = sum;
+    }
+}
+
 // The general kernels' packed filters (GatherConv::wp) from w[K][C][R][S]: of the whole filter (one class with R2 = R, S2 = S, no
 // stride) or of the sub-filters that the residue classes of a strided backward-data pass multiply.  Forward: rows = K, reduction
 // over C; backward: rows = C, reduction over K.  Rows up to Mp and channels up to a multiple of 16 are written, zeros where the
@@ -2204,6 +2243,21 @@ int check_desc(const dopt_hip_conv_desc *d, size_t *P, size_t *Q, const char *wh
     const size_t lim = (size_t)1 << 29;  // byte offsets of valid elements stay below 2^31
     DOPT_REQUIRE(d->N * d->C * d->H * d->W < lim && d->N * d->K * *P * *Q < lim && d->K * d->C * d->R * d->S < lim,
                  "%s: tensors of 2^29 elements or more are not supported", who);
+    return DOPT_HIP_OK;
+}
+
+// Floats from one partial copy of a general kernel's result, or of a filter gradient, to the next.
+size_t copy_stride(size_t elems) { return (elems + 3) / 4 * 4; }
+
+int launch_splitk_exact(size_t elems, int splits, const float *partial, float *out)
+{
+    const size_t n4 = copy_stride(elems) / 4;
+    const dim3 grid((unsigned)std::min(ceil_div(n4, (size_t)256), (size_t)num_cus() * 8));
+    if (elems % 4 != 0 || !aligned16(out))
+        hipLaunchKernelGGL(splitk_exact_k<true>, grid, dim3(256), 0, stream(), n4, splits, (const float4 *)partial, (float4 *)out, elems);
+    else
+        hipLaunchKernelGGL(splitk_exact_k<false>, grid, dim3(256), 0, stream(), n4, splits, (const float4 *)partial, (float4 *)out, elems);
+    DOPT_LAUNCH_CHECK();
     return DOPT_HIP_OK;
 }
 
@@ -2432,7 +2486,8 @@ int patch_splits(int tiles, int chunks, int slots, int BM, int BN, size_t out_el
 // The same estimate for the general kernels, whose unit is a slab of 16 reduction steps, at the rate that one CU sustains (0.33 on the
 // fp32 instruction; measured above).
 constexpr double kGatherRate = 0.6;
-int gather_splits(int tiles, int slabs, int slots, int BM, int BN, size_t out_elems, double cu_tflops, int cap)
+// sum_us: what the launch that adds the parts takes beside their bytes, where there would be none without a cut.
+int gather_splits(int tiles, int slabs, int slots, int BM, int BN, size_t out_elems, double cu_tflops, int cap, double sum_us)
 {
     const double per_cu = (double)slots / num_cus();
     const double t_slab = 2.0 * BM * BN * 16 / (cu_tflops * 1e6 / per_cu);
@@ -2443,7 +2498,7 @@ int gather_splits(int tiles, int slabs, int slots, int BM, int BN, size_t out_el
         if (sp > 1 && (slabs + per_block - 1) / per_block != sp) continue;
         const double rounds = (double)(((long long)tiles * sp + slots - 1) / slots);
         double cost = rounds * (per_block * t_slab + 6.0);
-        if (sp > 1) cost += 3.0 + (sp + 1.0) * out_elems * 4.0 / 4.5e6;
+        if (sp > 1) cost += sum_us + (sp + 1.0) * out_elems * 4.0 / 4.5e6;
         if (sp == 1 || cost < best_cost * 0.97) {
             best = sp;
             best_cost = cost;
@@ -2927,9 +2982,10 @@ int gather_launch(GatherConv g, bool bwd, int K, int C, const float *in, const f
     g.mtiles = (g.Mout + BM - 1) / BM;
     g.ntiles = (g.ncols + BN - 1) / BN;
     const int tiles = g.mtiles * g.ntiles;
-    int splits = gather_splits(tiles, g.slabs_total, num_cus(), BM, BN, g.out_elems, kGatherRate, 64);
-    // the split reduction works on float4 over a dense output
-    if (g.out_elems % 4 != 0 || !aligned16(out) || !dense) splits = 1;
+    int splits = gather_splits(tiles, g.slabs_total, num_cus(), BM, BN, g.out_elems, kGatherRate, 64, 4.5);
+    if (!dense) splits = 1;   // (the copies would be whole tensors)
+    const size_t elems = g.out_elems;
+    g.out_elems = copy_stride(elems);
     g.slabs_per_split = (g.slabs_total + splits - 1) / splits;
     splits = (g.slabs_total + g.slabs_per_split - 1) / g.slabs_per_split;  // no empty split
     g.splits = splits;
@@ -2963,7 +3019,7 @@ int gather_launch(GatherConv g, bool bwd, int K, int C, const float *in, const f
     if (int rc = brief ? (wide ? launch_gather<GatherWide, 1>(bwd, g, grid) : launch_gather<GatherSquare, 1>(bwd, g, grid))
                        : (wide ? launch_gather<GatherWide, 2>(bwd, g, grid) : launch_gather<GatherSquare, 2>(bwd, g, grid)))
         return rc;
-    if (splits > 1) return launch_splitk_reduce(g.out_elems, splits, partial, out);
+    if (splits > 1) return launch_splitk_exact(elems, splits, partial, out);
     return DOPT_HIP_OK;
 }
 
@@ -3030,15 +3086,41 @@ int run_bwd_strided(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float
         const int KPad = round_up(K, BK), Mp = round_up(C, 4);
         if ((size_t)BK * Mp * sizeof(float) > 0x7fffffffu)
             return fail(DOPT_HIP_ERR_UNSUPPORTED, "convolution: more than 2^25 output channels are not supported");
+        // The classes' reductions are cut into the same number of parts, each a partial copy of the whole of dx: where a handful of
+        // tiles would be as many workgroups of a long chain (47 images of 4 x 11, 300 channels to 5: 60 us, now 14 with the sum).
+        const bool wide = C <= 64 || (C + 63) / 64 * 64 < (C + 127) / 128 * 128;
+        const int BM = wide ? 64 : 128, BN = wide ? 256 : 128;
+        const size_t elems = d->N * d->C * d->H * d->W;
+        int splits = 1;
+        if (!gaps) {   // (a copy has no value where no tap reaches)
+            const double t_slab = 2.0 * BM * BN * 16 / (kGatherRate * 1e6);
+            double best = 0;
+            for (int sp = 1; sp <= 32; sp++) {
+                double total = 0, longest = 0;
+                bool full = true;
+                for (int j = 0; j < njobs; j++) {
+                    const int slabs = jobs[j].ch.taps * jobs[j].cw.taps * KPad / BK, per = (slabs + sp - 1) / sp;
+                    const double tiles = ceil_div((size_t)C, (size_t)BM) * ceil_div((size_t)d->N * jobs[j].ch.n * jobs[j].cw.n, (size_t)BN);
+                    full = full && (sp - 1) * per < slabs;
+                    total += tiles * sp * (per * t_slab + 6.0);
+                    longest = std::max(longest, per * t_slab + 6.0);
+                }
+                if (!full) continue;
+                const double cost = std::max(total / num_cus(), longest) + (sp > 1 ? 4.5 + (sp + 1.0) * elems * 4.0 / 4.5e6 : 0.0);
+                if (sp == 1 || cost < best * 0.9) {
+                    splits = sp;
+                    best = cost;
+                }
+            }
+        }
         size_t wp_off[kGatherJobs + 1] = {0};
         for (int j = 0; j < njobs; j++) {
             const size_t slabs = (size_t)jobs[j].ch.taps * jobs[j].cw.taps * KPad / BK;
             wp_off[j + 1] = wp_off[j] + (slabs * Mp * 96 + 255) / 256 * 256;
         }
-        char *ws = (char *)workspace(wp_off[njobs]);
+        char *ws = (char *)workspace(wp_off[njobs] + (splits > 1 ? (size_t)splits * copy_stride(elems) * sizeof(float) : 0));
         if (!ws) return DOPT_HIP_ERR_OOM;
-        const bool wide = C <= 64 || (C + 63) / 64 * 64 < (C + 127) / 128 * 128;
-        const int BM = wide ? 64 : 128, BN = wide ? 256 : 128;
+        float *const partial = (float *)(ws + wp_off[njobs]);
         SubFilters subs{};
         GatherGroup gg{};
         subs.n = gg.n = njobs;
@@ -3059,21 +3141,24 @@ int run_bwd_strided(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float
             g.Mp = Mp;
             g.ncols = g.N * g.OH * g.OW;
             g.slabs_total = g.R * g.S * KPad / BK;
-            g.slabs_per_split = g.slabs_total;
-            g.splits = 1;   // a class's pixels are scattered over dx: nothing for a split sum to add in place
-            g.out_elems = (size_t)g.ncols * g.Mout;
+            g.slabs_per_split = (g.slabs_total + splits - 1) / splits;
+            g.splits = splits;
+            g.out_elems = copy_stride(elems);
             g.mtiles = (g.Mout + BM - 1) / BM;
             g.ntiles = (g.ncols + BN - 1) / BN;
             g.in = dy;
             g.wp = subs.f[j].wp;
-            g.out = dx;
+            g.out = splits > 1 ? partial : dx;
             g.in_bytes = (size_t)g.N * g.Cin * g.IH * g.IW * sizeof(float);
-            gg.per[j] = ((unsigned)(g.mtiles * g.ntiles) + 7u) / 8u;
+            gg.per[j] = ((unsigned)(g.mtiles * g.ntiles * splits) + 7u) / 8u;
             blocks += 8u * gg.per[j];
         }
         if (int rc = launch_pack_gather(true, K, C, R, S, sH, sW, Mp, w, subs)) return rc;
-        if (wide) return launch_gather_kernel<GatherWide, 2, conv_gather_group_k<GatherWide, 2, true>>(gg, blocks);
-        return launch_gather_kernel<GatherSquare, 2, conv_gather_group_k<GatherSquare, 2, true>>(gg, blocks);
+        if (int rc = wide ? launch_gather_kernel<GatherWide, 2, conv_gather_group_k<GatherWide, 2, true>>(gg, blocks)
+                          : launch_gather_kernel<GatherSquare, 2, conv_gather_group_k<GatherSquare, 2, true>>(gg, blocks))
+            return rc;
+        if (splits > 1) return launch_splitk_exact(elems, splits, partial, dx);
+        return DOPT_HIP_OK;
     }
     void *sub = nullptr;
     if (int rc = scratch_alloc(&sub, d->K * d->C * d->R * d->S * sizeof(float))) return rc;
@@ -3197,6 +3282,7 @@ struct WgradSetup {
     WgradPatch wp;
     bool tall;            // 128 rows x 32 channels per block
     bool pre;             // x is split when it is stored
+    bool quads;           // the result is whole quads on the 16-byte grid (else its partial copies are added here, never left open)
     int rows;             // output channels per block: 128 (tall), 160 (x 32 channels) or 64 (x 64 channels)
     int geo, tiles, splits;
     size_t out_elems, lds_bytes;
@@ -3280,12 +3366,11 @@ WgradSetup wgrad_patch_setup(const dopt_hip_conv_desc *d, const float *dw)
             }
         }
     }
-    const bool whole = out_elems % 4 != 0 || !aligned16(dw);
-    if (whole) splits = 1;  // the split sum works on float4
+    u.quads = out_elems % 4 == 0 && aligned16(dw);
     // 64-row tiles on 4 x 4 images: few workgroups of a long set-up unless the layer or the batch is large, and one without a split
     // (16 images, 64 -> 64 channels: 20 us, the general kernel 10; 140, 62 -> 27: 135 and 18; 128, 128 -> 48: 21 and 18; but 256, 16 -> 16:
     // 18 and 26; 512, 64 -> 64: 25 and 29; 128, 320 -> 320: 41 and 59; 192 -> 192, nine tiles, 8 to 128 images: within a tenth)
-    if (geo == 1 && BM == 64 && (whole || (tiles < 8 && d->N < 256))) return u;
+    if (geo == 1 && BM == 64 && (!u.quads || (tiles < 8 && d->N < 256))) return u;
     wp.chunks_per_split = (wp.chunks_total + splits - 1) / splits;
     splits = (wp.chunks_total + wp.chunks_per_split - 1) / wp.chunks_per_split;
     wp.splits = splits;
@@ -3293,7 +3378,7 @@ WgradSetup wgrad_patch_setup(const dopt_hip_conv_desc *d, const float *dw)
     const size_t lds_epi = (size_t)32 * (BC * 9 + 1) * sizeof(float);
     u.lds_bytes = lds_main > lds_epi ? lds_main : lds_epi;
     if (u.lds_bytes > 160 * 1024) return u;
-    wp.split_stride = out_elems;
+    wp.split_stride = copy_stride(out_elems);
     u.tall = tall; u.pre = pre; u.rows = BM; u.geo = geo; u.tiles = tiles; u.splits = splits; u.out_elems = out_elems;
     u.ok = true;
     return u;
@@ -3321,7 +3406,15 @@ int launch_split_sum(size_t n4, int splits, int lanes, const float *partial, flo
 // dw = the partial filters added in split order
 int wgrad_split_sum(const WgradSetup &u, const float *partial, float *dw)
 {
-    const size_t n4 = u.out_elems / 4;
+    const size_t n4 = u.wp.split_stride / 4;
+    if (!u.quads) {
+        const bool few = wgrad_sum_lanes(n4) == 16;
+        const dim3 grid((unsigned)ceil_div(n4, (size_t)(few ? 16 : 64)));
+        if (few) hipLaunchKernelGGL((split_sum_k<16, true>), grid, dim3(256), 0, stream(), n4, u.splits, n4, (const float4 *)partial, (float4 *)dw, u.out_elems);
+        else hipLaunchKernelGGL((split_sum_k<4, true>), grid, dim3(256), 0, stream(), n4, u.splits, n4, (const float4 *)partial, (float4 *)dw, u.out_elems);
+        DOPT_LAUNCH_CHECK();
+        return DOPT_HIP_OK;
+    }
     return launch_split_sum(n4, u.splits, wgrad_sum_lanes(n4), partial, dw);
 }
 
@@ -3351,7 +3444,7 @@ int run_wgrad_patch(const dopt_hip_conv_desc *d, const float *dy, const float *x
     WgradPatch &wp = u.wp;
     float *partial = nullptr;
     if (u.splits > 1) {
-        partial = (float *)workspace((size_t)u.splits * u.out_elems * sizeof(float));
+        partial = (float *)workspace((size_t)u.splits * wp.split_stride * sizeof(float));
         if (!partial) return DOPT_HIP_ERR_OOM;
     }
     wp.dy = dy; wp.x = x;
@@ -3401,13 +3494,13 @@ int run_bwd_pair(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float *d
     // sum rides in the batch-norm gradient there instead of being a launch of its own.  (The same for the 64-row layers
     // was measured and does not pay: they are followed by the multi-block batch norm, whose workgroups fill every CU,
     // so the riders only start when those have finished - 20 us per layer instead of the 7.6 us of the separate sum.)
-    const bool two = combo < 0 && a.shape == 4 && a.BM == 128 && open_dw != nullptr && b.splits > 1;
+    const bool two = combo < 0 && a.shape == 4 && a.BM == 128 && open_dw != nullptr && b.splits > 1 && b.quads;
     if (combo < 0 && !two) return DOPT_HIP_OK;
     PatchConv &pc = a.pc;
     WgradPatch &wp = b.wp;
     const int splits_a = patch_decide_splits(&a, dx);
     const size_t part_a = splits_a > 1 ? ((size_t)splits_a * pc.out_elems * sizeof(float) + 255) / 256 * 256 : 0;
-    const size_t part_b = b.splits > 1 ? (size_t)b.splits * b.out_elems * sizeof(float) : 0;
+    const size_t part_b = b.splits > 1 ? (size_t)b.splits * wp.split_stride * sizeof(float) : 0;
     char *ws = part_a + part_b > 0 ? (char *)workspace(part_a + part_b) : nullptr;
     if (part_a + part_b > 0 && !ws) return DOPT_HIP_ERR_OOM;
     float *partial_a = (float *)ws, *partial_b = (float *)(ws + part_a);
@@ -3438,7 +3531,7 @@ int run_bwd_pair(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float *d
         probe.bytes += 4.0 * (2.0 * px * d->C + px * d->K + 2.0 * (double)d->K * d->C * 9.0);   // dy, x, dx, filter, dw once each
     }
     *done = true;
-    if (b.splits > 1 && open_dw) {   // the caller's next call adds the copies
+    if (b.splits > 1 && open_dw && b.quads) {   // the caller's next call adds the copies
         open_dw->partial = partial_b;
         open_dw->splits = b.splits;
         open_dw->elems = b.out_elems;
@@ -3756,7 +3849,7 @@ int dopt_hip_conv_bwd_filter(const dopt_hip_conv_desc *d, const float *dy, const
     f.ntiles = (f.ncols + BN - 1) / BN;
     const int tiles = f.mtiles * f.ntiles;
     // filter gradients are short and wide (small output, long pixel reduction): allow deep splits
-    int splits = gather_splits(tiles, f.slabs_total, big ? num_cus() : 2 * num_cus(), BM, BN, f.out_elems, kGatherRate, 512);
+    int splits = gather_splits(tiles, f.slabs_total, big ? num_cus() : 2 * num_cus(), BM, BN, f.out_elems, kGatherRate, 512, 3.0);
     f.slabs_per_split = (f.slabs_total + splits - 1) / splits;
     splits = (f.slabs_total + f.slabs_per_split - 1) / f.slabs_per_split;
     f.splits = splits;

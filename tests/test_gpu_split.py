@@ -502,6 +502,51 @@ def test_general_convolution_of_short_reductions(shape):
         assert not fine.all() and fine.mean() > 0.9 and np.array_equal(again[fine], plain[fine])
 
 
+# results of odd counts whose reductions are cut: forward, backward-data, both; the classes of a stride (with classes that no tap reaches);
+# filter gradients of K C 9 values (128 x 32 and 64 x 64 tiles, rows of 8, 16 and 32 pixels)
+@pytest.mark.parametrize("shape", [(3, 116, 21, 11, 9, 5, 2, 1), (1, 507, 9, 13, 215, 3, 0, 1), (3, 51, 23, 7, 617, 3, 1, 1), (1, 66, 23, 7, 13, 3, 1, 1), (5, 459, 5, 11, 407, 1, 0, 1),
+                                   (47, 5, 4, 11, 300, 3, 0, 2), (1, 123, 5, 7, 366, 3, 0, 2), (3, 7, 9, 7, 385, 5, 2, 3), (2, 9, 11, 7, 333, 1, 0, 2), (1, 86, 5, 8, 128, 3, 1, 2),
+                                   (100, 33, 16, 16, 43, 3, 1, 1), (64, 35, 8, 8, 131, 3, 1, 1), (12, 17, 32, 32, 21, 3, 1, 1)])
+def test_results_of_odd_counts_are_cut_too(shape):
+    N, C, H, W, K, R, pad, stride = shape
+    r = rng(C + K + R)
+    x, w = r.standard_normal((N, C, H, W), np.float32), r.standard_normal((K, C, R, R), np.float32)
+    ps = ((pad, pad), (stride, stride))
+    got = ops.convolution(T(x), T(w), *ps).numpy()
+    dy = r.standard_normal(got.shape, np.float32)
+    dx, dw = ops.conv_bwd_data(T(dy), T(w), x.shape, *ps).numpy(), ops.conv_bwd_filter(T(dy), T(x), w.shape, *ps).numpy()
+    wants = general_gradients(x, w, dy, pad, stride)
+    check_norm(got, general(x, w, pad, stride), C * R * R, shape)
+    check_norm(dx, wants[0], K * R * R / stride ** 2, shape)
+    check_norm(dw, wants[1], dy[:, 0].size, shape)
+    # into results off the 16-byte grid: nothing around them is touched
+    for want, run in ((got, lambda o: ops.convolution(T(x), T(w), *ps, out=o)), (dx, lambda o: ops.conv_bwd_data(T(dy), T(w), x.shape, *ps, out=o)),
+                      (dw, lambda o: ops.conv_bwd_filter(T(dy), T(x), w.shape, *ps, out=o))):
+        whole = T(np.full(want.size + 8, 7.0, np.float32))
+        run(whole.view(1, want.shape))
+        flat = whole.numpy()
+        assert (flat[:1] == 7.0).all() and (flat[1 + want.size:] == 7.0).all()
+        assert np.allclose(flat[1:1 + want.size], want.ravel(), rtol=1e-4, atol=1e-5 * np.sqrt(C * R * R + K * R * R))
+
+
+def test_odd_filter_gradients_in_a_plan():
+    """A backward pair whose filter gradient has an odd count beside the batch norm that adds riding sums: it adds its own."""
+    from dopt_amd import core, nnet
+    x, y = core.float32([64, 65, 8, 8]), core.float32([64, 10])
+    init = nnet.Init(3)
+    h = nnet.relu(nnet.batchNorm(nnet.conv2D(nnet.dataSource(x), 33, (3, 3), init, padding=(1, 1))))
+    h = nnet.relu(nnet.batchNorm(nnet.conv2D(h, 143, (3, 3), init, padding=(1, 1))))
+    h = nnet.relu(nnet.batchNorm(nnet.conv2D(h, 145, (3, 3), init, padding=(1, 1))))
+    net = nnet.DAGNetwork([x], [nnet.softmax(nnet.dense(h, 10, init))])
+    loss = nnet.crossEntropy(net.outputs[0].trainOutput, y)
+    outs = [loss] + core.grad(loss, net.params)
+    r = rng(4)
+    args = {x: r.standard_normal((64, 65, 8, 8), np.float32), y: np.eye(10, dtype=np.float32)[r.integers(0, 10, 64)]}
+    a, b = (core.compile(outs, f).execute(args) for f in (core.PLAN_VIEWS, core.PLAN_VIEWS | core.PLAN_FUSE))
+    for p, q, o in zip(a, b, outs):
+        assert np.allclose(p, q, rtol=1e-4, atol=1e-5 * max(1.0, float(np.abs(p).max()))), o.shape
+
+
 def test_general_convolution_operands_that_are_not_finite():
     """A value far from every bad one is what it is without them; an infinity stays one and a NaN stays one."""
     r = rng(3)
