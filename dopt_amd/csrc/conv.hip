@@ -2284,6 +2284,9 @@ int launch_splitk_reduce(size_t elems, int splits, const float *partial, float *
 
 // Eight wavefronts of 32 x 64, one workgroup per CU.  (Four of 64 x 64, two workgroups per CU, hid their loads as well but had
 // twice the values to split per wavefront: 5 x 5 layers backward-data 104 against 101 us before the splitting was overlapped.)
+// Up to 32 output channels: 64 rows would multiply as many zeros (3 x 3, 108 images of 16 x 57, 11 -> 16 channels: 27 -> 21 us; 418 -> 28, 222
+// of 10 x 35, 174 -> 142).
+using GatherNarrow = Tile<32, 256, 1, 8>;
 using GatherWide = Tile<64, 256, 2, 4>;     // few output channels, many pixels
 using GatherSquare = Tile<128, 128, 4, 2>;
 
@@ -2977,12 +2980,13 @@ int gather_launch(GatherConv g, bool bwd, int K, int C, const float *in, const f
 
     // tile shape: 64-row tiles for <= 64 output channels and wherever 128-row tiles would pad more;
     // otherwise 128x128
-    const bool wide = g.Mout <= 64 || (g.Mout + 63) / 64 * 64 < (g.Mout + 127) / 128 * 128;
-    const int BM = wide ? 64 : 128, BN = wide ? 256 : 128;
+    const bool narrow = g.Mout <= 32, wide = !narrow && (g.Mout <= 64 || (g.Mout + 63) / 64 * 64 < (g.Mout + 127) / 128 * 128);
+    const int BM = narrow ? 32 : wide ? 64 : 128, BN = narrow || wide ? 256 : 128;
     g.mtiles = (g.Mout + BM - 1) / BM;
     g.ntiles = (g.ncols + BN - 1) / BN;
     const int tiles = g.mtiles * g.ntiles;
-    int splits = gather_splits(tiles, g.slabs_total, num_cus(), BM, BN, g.out_elems, kGatherRate, 64, 4.5);
+    // (tiles of 32 rows are cut as those of 64: staging is most of a slab there, and longer chains would be further off)
+    int splits = gather_splits(tiles, g.slabs_total, num_cus(), std::max(BM, 64), BN, g.out_elems, kGatherRate, 64, 4.5);
     if (!dense) splits = 1;   // (the copies would be whole tensors)
     const size_t elems = g.out_elems;
     g.out_elems = copy_stride(elems);
@@ -3016,7 +3020,9 @@ int gather_launch(GatherConv g, bool bwd, int K, int C, const float *in, const f
     // slabs, 275 -> 266; but 42 -> 592, 3 x 3, 515 tiles of 27 slabs, 1.3 times as far off).
     const int cus = num_cus();
     const bool brief = splits == 1 && g.slabs_total <= (tiles >= 4 * cus ? 32 : tiles >= 2 * cus ? 9 : tiles > cus ? 3 : 0);
-    if (int rc = brief ? (wide ? launch_gather<GatherWide, 1>(bwd, g, grid) : launch_gather<GatherSquare, 1>(bwd, g, grid))
+    if (narrow) {
+        if (int rc = brief ? launch_gather<GatherNarrow, 1>(bwd, g, grid) : launch_gather<GatherNarrow, 2>(bwd, g, grid)) return rc;
+    } else if (int rc = brief ? (wide ? launch_gather<GatherWide, 1>(bwd, g, grid) : launch_gather<GatherSquare, 1>(bwd, g, grid))
                        : (wide ? launch_gather<GatherWide, 2>(bwd, g, grid) : launch_gather<GatherSquare, 2>(bwd, g, grid)))
         return rc;
     if (splits > 1) return launch_splitk_exact(elems, splits, partial, out);
@@ -3088,12 +3094,12 @@ int run_bwd_strided(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float
             return fail(DOPT_HIP_ERR_UNSUPPORTED, "convolution: more than 2^25 output channels are not supported");
         // The classes' reductions are cut into the same number of parts, each a partial copy of the whole of dx: where a handful of
         // tiles would be as many workgroups of a long chain (47 images of 4 x 11, 300 channels to 5: 60 us, now 14 with the sum).
-        const bool wide = C <= 64 || (C + 63) / 64 * 64 < (C + 127) / 128 * 128;
-        const int BM = wide ? 64 : 128, BN = wide ? 256 : 128;
+        const bool narrow = C <= 32, wide = !narrow && (C <= 64 || (C + 63) / 64 * 64 < (C + 127) / 128 * 128);
+        const int BM = narrow ? 32 : wide ? 64 : 128, BN = narrow || wide ? 256 : 128;
         const size_t elems = d->N * d->C * d->H * d->W;
         int splits = 1;
         if (!gaps) {   // (a copy has no value where no tap reaches)
-            const double t_slab = 2.0 * BM * BN * 16 / (kGatherRate * 1e6);
+            const double t_slab = 2.0 * std::max(BM, 64) * BN * 16 / (kGatherRate * 1e6);
             double best = 0;
             for (int sp = 1; sp <= 32; sp++) {
                 double total = 0, longest = 0;
@@ -3154,7 +3160,8 @@ int run_bwd_strided(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float
             blocks += 8u * gg.per[j];
         }
         if (int rc = launch_pack_gather(true, K, C, R, S, sH, sW, Mp, w, subs)) return rc;
-        if (int rc = wide ? launch_gather_kernel<GatherWide, 2, conv_gather_group_k<GatherWide, 2, true>>(gg, blocks)
+        if (int rc = narrow ? launch_gather_kernel<GatherNarrow, 2, conv_gather_group_k<GatherNarrow, 2, true>>(gg, blocks)
+                   : wide ? launch_gather_kernel<GatherWide, 2, conv_gather_group_k<GatherWide, 2, true>>(gg, blocks)
                           : launch_gather_kernel<GatherSquare, 2, conv_gather_group_k<GatherSquare, 2, true>>(gg, blocks))
             return rc;
         if (splits > 1) return launch_splitk_exact(elems, splits, partial, dx);
