@@ -1566,7 +1566,8 @@ __device__ __forceinline__ void store_loose(float *out, size_t n, size_t i, floa
 // The same for small filters of many copies, where K blocks a chunk leave the chip idle and a thread goes through its copies several
 // times: a block takes 64 of a row's elements in the copies' order and sixteen split lanes (lane sl: copies sl, sl + 16 .., four
 // chains), whose sums are added in order, all in float64 (with sixteen roundings in a row the error was 1.1 times wgrad_reduce_k's).
-// Results are written a word at a time.  32 x 16 x 9 values from 256 copies 9.3 -> 4.6 us, 100 x 48 x 25 from 23 10.1 -> 7.0.
+// Results are written a word at a time.  The five such layers of a WRN-10-2 step on 64 images 9.3 -> 5 us each, 100 x 48 x 25 values
+// 10.1 -> 7.4.
 __global__ __launch_bounds__(1024) void wgrad_reduce_small_k(int C, int Cp, int taps, int splits, size_t split_stride, const float *partial, float *dw)
 {
     __shared__ double part[16][64];
@@ -2166,7 +2167,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_k(size_t n4, int splits, co
 // rounding per part was most of the error: 66 -> 13 channels, 3 x 3, one image of 23 x 7, 1.3e-7 off float64, so 0.7e-7; the time
 // is that of the copies' bytes).  kLoose: the result's n values are no whole quads, or not on the 16-byte grid.
 template <bool kLoose>
-__global__ __launch_bounds__(256) void splitk_exact_k(size_t n4, int splits, const float4 *partial, float4 *out, size_t n)
+__global__ __launch_bounds__(256) void splitk_exact_k(size_t n4, int splits, const float4 *partial, float4 *out, size_t n, const float *bias, unsigned C,
+                                                       unsigned inner)
 {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256) {
         double x = 0, y = 0, z = 0, w = 0;
@@ -2185,7 +2187,14 @@ __global__ __launch_bounds__(256) void splitk_exact_k(size_t n4, int splits, con
                 }
             }
         }
-        const float4 sum = make_float4((float)x, (float)y, (float)z, (float)w);
+        float4 sum = make_float4((float)x, (float)y, (float)z, (float)w);
+        if (bias) {
+            const size_t e = i * 4;
+            sum.x += bias[(e / inner) % C];
+            sum.y += bias[((e + 1) / inner) % C];
+            sum.z += bias[((e + 2) / inner) % C];
+            sum.w += bias[((e + 3) / inner) % C];
+        }
         if constexpr (kLoose) store_loose((float *)out, n, i, sum);
         else out[i] = sum;
     }
@@ -2284,14 +2293,14 @@ int check_desc(const dopt_hip_conv_desc *d, size_t *P, size_t *Q, const char *wh
 // Floats from one partial copy of a general kernel's result, or of a filter gradient, to the next.
 size_t copy_stride(size_t elems) { return (elems + 3) / 4 * 4; }
 
-int launch_splitk_exact(size_t elems, int splits, const float *partial, float *out)
+int launch_splitk_exact(size_t elems, int splits, const float *partial, float *out, const float *bias = nullptr, unsigned C = 1, unsigned inner = 1)
 {
     const size_t n4 = copy_stride(elems) / 4;
     const dim3 grid((unsigned)std::min(ceil_div(n4, (size_t)256), (size_t)num_cus() * 8));
     if (elems % 4 != 0 || !aligned16(out))
-        hipLaunchKernelGGL(splitk_exact_k<true>, grid, dim3(256), 0, stream(), n4, splits, (const float4 *)partial, (float4 *)out, elems);
+        hipLaunchKernelGGL(splitk_exact_k<true>, grid, dim3(256), 0, stream(), n4, splits, (const float4 *)partial, (float4 *)out, elems, bias, C, inner);
     else
-        hipLaunchKernelGGL(splitk_exact_k<false>, grid, dim3(256), 0, stream(), n4, splits, (const float4 *)partial, (float4 *)out, elems);
+        hipLaunchKernelGGL(splitk_exact_k<false>, grid, dim3(256), 0, stream(), n4, splits, (const float4 *)partial, (float4 *)out, elems, bias, C, inner);
     DOPT_LAUNCH_CHECK();
     return DOPT_HIP_OK;
 }
@@ -2979,6 +2988,199 @@ int run_dense2x2_wgrad(const dopt_hip_conv_desc *d, const float *dy, const float
     return rc;
 }
 
+// ---- few output pixels: one image through a network ----------------------------------------------
+// Forward of up to 64 output pixels.  The filter is most of what such a layer moves and nothing of it is used more than 64 times, so it
+// is read once, as it lies: a row of it, [C][R][S], is the reduction in order, four steps of which a lane loads as 16 bytes whatever
+// their alignment, and the fp32 matrix instruction takes (32 rows, two steps).  A workgroup owns 32 rows, all pixels and a part
+// of the reduction, its eight wavefronts an eighth of that each.  The input under the part's channels lies in LDS with a halo of
+// zeros; a step's offset in it is read from a table.  Bound by the filter's bytes through launch and latency (512 -> 512 channels, 3 x 3, 16 pixels: 9.4 MB).
+// VGG-16 on one image, 261 us, now 191: its nine layers on 8 x 8, 4 x 4 and 2 x 2 images 7 to 9 us each (Winograd 9 to 11 and 17 to pack
+// their filters, conv2x2_direct_k 15).
+struct FewConv {
+    const float *x, *w, *bias;
+    float *out;                     // [N][K][P][Q], or `cuts` copies of it, out_elems apart
+    int N, C, H, W, K, R, S, padH, padW, strideH, strideW, P, Q;
+    int PR, PC, depth;              // extents of an image with its halo; steps of the reduction per part
+    size_t out_elems, w_bytes, x_bytes;
+};
+constexpr int kFewPixels = 64, kFewWaves = 8, kFewDepthMax = 1024;
+
+template <int NP>   // groups of 32 pixels
+__global__ __launch_bounds__(64 * kFewWaves) void conv_few_k(FewConv p)
+{
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    float *const red = lds;                                        // [wavefront][group][32][33]
+    int *const offs = (int *)(lds + kFewWaves * NP * 32 * 33);     // of the part's steps, a multiple of eight
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int taps = p.R * p.S, total = p.C * taps, m0 = blockIdx.x * 32;
+    const int k0 = (int)blockIdx.y * p.depth, k1 = min(total, k0 + p.depth), steps = (k1 - k0 + 7) / 8 * 8;
+    float *const patch = (float *)(offs + (p.depth + 7) / 8 * 8);
+    const int c0 = k0 / taps, chans = (k1 - 1) / taps - c0 + 1, plane = p.PR * p.PC, chan = p.N * plane;
+
+    const int slice = (steps / 8 + kFewWaves - 1) / kFewWaves * 8, kb = k0 + wave * slice, ke = min(k1, kb + slice);
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(p.w, p.w_bytes);
+    const unsigned row = m0 + l32 < p.K ? (unsigned)(m0 + l32) * (unsigned)total * 4u : kOobOffset;
+    constexpr int DEPTH = 4;   // steps of eight in flight
+    float4 a[DEPTH];
+    auto load = [&](int k) { return buffer_load_f32x4(rw, k < ke ? row + (unsigned)k * 4u : kOobOffset, 0); };
+#pragma unroll
+    for (int j = 0; j < DEPTH; j++) a[j] = load(kb + 8 * j + 4 * half);
+
+    for (int i = tid; i < steps; i += 64 * kFewWaves) {
+        const int k = k0 + i, c = k / taps, t = k - c * taps, r = t / p.S, s = t - r * p.S;
+        offs[i] = k < k1 ? (c - c0) * chan + (p.R - 1 - r) * p.PC + (p.S - 1 - s) : 0;   // a true convolution
+    }
+    // a thread takes one place of every few channels: where it lies is found once
+    const int span = min(chan, 64 * kFewWaves), together = 64 * kFewWaves / span, first = tid / span;
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x, p.x_bytes);
+    for (int e = first < together ? tid - first * span : chan; e < chan; e += span) {
+        const int n = e / plane, f = e - n * plane, fr = f / p.PC, ih = fr - p.padH, iw = f - fr * p.PC - p.padW;
+        const bool in = ih >= 0 && ih < p.H && iw >= 0 && iw < p.W;
+        const unsigned hw4 = (unsigned)(p.H * p.W) * 4u, from = (unsigned)(((n * p.C + c0) * p.H + ih) * p.W + iw) * 4u;
+#pragma unroll 8
+        for (int c = first; c < chans; c += together)
+            patch[c * chan + e] = buffer_load_f32(rx, in ? from + (unsigned)c * hw4 : kOobOffset, 0);
+    }
+    __syncthreads();
+
+    int base[NP];
+    v16f acc[NP];
+#pragma unroll
+    for (int g = 0; g < NP; g++) {
+        const int px = min(32 * g + l32, p.N * p.P * p.Q - 1), n = px / (p.P * p.Q), pq = px - n * p.P * p.Q, oh = pq / p.Q, ow = pq - oh * p.Q;
+        base[g] = n * plane + oh * p.strideH * p.PC + ow * p.strideW;
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[g][v] = 0.0f;
+    }
+    for (int k = kb; k < ke; k += 8 * DEPTH) {
+#pragma unroll
+        for (int j = 0; j < DEPTH; j++) {
+            const int kk = k + 8 * j + 4 * half;
+            const float av[4] = {a[j].x, a[j].y, a[j].z, a[j].w};
+            const int4 at = *(const int4 *)(offs + min(kk - k0, steps - 4));
+            const int o[4] = {at.x, at.y, at.z, at.w};
+            float in[NP][4];
+#pragma unroll
+            for (int g = 0; g < NP; g++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) in[g][e] = patch[o[e] + base[g]];
+            // what lies past the end counts as zero on both sides
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int g = 0; g < NP; g++)
+                    acc[g] = __builtin_amdgcn_mfma_f32_32x32x2f32(kk + e < ke ? av[e] : 0.0f, kk + e < ke ? in[g][e] : 0.0f, acc[g], 0, 0, 0);
+            a[j] = load(kk + 8 * DEPTH);
+            __builtin_amdgcn_sched_barrier(0);   // each refill stays behind its own step
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < NP; g++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) red[((wave * NP + g) * 32 + acc_row(v, lane)) * 33 + l32] = acc[g][v];
+    __syncthreads();
+    float *const out = p.out + (size_t)blockIdx.y * p.out_elems;
+#pragma unroll
+    for (int i = 0; i < 2 * NP; i++) {
+        const int idx = tid + i * 64 * kFewWaves, r = idx / (32 * NP), px = idx % (32 * NP);
+        const float *const from = red + ((px >> 5) * 32 + r) * 33 + (px & 31);
+        float sum = from[0];
+#pragma unroll
+        for (int w = 1; w < kFewWaves; w++) sum += from[w * NP * 32 * 33];
+        if (m0 + r < p.K && px < p.N * p.P * p.Q) {
+            const int n = px / (p.P * p.Q), pq = px - n * p.P * p.Q;
+            if (p.bias) sum += p.bias[m0 + r];
+            out[((size_t)n * p.K + m0 + r) * (p.P * p.Q) + pq] = sum;
+        }
+    }
+}
+
+struct FewSetup {
+    bool ok = false;
+    FewConv f{};
+    int cuts = 1;
+    size_t elems = 0, lds_bytes = 0;
+};
+// Against the kernels that run without it (transposed bf16 tiles, Winograd with its packing, a copy of the filter in rows and general
+// tiles): 512 -> 512 channels on 4 x 4 34 us, now 12; 640 -> 640 on 8 x 8 36, now 17; 320 -> 640 at stride 2 to 8 x 8 32, now 15;
+// 100 -> 201 on 7 x 9 48, now 11; 256 -> 32 on 4 x 4 20, now 9; 400 -> 300 on one pixel 15, now 8; nothing of 35 shapes slower.
+// The kernels of 2 x 2 images keep more than 32 pixels (512 -> 512 of 16 images: 14 us, 17 here), conv2x2_direct_k fewer than 384
+// input channels too (320 -> 320 of 8 images: 9.9 us, 10.7 here; 512 -> 512 of 8 images 14.0, 12.8 here, of one 13.8, 11.3 here).  Filters of
+// 2^27 values and more keep the kernels that are checked at such sizes (5120 -> 512 on 4 x 4, 94 MB, 117 us, now 39).
+FewSetup few_setup(const dopt_hip_conv_desc *d, size_t P, size_t Q)
+{
+    FewSetup u;
+    const size_t pixels = d->N * P * Q, total = d->C * d->R * d->S;
+    if (pixels > (size_t)kFewPixels || total < 256 || d->K < 32 || d->K * total >= (size_t)1 << 27 ||
+        d->N * d->C * d->H * d->W * sizeof(float) >= (size_t)kOobOffset)
+        return u;
+    if ((dense2x2_takes(d) && pixels > 32) || (direct2x2_takes(d) && d->C < 384)) return u;
+    const size_t PR = d->H + 2 * d->padH, PC = d->W + 2 * d->padW, taps = d->R * d->S;
+    const size_t tiles = ceil_div(d->K, (size_t)32);
+    size_t cuts = std::min({std::max((size_t)num_cus() / tiles, (size_t)1), total / 64, (size_t)16});
+    cuts = std::max(cuts, ceil_div(total, (size_t)kFewDepthMax));
+    const size_t depth = ceil_div(ceil_div(total, cuts), (size_t)8) * 8;
+    cuts = ceil_div(total, depth);
+    const size_t groups = pixels > 32 ? 2 : 1, chans = std::min((depth + taps - 2) / taps + 1, d->C);
+    u.lds_bytes = (kFewWaves * groups * 32 * 33 + depth + chans * d->N * PR * PC) * sizeof(float);
+    if (u.lds_bytes > 150 * 1024 || cuts > 64) return u;
+    FewConv &f = u.f;
+    f.N = (int)d->N; f.C = (int)d->C; f.H = (int)d->H; f.W = (int)d->W; f.K = (int)d->K; f.R = (int)d->R; f.S = (int)d->S;
+    f.padH = (int)d->padH; f.padW = (int)d->padW; f.strideH = (int)d->strideH; f.strideW = (int)d->strideW;
+    f.P = (int)P; f.Q = (int)Q; f.PR = (int)PR; f.PC = (int)PC; f.depth = (int)depth;
+    u.elems = pixels * d->K;
+    f.out_elems = copy_stride(u.elems);
+    f.w_bytes = d->K * total * sizeof(float);
+    f.x_bytes = d->N * d->C * d->H * d->W * sizeof(float);
+    u.cuts = (int)cuts;
+    u.ok = true;
+    return u;
+}
+
+// `open` as in run_patch.
+int run_few(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float *x, const float *w, const float *bias, float *y, bool *done,
+            dopt_hip_split_sum *open = nullptr)
+{
+    *done = false;
+    FewSetup u = few_setup(d, P, Q);
+    if (!u.ok) return DOPT_HIP_OK;
+    FewConv &f = u.f;
+    float *partial = nullptr;
+    if (u.cuts > 1 && !(partial = (float *)workspace((size_t)u.cuts * f.out_elems * sizeof(float)))) return DOPT_HIP_ERR_OOM;
+    f.x = x;
+    f.w = w;
+    f.bias = u.cuts == 1 ? bias : nullptr;
+    f.out = u.cuts > 1 ? partial : y;
+    const dim3 grid((unsigned)ceil_div(d->K, (size_t)32), (unsigned)u.cuts), block(64 * kFewWaves);
+    const bool two = d->N * P * Q > 32;
+    static bool raised = false;   // above 64 KB of dynamic LDS a kernel has to be told once
+    if (!raised) {
+        DOPT_HIP_CHECK(hipFuncSetAttribute((const void *)conv_few_k<1>, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
+        DOPT_HIP_CHECK(hipFuncSetAttribute((const void *)conv_few_k<2>, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
+        raised = true;
+    }
+    if (two) hipLaunchKernelGGL(conv_few_k<2>, grid, block, u.lds_bytes, stream(), f);
+    else hipLaunchKernelGGL(conv_few_k<1>, grid, block, u.lds_bytes, stream(), f);
+    DOPT_LAUNCH_CHECK();
+    *done = true;
+    if (u.cuts == 1) return DOPT_HIP_OK;
+    if (open && u.elems % 4 == 0 && aligned16(y)) {   // the caller's next call adds the copies
+        open->partial = partial;
+        open->splits = u.cuts;
+        open->elems = u.elems;
+        open->C = d->K;
+        open->inner = P * Q;
+        open->bias = bias;
+        open->value = y;
+        open_split_set(partial);
+        return DOPT_HIP_OK;
+    }
+    if (u.elems % 4 == 0 && aligned16(y))   // in the order in which a later call adds the open copies
+        return launch_splitk_reduce(u.elems, u.cuts, partial, y, bias, (unsigned)d->K, (unsigned)(P * Q));
+    return launch_splitk_exact(u.elems, u.cuts, partial, y, bias, (unsigned)d->K, (unsigned)(P * Q));
+}
+
 template <class T, int SL, auto kKernel, class Args>
 int launch_gather_kernel(const Args &args, dim3 grid)
 {
@@ -3239,6 +3441,8 @@ int run_gather(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float *in,
     if (!kBwd) {
         bool done = false;
         if (int rc = conv_smallc_fwd(d, in, w, bias, out, &done)) return rc;
+        if (done) return DOPT_HIP_OK;
+        if (int rc = run_few(d, P, Q, in, w, bias, out, &done)) return rc;
         if (done) return DOPT_HIP_OK;
     }
     if (dense2x2_takes(d)) {
@@ -3645,7 +3849,7 @@ size_t dopt_hip_conv_packed_bytes(const dopt_hip_conv_desc *d, int bwd_data)
     size_t P, Q;
     if (check_desc(d, &P, &Q, "dopt_hip_conv_packed_bytes") || !ensure_init()) return 0;
     if (!bwd_data && conv_smallc_takes(d)) return 0;   // that forward kernel reads the filter as it is
-    if (direct2x2_takes(d)) return d->K * d->C * 9 * sizeof(float);   // the filter as it is
+    if (direct2x2_takes(d) || (!bwd_data && few_setup(d, P, Q).ok)) return d->K * d->C * d->R * d->S * sizeof(float);   // the filter as it is
     if (dense2x2_takes(d)) return dense2x2_elems(d) * sizeof(float);
     const PatchSetup u = bwd_data ? patch_setup<true>(d, P, Q) : patch_setup<false>(d, P, Q);
     // PackJob keeps strides in 32 bits
@@ -3656,6 +3860,8 @@ int dopt_hip_conv_packed_layout(const dopt_hip_conv_desc *d, int bwd_data)
 {
     if (dopt_hip_conv_packed_bytes(d, bwd_data) == 0) return -1;
     if (direct2x2_takes(d)) return 3;  // the filter itself: such kernels read [K][C][3][3], and a caller may pass the filter
+    size_t P, Q;
+    if (!bwd_data && check_desc(d, &P, &Q, "dopt_hip_conv_packed_layout") == 0 && few_setup(d, P, Q).ok) return 3;
     if (dense2x2_takes(d)) return 2;   // the same matrix, read transposed by backward-data
     return bwd_data ? 1 : 0;
 }
@@ -3680,10 +3886,10 @@ int dopt_hip_conv_pack_batch(int n, const dopt_hip_conv_desc *descs, const int *
         size_t P, Q;
         if (int rc = check_desc(&descs[i], &P, &Q, "dopt_hip_conv_pack_batch")) return rc;
         DOPT_REQUIRE(w[i] && packed[i] && aligned16(packed[i]), "dopt_hip_conv_pack_batch: filter %d: null or unaligned pointer", i);
-        if (direct2x2_takes(&descs[i])) {   // "packed" is a plain copy (callers that know pass the filter itself instead)
+        if (dopt_hip_conv_packed_layout(&descs[i], bwd_data[i]) == 3) {   // "packed" is a plain copy (callers that know pass the filter itself instead)
             if (int rc = flush()) return rc;
             if (packed[i] != w[i])
-                if (int rc = dopt_hip_copy_d2d(packed[i], w[i], descs[i].K * descs[i].C * 9 * sizeof(float))) return rc;
+                if (int rc = dopt_hip_copy_d2d(packed[i], w[i], descs[i].K * descs[i].C * descs[i].R * descs[i].S * sizeof(float))) return rc;
             continue;
         }
         if (dense2x2_takes(&descs[i]) && !(!bwd_data[i] && conv_smallc_takes(&descs[i]))) {
@@ -3716,6 +3922,8 @@ int dopt_hip_conv_fwd_bias_packed_open(const dopt_hip_conv_desc *d, const float 
     DOPT_ENSURE_INIT();
     if (dopt_hip_conv_packed_layout(d, 0) == 3) {
         bool done = false;
+        if (int rc = run_few(d, P, Q, x, packed, bias, y, &done, open)) return rc;
+        if (done) return DOPT_HIP_OK;
         if (int rc = run_direct2x2<false>(d, x, packed, bias, y, &done)) return rc;
         if (done) return DOPT_HIP_OK;
         return run_dense2x2<false>(d, x, packed, nullptr, bias, y);   // operands it cannot read as quads: from the filter

@@ -529,6 +529,37 @@ def test_results_of_odd_counts_are_cut_too(shape):
         assert np.allclose(flat[1:1 + want.size], want.ravel(), rtol=1e-4, atol=1e-5 * np.sqrt(C * R * R + K * R * R))
 
 
+# forward of up to 64 output pixels: 1, 25, 31, 32, 33, 64 of them and 65; rows of 32 and of one more; reductions of 256 steps, of no whole
+# quads, of one part and of many; strides, no padding, several images; a count of results that is no multiple of four
+@pytest.mark.parametrize("shape", [(1, 400, 1, 1, 300, 1, 0, 1), (1, 257, 5, 5, 33, 5, 2, 1), (31, 29, 3, 3, 45, 3, 0, 1), (1, 64, 4, 8, 32, 3, 1, 1), (3, 131, 1, 11, 65, 3, 1, 1),
+                                   (1, 256, 1, 1, 31, 1, 0, 1), (1, 256, 8, 8, 32, 1, 0, 1), (1, 640, 8, 8, 640, 3, 1, 1), (1, 99, 16, 16, 70, 3, 1, 2), (2, 37, 17, 13, 34, 7, 0, 3),
+                                   (4, 512, 2, 2, 64, 3, 1, 1), (1, 2049, 7, 7, 36, 1, 0, 1), (5, 61, 13, 1, 40, 3, 1, 1), (1, 5000, 2, 3, 32, 3, 1, 1)])
+def test_convolution_of_few_pixels(shape):
+    import ctypes as C_
+    N, C, H, W, K, R, pad, stride = shape
+    r = rng(C + K + R)
+    x, w, b = r.standard_normal((N, C, H, W), np.float32), r.standard_normal((K, C, R, R), np.float32), r.standard_normal(K, np.float32)
+    ps = ((pad, pad), (stride, stride))
+    want = general(x, w, pad, stride)
+    got = ops.convolution(T(x), T(w), *ps).numpy()
+    check_norm(got, want, C * R * R, shape)
+    whole = T(np.full(want.size + 8, 7.0, np.float32))   # into results off the 16-byte grid, from operands off it
+    off = lambda v: T(np.append(np.zeros(1, np.float32), v.ravel())).view(1, v.shape)
+    ops.convolution(off(x), off(w), *ps, out=whole.view(1, want.shape))
+    flat = whole.numpy()
+    assert (flat[:1] == 7.0).all() and (flat[1 + want.size:] == 7.0).all()
+    check_norm(flat[1:1 + want.size].reshape(want.shape), want, C * R * R, shape)
+    lib, d = capi.load(), ops.conv_desc(x.shape, w.shape, *ps)
+    if lib.dopt_hip_conv_packed_layout(C_.byref(d), 0) == 3:   # left open and closed: the same bits
+        tx, tw, tb, o = T(x), T(w), T(b), capi.SplitSum()
+        closed, opened = ops.Tensor(want.shape), ops.Tensor(want.shape)
+        capi.check(lib.dopt_hip_conv_fwd_bias_packed(C_.byref(d), tx.ptr, tw.ptr, tb.ptr, closed.ptr))
+        capi.check(lib.dopt_hip_conv_fwd_bias_packed_open(C_.byref(d), tx.ptr, tw.ptr, tb.ptr, opened.ptr, C_.byref(o)))
+        capi.check(lib.dopt_hip_split_sum_close(C_.byref(o)))
+        assert np.array_equal(opened.numpy(), closed.numpy())
+        check_norm(closed.numpy(), want + b.astype(np.float64)[:, None, None], C * R * R, shape)
+
+
 def test_odd_filter_gradients_in_a_plan():
     """A backward pair whose filter gradient has an odd count beside the batch norm that adds riding sums: it adds its own."""
     from dopt_amd import core, nnet
