@@ -560,6 +560,21 @@ def test_convolution_of_few_pixels(shape):
         check_norm(closed.numpy(), want + b.astype(np.float64)[:, None, None], C * R * R, shape)
 
 
+# filter gradients from many copies: either side of 2^17 values; rows of values that are no whole block, one block, several
+@pytest.mark.parametrize("shape", [(64, 128, 16, 16, 113, 3, 1, 1), (64, 128, 16, 16, 114, 3, 1, 1), (100, 48, 31, 29, 25, 5, 2, 2), (64, 64, 32, 32, 7, 1, 0, 1),
+                                   (130, 65, 28, 28, 3, 1, 0, 1), (64, 16, 32, 32, 32, 3, 1, 1), (40, 3, 33, 31, 17, 7, 3, 2)])
+def test_filter_gradients_of_few_values(shape):
+    N, C, H, W, K, R, pad, stride = shape
+    r = rng(C + K + R)
+    x, P = r.standard_normal((N, C, H, W), np.float32), [(n + 2 * pad - R) // stride + 1 for n in (H, W)]
+    dy, w = r.standard_normal((N, K, *P), np.float32), np.zeros((K, C, R, R), np.float32)
+    whole = T(np.full(w.size + 8, 7.0, np.float32))
+    ops.conv_bwd_filter(T(dy), T(x), w.shape, (pad, pad), (stride, stride), out=whole.view(4, w.shape))
+    flat = whole.numpy()
+    assert (flat[:4] == 7.0).all() and (flat[4 + w.size:] == 7.0).all()
+    check_norm(flat[4:4 + w.size].reshape(w.shape), general_gradients(x, w, dy, pad, stride)[1], dy[:, 0].size, shape)
+
+
 def test_odd_filter_gradients_in_a_plan():
     """A backward pair whose filter gradient has an odd count beside the batch norm that adds riding sums: it adds its own."""
     from dopt_amd import core, nnet
