@@ -2164,8 +2164,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_k(size_t n4, int splits, co
 }
 
 // The same for the general kernels, whose reductions are cut into up to sixty-four parts: added in float64 and rounded once (one fp32
-// rounding per part was most of the error: 66 -> 13 channels, 3 x 3, one image of 23 x 7, 1.3e-7 off float64, so 0.7e-7; the time
-// is that of the copies' bytes).  kLoose: the result's n values are no whole quads, or not on the 16-byte grid.
+// rounding per part was most of the error: 66 -> 13 channels, 3 x 3, one image of 23 x 7, 1.3e-7 off float64, so 3.8e-8, in one
+// part 7e-8; the time is that of the copies' bytes).  kLoose: the result's n values are no whole quads, or not on the 16-byte grid.
 template <bool kLoose>
 __global__ __launch_bounds__(256) void splitk_exact_k(size_t n4, int splits, const float4 *partial, float4 *out, size_t n, const float *bias, unsigned C,
                                                        unsigned inner)
@@ -3330,7 +3330,7 @@ int run_bwd_strided(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float
         if ((size_t)BK * Mp * sizeof(float) > 0x7fffffffu)
             return fail(DOPT_HIP_ERR_UNSUPPORTED, "convolution: more than 2^25 output channels are not supported");
         // The classes' reductions are cut into the same number of parts, each a partial copy of the whole of dx: where a handful of
-        // tiles would be as many workgroups of a long chain (47 images of 4 x 11, 300 channels to 5: 60 us, now 14 with the sum).
+        // tiles would be as many workgroups of a long chain (47 images of 4 x 11, 300 channels to 5: 61 us, now 13 with the sum).
         const bool narrow = C <= 32, wide = !narrow && (C <= 64 || (C + 63) / 64 * 64 < (C + 127) / 128 * 128);
         const int BM = narrow ? 32 : wide ? 64 : 128, BN = narrow || wide ? 256 : 128;
         const size_t elems = d->N * d->C * d->H * d->W;

@@ -492,7 +492,7 @@ extern "C" __global__ __launch_bounds__(BLOCK) void red_cols(const T *in, T *out
 // latency times R / 8).  A block folds rows [s * rows_per, + rows_per) of `width` columns of one outer index: its threads are
 // blockDim / width rows side by side (consecutive threads, consecutive addresses where a row is one tile), each folds every
 // blockDim / width-th row, and the rows meet in LDS pairwise.  A slice's fold goes to out[(o * slices + s) * inner + j].
-// Bound by memory from a few MB on; sum of [17310, 17] over its rows 572 -> 6 us, of [7550, 786] 336 -> 9 us (both launches).
+// Bound by memory from a few MB on; sum of [17310, 17] over its rows 555 -> 8 us, of [7550, 786] 334 -> 15 us (both launches).
 extern "C" __global__ __launch_bounds__(1024) void red_cols_split(const T *in, T *out, size_t R, size_t inner, size_t rows_per,
                                                                    unsigned width, unsigned tiles, unsigned slices)
 {
