@@ -1228,6 +1228,19 @@ def test_graph_flag_leaves_plans_with_random_draws_direct():
     assert all(not np.array_equal(draws[0], d) for d in draws[1:])     # a replayed kernel would repeat its draws
 
 
+# 4, 5, 6, 16, 18 and 34 copies: either side of five, one and several groups of sixteen behind the first
+@pytest.mark.parametrize("channels", [256, 320, 384, 1100, 17500, 34000])
+@pytest.mark.parametrize("image", [(2, 2), (4, 4), (1, 4)], ids=str)
+def test_inference_batch_norm_adds_any_count_of_copies(channels, image):
+    r = np.random.default_rng(channels)
+    v = lambda *s: float32(list(s), r.standard_normal(s).astype(np.float32))
+    y = core.addBias(core.convolution(v(1, channels, *image), v(32, channels, 1, 1), [0, 0], [1, 1]), v(32))
+    b = core.relu(core.batchNormInference(y, v(1, 32, 1, 1), v(32), v(32), float32([32], (r.random(32) + 0.5).astype(np.float32))))
+    for out in [b] + ([core.maxpool(b, [2, 2])] if image[0] > 1 else []):
+        want = core.compile([out]).execute()[0]
+        assert np.array_equal(core.compile([out], core.PLAN_VIEWS | core.PLAN_FUSE).execute()[0], want)
+
+
 @pytest.mark.parametrize("shape", [(1, 512, 2, 2), (3, 64, 4, 4), (1, 96, 16, 16), (2, 5, 6, 6), (5, 7, 3, 3), (2, 16, 8, 4), (7, 24, 2, 4),
                                    (40, 300, 32, 32), (1, 4, 64, 64)], ids=str)
 @pytest.mark.parametrize("conv", [0, 1], ids=["plain", "behind a convolution"])
