@@ -10,6 +10,7 @@
 //   2. finalize: one thread per channel folds the slices in float64, derives mean / 1/std and the
 //      small per-channel outputs, and writes a per-channel coefficient table;
 //   3. apply: a flat 128-bit streaming pass over the tensor using the table.
+#include "bn_infer.h"
 #include "common.h"
 #include "pool2x2.h"
 
@@ -276,52 +277,34 @@ __global__ __launch_bounds__(kBlock) void bn_infer_prepare_k(size_t C, double ep
 // in front of it: y = relu(a * (x - mean) + b) and / or its pooled tensor.  Bound by memory traffic where the tensor is large
 // and by the kernel boundary where it is small, so what counts is that these are one pass and one launch: a layer of a
 // single image was three to five launches (sum of copies, coefficient table, batch norm, relu, pool).
-// A block takes kU * 256 units of consecutive quads - a unit is one quad, or, pooled, the quads of one or two windows -, starts their
-// loads (kN of a value's copies at once: VGG-16 on one image, 13 such launches of up to sixteen copies, 191 us, with four in flight
-// behind the coefficients, now 180) and puts the coefficients of the channels they lie in into LDS (one float64 reciprocal square root each; rows of
+// A block takes kU * 256 units of consecutive quads - a unit is one quad, or, pooled, the quads of one or two windows - and
+// first puts the coefficients of the channels they lie in into LDS (one float64 reciprocal square root each; rows of
 // the [N * C, inner] view, so at most as many as it has units).  Same arithmetic as bn_infer_prepare_k, bn_apply_k, relu_fwd_k
 // and maxpool2x2_fwd_k; the copies are added as splitk_reduce_k adds them.
-struct InferArgs {
-    const float4 *x;         // the operand, or null: [splits] copies of it at `partial`, to be added, and `addend` per channel
-    const float4 *partial;
-    const float *addend;
-    int splits;
-    unsigned n4, C, inner4, units, upr, W;   // quads; channels; quads of a row; units in all and of a row; pixels of an image row
-    double eps;
-    const float *scale, *bias, *mean, *var;
-    float4 *y;               // either may be null
-    float *pooled;
-    int relu;
-};
-
-// Copies s to s + kN - 1, as far as there are any, onto acc: all loads in flight, added in ascending order.
-template <int kN>
-__device__ inline void infer_add(const InferArgs &g, unsigned i, int s, float4 &acc)
-{
-    float4 v[kN];
-    const int last = g.splits - 1;
-#pragma unroll
-    for (int j = 0; j < kN; j++) v[j] = g.partial[(size_t)min(s + j, last) * g.n4 + i];
-#pragma unroll
-    for (int j = 0; j < kN; j++)
-        if (s + j <= last) acc = make_float4(acc.x + v[j].x, acc.y + v[j].y, acc.z + v[j].z, acc.w + v[j].w);
-}
-
-template <int kN>
-__device__ inline float4 infer_load(const InferArgs &g, unsigned i)
+__device__ inline float4 infer_load(const InferArgs &g, unsigned i, unsigned c)
 {
     if (g.x) return g.x[i];
     float4 acc = g.partial[i];
-    for (int s = 1; s < g.splits; s += kN) infer_add<kN>(g, i, s, acc);
+    const int last = g.splits - 1;
+    for (int s = 1; s < g.splits; s += 4) {   // four loads in flight, added in ascending order
+        const float4 v0 = g.partial[(size_t)s * g.n4 + i];
+        const float4 v1 = g.partial[(size_t)min(s + 1, last) * g.n4 + i];
+        const float4 v2 = g.partial[(size_t)min(s + 2, last) * g.n4 + i];
+        const float4 v3 = g.partial[(size_t)min(s + 3, last) * g.n4 + i];
+        acc = make_float4(acc.x + v0.x, acc.y + v0.y, acc.z + v0.z, acc.w + v0.w);
+        if (s + 1 <= last) acc = make_float4(acc.x + v1.x, acc.y + v1.y, acc.z + v1.z, acc.w + v1.w);
+        if (s + 2 <= last) acc = make_float4(acc.x + v2.x, acc.y + v2.y, acc.z + v2.z, acc.w + v2.w);
+        if (s + 3 <= last) acc = make_float4(acc.x + v3.x, acc.y + v3.y, acc.z + v3.z, acc.w + v3.w);
+    }
+    if (g.addend) {
+        const float b = g.addend[c];
+        acc = make_float4(acc.x + b, acc.y + b, acc.z + b, acc.w + b);
+    }
     return acc;
 }
 
-__device__ inline float4 infer_value(const InferArgs &g, float4 v, unsigned c, const Coef &k)
+__device__ inline float4 infer_value(const InferArgs &g, float4 v, const Coef &k)
 {
-    if (!g.x && g.addend) {
-        const float b = g.addend[c];
-        v = make_float4(v.x + b, v.y + b, v.z + b, v.w + b);
-    }
     float4 r;
     r.x = k.a * ((v.x - k.mean) - k.mean_lo) + k.b;
     r.y = k.a * ((v.y - k.mean) - k.mean_lo) + k.b;
@@ -330,62 +313,60 @@ __device__ inline float4 infer_value(const InferArgs &g, float4 v, unsigned c, c
     return g.relu ? make_float4(relu1(r.x), relu1(r.y), relu1(r.z), relu1(r.w)) : r;
 }
 
-template <int kU, bool kPool, int kN>
+template <int kU, bool kPool>
 __global__ __launch_bounds__(kBlock) void bn_infer_k(InferArgs g)
 {
     __shared__ Coef coef[kU * kBlock + 1];
     __shared__ unsigned channel[kU * kBlock + 1];
     const unsigned begin = blockIdx.x * (kU * kBlock), end = min(begin + kU * kBlock, g.units);
     const unsigned row0 = begin / g.upr, rows = (end - 1) / g.upr - row0 + 1;
-    float4 v[kPool ? 2 : kU];
-    unsigned at[kU], q[kPool ? 2 : kU];
-#pragma unroll
-    for (int u = 0; u < kU; u++) {
-        const unsigned i = begin + u * kBlock + threadIdx.x;
-        if (i >= end) break;
-        const unsigned row = i / g.upr;
-        at[u] = row - row0;
-        q[u] = i;
-        if constexpr (kPool) {   // (kU is 1)
-            const unsigned j = i - row * g.upr, W4 = g.W / 4;
-            if (g.W == 2) {   // a quad is a window
-                q[0] = row * g.inner4 + j;
-            } else {
-                const unsigned p = j / W4;
-                q[0] = row * g.inner4 + 2 * p * W4 + (j - p * W4);
-                q[1] = q[0] + W4;
-                v[1] = infer_load<kN>(g, q[1]);
-            }
-        }
-        v[u] = infer_load<kN>(g, q[u]);
-    }
     for (unsigned k = threadIdx.x; k < rows; k += kBlock) {
         const unsigned c = (row0 + k) % g.C;
         const double rstd = 1.0 / sqrt((double)g.var[c] + g.eps);
-        Coef f;
-        f.mean = g.mean[c];
-        f.a = (float)((double)g.scale[c] * rstd);
-        f.b = g.bias[c];
-        f.mean_lo = 0.0f;
-        coef[k] = f;
+        Coef q;
+        q.mean = g.mean[c];
+        q.a = (float)((double)g.scale[c] * rstd);
+        q.b = g.bias[c];
+        q.mean_lo = 0.0f;
+        coef[k] = q;
         channel[k] = c;
     }
     __syncthreads();
+    if constexpr (!kPool) {
+        float4 v[kU];
+        unsigned at[kU];
 #pragma unroll
-    for (int u = 0; u < kU; u++) {
-        const unsigned i = begin + u * kBlock + threadIdx.x;
-        if (i >= end) break;
-        const float4 a = infer_value(g, v[u], channel[at[u]], coef[at[u]]);
-        if (!kPool || g.y) g.y[q[u]] = a;
-        if constexpr (kPool) {
-            if (g.W == 2) {
-                g.pooled[i] = pool2x2(a.x, a.y, a.z, a.w);
-                continue;
-            }
-            const float4 b = infer_value(g, v[1], channel[at[u]], coef[at[u]]);
-            if (g.y) g.y[q[1]] = b;
-            ((float2 *)g.pooled)[i] = make_float2(pool2x2(a.x, a.y, b.x, b.y), pool2x2(a.z, a.w, b.z, b.w));
+        for (int u = 0; u < kU; u++) {
+            const unsigned i = begin + u * kBlock + threadIdx.x;
+            if (i >= end) break;
+            at[u] = i / g.upr - row0;
+            v[u] = infer_load(g, i, channel[at[u]]);
         }
+#pragma unroll
+        for (int u = 0; u < kU; u++) {
+            const unsigned i = begin + u * kBlock + threadIdx.x;
+            if (i >= end) break;
+            g.y[i] = infer_value(g, v[u], coef[at[u]]);
+        }
+    } else {
+        const unsigned i = begin + threadIdx.x;   // (kU is 1)
+        if (i >= end) return;
+        const unsigned row = i / g.upr, j = i - row * g.upr, k = row - row0;
+        if (g.W == 2) {   // a quad is a window
+            const unsigned q = row * g.inner4 + j;
+            const float4 r = infer_value(g, infer_load(g, q, channel[k]), coef[k]);
+            if (g.y) g.y[q] = r;
+            g.pooled[i] = pool2x2(r.x, r.y, r.z, r.w);
+            return;
+        }
+        const unsigned W4 = g.W / 4, p = j / W4, q = row * g.inner4 + 2 * p * W4 + (j - p * W4);
+        const float4 v0 = infer_load(g, q, channel[k]), v1 = infer_load(g, q + W4, channel[k]);
+        const float4 a = infer_value(g, v0, coef[k]), b = infer_value(g, v1, coef[k]);
+        if (g.y) {
+            g.y[q] = a;
+            g.y[q + W4] = b;
+        }
+        ((float2 *)g.pooled)[i] = make_float2(pool2x2(a.x, a.y, b.x, b.y), pool2x2(a.z, a.w, b.z, b.w));
     }
 }
 
@@ -1510,15 +1491,15 @@ int launch_infer(size_t N, size_t C, size_t inner, size_t W, const float *x, con
     g.pooled = pooled;
     g.relu = relu;
     if (split) open_split_clear(open->partial);
-    // four quads a thread once that still gives every CU two blocks; below that, sixteen copies in flight where there are more than
-    // five (in large launches the registers cost more: WRN-28-10 on 250 images 0.4% slower)
-    const bool large = g.units >= 2u * 4 * kBlock * (unsigned)num_cus(), wide = !large && g.splits > 5;
-    const dim3 grid((unsigned)ceil_div(g.units, (large && !pooled ? 4 : 1) * kBlock)), block(kBlock);
-    if (pooled && wide) hipLaunchKernelGGL((bn_infer_k<1, true, 16>), grid, block, 0, stream(), g);
-    else if (pooled) hipLaunchKernelGGL((bn_infer_k<1, true, 4>), grid, block, 0, stream(), g);
-    else if (large) hipLaunchKernelGGL((bn_infer_k<4, false, 4>), grid, block, 0, stream(), g);
-    else if (wide) hipLaunchKernelGGL((bn_infer_k<1, false, 16>), grid, block, 0, stream(), g);
-    else hipLaunchKernelGGL((bn_infer_k<1, false, 4>), grid, block, 0, stream(), g);
+    const bool large = g.units >= 2u * 4 * kBlock * (unsigned)num_cus();
+    // many copies: more than five are more than two rounds of bn_infer_k's loads.  Large launches hide their waits behind each other and
+    // lose by the registers (WRN-28-10 on 250 images 0.4%)
+    if (split && g.splits > 5 && !large) return bn_infer_copies(g);
+    // four quads a thread once that still gives every CU two blocks
+    if (pooled) hipLaunchKernelGGL((bn_infer_k<1, true>), dim3((unsigned)ceil_div(g.units, kBlock)), dim3(kBlock), 0, stream(), g);
+    else if (large)
+        hipLaunchKernelGGL((bn_infer_k<4, false>), dim3((unsigned)ceil_div(g.units, 4 * kBlock)), dim3(kBlock), 0, stream(), g);
+    else hipLaunchKernelGGL((bn_infer_k<1, false>), dim3((unsigned)ceil_div(g.units, kBlock)), dim3(kBlock), 0, stream(), g);
     DOPT_LAUNCH_CHECK();
     return DOPT_HIP_OK;
 }
