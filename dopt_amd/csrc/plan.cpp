@@ -1901,7 +1901,9 @@ int HIPPlan::Builder::allocateBuffers()
         if (buf) p->mOwned.push_back(buf);
         p->mBufferBytes += g.ops[id].bytes();
         p->mResults[id] = buf;
+        if (buf) p->mResultRanges.emplace_back((const char *)buf, (const char *)buf + g.ops[id].bytes());
     }
+    std::sort(p->mResultRanges.begin(), p->mResultRanges.end());
     return DOPT_HIP_OK;
 }
 
@@ -2060,6 +2062,8 @@ int HIPPlan::Builder::buildSteps()
 // dopt_hip_sgemm_batch, the filter gradients of 2x2-image layers one dopt_hip_conv_bwd_filter_batch, each placed
 // where the last of its members stood (everything they read is older than that, and nothing was going to read them
 // before).  The members run the kernel bodies they would have run alone: no value changes (DOPT_HIP_PLAN_FUSE).
+// An argument that lies in one of the plan's own buffers would change: its readers are moved past what fills that buffer,
+// or run beside it.  So the members stay in the list where they stood, for the executions that are given one (HIPPlan::mInOrder).
 void HIPPlan::Builder::batchIndependent()
 {
     if (!(flags & DOPT_HIP_PLAN_FUSE)) return;
@@ -2090,7 +2094,12 @@ void HIPPlan::Builder::batchIndependent()
             wgrads.push_back({i, conv_desc(x, op.shape, *pad, *stride)});
         }
     }
-    std::vector<char> drop(p->mSteps.size(), 0);
+    std::vector<Step> batchAt(p->mSteps.size());   // behind the step of that place, where it has a kernel
+    auto member = [&](size_t step) { p->mSteps[step].when = Step::kInOrder; };
+    auto batch = [&](size_t step, Step &&b) {
+        b.when = Step::kBatched;
+        batchAt[step] = std::move(b);
+    };
     const bool shapes = (flags & DOPT_HIP_PLAN_TIMING_SHAPES) != 0;
     if (products.size() >= 2) {
         Step b;
@@ -2105,7 +2114,7 @@ void HIPPlan::Builder::batchIndependent()
             b.inputOps.push_back(c.mi.a);
             b.inputOps.push_back(c.mi.b);
             outs.push_back((float *)p->mResults[p->mSteps[c.step].op]);
-            drop[c.step] = 1;
+            member(c.step);
         }
         const int n = (int)products.size();
         b.kernel = make([=](const std::vector<const void *> &in, void *) {
@@ -2119,9 +2128,7 @@ void HIPPlan::Builder::batchIndependent()
         b.inputs.resize(b.inputOps.size());
         b.inputBytes.resize(b.inputOps.size());
         for (size_t i = 0; i < b.inputOps.size(); i++) b.inputBytes[i] = g.ops[b.inputOps[i]].bytes();
-        const size_t at = products.back().step;
-        drop[at] = 0;
-        p->mSteps[at] = std::move(b);
+        batch(products.back().step, std::move(b));
     }
     if (wgrads.size() >= 2) {
         Step b;
@@ -2135,7 +2142,7 @@ void HIPPlan::Builder::batchIndependent()
             b.inputOps.push_back(op.deps[0]);
             b.inputOps.push_back(op.deps[1]);
             outs.push_back((float *)p->mResults[p->mSteps[c.step].op]);
-            drop[c.step] = 1;
+            member(c.step);
         }
         const int n = (int)wgrads.size();
         b.kernel = make([=](const std::vector<const void *> &in, void *) {
@@ -2149,9 +2156,7 @@ void HIPPlan::Builder::batchIndependent()
         b.inputs.resize(b.inputOps.size());
         b.inputBytes.resize(b.inputOps.size());
         for (size_t i = 0; i < b.inputOps.size(); i++) b.inputBytes[i] = g.ops[b.inputOps[i]].bytes();
-        const size_t at = wgrads.back().step;
-        drop[at] = 0;
-        p->mSteps[at] = std::move(b);
+        batch(wgrads.back().step, std::move(b));
     }
     // Products that a later step reads (a dense layer's gradients in front of an update rule) can wait for each other while no
     // step in between reads one of them.
@@ -2186,8 +2191,8 @@ void HIPPlan::Builder::batchIndependent()
             for (size_t k = from; k + 1 < to; k++) {   // (their buffers come as inputs, as those of a group's members do)
                 b.inputOps.push_back(p->mSteps[fed[k].step].op);
                 b.writes.push_back(p->mSteps[fed[k].step].op);
-                drop[fed[k].step] = 1;
             }
+            for (size_t k = from; k < to; k++) member(fed[k].step);
             b.kernel = make([=](const std::vector<const void *> &in, void *out) {
                 std::vector<const float *> A(n), B(n);
                 std::vector<float *> C(n);
@@ -2201,16 +2206,17 @@ void HIPPlan::Builder::batchIndependent()
             b.inputs.resize(b.inputOps.size());
             b.inputBytes.resize(b.inputOps.size());
             for (size_t i = 0; i < b.inputOps.size(); i++) b.inputBytes[i] = g.ops[b.inputOps[i]].bytes();
-            p->mSteps[at] = std::move(b);
+            batch(at, std::move(b));
         }
         from = to;
     }
-    // close the ranks; the convolution steps remembered for openSplitSums move with them
+    // the batches take their places; the convolution steps remembered for openSplitSums move with the others
     std::vector<size_t> moved(p->mSteps.size(), 0);
     std::vector<Step> kept;
     for (size_t i = 0; i < p->mSteps.size(); i++) {
         moved[i] = kept.size();
-        if (!drop[i]) kept.push_back(std::move(p->mSteps[i]));
+        kept.push_back(std::move(p->mSteps[i]));
+        if (batchAt[i].kernel) kept.push_back(std::move(batchAt[i]));
     }
     p->mSteps = std::move(kept);
     for (ConvStep &cs : convSteps) cs.step = moved[cs.step];
@@ -2391,7 +2397,7 @@ int HIPPlan::Builder::assignQueues()
         std::vector<char> side(n, 0);
         for (size_t i = n; i-- > 0;) {   // readers come later in the order, so they are decided first
             const Step &st = p->mSteps[i];
-            if (st.op < 0 || biasGradOf[st.op] >= 0 || producers[i].empty()) continue;
+            if (st.op < 0 || st.when != Step::kAlways || biasGradOf[st.op] >= 0 || producers[i].empty()) continue;
             // by label: a fused step carries the operation it ends in (convolution+addBias ends in an addBias), and a
             // convolution must stay behind the step that packs its filter
             const std::string &t = g.ops[st.op].opType;
@@ -2524,8 +2530,8 @@ int HIPPlan::create(Graph *graph, const std::vector<int> &outputs, unsigned flag
         if (dump[0] && dump[0] != '0')
             for (size_t i = 0; i < p->mSteps.size(); i++) {
                 const Step &st = p->mSteps[i];
-                std::fprintf(stderr, "plan step %3zu queue %d%s%s %-44s op %d <-", i, st.lane, st.fenceBefore ? " (waits)" : "",
-                             st.joinSide ? " (joins)" : "", st.label.c_str(), st.op);
+                std::fprintf(stderr, "plan step %3zu queue %d%s%s%s %-44s op %d <-", i, st.lane, st.fenceBefore ? " (waits)" : "",
+                             st.joinSide ? " (joins)" : "", st.when == Step::kInOrder ? " (in order)" : "", st.label.c_str(), st.op);
                 for (int in : st.inputOps) std::fprintf(stderr, " %d", in);
                 std::fprintf(stderr, "\n");
             }
@@ -2576,6 +2582,7 @@ int HIPPlan::resolve(int nargs, const int *argOps, const void *const *argPtrs, c
     for (int id : mOps)
         if (mNeeded[id] && is_leaf(g.ops[id])) mResults[id] = g.ops[id].value;
     int slot = -1;   // the pair of copies this execution's host arguments go through
+    mInOrder = false;
     for (int a = 0; a < nargs; a++) {
         const int id = argOps[a];
         if (id < 0 || id >= (int)g.ops.size() || g.ops[id].opType != "variable")
@@ -2612,6 +2619,10 @@ int HIPPlan::resolve(int nargs, const int *argOps, const void *const *argPtrs, c
             mResults[id] = h.dev;
         } else {
             mResults[id] = const_cast<void *>(argPtrs[a]);
+            // (the last of the plan's buffers that starts before the argument ends)
+            const char *const lo = (const char *)argPtrs[a];
+            auto at = std::lower_bound(mResultRanges.begin(), mResultRanges.end(), std::make_pair(lo + g.ops[id].bytes(), (const char *)nullptr));
+            if (at != mResultRanges.begin() && (--at)->second > lo) mInOrder = true;
         }
     }
     if (slot >= 0) {
@@ -2631,6 +2642,7 @@ int HIPPlan::resolve(int nargs, const int *argOps, const void *const *argPtrs, c
 int HIPPlan::enqueue(int nrets, void *const *rets)
 {
     const bool timing = !mEvents.empty();
+    auto runs = [&](const Step &s) { return s.when == Step::kAlways || (s.when == Step::kInOrder) == mInOrder; };
     size_t fence = 0;
     auto order = [&](int first, int then) -> int {   // work queued on `then` from here on follows all of `first` so far
         DOPT_HIP_CHECK(hipEventRecord(mFences[fence], lane_stream(first)));
@@ -2640,6 +2652,7 @@ int HIPPlan::enqueue(int nrets, void *const *rets)
     };
     for (size_t i = 0; i < mSteps.size(); i++) {
         Step &s = mSteps[i];
+        if (!runs(s)) continue;
         if (s.lane == 1 && s.fenceBefore) {
             if (int rc = order(0, 1)) return rc;   // its inputs come from main-queue steps before it
         } else if (s.joinSide) {
@@ -2659,6 +2672,7 @@ int HIPPlan::enqueue(int nrets, void *const *rets)
     if (timing) {
         DOPT_HIP_CHECK(hipStreamSynchronize(stream()));
         for (size_t i = 0; i < mSteps.size(); i++) {
+            if (!runs(mSteps[i])) continue;
             float ms = 0.0f;
             DOPT_HIP_CHECK(hipEventElapsedTime(&ms, mEvents[i].first, mEvents[i].second));
             auto &slot = profiler[mSteps[i].label];

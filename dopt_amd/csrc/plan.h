@@ -84,7 +84,12 @@ public:
     int execute(int nargs, const int *argOps, const void *const *argPtrs, const int *argOnHost, int nrets,
                 void *const *rets);
     int result(int op, void **ptr, size_t *bytes) const;
-    size_t kernelCount() const { return mSteps.size(); }
+    size_t kernelCount() const
+    {
+        size_t n = 0;
+        for (const Step &s : mSteps) n += s.when != Step::kInOrder;
+        return n;
+    }
     void recordings(size_t *recorded, size_t *replays) const
     {
         size_t n = 0;
@@ -110,6 +115,9 @@ private:
         int lane = 0;                            // 1: runs on the side queue, beside the main chain
         bool fenceBefore = false;                // side-queue step: first wait for what the main queue holds so far
         bool joinSide = false;                   // main-queue step that reads a side-queue result
+        // A batch of steps that stood apart, and each of its members where it stood: an execution runs one or the other
+        // (see mInOrder).
+        enum { kAlways, kBatched, kInOrder } when = kAlways;
     };
     Graph *mGraph = nullptr;
     unsigned mFlags = 0;
@@ -118,6 +126,10 @@ private:
     std::vector<Step> mSteps;                    // kernels to run, in order
     std::unordered_map<int, void *> mResults;    // op -> buffer
     std::vector<void *> mOwned;                  // buffers to free in cleanup
+    std::vector<std::pair<const char *, const char *>> mResultRanges;   // of the buffers that steps fill, ascending
+    // This execution was given an argument that lies in a buffer which a step fills.  What reads it reads it where it stands:
+    // batches of steps that stood apart, whose members may be done in any order, are replaced by their members.
+    bool mInOrder = false;
     // Arguments that arrive as host arrays (cuda/package.d:367-401 uploads them with a blocking copy on every
     // execution): two slots per argument, each a page-locked staging copy and a device copy, used in turn.  The host
     // array is copied into the staging memory before the call returns (the caller may change it at once, as after the

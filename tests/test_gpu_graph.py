@@ -643,6 +643,29 @@ def test_output_only_products_of_a_plan_share_a_launch():
         assert np.array_equal(a, b) or (a.ndim == 1 and np.allclose(a, b, rtol=0, atol=2e-5))
 
 
+@pytest.mark.parametrize("where", ["product", "between"])
+@pytest.mark.parametrize("read", [True, False], ids=["read later", "outputs"])
+def test_batched_products_with_an_argument_in_a_result(read, where):
+    """Products that stood apart run as one launch where the last of them stood.  An argument that lies in the other product's
+    result, or in what a step between them fills, is read where its reader stood: the values of the plan without rewrites."""
+    r = np.random.default_rng(73)
+    x, w, u = (float32([128, 96]) for _ in range(3))
+    A, B = (float32([96, 96], (r.standard_normal((96, 96)) / 10).astype(np.float32)) for _ in range(2))
+    z, s, y = core.matmul(x, B), core.softmax(u), core.matmul(w, A)
+    outs = [z + (s + y)] if read else [z, s, y]
+    plans = [core.compile(outs, f | core.PLAN_TIMING) for f in (0, core.PLAN_VIEWS | core.PLAN_FUSE)]
+    v = lambda: r.standard_normal((128, 96)).astype(np.float32)
+    first, later = {x: v(), w: v(), u: v()}, {w: v(), u: v()}
+    got = []
+    for p in plans:
+        p.execute(first)
+        ptr, _ = p.result_ptr(y if where == "product" else s)
+        got.append(p.execute({x: ops.Tensor((128, 96), _ptr=ptr, _owner=p), **later}) + p.execute(first))
+    assert plans[1].profile()["matmul*2"][1] == 2 and plans[1].profile()["matmul"][1] == 2, plans[1].profile()
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+
+
 def test_host_arguments_are_consumed_when_the_call_returns():
     """A plan's host arguments (cuda/package.d:367-401 uploads them with a blocking copy) are copied into the plan's
     own page-locked staging memory before the call returns and uploaded beside the kernels still queued, two copies
