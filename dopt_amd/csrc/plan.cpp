@@ -2343,12 +2343,11 @@ int HIPPlan::Builder::assignQueues()
         };
         int fences = 1;   // the final join
         for (Step &st : p->mSteps) {
-            if (st.op < 0) continue;
             bool reads_side = false;
             for (int in : st.inputOps) reads_side = reads_side || onSide[producer(in)];
-            const bool wgrad = g.ops[st.op].opType == "convolutionFiltersGrad";
-            // a step with a second output (the absorbed bias gradient) stays on the main queue
-            if ((wgrad || reads_side) && biasGradOf[st.op] < 0 && poolOf[st.op] < 0 && pairOf[st.op] < 0) {
+            const bool wgrad = st.op >= 0 && g.ops[st.op].opType == "convolutionFiltersGrad";
+            // a step with a second output (the absorbed bias gradient), or that serves other steps, stays on the main queue
+            if (st.op >= 0 && (wgrad || reads_side) && biasGradOf[st.op] < 0 && poolOf[st.op] < 0 && pairOf[st.op] < 0) {
                 st.lane = 1;
                 st.fenceBefore = true;
                 onSide[st.op] = 1;

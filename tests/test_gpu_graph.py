@@ -1062,6 +1062,25 @@ def test_overlapped_filter_gradients_change_nothing(maker):
     assert np.allclose(runs[0][0], runs[3][0], rtol=1e-4)
 
 
+def test_a_batch_of_products_waits_for_the_second_queue(monkeypatch, capfd):
+    """Two products of a filter gradient, which DOPT_HIP_PLAN_OVERLAP computes on the second queue: the launch they share is on
+    the main one and waits for it."""
+    r = np.random.default_rng(74)
+    v = lambda *s: float32(list(s), r.standard_normal(s).astype(np.float32))
+    dy, x = v(64, 48, 16, 16), v(64, 32, 16, 16)
+    dw = core.Operation("convolutionFiltersGrad", [dy, x], {"filtersShape": [48, 32, 3, 3], "padding": [1, 1], "stride": [1, 1]})
+    m = dw.reshape([48, 288])
+    outs = [core.matmul(m, v(288, 100)), core.matmul(m, v(288, 70))]
+    want = core.compile(outs, core.PLAN_VIEWS | core.PLAN_FUSE).execute()
+    monkeypatch.setenv("DOPT_HIP_PLAN_DUMP", "1")
+    plan = core.compile(outs, core.PLAN_VIEWS | core.PLAN_FUSE | core.PLAN_OVERLAP)
+    line = [t for t in capfd.readouterr().err.splitlines() if "matmul*2" in t]
+    assert len(line) == 1 and ("queue 1 (waits)" in line[0] or "queue 0 (joins)" in line[0])
+    for _ in range(3):
+        for a, b in zip(want, plan.execute()):
+            assert np.array_equal(a, b)
+
+
 def test_second_queue_beside_batch_norms_whose_blocks_share_a_channel():
     """The first two layers of the benchmark network at batch 128 hold 131072 values per channel: their batch norms run
     as four blocks per channel that wait for each other, sized for an otherwise idle device.  With a second queue live
