@@ -115,7 +115,8 @@ int reduce_squares_batch(int count, const float *const *in, const size_t *n, flo
 
 // tiny_rtc.cpp: a run of operations on tiny tensors (dopt_hip_tiny_graph's nodes) as a kernel of its own, compiled when it is first
 // launched.  The results' buffers must not overlap each other, which a plan's own do not.  `done` stays false, with nothing
-// launched, for runs it does not take and where what is read from outside overlaps a result: those are dopt_hip_tiny_graph's.
+// launched, for runs it does not take, where what is read from outside overlaps a result and where the kernel cannot be compiled or
+// loaded (which is tried once): those are dopt_hip_tiny_graph's.
 struct TinyRun {
     TinyRun(int nslots, const std::vector<dopt_hip_tiny_node> &nodes);
     int launch(void *const *slots, bool *done) const;
@@ -123,6 +124,7 @@ struct TinyRun {
 private:
     struct Range { int slot, offset, bytes; };
     int slots, threads = 0;
+    mutable bool refused = false;
     std::string source, key;
     std::vector<Range> reads, writes;
 };

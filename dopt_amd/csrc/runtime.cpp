@@ -242,10 +242,16 @@ int rtc_get(const std::string &key, const std::string &source, const char *kerne
     int rc = rtc_compile(source, r.arch.c_str(), &code, nullptr);
     if (rc) return rc;
     hipModule_t mod;
-    DOPT_HIP_CHECK(hipModuleLoadData(&mod, code.data()));
-    r.modules.push_back(mod);
+    hipError_t e = hipModuleLoadData(&mod, code.data());
     hipFunction_t f;
-    DOPT_HIP_CHECK(hipModuleGetFunction(&f, mod, kernel_name));
+    if (e == hipSuccess) {
+        r.modules.push_back(mod);
+        e = hipModuleGetFunction(&f, mod, kernel_name);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // reported here: a caller that can do without must not find it behind its next launch
+        return fail(DOPT_HIP_ERR_RUNTIME, "loading the compiled kernel %s failed: %s", kernel_name, hipGetErrorString(e));
+    }
     r.kernels[key] = f;
     *fn = f;
     return DOPT_HIP_OK;

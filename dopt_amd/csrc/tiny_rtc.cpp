@@ -442,7 +442,7 @@ TinyRun::TinyRun(int nslots, const std::vector<dopt_hip_tiny_node> &nodes) : slo
 int TinyRun::launch(void *const *ptrs, bool *done) const
 {
     *done = false;
-    if (threads == 0) return DOPT_HIP_OK;
+    if (threads == 0 || refused) return DOPT_HIP_OK;
     for (const Range &r : reads) {
         const char *lo = (const char *)ptrs[r.slot] + r.offset;
         for (const Range &w : writes) {
@@ -451,8 +451,14 @@ int TinyRun::launch(void *const *ptrs, bool *done) const
         }
     }
     hipFunction_t fn;
-    if (!rtc_find(key, &fn))
-        if (int rc = rtc_get(key, source, "tiny_run", &fn)) return rc;
+    if (!rtc_find(key, &fn)) {
+        const std::string said = dopt_hip_last_error();
+        if (rtc_get(key, source, "tiny_run", &fn)) {   // no compiler, no memory for the code: dopt_hip_tiny_graph needs neither
+            refused = true;
+            fail(DOPT_HIP_OK, "%s", said.c_str());   // what this call puts right is no error of its caller
+            return DOPT_HIP_OK;
+        }
+    }
     void *args[DOPT_HIP_TINY_SLOTS];
     for (int i = 0; i < slots; i++) args[i] = (void *)&ptrs[i];
     *done = true;

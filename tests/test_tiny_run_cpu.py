@@ -1,0 +1,113 @@
+"""A plan's compiled runs of tiny operations (tiny_rtc.cpp) against a run-time compiler that is played by a table: what a run does
+when it cannot be compiled, without a device."""
+import os
+import subprocess
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "dopt_amd", "csrc")
+
+HARNESS = r"""
+#include <cassert>
+#include <cstdarg>
+#include <map>
+#include <memory>
+#include "common.h"
+
+static std::string error_text;
+static std::map<std::string, hipFunction_t> compiled;
+static bool broken = false;
+static int attempts = 0, launches = 0;
+
+extern "C" const char *dopt_hip_last_error(void) { return error_text.c_str(); }
+
+namespace dopt {
+int fail(int code, const char *fmt, ...)
+{
+    char buf[2048];
+    va_list ap;
+    va_start(ap, fmt);
+    vsnprintf(buf, sizeof(buf), fmt, ap);
+    va_end(ap);
+    error_text = buf;
+    return code;
+}
+bool rtc_find(const std::string &key, hipFunction_t *fn)
+{
+    auto it = compiled.find(key);
+    if (it != compiled.end()) *fn = it->second;
+    return it != compiled.end();
+}
+int rtc_get(const std::string &key, const std::string &, const char *, hipFunction_t *fn)
+{
+    attempts++;
+    if (broken) return fail(DOPT_HIP_ERR_RTC, "hipRTC compilation failed");
+    *fn = compiled[key] = (hipFunction_t)(compiled.size() + 1);
+    return DOPT_HIP_OK;
+}
+int rtc_launch(hipFunction_t, unsigned, unsigned, void **)
+{
+    launches++;
+    return DOPT_HIP_OK;
+}
+}
+
+using namespace dopt;
+
+// out = (a + b) * a over n values
+static std::unique_ptr<TinyRun> make_run(int n)
+{
+    std::vector<dopt_hip_tiny_node> nodes(2);
+    for (int k = 0; k < 2; k++) {
+        dopt_hip_tiny_node nd{};
+        nd.kind = DOPT_HIP_TINY_POINTWISE;
+        nd.op = k ? 2 : 0;   // mul, add
+        nd.dst = 2 + k;
+        nd.a = k ? 2 : 0;
+        nd.b = k ? 0 : 1;
+        nd.n = n;
+        nodes[(size_t)k] = nd;
+    }
+    return std::unique_ptr<TinyRun>(new TinyRun(4, nodes));
+}
+
+static float memory[4][64];
+static void *slots[4] = {memory[0], memory[1], memory[2], memory[3]};
+
+#define CHECK(x) do { if (!(x)) { printf("line %d: %s\n", __LINE__, #x); return 1; } } while (0)
+
+int main()
+{
+BODY
+    puts("ok");
+    return 0;
+}
+"""
+
+
+def _run(tmp_path, body):
+    src, exe = os.path.join(str(tmp_path), "harness.cpp"), os.path.join(str(tmp_path), "harness")
+    with open(src, "w") as f:
+        f.write(HARNESS.replace("BODY", body))
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I", CSRC, "-w", "-o", exe, src,
+                    os.path.join(CSRC, "tiny_rtc.cpp")], check=True)
+    out = subprocess.run([exe], capture_output=True, text=True)
+    assert out.returncode == 0 and out.stdout.strip() == "ok", out.stdout + out.stderr
+
+
+def test_a_run_that_cannot_be_compiled_is_left_to_the_interpreter(tmp_path):
+    _run(tmp_path, r"""
+    auto run = make_run(10), other = make_run(11);
+    bool done = true;
+    error_text = "what an earlier call reported";
+    broken = true;
+    for (int i = 0; i < 3; i++) {
+        CHECK(run->launch(slots, &done) == DOPT_HIP_OK);
+        CHECK(!done && launches == 0 && attempts == 1);   // and is not tried again
+        CHECK(error_text == "what an earlier call reported");
+    }
+    broken = false;
+    for (int i = 0; i < 2; i++) {
+        CHECK(other->launch(slots, &done) == DOPT_HIP_OK && done);
+        CHECK(launches == i + 1 && attempts == 2);
+    }
+""")
