@@ -7,6 +7,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <cstdio>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -119,17 +120,29 @@ int reduce_squares_batch(int count, const float *const *in, const size_t *n, flo
 // loaded (which is tried once): those are dopt_hip_tiny_graph's.
 struct TinyRun {
     TinyRun(int nslots, const std::vector<dopt_hip_tiny_node> &nodes);
+    ~TinyRun();
+    TinyRun(const TinyRun &) = delete;
+    TinyRun &operator=(const TinyRun &) = delete;
     int launch(void *const *slots, bool *done) const;
+    struct Code;   // shared by the runs with one source
 
 private:
+    int compile() const;
     struct Range { int slot, offset, bytes; };
     int slots, threads = 0;
     mutable bool refused = false;
-    std::string source, key;
+    mutable std::shared_ptr<Code> code;
+    std::string source;
     std::vector<Range> reads, writes;
 };
+void tiny_codes_trim();       // unloads the code of runs that are gone
+void tiny_codes_shutdown();   // unloads all of it, with the queues idle; runs that are left compile theirs again
 
-// hipRTC: compile `source` (once per distinct `key`) and return the named kernel.
+// hipRTC: compile `source`, load it and find the named kernel in it; wait for all that is queued; unload.
+int rtc_load(const std::string &source, const char *kernel_name, hipModule_t *module, hipFunction_t *fn);
+void rtc_idle();
+void rtc_unload(hipModule_t module);
+// The same once per distinct `key`, for the life of the library.
 int rtc_get(const std::string &key, const std::string &source, const char *kernel_name, hipFunction_t *fn);
 bool rtc_find(const std::string &key, hipFunction_t *fn);   // a kernel compiled before (its source need not be put together again)
 int rtc_compile_only(const std::string &source, const char *arch, std::string *log);

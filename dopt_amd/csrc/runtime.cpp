@@ -230,6 +230,26 @@ bool rtc_find(const std::string &key, hipFunction_t *fn)
     return true;
 }
 
+int rtc_load(const std::string &source, const char *kernel_name, hipModule_t *module, hipFunction_t *fn)
+{
+    std::vector<char> code;
+    if (int rc = rtc_compile(source, rt().arch.c_str(), &code, nullptr)) return rc;
+    hipError_t e = hipModuleLoadData(module, code.data());
+    if (e == hipSuccess && (e = hipModuleGetFunction(fn, *module, kernel_name)) != hipSuccess) (void)hipModuleUnload(*module);
+    if (e == hipSuccess) return DOPT_HIP_OK;
+    (void)hipGetLastError();   // reported here: a caller that can do without must not find it behind its next launch
+    return fail(DOPT_HIP_ERR_RUNTIME, "loading the compiled kernel %s failed: %s", kernel_name, hipGetErrorString(e));
+}
+
+void rtc_idle()
+{
+    if (!rt().ready) return;
+    (void)hipStreamSynchronize(rt().stream);
+    (void)hipStreamSynchronize(rt().side);
+}
+
+void rtc_unload(hipModule_t module) { (void)hipModuleUnload(module); }
+
 int rtc_get(const std::string &key, const std::string &source, const char *kernel_name, hipFunction_t *fn)
 {
     Runtime &r = rt();
@@ -238,20 +258,10 @@ int rtc_get(const std::string &key, const std::string &source, const char *kerne
         *fn = it->second;
         return DOPT_HIP_OK;
     }
-    std::vector<char> code;
-    int rc = rtc_compile(source, r.arch.c_str(), &code, nullptr);
-    if (rc) return rc;
     hipModule_t mod;
-    hipError_t e = hipModuleLoadData(&mod, code.data());
     hipFunction_t f;
-    if (e == hipSuccess) {
-        r.modules.push_back(mod);
-        e = hipModuleGetFunction(&f, mod, kernel_name);
-    }
-    if (e != hipSuccess) {
-        (void)hipGetLastError();   // reported here: a caller that can do without must not find it behind its next launch
-        return fail(DOPT_HIP_ERR_RUNTIME, "loading the compiled kernel %s failed: %s", kernel_name, hipGetErrorString(e));
-    }
+    if (int rc = rtc_load(source, kernel_name, &mod, &f)) return rc;
+    r.modules.push_back(mod);
     r.kernels[key] = f;
     *fn = f;
     return DOPT_HIP_OK;
@@ -301,6 +311,7 @@ int dopt_hip_shutdown(void)
     for (hipModule_t m : r.modules) (void)hipModuleUnload(m);
     r.modules.clear();
     r.kernels.clear();
+    tiny_codes_shutdown();
     if (r.uploads) (void)hipEventDestroy(r.uploads);
     r.uploads = nullptr;
     (void)hipStreamDestroy(r.stream);
@@ -397,6 +408,7 @@ int dopt_hip_pool_trim(void)
         lane_cache.clear();
     }
     r.cached_bytes = 0;
+    tiny_codes_trim();
     return DOPT_HIP_OK;
 }
 

@@ -11,7 +11,7 @@
 // loss of the 784-512-512-10 network, 13 on 2560 values, 18 -> 4.7; of VGG-16, 13 on 1280, 25 -> 5.
 #include <algorithm>
 #include <cstring>
-#include <map>
+#include <list>
 #include <mutex>
 #include <string>
 
@@ -418,6 +418,68 @@ struct Generator {
 
 namespace dopt {
 
+// The code objects of compiled runs, by their sources, the one that was asked for last at the back.  Runs with the same source
+// share one.  Those that no run holds any more are kept for the next plan of the same network - compiling one takes 0.1 s - but
+// only the kIdleCodes newest: a program that makes a plan for every batch size it meets would collect them.
+struct TinyRun::Code {
+    std::string source;
+    hipModule_t module;
+    hipFunction_t fn;   // null once the library has been shut down
+};
+
+namespace {
+
+constexpr size_t kIdleCodes = 64;
+
+struct Codes {
+    std::mutex mutex;
+    std::list<std::shared_ptr<TinyRun::Code>> all;
+};
+Codes &codes()
+{
+    static Codes *const c = new Codes;   // plans may be destroyed behind the end of main
+    return *c;
+}
+
+// (mutex held)
+void drop_idle(Codes &c, size_t keep)
+{
+    if (capturing()) return;   // nothing can be waited for now
+    size_t idle = 0;
+    for (const auto &code : c.all) idle += code.use_count() == 1;
+    if (idle <= keep) return;
+    rtc_idle();   // a kernel of a run that is gone may still be queued
+    for (auto it = c.all.begin(); it != c.all.end() && idle > keep;) {
+        if (it->use_count() != 1) {
+            ++it;
+            continue;
+        }
+        rtc_unload((*it)->module);
+        it = c.all.erase(it);
+        idle--;
+    }
+}
+
+}  // namespace
+
+void tiny_codes_trim()
+{
+    Codes &c = codes();
+    std::lock_guard<std::mutex> lock(c.mutex);
+    drop_idle(c, 0);
+}
+
+void tiny_codes_shutdown()
+{
+    Codes &c = codes();
+    std::lock_guard<std::mutex> lock(c.mutex);
+    for (const auto &code : c.all) {
+        rtc_unload(code->module);
+        code->fn = nullptr;
+    }
+    c.all.clear();
+}
+
 TinyRun::TinyRun(int nslots, const std::vector<dopt_hip_tiny_node> &nodes) : slots(nslots)
 {
     Generator g(nodes);
@@ -428,15 +490,38 @@ TinyRun::TinyRun(int nslots, const std::vector<dopt_hip_tiny_node> &nodes) : slo
     g.pass();
     threads = g.threads;
     source = g.source(nslots);
-    // (a short name for the source: it is looked up at every launch)
-    static std::mutex mutex;
-    static std::map<std::string, size_t> names;
-    {
-        std::lock_guard<std::mutex> lock(mutex);
-        key = "tiny:" + std::to_string(names.emplace(source, names.size()).first->second);
-    }
     for (size_t v = 0; v < g.values.size(); v++)
         (v < nodes.size() ? writes : reads).push_back({g.values[v].slot, g.values[v].offset, 4 * g.values[v].n});
+}
+
+TinyRun::~TinyRun()
+{
+    if (!code) return;
+    Codes &c = codes();
+    std::lock_guard<std::mutex> lock(c.mutex);
+    code.reset();
+    drop_idle(c, kIdleCodes);
+}
+
+// The run's kernel, compiled where no run with the same source has been.
+int TinyRun::compile() const
+{
+    Codes &c = codes();
+    std::lock_guard<std::mutex> lock(c.mutex);
+    code.reset();
+    for (auto it = c.all.begin(); it != c.all.end(); ++it)
+        if ((*it)->source == source) {
+            code = *it;
+            c.all.splice(c.all.end(), c.all, it);
+            return DOPT_HIP_OK;
+        }
+    auto made = std::make_shared<Code>();
+    made->source = source;
+    if (int rc = rtc_load(source, "tiny_run", &made->module, &made->fn)) return rc;
+    c.all.push_back(made);
+    code = made;
+    drop_idle(c, kIdleCodes);
+    return DOPT_HIP_OK;
 }
 
 int TinyRun::launch(void *const *ptrs, bool *done) const
@@ -450,10 +535,9 @@ int TinyRun::launch(void *const *ptrs, bool *done) const
             if (lo < wlo + w.bytes && wlo < lo + r.bytes) return DOPT_HIP_OK;   // a caller's argument lies in what the run writes
         }
     }
-    hipFunction_t fn;
-    if (!rtc_find(key, &fn)) {
+    if (!code || !code->fn) {
         const std::string said = dopt_hip_last_error();
-        if (rtc_get(key, source, "tiny_run", &fn)) {   // no compiler, no memory for the code: dopt_hip_tiny_graph needs neither
+        if (compile()) {   // no compiler, no memory for the code: dopt_hip_tiny_graph needs neither
             refused = true;
             fail(DOPT_HIP_OK, "%s", said.c_str());   // what this call puts right is no error of its caller
             return DOPT_HIP_OK;
@@ -462,7 +546,7 @@ int TinyRun::launch(void *const *ptrs, bool *done) const
     void *args[DOPT_HIP_TINY_SLOTS];
     for (int i = 0; i < slots; i++) args[i] = (void *)&ptrs[i];
     *done = true;
-    return rtc_launch(fn, 1, (unsigned)threads, args);
+    return rtc_launch(code->fn, 1, (unsigned)threads, args);
 }
 
 }  // namespace dopt

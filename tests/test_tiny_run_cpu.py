@@ -1,5 +1,5 @@
 """A plan's compiled runs of tiny operations (tiny_rtc.cpp) against a run-time compiler that is played by a table: what a run does
-when it cannot be compiled, without a device."""
+when it cannot be compiled, and what becomes of the code of runs that are gone, without a device."""
 import os
 import subprocess
 
@@ -9,14 +9,12 @@ CSRC = os.path.join(ROOT, "dopt_amd", "csrc")
 HARNESS = r"""
 #include <cassert>
 #include <cstdarg>
-#include <map>
 #include <memory>
 #include "common.h"
 
 static std::string error_text;
-static std::map<std::string, hipFunction_t> compiled;
-static bool broken = false;
-static int attempts = 0, launches = 0;
+static bool broken = false, recording = false;
+static int attempts = 0, launches = 0, loaded = 0, waits = 0;
 
 extern "C" const char *dopt_hip_last_error(void) { return error_text.c_str(); }
 
@@ -31,19 +29,18 @@ int fail(int code, const char *fmt, ...)
     error_text = buf;
     return code;
 }
-bool rtc_find(const std::string &key, hipFunction_t *fn)
-{
-    auto it = compiled.find(key);
-    if (it != compiled.end()) *fn = it->second;
-    return it != compiled.end();
-}
-int rtc_get(const std::string &key, const std::string &, const char *, hipFunction_t *fn)
+int rtc_load(const std::string &, const char *, hipModule_t *module, hipFunction_t *fn)
 {
     attempts++;
     if (broken) return fail(DOPT_HIP_ERR_RTC, "hipRTC compilation failed");
-    *fn = compiled[key] = (hipFunction_t)(compiled.size() + 1);
+    loaded++;
+    *module = (hipModule_t)1;
+    *fn = (hipFunction_t)1;
     return DOPT_HIP_OK;
 }
+void rtc_idle() { waits++; }
+void rtc_unload(hipModule_t) { loaded--; }
+bool capturing() { return recording; }
 int rtc_launch(hipFunction_t, unsigned, unsigned, void **)
 {
     launches++;
@@ -70,7 +67,7 @@ static std::unique_ptr<TinyRun> make_run(int n)
     return std::unique_ptr<TinyRun>(new TinyRun(4, nodes));
 }
 
-static float memory[4][64];
+static float memory[4][256];
 static void *slots[4] = {memory[0], memory[1], memory[2], memory[3]};
 
 #define CHECK(x) do { if (!(x)) { printf("line %d: %s\n", __LINE__, #x); return 1; } } while (0)
@@ -110,4 +107,46 @@ def test_a_run_that_cannot_be_compiled_is_left_to_the_interpreter(tmp_path):
         CHECK(other->launch(slots, &done) == DOPT_HIP_OK && done);
         CHECK(launches == i + 1 && attempts == 2);
     }
+""")
+
+
+def test_the_code_of_runs_that_are_gone_is_bounded(tmp_path):
+    _run(tmp_path, r"""
+    bool done;
+    std::vector<std::unique_ptr<TinyRun>> live;
+    for (int n = 1; n <= 200; n++) {   // a plan for every batch size
+        make_run(n)->launch(slots, &done);
+        CHECK(done && attempts == n && loaded == std::min(n, 64));
+    }
+    make_run(200)->launch(slots, &done);   // the newest are still there
+    CHECK(done && attempts == 200);
+    for (int n = 1; n <= 200; n++) {   // all at once: none is taken from a run that holds it
+        live.push_back(make_run(n));
+        live.back()->launch(slots, &done);
+        live.back()->launch(slots, &done);
+        CHECK(done);
+    }
+    CHECK(loaded >= 200 && loaded <= 264);
+    auto second = make_run(7);   // shares the code of the one above
+    const int before = attempts;
+    second->launch(slots, &done);
+    CHECK(done && attempts == before);
+    recording = true;   // nothing can be waited for, so nothing is unloaded
+    const int kept = loaded, waited = waits;
+    for (int n = 0; n < 150; n++) live[(size_t)n].reset();
+    CHECK(loaded == kept && waits == waited);
+    recording = false;
+    live.clear();
+    CHECK(loaded <= 65 && waits > waited);
+    tiny_codes_trim();
+    CHECK(loaded == 1);
+    second->launch(slots, &done);
+    CHECK(done && attempts == before);
+    tiny_codes_shutdown();   // and the run compiles its kernel again
+    CHECK(loaded == 0);
+    second->launch(slots, &done);
+    CHECK(done && attempts == before + 1 && loaded == 1);
+    second.reset();
+    tiny_codes_trim();
+    CHECK(loaded == 0);
 """)
