@@ -115,9 +115,9 @@ int pointwise_group(const PointwiseProgram &program, const std::vector<Pointwise
 int reduce_squares_batch(int count, const float *const *in, const size_t *n, float *const *out);
 
 // tiny_rtc.cpp: a run of operations on tiny tensors (dopt_hip_tiny_graph's nodes) as a kernel of its own, compiled when it is first
-// launched.  The results' buffers must not overlap each other, which a plan's own do not.  `done` stays false, with nothing
-// launched, for runs it does not take, where what is read from outside overlaps a result and where the kernel cannot be compiled or
-// loaded (which is tried once): those are dopt_hip_tiny_graph's.
+// launched.  The results' buffers must overlap neither each other nor what is read from outside: a plan's own do not, and a plan
+// that is given an argument in one of them (HIPPlan::mInOrder) does not call this.  `done` stays false, with nothing launched, for
+// runs it does not take and where the kernel cannot be compiled or loaded (which is tried once): those are dopt_hip_tiny_graph's.
 struct TinyRun {
     TinyRun(int nslots, const std::vector<dopt_hip_tiny_node> &nodes);
     ~TinyRun();
@@ -128,12 +128,10 @@ struct TinyRun {
 
 private:
     int compile() const;
-    struct Range { int slot, offset, bytes; };
     int slots, threads = 0;
     mutable bool refused = false;
     mutable std::shared_ptr<Code> code;
     std::string source;
-    std::vector<Range> reads, writes;
 };
 void tiny_codes_trim();       // unloads the code of runs that are gone
 void tiny_codes_shutdown();   // unloads all of it, with the queues idle; runs that are left compile theirs again

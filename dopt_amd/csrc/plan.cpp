@@ -1390,11 +1390,13 @@ void HIPPlan::Builder::formTinyRuns()
                     if (m.op != last) tinyWrites[last].push_back(m.op);
                 const int nslots = (int)slots.size();
                 const auto own = std::make_shared<TinyRun>(nslots, nodes);
+                const HIPPlan *const plan = p;
                 prebuilt[last] = make([=](const std::vector<const void *> &in, void *out) {
                     void *ptrs[DOPT_HIP_TINY_SLOTS];
                     for (int k = 0; k < nslots; k++) ptrs[k] = slotIn[(size_t)k] >= 0 ? const_cast<void *>(in[(size_t)slotIn[(size_t)k]]) : out;
-                    bool done;
-                    if (int rc = own->launch(ptrs, &done)) return rc;
+                    bool done = false;
+                    if (!plan->mInOrder)   // (the interpreter goes through memory in the nodes' order)
+                        if (int rc = own->launch(ptrs, &done)) return rc;
                     if (done) return (int)DOPT_HIP_OK;
                     return dopt_hip_tiny_graph(nslots, ptrs, (int)nodes.size(), nodes.data());
                 });

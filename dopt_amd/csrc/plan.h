@@ -128,7 +128,8 @@ private:
     std::vector<void *> mOwned;                  // buffers to free in cleanup
     std::vector<std::pair<const char *, const char *>> mResultRanges;   // of the buffers that steps fill, ascending
     // This execution was given an argument that lies in a buffer which a step fills.  What reads it reads it where it stands:
-    // batches of steps that stood apart, whose members may be done in any order, are replaced by their members.
+    // batches of steps that stood apart, whose members may be done in any order, are replaced by their members, and compiled runs
+    // of tiny operations, which load everything first, by the interpreter.
     bool mInOrder = false;
     // Arguments that arrive as host arrays (cuda/package.d:367-401 uploads them with a blocking copy on every
     // execution): two slots per argument, each a page-locked staging copy and a device copy, used in turn.  The host

@@ -490,8 +490,6 @@ TinyRun::TinyRun(int nslots, const std::vector<dopt_hip_tiny_node> &nodes) : slo
     g.pass();
     threads = g.threads;
     source = g.source(nslots);
-    for (size_t v = 0; v < g.values.size(); v++)
-        (v < nodes.size() ? writes : reads).push_back({g.values[v].slot, g.values[v].offset, 4 * g.values[v].n});
 }
 
 TinyRun::~TinyRun()
@@ -528,13 +526,6 @@ int TinyRun::launch(void *const *ptrs, bool *done) const
 {
     *done = false;
     if (threads == 0 || refused) return DOPT_HIP_OK;
-    for (const Range &r : reads) {
-        const char *lo = (const char *)ptrs[r.slot] + r.offset;
-        for (const Range &w : writes) {
-            const char *wlo = (const char *)ptrs[w.slot] + w.offset;
-            if (lo < wlo + w.bytes && wlo < lo + r.bytes) return DOPT_HIP_OK;   // a caller's argument lies in what the run writes
-        }
-    }
     if (!code || !code->fn) {
         const std::string said = dopt_hip_last_error();
         if (compile()) {   // no compiler, no memory for the code: dopt_hip_tiny_graph needs neither
