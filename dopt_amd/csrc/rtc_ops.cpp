@@ -493,6 +493,34 @@ extern "C" __global__ __launch_bounds__(BLOCK) void red_cols(const T *in, T *out
 // blockDim / width rows side by side (consecutive threads, consecutive addresses where a row is one tile), each folds every
 // blockDim / width-th row, and the rows meet in LDS pairwise.  A slice's fold goes to out[(o * slices + s) * inner + j].
 // Bound by memory from a few MB on; sum of [17310, 17] over its rows 555 -> 8 us, of [7550, 786] 334 -> 15 us (both launches).
+__device__ inline T fold_rows(const T *p, size_t r, size_t r1, size_t inner, unsigned rows)
+{
+    T acc = (T)(IDENT);
+    for (; r + 7 * rows < r1; r += 8 * rows) {
+        T v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = PRE(p[(r + u * rows) * inner]);
+#pragma unroll
+        for (int u = 0; u < 8; u++) acc = combine(acc, v[u]);
+    }
+    for (; r < r1; r += rows) acc = combine(acc, PRE(p[r * inner]));
+    return acc;
+}
+
+// The rows that lie side by side, into the first of them (every thread of the block calls this).
+__device__ inline T meet_rows(T *part, T acc, unsigned rows, unsigned width, bool mine)
+{
+    const unsigned ty = threadIdx.x / width;
+    part[threadIdx.x] = acc;
+    for (unsigned n = rows; n > 1;) {
+        const unsigned half = (n + 1) / 2;
+        __syncthreads();
+        if (mine && ty + half < n) part[threadIdx.x] = acc = combine(acc, part[threadIdx.x + half * width]);
+        n = half;
+    }
+    return acc;
+}
+
 extern "C" __global__ __launch_bounds__(1024) void red_cols_split(const T *in, T *out, size_t R, size_t inner, size_t rows_per,
                                                                    unsigned width, unsigned tiles, unsigned slices)
 {
@@ -504,25 +532,38 @@ extern "C" __global__ __launch_bounds__(1024) void red_cols_split(const T *in, T
     T acc = (T)(IDENT);
     if (mine) {
         const size_t r0 = (size_t)s * rows_per, r1 = r0 + rows_per < R ? r0 + rows_per : R;
-        const T *p = in + (size_t)o * R * inner + j;
-        size_t r = r0 + ty;
-        for (; r + 7 * rows < r1; r += 8 * rows) {
-            T v[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) v[u] = PRE(p[(r + u * rows) * inner]);
-#pragma unroll
-            for (int u = 0; u < 8; u++) acc = combine(acc, v[u]);
-        }
-        for (; r < r1; r += rows) acc = combine(acc, PRE(p[r * inner]));
+        acc = fold_rows(in + (size_t)o * R * inner + j, r0 + ty, r1, inner, rows);
     }
-    part[threadIdx.x] = acc;
-    for (unsigned n = rows; n > 1;) {
-        const unsigned half = (n + 1) / 2;
-        __syncthreads();
-        if (mine && ty + half < n) part[threadIdx.x] = acc = combine(acc, part[threadIdx.x + half * width]);
-        n = half;
-    }
+    acc = meet_rows(part, acc, rows, width, mine);
     if (mine && ty == 0) out[(size_t)os * inner + j] = acc;
+}
+
+// Both launches' folds as one, in their order, for where the slices' folds have no memory to go to: a block takes all slices of
+// its columns, one after the other.
+#define SLICE_FOLDS 16384   // slices x width at most (cols_split)
+extern "C" __global__ __launch_bounds__(1024) void red_cols_whole(const T *in, T *out, size_t R, size_t inner, size_t rows_per,
+                                                                   unsigned width, unsigned tiles, unsigned slices)
+{
+    __shared__ T part[1024], folds[SLICE_FOLDS];
+    const unsigned tile = blockIdx.x % tiles, o = blockIdx.x / tiles;
+    const unsigned rows = blockDim.x / width, ty = threadIdx.x / width, tx = threadIdx.x - ty * width;
+    const size_t j = (size_t)tile * width + tx;
+    const bool mine = ty < rows && j < inner;
+    for (unsigned s = 0; s < slices; s++) {
+        T acc = (T)(IDENT);
+        if (mine) {
+            const size_t r0 = (size_t)s * rows_per, r1 = r0 + rows_per < R ? r0 + rows_per : R;
+            acc = fold_rows(in + (size_t)o * R * inner + j, r0 + ty, r1, inner, rows);
+        }
+        acc = meet_rows(part, acc, rows, width, mine);
+        if (mine && ty == 0) folds[s * width + tx] = acc;
+        __syncthreads();
+    }
+    T acc = (T)(IDENT);
+    if (mine)
+        for (unsigned s = ty; s < slices; s += rows) acc = combine(acc, folds[s * width + tx]);
+    acc = meet_rows(part, acc, rows, width, mine);
+    if (mine && ty == 0) out[(size_t)o * inner + j] = acc;
 }
 )SRC";
 
@@ -676,19 +717,20 @@ int check_dtype(int dtype)
 // One (outer, R, inner) reduction pass on the device.
 // `later` folds partial results: the first stage may fold PRE(element), the second never does.
 struct ReduceKernels {
-    hipFunction_t rows, rows4, rows4u, cols, split;
+    hipFunction_t rows, rows4, rows4u, cols, split, whole;
 };
 int reduce_kernels(const std::string &key, bool is_sum, int dtype, bool square, ReduceKernels *k)
 {
     if (rtc_find(key + ":rows", &k->rows) && rtc_find(key + ":rows4", &k->rows4) && rtc_find(key + ":rows4u", &k->rows4u) &&
-        rtc_find(key + ":cols", &k->cols) && rtc_find(key + ":split", &k->split))
+        rtc_find(key + ":cols", &k->cols) && rtc_find(key + ":split", &k->split) && rtc_find(key + ":whole", &k->whole))
         return DOPT_HIP_OK;
     const std::string src = reduce_source(is_sum, dtype, square);
     if (int rc = rtc_get(key + ":rows", src, "red_rows", &k->rows)) return rc;
     if (int rc = rtc_get(key + ":rows4", src, "red_rows4", &k->rows4)) return rc;
     if (int rc = rtc_get(key + ":rows4u", src, "red_rows4u", &k->rows4u)) return rc;
     if (int rc = rtc_get(key + ":cols", src, "red_cols", &k->cols)) return rc;
-    return rtc_get(key + ":split", src, "red_cols_split", &k->split);
+    if (int rc = rtc_get(key + ":split", src, "red_cols_split", &k->split)) return rc;
+    return rtc_get(key + ":whole", src, "red_cols_whole", &k->whole);
 }
 
 // How much of a contiguous row of R values one workgroup folds.
@@ -718,7 +760,7 @@ bool cols_split(size_t outer, size_t R, size_t inner, ColsSplit *c)
     c->tiles = (unsigned)tiles;
     c->width = (unsigned)ceil_div(inner, tiles);
     // one launch while a thread has no more than 64 rows; else two blocks on every CU with at least 8 rows a thread, and no more
-    // slices than the launch that adds them folds in 16 rows a thread
+    // slices than the launch that adds them folds in 16 rows a thread (SLICE_FOLDS)
     const size_t side = 1024 / c->width;
     size_t slices = 1;
     if (R > side * 64) slices = std::min({ceil_div((size_t)num_cus() * 2, outer * tiles), ceil_div(R, side * 8), side * 16});
@@ -737,9 +779,8 @@ int reduce_pass(const ReduceKernels &k, const void *in, void *out, size_t outer,
     if (cols_split(outer, R, inner, &c)) {
         void *first = out;
         if (c.slices > 1 && !(first = workspace_if_free(outer * c.slices * inner * esize))) {
-            first = out;
-            c.slices = 1;
-            c.rows_per = R;
+            void *all[] = {(void *)&in, (void *)&out, (void *)&R, (void *)&inner, (void *)&c.rows_per, (void *)&c.width, (void *)&c.tiles, (void *)&c.slices};
+            return rtc_launch(k.whole, (unsigned)(outer * c.tiles), 1024, all);
         }
         void *args[] = {(void *)&in, (void *)&first, (void *)&R, (void *)&inner, (void *)&c.rows_per, (void *)&c.width, (void *)&c.tiles,
                         (void *)&c.slices};

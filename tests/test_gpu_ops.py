@@ -200,6 +200,32 @@ def test_folds_of_few_columns_over_many_rows(outer, rows, inner):
         assert np.array_equal(ops.sum(whole.view(1, x.shape), [1]).numpy(), got)
 
 
+@pytest.mark.parametrize("outer,rows,inner", [(1, 70000, 2), (1, 20001, 3), (1, 17310, 17), (2, 40000, 64), (1, 9000, 305), (3, 9001, 65)])
+def test_folds_of_few_columns_do_not_depend_on_scratch(outer, rows, inner):
+    """Folds in slices while an open convolution result occupies the workspace: the bits of the fold that may use it."""
+    import ctypes as C
+    from dopt_amd import capi
+    lib, r = capi.load(), rng(outer + rows)
+    x, w, y = T(r.standard_normal((8, 256, 4, 4)).astype(np.float32)), T(r.standard_normal((512, 256, 3, 3)).astype(np.float32)), ops.Tensor((8, 512, 4, 4))
+    d = ops.conv_desc(x.shape, w.shape, (1, 1), (1, 1))
+    packed, want = ops.Tensor((lib.dopt_hip_conv_packed_bytes(C.byref(d), 0) // 4,)), ops.convolution(x, w, (1, 1), (1, 1)).numpy()
+    capi.check(lib.dopt_hip_conv_pack_batch(1, (capi.ConvDesc * 1)(d), (C.c_int * 1)(0), (C.c_void_p * 1)(w.ptr), (C.c_void_p * 1)(packed.ptr)))
+    f = T(r.standard_normal((outer, rows, inner)).astype(np.float32))
+    i = T(r.integers(-2**31, 2**31 - 1, f.shape).astype(np.int32))
+    folds = [lambda o: ops.sum(f, [1], out=o), lambda o: ops.max_element(f, [1], out=o), lambda o: ops.sum_of_squares(f, [1], out=o),
+             lambda o: ops.sum(i, [1], out=o)]
+    for k, fold in enumerate(folds):
+        a, b = (ops.Tensor((outer, inner), np.int32 if k == 3 else np.float32) for _ in range(2))
+        fold(a)
+        o = capi.SplitSum()
+        capi.check(lib.dopt_hip_conv_fwd_bias_packed_open(C.byref(d), x.ptr, packed.ptr, None, y.ptr, C.byref(o)))
+        assert o.splits > 1
+        fold(b)
+        capi.check(lib.dopt_hip_split_sum_close(C.byref(o)))
+        assert np.array_equal(a.numpy(), b.numpy()), k
+        assert np.array_equal(y.numpy(), want)
+
+
 def test_max_identity_is_minus_type_max():
     x = np.full((3, 5), -2**31, np.int32)
     assert np.array_equal(ops.max_element(T(x), (1,)).numpy(), O.max_element(x, (1,)))
