@@ -136,12 +136,14 @@ private:
 void tiny_codes_trim();       // unloads the code of runs that are gone
 void tiny_codes_shutdown();   // unloads all of it, with the queues idle; runs that are left compile theirs again
 
-// hipRTC: compile `source`, load it and find the named kernel in it; wait for all that is queued; unload.
-int rtc_load(const std::string &source, const char *kernel_name, hipModule_t *module, hipFunction_t *fn);
+// hipRTC: compile `source`, load it and find the named kernels in it; wait for all that is queued; unload.
+int rtc_load(const std::string &source, int n, const char *const *names, hipModule_t *module, hipFunction_t *fns);
 void rtc_idle();
 void rtc_unload(hipModule_t module);
 // The same once per distinct `key`, for the life of the library.
 int rtc_get(const std::string &key, const std::string &source, const char *kernel_name, hipFunction_t *fn);
+// ... and several kernels of one source (under key:name), which is compiled once for all of them.
+int rtc_get_all(const std::string &key, const std::string &source, int n, const char *const *names, hipFunction_t *fns);
 bool rtc_find(const std::string &key, hipFunction_t *fn);   // a kernel compiled before (its source need not be put together again)
 int rtc_compile_only(const std::string &source, const char *arch, std::string *log);
 int rtc_launch(hipFunction_t fn, unsigned grid, unsigned block, void **args);

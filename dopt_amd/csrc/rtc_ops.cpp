@@ -538,6 +538,7 @@ extern "C" __global__ __launch_bounds__(1024) void red_cols_split(const T *in, T
     if (mine && ty == 0) out[(size_t)os * inner + j] = acc;
 }
 
+#ifdef WHOLE   // compiled when it is needed: it takes as long as all of the above
 // Both launches' folds as one, in their order, for where the slices' folds have no memory to go to: a block takes all slices of
 // its columns, one after the other.
 #define SLICE_FOLDS 16384   // slices x width at most (cols_split)
@@ -565,6 +566,7 @@ extern "C" __global__ __launch_bounds__(1024) void red_cols_whole(const T *in, T
     acc = meet_rows(part, acc, rows, width, mine);
     if (mine && ty == 0) out[(size_t)o * inner + j] = acc;
 }
+#endif
 )SRC";
 
 const char *kArgminBody = R"SRC(
@@ -717,20 +719,22 @@ int check_dtype(int dtype)
 // One (outer, R, inner) reduction pass on the device.
 // `later` folds partial results: the first stage may fold PRE(element), the second never does.
 struct ReduceKernels {
-    hipFunction_t rows, rows4, rows4u, cols, split, whole;
+    hipFunction_t rows, rows4, rows4u, cols, split;
+    std::string key;
+    bool is_sum, square;
+    int dtype;
 };
 int reduce_kernels(const std::string &key, bool is_sum, int dtype, bool square, ReduceKernels *k)
 {
-    if (rtc_find(key + ":rows", &k->rows) && rtc_find(key + ":rows4", &k->rows4) && rtc_find(key + ":rows4u", &k->rows4u) &&
-        rtc_find(key + ":cols", &k->cols) && rtc_find(key + ":split", &k->split) && rtc_find(key + ":whole", &k->whole))
-        return DOPT_HIP_OK;
-    const std::string src = reduce_source(is_sum, dtype, square);
-    if (int rc = rtc_get(key + ":rows", src, "red_rows", &k->rows)) return rc;
-    if (int rc = rtc_get(key + ":rows4", src, "red_rows4", &k->rows4)) return rc;
-    if (int rc = rtc_get(key + ":rows4u", src, "red_rows4u", &k->rows4u)) return rc;
-    if (int rc = rtc_get(key + ":cols", src, "red_cols", &k->cols)) return rc;
-    if (int rc = rtc_get(key + ":split", src, "red_cols_split", &k->split)) return rc;
-    return rtc_get(key + ":whole", src, "red_cols_whole", &k->whole);
+    const char *const names[] = {"red_rows", "red_rows4", "red_rows4u", "red_cols", "red_cols_split"};
+    constexpr int n = sizeof(names) / sizeof(names[0]);
+    hipFunction_t fns[n];
+    bool all = true;
+    for (int i = 0; i < n && all; i++) all = rtc_find(key + ":" + names[i], &fns[i]);
+    if (!all)
+        if (int rc = rtc_get_all(key, reduce_source(is_sum, dtype, square), n, names, fns)) return rc;
+    *k = ReduceKernels{fns[0], fns[1], fns[2], fns[3], fns[4], key, is_sum, square, dtype};
+    return DOPT_HIP_OK;
 }
 
 // How much of a contiguous row of R values one workgroup folds.
@@ -780,7 +784,11 @@ int reduce_pass(const ReduceKernels &k, const void *in, void *out, size_t outer,
         void *first = out;
         if (c.slices > 1 && !(first = workspace_if_free(outer * c.slices * inner * esize))) {
             void *all[] = {(void *)&in, (void *)&out, (void *)&R, (void *)&inner, (void *)&c.rows_per, (void *)&c.width, (void *)&c.tiles, (void *)&c.slices};
-            return rtc_launch(k.whole, (unsigned)(outer * c.tiles), 1024, all);
+            hipFunction_t whole;
+            const std::string key = k.key + ":red_cols_whole";
+            if (!rtc_find(key, &whole))
+                if (int rc = rtc_get(key, "#define WHOLE\n" + reduce_source(k.is_sum, k.dtype, k.square), "red_cols_whole", &whole)) return rc;
+            return rtc_launch(whole, (unsigned)(outer * c.tiles), 1024, all);
         }
         void *args[] = {(void *)&in, (void *)&first, (void *)&R, (void *)&inner, (void *)&c.rows_per, (void *)&c.width, (void *)&c.tiles,
                         (void *)&c.slices};

@@ -230,15 +230,18 @@ bool rtc_find(const std::string &key, hipFunction_t *fn)
     return true;
 }
 
-int rtc_load(const std::string &source, const char *kernel_name, hipModule_t *module, hipFunction_t *fn)
+int rtc_load(const std::string &source, int n, const char *const *names, hipModule_t *module, hipFunction_t *fns)
 {
     std::vector<char> code;
     if (int rc = rtc_compile(source, rt().arch.c_str(), &code, nullptr)) return rc;
     hipError_t e = hipModuleLoadData(module, code.data());
-    if (e == hipSuccess && (e = hipModuleGetFunction(fn, *module, kernel_name)) != hipSuccess) (void)hipModuleUnload(*module);
-    if (e == hipSuccess) return DOPT_HIP_OK;
+    if (e == hipSuccess) {
+        for (int i = 0; i < n && e == hipSuccess; i++) e = hipModuleGetFunction(&fns[i], *module, names[i]);
+        if (e == hipSuccess) return DOPT_HIP_OK;
+        (void)hipModuleUnload(*module);
+    }
     (void)hipGetLastError();   // reported here: a caller that can do without must not find it behind its next launch
-    return fail(DOPT_HIP_ERR_RUNTIME, "loading the compiled kernel %s failed: %s", kernel_name, hipGetErrorString(e));
+    return fail(DOPT_HIP_ERR_RUNTIME, "loading the compiled kernel %s failed: %s", names[0], hipGetErrorString(e));
 }
 
 void rtc_idle()
@@ -252,18 +255,22 @@ void rtc_unload(hipModule_t module) { (void)hipModuleUnload(module); }
 
 int rtc_get(const std::string &key, const std::string &source, const char *kernel_name, hipFunction_t *fn)
 {
+    if (rtc_find(key, fn)) return DOPT_HIP_OK;
     Runtime &r = rt();
-    auto it = r.kernels.find(key);
-    if (it != r.kernels.end()) {
-        *fn = it->second;
-        return DOPT_HIP_OK;
-    }
     hipModule_t mod;
-    hipFunction_t f;
-    if (int rc = rtc_load(source, kernel_name, &mod, &f)) return rc;
+    if (int rc = rtc_load(source, 1, &kernel_name, &mod, fn)) return rc;
     r.modules.push_back(mod);
-    r.kernels[key] = f;
-    *fn = f;
+    r.kernels[key] = *fn;
+    return DOPT_HIP_OK;
+}
+
+int rtc_get_all(const std::string &key, const std::string &source, int n, const char *const *names, hipFunction_t *fns)
+{
+    Runtime &r = rt();
+    hipModule_t mod;
+    if (int rc = rtc_load(source, n, names, &mod, fns)) return rc;
+    r.modules.push_back(mod);
+    for (int i = 0; i < n; i++) r.kernels[key + ":" + names[i]] = fns[i];
     return DOPT_HIP_OK;
 }
 

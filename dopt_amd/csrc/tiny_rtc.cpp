@@ -515,7 +515,8 @@ int TinyRun::compile() const
         }
     auto made = std::make_shared<Code>();
     made->source = source;
-    if (int rc = rtc_load(source, "tiny_run", &made->module, &made->fn)) return rc;
+    const char *const name = "tiny_run";
+    if (int rc = rtc_load(source, 1, &name, &made->module, &made->fn)) return rc;
     c.all.push_back(made);
     code = made;
     drop_idle(c, kIdleCodes);

@@ -29,7 +29,7 @@ int fail(int code, const char *fmt, ...)
     error_text = buf;
     return code;
 }
-int rtc_load(const std::string &, const char *, hipModule_t *module, hipFunction_t *fn)
+int rtc_load(const std::string &, int, const char *const *, hipModule_t *module, hipFunction_t *fn)
 {
     attempts++;
     if (broken) return fail(DOPT_HIP_ERR_RTC, "hipRTC compilation failed");
