@@ -838,37 +838,51 @@ struct VectorEpilogue {   // + rowvec[row] * colbias[col >> shift], relu, mask, 
 };
 
 // The matrix is stored row by row along the reduction: a wavefront per result, a lane per chain.
+// kFew: up to four steps of 64, where all the rest is only what a wavefront has to go through (3 000 000 rows of 2 steps 437 us with the
+// loops below, 314 so; 30000 of 64 6.7 and 4.5, of 129 7.7 and 5.4).
+template <bool kFew>
 __global__ __launch_bounds__(256) void gemv_rows_k(size_t M, size_t K, const float *A, const float *b, float *c, VectorEpilogue ep)
 {
     const size_t row = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= M) return;
     const int lane = threadIdx.x & 63;
     const float *ar = A + row * K;
+    if constexpr (kFew) {
+        float acc = 0.0f;
+        for (size_t k = lane; k < K; k += 64) acc += ar[k] * b[k];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
+        if (lane == 0) c[row] = ep(acc, row);
+        return;
+    }
     float total = 0.0f;
     for (size_t k0 = 0; k0 < K; k0 += kGemvSlice) {
         const size_t k1 = min(K, k0 + kGemvSlice);
         float acc = 0.0f;
-        size_t k = k0 + lane;
-        for (; k + 448 < k1; k += 512) {   // eight steps in flight
+        size_t k = k0;
+        for (; k + 512 <= k1; k += 512) {   // eight steps in flight
             float x[8], y[8];
 #pragma unroll
             for (int u = 0; u < 8; u++) {
-                x[u] = ar[k + 64 * u];
-                y[u] = b[k + 64 * u];
+                x[u] = ar[k + 64 * u + lane];
+                y[u] = b[k + 64 * u + lane];
             }
 #pragma unroll
             for (int u = 0; u < 8; u++) acc += x[u] * y[u];
         }
-        float x[7], y[7];   // what is left: up to seven steps, together as well
+        // what is left, as many steps as there are
+        const int left = (int)(k1 - k);
+        float x[8], y[8];
 #pragma unroll
-        for (int u = 0; u < 7; u++) {
-            const size_t at = min(k + 64 * u, K - 1);
-            x[u] = ar[at];
-            y[u] = b[at];
-        }
+        for (int u = 0; u < 8; u++)
+            if (64 * u < left) {   // (the same in every lane)
+                const size_t at = min(k + 64 * u + lane, k1 - 1);
+                x[u] = ar[at];
+                y[u] = b[at];
+            }
 #pragma unroll
-        for (int u = 0; u < 7; u++)
-            if (k + 64 * u < k1) acc += x[u] * y[u];
+        for (int u = 0; u < 8; u++)
+            if (64 * u + lane < left) acc += x[u] * y[u];
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
         total = k0 == 0 ? acc : total + acc;
@@ -876,66 +890,77 @@ __global__ __launch_bounds__(256) void gemv_rows_k(size_t M, size_t K, const flo
     if (lane == 0) c[row] = ep(total, row);
 }
 
-// The matrix is stored [K][N]: a block folds one slice of 32 columns, a thread eight neighbouring chains of a column.
-constexpr int kGemvCols = 32;
+// The matrix is stored [K][N]: a block of 256 threads folds one slice of 256 / kGroups columns, a thread 64 / kGroups neighbouring
+// chains of a column.  kLive: a reduction of so many steps at most, whose other chains are zeros that change nothing.
+template <int kGroups, int kLive = 64>
 struct GemvLds {
-    float chain[8][8][kGemvCols];   // group of chains, chain, column
+    static constexpr int kCols = 256 / kGroups, kChains = kLive / kGroups;
+    float chain[kGroups / 2][kChains][kCols];   // upper half of the groups, chain, column
 };
 // (`on`: false for the threads of a larger block that only keep the barriers company)
-template <class Store>
-__device__ __forceinline__ void gemv_cols_body(int K, int N, const float *a, const float *B, int bx, int k0, bool on, GemvLds &lds, Store &&store)
+template <int kGroups, int kLive = 64, class Store>
+__device__ __forceinline__ void gemv_cols_body(int K, int N, const float *a, const float *B, int bx, int k0, bool on, GemvLds<kGroups, kLive> &lds, Store &&store)
 {
-    const int col = threadIdx.x & 31, g = (threadIdx.x >> 5) & 7, k1 = min(K, k0 + kGemvSlice);
-    const int n = min(bx * kGemvCols + col, N - 1);
-    float acc[8];
+    constexpr int kCols = GemvLds<kGroups, kLive>::kCols, kChains = GemvLds<kGroups, kLive>::kChains;
+    constexpr int kSteps = kLive == 64 && kChains < 16 ? 16 / kChains : 1;   // sixteen loads in flight
+    const int col = threadIdx.x % kCols, g = threadIdx.x / kCols % kGroups, k1 = min(K, k0 + kGemvSlice);
+    const int n = min(bx * kCols + col, N - 1);
+    float acc[kChains];
 #pragma unroll
-    for (int j = 0; j < 8; j++) acc[j] = 0.0f;
+    for (int j = 0; j < kChains; j++) acc[j] = 0.0f;
     if (on) {
-        for (int k = k0 + 8 * g; k < k1; k += 128) {   // sixteen loads in flight (clamped, not branched)
-            float av[2][8], bv[2][8];
+        for (int k = k0 + kChains * g; k < k1; k += 64 * kSteps) {   // (clamped, not branched)
+            float av[kSteps][kChains], bv[kSteps][kChains];
 #pragma unroll
-            for (int u = 0; u < 2; u++)
+            for (int u = 0; u < kSteps; u++)
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
+                for (int j = 0; j < kChains; j++) {
                     const int at = min(k + 64 * u + j, K - 1);
                     av[u][j] = a[at];
                     bv[u][j] = B[(size_t)at * N + n];
                 }
 #pragma unroll
-            for (int u = 0; u < 2; u++)
+            for (int u = 0; u < kSteps; u++)
 #pragma unroll
-                for (int j = 0; j < 8; j++)
+                for (int j = 0; j < kChains; j++)
                     if (k + 64 * u + j < k1) acc[j] += av[u][j] * bv[u][j];
         }
     }
 #pragma unroll
-    for (int half = 4; half > 0; half >>= 1) {   // chains 32, 16 and 8 apart: groups
+    for (int half = kGroups / 2; half > 0; half >>= 1) {   // groups: chains kLive / 2, kLive / 4 .. apart
         if (on && g >= half && g < 2 * half) {
 #pragma unroll
-            for (int j = 0; j < 8; j++) lds.chain[g][j][col] = acc[j];
+            for (int j = 0; j < kChains; j++) lds.chain[g - half][j][col] = acc[j];
         }
         __syncthreads();
         if (on && g < half) {
 #pragma unroll
-            for (int j = 0; j < 8; j++) acc[j] += lds.chain[g + half][j][col];
+            for (int j = 0; j < kChains; j++) acc[j] += lds.chain[g][j][col];
         }
+        if (half > 1) __syncthreads();
     }
 #pragma unroll
-    for (int half = 4; half > 0; half >>= 1)
+    for (int half = kChains / 2; half > 0; half >>= 1)
 #pragma unroll
         for (int j = 0; j < half; j++) acc[j] += acc[j + half];
-    if (on && g == 0 && bx * kGemvCols + col < N) store(bx * kGemvCols + col, acc[0]);
+    if (on && g == 0 && bx * kCols + col < N) store(bx * kCols + col, acc[0]);
 }
 
 // blockIdx.y: the slice.  With more than one their sums go to consecutive copies of the result, which splitk_epilogue_k adds
 // (and `ep` does nothing).
+template <int kGroups, int kLive>
 __global__ __launch_bounds__(256) void gemv_cols_k(int K, int N, const float *a, const float *B, float *c, VectorEpilogue ep)
 {
-    __shared__ GemvLds lds;
+    __shared__ GemvLds<kGroups, kLive> lds;
     float *const to = c + (size_t)blockIdx.y * N;
-    gemv_cols_body(K, N, a, B, (int)blockIdx.x, (int)blockIdx.y * kGemvSlice, true, lds,
-                   [&](int n, float v) { to[n] = ep(v, (size_t)n); });
+    gemv_cols_body<kGroups, kLive>(K, N, a, B, (int)blockIdx.x, (int)blockIdx.y * kGemvSlice, true, lds,
+                                   [&](int n, float v) { to[n] = ep(v, (size_t)n); });
 }
+// Eight groups, so that few columns make as many threads as they can.  Four where there are 96 columns a CU, as sums that meet in LDS
+// and groups without a step of their own cost more then (30000 columns of 256 steps 7.8 us with eight, 7.0 with four; 16384 of 512
+// 5.1 and 7.0), and for reductions of up to 64 steps, of which a thread takes no more chains than there are (3 000 000 columns of 2 steps
+// 62 us with eight groups, 16 so; of 64 170 and 137; one group of all chains 13 and 139, but 300000 of 64 15.4, 13.8 with eight, 12.8 so).
+constexpr int kGemvGroups = 8;
 
 // Several independent small products in ONE launch: the weight and bias gradients of a dense head are six kernels of a
 // few microseconds each that wait for nothing but the gradient in front of them, and a kernel boundary costs as much as
@@ -963,14 +988,14 @@ __global__ __launch_bounds__(64 * kSmallWaves) void sgemm_small_group_k(SmallGro
 {
     __shared__ union {
         float red[kSmallWaves][32 * 33];
-        GemvLds gemv;
+        GemvLds<kGemvGroups> gemv;
     } lds;
     const int b = (int)blockIdx.x;   // uniform: the scans below stay scalar
     if (g.nv > 0 && b >= g.v[0].first) {
         int j = 0;
         while (j + 1 < g.nv && b >= g.v[j + 1].first) j++;
         const GemvJob &q = g.v[j];
-        gemv_cols_body(q.K, q.N, q.a, q.B, b - q.first, 0, threadIdx.x < 256, lds.gemv, [&](int n, float v) { q.c[n] = v; });
+        gemv_cols_body<kGemvGroups>(q.K, q.N, q.a, q.B, b - q.first, 0, threadIdx.x < 256, lds.gemv, [&](int n, float v) { q.c[n] = v; });
         return;
     }
     int j = 0;
@@ -1080,6 +1105,22 @@ struct Extras {
 
 // Whether a matrix times a vector finds the matrix stored row by row along the reduction (where both sides are vectors it does).
 bool gemv_by_rows(int transA, int transB, size_t M, size_t N) { return (N == 1 && !transA) || (M == 1 && transB) || (M == 1 && N == 1); }
+
+template <int kGroups, int kLive = 64>
+void launch_gemv_groups(int K, int N, size_t slices, const float *a, const float *B, float *c, const VectorEpilogue &ep)
+{
+    const dim3 grid((unsigned)ceil_div((size_t)N, (size_t)GemvLds<kGroups, kLive>::kCols), (unsigned)slices);
+    hipLaunchKernelGGL((gemv_cols_k<kGroups, kLive>), grid, dim3(256), 0, stream(), K, N, a, B, c, ep);
+}
+int launch_gemv_cols(int K, int N, size_t slices, const float *a, const float *B, float *c, const VectorEpilogue &ep)
+{
+    if (K <= 16) launch_gemv_groups<4, 16>(K, N, slices, a, B, c, ep);
+    else if (K <= 32) launch_gemv_groups<4, 32>(K, N, slices, a, B, c, ep);
+    else if (K <= 64 || N >= 96 * num_cus()) launch_gemv_groups<4>(K, N, slices, a, B, c, ep);
+    else launch_gemv_groups<kGemvGroups>(K, N, slices, a, B, c, ep);
+    DOPT_LAUNCH_CHECK();
+    return DOPT_HIP_OK;
+}
 
 int sgemm_epilogue(int transA, int transB, size_t M, size_t N, size_t K, const float *A, const float *B, float *C,
                    const float *colbias, int bias_shift, const float *rowvec, int relu, bool *biased, const Extras &ex = Extras{});
@@ -1285,16 +1326,18 @@ int sgemm_epilogue(int transA, int transB, size_t M, size_t N, size_t K, const f
         const VectorEpilogue ep{colbias, rowvec, ex.mask, bias_shift, relu, N}, none{nullptr, nullptr, nullptr, 0, 0, 1};
         *biased = true;
         if (gemv_by_rows(transA, transB, M, N)) {
-            hipLaunchKernelGGL(gemv_rows_k, dim3((unsigned)ceil_div(R, (size_t)4)), dim3(256), 0, stream(), R, K, mat, vec, C, ep);
+            const dim3 grid((unsigned)ceil_div(R, (size_t)4));
+            if (K <= 256) hipLaunchKernelGGL(gemv_rows_k<true>, grid, dim3(256), 0, stream(), R, K, mat, vec, C, ep);
+            else hipLaunchKernelGGL(gemv_rows_k<false>, grid, dim3(256), 0, stream(), R, K, mat, vec, C, ep);
             DOPT_LAUNCH_CHECK();
             return DOPT_HIP_OK;
         }
         float *to = C;
         if (slices > 1 && !(to = (float *)workspace(slices * R * sizeof(float)))) return DOPT_HIP_ERR_OOM;
         for (size_t s0 = 0; s0 < slices; s0 += 65535)   // (a grid's second dimension)
-            hipLaunchKernelGGL(gemv_cols_k, dim3((unsigned)ceil_div(R, (size_t)kGemvCols), (unsigned)std::min(slices - s0, (size_t)65535)), dim3(256), 0, stream(),
-                               (int)(K - s0 * kGemvSlice), (int)R, vec + s0 * kGemvSlice, mat + s0 * kGemvSlice * R, to + s0 * R, slices > 1 ? none : ep);
-        DOPT_LAUNCH_CHECK();
+            if (int rc = launch_gemv_cols((int)(K - s0 * kGemvSlice), (int)R, std::min(slices - s0, (size_t)65535), vec + s0 * kGemvSlice,
+                                          mat + s0 * kGemvSlice * R, to + s0 * R, slices > 1 ? none : ep))
+                return rc;
         if (slices > 1) {
             hipLaunchKernelGGL(splitk_epilogue_k, dim3(flat_grid(R)), dim3(256), 0, stream(), M, N, (int)slices, to, C, colbias, bias_shift, rowvec, relu,
                                ex.mask);
@@ -1476,7 +1519,7 @@ int dopt_hip_sgemm_batch(int n, const int *transA, const int *transB, const size
                 GemvJob &q = in.g.v[in.g.nv++];
                 q = v;
                 q.first = (int)in.blocks;
-                in.blocks += (unsigned)ceil_div((size_t)v.N, (size_t)kGemvCols);
+                in.blocks += (unsigned)ceil_div((size_t)v.N, (size_t)GemvLds<kGemvGroups>::kCols);
             }
             gemvs.clear();
         }
@@ -1490,9 +1533,7 @@ int dopt_hip_sgemm_batch(int n, const int *transA, const int *transB, const size
         DOPT_LAUNCH_CHECK();
     }
     for (const GemvJob &v : gemvs) {   // no 32 x 32-tile launch to ride in
-        hipLaunchKernelGGL(gemv_cols_k, dim3((unsigned)ceil_div((size_t)v.N, (size_t)kGemvCols)), dim3(256), 0, stream(), v.K, v.N, v.a, v.B, v.c,
-                           VectorEpilogue{nullptr, nullptr, nullptr, 0, 0, 1});
-        DOPT_LAUNCH_CHECK();
+        if (int rc = launch_gemv_cols(v.K, v.N, 1, v.a, v.B, v.c, VectorEpilogue{nullptr, nullptr, nullptr, 0, 0, 1})) return rc;
     }
     for (int i : single)
         if (int rc = dopt_hip_sgemm_t(transA[i], transB[i], M[i], N[i], K[i], A[i], B[i], C[i])) return rc;

@@ -7,6 +7,8 @@ has magnitude sqrt(n) and atol is scaled by that; the same kernel is then run ag
 as the configurations scale them (He-scaled weights, gradients that carry the 1/batch of a mean loss),
 where results are O(1) or smaller, and must meet the stated tolerance with no rescaling.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -976,7 +978,8 @@ def test_products_of_few_tiles_cut_their_reduction(shape):
 
 
 @pytest.mark.parametrize("n,k", [(512, 512), (1252, 784), (10, 25088), (777, 2500), (1, 70000), (33, 65), (5000, 3), (7, 1025), (31, 1024),
-                                 (64, 2), (1, 2), (100001, 130), (3, 5000), (32, 63)])
+                                 (64, 2), (1, 2), (100001, 130), (3, 5000), (32, 63), (70001, 2), (333, 16), (65, 17), (129, 32), (63, 33),
+                                 (66, 64), (24575, 65), (24576, 65), (24577, 513), (9, 256), (9, 257), (5, 512), (5, 1023)])
 def test_vector_products_have_one_order(n, k):
     """A matrix times a vector: the same bits whether the matrix is stored by rows or by columns, whichever side it stands on, with
     the epilogues and in a batch.  Bound: six standard deviations of 32 roundings of partial sums no larger than sqrt(k)."""
@@ -1001,6 +1004,19 @@ def test_vector_products_have_one_order(n, k):
         g, x = ops.Tensor((n,)), T(mask)
         capi.check(lib.dopt_hip_sgemm_relu_grad(ta, tb, M, N, k, a.ptr, b.ptr, x.ptr, g.ptr))
         assert np.array_equal(g.numpy(), np.where(mask > 0, got, np.float32(0)))
+    # in a batch: alone, and as blocks of a launch that also computes a small product
+    for beside in (0, 1):
+        jobs = [(a, b, ta, tb, M, N, k) for a, b, ta, tb, M, N in forms]
+        if beside:
+            jobs.append((T(r.standard_normal((40, 24)).astype(np.float32)), T(r.standard_normal((24, 50)).astype(np.float32)), 0, 0, 40, 50, 24))
+        outs, cnt = [T(np.full(j[4] * j[5], 7.0, np.float32)) for j in jobs], len(jobs)
+        arr = lambda t, v: (t * cnt)(*v)
+        capi.check(lib.dopt_hip_sgemm_batch(cnt, arr(C.c_int, [j[2] for j in jobs]), arr(C.c_int, [j[3] for j in jobs]), *[arr(C.c_size_t, [j[q] for j in jobs]) for q in (4, 5, 6)],
+                                            arr(C.c_void_p, [j[0].ptr for j in jobs]), arr(C.c_void_p, [j[1].ptr for j in jobs]), arr(C.c_void_p, [t.ptr for t in outs])))
+        for t in outs[:len(forms)]:
+            assert np.array_equal(t.numpy(), got)
+        if beside:
+            assert np.array_equal(outs[-1].numpy().reshape(40, 50), ops.matmul(jobs[-1][0], jobs[-1][1]).numpy())
 
 
 @pytest.mark.parametrize("shape", [(12, 32768, 32), (32768, 12, 16), (12, 32768, 100), (64, 8192, 512), (8192, 64, 512),
