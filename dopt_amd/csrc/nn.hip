@@ -745,12 +745,14 @@ int dopt_hip_softmax_fwd(size_t N, size_t C, size_t inner, const float *x, float
     } else if (inner == 1 && C >= 64)
         hipLaunchKernelGGL(softmax_rows_fwd_k, dim3((unsigned)ceil_div(N, (size_t)(kBlock / 64))), dim3(kBlock), 0, stream(),
                            N, C, x, y);
+    else if (C == 1 || C > 32)
+        hipLaunchKernelGGL(softmax_fwd_k, dim3(flat_grid(N * inner)), dim3(kBlock), 0, stream(), N, C, inner, x, y);
+    else if (C <= 4)   // (as up to 16 a million rows of two and three took 13.5 and 14.5 us, 6.7 and 7.3 so; one after the other 8 and 11.5)
+        hipLaunchKernelGGL(softmax_few_fwd_k<4>, dim3(flat_grid(N * inner)), dim3(kBlock), 0, stream(), N, (int)C, inner, x, y);
     else if (C <= 16)
         hipLaunchKernelGGL(softmax_few_fwd_k<16>, dim3(flat_grid(N * inner)), dim3(kBlock), 0, stream(), N, (int)C, inner, x, y);
-    else if (C <= 32)
-        hipLaunchKernelGGL(softmax_few_fwd_k<32>, dim3(flat_grid(N * inner)), dim3(kBlock), 0, stream(), N, (int)C, inner, x, y);
     else
-        hipLaunchKernelGGL(softmax_fwd_k, dim3(flat_grid(N * inner)), dim3(kBlock), 0, stream(), N, C, inner, x, y);
+        hipLaunchKernelGGL(softmax_few_fwd_k<32>, dim3(flat_grid(N * inner)), dim3(kBlock), 0, stream(), N, (int)C, inner, x, y);
     DOPT_LAUNCH_CHECK();
     return DOPT_HIP_OK;
 }

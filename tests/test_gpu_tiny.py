@@ -95,7 +95,7 @@ def test_reductions_as_nodes_equal_dopt_hip_reduce(shape, axes, op):
     assert np.array_equal(out.numpy().ravel(), want.ravel(), equal_nan=True)
 
 
-@pytest.mark.parametrize("shape", [(5, 1), (300, 2), (33, 15), (3, 16), (200, 17), (9, 31), (4, 32), (11, 33), (3, 16, 5), (2, 17, 3, 2)])
+@pytest.mark.parametrize("shape", [(5, 1), (300, 2), (100, 3), (70, 4), (64, 5), (9, 1, 7), (33, 15), (3, 16), (200, 17), (9, 31), (4, 32), (11, 33), (3, 16, 5), (2, 17, 3, 2)])
 def test_softmax_of_few_classes(shape):
     """Kept in registers up to 16 and 32 classes: the bits of the node, which takes the classes in the reference's order."""
     r = np.random.default_rng(int(np.prod(shape)))
