@@ -759,8 +759,11 @@ struct ColsSplit {
 };
 bool cols_split(size_t outer, size_t R, size_t inner, ColsSplit *c)
 {
-    if (inner < 2 || R <= 128 || outer * inner >= (size_t)num_cus() * 256 || outer * R * inner <= 4096) return false;
+    if (inner < 2 || outer * inner >= (size_t)num_cus() * 256 || outer * R * inner <= 4096) return false;
     const size_t tiles = ceil_div(inner, (size_t)64);   // (fewer than 2^16 columns)
+    // With more than two blocks a CU a short fold is a wavefront's work either way, and blocks take turns: [3000, 129, 2] 9.5 us by
+    // red_cols, 16.2 so; [300, 200, 65] 7.0 and 8.3; but [600 tiles, 500] 27 and 16, [3000, 500, 10] 30 and 22.
+    if (R <= (outer * tiles > (size_t)num_cus() * 2 ? 256 : 128)) return false;
     c->tiles = (unsigned)tiles;
     c->width = (unsigned)ceil_div(inner, tiles);
     // one launch while a thread has no more than 64 rows; else two blocks on every CU with at least 8 rows a thread, and no more

@@ -176,7 +176,8 @@ def test_sum_of_squares_is_the_sum_of_the_stored_product(shape, axes):
 
 @pytest.mark.parametrize("outer,rows,inner", [
     (1, 129, 32), (1, 1000, 2), (3, 700, 17), (1, 1480, 11), (2, 2049, 64), (1, 1025, 65), (1, 20001, 3), (1, 17310, 17),
-    (1, 9000, 305), (2, 40000, 64), (1, 300, 65535), (1, 129, 65537), (5, 65, 200), (1, 4096, 1024)])
+    (1, 9000, 305), (2, 40000, 64), (1, 300, 65535), (1, 129, 65537), (5, 65, 200), (1, 4096, 1024),
+    (513, 256, 2), (513, 257, 2), (512, 129, 3), (3000, 300, 10)])
 def test_folds_of_few_columns_over_many_rows(outer, rows, inner):
     """Sums and maxima over a middle or leading axis: one thread per column, a workgroup per tile of columns, or slices of rows
     that a second launch adds.  Bound for sums: six standard deviations of 256 roundings (the longest chain) of partial sums that
