@@ -513,8 +513,7 @@ constexpr int kGroupJobs = 8;   // jobs one grouped launch may hold (its descrip
 // when r lies outside the matrix; `pitch`: bytes between consecutive reductions of an r-contiguous operand.
 // A k-contiguous operand is loaded as one 16-byte piece whatever its alignment (see Stage3): word by word, each load touched a
 // line per row, and [29 x 2146] x [2146 x 2424], B stored [2424][2146], took 49 us instead of 20.
-// kCut: the reduction is no multiple of four; what a piece holds past its end is zeroed.
-template <bool kKContig, bool kCut>
+template <bool kKContig>
 __device__ __forceinline__ void small_load(__amdgpu_buffer_rsrc_t rs, unsigned base, unsigned pitch, int kk, int k_end,
                                            float (&v)[4])
 {
@@ -527,7 +526,8 @@ __device__ __forceinline__ void small_load(__amdgpu_buffer_rsrc_t rs, unsigned b
     }
 }
 
-// What the last pieces of a k-contiguous operand hold past the end of the reduction counts as zero.
+// What the last pieces of a k-contiguous operand hold past the end of the reduction counts as zero.  kCut: a reduction of no
+// multiple of four, whose last pieces do.
 template <bool kKContig, bool kCut>
 __device__ __forceinline__ float small_value(const float (&v)[4], int e, int kk, int k_end)
 {
@@ -559,8 +559,8 @@ __device__ __forceinline__ void sgemm_small_body(int M, int N, int K, int lda, i
     const int nsteps = k_begin < k_end ? (k_end - k_begin + 7) / 8 : 0;
 #pragma unroll
     for (int j = 0; j < kSmallDepth; j++) {   // steps past the end fetch nothing
-        small_load<!kTA, kCut>(rsa, abase, apitch, k_begin + 8 * j + 4 * half, k_end, a[j]);
-        small_load<kTB, kCut>(rsb, bbase, bpitch, k_begin + 8 * j + 4 * half, k_end, b[j]);
+        small_load<!kTA>(rsa, abase, apitch, k_begin + 8 * j + 4 * half, k_end, a[j]);
+        small_load<kTB>(rsb, bbase, bpitch, k_begin + 8 * j + 4 * half, k_end, b[j]);
         __builtin_amdgcn_sched_barrier(0);   // in this order: the first step's operands are waited for first
     }
     auto value_a = [&](int j, int s, int e) { return small_value<!kTA, kCut>(a[j], e, k_begin + 8 * (s + j) + 4 * half, k_end); };
@@ -575,8 +575,8 @@ __device__ __forceinline__ void sgemm_small_body(int M, int N, int K, int lda, i
 #pragma unroll
             for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(value_a(j, s, e), value_b(j, s, e), acc, 0, 0, 0);
             const int kk = k_begin + 8 * (s + j + kSmallDepth) + 4 * half;   // this register set's next step
-            small_load<!kTA, kCut>(rsa, abase, apitch, kk, k_end, a[j]);
-            small_load<kTB, kCut>(rsb, bbase, bpitch, kk, k_end, b[j]);
+            small_load<!kTA>(rsa, abase, apitch, kk, k_end, a[j]);
+            small_load<kTB>(rsb, bbase, bpitch, kk, k_end, b[j]);
             __builtin_amdgcn_sched_barrier(0);   // keep each refill behind its own step: sunk to the loop's end, all of them are waited for at once
         }
     }
