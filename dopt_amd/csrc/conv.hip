@@ -2116,10 +2116,11 @@ __global__ __launch_bounds__(768, 1) void conv_bwd_pair_k(PatchConv a, WgradPatc
 
 // out[i] = sum_s partial[s][i], s ascending; plus bias[channel of i] when a bias is given
 // (channel = (i / inner) % C for an [N, C, inner] output).
-// kS > 0: exactly kS splits, all loads issued before the first add.
-template <int kS>
+// kS > 0: exactly kS splits, all loads issued before the first add.  kLoose: the result's n values are no whole quads, or not on
+// the 16-byte grid.
+template <int kS, bool kLoose = false>
 __global__ __launch_bounds__(256) void splitk_reduce_k(size_t n4, int splits, const float4 *partial, float4 *out,
-                                                        const float *bias, unsigned C, unsigned inner)
+                                                        const float *bias, unsigned C, unsigned inner, size_t n = 0)
 {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256) {
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -2159,7 +2160,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_k(size_t n4, int splits, co
             acc.z += bias[((e + 2) / inner) % C];
             acc.w += bias[((e + 3) / inner) % C];
         }
-        out[i] = acc;
+        if constexpr (kLoose) store_loose((float *)out, n, i, acc);
+        else out[i] = acc;
     }
 }
 
@@ -2167,8 +2169,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_k(size_t n4, int splits, co
 // rounding per part was most of the error: 66 -> 13 channels, 3 x 3, one image of 23 x 7, 1.3e-7 off float64, so 3.8e-8, in one
 // part 7e-8; the time is that of the copies' bytes).  kLoose: the result's n values are no whole quads, or not on the 16-byte grid.
 template <bool kLoose>
-__global__ __launch_bounds__(256) void splitk_exact_k(size_t n4, int splits, const float4 *partial, float4 *out, size_t n, const float *bias, unsigned C,
-                                                       unsigned inner)
+__global__ __launch_bounds__(256) void splitk_exact_k(size_t n4, int splits, const float4 *partial, float4 *out, size_t n)
 {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256) {
         double x = 0, y = 0, z = 0, w = 0;
@@ -2187,14 +2188,7 @@ __global__ __launch_bounds__(256) void splitk_exact_k(size_t n4, int splits, con
                 }
             }
         }
-        float4 sum = make_float4((float)x, (float)y, (float)z, (float)w);
-        if (bias) {
-            const size_t e = i * 4;
-            sum.x += bias[(e / inner) % C];
-            sum.y += bias[((e + 1) / inner) % C];
-            sum.z += bias[((e + 2) / inner) % C];
-            sum.w += bias[((e + 3) / inner) % C];
-        }
+        const float4 sum = make_float4((float)x, (float)y, (float)z, (float)w);
         if constexpr (kLoose) store_loose((float *)out, n, i, sum);
         else out[i] = sum;
     }
@@ -2293,14 +2287,14 @@ int check_desc(const dopt_hip_conv_desc *d, size_t *P, size_t *Q, const char *wh
 // Floats from one partial copy of a general kernel's result, or of a filter gradient, to the next.
 size_t copy_stride(size_t elems) { return (elems + 3) / 4 * 4; }
 
-int launch_splitk_exact(size_t elems, int splits, const float *partial, float *out, const float *bias = nullptr, unsigned C = 1, unsigned inner = 1)
+int launch_splitk_exact(size_t elems, int splits, const float *partial, float *out)
 {
     const size_t n4 = copy_stride(elems) / 4;
     const dim3 grid((unsigned)std::min(ceil_div(n4, (size_t)256), (size_t)num_cus() * 8));
     if (elems % 4 != 0 || !aligned16(out))
-        hipLaunchKernelGGL(splitk_exact_k<true>, grid, dim3(256), 0, stream(), n4, splits, (const float4 *)partial, (float4 *)out, elems, bias, C, inner);
+        hipLaunchKernelGGL(splitk_exact_k<true>, grid, dim3(256), 0, stream(), n4, splits, (const float4 *)partial, (float4 *)out, elems);
     else
-        hipLaunchKernelGGL(splitk_exact_k<false>, grid, dim3(256), 0, stream(), n4, splits, (const float4 *)partial, (float4 *)out, elems, bias, C, inner);
+        hipLaunchKernelGGL(splitk_exact_k<false>, grid, dim3(256), 0, stream(), n4, splits, (const float4 *)partial, (float4 *)out, elems);
     DOPT_LAUNCH_CHECK();
     return DOPT_HIP_OK;
 }
@@ -2308,19 +2302,23 @@ int launch_splitk_exact(size_t elems, int splits, const float *partial, float *o
 int launch_splitk_reduce(size_t elems, int splits, const float *partial, float *out, const float *bias = nullptr,
                          unsigned C = 1, unsigned inner = 1)
 {
-    // float4 passes: the caller only splits when elems % 4 == 0, and the partial copies start on
-    // 256-byte boundaries of the workspace; `out` comes from the pool or is checked by the caller
-    const size_t n4 = elems / 4;
+    // float4 passes: the partial copies are whole quads (copy_stride) and start on 256-byte boundaries of the workspace
+    const size_t n4 = copy_stride(elems) / 4;
     size_t blocks = ceil_div(n4, (size_t)256);
     size_t cap = (size_t)num_cus() * 8;
     const dim3 grid((unsigned)(blocks > cap ? cap : (blocks < 1 ? 1 : blocks)));
     const float4 *p4 = (const float4 *)partial;
     float4 *o4 = (float4 *)out;
+    if (elems % 4 != 0 || !aligned16(out)) {   // (the same order)
+        hipLaunchKernelGGL((splitk_reduce_k<0, true>), grid, dim3(256), 0, stream(), n4, splits, p4, o4, bias, C, inner, elems);
+        DOPT_LAUNCH_CHECK();
+        return DOPT_HIP_OK;
+    }
     switch (splits) {
-    case 2: hipLaunchKernelGGL(splitk_reduce_k<2>, grid, dim3(256), 0, stream(), n4, splits, p4, o4, bias, C, inner); break;
-    case 3: hipLaunchKernelGGL(splitk_reduce_k<3>, grid, dim3(256), 0, stream(), n4, splits, p4, o4, bias, C, inner); break;
-    case 4: hipLaunchKernelGGL(splitk_reduce_k<4>, grid, dim3(256), 0, stream(), n4, splits, p4, o4, bias, C, inner); break;
-    default: hipLaunchKernelGGL(splitk_reduce_k<0>, grid, dim3(256), 0, stream(), n4, splits, p4, o4, bias, C, inner); break;
+    case 2: hipLaunchKernelGGL(splitk_reduce_k<2>, grid, dim3(256), 0, stream(), n4, splits, p4, o4, bias, C, inner, elems); break;
+    case 3: hipLaunchKernelGGL(splitk_reduce_k<3>, grid, dim3(256), 0, stream(), n4, splits, p4, o4, bias, C, inner, elems); break;
+    case 4: hipLaunchKernelGGL(splitk_reduce_k<4>, grid, dim3(256), 0, stream(), n4, splits, p4, o4, bias, C, inner, elems); break;
+    default: hipLaunchKernelGGL(splitk_reduce_k<0>, grid, dim3(256), 0, stream(), n4, splits, p4, o4, bias, C, inner, elems); break;
     }
     DOPT_LAUNCH_CHECK();
     return DOPT_HIP_OK;
@@ -3176,9 +3174,8 @@ int run_few(const dopt_hip_conv_desc *d, size_t P, size_t Q, const float *x, con
         open_split_set(partial);
         return DOPT_HIP_OK;
     }
-    if (u.elems % 4 == 0 && aligned16(y))   // in the order in which a later call adds the open copies
-        return launch_splitk_reduce(u.elems, u.cuts, partial, y, bias, (unsigned)d->K, (unsigned)(P * Q));
-    return launch_splitk_exact(u.elems, u.cuts, partial, y, bias, (unsigned)d->K, (unsigned)(P * Q));
+    // in the order in which a later call adds the open copies, wherever the result lies
+    return launch_splitk_reduce(u.elems, u.cuts, partial, y, bias, (unsigned)d->K, (unsigned)(P * Q));
 }
 
 template <class T, int SL, auto kKernel, class Args>

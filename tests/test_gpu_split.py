@@ -533,7 +533,7 @@ def test_results_of_odd_counts_are_cut_too(shape):
 # quads, of one part and of many; strides, no padding, several images; a count of results that is no multiple of four
 @pytest.mark.parametrize("shape", [(1, 400, 1, 1, 300, 1, 0, 1), (1, 257, 5, 5, 33, 5, 2, 1), (31, 29, 3, 3, 45, 3, 0, 1), (1, 64, 4, 8, 32, 3, 1, 1), (3, 131, 1, 11, 65, 3, 1, 1),
                                    (1, 256, 1, 1, 31, 1, 0, 1), (1, 256, 8, 8, 32, 1, 0, 1), (1, 640, 8, 8, 640, 3, 1, 1), (1, 99, 16, 16, 70, 3, 1, 2), (2, 37, 17, 13, 34, 7, 0, 3),
-                                   (4, 512, 2, 2, 64, 3, 1, 1), (1, 2049, 7, 7, 36, 1, 0, 1), (5, 61, 13, 1, 40, 3, 1, 1), (1, 5000, 2, 3, 32, 3, 1, 1)])
+                                   (4, 512, 2, 2, 64, 3, 1, 1), (1, 1024, 4, 4, 32, 1, 0, 1), (1, 2049, 7, 7, 36, 1, 0, 1), (5, 61, 13, 1, 40, 3, 1, 1), (1, 5000, 2, 3, 32, 3, 1, 1)])
 def test_convolution_of_few_pixels(shape):
     import ctypes as C_
     N, C, H, W, K, R, pad, stride = shape
@@ -549,6 +549,7 @@ def test_convolution_of_few_pixels(shape):
     flat = whole.numpy()
     assert (flat[:1] == 7.0).all() and (flat[1 + want.size:] == 7.0).all()
     check_norm(flat[1:1 + want.size].reshape(want.shape), want, C * R * R, shape)
+    assert np.array_equal(flat[1:1 + want.size].reshape(want.shape), got)   # the same sums wherever the result lies
     lib, d = capi.load(), ops.conv_desc(x.shape, w.shape, *ps)
     if lib.dopt_hip_conv_packed_layout(C_.byref(d), 0) == 3:   # left open and closed: the same bits
         tx, tw, tb, o = T(x), T(w), T(b), capi.SplitSum()
