@@ -3910,7 +3910,7 @@ int dopt_hip_conv_fwd_bias_packed_open(const dopt_hip_conv_desc *d, const float 
                                        const float *bias, float *y, dopt_hip_split_sum *open)
 {
     size_t P, Q;
-    if (open) {   // complete unless the patch kernel splits below
+    if (open) {   // complete unless a kernel below leaves parts
         *open = dopt_hip_split_sum{};
         open->value = y;
     }
