@@ -1390,7 +1390,7 @@ void HIPPlan::Builder::formTinyRuns()
                     if (m.op != last) tinyWrites[last].push_back(m.op);
                 const int nslots = (int)slots.size();
                 const auto own = std::make_shared<TinyRun>(nslots, nodes);
-                const HIPPlan *const plan = p;
+                HIPPlan *const plan = p;
                 prebuilt[last] = make([=](const std::vector<const void *> &in, void *out) {
                     void *ptrs[DOPT_HIP_TINY_SLOTS];
                     for (int k = 0; k < nslots; k++) ptrs[k] = slotIn[(size_t)k] >= 0 ? const_cast<void *>(in[(size_t)slotIn[(size_t)k]]) : out;
@@ -1398,6 +1398,7 @@ void HIPPlan::Builder::formTinyRuns()
                     if (!plan->mInOrder)   // (the interpreter goes through memory in the nodes' order)
                         if (int rc = own->launch(ptrs, &done)) return rc;
                     if (done) return (int)DOPT_HIP_OK;
+                    plan->mInterpreted++;
                     return dopt_hip_tiny_graph(nslots, ptrs, (int)nodes.size(), nodes.data());
                 });
                 prebuiltLabel[last] = "tiny*" + std::to_string(nodes.size());
@@ -2794,6 +2795,7 @@ std::string HIPPlan::profile()
         snprintf(line, sizeof(line), "%s %.1f %zu\n", kv.first.c_str(), kv.second.first, kv.second.second);
         s += line;
     }
+    if (mInterpreted && (mFlags & DOPT_HIP_PLAN_TIMING)) s += "tiny(interpreted) 0.0 " + std::to_string(mInterpreted) + "\n";
     return s;
 }
 

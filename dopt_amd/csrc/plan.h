@@ -131,6 +131,7 @@ private:
     // batches of steps that stood apart, whose members may be done in any order, are replaced by their members, and compiled runs
     // of tiny operations, which load everything first, by the interpreter.
     bool mInOrder = false;
+    size_t mInterpreted = 0;                     // runs of tiny operations that were launched without a kernel of their own
     // Arguments that arrive as host arrays (cuda/package.d:367-401 uploads them with a blocking copy on every
     // execution): two slots per argument, each a page-locked staging copy and a device copy, used in turn.  The host
     // array is copied into the staging memory before the call returns (the caller may change it at once, as after the

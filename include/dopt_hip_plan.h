@@ -117,7 +117,8 @@ int dopt_hip_plan_stats(void *plan, size_t *kernels, size_t *buffer_bytes);
    many executions so far were replays of one. */
 int dopt_hip_plan_recordings(void *plan, size_t *recorded, size_t *replays);
 /* CUDAPlan.profiler (cuda/package.d:265): accumulated device microseconds per op type as
-   "opType usec count\n" lines; needs DOPT_HIP_PLAN_TIMING. */
+   "opType usec count\n" lines; needs DOPT_HIP_PLAN_TIMING.  "tiny(interpreted) 0.0 count" among them: how many of the runs of tiny
+   operations were launched without a kernel compiled for them. */
 int dopt_hip_plan_profile(void *plan, char *buf, size_t buf_bytes, size_t *needed);
 /* CUDAPlan.cleanup (cuda/package.d:322-338) */
 int dopt_hip_plan_destroy(void *plan);

@@ -192,18 +192,21 @@ def test_a_loss_tail_as_one_launch_matches_the_oracle():
 UNARY, BINARY = ["neg", "abs", "sgn", "exp", "sqrt", "tanh", "relu"], ["add", "sub", "mul", "div", "max", "min", "lt", "pow"]
 
 
-def _random_run(seed):
-    """A graph of tiny operations of every kind a run may hold, over tensors of odd and even sizes, and its variables."""
+def _random_run(seed, wide=False):
+    """A graph of tiny operations of every kind a run may hold, over tensors of odd and even sizes, and its variables; `wide`: rows
+    of 33 values and more, where a softmax is kept in memory and a fold of several rows is the work of a workgroup."""
     from dopt_amd import core, nnet
     r = np.random.default_rng(seed)
     rows, cols = int(r.choice([1, 2, 7, 33, 64, 100, 257, 400])), int(r.choice([1, 2, 3, 8, 10, 16, 40]))
+    if wide:
+        rows, cols = int(r.choice([1, 2, 3, 4, 5, 11, 40, 64])), int(r.choice([33, 48, 63, 64, 65, 68, 100, 129, 256, 1000, 1025]))
     if rows * cols > 4096:
         cols = 4096 // rows
     var = [core.float32([rows, cols]) for _ in range(3)] + [core.float32([1]), core.float32([rows, 1]), core.float32([1, cols])]
     full, single = list(var[:3]), [var[3]]
     outs = []
     for _ in range(int(r.integers(6, 22))):
-        k, x = r.integers(0, 11), full[r.integers(len(full))]
+        k, x = r.integers(0, 13 if wide else 11), full[r.integers(len(full))]
         y = full[r.integers(len(full))]
         if k < 3:
             op = BINARY[r.integers(len(BINARY))]
@@ -223,8 +226,12 @@ def _random_run(seed):
             full.append(core.matmul(core.matmul(x, core.float32([cols, 1], np.ones(cols, np.float32))), var[5]))
         elif k == 9:
             full.append(core.repeat(single[r.integers(len(single))], [rows * cols]).reshape([rows, cols]) * x)
-        else:
+        elif k == 10:
             single.append(single[r.integers(len(single))] * single[r.integers(len(single))] + var[3])
+        elif k == 11:
+            full.append(core.Operation("softmaxGrad", [x, y], {}) if cols < 64 else x * y)
+        else:
+            full.append(core.repeat((core.sum(x, [1]) if r.random() < 0.5 else core.maxElement(x, [1])).reshape([rows, 1]), [1, cols]) - y)
         if r.random() < 0.3:
             outs.append(full[-1])
     outs += [full[-1], single[-1], core.sum(full[-1] * full[0], [1])]
@@ -247,6 +254,44 @@ def test_runs_compiled_for_a_plan_equal_their_operations(seed):
             a[a.size // 2] = np.inf
         for x, y in zip(plain.execute(args), fused.execute(args)):
             assert np.array_equal(x, y, equal_nan=True)
+
+
+@pytest.mark.parametrize("wide", [False, True], ids=["narrow", "wide"])
+@pytest.mark.parametrize("seed", range(30))
+def test_runs_have_a_kernel_of_their_own(seed, wide):
+    """The runs of a plan are compiled: none is left to the interpreter, and their bits are those of the plan that runs every
+    operation by itself, on one and the other queue and replayed."""
+    from dopt_amd import core
+    var, outs = _random_run(2000 + seed, wide)
+    r = np.random.default_rng(3000 + seed)
+    base = core.PLAN_VIEWS | core.PLAN_FUSE
+    plain = core.compile(outs, 0)
+    plans = [core.compile(outs, base | f) for f in (core.PLAN_TIMING, core.PLAN_OVERLAP_LIGHT, core.PLAN_GRAPH)]
+    dev = {v: ops.Tensor(v.shape) for v in var}
+    for case in range(4):
+        for v, t in dev.items():
+            a = r.standard_normal(v.shape).astype(np.float32)
+            if case == 1 and v is var[0]:
+                a.ravel()[:: max(1, a.size // 3)] = np.nan
+                a.ravel()[a.size // 2] = -np.inf
+            t.set(a)
+        want = plain.execute(dev)
+        for p in plans:
+            for x, y in zip(want, p.execute(dev)):
+                assert np.array_equal(x, y, equal_nan=True)
+    assert "tiny(interpreted)" not in plans[0].profile()
+    assert any(label.startswith("tiny*") for label in plans[0].profile())
+
+
+def test_a_run_with_an_argument_in_its_result_is_interpreted():
+    from dopt_amd import core
+    x, w = core.float32([10, 10]), core.float32([10, 10])
+    a = x * w
+    plan = core.compile([a, core.repeat(core.sum(a, [0]).reshape([1, 10]), [10, 1]) + a * x], core.PLAN_VIEWS | core.PLAN_FUSE | core.PLAN_TIMING)
+    ones = np.ones((10, 10), np.float32)
+    for given, interpreted in ((ones, 0), (ops.Tensor((10, 10), _ptr=plan.result_ptr(a)[0], _owner=plan), 1), (ones, 1)):
+        plan.execute({x: given, w: ones})
+        assert plan.profile().get("tiny(interpreted)", (0, 0))[1] == interpreted
 
 
 def test_a_run_whose_argument_lies_in_its_own_result():
