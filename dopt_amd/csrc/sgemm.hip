@@ -1222,21 +1222,17 @@ Route sgemm_route(int transA, int transB, size_t M, size_t N, size_t K, bool pan
     const size_t tiles32 = ceil_div(M, (size_t)32) * ceil_div(N, (size_t)32);
     const double traffic = (double)tiles32 * 64 * K * sizeof(float);
     const bool small = offsets32 && tiles32 <= 4096 && traffic <= (double)(256 << 20);   // (32-bit byte offsets)
-    // no operand's rows run along the reduction: whether that is whole quads changes nothing ([5112 x 19] from 2575 steps 30 us by
-    // sgemm_rows_k, 24 in eleven parts here)
-    const bool across = transA && !transB;
+    // the rows of the larger operand do not run along the reduction: whether that is whole quads changes little ([5112 x 19] from 2575
+    // steps, A across, 30 us by sgemm_rows_k, 24 in eleven parts here; [11 x 4459] from 5058, B across, 32 uncut, 41 in parts)
+    const bool across = M >= N ? transA : !transB;
     const double traffic_us = traffic / (K % 4 && !across ? 4.5e6 : 10e6);
     // (small_us, which decides between this kernel uncut and sgemm_rows_k, keeps the factor there too: without it [5112 x 19] ran here uncut in
     // 19 us, 3.3e-7 off float64 instead of 1.6e-7)
     const double small_us = 4 + (K % 4 ? 2 : 1) * std::max(traffic / 10e6, 5.5e-3 * K);
-    const double plain_us = 4 + std::max(traffic / 10e6, 5.5e-3 * K);
-    // Only the rows of the smaller operand do: they change little either ([11 x 4459] from 5058 steps, B across, 32 us uncut, 41 in the two
-    // parts that the factor asked for).  Beside plain_us, which is close, what parts take is as well: 8 us, and 8 TB/s.
-    const bool smaller = !across && (M >= N ? transA : !transB);
-    auto parts = [&]() {
-        if (smaller) return small_cuts(M, N, K, tiles32, traffic / 8e6, plain_us, 8.0);
-        return small_cuts(M, N, K, tiles32, traffic_us, across ? plain_us : small_us, 9.5);
-    };
+    const double uncut_us = across ? 4 + std::max(traffic / 10e6, 5.5e-3 * K) : small_us;
+    // Beside that estimate, which is close, what parts take is as well: 8 us, and 8 TB/s where many blocks share the L2 ([21 x 4937] from
+    // 5244 steps 31 us uncut, 34 in three parts; [43 x 1021] from 1770 12 and 8).  The others' are long on both sides.
+    auto parts = [&]() { return across ? small_cuts(M, N, K, tiles32, traffic / 8e6, uncut_us, 8.0) : small_cuts(M, N, K, tiles32, traffic_us, uncut_us, 9.5); };
     const size_t slabs_total = ceil_div(K, (size_t)BK);
     if (M <= 64 || !offsets32) {
         if (small) return parts();
