@@ -1179,8 +1179,8 @@ constexpr RowsShape kRowsShapes[] = {{256, 256, 2.4}, {128, 256, 1.45}, {256, 12
 // parts; [16 x 132] from 944 6.7 us uncut, 8.1 in eight.  The parts take no more space than the operands.  A round is one block per CU, as two
 // on a CU share what it can load: [36 x 2052] from 4000 steps 22.6 us uncut, 29 in two parts (260 blocks), 22.4 in seven; [51 x 1500] from
 // 3000 19.2 in three (282 blocks), 15.5 in five.
-// `us`: what has to be undercut; `fixed_us`: what parts take beside their bytes and steps; `longest`: steps of a part.
-Route small_cuts(size_t M, size_t N, size_t K, size_t tiles, double traffic_us, double us, double fixed_us, size_t longest = ~(size_t)0)
+// `us`: what has to be undercut; `longest`: steps of a part.
+Route small_cuts(size_t M, size_t N, size_t K, size_t tiles, double traffic_us, double us, size_t longest = ~(size_t)0)
 {
     Route r{Route::kSmall, 1, K, 0, 0, 0};
     const unsigned slots = (unsigned)num_cus(), k = (unsigned)K, t = (unsigned)tiles;
@@ -1190,7 +1190,7 @@ Route small_cuts(size_t M, size_t N, size_t K, size_t tiles, double traffic_us, 
         if (depth < 128 || cuts * M * N > M * K + K * N) break;
         if (depth > longest || (k + depth - 1) / depth != cuts) continue;
         const unsigned rounds = (t * cuts + slots - 1) / slots;
-        const double cost = fixed_us + std::max(traffic_us, 5.5e-3 * depth * rounds) + copy_us * cuts;
+        const double cost = 9.5 + std::max(traffic_us, 5.5e-3 * depth * rounds) + copy_us * cuts;
         if (cost >= us) continue;
         us = cost;
         r.cuts = cuts;
@@ -1222,20 +1222,17 @@ Route sgemm_route(int transA, int transB, size_t M, size_t N, size_t K, bool pan
     const size_t tiles32 = ceil_div(M, (size_t)32) * ceil_div(N, (size_t)32);
     const double traffic = (double)tiles32 * 64 * K * sizeof(float);
     const bool small = offsets32 && tiles32 <= 4096 && traffic <= (double)(256 << 20);   // (32-bit byte offsets)
-    // the rows of the larger operand do not run along the reduction: whether that is whole quads changes little ([5112 x 19] from 2575
-    // steps, A across, 30 us by sgemm_rows_k, 24 in eleven parts here; [11 x 4459] from 5058, B across, 32 uncut, 41 in parts)
-    const bool across = M >= N ? transA : !transB;
+    // no operand's rows run along the reduction: whether that is whole quads changes nothing ([5112 x 19] from 2575 steps 30 us by
+    // sgemm_rows_k, 24 in eleven parts here)
+    const bool across = transA && !transB;
     const double traffic_us = traffic / (K % 4 && !across ? 4.5e6 : 10e6);
     // (small_us, which decides between this kernel uncut and sgemm_rows_k, keeps the factor there too: without it [5112 x 19] ran here uncut in
     // 19 us, 3.3e-7 off float64 instead of 1.6e-7)
     const double small_us = 4 + (K % 4 ? 2 : 1) * std::max(traffic / 10e6, 5.5e-3 * K);
     const double uncut_us = across ? 4 + std::max(traffic / 10e6, 5.5e-3 * K) : small_us;
-    // Beside that estimate, which is close, what parts take is as well: 8 us, and 8 TB/s where many blocks share the L2 ([21 x 4937] from
-    // 5244 steps 31 us uncut, 34 in three parts; [43 x 1021] from 1770 12 and 8).  The others' are long on both sides.
-    auto parts = [&]() { return across ? small_cuts(M, N, K, tiles32, traffic / 8e6, uncut_us, 8.0) : small_cuts(M, N, K, tiles32, traffic_us, uncut_us, 9.5); };
     const size_t slabs_total = ceil_div(K, (size_t)BK);
     if (M <= 64 || !offsets32) {
-        if (small) return parts();
+        if (small) return small_cuts(M, N, K, tiles32, traffic_us, uncut_us);
         r.kind = M <= 64 ? Route::kTile64 : Route::kTile128;
         r.bm = M <= 64 ? 64 : 128;
         r.bn = M <= 64 ? 256 : 128;
@@ -1289,11 +1286,11 @@ Route sgemm_route(int transA, int transB, size_t M, size_t N, size_t K, bool pan
             }
         }
     }
-    if (small && small_us < best) return parts();
+    if (small && small_us < best) return small_cuts(M, N, K, tiles32, traffic_us, uncut_us);
     // Else the 32 x 32 tiles only where the reduction is cut into parts whose sums are as close as sgemm_rows_k's: 506 x 36 from 1127
     // steps 13 us and 1.2e-7 off float64; in parts of 256 steps 8 us and 1.2e-7; uncut 9 us and 2.2e-7.
     if (small) {
-        const Route cut = small_cuts(M, N, K, tiles32, traffic_us, best, 9.5, 256);
+        const Route cut = small_cuts(M, N, K, tiles32, traffic_us, best, 256);
         if (cut.cuts > 1) return cut;
     }
     return r;
