@@ -52,6 +52,16 @@ int scratch_alloc(void **ptr, size_t bytes);   // pooled block, NOT zero-filled;
 // shape takes a kernel with that epilogue; *biased says whether it did).
 int sgemm_bias(int transA, int transB, size_t M, size_t N, size_t K, const float *A, const float *B, float *C,
                const float *colbias, int bias_shift, bool *biased);
+// sgemm.hip: dopt_hip_sgemm_t, _rank1, _relu_grad, _batch and _order.  `written`, as a plan calls them: the reduction is cut the same
+// however the operands are stored, so a product that reads a transposed matrix in place gives the bits of the product of its copy.
+// Else it is cut as suits the storage ([52 x 2052] from 4403 steps, both operands across, 24 us; cut as the product of copies 31).
+int product(bool written, int transA, int transB, size_t M, size_t N, size_t K, const float *A, const float *B, float *C);
+int product_rank1(bool written, int transA, int transB, size_t M, size_t N, size_t K, const float *A, const float *B, const float *u, const float *v, int relu,
+                  float *C);
+int product_relu_grad(bool written, int transA, int transB, size_t M, size_t N, size_t K, const float *A, const float *B, const float *x, float *C);
+int product_batch(bool written, int n, const int *transA, const int *transB, const size_t *M, const size_t *N, const size_t *K, const float *const *A,
+                  const float *const *B, float *const *C);
+uint64_t product_order(bool written, int transA, int transB, size_t M, size_t N, size_t K);
 // sgemm.hip: dw[K][C][3][3] = filter gradient of a 3x3, pad-1 convolution over 2x2 images, from x[N][4C]
 // and dy[N][4K] in one launch.  Returns false, with nothing launched, for shapes it does not take.
 bool sgemm_fold2x2(size_t C, size_t K, size_t N, const float *x, const float *dy, float *dw, int *rc);

@@ -181,7 +181,7 @@ void registerBuiltinsOnce()
         }
         const size_t M = a[0], K = a[1], N = b[1];
         return make([=](const std::vector<const void *> &in, void *out) {
-            return dopt_hip_sgemm(M, N, K, (const float *)in[0], (const float *)in[1], (float *)out);
+            return product(true, 0, 0, M, N, K, (const float *)in[0], (const float *)in[1], (float *)out);
         });
     };
 
@@ -803,7 +803,7 @@ void HIPPlan::Builder::foldTransposes()
     // matmul reads a transposed operand in place instead of a copy made by `transpose`, and
     // transpose(matmul(A, B)) is computed as matmul(B^T, A^T); the transposes left without a
     // reader drop out.  Only where the product as rewritten adds its terms in the order of the product
-    // as written (dopt_hip_sgemm_order): a flag or exchanged dimensions can select another kernel, and
+    // as written (product_order): a flag or exchanged dimensions can select another kernel, and
     // a plan with rewrites has to give the bits of the plan without.
     auto is_swap = [&](int t) {
         const Operation &o = g.ops[t];
@@ -833,7 +833,7 @@ void HIPPlan::Builder::foldTransposes()
         f.M = g.ops[mm].shape[0];
         f.N = g.ops[mm].shape[1];
         f.K = g.ops[g.ops[mm].deps[0]].shape[1];
-        const uint64_t as_written = dopt_hip_sgemm_order(0, 0, f.M, f.N, f.K);
+        const uint64_t as_written = product_order(true, 0, 0, f.M, f.N, f.K);
         if (outT) {  // (A B)^T = B^T A^T
             std::swap(f.a, f.b);
             const bool na = !f.tB, nb = !f.tA;
@@ -841,7 +841,7 @@ void HIPPlan::Builder::foldTransposes()
             f.tB = nb;
             std::swap(f.M, f.N);
         }
-        f.same_order = as_written != 0 && dopt_hip_sgemm_order(f.tA, f.tB, f.M, f.N, f.K) == as_written;
+        f.same_order = as_written != 0 && product_order(true, f.tA, f.tB, f.M, f.N, f.K) == as_written;
         return f;
     };
     auto feeds_a_transpose_only = [&](int mm) {
@@ -872,7 +872,7 @@ void HIPPlan::Builder::foldTransposes()
         mmInfo[id].a = a; mmInfo[id].b = b; mmInfo[id].tA = ta; mmInfo[id].tB = tb;
         mmInfo[id].M = M; mmInfo[id].N = N; mmInfo[id].K = K;
         prebuilt[id] = make([=](const std::vector<const void *> &in, void *out) {
-            return dopt_hip_sgemm_t(ta, tb, M, N, K, (const float *)in[0], (const float *)in[1], (float *)out);
+            return product(true, ta, tb, M, N, K, (const float *)in[0], (const float *)in[1], (float *)out);
         });
         prebuiltLabel[id] = outT ? "matmul+transpose" : "matmul";
     }
@@ -916,8 +916,8 @@ void HIPPlan::Builder::fuseDenseLayers()
             const MatmulInfo mi = prod;
             const int relu = clamp ? 1 : 0;
             prebuilt[id] = make([=](const std::vector<const void *> &in, void *out) {
-                return dopt_hip_sgemm_rank1(mi.tA, mi.tB, mi.M, mi.N, mi.K, (const float *)in[0], (const float *)in[1],
-                                            (const float *)in[2], (const float *)in[3], relu, (float *)out);
+                return product_rank1(true, mi.tA, mi.tB, mi.M, mi.N, mi.K, (const float *)in[0], (const float *)in[1],
+                                     (const float *)in[2], (const float *)in[3], relu, (float *)out);
             });
             prebuiltLabel[id] = clamp ? "matmul+broadcast+relu" : "matmul+broadcast";
             prebuilt[pid].reset();   // the product no longer runs on its own
@@ -984,8 +984,8 @@ void HIPPlan::Builder::fuseDenseBackward()
             fusedKind[id] = 9;
             inputsOf[id] = {mi.a, mi.b, op.deps[2]};
             prebuilt[id] = make([=](const std::vector<const void *> &in, void *out) {
-                return dopt_hip_sgemm_relu_grad(mi.tA, mi.tB, mi.M, mi.N, mi.K, (const float *)in[0], (const float *)in[1],
-                                                (const float *)in[2], (float *)out);
+                return product_relu_grad(true, mi.tA, mi.tB, mi.M, mi.N, mi.K, (const float *)in[0], (const float *)in[1],
+                                         (const float *)in[2], (float *)out);
             });
             prebuiltLabel[id] = "matmul+reluGrad";
             prebuilt[pid].reset();   // the product no longer runs on its own
@@ -2126,7 +2126,7 @@ void HIPPlan::Builder::batchIndependent()
                 A[(size_t)j] = (const float *)in[(size_t)(2 * j)];
                 B[(size_t)j] = (const float *)in[(size_t)(2 * j + 1)];
             }
-            return dopt_hip_sgemm_batch(n, tA.data(), tB.data(), M.data(), N.data(), K.data(), A.data(), B.data(), outs.data());
+            return product_batch(true, n, tA.data(), tB.data(), M.data(), N.data(), K.data(), A.data(), B.data(), outs.data());
         });
         b.inputs.resize(b.inputOps.size());
         b.inputBytes.resize(b.inputOps.size());
@@ -2204,7 +2204,7 @@ void HIPPlan::Builder::batchIndependent()
                     B[j] = (const float *)in[2 * j + 1];
                     C[j] = j + 1 < n ? (float *)const_cast<void *>(in[2 * n + j]) : (float *)out;
                 }
-                return dopt_hip_sgemm_batch((int)n, tA.data(), tB.data(), M.data(), N.data(), K.data(), A.data(), B.data(), C.data());
+                return product_batch(true, (int)n, tA.data(), tB.data(), M.data(), N.data(), K.data(), A.data(), B.data(), C.data());
             });
             b.inputs.resize(b.inputOps.size());
             b.inputBytes.resize(b.inputOps.size());

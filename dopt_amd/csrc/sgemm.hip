@@ -1101,6 +1101,7 @@ namespace dopt {
 // What may ride in a product's epilogue besides the bias forms: a reluGrad mask (C = mask > 0 ? product : 0).
 struct Extras {
     const float *mask = nullptr;
+    bool written = false;   // see sgemm_route
 };
 
 // Whether a matrix times a vector finds the matrix stored row by row along the reduction (where both sides are vectors it does).
@@ -1199,7 +1200,9 @@ Route small_cuts(size_t M, size_t N, size_t K, size_t tiles, double traffic_us, 
     return r;
 }
 
-Route sgemm_route(int transA, int transB, size_t M, size_t N, size_t K, bool panel_allowed = true)
+// `written`: the product of a plan, whose reduction is cut the same however its operands are stored - one that reads a transposed
+// matrix in place has to add its terms in the order of the product that was written, of a copy of it.
+Route sgemm_route(int transA, int transB, size_t M, size_t N, size_t K, bool written, bool panel_allowed = true)
 {
     Route r{Route::kNone, 1, K, 0, 0, 0};
     if (M * N == 0 || K == 0) return r;
@@ -1224,7 +1227,7 @@ Route sgemm_route(int transA, int transB, size_t M, size_t N, size_t K, bool pan
     const bool small = offsets32 && tiles32 <= 4096 && traffic <= (double)(256 << 20);   // (32-bit byte offsets)
     // no operand's rows run along the reduction: whether that is whole quads changes nothing ([5112 x 19] from 2575 steps 30 us by
     // sgemm_rows_k, 24 in eleven parts here)
-    const bool across = transA && !transB;
+    const bool across = transA && !transB && !written;
     const double traffic_us = traffic / (K % 4 && !across ? 4.5e6 : 10e6);
     // (small_us, which decides between this kernel uncut and sgemm_rows_k, keeps the factor there too: without it [5112 x 19] ran here uncut in
     // 19 us, 3.3e-7 off float64 instead of 1.6e-7)
@@ -1311,9 +1314,9 @@ int sgemm_epilogue(int transA, int transB, size_t M, size_t N, size_t K, const f
                      M * N < ((size_t)1 << 40),
                  "dopt_hip_sgemm: dimensions too large");
 
-    Route route = sgemm_route(transA, transB, M, N, K);
+    Route route = sgemm_route(transA, transB, M, N, K, ex.written);
     if (route.kind == Route::kPanel && !panel_takes(M, N, K, A, B))   // operands off the 16-byte grid: as if it were not there
-        route = sgemm_route(transA, transB, M, N, K, false);
+        route = sgemm_route(transA, transB, M, N, K, ex.written, false);
     const Route::Kind kind = route.kind;
     if (kind == Route::kOuter) {  // vectors: a transposed vector is the same memory
         hipLaunchKernelGGL(outer_k, dim3(flat_grid(M * N)), dim3(256), 0, stream(), M, N, A, B, C);
@@ -1463,14 +1466,17 @@ bool sgemm_fold2x2_batch(int n, const size_t *C, const size_t *K, const size_t *
     return true;
 }
 
-}  // namespace dopt
-
-extern "C" {
-
-int dopt_hip_sgemm_batch(int n, const int *transA, const int *transB, const size_t *M, const size_t *N, const size_t *K,
-                         const float *const *A, const float *const *B, float *const *C)
+int product(bool written, int transA, int transB, size_t M, size_t N, size_t K, const float *A, const float *B, float *C)
 {
-    using namespace dopt;
+    Extras ex;
+    ex.written = written;
+    bool applied;
+    return sgemm_epilogue(transA, transB, M, N, K, A, B, C, nullptr, 0, nullptr, 0, &applied, ex);
+}
+
+int product_batch(bool written, int n, const int *transA, const int *transB, const size_t *M, const size_t *N, const size_t *K, const float *const *A,
+                  const float *const *B, float *const *C)
+{
     DOPT_REQUIRE(n >= 0 && (n == 0 || (transA && transB && M && N && K && A && B && C)), "dopt_hip_sgemm_batch: null argument");
     DOPT_ENSURE_INIT();
     // Products that take the 32 x 32-tile kernel (grouped per template instance) or the short column sum share launches;
@@ -1482,7 +1488,7 @@ int dopt_hip_sgemm_batch(int n, const int *transA, const int *transB, const size
     for (int i = 0; i < n; i++) {
         if (M[i] * N[i] == 0) continue;
         const bool plain = K[i] > 0 && A[i] && B[i] && C[i] && M[i] < ((size_t)1 << 30) && N[i] < ((size_t)1 << 30) && K[i] < ((size_t)1 << 30);
-        const Route r = plain ? sgemm_route(transA[i], transB[i], M[i], N[i], K[i]) : Route{Route::kNone, 1, 0, 0, 0, 0};
+        const Route r = plain ? sgemm_route(transA[i], transB[i], M[i], N[i], K[i], written) : Route{Route::kNone, 1, 0, 0, 0, 0};
         if (r.kind == Route::kGemv && r.cuts == 1 && !gemv_by_rows(transA[i], transB[i], M[i], N[i]) && gemvs.size() < (size_t)kGroupJobs) {
             const size_t R = M[i] == 1 ? N[i] : M[i];
             GemvJob q{};
@@ -1536,45 +1542,70 @@ int dopt_hip_sgemm_batch(int n, const int *transA, const int *transB, const size
         if (int rc = launch_gemv_cols(v.K, v.N, 1, v.a, v.B, v.c, VectorEpilogue{nullptr, nullptr, nullptr, 0, 0, 1})) return rc;
     }
     for (int i : single)
-        if (int rc = dopt_hip_sgemm_t(transA[i], transB[i], M[i], N[i], K[i], A[i], B[i], C[i])) return rc;
+        if (int rc = product(written, transA[i], transB[i], M[i], N[i], K[i], A[i], B[i], C[i])) return rc;
     return DOPT_HIP_OK;
+}
+
+int product_rank1(bool written, int transA, int transB, size_t M, size_t N, size_t K, const float *A, const float *B, const float *u, const float *v, int relu,
+                  float *C)
+{
+    DOPT_REQUIRE((u == nullptr) == (v == nullptr), "dopt_hip_sgemm_rank1: u and v go together");
+    Extras ex;
+    ex.written = written;
+    bool applied = false;
+    if (int rc = sgemm_epilogue(transA, transB, M, N, K, A, B, C, v, 0, u, relu, &applied, ex)) return rc;
+    if (applied || M * N == 0 || (!v && !relu)) return DOPT_HIP_OK;
+    hipLaunchKernelGGL(rank1_epilogue_k, dim3(flat_grid(M * N)), dim3(256), 0, stream(), M, N, u, v, relu, C);
+    DOPT_LAUNCH_CHECK();
+    return DOPT_HIP_OK;
+}
+
+int product_relu_grad(bool written, int transA, int transB, size_t M, size_t N, size_t K, const float *A, const float *B, const float *x, float *C)
+{
+    DOPT_REQUIRE(x != nullptr || M * N == 0, "dopt_hip_sgemm_relu_grad: null argument");
+    Extras ex;
+    ex.mask = x;
+    ex.written = written;
+    bool applied = false;
+    if (int rc = sgemm_epilogue(transA, transB, M, N, K, A, B, C, nullptr, 0, nullptr, 0, &applied, ex)) return rc;
+    if (applied || M * N == 0) return DOPT_HIP_OK;
+    return dopt_hip_relu_bwd(M * N, C, x, C);   // in place: every element is read before it is written
+}
+
+uint64_t product_order(bool written, int transA, int transB, size_t M, size_t N, size_t K)
+{
+    if (!ensure_init()) return 0;   // the cut of a reduction follows the device's size
+    const Route r = sgemm_route(transA, transB, M, N, K, written);
+    return (uint64_t)r.kind | (uint64_t)r.cuts << 8 | (uint64_t)r.depth << 24 | (uint64_t)r.pass << 52;
+}
+
+}  // namespace dopt
+
+extern "C" {
+
+int dopt_hip_sgemm_batch(int n, const int *transA, const int *transB, const size_t *M, const size_t *N, const size_t *K,
+                         const float *const *A, const float *const *B, float *const *C)
+{
+    return product_batch(false, n, transA, transB, M, N, K, A, B, C);
 }
 
 int dopt_hip_sgemm_rank1(int transA, int transB, size_t M, size_t N, size_t K, const float *A, const float *B,
                          const float *u, const float *v, int relu, float *C)
 {
-    DOPT_REQUIRE((u == nullptr) == (v == nullptr), "dopt_hip_sgemm_rank1: u and v go together");
-    bool applied = false;
-    if (int rc = dopt::sgemm_epilogue(transA, transB, M, N, K, A, B, C, v, 0, u, relu, &applied)) return rc;
-    if (applied || M * N == 0 || (!v && !relu)) return DOPT_HIP_OK;
-    hipLaunchKernelGGL(rank1_epilogue_k, dim3(flat_grid(M * N)), dim3(256), 0, dopt::stream(), M, N, u, v, relu, C);
-    DOPT_LAUNCH_CHECK();
-    return DOPT_HIP_OK;
+    return product_rank1(false, transA, transB, M, N, K, A, B, u, v, relu, C);
 }
 
 int dopt_hip_sgemm_relu_grad(int transA, int transB, size_t M, size_t N, size_t K, const float *A, const float *B,
                              const float *x, float *C)
 {
-    DOPT_REQUIRE(x != nullptr || M * N == 0, "dopt_hip_sgemm_relu_grad: null argument");
-    dopt::Extras ex;
-    ex.mask = x;
-    bool applied = false;
-    if (int rc = dopt::sgemm_epilogue(transA, transB, M, N, K, A, B, C, nullptr, 0, nullptr, 0, &applied, ex)) return rc;
-    if (applied || M * N == 0) return DOPT_HIP_OK;
-    return dopt_hip_relu_bwd(M * N, C, x, C);   // in place: every element is read before it is written
+    return product_relu_grad(false, transA, transB, M, N, K, A, B, x, C);
 }
 
-uint64_t dopt_hip_sgemm_order(int transA, int transB, size_t M, size_t N, size_t K)
-{
-    if (!dopt::ensure_init()) return 0;   // the cut of a reduction follows the device's size
-    const dopt::Route r = dopt::sgemm_route(transA, transB, M, N, K);
-    return (uint64_t)r.kind | (uint64_t)r.cuts << 8 | (uint64_t)r.depth << 24 | (uint64_t)r.pass << 52;
-}
+uint64_t dopt_hip_sgemm_order(int transA, int transB, size_t M, size_t N, size_t K) { return product_order(false, transA, transB, M, N, K); }
 
 int dopt_hip_sgemm_t(int transA, int transB, size_t M, size_t N, size_t K, const float *A, const float *B, float *C)
 {
-    bool biased;
-    return dopt::sgemm_bias(transA, transB, M, N, K, A, B, C, nullptr, 0, &biased);
+    return product(false, transA, transB, M, N, K, A, B, C);
 }
 
 int dopt_hip_sgemm(size_t M, size_t N, size_t K, const float *A, const float *B, float *C)

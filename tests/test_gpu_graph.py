@@ -643,6 +643,22 @@ def test_output_only_products_of_a_plan_share_a_launch():
         assert np.array_equal(a, b) or (a.ndim == 1 and np.allclose(a, b, rtol=0, atol=2e-5))
 
 
+# reductions of odd lengths, whose cut depends on how the operands of a call of its own are stored
+@pytest.mark.parametrize("M,N,K", [(88, 632, 2990), (607, 11, 2019), (34, 574, 927), (978, 52, 8010), (312, 8, 3279), (64, 32, 959), (2, 191, 905), (3170, 21, 4739)])
+@pytest.mark.parametrize("tA,tB", [(1, 0), (0, 1), (1, 1)])
+def test_products_read_transposed_operands_of_odd_reductions_in_place(M, N, K, tA, tB):
+    r = np.random.default_rng(M + N)
+    a, b = (float32(list(s), r.standard_normal(s).astype(np.float32)) for s in ((K, M) if tA else (M, K), (N, K) if tB else (K, N)))
+    left, right = core.transpose(a, (1, 0)) if tA else a, core.transpose(b, (1, 0)) if tB else b
+    y = core.matmul(left, right)
+    outs = [y, core.relu(y + core.matmul(float32([M, 1], np.ones((M, 1), np.float32)), float32([1, N], r.standard_normal((1, N)).astype(np.float32))))]
+    want = core.compile(outs, 0).execute()
+    plan = core.compile(outs, core.PLAN_VIEWS | core.PLAN_FUSE | core.PLAN_TIMING)
+    for x, w in zip(plan.execute(), want):
+        assert np.array_equal(x, w)
+    assert not any("transpose" in label for label in plan.profile()), plan.profile()
+
+
 @pytest.mark.parametrize("where", ["product", "between"])
 @pytest.mark.parametrize("read", [True, False], ids=["read later", "outputs"])
 def test_batched_products_with_an_argument_in_a_result(read, where):
