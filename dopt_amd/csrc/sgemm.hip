@@ -838,18 +838,32 @@ struct VectorEpilogue {   // + rowvec[row] * colbias[col >> shift], relu, mask, 
 };
 
 // The matrix is stored row by row along the reduction: a wavefront per result, a lane per chain.
-// kFew: up to four steps of 64, where all the rest is only what a wavefront has to go through (3 000 000 rows of 2 steps 437 us with the
-// loops below, 314 so; 30000 of 64 6.7 and 4.5, of 129 7.7 and 5.4).
-template <bool kFew>
+// kSteps > 0: at most so many steps of 64, where all of the loops below is only what a wavefront has to go through.  Up to four one
+// after the other (3 000 000 rows of 2 steps 437 us with the loops, 314 so; 30000 of 64 6.7 and 4.5, of 129 7.7 and 5.4), more all
+// together (8333 rows of 512 4.5 us one after the other, 3.8 with the loops, 3.6 so; 6057 of 429 3.8, 3.8 and 3.1; 25648 of 272 9.1, 8.2 and 6.5).
+template <int kSteps>
 __global__ __launch_bounds__(256) void gemv_rows_k(size_t M, size_t K, const float *A, const float *b, float *c, VectorEpilogue ep)
 {
     const size_t row = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= M) return;
     const int lane = threadIdx.x & 63;
     const float *ar = A + row * K;
-    if constexpr (kFew) {
+    if constexpr (kSteps > 0) {
         float acc = 0.0f;
-        for (size_t k = lane; k < K; k += 64) acc += ar[k] * b[k];
+        if constexpr (kSteps <= 4) {
+            for (size_t k = lane; k < K; k += 64) acc += ar[k] * b[k];
+        } else {
+            const int last = (int)K - 1;
+            float x[kSteps], y[kSteps];
+#pragma unroll
+            for (int u = 0; u < kSteps; u++) {   // (clamped, not branched)
+                x[u] = ar[min(64 * u + lane, last)];
+                y[u] = b[min(64 * u + lane, last)];
+            }
+#pragma unroll
+            for (int u = 0; u < kSteps; u++)
+                if (64 * u + lane <= last) acc += x[u] * y[u];
+        }
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
         if (lane == 0) c[row] = ep(acc, row);
@@ -890,32 +904,34 @@ __global__ __launch_bounds__(256) void gemv_rows_k(size_t M, size_t K, const flo
     if (lane == 0) c[row] = ep(total, row);
 }
 
-// The matrix is stored [K][N]: a block of 256 threads folds one slice of 256 / kGroups columns, a thread 64 / kGroups neighbouring
-// chains of a column.  kLive: a reduction of so many steps at most, whose other chains are zeros that change nothing.
-template <int kGroups, int kLive = 64>
+// The matrix is stored [K][N]: a block of 256 threads folds one slice of 256 / kGroups columns, a thread every kGroups-th chain of a
+// column, so that all halves but the last are added in its registers and one value a thread meets the others' in LDS (with
+// neighbouring chains, all of which met there, 2855 columns of 64 steps 2.8 us, 2.5 so; 7182 of 799 9.7 and 8.9).  kLive: a reduction of so many steps at most; chains
+// beyond them are zeros that change nothing.
+template <int kGroups, int kLive = kGemvSlice>
 struct GemvLds {
-    static constexpr int kCols = 256 / kGroups, kChains = kLive / kGroups;
-    float chain[kGroups / 2][kChains][kCols];   // upper half of the groups, chain, column
+    static constexpr int kCols = 256 / kGroups, kChains = (kLive < 64 ? kLive : 64) / kGroups;
+    float sum[kGroups][kCols];
 };
-// (`on`: false for the threads of a larger block that only keep the barriers company)
-template <int kGroups, int kLive = 64, class Store>
+// (`on`: false for the threads of a larger block that only keep the barrier company)
+template <int kGroups, int kLive = kGemvSlice, class Store>
 __device__ __forceinline__ void gemv_cols_body(int K, int N, const float *a, const float *B, int bx, int k0, bool on, GemvLds<kGroups, kLive> &lds, Store &&store)
 {
     constexpr int kCols = GemvLds<kGroups, kLive>::kCols, kChains = GemvLds<kGroups, kLive>::kChains;
-    constexpr int kSteps = kLive == 64 && kChains < 16 ? 16 / kChains : 1;   // sixteen loads in flight
+    constexpr int kSteps = kLive > 64 && kChains < 16 ? 16 / kChains : 1;   // sixteen loads in flight
     const int col = threadIdx.x % kCols, g = threadIdx.x / kCols % kGroups, k1 = min(K, k0 + kGemvSlice);
     const int n = min(bx * kCols + col, N - 1);
     float acc[kChains];
 #pragma unroll
     for (int j = 0; j < kChains; j++) acc[j] = 0.0f;
     if (on) {
-        for (int k = k0 + kChains * g; k < k1; k += 64 * kSteps) {   // (clamped, not branched)
+        auto steps = [&](int k, auto whole) {   // (the last ones clamped, not branched)
             float av[kSteps][kChains], bv[kSteps][kChains];
 #pragma unroll
             for (int u = 0; u < kSteps; u++)
 #pragma unroll
                 for (int j = 0; j < kChains; j++) {
-                    const int at = min(k + 64 * u + j, K - 1);
+                    const int step = k + 64 * u + kGroups * j + g, at = whole ? step : min(step, k1 - 1);
                     av[u][j] = a[at];
                     bv[u][j] = B[(size_t)at * N + n];
                 }
@@ -923,27 +939,30 @@ __device__ __forceinline__ void gemv_cols_body(int K, int N, const float *a, con
             for (int u = 0; u < kSteps; u++)
 #pragma unroll
                 for (int j = 0; j < kChains; j++)
-                    if (k + 64 * u + j < k1) acc[j] += av[u][j] * bv[u][j];
-        }
+                    if (whole || k + 64 * u + kGroups * j + g < k1) acc[j] += av[u][j] * bv[u][j];
+        };
+        int k = k0;
+        if constexpr (kLive > 64)
+            for (; k + 64 * kSteps <= k1; k += 64 * kSteps) steps(k, std::true_type());
+        if (kLive <= 64 || k < k1) steps(k, std::false_type());
     }
 #pragma unroll
-    for (int half = kGroups / 2; half > 0; half >>= 1) {   // groups: chains kLive / 2, kLive / 4 .. apart
-        if (on && g >= half && g < 2 * half) {
-#pragma unroll
-            for (int j = 0; j < kChains; j++) lds.chain[g - half][j][col] = acc[j];
-        }
-        __syncthreads();
-        if (on && g < half) {
-#pragma unroll
-            for (int j = 0; j < kChains; j++) acc[j] += lds.chain[g][j][col];
-        }
-        if (half > 1) __syncthreads();
-    }
-#pragma unroll
-    for (int half = kChains / 2; half > 0; half >>= 1)
+    for (int half = kChains / 2; half > 0; half >>= 1)   // chains 32 (fewer, if fewer are live) .. kGroups apart
 #pragma unroll
         for (int j = 0; j < half; j++) acc[j] += acc[j + half];
-    if (on && g == 0 && bx * kCols + col < N) store(bx * kCols + col, acc[0]);
+    if (on && g > 0) lds.sum[g][col] = acc[0];
+    __syncthreads();
+    if (on && g == 0) {
+        float s[kGroups];
+        s[0] = acc[0];
+#pragma unroll
+        for (int i = 1; i < kGroups; i++) s[i] = lds.sum[i][col];
+#pragma unroll
+        for (int half = kGroups / 2; half > 0; half >>= 1)
+#pragma unroll
+            for (int i = 0; i < half; i++) s[i] += s[i + half];
+        if (bx * kCols + col < N) store(bx * kCols + col, s[0]);
+    }
 }
 
 // blockIdx.y: the slice.  With more than one their sums go to consecutive copies of the result, which splitk_epilogue_k adds
@@ -956,10 +975,11 @@ __global__ __launch_bounds__(256) void gemv_cols_k(int K, int N, const float *a,
     gemv_cols_body<kGroups, kLive>(K, N, a, B, (int)blockIdx.x, (int)blockIdx.y * kGemvSlice, true, lds,
                                    [&](int n, float v) { to[n] = ep(v, (size_t)n); });
 }
-// Eight groups, so that few columns make as many threads as they can.  Four where there are 96 columns a CU, as sums that meet in LDS
-// and groups without a step of their own cost more then (30000 columns of 256 steps 7.8 us with eight, 7.0 with four; 16384 of 512
-// 5.1 and 7.0), and for reductions of up to 64 steps, of which a thread takes no more chains than there are (3 000 000 columns of 2 steps
-// 62 us with eight groups, 16 so; of 64 170 and 137; one group of all chains 13 and 139, but 300000 of 64 15.4, 13.8 with eight, 12.8 so).
+// Eight groups, so that few columns make as many threads as they can.  Four where there are 64 columns a CU, a block of 64 for each
+// (16913 columns of 679 steps 15.4 us with eight, 11.8 so; 22431 of 192 5.1 and 4.1; 14186 of 752 14.1 and 11.4, but 13302 of 244 4.1 and 4.7),
+// but eight up to 96 columns a CU while they have all of the reduction in flight at once (18260 of 68 3.0 us with eight, 3.3 with four; 44921
+// of 111 6.3 and 4.3), and for reductions of up to 64 steps, of which a thread takes no more chains than there are (3 000 000 columns of 2 steps 62 us
+// with eight groups, 16 so; of 64 170 and 137; one group of all chains 13 and 139, but 300000 of 64 15.4, 13.8 with eight, 12.8 so).
 constexpr int kGemvGroups = 8;
 
 // Several independent small products in ONE launch: the weight and bias gradients of a dense head are six kernels of a
@@ -1107,7 +1127,7 @@ struct Extras {
 // Whether a matrix times a vector finds the matrix stored row by row along the reduction (where both sides are vectors it does).
 bool gemv_by_rows(int transA, int transB, size_t M, size_t N) { return (N == 1 && !transA) || (M == 1 && transB) || (M == 1 && N == 1); }
 
-template <int kGroups, int kLive = 64>
+template <int kGroups, int kLive = kGemvSlice>
 void launch_gemv_groups(int K, int N, size_t slices, const float *a, const float *B, float *c, const VectorEpilogue &ep)
 {
     const dim3 grid((unsigned)ceil_div((size_t)N, (size_t)GemvLds<kGroups, kLive>::kCols), (unsigned)slices);
@@ -1117,7 +1137,8 @@ int launch_gemv_cols(int K, int N, size_t slices, const float *a, const float *B
 {
     if (K <= 16) launch_gemv_groups<4, 16>(K, N, slices, a, B, c, ep);
     else if (K <= 32) launch_gemv_groups<4, 32>(K, N, slices, a, B, c, ep);
-    else if (K <= 64 || N >= 96 * num_cus()) launch_gemv_groups<4>(K, N, slices, a, B, c, ep);
+    else if (K <= 64) launch_gemv_groups<4, 64>(K, N, slices, a, B, c, ep);
+    else if (N >= (K <= 128 ? 96 : 64) * num_cus()) launch_gemv_groups<4>(K, N, slices, a, B, c, ep);
     else launch_gemv_groups<kGemvGroups>(K, N, slices, a, B, c, ep);
     DOPT_LAUNCH_CHECK();
     return DOPT_HIP_OK;
@@ -1330,8 +1351,10 @@ int sgemm_epilogue(int transA, int transB, size_t M, size_t N, size_t K, const f
         *biased = true;
         if (gemv_by_rows(transA, transB, M, N)) {
             const dim3 grid((unsigned)ceil_div(R, (size_t)4));
-            if (K <= 256) hipLaunchKernelGGL(gemv_rows_k<true>, grid, dim3(256), 0, stream(), R, K, mat, vec, C, ep);
-            else hipLaunchKernelGGL(gemv_rows_k<false>, grid, dim3(256), 0, stream(), R, K, mat, vec, C, ep);
+            if (K <= 256) hipLaunchKernelGGL(gemv_rows_k<4>, grid, dim3(256), 0, stream(), R, K, mat, vec, C, ep);
+            else if (K <= 384) hipLaunchKernelGGL(gemv_rows_k<6>, grid, dim3(256), 0, stream(), R, K, mat, vec, C, ep);
+            else if (K <= 512) hipLaunchKernelGGL(gemv_rows_k<8>, grid, dim3(256), 0, stream(), R, K, mat, vec, C, ep);
+            else hipLaunchKernelGGL(gemv_rows_k<0>, grid, dim3(256), 0, stream(), R, K, mat, vec, C, ep);
             DOPT_LAUNCH_CHECK();
             return DOPT_HIP_OK;
         }

@@ -980,7 +980,8 @@ def test_products_of_few_tiles_cut_their_reduction(shape):
 
 @pytest.mark.parametrize("n,k", [(512, 512), (1252, 784), (10, 25088), (777, 2500), (1, 70000), (33, 65), (5000, 3), (7, 1025), (31, 1024),
                                  (64, 2), (1, 2), (100001, 130), (3, 5000), (32, 63), (70001, 2), (333, 16), (65, 17), (129, 32), (63, 33),
-                                 (66, 64), (24575, 65), (24576, 65), (24577, 513), (9, 256), (9, 257), (5, 512), (5, 1023)])
+                                 (66, 64), (24575, 65), (24576, 65), (24577, 513), (9, 256), (9, 257), (5, 512), (5, 1023),
+                                 (5, 384), (6, 385), (5, 513), (16383, 129), (16384, 129), (24575, 128), (24576, 128)])
 def test_vector_products_have_one_order(n, k):
     """A matrix times a vector: the same bits whether the matrix is stored by rows or by columns, whichever side it stands on, with
     the epilogues and in a batch.  Bound: six standard deviations of 32 roundings of partial sums no larger than sqrt(k)."""
