@@ -1201,20 +1201,25 @@ constexpr RowsShape kRowsShapes[] = {{256, 256, 2.4}, {128, 256, 1.45}, {256, 12
 // parts; [16 x 132] from 944 6.7 us uncut, 8.1 in eight.  The parts take no more space than the operands.  A round is one block per CU, as two
 // on a CU share what it can load: [36 x 2052] from 4000 steps 22.6 us uncut, 29 in two parts (260 blocks), 22.4 in seven; [51 x 1500] from
 // 3000 19.2 in three (282 blocks), 15.5 in five.
-// `us`: what has to be undercut; `longest`: steps of a part.
+// `us`: what has to be undercut; `longest`: steps of a part.  Where rows off the 16-byte grid have raised `traffic_us` it hides what more
+// parts give, so there they are also taken if they give half a microsecond without that ([64 x 640] from 8001 steps 24 us in three
+// parts, 16 in six; [11 x 4459] from 5058 42 in two, 30 in five; [9 x 1538] from 4446 19 in two, 11 in five).
 Route small_cuts(size_t M, size_t N, size_t K, size_t tiles, double traffic_us, double us, size_t longest = ~(size_t)0)
 {
     Route r{Route::kSmall, 1, K, 0, 0, 0};
     const unsigned slots = (unsigned)num_cus(), k = (unsigned)K, t = (unsigned)tiles;
-    const double copy_us = 8.0 * M * N / 5e6;
+    const double copy_us = 8.0 * M * N / 5e6, grid_us = (double)tiles * 64 * K * sizeof(float) / 10e6;
+    double on_grid = 0;
     for (unsigned cuts = 2; cuts <= 32; cuts++) {
         const unsigned depth = ((k + cuts - 1) / cuts + 63) / 64 * 64;
         if (depth < 128 || cuts * M * N > M * K + K * N) break;
         if (depth > longest || (k + depth - 1) / depth != cuts) continue;
         const unsigned rounds = (t * cuts + slots - 1) / slots;
-        const double cost = 9.5 + std::max(traffic_us, 5.5e-3 * depth * rounds) + copy_us * cuts;
-        if (cost >= us) continue;
-        us = cost;
+        const double lasts = 5.5e-3 * depth * rounds, cost = 9.5 + std::max(traffic_us, lasts) + copy_us * cuts;
+        const double even = std::max(grid_us, lasts) + copy_us * cuts;
+        if (cost >= us && (r.cuts == 1 || even >= on_grid - 0.5)) continue;
+        us = std::min(us, cost);
+        on_grid = even;
         r.cuts = cuts;
         r.depth = depth;
     }

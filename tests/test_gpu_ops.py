@@ -978,6 +978,14 @@ def test_products_of_few_tiles_cut_their_reduction(shape):
             assert np.array_equal(g.numpy(), np.where(mask > 0, got, np.float32(0)))
 
 
+@pytest.mark.parametrize("M,N,even,odd", [(64, 640, 8000, 8001), (20, 1100, 7000, 7001), (16, 2000, 6000, 6001), (11, 4459, 5056, 5058)])
+def test_reductions_off_the_grid_are_cut_as_those_on_it(M, N, even, odd):
+    from dopt_amd import capi
+    parts = lambda ta, tb, K: capi.load().dopt_hip_sgemm_order(ta, tb, M, N, K) >> 8 & 0xffff
+    for ta, tb in [(0, 0), (0, 1), (1, 1)]:
+        assert 1.5 * parts(ta, tb, odd) >= parts(ta, tb, even) > 1
+
+
 @pytest.mark.parametrize("n,k", [(512, 512), (1252, 784), (10, 25088), (777, 2500), (1, 70000), (33, 65), (5000, 3), (7, 1025), (31, 1024),
                                  (64, 2), (1, 2), (100001, 130), (3, 5000), (32, 63), (70001, 2), (333, 16), (65, 17), (129, 32), (63, 33),
                                  (66, 64), (24575, 65), (24576, 65), (24577, 513), (9, 256), (9, 257), (5, 512), (5, 1023),
