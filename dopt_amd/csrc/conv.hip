@@ -2991,7 +2991,8 @@ int run_dense2x2_wgrad(const dopt_hip_conv_desc *d, const float *dy, const float
 // is read once, as it lies: a row of it, [C][R][S], is the reduction in order, four steps of which a lane loads as 16 bytes whatever
 // their alignment, and the fp32 matrix instruction takes (32 rows, two steps).  A workgroup owns 32 rows, all pixels and a part
 // of the reduction, its eight wavefronts an eighth of that each.  The input under the part's channels lies in LDS with a halo of
-// zeros; a step's offset in it is read from a table.  Bound by the filter's bytes through launch and latency (512 -> 512 channels, 3 x 3, 16 pixels: 9.4 MB).
+// zeros; a step's offset in it is read from a table.  Bound by launch and latency: 8.9 MB read (256 and 512 -> 512 channels, 3 x 3, 16 and 4 pixels,
+// on average) in 7.9 us are 1.1 TB/s, the CUs have work during 44 % of the cycles counted around a launch, the matrix cores during 10.
 // VGG-16 on one image, 261 us, now 191: its nine layers on 8 x 8, 4 x 4 and 2 x 2 images 7 to 9 us each (Winograd 9 to 11 and 17 to pack
 // their filters, conv2x2_direct_k 15).
 struct FewConv {
@@ -3102,7 +3103,7 @@ struct FewSetup {
 };
 // Against the kernels that run without it (transposed bf16 tiles, Winograd with its packing, a copy of the filter in rows and general
 // tiles): 512 -> 512 channels on 4 x 4 34 us, now 12; 640 -> 640 on 8 x 8 36, now 17; 320 -> 640 at stride 2 to 8 x 8 32, now 15;
-// 100 -> 201 on 7 x 9 48, now 11; 256 -> 32 on 4 x 4 20, now 9; 400 -> 300 on one pixel 15, now 8; nothing of 35 shapes slower.
+// 100 -> 201 on 7 x 9 48, now 11; 256 -> 32 on 4 x 4 20, now 9; 400 -> 300 on one pixel 15, now 8.
 // The kernels of 2 x 2 images keep more than 32 pixels (512 -> 512 of 16 images: 14 us, 17 here), conv2x2_direct_k fewer than 384
 // input channels too (320 -> 320 of 8 images: 9.9 us, 10.7 here; 512 -> 512 of 8 images 14.0, 12.8 here, of one 13.8, 11.3 here).  Filters of
 // 2^27 values and more keep the kernels that are checked at such sizes (5120 -> 512 on 4 x 4, 94 MB, 117 us, now 39).
